@@ -630,6 +630,13 @@ int fc_run(const float* X, uint32_t ldx, const float* W, uint32_t ldw, int trans
            uint32_t* seg_width, void* out_planes)
 {
     if (seg_width) *seg_width = 0;
+    const bool small = !transposed && !accumulate && ((uintptr_t)X % 16) == 0 && (ldx % 4) == 0 && (k == 128 || k == 256) &&
+                       (uint64_t)batch * n <= (1u << 20);   // the one-round-trip kernel's shapes
+    if (!(small && n < 4096) && fc_rows_takes(batch, k, n, ldx, ldw, transposed)) {
+        int rc = fc_rows_run(X, ldx, W, ldw, bias, Z, ldz, batch, k, n, accumulate, activation, params, seg_max, seg_width);
+        if (rc == DSX_OK && out_planes) rc = fc_split_planes_run(Z, ldz, 1, batch, n, out_planes);
+        return rc;
+    }
     FcArgs a{};
     a.X = X; a.W = W; a.bias = bias; a.Z = Z;
     a.ldx = ldx; a.ldw = ldw; a.ldz = ldz;
@@ -657,7 +664,7 @@ int fc_run(const float* X, uint32_t ldx, const float* W, uint32_t ldw, int trans
         // and the kernels of other streams that share the CUs find 17 KiB of LDS taken per workgroup instead of 34.
         if (k <= 256) launch_fc_shape<2, 2, 8>(a, xv, wv, transposed != 0);
         else launch_fc_shape<2, 2, 16>(a, xv, wv, transposed != 0);
-    } else if (!transposed && !accumulate && xv == 4 && (k == 128 || k == 256) && (uint64_t)batch * n <= (1u << 20)) {
+    } else if (small) {
         if (out_planes) {   // the result also as the next layer's planes, written by the same workgroups
             a.out_planes = reinterpret_cast<uint4*>(out_planes);
             a.out_rows_padded = split_rows_padded(batch);

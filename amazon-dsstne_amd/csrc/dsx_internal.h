@@ -102,6 +102,11 @@ int topk_merge(const uint64_t* partial, uint32_t slots, uint32_t k, float* keys,
 int fc_run(const float* X, uint32_t ldx, const float* W, uint32_t ldw, int transposed, const float* bias, float* Z, uint32_t ldz,
            uint32_t batch, uint32_t k, uint32_t n, int accumulate, uint32_t activation, const dsx_act_params* params,
            float* seg_max = nullptr, uint32_t* seg_width = nullptr, void* out_planes = nullptr);
+// The same for few rows or few output tiles (dsx_fc_rows.hip): whether that kernel is the one for a shape, and the launch.
+bool fc_rows_takes(uint32_t batch, uint32_t k, uint32_t n, uint32_t ldx, uint32_t ldw, int transposed);
+int fc_rows_run(const float* X, uint32_t ldx, const float* W, uint32_t ldw, const float* bias, float* Z, uint32_t ldz, uint32_t batch,
+                uint32_t k, uint32_t n, int accumulate, uint32_t activation, const dsx_act_params* params, float* seg_max,
+                uint32_t* seg_width);
 // Candidate mode of the same kernel (exact KNN): scores are compared with the rows' bounds and the survivors appended to
 // per-row lists as packed words (CandArgs); nothing else is written.  knn_refresh folds a row's candidates into its best
 // list.  The caller guarantees 16-byte aligned operands with pitches that are multiples of four floats.
