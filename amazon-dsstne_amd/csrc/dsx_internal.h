@@ -97,6 +97,15 @@ int topk_run(const float* in, uint32_t pitch, uint32_t width, uint32_t batch, ui
 // Looks up this device's address of the fixed scratch array behind dsx_topk_filtered_static (called by dsx_init with the
 // device current).
 int topk_static_setup(int device);
+// The same for scores whose producer left the maxima of their 64-column segments (row pitch of seg_max: ceil(width / 64)); rows
+// are cut into topk_guided_parts(width, batch) parts, each with a list of its own in partial (or in the library's scratch).
+uint32_t topk_guided_parts(uint32_t width, uint32_t batch);
+int topk_guided_launch(const float* in, uint32_t pitch, uint32_t width, uint32_t batch, uint32_t k, float* keys, uint32_t* values,
+                       const float* seg_max, uint32_t position, const uint32_t* index, const uint64_t* fstart, const uint64_t* fend,
+                       const uint32_t* fidx, const float* fmul, uint32_t col_offset, uint64_t* partial, uint32_t partial_slots,
+                       uint32_t partial_slot0, uint32_t* row_bound);
+// Workgroups per row that topk_run takes on its own (forced_segments = 0).
+uint32_t topk_segments(uint32_t batch, uint32_t width, bool filtered);
 int topk_merge(const uint64_t* partial, uint32_t slots, uint32_t k, float* keys, uint32_t* values, uint32_t batch);
 // GEMM building block shared with the KNN search (dsx_fc.hip): Z = X.W (+bias, activation), see dsx_fc_forward.
 int fc_run(const float* X, uint32_t ldx, const float* W, uint32_t ldw, int transposed, const float* bias, float* Z, uint32_t ldz,

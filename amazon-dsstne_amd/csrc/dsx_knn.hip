@@ -45,7 +45,8 @@ constexpr uint32_t kCandCap = 4096;   // candidate words per query and column ra
 
 struct KnnWorkspace {
     float* block_scores;
-    uint64_t* partial;      // block path: [queries][blocks][k]; candidate path: [queries][k], the best lists
+    float* seg_max;         // [queries][block columns / 64], few queries only: maxima of the block's 64-column segments
+    uint64_t* partial;      // block path: [queries][lists of all blocks][k]; candidate path: [queries][k], the best lists
     uint32_t* row_bound;    // [queries] key of a score that k items seen so far reach; later columns admit nothing below it
     uint32_t* cand_count;   // [queries]
     uint32_t* overflow;     // [1] (+ padding)
@@ -56,6 +57,16 @@ struct KnnWorkspace {
     size_t bytes;
 };
 
+// A search of few queries is bound by reading the table once: its scores are stored (64 queries x 1,000,000 items: 256 MB against
+// 512 MB of table at 128 components) by the kernel for few rows, which leaves segment maxima for the top-K.
+static bool knn_few_queries(uint32_t num_queries) { return num_queries <= 64; }
+
+// Lists per query that the top-K of a block of ncols columns leaves: enough workgroups per query to fill the GPU.
+static uint32_t knn_block_lists(uint32_t num_queries, uint32_t ncols)
+{
+    return knn_few_queries(num_queries) ? topk_guided_parts(ncols, num_queries) : topk_segments(num_queries, ncols, false);
+}
+
 static KnnWorkspace knn_layout(void* base, uint32_t rows_padded, uint32_t num_queries, uint32_t k, bool f16 = false, uint32_t dim = 0,
                                bool split = false)
 {
@@ -65,8 +76,10 @@ static KnnWorkspace knn_layout(void* base, uint32_t rows_padded, uint32_t num_qu
     char* p = (char*)base;
     w.block_scores = (float*)p;
     p += align256((size_t)num_queries * cb * sizeof(float));
+    w.seg_max = knn_few_queries(num_queries) ? (float*)p : nullptr;
+    if (w.seg_max) p += align256((size_t)num_queries * ((cb + 63) / 64) * sizeof(float));
     w.partial = (uint64_t*)p;
-    p += align256((size_t)num_queries * blocks * k * sizeof(uint64_t));
+    p += align256((size_t)num_queries * blocks * knn_block_lists(num_queries, cb) * k * sizeof(uint64_t));
     w.row_bound = (uint32_t*)p;             // row_bound, cand_count and overflow are cleared together
     w.cand_count = w.row_bound + num_queries;
     w.overflow = w.cand_count + num_queries;
@@ -100,13 +113,14 @@ struct KnnOperands {
     const void* queries16 = nullptr;
     uint32_t rows_padded = 0, dim = 0, ld16 = 0;
 
-    int into_matrix(uint32_t c0, uint32_t ncols, uint32_t num_queries, float* Z, uint32_t ldz) const
+    int into_matrix(uint32_t c0, uint32_t ncols, uint32_t num_queries, float* Z, uint32_t ldz, float* seg_max = nullptr,
+                    uint32_t* seg_width = nullptr) const
     {
         if (f16) return knn_f16_scores_run(queries16, items16 + (uint64_t)c0 * ld16 * 2, ld16, num_queries, ncols, Z, ldz, nullptr);
         if (split)
             return fc_split_run(query_planes, item_planes, split_rows_padded(rows_padded), c0, nullptr, Z, ldz, num_queries, dim, ncols, 0,
                                 DSX_ACT_LINEAR, nullptr, nullptr, nullptr);
-        return fc_run(queries, dim, items + c0, rows_padded, 0, nullptr, Z, ldz, num_queries, dim, ncols, 0, DSX_ACT_LINEAR, nullptr);
+        return fc_run(queries, dim, items + c0, rows_padded, 0, nullptr, Z, ldz, num_queries, dim, ncols, 0, DSX_ACT_LINEAR, nullptr, seg_max, seg_width);
     }
     // *chunks_used: how many (row, chunk) lists of seg the range filled besides the shared lists (0: none)
     int into_candidates(uint32_t c0, uint32_t ncols, uint32_t num_queries, const CandArgs& cand, uint64_t* seg, uint32_t* seg_count,
@@ -144,22 +158,29 @@ static int knn_search_blocks(const KnnWorkspace& w, const KnnOperands& op, uint3
     hipStream_t s = ctx().stream;
     const uint32_t cb = knn_block_columns(op.rows_padded, num_queries);
     const uint32_t blocks = (M + cb - 1) / cb;
+    const uint32_t lists_per_block = knn_block_lists(num_queries, cb);
+    const uint32_t lists = (blocks - 1) * lists_per_block + knn_block_lists(num_queries, M - (blocks - 1) * cb);
     hipLaunchKernelGGL(knn_clear_kernel, dim3((num_queries + 255) / 256), dim3(256), 0, s, w.row_bound, num_queries);
     for (uint32_t blk = 0; blk < blocks; blk++) {
         const uint32_t c0 = blk * cb;
         const uint32_t ncols = std::min(cb, M - c0);
         t.start(s);
-        int rc = op.into_matrix(c0, ncols, num_queries, w.block_scores, cb);
+        uint32_t seg_width = 0;
+        int rc = op.into_matrix(c0, ncols, num_queries, w.block_scores, cb, w.seg_max, w.seg_max ? &seg_width : nullptr);
         if (rc) return rc;
         t.stop(s, t.gemm);
         t.start(s);
-        rc = topk_run(w.block_scores, cb, ncols, num_queries, k, nullptr, nullptr, 0, nullptr, nullptr, nullptr, nullptr, nullptr, c0,
-                      w.partial, blocks, blk, 1, w.row_bound);
+        if (seg_width != 0)
+            rc = topk_guided_launch(w.block_scores, cb, ncols, num_queries, k, nullptr, nullptr, w.seg_max, 0, nullptr, nullptr, nullptr, nullptr,
+                                    nullptr, c0, w.partial, lists, blk * lists_per_block, w.row_bound);
+        else
+            rc = topk_run(w.block_scores, cb, ncols, num_queries, k, nullptr, nullptr, 0, nullptr, nullptr, nullptr, nullptr, nullptr, c0,
+                          w.partial, lists, blk * lists_per_block, knn_block_lists(num_queries, ncols), w.row_bound);
         if (rc) return rc;
         t.stop(s, t.topk);
     }
     t.start(s);
-    int rc = topk_merge(w.partial, blocks, k, scores, indexes, num_queries);
+    int rc = topk_merge(w.partial, lists, k, scores, indexes, num_queries);
     t.stop(s, t.topk);
     return rc;
 }
@@ -301,7 +322,9 @@ static int knn_search_common(KnnOperands& op, uint32_t padding, uint32_t num_que
     }
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
     hipStreamIsCapturing(s, &capturing);
-    const bool candidates = aligned && capturing == hipStreamCaptureStatusNone && M > knn_block_columns(op.rows_padded, num_queries);
+    // (few queries against an fp32 table stay with the blocks, however many there are; a width set by the caller is kept)
+    const bool few = knn_few_queries(num_queries) && !op.f16 && !op.split && !ctx().knobs.knn_block_columns;
+    const bool candidates = aligned && !few && capturing == hipStreamCaptureStatusNone && M > knn_block_columns(op.rows_padded, num_queries);
     bool redo = !candidates;
     if (rc == DSX_OK && candidates) rc = knn_search_candidates(w, op, M, num_queries, k, scores, indexes, t, &redo);
     g_knn_last_path = !candidates ? DSX_KNN_PATH_BLOCKS : (redo ? DSX_KNN_PATH_CANDIDATES_REDONE : DSX_KNN_PATH_CANDIDATES);

@@ -141,7 +141,11 @@ template <int R> __device__ __forceinline__ void bitonic_merge_desc(uint64_t (&v
 template <int R> struct WaveTopK {
     static constexpr int L = kWave * R;
     static constexpr int kBurst = 5 * kWave;            // most words staged between two checks of the fill level
-    static constexpr int kStageWords = L + kBurst;
+    // Words that may wait before they are merged into the list.  A workgroup none of whose wavefronts ever merged finishes by
+    // counting instead of sorting (finish_row), so for the shorter lists there is room for twice their length.
+    static constexpr int kDrainAt = (R <= 2) ? 2 * L : L;
+    static constexpr int kStageWords = kDrainAt + kBurst;
+    static constexpr int kCountWords = (R == 1) ? 256 : 512;   // most words of a workgroup that finish_row counts
 
     uint64_t q[R];        // sorted descending over position r*64 + lane; 0 = empty slot
     uint64_t thr;         // current k-th word: candidates must be strictly larger
@@ -254,7 +258,7 @@ template <int R> struct WaveTopK {
     }
 
     // Stage the lanes' words that beat the threshold.  All 64 lanes must call this together.  Nothing is merged here: after
-    // at most five calls the caller runs drain(), which keeps count < L between bursts.
+    // at most five calls the caller runs drain(), which keeps count < kDrainAt between bursts.
     __device__ __forceinline__ void stage_only(bool valid, uint64_t word)
     {
         const bool cand = valid && (word > thr);
@@ -267,10 +271,10 @@ template <int R> struct WaveTopK {
 
     __device__ __forceinline__ void drain()
     {
-        while (count >= (uint32_t)L) flush();
+        while (count >= (uint32_t)kDrainAt) flush();
     }
 
-    // Offer one word per lane (valid lanes only) and merge when L are waiting.
+    // Offer one word per lane (valid lanes only) and merge when kDrainAt are waiting.
     __device__ __forceinline__ void offer(bool valid, uint64_t word)
     {
         stage_only(valid, word);
@@ -308,6 +312,7 @@ struct TopKArgs {
     // guided variant: maxima of the row's 64-column segments, left by the producer of `in`
     const float* seg_max;       // [batch][nseg]
     uint32_t nseg;
+    uint32_t part_segs;         // segments per workgroup (nseg: one workgroup per row)
 };
 
 template <int R>
@@ -338,9 +343,10 @@ __device__ __forceinline__ void finish_row(WaveTopK<R>& list, uint64_t (*sStage)
 {
     // Merge the four waves into wave 0.  A wave that never had to flush hands over its staged words as they are (they
     // already sit in LDS); a wave with a register list flushes what is left and publishes its first k words.
+    constexpr int kCount = WaveTopK<R>::kCountWords, M = kCount / kWave;
     __shared__ uint32_t sPublished[kTopkWaves];
     __shared__ uint32_t sFlushed[kTopkWaves];
-    __shared__ uint32_t sPlace[2 * kWave];
+    __shared__ uint32_t sPlace[kCount];
     if (wave != 0 && list.flushed) {
         list.finish();
 #pragma unroll
@@ -353,10 +359,7 @@ __device__ __forceinline__ void finish_row(WaveTopK<R>& list, uint64_t (*sStage)
         sPublished[wave] = (wave != 0 && list.flushed) ? a.k : list.count;
         sFlushed[wave] = list.flushed ? 1u : 0u;
     }
-    if (wave == 1) {
-        sPlace[lane] = 0;
-        sPlace[kWave + lane] = 0;
-    }
+    for (uint32_t i = wave * kWave + lane; i < (uint32_t)kCount; i += kTopkThreads) sPlace[i] = 0;
     __syncthreads();
 
     uint64_t* partial = a.partial ? a.partial + ((uint64_t)b * a.partial_slots + a.partial_slot0 + seg) * a.k : nullptr;
@@ -381,43 +384,56 @@ __device__ __forceinline__ void finish_row(WaveTopK<R>& list, uint64_t (*sStage)
     const uint32_t n0 = sPublished[0], n1 = sPublished[1], n2 = sPublished[2], n3 = sPublished[3];
     const uint32_t total = n0 + n1 + n2 + n3;
     const bool any_flushed = (sFlushed[0] | sFlushed[1] | sFlushed[2] | sFlushed[3]) != 0;   // the same for every wave
-    if (!any_flushed && total <= 2 * kWave) {
-        // Common case for small k: at most 128 staged words in all.  Lane i takes the i-th (and the 64 + i-th) of them; the
-        // number of staged words that are larger is its place in the result, so no sorting network runs at all.  The
-        // counting is shared: every wave compares all words with its own staged ones and adds its count in LDS.
+    if (!any_flushed && total <= (uint32_t)kCount) {
+        // Common case: a few words more than k in all, none of them merged yet.  The number of staged words that are larger is a
+        // word's place in the result, so no sorting network runs at all.  Every lane holds the i-th, (64 + i)-th, ... of the words,
+        // every wave compares them with its own staged ones and adds its counts in LDS.  (256 words of a k = 128 row: about 750
+        // instructions per wave, spread over four waves, against a chain of six sorts and merges in one of them.)
         auto fetch = [&](uint32_t i) -> uint64_t {
             if (i >= total) return 0ull;   // never larger than anything
             const uint32_t w = (i >= n0) + (i >= n0 + n1) + (i >= n0 + n1 + n2);
             const uint32_t first = (w == 0) ? 0 : (w == 1) ? n0 : (w == 2) ? n0 + n1 : n0 + n1 + n2;
             return sStage[w][i - first];
         };
-        const bool two = total > kWave;   // workgroup-uniform
-        const uint64_t word0 = fetch(lane), word1 = two ? fetch(kWave + lane) : 0ull;
         const uint32_t mine = sPublished[wave];
-        uint32_t part0 = 0, part1 = 0;
-        for (uint32_t i = 0; i < mine; i += 4) {   // broadcast reads, four in flight (a staging row has room beyond any count)
-            uint64_t o[4];
+        auto count = [&](auto lanes_words) __attribute__((always_inline)) {
+            constexpr int N = decltype(lanes_words)::value;   // words per lane
+            uint64_t word[N];
+            uint32_t part[N];
 #pragma unroll
-            for (int u = 0; u < 4; u++) o[u] = sStage[wave][i + u];
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                if (i + u >= mine) o[u] = 0ull;   // stale words beyond the count
-                part0 += (o[u] > word0) ? 1u : 0u;
-                if (two) part1 += (o[u] > word1) ? 1u : 0u;
+            for (int m = 0; m < N; m++) {
+                word[m] = fetch(m * kWave + lane);
+                part[m] = 0;
             }
-        }
-        if (part0 != 0) atomicAdd(&sPlace[lane], part0);
-        if (part1 != 0) atomicAdd(&sPlace[kWave + lane], part1);
+            for (uint32_t i = 0; i < mine; i += 4) {   // broadcast reads, four in flight (a staging row has room beyond any count)
+                uint64_t o[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) o[u] = sStage[wave][i + u];
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    if (i + u >= mine) o[u] = 0ull;   // stale words beyond the count
+#pragma unroll
+                    for (int m = 0; m < N; m++) part[m] += (o[u] > word[m]) ? 1u : 0u;
+                }
+            }
+#pragma unroll
+            for (int m = 0; m < N; m++)
+                if (part[m] != 0) atomicAdd(&sPlace[m * kWave + lane], part[m]);
+        };
+        if (total <= kWave) count(std::integral_constant<int, 1>());   // the same for the whole workgroup
+        else if (total <= 2 * kWave) count(std::integral_constant<int, 2>());
+        else if (M <= 4 || total <= 4 * kWave) count(std::integral_constant<int, 4>());
+        else count(std::integral_constant<int, M>());
         __syncthreads();
-        if (wave != 0) return;
-        const uint32_t place0 = sPlace[lane], place1 = sPlace[kWave + lane];
-        if (word0 != 0 && place0 < a.k) write_slot(place0, word0);
-        if (word1 != 0 && place1 < a.k) write_slot(place1, word1);
-        for (uint32_t p = total + lane; p < a.k; p += kWave) write_slot(p, 0ull);
-        if (a.row_bound) {   // this block's k-th score bounds the row's final k-th from below
-            if (word0 != 0 && place0 == a.k - 1) atomicMax(&a.row_bound[b], (uint32_t)(word0 >> 32));
-            if (word1 != 0 && place1 == a.k - 1) atomicMax(&a.row_bound[b], (uint32_t)(word1 >> 32));
+        for (uint32_t i = wave * kWave + lane; i < total; i += kTopkThreads) {
+            const uint64_t word = fetch(i);
+            const uint32_t place = sPlace[i];
+            if (word == 0 || place >= a.k) continue;
+            write_slot(place, word);
+            // this block's k-th score bounds the row's final k-th from below
+            if (a.row_bound && place == a.k - 1) atomicMax(&a.row_bound[b], (uint32_t)(word >> 32));
         }
+        for (uint32_t p = total + wave * kWave + lane; p < a.k; p += kTopkThreads) write_slot(p, 0ull);
         return;
     }
     if (wave != 0) return;
@@ -759,7 +775,7 @@ __global__ __launch_bounds__(kTopkThreads, (R <= 2) ? 4 : 2) void topk_scan_kern
     finish_row<R>(list, sStage, a, b, seg, wave, lane);
 }
 
-// Guided top-K (k <= 64): the producer of the scores also left the maximum of every 64-column segment of every row (the
+// Guided top-K: the producer of the scores also left the maximum of every 64-column segment of every row (the
 // dense layer's epilogue has them in registers anyway).  The k-th largest of a row's segment maxima is a score that at least
 // k items reach, so only segments whose maximum reaches it can hold a result: about k of them.  The kernel reads the
 // row's maxima (1/64 of the row), picks that bound with the same key-bit search the scan uses for priming, and then reads
@@ -767,32 +783,38 @@ __global__ __launch_bounds__(kTopkThreads, (R <= 2) ? 4 : 2) void topk_scan_kern
 // ones: it is left out of the bound (its segment is still read).  Rows full of ties read more segments and still come out
 // right: the survivors go through the same lists as in the scan.
 constexpr uint32_t kGuidedSegWidth = 64;
-constexpr uint32_t kGuidedMaxSegs = 2048;
-constexpr uint32_t kGuidedMaxK = 64;
+constexpr uint32_t kGuidedMaxSegs = 2048;   // per workgroup
 
-// E: segment maxima per lane (256 * E >= number of segments); the key search costs in proportion.
-template <bool FILTERED, int E>
-__global__ __launch_bounds__(kTopkThreads, 4) void topk_guided_kernel(TopKArgs a)
+// E: segment maxima per lane (256 * E >= number of segments); the key search costs in proportion.  R: length of the lists / 64.
+// Wide rows are cut into parts of a.part_segs segments, a workgroup each (blockIdx.y); the parts' lists are merged afterwards.
+template <int R, bool FILTERED, int E>
+__global__ __launch_bounds__(kTopkThreads, R <= 2 ? 4 : 2) void topk_guided_kernel(TopKArgs a)
 {
     __builtin_amdgcn_s_setprio(3);   // short kernels issue ahead of a GEMM's wavefronts that share their SIMD
-    using List = WaveTopK<1>;
+    using List = WaveTopK<R>;
     static_assert(E * kTopkThreads <= kGuidedMaxSegs, "at most kGuidedMaxSegs segments");
     __shared__ uint64_t sStage[kTopkWaves][List::kStageWords];
-    __shared__ uint32_t sPrime[kTopkWaves][kGuidedMaxK];
+    __shared__ uint32_t sPrime[kTopkWaves][R * kWave];
     __shared__ uint32_t sListCount, sBound;
     __shared__ uint32_t sChunk[8 * kTopkWaves];   // listed segments per group of 64 maxima
     extern __shared__ uint32_t sDyn[];   // segments to read [nseg] | their maxima [nseg] | best listed score per segment [nseg] | bitmap of listed columns
-    uint32_t* sList = sDyn;
-    uint32_t* sListKey = sDyn + a.nseg;
-    uint32_t* sFiltMax = sDyn + 2 * a.nseg;
-    uint32_t* sBitmap = sDyn + 3 * a.nseg;
-
     const uint32_t b = blockIdx.x;
+    const uint32_t seg0 = blockIdx.y * a.part_segs, nseg = min(a.nseg - seg0, a.part_segs);   // this part's segments
+    const uint32_t lo = seg0 * kGuidedSegWidth, hi = min(a.width, lo + nseg * kGuidedSegWidth);
+    uint32_t* sList = sDyn;
+    uint32_t* sListKey = sDyn + nseg;
+    uint32_t* sFiltMax = sDyn + 2 * nseg;
+    uint32_t* sBitmap = sDyn + 3 * nseg;
+
     const uint32_t wave = threadIdx.x / kWave;
     const uint32_t lane = threadIdx.x % kWave;
     const float* row = a.in + (uint64_t)b * a.pitch;
     List list;
     list.init(sStage[wave], lane, a.k);
+    if (a.row_bound) {
+        const uint32_t t = a.row_bound[b];   // k columns of earlier blocks of this row reach this score
+        if (t > score_key(-__builtin_inff())) list.prime(t);
+    }
 
     uint64_t fs = 0, fe = 0;
     if constexpr (FILTERED) {
@@ -803,14 +825,16 @@ __global__ __launch_bounds__(kTopkThreads, 4) void topk_guided_kernel(TopKArgs a
     }
     uint32_t mk[E];   // keys of this lane's segment maxima; 0 = no such segment
     {
-        const float* mrow = a.seg_max + (uint64_t)b * a.nseg;
+        const float* mrow = a.seg_max + (uint64_t)b * a.nseg + seg0;
 #pragma unroll
         for (int e = 0; e < E; e++) {
             const uint32_t idx = e * kTopkThreads + threadIdx.x;
-            mk[e] = (idx < a.nseg) ? score_key(mrow[idx]) : 0u;
+            mk[e] = (idx < nseg) ? score_key(mrow[idx]) : 0u;
         }
     }
-    sPrime[wave][lane] = 0;
+    
+#pragma unroll
+    for (int r = 0; r < R; r++) sPrime[wave][r * kWave + lane] = 0;
     if (threadIdx.x == 0) sListCount = 0;
 
     constexpr int kFU = 4;
@@ -822,7 +846,7 @@ __global__ __launch_bounds__(kTopkThreads, 4) void topk_guided_kernel(TopKArgs a
     // and rows with multipliers, read the listed scores first and leave out only the segments whose maximum is one of them.
     bool light = false;   // the same for the whole workgroup
     if constexpr (FILTERED) {
-        light = !a.fmul && (fe - fs) * 2 <= a.nseg;
+        light = !a.fmul && (fe - fs) * 2 <= nseg;
         // (the listed columns are requested before the barrier below, which waits for everything in flight: the row's range,
         // the maxima and the first listed columns then cost two round trips, not three)
 #pragma unroll
@@ -835,35 +859,35 @@ __global__ __launch_bounds__(kTopkThreads, 4) void topk_guided_kernel(TopKArgs a
                 if (a.fmul) fm[u] = a.fmul[t];
             }
         }
-        const uint32_t words = (a.width + 31) / 32;
+        const uint32_t words = (hi - lo + 31) / 32;
         for (uint32_t i = threadIdx.x; i < words; i += kTopkThreads) sBitmap[i] = 0;
-        for (uint32_t i = threadIdx.x; i < a.nseg; i += kTopkThreads) sFiltMax[i] = 0;
+        for (uint32_t i = threadIdx.x; i < nseg; i += kTopkThreads) sFiltMax[i] = 0;
         __syncthreads();
         auto mark = [&](uint32_t c, float v) {
-            atomicOr(&sBitmap[c >> 5], 1u << (c & 31));
-            if (v == v) atomicMax(&sFiltMax[c / kGuidedSegWidth], score_key(v));   // a NaN is never a segment's maximum
+            atomicOr(&sBitmap[(c - lo) >> 5], 1u << ((c - lo) & 31));
+            if (v == v) atomicMax(&sFiltMax[(c - lo) / kGuidedSegWidth], score_key(v));   // a NaN is never a segment's maximum
         };
         if (light) {   // (at most nseg / 2 <= 1024 listed columns: they are all in fcol)
 #pragma unroll
             for (int u = 0; u < kFU; u++) {
                 fv[u] = 0.0f;
-                if (fcol[u] < a.width) {
-                    atomicOr(&sBitmap[fcol[u] >> 5], 1u << (fcol[u] & 31));
-                    sFiltMax[fcol[u] / kGuidedSegWidth] = 0xffffffffu;   // equal to no key of a maximum that takes part (NaN patterns aside, which are 0 here)
+                if (fcol[u] >= lo && fcol[u] < hi) {
+                    atomicOr(&sBitmap[(fcol[u] - lo) >> 5], 1u << ((fcol[u] - lo) & 31));
+                    sFiltMax[(fcol[u] - lo) / kGuidedSegWidth] = 0xffffffffu;   // equal to no key of a maximum that takes part (NaN patterns aside, which are 0 here)
                 }
             }
         } else {
 #pragma unroll
             for (int u = 0; u < kFU; u++) {
                 fv[u] = 0.0f;
-                if (fcol[u] < a.width) fv[u] = row[fcol[u]];
+                if (fcol[u] >= lo && fcol[u] < hi) fv[u] = row[fcol[u]];
             }
 #pragma unroll
             for (int u = 0; u < kFU; u++)
-                if (fcol[u] < a.width) mark(fcol[u], fv[u]);
+                if (fcol[u] >= lo && fcol[u] < hi) mark(fcol[u], fv[u]);
             for (uint64_t t = fs + (uint64_t)kFU * kTopkThreads + threadIdx.x; t < fe; t += kTopkThreads) {
                 const uint32_t c = a.fidx[t];
-                if (c < a.width) mark(c, row[c]);
+                if (c >= lo && c < hi) mark(c, row[c]);
             }
         }
     }
@@ -871,7 +895,7 @@ __global__ __launch_bounds__(kTopkThreads, 4) void topk_guided_kernel(TopKArgs a
 
     auto filtered_out = [&](uint32_t col) -> bool {
         if constexpr (FILTERED) {
-            return (sBitmap[col >> 5] >> (col & 31)) & 1u;
+            return (sBitmap[(col - lo) >> 5] >> ((col - lo) & 31)) & 1u;
         } else {
             return false;
         }
@@ -887,7 +911,7 @@ __global__ __launch_bounds__(kTopkThreads, 4) void topk_guided_kernel(TopKArgs a
             tk[e] = mk[e];
             if constexpr (FILTERED) {
                 const uint32_t idx = e * kTopkThreads + threadIdx.x;
-                if (idx < a.nseg && (light ? sFiltMax[idx] != 0 : sFiltMax[idx] == mk[e])) tk[e] = 0;
+                if (idx < nseg && (light ? sFiltMax[idx] != 0 : sFiltMax[idx] == mk[e])) tk[e] = 0;
             }
         }
         if (a.k <= 16) {   // the same for the whole workgroup
@@ -898,12 +922,12 @@ __global__ __launch_bounds__(kTopkThreads, 4) void topk_guided_kernel(TopKArgs a
 #pragma unroll
             for (int e = 0; e < E; e++) {
                 const uint32_t idx = e * kTopkThreads + threadIdx.x;
-                if (idx < a.nseg) sListKey[idx] = tk[e];   // (the list of segments is built later)
+                if (idx < nseg) sListKey[idx] = tk[e];   // (the list of segments is built later)
             }
             __syncthreads();
             if (wave == 0) {
                 uint32_t best[1] = {0u};
-                for (uint32_t i = lane; i < a.nseg; i += kWave) best[0] = max(best[0], sListKey[i]);
+                for (uint32_t i = lane; i < nseg; i += kWave) best[0] = max(best[0], sListKey[i]);
                 const uint32_t t = wave_kth_key<1>(best, a.k);
                 if (lane == 0) sBound = t;
             }
@@ -922,15 +946,15 @@ __global__ __launch_bounds__(kTopkThreads, 4) void topk_guided_kernel(TopKArgs a
             // (one wavefront searches, the others wait: four workgroups share a CU, and what the searches of sixteen wavefronts
             // cost is instruction issue, not latency)
             if (wave == 0) {
-                uint32_t all[4];
+                uint32_t all[4 * R];
 #pragma unroll
-                for (int n = 0; n < 4; n++) {
+                for (int n = 0; n < 4 * R; n++) {
                     const uint32_t i = n * kWave + lane;
                     all[n] = (i < kTopkWaves * a.k) ? sPrime[i / a.k][i % a.k] : 0u;
                 }
                 uint32_t t;
-                if (a.k <= 32) t = wave_kth_key<2>(reinterpret_cast<const uint32_t(&)[2]>(all), a.k);
-                else t = wave_kth_key<4>(all, a.k);
+                if (R == 1 && a.k <= 32) t = wave_kth_key<2>(reinterpret_cast<const uint32_t(&)[2]>(all), a.k);
+                else t = wave_kth_key<4 * R>(all, a.k);
                 if (lane == 0) sBound = t;
             }
         }
@@ -947,7 +971,7 @@ __global__ __launch_bounds__(kTopkThreads, 4) void topk_guided_kernel(TopKArgs a
 #pragma unroll
     for (int e = 0; e < E; e++) {
         const uint32_t idx = e * kTopkThreads + threadIdx.x;
-        const bool flagged = idx < a.nseg && mk[e] >= bound;
+        const bool flagged = idx < nseg && mk[e] >= bound;
         const uint64_t m = __ballot(flagged);
         listed[e] = m;
         if (m == 0) continue;
@@ -963,10 +987,10 @@ __global__ __launch_bounds__(kTopkThreads, 4) void topk_guided_kernel(TopKArgs a
     __syncthreads();
     const uint32_t count = sListCount;
     constexpr int kSegsInFlight = 8;
-    // More segments than one round of reads takes (rows of tied scores, mostly): the list is written again in ascending
+    // More segments than one round of reads takes, and many more than k (rows of tied scores, mostly): the list is written again in ascending
     // order, so that the first round reads the lowest columns and what only ties behind them can be left out.  Lane j holds
     // the count of the j-th group of 64 maxima; a scan over the first lanes gives every group its place.
-    const bool heavy = bound != 0 && count > kTopkWaves * kSegsInFlight;   // the same for the whole workgroup
+    const bool heavy = bound != 0 && count > max((uint32_t)(kTopkWaves * kSegsInFlight), 2 * a.k);   // the same for the whole workgroup
     if (heavy) {
         if (lane == 0) {
 #pragma unroll
@@ -1008,10 +1032,10 @@ __global__ __launch_bounds__(kTopkThreads, 4) void topk_guided_kernel(TopKArgs a
             col[u] = 0;
             const uint32_t i = i0 + u * kTopkWaves;
             if (i < count) {
-                const uint32_t first = sList[i] * kGuidedSegWidth;
+                const uint32_t first = lo + sList[i] * kGuidedSegWidth;
                 if (key_score(sListKey[i]) >= list.admission_score(first)) {   // wave-uniform
                     col[u] = first + lane;
-                    if (col[u] < a.width) v[u] = row[col[u]];
+                    if (col[u] < hi) v[u] = row[col[u]];
                 }
             }
         }
@@ -1095,16 +1119,16 @@ __global__ __launch_bounds__(kTopkThreads, 4) void topk_guided_kernel(TopKArgs a
 #pragma unroll
                 for (int u = 0; u < kFU; u++) {
                     fv[u] = 0.0f;
-                    if (fcol[u] < a.width) fv[u] = row[fcol[u]];
+                    if (fcol[u] >= lo && fcol[u] < hi) fv[u] = row[fcol[u]];
                 }
             }
 #pragma unroll
             for (int u = 0; u < kFU; u++) {
                 if (base + (uint64_t)u * kTopkThreads + wave * kWave >= fe) break;   // wave-uniform
                 bool own = false;
-                if (fcol[u] < a.width) {
-                    const uint32_t bit = 1u << (fcol[u] & 31);
-                    own = (atomicAnd(&sBitmap[fcol[u] >> 5], ~bit) & bit) != 0;
+                if (fcol[u] >= lo && fcol[u] < hi) {
+                    const uint32_t bit = 1u << ((fcol[u] - lo) & 31);
+                    own = (atomicAnd(&sBitmap[(fcol[u] - lo) >> 5], ~bit) & bit) != 0;
                 }
                 const float v = fm[u] * fv[u];   // utils/Filters.cpp:62
                 list.stage_only(own && v == v, pack_score(v, fcol[u]));
@@ -1112,31 +1136,67 @@ __global__ __launch_bounds__(kTopkThreads, 4) void topk_guided_kernel(TopKArgs a
             list.drain();
         }
     }
-    finish_row<1>(list, sStage, a, b, 0, wave, lane);
+    finish_row<R>(list, sStage, a, b, blockIdx.y, wave, lane);
 }
 
-// Second stage: one wavefront per row merges `slots` packed partial lists of k words each.
+// Second stage: one workgroup per row merges `slots` packed partial lists of k words each (every list best first).  A bound
+// comes first: if q lists have a d-th word of at least t, then q * d words of the row reach t, so the ceil(k / d)-th largest of
+// the lists' d-th words bounds the k-th word; with d about 2 k / slots that rank is in the middle of the lists, and what
+// passes is little more than k words, which finish_row puts in order by counting.  (61 lists of 50 words, one row: 27 -> 6 us
+// against one wavefront that sorts and merges 64 words at a time.)
 template <int R>
-__global__ __launch_bounds__(kWave) void topk_merge_kernel(const uint64_t* partial, uint32_t slots, uint32_t k, float* keys,
-                                                           uint32_t* values)
+__global__ __launch_bounds__(kTopkThreads) void topk_merge_kernel(const uint64_t* partial, uint32_t slots, uint32_t k, float* keys,
+                                                                  uint32_t* values)
 {
     __builtin_amdgcn_s_setprio(3);   // short kernels issue ahead of a GEMM's wavefronts that share their SIMD
     using List = WaveTopK<R>;
-    __shared__ uint64_t sStage[List::kStageWords];
+    __shared__ uint64_t sStage[kTopkWaves][List::kStageWords];
     const uint32_t b = blockIdx.x;
-    const uint32_t lane = threadIdx.x;
-    List list;
-    list.init(sStage, lane, k);
+    const uint32_t wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
     const uint64_t* src = partial + (uint64_t)b * slots * k;
-    const uint32_t total = slots * k;
-    for (uint32_t p0 = 0; p0 < total; p0 += kWave) {
-        const uint32_t p = p0 + lane;
-        uint64_t word = 0;
-        if (p < total) word = src[p];
-        list.offer(word != 0, word);
+    TopKArgs a{};
+    a.k = k;
+    a.keys = keys;
+    a.values = values;
+    if (slots == 1) {   // already in order
+        for (uint32_t p = threadIdx.x; p < k; p += kTopkThreads) {
+            float key = -kMaxValue;
+            uint32_t col = 0;
+            if (src[p] != 0) unpack_score(src[p], key, col);
+            keys[(uint64_t)b * k + p] = key;
+            values[(uint64_t)b * k + p] = col;
+        }
+        return;
     }
-    list.finish();
-    write_final<R>(list.q, lane, k, 0, keys + (uint64_t)b * k, values + (uint64_t)b * k);
+    List list;
+    list.init(sStage[wave], lane, k);
+    const uint32_t total = slots * k;
+    constexpr int U = 4;
+    uint64_t word[U], next[U];
+    auto load = [&](uint64_t (&w)[U], uint32_t p0) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const uint32_t p = p0 + u * kTopkThreads + threadIdx.x;
+            w[u] = (p < total) ? src[p] : 0ull;
+        }
+    };
+    load(word, 0);
+    {
+        const uint32_t d = min(k, max((2 * k + slots - 1) / slots, (k + 31) / 32));   // (64 lanes: a rank of 32 at most)
+        uint32_t best[1] = {0u};   // a lane's best d-th word (its lists are every 64th)
+        for (uint32_t s = lane; s < slots; s += kWave) best[0] = max(best[0], (uint32_t)(src[(uint64_t)s * k + d - 1] >> 32));
+        const uint32_t t = wave_kth_key<1>(best, (k + d - 1) / d);
+        if (t > score_key(-__builtin_inff())) list.prime(t);
+    }
+    for (uint32_t p0 = 0; p0 < total; p0 += U * kTopkThreads) {
+        if (p0 + U * kTopkThreads < total) load(next, p0 + U * kTopkThreads);
+#pragma unroll
+        for (int u = 0; u < U; u++) list.stage_only(word[u] != 0, word[u]);
+        list.drain();
+#pragma unroll
+        for (int u = 0; u < U; u++) word[u] = next[u];
+    }
+    finish_row<R>(list, sStage, a, b, 0, wave, lane);
 }
 
 // In-place payload gather for the key/value overloads: values[b][j] holds a column number on entry.
@@ -1173,13 +1233,13 @@ template <int R> static int launch_scan(const TopKArgs& a, uint32_t batch, bool 
 
 template <int R> static int launch_merge(const uint64_t* partial, uint32_t slots, uint32_t k, float* keys, uint32_t* values, uint32_t batch)
 {
-    hipLaunchKernelGGL((topk_merge_kernel<R>), dim3(batch), dim3(kWave), 0, ctx().stream, partial, slots, k, keys, values);
+    hipLaunchKernelGGL((topk_merge_kernel<R>), dim3(batch), dim3(kTopkThreads), 0, ctx().stream, partial, slots, k, keys, values);
     DSX_LAUNCH_CHECK("topk_merge_kernel");
     return DSX_OK;
 }
 
 // Number of workgroups per row: enough to fill the device, and small enough segments for the LDS bitmap.
-static uint32_t choose_segments(uint32_t batch, uint32_t width, bool filtered)
+uint32_t topk_segments(uint32_t batch, uint32_t width, bool filtered)
 {
     uint32_t s = 1;
     const uint32_t target_blocks = (uint32_t)ctx().num_cus * 4;
@@ -1216,7 +1276,7 @@ int topk_run(const float* in, uint32_t pitch, uint32_t width, uint32_t batch, ui
     a.keys = keys;
     a.values = values;
     a.row_bound = row_bound;
-    a.segments = forced_segments ? forced_segments : choose_segments(batch, width, filtered);
+    a.segments = forced_segments ? forced_segments : topk_segments(batch, width, filtered);
     if (fixed_scratch && !partial && a.segments > 1 && (size_t)batch * a.segments * k > fixed_scratch_words)
         return set_error(DSX_EINVAL, "top-K: %u rows x %u segments x k = %u need %zu bytes of partial lists, the fixed scratch holds %zu",
                          batch, a.segments, k, (size_t)batch * a.segments * k * sizeof(uint64_t), fixed_scratch_words * sizeof(uint64_t));
@@ -1582,23 +1642,45 @@ int layer_refresh_run(const LayerRefresh& r, uint32_t batch)
     return DSX_OK;
 }
 
-// Guided top-K when it applies (k <= 64, 64-column segments, at most kGuidedMaxSegs of them), the scan otherwise.
-int topk_guided_run(const float* in, uint32_t width, uint32_t batch, uint32_t k, float* keys, uint32_t* values, const float* seg_max,
-                    uint32_t seg_width, uint32_t position, const uint32_t* index, const uint64_t* fstart, const uint64_t* fend,
-                    const uint32_t* fidx, const float* fmul)
+// Segments per workgroup of the guided top-K: up to 2,048, and no more than 1,024 where the rows alone leave the GPU idle.
+static uint32_t guided_part_segs(uint32_t nseg, uint32_t batch)
 {
-    const bool filtered = fidx != nullptr;
-    const uint32_t nseg = (width + kGuidedSegWidth - 1) / kGuidedSegWidth;
-    size_t lds = (size_t)nseg * 8;
-    if (filtered) lds += (size_t)nseg * 4 + ((size_t)(width + 31) / 32) * 4;
-    if (!seg_max || seg_width != kGuidedSegWidth || k > kGuidedMaxK || nseg > kGuidedMaxSegs || lds > 40 * 1024)
-        return topk_run(in, width, width, batch, k, keys, values, position, index, fstart, fend, fidx, fmul, 0, nullptr, 0, 0, 0);
+    const uint32_t most = (batch < (uint32_t)ctx().num_cus) ? kGuidedMaxSegs / 2 : kGuidedMaxSegs;
+    const uint32_t parts = (nseg + most - 1) / most;
+    return (nseg + parts - 1) / parts;
+}
+
+uint32_t topk_guided_parts(uint32_t width, uint32_t batch)
+{
+    const uint32_t nseg = (width + kGuidedSegWidth - 1) / kGuidedSegWidth, per = guided_part_segs(nseg, batch);
+    return (nseg + per - 1) / per;
+}
+
+template <int R, bool FILTERED> static void launch_guided(const TopKArgs& a, uint32_t batch, uint32_t parts)
+{
+    size_t lds = (size_t)a.part_segs * 8;
+    if (FILTERED) lds += (size_t)a.part_segs * (4 + kGuidedSegWidth / 8);
+    const dim3 grid(batch, parts), block(kTopkThreads);
+    hipStream_t s = ctx().stream;
+    if (a.part_segs <= 2 * kTopkThreads) hipLaunchKernelGGL((topk_guided_kernel<R, FILTERED, 2>), grid, block, lds, s, a);
+    else if (a.part_segs <= 4 * kTopkThreads) hipLaunchKernelGGL((topk_guided_kernel<R, FILTERED, 4>), grid, block, lds, s, a);
+    else hipLaunchKernelGGL((topk_guided_kernel<R, FILTERED, 8>), grid, block, lds, s, a);
+}
+
+// Guided top-K over in[batch][pitch] with the maxima of its 64-column segments; with partial != NULL the parts' packed lists go to
+// partial[b][partial_slot0 + part] (as topk_run).
+int topk_guided_launch(const float* in, uint32_t pitch, uint32_t width, uint32_t batch, uint32_t k, float* keys, uint32_t* values,
+                       const float* seg_max, uint32_t position, const uint32_t* index, const uint64_t* fstart, const uint64_t* fend,
+                       const uint32_t* fidx, const float* fmul, uint32_t col_offset, uint64_t* partial, uint32_t partial_slots,
+                       uint32_t partial_slot0, uint32_t* row_bound)
+{
     TopKArgs a{};
     a.in = in;
-    a.pitch = width;
+    a.pitch = pitch;
     a.width = width;
     a.k = k;
     a.segments = 1;
+    a.col_offset = col_offset;
     a.position = position;
     a.index = index;
     a.fstart = fstart;
@@ -1607,19 +1689,44 @@ int topk_guided_run(const float* in, uint32_t width, uint32_t batch, uint32_t k,
     a.fmul = fmul;
     a.keys = keys;
     a.values = values;
+    a.row_bound = row_bound;
     a.seg_max = seg_max;
-    a.nseg = nseg;
-#define DSX_GUIDED(F, E) hipLaunchKernelGGL((topk_guided_kernel<F, E>), dim3(batch), dim3(kTopkThreads), lds, ctx().stream, a)
-    if (nseg <= 2 * kTopkThreads) {
-        if (filtered) DSX_GUIDED(true, 2); else DSX_GUIDED(false, 2);
-    } else if (nseg <= 4 * kTopkThreads) {
-        if (filtered) DSX_GUIDED(true, 4); else DSX_GUIDED(false, 4);
-    } else {
-        if (filtered) DSX_GUIDED(true, 8); else DSX_GUIDED(false, 8);
+    a.nseg = (width + kGuidedSegWidth - 1) / kGuidedSegWidth;
+    a.part_segs = guided_part_segs(a.nseg, batch);
+    const uint32_t parts = (a.nseg + a.part_segs - 1) / a.part_segs;
+    if (partial) {
+        a.partial = partial;
+        a.partial_slots = partial_slots;
+        a.partial_slot0 = partial_slot0;
+    } else if (parts > 1) {
+        if (int rc = ensure_partial((size_t)batch * parts * k * sizeof(uint64_t), &a.partial)) return rc;
+        a.partial_slots = parts;
     }
-#undef DSX_GUIDED
+    if (fidx) {
+        if (k <= 64) launch_guided<1, true>(a, batch, parts);
+        else if (k <= 128) launch_guided<2, true>(a, batch, parts);
+        else launch_guided<4, true>(a, batch, parts);
+    } else {
+        if (k <= 64) launch_guided<1, false>(a, batch, parts);
+        else if (k <= 128) launch_guided<2, false>(a, batch, parts);
+        else launch_guided<4, false>(a, batch, parts);
+    }
     DSX_LAUNCH_CHECK("topk_guided_kernel");
+    if (!partial && parts > 1) return topk_merge(a.partial, parts, k, keys, values, batch);
     return DSX_OK;
+}
+
+// Guided top-K when it applies (64-column segments, enough of them that k segments are a small part of the row), the scan
+// otherwise.
+int topk_guided_run(const float* in, uint32_t width, uint32_t batch, uint32_t k, float* keys, uint32_t* values, const float* seg_max,
+                    uint32_t seg_width, uint32_t position, const uint32_t* index, const uint64_t* fstart, const uint64_t* fend,
+                    const uint32_t* fidx, const float* fmul)
+{
+    const uint32_t nseg = (width + kGuidedSegWidth - 1) / kGuidedSegWidth;
+    if (!seg_max || seg_width != kGuidedSegWidth || (k > 64 && nseg < 3 * k))
+        return topk_run(in, width, width, batch, k, keys, values, position, index, fstart, fend, fidx, fmul, 0, nullptr, 0, 0, 0);
+    return topk_guided_launch(in, width, width, batch, k, keys, values, seg_max, position, index, fstart, fend, fidx, fmul, 0, nullptr, 0, 0,
+                              nullptr);
 }
 
 // Fixed scratch of dsx_topk_filtered_static: the packed partial lists of rows split over several workgroups,
