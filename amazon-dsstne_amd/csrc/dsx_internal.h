@@ -99,6 +99,8 @@ int topk_run(const float* in, uint32_t pitch, uint32_t width, uint32_t batch, ui
 int topk_static_setup(int device);
 // The same for scores whose producer left the maxima of their 64-column segments (row pitch of seg_max: ceil(width / 64)); rows
 // are cut into topk_guided_parts(width, batch) parts, each with a list of its own in partial (or in the library's scratch).
+// k <= 128; topk_guided_pays: whether this is the faster way.
+bool topk_guided_pays(uint32_t batch, uint32_t width, uint32_t k);
 uint32_t topk_guided_parts(uint32_t width, uint32_t batch);
 int topk_guided_launch(const float* in, uint32_t pitch, uint32_t width, uint32_t batch, uint32_t k, float* keys, uint32_t* values,
                        const float* seg_max, uint32_t position, const uint32_t* index, const uint64_t* fstart, const uint64_t* fend,

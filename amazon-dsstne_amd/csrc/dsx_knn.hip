@@ -62,9 +62,10 @@ struct KnnWorkspace {
 static bool knn_few_queries(uint32_t num_queries) { return num_queries <= 64; }
 
 // Lists per query that the top-K of a block of ncols columns leaves: enough workgroups per query to fill the GPU.
-static uint32_t knn_block_lists(uint32_t num_queries, uint32_t ncols)
+static bool knn_block_guided(uint32_t num_queries, uint32_t ncols, uint32_t k) { return knn_few_queries(num_queries) && topk_guided_pays(num_queries, ncols, k); }
+static uint32_t knn_block_lists(uint32_t num_queries, uint32_t ncols, uint32_t k)
 {
-    return knn_few_queries(num_queries) ? topk_guided_parts(ncols, num_queries) : topk_segments(num_queries, ncols, false);
+    return knn_block_guided(num_queries, ncols, k) ? topk_guided_parts(ncols, num_queries) : topk_segments(num_queries, ncols, false);
 }
 
 static KnnWorkspace knn_layout(void* base, uint32_t rows_padded, uint32_t num_queries, uint32_t k, bool f16 = false, uint32_t dim = 0,
@@ -79,7 +80,9 @@ static KnnWorkspace knn_layout(void* base, uint32_t rows_padded, uint32_t num_qu
     w.seg_max = knn_few_queries(num_queries) ? (float*)p : nullptr;
     if (w.seg_max) p += align256((size_t)num_queries * ((cb + 63) / 64) * sizeof(float));
     w.partial = (uint64_t*)p;
-    p += align256((size_t)num_queries * blocks * knn_block_lists(num_queries, cb) * k * sizeof(uint64_t));
+    // (a last block narrower than the others may be cut into more parts than they are, but not into more than fill half the GPU)
+    const uint32_t lists = std::max(knn_block_lists(num_queries, cb, k), std::max(topk_segments(num_queries, cb, false), (uint32_t)ctx().num_cus / (2 * std::max(1u, num_queries)) + 2));
+    p += align256((size_t)num_queries * blocks * lists * k * sizeof(uint64_t));
     w.row_bound = (uint32_t*)p;             // row_bound, cand_count and overflow are cleared together
     w.cand_count = w.row_bound + num_queries;
     w.overflow = w.cand_count + num_queries;
@@ -158,15 +161,16 @@ static int knn_search_blocks(const KnnWorkspace& w, const KnnOperands& op, uint3
     hipStream_t s = ctx().stream;
     const uint32_t cb = knn_block_columns(op.rows_padded, num_queries);
     const uint32_t blocks = (M + cb - 1) / cb;
-    const uint32_t lists_per_block = knn_block_lists(num_queries, cb);
-    const uint32_t lists = (blocks - 1) * lists_per_block + knn_block_lists(num_queries, M - (blocks - 1) * cb);
+    const uint32_t lists_per_block = knn_block_lists(num_queries, cb, k);
+    const uint32_t lists = (blocks - 1) * lists_per_block + knn_block_lists(num_queries, M - (blocks - 1) * cb, k);
     hipLaunchKernelGGL(knn_clear_kernel, dim3((num_queries + 255) / 256), dim3(256), 0, s, w.row_bound, num_queries);
     for (uint32_t blk = 0; blk < blocks; blk++) {
         const uint32_t c0 = blk * cb;
         const uint32_t ncols = std::min(cb, M - c0);
         t.start(s);
         uint32_t seg_width = 0;
-        int rc = op.into_matrix(c0, ncols, num_queries, w.block_scores, cb, w.seg_max, w.seg_max ? &seg_width : nullptr);
+        const bool guided = knn_block_guided(num_queries, ncols, k);
+        int rc = op.into_matrix(c0, ncols, num_queries, w.block_scores, cb, guided ? w.seg_max : nullptr, guided ? &seg_width : nullptr);
         if (rc) return rc;
         t.stop(s, t.gemm);
         t.start(s);
@@ -175,7 +179,7 @@ static int knn_search_blocks(const KnnWorkspace& w, const KnnOperands& op, uint3
                                     nullptr, c0, w.partial, lists, blk * lists_per_block, w.row_bound);
         else
             rc = topk_run(w.block_scores, cb, ncols, num_queries, k, nullptr, nullptr, 0, nullptr, nullptr, nullptr, nullptr, nullptr, c0,
-                          w.partial, lists, blk * lists_per_block, knn_block_lists(num_queries, ncols), w.row_bound);
+                          w.partial, lists, blk * lists_per_block, knn_block_lists(num_queries, ncols, k), w.row_bound);
         if (rc) return rc;
         t.stop(s, t.topk);
     }

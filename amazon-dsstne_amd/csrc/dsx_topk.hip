@@ -25,6 +25,9 @@
 
 namespace dsx {
 
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));   // 128-bit loads of any row
+
 constexpr int kTopkThreads = 256;
 constexpr int kTopkWaves = kTopkThreads / kWave;
 constexpr uint32_t kMaxBitmapBits = 256 * 1024;   // 32 KiB of LDS per workgroup
@@ -38,11 +41,12 @@ __device__ __forceinline__ uint64_t pack_score(float key, uint32_t col)
 // >= the result.  A radix-4 search over key bits 31..12; each step is three vector compares per key and scalar bookkeeping.
 // Twelve bits of slack admit a handful of extra candidates, and save a third of a dependent chain that every wave runs
 // before it can ask for more data.
-template <int N> __device__ __forceinline__ uint32_t wave_kth_key(const uint32_t (&key)[N], uint32_t k)
+// LOW = 0 searches all bits: the k-th largest key itself.
+template <int N, int LOW = 12> __device__ __forceinline__ uint32_t wave_kth_key(const uint32_t (&key)[N], uint32_t k)
 {
     uint32_t t = 0;
 #pragma unroll 1
-    for (int bit = 30; bit >= 12; bit -= 2) {
+    for (int bit = 30; bit >= LOW; bit -= 2) {
         const uint32_t c1 = t | (1u << bit), c2 = t | (2u << bit), c3 = t | (3u << bit);
         uint32_t n1 = 0, n2 = 0, n3 = 0;
 #pragma unroll
@@ -142,10 +146,10 @@ template <int R> struct WaveTopK {
     static constexpr int L = kWave * R;
     static constexpr int kBurst = 5 * kWave;            // most words staged between two checks of the fill level
     // Words that may wait before they are merged into the list.  A workgroup none of whose wavefronts ever merged finishes by
-    // counting instead of sorting (finish_row), so for the shorter lists there is room for twice their length.
-    static constexpr int kDrainAt = (R <= 2) ? 2 * L : L;
+    // counting instead of sorting (finish_row), so there is room for about three times k of them in the four wavefronts.
+    static constexpr int kDrainAt = (R == 1) ? 128 : 192;
     static constexpr int kStageWords = kDrainAt + kBurst;
-    static constexpr int kCountWords = (R == 1) ? 256 : 512;   // most words of a workgroup that finish_row counts
+    static constexpr int kCountWords = (R == 4) ? 512 : 256;   // most words of a workgroup that finish_row counts
 
     uint64_t q[R];        // sorted descending over position r*64 + lane; 0 = empty slot
     uint64_t thr;         // current k-th word: candidates must be strictly larger
@@ -381,20 +385,56 @@ __device__ __forceinline__ void finish_row(WaveTopK<R>& list, uint64_t (*sStage)
         }
     };
 
-    const uint32_t n0 = sPublished[0], n1 = sPublished[1], n2 = sPublished[2], n3 = sPublished[3];
-    const uint32_t total = n0 + n1 + n2 + n3;
+    uint32_t n0 = sPublished[0], n1 = sPublished[1], n2 = sPublished[2], n3 = sPublished[3];
+    uint32_t total = n0 + n1 + n2 + n3;
     const bool any_flushed = (sFlushed[0] | sFlushed[1] | sFlushed[2] | sFlushed[3]) != 0;   // the same for every wave
+    auto fetch = [&](uint32_t i) -> uint64_t {   // the i-th of all staged words
+        if (i >= total) return 0ull;   // never larger than anything
+        const uint32_t w = (i >= n0) + (i >= n0 + n1) + (i >= n0 + n1 + n2);
+        const uint32_t first = (w == 0) ? 0 : (w == 1) ? n0 : (w == 2) ? n0 + n1 : n0 + n1 + n2;
+        return sStage[w][i - first];
+    };
+    if (R > 1 && !any_flushed && total > (uint32_t)(R == 2 ? 4 : 5) * kWave && total > a.k) {
+        // The general scan stages up to twice k words, and counting costs their number squared: the exact k-th key first (one
+        // wavefront searches; which one depends on the row, so that the four SIMDs of a compute unit share the work of the
+        // workgroups on it), then every wave drops its words below it.
+        constexpr int N = (4 * WaveTopK<R>::kDrainAt) / kWave;
+        __shared__ uint32_t sKth;
+        if (wave == ((b >> 8) & 3u)) {
+            uint32_t t;
+            auto search = [&](auto lanes_words) __attribute__((always_inline)) {
+                constexpr int C = decltype(lanes_words)::value;
+                uint32_t key[C];
+#pragma unroll
+                for (int m = 0; m < C; m++) key[m] = (uint32_t)(fetch(m * kWave + lane) >> 32);
+                return wave_kth_key<C, 0>(key, a.k);
+            };
+            if (total <= 4 * kWave) t = search(std::integral_constant<int, 4>());
+            else if (total <= 6 * kWave) t = search(std::integral_constant<int, 6>());
+            else t = search(std::integral_constant<int, N>());
+            if (lane == 0) sKth = t;
+        }
+        __syncthreads();
+        const uint32_t t = sKth, had = sPublished[wave];
+        uint32_t kept = 0;
+        for (uint32_t i0 = 0; i0 < had; i0 += kWave) {   // (in place: nothing moves to a later position)
+            const uint64_t word = (i0 + lane < had) ? sStage[wave][i0 + lane] : 0ull;
+            const bool keep = (uint32_t)(word >> 32) >= t && word != 0;
+            const uint64_t m = __ballot(keep);
+            __builtin_amdgcn_wave_barrier();
+            if (keep) sStage[wave][kept + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))] = word;
+            kept += (uint32_t)__popcll(m);
+        }
+        if (lane == 0) sPublished[wave] = kept;
+        list.count = kept;
+        __syncthreads();
+        n0 = sPublished[0], n1 = sPublished[1], n2 = sPublished[2], n3 = sPublished[3];
+        total = n0 + n1 + n2 + n3;
+    }
     if (!any_flushed && total <= (uint32_t)kCount) {
         // Common case: a few words more than k in all, none of them merged yet.  The number of staged words that are larger is a
         // word's place in the result, so no sorting network runs at all.  Every lane holds the i-th, (64 + i)-th, ... of the words,
-        // every wave compares them with its own staged ones and adds its counts in LDS.  (256 words of a k = 128 row: about 750
-        // instructions per wave, spread over four waves, against a chain of six sorts and merges in one of them.)
-        auto fetch = [&](uint32_t i) -> uint64_t {
-            if (i >= total) return 0ull;   // never larger than anything
-            const uint32_t w = (i >= n0) + (i >= n0 + n1) + (i >= n0 + n1 + n2);
-            const uint32_t first = (w == 0) ? 0 : (w == 1) ? n0 : (w == 2) ? n0 + n1 : n0 + n1 + n2;
-            return sStage[w][i - first];
-        };
+        // every wave compares them with its own staged ones and adds its counts in LDS.
         const uint32_t mine = sPublished[wave];
         auto count = [&](auto lanes_words) __attribute__((always_inline)) {
             constexpr int N = decltype(lanes_words)::value;   // words per lane
@@ -422,7 +462,9 @@ __device__ __forceinline__ void finish_row(WaveTopK<R>& list, uint64_t (*sStage)
         };
         if (total <= kWave) count(std::integral_constant<int, 1>());   // the same for the whole workgroup
         else if (total <= 2 * kWave) count(std::integral_constant<int, 2>());
+        else if (total <= 3 * kWave) count(std::integral_constant<int, 3>());
         else if (M <= 4 || total <= 4 * kWave) count(std::integral_constant<int, 4>());
+        else if (total <= 5 * kWave) count(std::integral_constant<int, 5>());
         else count(std::integral_constant<int, M>());
         __syncthreads();
         for (uint32_t i = wave * kWave + lane; i < total; i += kTopkThreads) {
@@ -456,13 +498,11 @@ __device__ __forceinline__ void finish_row(WaveTopK<R>& list, uint64_t (*sStage)
     }
 }
 
+// The scan of a (row, segment) of any width: sBitmap holds a bit for every column of the segment when FILTERED.
 template <int R, bool FILTERED>
-__global__ __launch_bounds__(kTopkThreads, (R <= 2) ? 4 : 2) void topk_scan_kernel(TopKArgs a)
+__device__ __forceinline__ void scan_segment(const TopKArgs& a, uint64_t (*sStage)[WaveTopK<R>::kStageWords], uint32_t* sBitmap)
 {
     using List = WaveTopK<R>;
-    __shared__ uint64_t sStage[kTopkWaves][List::kStageWords];
-    extern __shared__ uint32_t sBitmap[];
-
     const uint32_t b = blockIdx.x;
     const uint32_t seg = blockIdx.y;
     const uint32_t wave = threadIdx.x / kWave;
@@ -584,7 +624,7 @@ __global__ __launch_bounds__(kTopkThreads, (R <= 2) ? 4 : 2) void topk_scan_kern
         }
     };
 
-    // Priming (k <= 128): before anything is admitted, every lane takes the best score of its groups in each of the first two spans.
+    // Priming: before anything is admitted, every lane takes the best score of its groups in each of the first two spans.
     // The k-th best of a wave's 128 maxima is a score that at least k unfiltered items reach, so nothing below it can be in the
     // result; the k-th best of the 4k scores the four waves publish is a bound for the whole workgroup.  It is found by
     // binary search on the key bits (no sorting), and the scan then admits a few dozen items per row instead of a few
@@ -594,6 +634,7 @@ __global__ __launch_bounds__(kTopkThreads, (R <= 2) ? 4 : 2) void topk_scan_kern
     // the segment, 60 % of a 27,278-column row.  (A bound from the first span alone admits twice as many items on average
     // and, in the unlucky row of a large batch, ten times as many: the slowest row sets the kernel's time.)
     __shared__ uint32_t sPrime[kTopkWaves][2 * kWave];
+    __shared__ uint32_t sPrimeKey;
     auto prime_from_first_spans = [&]() {
         constexpr int PV = 2;
         uint32_t taint = 0;
@@ -610,28 +651,44 @@ __global__ __launch_bounds__(kTopkThreads, (R <= 2) ? 4 : 2) void topk_scan_kern
             }
             key[v] = score_key(m);
         }
-        const uint32_t tw = wave_kth_key<PV>(key, a.k);
-        uint32_t published = 0;   // wave-uniform
-#pragma unroll
-        for (int v = 0; v < PV; v++) {
-            const bool pub = key[v] >= tw;   // at least k values of the wavefront
-            const uint64_t pm = __ballot(pub);
-            const uint32_t pos = published + __builtin_amdgcn_mbcnt_hi((uint32_t)(pm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)pm, 0u));
-            if (pub && pos < a.k) sPrime[wave][pos] = key[v];
-            published += (uint32_t)__popcll(pm);
-        }
-        __syncthreads();
-        uint32_t all[4 * PV];   // the 4k published keys, side by side
-#pragma unroll
-        for (int n = 0; n < 4 * PV; n++) {
-            const uint32_t i = n * kWave + lane;
-            all[n] = (i < kTopkWaves * a.k) ? sPrime[i / a.k][i % a.k] : 0u;
-        }
         uint32_t t;
-        if (a.k <= 16) t = wave_kth_key<1>(reinterpret_cast<const uint32_t(&)[1]>(all), a.k);
-        else if (a.k <= 32) t = wave_kth_key<2>(reinterpret_cast<const uint32_t(&)[2]>(all), a.k);
-        else if (a.k <= 64) t = wave_kth_key<4>(reinterpret_cast<const uint32_t(&)[4]>(all), a.k);
-        else t = wave_kth_key<4 * PV>(all, a.k);
+        if constexpr (R == 1) {
+            const uint32_t tw = wave_kth_key<PV>(key, a.k);
+            uint32_t published = 0;   // wave-uniform
+#pragma unroll
+            for (int v = 0; v < PV; v++) {
+                const bool pub = key[v] >= tw;   // at least k values of the wavefront
+                const uint64_t pm = __ballot(pub);
+                const uint32_t pos = published + __builtin_amdgcn_mbcnt_hi((uint32_t)(pm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)pm, 0u));
+                if (pub && pos < a.k) sPrime[wave][pos] = key[v];
+                published += (uint32_t)__popcll(pm);
+            }
+            __syncthreads();
+            uint32_t all[4];   // the 4k published keys, side by side
+#pragma unroll
+            for (int n = 0; n < 4; n++) {
+                const uint32_t i = n * kWave + lane;
+                all[n] = (i < kTopkWaves * a.k) ? sPrime[i / a.k][i % a.k] : 0u;
+            }
+            if (a.k <= 16) t = wave_kth_key<1>(reinterpret_cast<const uint32_t(&)[1]>(all), a.k);
+            else if (a.k <= 32) t = wave_kth_key<2>(reinterpret_cast<const uint32_t(&)[2]>(all), a.k);
+            else t = wave_kth_key<4>(all, a.k);
+        } else {
+            // k is a large part of the 512 maxima: they are searched at once, by one wavefront (a different one from row to row, so
+            // that the four SIMDs of a compute unit share the searches of the workgroups on it)
+#pragma unroll
+            for (int v = 0; v < PV; v++) sPrime[wave][v * kWave + lane] = key[v];
+            __syncthreads();
+            if (wave == ((b >> 8) & 3u)) {
+                uint32_t all[4 * PV];
+#pragma unroll
+                for (int n = 0; n < 4 * PV; n++) all[n] = sPrime[n / PV][(n % PV) * kWave + lane];
+                const uint32_t found = wave_kth_key<4 * PV>(all, a.k);
+                if (lane == 0) sPrimeKey = found;
+            }
+            __syncthreads();
+            t = sPrimeKey;
+        }
         if (t > score_key(-__builtin_inff())) {
             list.prime(t);
             // Rows whose best scores tie in their hundreds (saturated sigmoids: exactly 1.0f in every eighth column) would
@@ -668,7 +725,7 @@ __global__ __launch_bounds__(kTopkThreads, (R <= 2) ? 4 : 2) void topk_scan_kern
             }
         }
     };
-    if (R <= 2 && g0 < g1) prime_from_first_spans();   // (k <= 128)
+    if (g0 < g1) prime_from_first_spans();
 
     // The four scores of one 16-byte group; at most 4 * 64 words are staged.
     auto stage_group = [&](const float4& v, uint32_t col) {
@@ -773,6 +830,186 @@ __global__ __launch_bounds__(kTopkThreads, (R <= 2) ? 4 : 2) void topk_scan_kern
     }
 
     finish_row<R>(list, sStage, a, b, seg, wave, lane);
+}
+
+template <int R, bool FILTERED>
+__global__ __launch_bounds__(kTopkThreads, 4) void topk_scan_kernel(TopKArgs a)
+{
+    __shared__ uint64_t sStage[kTopkWaves][WaveTopK<R>::kStageWords];
+    extern __shared__ uint32_t sBitmap[];
+    scan_segment<R, FILTERED>(a, sStage, sBitmap);
+}
+
+// The same for a segment of at most G * 1,024 columns, which the workgroup holds in registers: every score is requested before
+// anything else happens, and the bound is taken over all of them, so that little more than k words pass it (the scan's bound has
+// seen 60 % of a 27,278-column row when it starts to admit words, and admits 1.9 k).  With 1,024 rows on the GPU at once a compute
+// unit's four workgroups get their data one after the other, and one's selection runs under the next one's loads.
+// Steps: R maxima per lane over its 16-byte groups that hold no listed column; their k-th largest is the bound; every wavefront
+// stages its scores that reach it, then strikes out the listed ones, and finish_row puts the words in order.  A segment that this
+// does not settle (fewer than k scores above 0 besides the listed ones, more survivors than the staging area holds: ties by the
+// hundred) is scanned again in the general way.
+template <int R, bool FILTERED, int G>
+__global__ __launch_bounds__(kTopkThreads, 4) void topk_block_kernel(TopKArgs a)
+{
+    using List = WaveTopK<R>;
+    __shared__ uint64_t sStage[kTopkWaves][List::kStageWords];
+    __shared__ uint32_t sMax[R * kTopkThreads];
+    __shared__ uint32_t sTaint[FILTERED ? kTopkThreads : 1];   // bit u: the lane's group u holds a listed column
+    __shared__ uint32_t sBound, sReach, sStaged;
+    extern __shared__ uint32_t sBitmap[];
+    const uint32_t b = blockIdx.x, seg = blockIdx.y;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+    const float* row = a.in + (uint64_t)b * a.pitch;
+    // (the segment is cut as the general scan cuts it: at most 6 columns more than its 16-byte groups hold)
+    const uint32_t head = min((4 - (uint32_t)(((uintptr_t)row >> 2) & 3)) & 3u, a.width);
+    const uint32_t nvec = (a.width - head) / 4, gps = (nvec + a.segments - 1) / a.segments;
+    const uint32_t g0 = min(seg * gps, nvec), g1 = min(g0 + gps, nvec);
+    const uint32_t lo = (seg == 0) ? 0 : head + 4 * g0, hi = (seg == a.segments - 1) ? a.width : head + 4 * g1;
+
+    uint64_t fs = 0, fe = 0;
+    if constexpr (FILTERED) {
+        uint32_t r = a.position + b;
+        if (a.index) r = a.index[r];
+        fs = a.fstart[r];
+        fe = a.fend[r];
+    }
+    f32x4 v[G];
+#pragma unroll
+    for (int u = 0; u < G; u++) {
+        const uint32_t first = lo + u * 4 * kTopkThreads;   // uniform
+        const uint32_t col = first + 4 * threadIdx.x;
+        if (first + 4 * kTopkThreads <= hi) {
+            v[u] = *reinterpret_cast<const float4u*>(row + col);
+        } else {
+            const float nan = __uint_as_float(0x7fc00000u);   // fails every comparison below
+            v[u] = f32x4{nan, nan, nan, nan};
+            if (col + 4 <= hi) v[u] = *reinterpret_cast<const float4u*>(row + col);
+            else {
+                if (col < hi) v[u].x = row[col];
+                if (col + 1 < hi) v[u].y = row[col + 1];
+                if (col + 2 < hi) v[u].z = row[col + 2];
+            }
+        }
+    }
+    uint32_t taint = 0;
+    if constexpr (FILTERED) {
+        const uint32_t words = (hi - lo + 31) / 32;
+        for (uint32_t i = threadIdx.x; i < words; i += kTopkThreads) sBitmap[i] = 0;
+        sTaint[threadIdx.x] = 0;
+    }
+    if (threadIdx.x == 0) sReach = sStaged = 0;
+    if constexpr (FILTERED) {
+        __syncthreads();
+        for (uint64_t t = fs + threadIdx.x; t < fe; t += kTopkThreads) {
+            const uint32_t c = a.fidx[t];
+            if (c >= lo && c < hi) {
+                atomicOr(&sBitmap[(c - lo) >> 5], 1u << ((c - lo) & 31));
+                atomicOr(&sTaint[((c - lo) / 4) % kTopkThreads], 1u << ((c - lo) / (4 * kTopkThreads)));
+            }
+        }
+        __syncthreads();
+        taint = sTaint[threadIdx.x];
+    }
+    // maximum i of a lane: its groups i, i + R, ...
+#pragma unroll
+    for (int i = 0; i < R; i++) {
+        float m = -__builtin_inff();
+#pragma unroll
+        for (int u = i; u < G; u += R) {
+            float g = fmaxf(fmaxf(v[u].x, v[u].y), fmaxf(v[u].z, v[u].w));   // fmaxf drops NaN
+            if constexpr (FILTERED) g = __uint_as_float(__float_as_uint(g) | (uint32_t)__builtin_amdgcn_sbfe((int)taint, u, 1));   // listed: NaN
+            m = fmaxf(m, g);
+        }
+        sMax[i * kTopkThreads + threadIdx.x] = score_key(m);
+    }
+    __syncthreads();
+    // (one wavefront searches, a different one from row to row, so that the four SIMDs of a compute unit share the searches)
+    if (wave == ((b >> 8) & 3u)) {
+        uint32_t t;
+        if (R == 1 && a.k <= 16) {   // the largest of each lane's four: the exact bound unless two of the k best share a lane
+            uint32_t best[1] = {0u};
+#pragma unroll
+            for (int n = 0; n < 4; n++) best[0] = max(best[0], sMax[n * kWave + lane]);
+            t = wave_kth_key<1>(best, a.k);
+        } else {
+            uint32_t all[4 * R];
+#pragma unroll
+            for (int n = 0; n < 4 * R; n++) all[n] = sMax[n * kWave + lane];
+            t = wave_kth_key<4 * R>(all, a.k);
+        }
+        if (lane == 0) sBound = t;
+    }
+    __syncthreads();
+    uint32_t t = sBound;
+    const uint32_t none = score_key(-__builtin_inff());
+    bool failed = t <= none;   // fewer than k maxima
+    if (FILTERED && t <= score_key(0.0f)) failed = true;   // listed columns score 0 and may belong in the result
+    if (a.row_bound) t = max(t, a.row_bound[b]);           // (a bound from earlier columns of the row: fewer than k words may pass)
+    // Saturated activations have thousands of scores at exactly 1.0.  Among equal scores the lower column wins: when k of the
+    // segment's first 1,024 columns reach the bound, later ones have to lie above it.
+    const float bound = key_score(t);
+    float later = bound;
+    {
+        uint32_t reach = 0;
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            bool ok = v[0][c] >= bound;
+            if constexpr (FILTERED) {
+                const uint32_t off = 4 * threadIdx.x + c;
+                if (ok) ok = !((sBitmap[off >> 5] >> (off & 31)) & 1u);
+            }
+            reach += (uint32_t)__popcll(__ballot(ok));
+        }
+        if (lane == 0 && reach != 0) atomicAdd(&sReach, reach);
+        __syncthreads();
+        if (sReach >= a.k) later = key_score(t + 1u);   // (above +inf this is NaN, which nothing reaches)
+    }
+    uint32_t count = 0;   // wave-uniform
+    if (!failed) {
+#pragma unroll
+        for (int u = 0; u < G; u++) {
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const float need = (u == 0) ? bound : later;
+                const uint64_t m = __ballot(v[u][c] >= need);
+                if (m == 0) continue;
+                const uint32_t at = count + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+                if (v[u][c] >= need && at < (uint32_t)List::kStageWords) sStage[wave][at] = pack_score(v[u][c], lo + (u * kTopkThreads + threadIdx.x) * 4 + c);
+                count += (uint32_t)__popcll(m);
+            }
+        }
+    }
+    const bool full = count > (uint32_t)List::kStageWords - 4;   // (finish_row reads up to three words beyond the last)
+    if (full) count = 0;
+    if constexpr (FILTERED) {   // the listed ones are struck out, 64 at a time and in place
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        uint32_t kept = 0;
+        for (uint32_t i0 = 0; i0 < count; i0 += kWave) {
+            const uint64_t word = (i0 + lane < count) ? sStage[wave][i0 + lane] : 0ull;
+            bool keep = word != 0;
+            if (keep) {
+                const uint32_t off = ~(uint32_t)word - lo;
+                keep = !((sBitmap[off >> 5] >> (off & 31)) & 1u);
+            }
+            const uint64_t m = __ballot(keep);
+            __builtin_amdgcn_wave_barrier();
+            if (keep) sStage[wave][kept + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))] = word;
+            kept += (uint32_t)__popcll(m);
+        }
+        count = kept;
+    }
+    List list;
+    list.init(sStage[wave], lane, a.k);
+    list.count = count;
+    if (lane == 0) atomicAdd(&sStaged, full ? 0x10000u : count);
+    __syncthreads();
+    failed = failed || sStaged > ((R == 1) ? (uint32_t)List::kCountWords : 4u * (uint32_t)List::kDrainAt);   // the same for the whole workgroup
+    if (!failed) {
+        finish_row<R>(list, sStage, a, b, seg, wave, lane);
+        return;
+    }
+    scan_segment<R, FILTERED>(a, sStage, sBitmap);
 }
 
 // Guided top-K: the producer of the scores also left the maximum of every 64-column segment of every row (the
@@ -931,6 +1168,21 @@ __global__ __launch_bounds__(kTopkThreads, R <= 2 ? 4 : 2) void topk_guided_kern
                 const uint32_t t = wave_kth_key<1>(best, a.k);
                 if (lane == 0) sBound = t;
             }
+        } else if (R > 1 && E <= 4) {
+            // k is a large part of the maxima: all of them are searched at once
+#pragma unroll
+            for (int e = 0; e < E; e++) {
+                const uint32_t idx = e * kTopkThreads + threadIdx.x;
+                if (idx < nseg) sListKey[idx] = tk[e];
+            }
+            __syncthreads();
+            if (wave == 0) {
+                uint32_t all[4 * E];
+#pragma unroll
+                for (int n = 0; n < 4 * E; n++) all[n] = (n * kWave + lane < nseg) ? sListKey[n * kWave + lane] : 0u;
+                const uint32_t t = wave_kth_key<4 * E>(all, a.k);
+                if (lane == 0) sBound = t;
+            }
         } else {
             const uint32_t tw = wave_kth_key<E>(tk, a.k);
             uint32_t published = 0;   // wave-uniform
@@ -986,7 +1238,7 @@ __global__ __launch_bounds__(kTopkThreads, R <= 2 ? 4 : 2) void topk_guided_kern
     }
     __syncthreads();
     const uint32_t count = sListCount;
-    constexpr int kSegsInFlight = 8;
+    constexpr int kSegsInFlight = (R == 1) ? 8 : 16;   // per wavefront
     // More segments than one round of reads takes, and many more than k (rows of tied scores, mostly): the list is written again in ascending
     // order, so that the first round reads the lowest columns and what only ties behind them can be left out.  Lane j holds
     // the count of the j-th group of 64 maxima; a scan over the first lanes gives every group its place.
@@ -1220,9 +1472,26 @@ static int ensure_partial(size_t bytes, uint64_t** out)
     return DSX_OK;
 }
 
+template <int R, int G> static void launch_block(const TopKArgs& a, uint32_t batch, bool filtered, size_t bitmap_bytes)
+{
+    const dim3 grid(batch, a.segments);
+    if (filtered) hipLaunchKernelGGL((topk_block_kernel<R, true, G>), grid, dim3(kTopkThreads), bitmap_bytes, ctx().stream, a);
+    else hipLaunchKernelGGL((topk_block_kernel<R, false, G>), grid, dim3(kTopkThreads), 0, ctx().stream, a);
+}
+
 template <int R> static int launch_scan(const TopKArgs& a, uint32_t batch, bool filtered, size_t bitmap_bytes)
 {
     dim3 grid(batch, a.segments);
+    // Segments that fit a workgroup's registers (multipliers other than 0 need the listed scores: the general scan).
+    const uint32_t columns = ((a.width / 4 + 1 + a.segments - 1) / a.segments) * 4 + 8;   // an upper bound of a segment's
+    if (!a.fmul && columns <= 27 * 4 * kTopkThreads) {
+        if (columns <= 2 * 4 * kTopkThreads) launch_block<R, 2>(a, batch, filtered, bitmap_bytes);
+        else if (columns <= 8 * 4 * kTopkThreads) launch_block<R, 8>(a, batch, filtered, bitmap_bytes);
+        else if (columns <= 16 * 4 * kTopkThreads) launch_block<R, 16>(a, batch, filtered, bitmap_bytes);
+        else launch_block<R, 27>(a, batch, filtered, bitmap_bytes);
+        DSX_LAUNCH_CHECK("topk_block_kernel");
+        return DSX_OK;
+    }
     if (filtered)
         hipLaunchKernelGGL((topk_scan_kernel<R, true>), grid, dim3(kTopkThreads), bitmap_bytes, ctx().stream, a);
     else
@@ -1642,10 +1911,12 @@ int layer_refresh_run(const LayerRefresh& r, uint32_t batch)
     return DSX_OK;
 }
 
-// Segments per workgroup of the guided top-K: up to 2,048, and no more than 1,024 where the rows alone leave the GPU idle.
+// Segments per workgroup of the guided top-K: up to 2,048, and down to 512 where that would leave three quarters of the compute
+// units without a workgroup (4 x 1,000,000 k = 10: 10.8 -> 9.7 us; a merge is the price, 100 x 60,000: 7.5 us whole, 10.2 cut).
 static uint32_t guided_part_segs(uint32_t nseg, uint32_t batch)
 {
-    const uint32_t most = (batch < (uint32_t)ctx().num_cus) ? kGuidedMaxSegs / 2 : kGuidedMaxSegs;
+    uint32_t most = kGuidedMaxSegs;
+    while (most > kGuidedMaxSegs / 4 && 4ull * batch * ((nseg + most - 1) / most) <= (uint64_t)ctx().num_cus) most /= 2;
     const uint32_t parts = (nseg + most - 1) / most;
     return (nseg + parts - 1) / parts;
 }
@@ -1702,28 +1973,34 @@ int topk_guided_launch(const float* in, uint32_t pitch, uint32_t width, uint32_t
         if (int rc = ensure_partial((size_t)batch * parts * k * sizeof(uint64_t), &a.partial)) return rc;
         a.partial_slots = parts;
     }
-    if (fidx) {
-        if (k <= 64) launch_guided<1, true>(a, batch, parts);
-        else if (k <= 128) launch_guided<2, true>(a, batch, parts);
-        else launch_guided<4, true>(a, batch, parts);
+    if (k <= 64) {
+        if (fidx) launch_guided<1, true>(a, batch, parts);
+        else launch_guided<1, false>(a, batch, parts);
     } else {
-        if (k <= 64) launch_guided<1, false>(a, batch, parts);
-        else if (k <= 128) launch_guided<2, false>(a, batch, parts);
-        else launch_guided<4, false>(a, batch, parts);
+        if (fidx) launch_guided<2, true>(a, batch, parts);
+        else launch_guided<2, false>(a, batch, parts);
     }
     DSX_LAUNCH_CHECK("topk_guided_kernel");
     if (!partial && parts > 1) return topk_merge(a.partial, parts, k, keys, values, batch);
     return DSX_OK;
 }
 
-// Guided top-K when it applies (64-column segments, enough of them that k segments are a small part of the row), the scan
-// otherwise.
+// Whether the guided top-K is the faster one, given segment maxima: k <= 64 and at least 3 k segments (us, guided / scan, filtered:
+// 1,024 x 27,278 k = 10 8.1 / 23, k = 64 20.8 / 26; 300 x 5,000 k = 32 11.0 / 10.7); up to 128, where k segments are a large part of
+// the row, for score matrices that do not stay in the caches anyway (4,096 x 27,278 k = 100 76 / 96, k = 128 94 / 99; 64 x 27,278
+// k = 100 19.5 / 17.6); never above (8 x 500,000 k = 200 40 / 34).
+bool topk_guided_pays(uint32_t batch, uint32_t width, uint32_t k)
+{
+    const uint32_t nseg = (width + kGuidedSegWidth - 1) / kGuidedSegWidth;
+    if (k <= 64) return nseg >= 3 * k;
+    return k <= 128 && nseg >= 4 * k && (uint64_t)batch * nseg >= 100000;
+}
+
 int topk_guided_run(const float* in, uint32_t width, uint32_t batch, uint32_t k, float* keys, uint32_t* values, const float* seg_max,
                     uint32_t seg_width, uint32_t position, const uint32_t* index, const uint64_t* fstart, const uint64_t* fend,
                     const uint32_t* fidx, const float* fmul)
 {
-    const uint32_t nseg = (width + kGuidedSegWidth - 1) / kGuidedSegWidth;
-    if (!seg_max || seg_width != kGuidedSegWidth || (k > 64 && nseg < 3 * k))
+    if (!seg_max || seg_width != kGuidedSegWidth || !topk_guided_pays(batch, width, k))
         return topk_run(in, width, width, batch, k, keys, values, position, index, fstart, fend, fidx, fmul, 0, nullptr, 0, 0, 0);
     return topk_guided_launch(in, width, width, batch, k, keys, values, seg_max, position, index, fstart, fend, fidx, fmul, 0, nullptr, 0, 0,
                               nullptr);
