@@ -1964,6 +1964,12 @@ int topk_guided_launch(const float* in, uint32_t pitch, uint32_t width, uint32_t
     a.seg_max = seg_max;
     a.nseg = (width + kGuidedSegWidth - 1) / kGuidedSegWidth;
     a.part_segs = guided_part_segs(a.nseg, batch);
+    if (!partial && a.part_segs < a.nseg && a.nseg <= kGuidedMaxSegs) {
+        // (a graph keeps no address of the library's scratch, which may have to be allocated now and may move when it grows)
+        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+        DSX_HIP(hipStreamIsCapturing(ctx().stream, &capturing));
+        if (capturing != hipStreamCaptureStatusNone) a.part_segs = a.nseg;
+    }
     const uint32_t parts = (a.nseg + a.part_segs - 1) / a.part_segs;
     if (partial) {
         a.partial = partial;
