@@ -26,6 +26,11 @@ public:
     // inputs: [size][featureSize] row-major queries; keys / scores: [size][k], best first.
     void search(int k, const float* inputs, int size, std::string* keys, float* scores);
     void search(int k, const float* inputs, std::string* keys, float* scores) override { search(k, inputs, data->batchSize, keys, scores); }
+    // The same with the rows of the table in place of their keys.
+    void searchRows(int k, const float* inputs, int size, uint32_t* rows, float* scores);
+
+private:
+    void searchDevice(int k, const float* inputs, int size);   // leaves [size][maxK] results in data's host buffers
 };
 
 // k-way merge of per-device result lists (each [batchSize][width], descending); ties go to the lower device id.

@@ -2,6 +2,7 @@
 #include <cstring>
 #include <cstdarg>
 #include <stdexcept>
+#include <unordered_map>
 
 #include "amazon/dsstne/engine/NNTypes.h"
 #include "amazon/dsstne/knn/KnnExactGpu.h"
@@ -466,6 +467,15 @@ struct dsstne_knn {
     astdl::knn::KnnData* data = nullptr;
     astdl::knn::KnnExactGpu* knn = nullptr;
     bool numericKeys = true;
+    std::vector<uint32_t> firstRow;   // labelled tables: the first row with the same label as row i
+    void orderKeys()
+    {
+        firstRow.clear();
+        if (numericKeys) return;
+        const auto& all = data->hKeys[0];
+        std::unordered_map<std::string, uint32_t> order;
+        for (uint32_t i = 0; i < all.size(); i++) firstRow.push_back(order.emplace(all[i], i).first->second);
+    }
 };
 
 dsstne_knn* dsstne_knn_create(uint32_t batch, uint32_t max_k) { return dsstne_knn_create_typed(batch, max_k, "fp32"); }
@@ -489,6 +499,7 @@ int dsstne_knn_load(dsstne_knn* k, const float* items, uint32_t rows, uint32_t d
     ArrayDataReader reader(items, rows, (int)dim, keys ? skeys.data() : nullptr);
     k->data->load(0, &reader);
     k->numericKeys = (keys == nullptr);
+    k->orderKeys();
     return 0;
     CAPI_CATCH(-1)
 }
@@ -499,6 +510,7 @@ int dsstne_knn_load_file(dsstne_knn* k, const char* file, char kv_delim, char ve
     std::map<int, std::string> files = {{0, file}};
     k->data->load(files, kv_delim, vec_delim);
     k->numericKeys = false;
+    k->orderKeys();
     return 0;
     CAPI_CATCH(-1)
 }
@@ -506,22 +518,12 @@ int dsstne_knn_load_file(dsstne_knn* k, const char* file, char kv_delim, char ve
 int dsstne_knn_search(dsstne_knn* k, uint32_t kk, const float* queries, uint32_t size, float* scores, uint32_t* indexes)
 {
     CAPI_TRY
-    vector<string> keys((size_t)size * kk);
-    k->knn->search((int)kk, queries, (int)size, keys.data(), scores);
-    if (indexes) {
-        if (k->numericKeys) {
-            for (size_t i = 0; i < keys.size(); i++) indexes[i] = keys[i].empty() ? 0xffffffffu : (uint32_t)stoul(keys[i]);
-        } else {
-            // keys are arbitrary labels: report their load order
-            std::map<string, uint32_t> order;
-            const auto& all = k->data->hKeys[0];
-            for (uint32_t i = 0; i < all.size(); i++) order.emplace(all[i], i);
-            for (size_t i = 0; i < keys.size(); i++) {
-                auto it = order.find(keys[i]);
-                indexes[i] = it == order.end() ? 0xffffffffu : it->second;
-            }
-        }
-    }
+    vector<uint32_t> unwanted(indexes ? 0 : (size_t)size * kk);
+    uint32_t* const rows = indexes ? indexes : unwanted.data();
+    k->knn->searchRows((int)kk, queries, (int)size, rows, scores);
+    // keys are arbitrary labels: report their load order, the first row of those that share one
+    if (indexes && !k->numericKeys)
+        for (size_t i = 0; i < (size_t)size * kk; i++) indexes[i] = indexes[i] < k->firstRow.size() ? k->firstRow[indexes[i]] : 0xffffffffu;
     return 0;
     CAPI_CATCH(-1)
 }
