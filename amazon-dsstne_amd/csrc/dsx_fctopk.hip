@@ -71,10 +71,12 @@ struct LayerWorkspace {
     uint32_t* row_flag;    // [batch]
     uint32_t* overflow;    // [64] unused flag word of the shared epilogue
     uint64_t* cand;        // [batch][cap]
+    ScreenWorkspace screen;   // where the ranges are screened in 16 bits
     size_t bytes;
 };
 
-static LayerWorkspace layer_layout(void* base, uint32_t batch, uint32_t n0, uint32_t k, uint32_t cap, bool ranges)
+static LayerWorkspace layer_layout(void* base, uint32_t batch, uint32_t n0, uint32_t k, uint32_t cap, bool ranges, bool screened,
+                                   uint32_t kdim, uint32_t n)
 {
     LayerWorkspace w;
     char* p = (char*)base;
@@ -90,6 +92,11 @@ static LayerWorkspace layer_layout(void* base, uint32_t batch, uint32_t n0, uint
     p += align256(((size_t)3 * batch + 64) * sizeof(uint32_t));
     w.cand = (uint64_t*)p;
     if (ranges) p += align256((size_t)batch * cap * sizeof(uint64_t));
+    w.screen = ScreenWorkspace{};
+    if (screened) {
+        w.screen = screen_layout(p, batch, kdim, n, true, kLayerCandCap);
+        p += w.screen.bytes;
+    }
     w.bytes = (size_t)(p - (char*)base);
     return w;
 }
@@ -179,10 +186,11 @@ static int fc_topk_common(const float* X, uint32_t ldx, const float* W, const fl
     const uint32_t cap = ctx().knobs.fc_topk_candidate_capacity ? ctx().knobs.fc_topk_candidate_capacity : kLayerCandCap;   // tests lower it to reach the overflow path with small inputs
     const uint32_t n0 = layer_first_columns(n, k);
     const bool ranges = n0 < n;
-    const size_t need = layer_layout(nullptr, batch, n0, k, cap, ranges).bytes;
+    const bool screened = ranges && !x_planes && screen_takes(batch, kdim, n, true);
+    const size_t need = layer_layout(nullptr, batch, n0, k, cap, ranges, screened, kdim, n).bytes;
     LibScratch& ws = g_layer_ws_of[current_lane()];
     if (int rc = lib_scratch_reserve(ws, need, "dsx_fc_topk workspace")) return rc;
-    const LayerWorkspace w = layer_layout(ws.ptr, batch, n0, k, cap, ranges);
+    const LayerWorkspace w = layer_layout(ws.ptr, batch, n0, k, cap, ranges, screened, kdim, n);
     const uint32_t ld0 = (n0 + 3) / 4 * 4;
     hipStream_t s = ctx().stream;
 
@@ -197,6 +205,10 @@ static int fc_topk_common(const float* X, uint32_t ldx, const float* W, const fl
     const uint32_t clear_words = 3 * batch + 64;
     hipLaunchKernelGGL(layer_clear_kernel, dim3((clear_words + 255) / 256), dim3(256), 0, s, w.row_bound, clear_words);
     DSX_LAUNCH_CHECK("layer_clear_kernel");
+    if (screened) {
+        rc = screen_prepare(w.screen, X, ldx, batch, W, n, bias, n, kdim, true, w.row_flag, flag_word);
+        if (rc) return rc;
+    }
     rc = topk_run(w.block_scores, ld0, n0, batch, k, nullptr, nullptr, position, index, filter_start, filter_end, filter_index, nullptr, 0,
                   w.best, 1, 0, 1, w.row_bound);
     if (rc) return rc;
@@ -219,8 +231,9 @@ static int fc_topk_common(const float* X, uint32_t ldx, const float* W, const fl
         cand.slope = params ? params->slope : 0.01f;
         cand.alpha = params ? params->alpha : 1.0f;
         cand.lambda = params ? params->lambda : 1.0f;
-        rc = x_planes ? fc_split_candidates_run(x_planes, w_planes, wrows, done, batch, kdim, ncols, cand, true, bias ? bias + done : nullptr)
-                      : fc_layer_candidates_run(X, ldx, W + done, n, bias ? bias + done : nullptr, batch, kdim, ncols, cand);
+        if (screened) rc = screen_candidates(w.screen, X, ldx, batch, kdim, true, bias, ncols, cand, false);
+        else rc = x_planes ? fc_split_candidates_run(x_planes, w_planes, wrows, done, batch, kdim, ncols, cand, true, bias ? bias + done : nullptr)
+                           : fc_layer_candidates_run(X, ldx, W + done, n, bias ? bias + done : nullptr, batch, kdim, ncols, cand);
         if (rc) return rc;
         done += ncols;
         LayerRefresh r{};

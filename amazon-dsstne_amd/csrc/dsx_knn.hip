@@ -55,6 +55,7 @@ struct KnnWorkspace {
     void* queries16;        // fp16 storage: the query batch, [queries rounded up to 256][ld] halves; split products: its bf16 planes
     uint64_t* seg;          // fp16 storage only: [queries][chunks][kCandCap / chunks], the lists of a sweep (knn_f16_sweep_run)
     uint32_t* seg_count;    // fp16 storage only: [queries][64]
+    ScreenWorkspace screen; // fp32 storage, where screen_takes says so
     size_t bytes;
 };
 
@@ -101,6 +102,11 @@ static KnnWorkspace knn_layout(void* base, uint32_t rows_padded, uint32_t num_qu
         p += align256((size_t)num_queries * 64 * sizeof(uint32_t));
     }
     if (split) p += align256((size_t)split_plane_bytes(num_queries, dim));
+    w.screen = ScreenWorkspace{};
+    if (!f16 && !split && screen_takes(num_queries, dim, rows_padded, false)) {
+        w.screen = screen_layout(p, num_queries, dim, rows_padded, false, kCandCap);
+        p += w.screen.bytes;
+    }
     w.bytes = (size_t)(p - (char*)base);
     return w;
 }
@@ -213,9 +219,10 @@ static int knn_search_blocks(const KnnWorkspace& w, const KnnOperands& op, uint3
     return rc;
 }
 
-// First block as above, the rest in candidate mode.  *overflowed tells the caller to redo the search block by block.
+// First block as above, the rest in candidate mode, screened in 16 bits where asked for (fp32 storage).  *overflowed tells the caller
+// to redo the search without screening, or block by block.
 static int knn_search_candidates(const KnnWorkspace& w, const KnnOperands& op, uint32_t M, uint32_t num_queries, uint32_t k, float* scores,
-                                 uint32_t* indexes, KnnTimer& t, bool* overflowed)
+                                 uint32_t* indexes, KnnTimer& t, bool screened, bool* overflowed)
 {
     hipStream_t s = ctx().stream;
     const uint32_t cb = knn_block_columns(op.rows_padded, num_queries);
@@ -225,9 +232,13 @@ static int knn_search_candidates(const KnnWorkspace& w, const KnnOperands& op, u
     // The first block only has to give every query a usable bound; a quarter of a column block does (measured on 2 M items x 4,096
     // queries: 8 K to 32 K columns are level, the full 64 K cost 0.1 ms more in stores and scan).  A width set by the caller is kept.
     uint32_t done = std::min(cb, M);
-    if (!ctx().knobs.knn_block_columns) done = std::min<uint32_t>(done, std::max<uint32_t>(1024, cb / 4 / 1024 * 1024));
+    // (screened, later columns cost a tenth of the first block's: 8 K)
+    if (!ctx().knobs.knn_block_columns) done = std::min<uint32_t>(done, screened ? 8192u : std::max<uint32_t>(1024, cb / 4 / 1024 * 1024));
     t.start(s);
-    int rc = op.into_matrix(0, done, num_queries, w.block_scores, cb);
+    int rc = DSX_OK;
+    if (screened) rc = screen_prepare(w.screen, op.queries, op.dim, num_queries, op.items, op.rows_padded, nullptr, M, op.dim, false, w.overflow, nullptr);
+    if (rc) return rc;
+    rc = op.into_matrix(0, done, num_queries, w.block_scores, cb);
     if (rc) return rc;
     t.stop(s, t.gemm);
     t.start(s);
@@ -241,7 +252,8 @@ static int knn_search_candidates(const KnnWorkspace& w, const KnnOperands& op, u
         t.start(s);
         const CandArgs cand{w.row_bound, w.cand, w.cand_count, kCandCap, done, w.overflow};
         uint32_t chunks = 0;
-        rc = op.into_candidates(done, ncols, num_queries, cand, w.seg, w.seg_count, &chunks);
+        rc = screened ? screen_candidates(w.screen, op.queries, op.dim, num_queries, op.dim, false, nullptr, ncols, cand, true)
+                      : op.into_candidates(done, ncols, num_queries, cand, w.seg, w.seg_count, &chunks);
         if (rc) return rc;
         t.stop(s, t.gemm);
         t.start(s);
@@ -285,8 +297,7 @@ int dsx_testing_set_knn_f16_sweep(int mode)
 
 size_t dsx_knn_workspace_bytes(uint32_t rows_padded, uint32_t dim, uint32_t num_queries, uint32_t k)
 {
-    (void)dim;
-    return knn_layout(nullptr, rows_padded, num_queries, k).bytes;
+    return knn_layout(nullptr, rows_padded, num_queries, k, false, dim).bytes;
 }
 
 size_t dsx_knn_workspace_bytes_f16(uint32_t rows_padded, uint32_t dim, uint32_t num_queries, uint32_t k)
@@ -349,9 +360,13 @@ static int knn_search_common(KnnOperands& op, uint32_t padding, uint32_t num_que
     hipStreamIsCapturing(s, &capturing);
     // (few queries against an fp32 table stay with the blocks, however many there are; a width set by the caller is kept)
     const bool few = knn_few_queries(num_queries) && !op.f16 && !op.split && !ctx().knobs.knn_block_columns;
-    const bool candidates = aligned && !few && capturing == hipStreamCaptureStatusNone && M > knn_block_columns(op.rows_padded, num_queries);
+    const bool may = aligned && !few && capturing == hipStreamCaptureStatusNone;
+    const bool screened = may && w.screen.bytes != 0 && !ctx().knobs.knn_block_columns;
+    const bool candidates = may && (screened || M > knn_block_columns(op.rows_padded, num_queries));
     bool redo = !candidates;
-    if (rc == DSX_OK && candidates) rc = knn_search_candidates(w, op, M, num_queries, k, scores, indexes, t, &redo);
+    if (rc == DSX_OK && screened) rc = knn_search_candidates(w, op, M, num_queries, k, scores, indexes, t, true, &redo);
+    if (rc == DSX_OK && candidates && (!screened || redo) && M > knn_block_columns(op.rows_padded, num_queries))
+        rc = knn_search_candidates(w, op, M, num_queries, k, scores, indexes, t, false, &redo);
     g_knn_last_path = !candidates ? DSX_KNN_PATH_BLOCKS : (redo ? DSX_KNN_PATH_CANDIDATES_REDONE : DSX_KNN_PATH_CANDIDATES);
     if (rc == DSX_OK && redo) rc = knn_search_blocks(w, op, M, num_queries, k, scores, indexes, t);
     if (elapsed_ms) {

@@ -1,0 +1,119 @@
+"""fp32 searches whose candidates are screened in 16 bits (dsx_screen.hip): the results must be those of the fp32 scores, for operands that
+f16 holds badly too (subnormal, above its range, norms of very different size), at the edges of the tables' padding and of both sweeps."""
+
+import numpy as np
+import pytest
+
+from test_gpu_kernels import dev
+from test_oracle import random_csr
+
+pytestmark = pytest.mark.gpu
+
+
+def search(pkg, dsx, items, queries, k):
+    n, dim = items.shape
+    rows = (n + 7) // 8 * 8
+    cm = np.full((dim, rows), 1e30, dtype=np.float32)      # pad rows: never looked at
+    cm[:, :n] = items.T
+    dI, dQ = dev(pkg, cm), dev(pkg, queries)
+    scores, idx = pkg.DeviceArray((len(queries), k), np.float32), pkg.DeviceArray((len(queries), k), np.uint32)
+    pkg.check(dsx.dsx_knn_search(dI.ptr, rows, rows - n, dim, dQ.ptr, len(queries), k, scores.ptr, idx.ptr, None, 0, None))
+    return scores.numpy(), idx.numpy()
+
+
+def best(full, k):
+    """The k best of every row: score descending, then column ascending (NaN last)."""
+    part = np.argsort(-full, axis=1, kind="stable")[:, :k]
+    return np.take_along_axis(full, part, axis=1), part.astype(np.uint32)
+
+
+def check_against_float64(got_s, got_i, full, k, unit):
+    """Scores right for the columns returned, and no column left out whose score lies above the k-th by more than the roundings."""
+    want, _ = best(np.nan_to_num(full, nan=-np.inf), k)
+    at = np.take_along_axis(full, got_i.astype(np.int64), axis=1)
+    assert np.abs(got_s - at).max() <= unit
+    assert np.abs(np.sort(at, axis=1)[:, ::-1] - want).max() <= unit
+    assert all(len(set(r)) == k for r in got_i.tolist())
+
+
+# dim on both sides of a step of 64 and no multiple of 4; more than 256 (the other sweep); the smallest batch and table; a ragged table
+@pytest.mark.parametrize("n,queries,dim,k", [(65536, 512, 32, 10), (70003, 520, 36, 64), (66001, 513, 64, 256), (131075, 700, 128, 100),
+                                             (80000, 512, 260, 20), (65543, 1030, 100, 1)])
+def test_integer_vectors(pkg, dsx, rng, n, queries, dim, k):
+    """Every score is exact in fp32 and in f16, whatever the order of the sums; many tie."""
+    print("[case] screened knn n=%d queries=%d dim=%d k=%d" % (n, queries, dim, k), flush=True)
+    items = rng.integers(-3, 4, size=(n, dim)).astype(np.float32)
+    q = rng.integers(-3, 4, size=(queries, dim)).astype(np.float32)
+    s, i = search(pkg, dsx, items, q, k)
+    assert dsx.dsx_knn_last_search_path() == 1
+    rs, ri = best(q @ items.T, k)
+    assert np.array_equal(s, rs) and np.array_equal(i, ri)
+
+
+@pytest.mark.parametrize("form", ["unit", "subnormal", "above the range", "one large item", "nan items", "rising", "huge queries"])
+def test_operands_that_f16_holds_badly(pkg, dsx, rng, form):
+    n, queries, dim, k = 70001, 516, 48, 50
+    print("[case] screened knn %s" % form, flush=True)
+    items = rng.standard_normal((n, dim), dtype=np.float32) / np.float32(np.sqrt(dim))
+    q = rng.standard_normal((queries, dim), dtype=np.float32)
+    if form == "subnormal":
+        items *= np.float32(3e-6)
+    elif form == "above the range":
+        items *= np.float32(3e5)
+    elif form == "one large item":
+        items[n // 2] *= np.float32(1e4)
+    elif form == "nan items":
+        items[7::13, 5] = np.nan
+    elif form == "rising":
+        items = np.sort(items, axis=0)
+    elif form == "huge queries":
+        q[3] *= np.float32(1e6)
+    s, i = search(pkg, dsx, items, q, k)
+    full = q.astype(np.float64) @ items.astype(np.float64).T
+    # dim products, each rounding at most 2^-24 of |q| |w|: rows are compared in units of |q| max |w|
+    scale = np.linalg.norm(q.astype(np.float64), axis=1)[:, None] * np.nanmax(np.linalg.norm(items.astype(np.float64), axis=1))
+    check_against_float64(s / scale, i, full / scale, k, dim * 2.0 ** -24)
+
+
+# activations with and without a flat part; columns whose norms span four orders; a bias; a filter; both sides of the padding
+@pytest.mark.parametrize("batch,kdim,n,k,act,biased,filtered", [(4096, 32, 16384, 10, 0, True, True), (2200, 60, 17003, 100, 3, True, False),
+                                                                (2050, 64, 66000, 256, 2, False, True), (520, 508, 70001, 20, 1, True, True)])
+def test_layer(pkg, dsx, rng, batch, kdim, n, k, act, biased, filtered):
+    print("[case] screened layer batch=%d kdim=%d n=%d k=%d act=%d" % (batch, kdim, n, k, act), flush=True)
+    ldx = (kdim + 3) // 4 * 4
+    X = np.maximum(rng.standard_normal((batch, ldx), dtype=np.float32), 0)
+    W = rng.standard_normal((kdim, n), dtype=np.float32) * np.float32(1 / np.sqrt(kdim))
+    W *= (10.0 ** rng.uniform(-4, 0, n)).astype(np.float32)
+    bias = (rng.standard_normal(n) - 3).astype(np.float32) if biased else None
+    start = end = fidx = None
+    if filtered:
+        start, end, fidx = random_csr(rng, batch, n, 300)
+    dX, dW, db, ds, de, dx = (dev(pkg, a) for a in (X, W, bias, start, end, fidx))
+    keys, vals = pkg.DeviceArray((batch, k), np.float32), pkg.DeviceArray((batch, k), np.uint32)
+    pkg.check(dsx.dsx_fc_topk(dX.ptr, ldx, dW.ptr, pkg.ptr(db), batch, kdim, n, act, None, k, keys.ptr, vals.ptr, 0, None, pkg.ptr(ds),
+                              pkg.ptr(de), pkg.ptr(dx)))
+    z = X[:, :kdim].astype(np.float64) @ W.astype(np.float64) + (bias if biased else 0.0)
+    y = {0: lambda v: 1 / (1 + np.exp(-v)), 1: np.tanh, 2: lambda v: np.maximum(v, 0), 3: lambda v: v}[act](z)
+    if filtered:
+        for b in range(batch):
+            y[b, fidx[int(start[b]):int(end[b])]] *= 0.0
+    # sums of kdim products and the bias, |x| |w| + |b| below 40 here: kdim roundings of 2^-24 of that at the very most, 1e-6 for the
+    # activations' own error; slopes are at most 1
+    check_against_float64(keys.numpy(), vals.numpy(), y, k, (kdim + 8) * 40 * 2.0 ** -24 / 8 + 1e-6)
+
+
+def test_layer_above_the_range_is_recomputed(pkg, dsx, rng):
+    """A row that f16 cannot hold: its error has no bound, it is computed from scratch; the others are not."""
+    batch, kdim, n, k = 512, 256, 65536, 10
+    X = rng.standard_normal((batch, kdim), dtype=np.float32)
+    X[17] *= np.float32(1e6)
+    W = rng.standard_normal((kdim, n), dtype=np.float32)
+    dX, dW = dev(pkg, X), dev(pkg, W)
+    keys, vals = pkg.DeviceArray((batch, k), np.float32), pkg.DeviceArray((batch, k), np.uint32)
+    dsx.dsx_fc_topk_flagged(1)
+    pkg.check(dsx.dsx_fc_topk(dX.ptr, kdim, dW.ptr, None, batch, kdim, n, 3, None, k, keys.ptr, vals.ptr, 0, None, None, None, None))
+    y = X.astype(np.float64) @ W.astype(np.float64)
+    scale = np.linalg.norm(X.astype(np.float64), axis=1)[:, None] * 25
+    check_against_float64(keys.numpy() / scale, vals.numpy(), y / scale, k, kdim * 2.0 ** -24)
+    pkg.check(dsx.dsx_sync())
+    assert dsx.dsx_fc_topk_flagged(1) == 1
