@@ -153,6 +153,22 @@ int dsx_fc_topk_flagged_for(const float* W, int reset)
     return seen;
 }
 
+// Where the line lies (us, layer stored and guided top-K / this call, filter of 144 columns a row):
+//   From 131,072 columns on always, but for batches of up to 64: those are bound by reading the layer's weights once; storing their
+//   scores and maxima adds little to that, and this call's tiles of 128 rows a lot (8 x 256 x 500,000, top 50: 135 / 440).
+//   Narrower layers where the ranges are screened in 16 bits and that is most of the work: 4,096 x 1,024 x 27,278 top 10 2,011 / 920,
+//   1,904 rows 913 / 517, 2,048 x 512 x 27,278 490 / 281, 4,096 x 128 x 60,000 716 / 413; 1,024 x 1,024 x 27,278 468 / 370, but with
+//   own items that score high (trained networks) the candidates double.  Candidates grow with k: top 100 2,084 / 1,852, 4,096 x 512 x
+//   60,000 2,056 / 1,465, but 2,048 x 512 x 27,278 515 / 593.  Sigmoids only: their scores are above 0, so that no row has to be
+//   computed again for a listed column's zero.
+int dsx_fc_topk_pays(uint32_t batch, uint32_t k_dim, uint32_t n, uint32_t activation, uint32_t k)
+{
+    if (n >= 131072) return batch > 64;
+    const double products = (double)batch * k_dim * n;
+    return activation == DSX_ACT_SIGMOID && screen_takes(batch, k_dim, n, true) &&
+           ((k <= 32 && batch >= 1536 && products >= 2e10) || (k <= 128 && batch >= 2048 && products >= 1e11));
+}
+
 int dsx_fc_topk_supported(uint32_t ldx, const float* X, uint32_t activation, const dsx_act_params* params, const float* filter_mul)
 {
     return layer_activation_supported(activation, params) && filter_mul == nullptr && ((uintptr_t)X % 16) == 0 && (ldx % 4) == 0;

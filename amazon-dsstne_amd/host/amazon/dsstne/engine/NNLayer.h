@@ -92,6 +92,8 @@ private:
     unique_ptr<GpuBuffer<uint32_t>> _pbSplitInput;
     bool _bSplitInputFresh = false;   // the layer before this one wrote the planes of the current batch itself (dsx_fc_forward_planes)
     void* SplitInputBuffer();         // this lane's buffer for them, allocated on first use
+    // Whether the deferred layer and a top-K of k entries are computed in one call (or the layer is stored first).
+    bool TopKFusionPays(uint32_t batch, uint32_t k);
     bool UseSplitProducts(uint32_t batch) const
     {
         if (!_bSplitProducts || _vIncomingLayer.empty()) return false;

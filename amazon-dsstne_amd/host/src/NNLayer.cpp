@@ -134,15 +134,18 @@ void NNLayer::ForwardPropagate(uint32_t position, uint32_t batch, bool bTraining
 
 // Narrower layers are cheap to scan in full.
 static const uint32_t kSegMaxMinWidth = 8192;
-// From this width on the output layer is not stored but computed together with its top-K.  What the GEMM kernel's epilogue
-// then does per 32 x 32 block depends on how many scores of the block reach the row's running k-th score: about
-// 1024 * (k / columns seen so far + the filter's density).  In a 27,278-wide catalogue with top-10 and 144 own items per sample
-// that is ten per block, every block takes the slow path and the fused call is no faster than storing the layer (measured:
-// 95 us against 76 us for the GEMM alone); in a 1,000,000-wide one it is one block in three, and 16 GB of stores and loads go away.
+// Whether the output layer is computed together with its top-K and not stored: dsx_fc_topk_pays, and with split products from this
+// width on.  What the GEMM kernel's epilogue does per 32 x 32 block depends on how many scores of the block reach the row's running
+// k-th score: about 1024 * (k / columns seen so far + the filter's density).  In a 27,278-wide catalogue with top-10 and 144 own
+// items per sample that is ten per block and every block takes the slow path; in a 1,000,000-wide one it is one block in three, and
+// 16 GB of stores and loads go away.
 static const uint32_t kDeferMinWidth = 131072;
-// A batch of few rows is bound by reading the layer's weights once; storing its scores and maxima adds little to that, and the
-// fused call's tiles of 128 rows a lot (8 x 256 x 500,000, top 50: 440 us fused, 135 stored).
-static const uint32_t kDeferMinBatch = 65;
+
+bool NNLayer::TopKFusionPays(uint32_t batch, uint32_t k)
+{
+    if (_localStride < kDeferMinWidth && UseSplitProducts(batch)) return false;
+    return dsx_fc_topk_pays(batch, _vIncomingLayer[0]->_stride, _localStride, (uint32_t)_activation, k) != 0;
+}
 
 void NNLayer::ForwardPropagateFullyConnected(uint32_t position, uint32_t batch, bool bTraining)
 {
@@ -170,7 +173,7 @@ void NNLayer::ForwardPropagateFullyConnected(uint32_t position, uint32_t batch, 
         } else if (_kind == Output && _localStride >= kSegMaxMinWidth) {
             // Wide output layer that feeds no other layer: what usually follows is a top-K, which can run together with the layer
             // without the layer's result ever being stored.  The layer is computed when somebody asks for it.
-            if (_bDeferOutput && _localStride >= kDeferMinWidth && batch >= kDeferMinBatch && !w->_bTransposed && _vOutgoingLayer.empty() && _vOutgoingSkip.empty() &&
+            if (_bDeferOutput && TopKFusionPays(batch, 1) && !w->_bTransposed && _vOutgoingLayer.empty() && _vOutgoingSkip.empty() &&
                 dsx_fc_topk_supported(src->_stride, src->GetUnitBuffer(), (uint32_t)_activation, &params, NULL)) {
                 if (dsx_fc_topk_flagged_for(wsrc->_pbWeight->_pDevData, 0)) {
                     // rows whose survivor lists filled up had to be recomputed one by one: this data (thousands of scores tied at the

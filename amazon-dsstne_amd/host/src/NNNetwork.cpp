@@ -383,6 +383,7 @@ void NNNetwork::CalculateTopK(const string& layer, uint32_t k, GpuBuffer<NNFloat
     }
     uint32_t batch = _batch;
     if (_position + batch > _examples) batch = _examples - _position;
+    if (pLayer->_deferred && !pLayer->TopKFusionPays(batch, k)) pLayer->Materialise();
     if (pLayer->_deferred)
         LayerWithTopK(pLayer, k, batch, NULL, NULL, NULL, NULL, pbKey->_pDevData, pbValue->_pDevData);
     else if (pLayer->_segWidth != 0 && pLayer->_pbSegMax)
@@ -425,12 +426,12 @@ void NNNetwork::CalculateFilteredTopK(const string& layer, uint32_t k, NNDataSet
     pFilter->NoteSparseRead();
     const uint32_t* pIndex = (pFilter->_attributes & NNDataSetEnums::Indexed) ? pFilter->_pbIndex->_pDevData : NULL;
     if (pLayer->_deferred) {
-        if (pMul == NULL) {
+        if (pMul == NULL && pLayer->TopKFusionPays(batch, k)) {
             LayerWithTopK(pLayer, k, batch, pIndex, pFilter->_pbSparseStart->_pDevData, pFilter->_pbSparseEnd->_pDevData,
                           pFilter->_pbSparseIndex->_pDevData, pbKey->_pDevData, pbValue->_pDevData);
             return;
         }
-        pLayer->Materialise();   // multipliers other than 0 need the listed items' scores
+        pLayer->Materialise();   // (multipliers other than 0 need the listed items' scores)
     }
     // with segment maxima of the current batch (left by the layer's dense kernel) only the segments that can hold a result are read
     const NNFloat* pSegMax = (pLayer->_segWidth != 0 && pLayer->_pbSegMax) ? pLayer->_pbSegMax->_pDevData : NULL;
@@ -456,7 +457,7 @@ void NNNetwork::CalculateFilteredTopK(const string& layer, uint32_t k, const uin
     uint32_t batch = _batch;
     if (_position + batch > _examples) batch = _examples - _position;
     if (pLayer->_deferred) {
-        if (pFilterMul == NULL) {
+        if (pFilterMul == NULL && pLayer->TopKFusionPays(batch, k)) {
             LayerWithTopK(pLayer, k, batch, NULL, pFilterStart, pFilterEnd, pFilterIndex, pKey, pValue);
             return;
         }

@@ -322,6 +322,8 @@ int dsx_fc_topk_split(const float* X, uint32_t ldx, const float* W, const void* 
                       uint32_t batch, uint32_t k_dim, uint32_t n, uint32_t activation, const dsx_act_params* params, uint32_t k, float* keys,
                       uint32_t* values, uint32_t position, const uint32_t* index, const uint64_t* filter_start, const uint64_t* filter_end,
                       const uint32_t* filter_index);
+/* 1 where dsx_fc_topk is the faster way to the top-K, 0 where dsx_fc_forward_segmax + dsx_topk_guided are. */
+int dsx_fc_topk_pays(uint32_t batch, uint32_t k_dim, uint32_t n, uint32_t activation, uint32_t k);
 int dsx_fc_topk_supported(uint32_t ldx, const float* X, uint32_t activation, const dsx_act_params* params, const float* filter_mul);
 /* 1 if any row of any dsx_fc_topk call so far had to be recomputed (reset != 0 clears the mark); dsx_fc_topk_flagged_for: the
  * same for the calls with this weight matrix only (the mark is kept per W pointer, for the 64 matrices used last). */
