@@ -129,3 +129,34 @@ def test_knn_few_queries(pkg, dsx, orc, rng, items, queries, dim, k):
     q = rng.integers(-3, 4, size=(queries, dim)).astype(np.float32)
     got_s, got_i, ref_s, ref_i, _ = knn_case(pkg, dsx, orc, it, q, k)
     assert np.array_equal(got_s, ref_s) and np.array_equal(got_i, ref_i)
+
+
+@pytest.mark.parametrize("items,most,fewer", [(500, 129, (128, 127, 64, 3)), (5000, 65, (64, 33, 1)), (20000, 43, (42, 7))])
+@pytest.mark.parametrize("storage", ["fp32", "fp16", "split"])
+def test_knn_workspace_of_a_batch_holds_smaller_ones(pkg, dsx, orc, rng, items, most, fewer, storage):
+    """Fewer queries leave more lists each, which must not need more than a workspace sized for the whole batch."""
+    dim, k = 24, 100
+    rows = (items + 7) // 8 * 8
+    suffix = "" if storage == "fp32" else "_f16" if storage == "fp16" else "_split"
+    it = rng.integers(-3, 4, size=(items, dim)).astype(np.float32)
+    cm = np.full((dim, rows), 50.0, dtype=np.float32)
+    cm[:, :items] = it.T
+    table = dev(pkg, cm)
+    if storage == "fp16":
+        made = pkg.DeviceArray((dsx.dsx_knn_f16_table_bytes(rows, dim),), np.uint8)
+        pkg.check(dsx.dsx_knn_f16_convert_items(table.ptr, rows, rows - items, dim, made.ptr))
+    elif storage == "split":
+        made = pkg.DeviceArray((dsx.dsx_fc_split_bytes(rows, dim),), np.uint8)
+        pkg.check(dsx.dsx_fc_split(table.ptr, rows, 1, rows, dim, made.ptr))
+    else:
+        made = table
+    room = getattr(dsx, "dsx_knn_workspace_bytes" + suffix)(rows, dim, most, k)
+    workspace = pkg.DeviceArray((room,), np.uint8)
+    for queries in (most,) + fewer:
+        print("[case] knn workspace items=%d most=%d queries=%d %s" % (items, most, queries, storage), flush=True)
+        q = rng.integers(-3, 4, size=(queries, dim)).astype(np.float32)
+        dq, scores, idx = dev(pkg, q), pkg.DeviceArray((queries, k), np.float32), pkg.DeviceArray((queries, k), np.uint32)
+        pkg.check(getattr(dsx, "dsx_knn_search" + suffix)(made.ptr, rows, rows - items, dim, dq.ptr, queries, k, scores.ptr, idx.ptr,
+                                                          workspace.ptr, room, None))
+        rs, ri = orc.knn_search(cm, rows, rows - items, dim, q, k)
+        assert np.array_equal(scores.numpy(), rs) and np.array_equal(idx.numpy(), ri)
