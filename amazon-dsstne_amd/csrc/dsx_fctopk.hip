@@ -202,10 +202,15 @@ static int fc_topk_common(const float* X, uint32_t ldx, const float* W, const fl
     const uint32_t cap = ctx().knobs.fc_topk_candidate_capacity ? ctx().knobs.fc_topk_candidate_capacity : kLayerCandCap;   // tests lower it to reach the overflow path with small inputs
     const uint32_t n0 = layer_first_columns(n, k);
     const bool ranges = n0 < n;
-    const bool screened = ranges && !x_planes && screen_takes(batch, kdim, n, true);
-    const size_t need = layer_layout(nullptr, batch, n0, k, cap, ranges, screened, kdim, n).bytes;
+    bool screened = ranges && !x_planes && screen_takes(batch, kdim, n, true);
     LibScratch& ws = g_layer_ws_of[current_lane()];
-    if (int rc = lib_scratch_reserve(ws, need, "dsx_fc_topk workspace")) return rc;
+    int reserved = lib_scratch_reserve(ws, layer_layout(nullptr, batch, n0, k, cap, ranges, screened, kdim, n).bytes, "dsx_fc_topk workspace");
+    if (reserved == DSX_ENOMEM && screened) {   // the 16-bit copies (up to 8 GiB) do not fit beside what is there: fp32 ranges need none
+        (void)hipGetLastError();
+        screened = false;
+        reserved = lib_scratch_reserve(ws, layer_layout(nullptr, batch, n0, k, cap, ranges, screened, kdim, n).bytes, "dsx_fc_topk workspace");
+    }
+    if (reserved) return reserved;
     const LayerWorkspace w = layer_layout(ws.ptr, batch, n0, k, cap, ranges, screened, kdim, n);
     const uint32_t ld0 = (n0 + 3) / 4 * 4;
     hipStream_t s = ctx().stream;

@@ -71,7 +71,7 @@ static uint32_t knn_block_lists(uint32_t num_queries, uint32_t ncols, uint32_t k
 }
 
 static KnnWorkspace knn_layout(void* base, uint32_t rows_padded, uint32_t num_queries, uint32_t k, bool f16 = false, uint32_t dim = 0,
-                               bool split = false)
+                               bool split = false, bool screen = true)
 {
     const uint32_t cb = knn_block_columns(rows_padded, num_queries);
     const uint32_t blocks = (rows_padded + cb - 1) / cb;
@@ -103,7 +103,7 @@ static KnnWorkspace knn_layout(void* base, uint32_t rows_padded, uint32_t num_qu
     }
     if (split) p += align256((size_t)split_plane_bytes(num_queries, dim));
     w.screen = ScreenWorkspace{};
-    if (!f16 && !split && screen_takes(num_queries, dim, rows_padded, false)) {
+    if (screen && !f16 && !split && screen_takes(num_queries, dim, rows_padded, false)) {
         w.screen = screen_layout(p, num_queries, dim, rows_padded, false, kCandCap);
         p += w.screen.bytes;
     }
@@ -339,15 +339,23 @@ static int knn_search_common(KnnOperands& op, uint32_t padding, uint32_t num_que
                              size_t workspace_bytes, float* elapsed_ms, bool aligned, const float* queries_f32)
 {
     const size_t need = knn_layout(nullptr, op.rows_padded, num_queries, k, op.f16, op.dim, op.split).bytes;
+    bool screen = true;
     if (workspace) {
         DSX_CHECK_ARG(workspace_bytes >= need, "dsx_knn_search: workspace of %zu bytes, %zu needed", workspace_bytes, need);
         DSX_CHECK_ARG(((uintptr_t)workspace % 256) == 0, "dsx_knn_search: workspace is not 256-byte aligned");
     } else {
         LibScratch& ws = g_knn_ws_of[current_lane()];
-        if (int rc = lib_scratch_reserve(ws, need, "dsx_knn_search workspace")) return rc;
+        int reserved = lib_scratch_reserve(ws, need, "dsx_knn_search workspace");
+        if (reserved == DSX_ENOMEM) {   // the screening's copies of the table (up to 8 GiB) may be what does not fit: fp32 needs none
+            (void)hipGetLastError();
+            screen = false;
+            reserved = lib_scratch_reserve(ws, knn_layout(nullptr, op.rows_padded, num_queries, k, op.f16, op.dim, op.split, screen).bytes,
+                                           "dsx_knn_search workspace");
+        }
+        if (reserved) return reserved;
         workspace = ws.ptr;
     }
-    const KnnWorkspace w = knn_layout(workspace, op.rows_padded, num_queries, k, op.f16, op.dim, op.split);
+    const KnnWorkspace w = knn_layout(workspace, op.rows_padded, num_queries, k, op.f16, op.dim, op.split, screen);
     const uint32_t M = op.rows_padded - padding;
     hipStream_t s = ctx().stream;
     KnnTimer t;
