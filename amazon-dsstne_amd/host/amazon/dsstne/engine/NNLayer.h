@@ -107,6 +107,8 @@ private:
     bool _deferred = false;
     uint32_t _deferredBatch = 0;
     void Materialise();
+    bool _bHandedOut = false;     // NNNetwork::GetUnitBuffer was called for this layer: its units may change at any time
+    void SettleConsumers();       // before this layer's units change: computes deferred layers that are fed by them
     void SwitchLane(uint32_t lane)
     {
         if (lane == _currentLane) return;

@@ -24,6 +24,9 @@ private:
     Transform _transform;
     bool _bLocked;
     NNWeight* _pSharedWeight;
+    vector<NNWeight*> _vSharing;    // the connections that use this one's matrix
+    bool _bHandedOut = false;       // GetWeightBuffer was called: the matrix may change at any time
+    void SettleUnits();             // before the matrix or the biases change
     uint32_t _sharingCount;
     uint32_t _dimensionality;
     uint64_t _width;              // output units
@@ -51,7 +54,7 @@ private:
     NNWeight(NNLayer& inputLayer, NNLayer& outputLayer, bool bShared = false, bool bTransposed = false, bool bLocked = false,
              NNFloat maxNorm = 0.0f);
     ~NNWeight();
-    NNFloat* GetWeightBuffer() { return _pbWeight ? _pbWeight->_pDevData : NULL; }
+    NNFloat* GetWeightBuffer();
     // Starting values by the output layer's scheme (engine/NNWeight.cpp:500-561); biases start at biasInit.
     void Randomize();
     uint64_t GetBufferSize() { return _localSize; }

@@ -173,7 +173,9 @@ void NNLayer::ForwardPropagateFullyConnected(uint32_t position, uint32_t batch, 
         } else if (_kind == Output && _localStride >= kSegMaxMinWidth) {
             // Wide output layer that feeds no other layer: what usually follows is a top-K, which can run together with the layer
             // without the layer's result ever being stored.  The layer is computed when somebody asks for it.
-            if (_bDeferOutput && TopKFusionPays(batch, 1) && !w->_bTransposed && _vOutgoingLayer.empty() && _vOutgoingSkip.empty() &&
+            // (a narrower one is not put off while a caller holds a pointer through which its operands may change meanwhile)
+            const bool bHeld = _localStride < kDeferMinWidth && (src->_bHandedOut || wsrc->_bHandedOut);
+            if (_bDeferOutput && !bHeld && TopKFusionPays(batch, 1) && !w->_bTransposed && _vOutgoingLayer.empty() && _vOutgoingSkip.empty() &&
                 dsx_fc_topk_supported(src->_stride, src->GetUnitBuffer(), (uint32_t)_activation, &params, NULL)) {
                 if (dsx_fc_topk_flagged_for(wsrc->_pbWeight->_pDevData, 0)) {
                     // rows whose survivor lists filled up had to be recomputed one by one: this data (thousands of scores tied at the
@@ -245,6 +247,12 @@ void NNLayer::Materialise()
                                    w->_pbBias->_pDevData, GetIncomingUnitBuffer(), _stride, _deferredBatch, src->_stride, _localStride,
                                    (uint32_t)_activation, &params, _pbSegMax->_pDevData, &_segWidth),
              "NNLayer::ForwardPropagate: GEMM failure");
+}
+
+void NNLayer::SettleConsumers()
+{
+    for (auto l : _vOutgoingLayer)
+        if (l->_deferred) l->Materialise();
 }
 
 void NNLayer::ForwardSplit(uint32_t batch, NNFloat* pSegMax, uint32_t* pSegWidth)
@@ -334,6 +342,7 @@ bool NNLayer::SetUnits(const vector<NNFloat>& vUnit)
         printf("NNLayer::SetUnits: Input unit data too small to set all units.\n");
         return false;
     }
+    SettleConsumers();
     _pbUnit->Upload(vUnit.data());
     _segWidth = 0;
     _deferred = false;

@@ -123,6 +123,7 @@ NNNetwork::NNNetwork(NNNetworkDescriptor& d, uint32_t batch)
                       pWeight->_inputLayer._name.c_str(), pWeight->_outputLayer._name.c_str());
             }
             pWeight->_pSharedWeight = c;
+            c->_vSharing.push_back(pWeight);
             if (c->_sharingCount == 1) _vSharedWeight.push_back(c);
             c->_sharingCount++;
             bFound = true;
@@ -541,6 +542,8 @@ NNFloat* NNNetwork::GetUnitBuffer(const string& layer)
         return NULL;
     }
     if (itr->second->_deferred) itr->second->Materialise();
+    itr->second->SettleConsumers();
+    itr->second->_bHandedOut = true;
     // the caller gets a writable device pointer: the segment maxima of the batch may not describe the units any longer
     itr->second->_segWidth = 0;
     // The reference's callers follow this call with a plain cudaMemcpy or a kernel of their own

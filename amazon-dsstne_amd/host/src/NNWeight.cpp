@@ -78,6 +78,7 @@ struct WeightStream {
 
 void NNWeight::Randomize()
 {
+    SettleUnits();
     if (!_bShared) {
         const WeightStream rng(getGpu()._randomSeed, _inputLayer._name, _outputLayer._name);
         const NNFloat s = _outputLayer._weightInitScale;
@@ -127,6 +128,22 @@ void NNWeight::Randomize()
     _pbBias->Upload(_vBias.data());
 }
 
+// Units that the forward pass has put off belong to the weights it ran with: they are computed before those change.
+void NNWeight::SettleUnits()
+{
+    if (_outputLayer._deferred) _outputLayer.Materialise();
+    for (auto w : _vSharing)
+        if (w->_outputLayer._deferred) w->_outputLayer.Materialise();
+}
+
+NNFloat* NNWeight::GetWeightBuffer()
+{
+    if (!_pbWeight) return NULL;
+    SettleUnits();
+    _bHandedOut = true;
+    return _pbWeight->_pDevData;
+}
+
 bool NNWeight::CopyWeights(const NNWeight* pSrcWeight)
 {
     NNWeight* pDstWeight = _bShared ? _pSharedWeight : this;
@@ -139,6 +156,8 @@ bool NNWeight::CopyWeights(const NNWeight* pSrcWeight)
         printf("NNWeight::CopyWeights: Mismatched weight dimensions.\n");
         return false;
     }
+    SettleUnits();
+    if (pDstWeight != this) pDstWeight->SettleUnits();
     pDstWeight->_vWeight = pSrc->_vWeight;
     _vBias = pSrcWeight->_vBias;
     if (pDstWeight->_pbWeight) pDstWeight->_pbWeight->Upload(pDstWeight->_vWeight.data());
@@ -154,6 +173,8 @@ bool NNWeight::SetWeights(const vector<NNFloat>& vWeight)
         printf("NNWeight::SetWeights: Input vector smaller than weight vector.\n");
         return false;
     }
+    SettleUnits();
+    if (pWeight != this) pWeight->SettleUnits();
     std::copy(vWeight.begin(), vWeight.begin() + pWeight->_vWeight.size(), pWeight->_vWeight.begin());
     if (pWeight->_pbWeight) pWeight->_pbWeight->Upload(pWeight->_vWeight.data());
     pWeight->InvalidateSplit();
@@ -183,6 +204,7 @@ bool NNWeight::SetBiases(const vector<NNFloat>& vBias)
         printf("NNWeight::SetBiases: Input vector smaller than bias vector.\n");
         return false;
     }
+    SettleUnits();
     std::copy(vBias.begin(), vBias.begin() + _vBias.size(), _vBias.begin());
     if (_pbBias) _pbBias->Upload(_vBias.data());
     return true;

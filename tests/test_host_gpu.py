@@ -582,3 +582,41 @@ def test_wide_output_layer_is_deferred_and_materialised_on_demand(pkg, dsx, orc,
         assert dsx.dsx_fc_topk_flagged(0) == 0
     finally:
         net.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("change", ["weights", "biases", "hidden units"])
+def test_layer_put_off_for_the_top_k_is_of_the_operands_it_was_predicted_with(pkg, dsx, synth, change):
+    """An output layer that PredictBatch leaves to the top-K (16-bit screening pays here) is computed before its weights, biases or inputs
+    change; the next batch sees the new ones."""
+    from amazon_dsstne_amd import host_api
+    p = synth.autoencoder("put-off", 77, 16500, [1024], 1536, 10, zipf_s=1.0, nnz_mean=20, nnz_sigma=0.5, nnz_clip=(1, 200))
+    assert dsx.dsx_fc_topk_pays(p.batch, 1024, 16500, 0, p.k) == 1
+    net = host_api.Network(p, max_k=p.k)
+    try:
+        net.bind_input()
+        got = {}
+        for deferred in (True, False):
+            net.set_deferred_output(deferred)
+            net.set_weights("Hidden1", "Output", weights=p.weights[1], biases=p.biases[1])
+            net.predict_batch(0)
+            if change == "weights":
+                net.set_weights("Hidden1", "Output", weights=-p.weights[1])
+            elif change == "biases":
+                net.set_weights("Hidden1", "Output", biases=np.linspace(-2, 2, 16500, dtype=np.float32))
+            else:
+                net.set_units(np.ones((p.batch, 1024), np.float32), "Hidden1")
+            net.topk(p.k)
+            before = net.get_topk(p.batch)
+            if change != "hidden units":
+                net.predict_batch(0)
+            net.topk(p.k)
+            got[deferred] = before + net.get_topk(p.batch)
+        for a, b in zip(got[True][::2], got[False][::2]):
+            # sums of 1,024 products below 1 in another order: 1e-5 is far above their roundings; a change that leaks in moves scores by 1e-2 and more
+            assert np.abs(a - b).max() < 1e-5
+        assert (got[True][1] == got[False][1]).mean() > 0.99
+        if change != "hidden units":
+            assert (got[True][1] == got[True][3]).mean() < 0.5
+    finally:
+        net.close()
