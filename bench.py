@@ -26,6 +26,7 @@ import __graft_entry__ as entry  # noqa: E402
 HBM_PEAK_GBS = 8000.0        # MI355X HBM3E, published
 FP32_MFMA_PEAK_TF = 157.3    # MI355X dense fp32 matrix, published
 BF16_MFMA_PEAK_TF = 2500.0       # dense bf16 MFMA, the published figure
+F16_MFMA_PEAK_TF = 2500.0        # dense f16 MFMA, the same
 
 # HBM bytes per launch, measured: profiles/pmc_hbm_traffic.json holds, per workload and kernel, what rocprofv3 --pmc FETCH_SIZE and
 # WRITE_SIZE read (KiB per dispatch) and the calibration factors from a plain 256 MiB device-to-device copy in the same runs; the
@@ -370,7 +371,7 @@ def network_bench(args, pkg, lib):
             g.update({"achieved": (moved["read"] + moved["write"]) / ms / 1e6, "peak": HBM_PEAK_GBS, "unit": "GB/s"})
             g["frac"] = g["achieved"] / g["peak"]
         kernels["topk_guided_kernel"] = g
-    deferred = N >= 131072      # NNLayer defers output layers from this width on
+    deferred = bool(lib.dsx_fc_topk_pays(B, p.widths[last], N, p.acts[last], K))      # as NNLayer decides
     if deferred:
         keys = pkg.DeviceArray((B, K), np.float32)
         vals = pkg.DeviceArray((B, K), np.uint32)
@@ -382,9 +383,9 @@ def network_bench(args, pkg, lib):
         flops = 2.0 * B * p.widths[last] * N
         ms = time_launches(pkg, lib, k_fused, max(5, reps // 4))
         kernels["dsx_fc_topk (output layer + filtered top-K, nothing stored)"] = {
-            "bound": "mfma", "ms": ms, "achieved": flops / ms / 1e9, "peak": FP32_MFMA_PEAK_TF, "unit": "TFLOP/s",
-            "algorithmic_flops": flops, "frac": flops / ms / 1e9 / FP32_MFMA_PEAK_TF,
-            "note": "what the timed step runs for this layer: first column block stored and scanned, the rest compared in registers"}
+            "bound": "mfma", "ms": ms, "achieved": flops / ms / 1e9, "peak": F16_MFMA_PEAK_TF, "unit": "TFLOP/s",
+            "algorithmic_flops": flops, "frac": flops / ms / 1e9 / F16_MFMA_PEAK_TF,
+            "note": "what the timed step runs for this layer: first column block stored and scanned, the rest screened in f16 and what passes scored in fp32; priced against the f16 peak"}
 
     # The output layer's kernel of the split-products mode (off by default, so never the dominant kernel of `roofline`): priced as the
     # bf16 matrix work it executes, six products per fp32 product, against the bf16 peak.
@@ -421,6 +422,7 @@ def network_bench(args, pkg, lib):
     candidates = [n for n in kernels if "frac" in kernels[n] and n != split_name and not (deferred and n in (gemm_name, "topk_scan_kernel"))]
     dominant = max(candidates, key=lambda n: kernels[n]["ms"])
     d = kernels[dominant]
+    step_peak = F16_MFMA_PEAK_TF if deferred else FP32_MFMA_PEAK_TF
     roofline = {"kernel": dominant, "bound": d["bound"], "achieved": round(d["achieved"], 3), "peak": d["peak"], "unit": d["unit"],
                 "frac": round(d["frac"], 4), "traffic": d.get("traffic"), "avg_launch_ms": round(d["ms"], 5),
                 "note": "isolated back-to-back launches, clocks settled; `pipeline` below prices the whole timed step"}
@@ -473,9 +475,9 @@ def network_bench(args, pkg, lib):
                     "min": round(min(windows), 5), "median": round(ms_step, 5), "max": round(max(windows), 5),
                     "note": "value is the median window; the timed steps cycle over the resident batches"},
         "roofline": roofline,
-        "pipeline": {"gemm_flops_per_step": flops_step, "achieved": round(flops_step / ms_step / 1e9, 3), "peak": FP32_MFMA_PEAK_TF,
-                     "unit": "TFLOP/s", "frac": round(flops_step / ms_step / 1e9 / FP32_MFMA_PEAK_TF, 4),
-                     "note": "all dense-layer flops of a step over the timed step itself (every kernel of the step included, batches on %d lanes)" % args.lanes + ": the fraction of the fp32 MFMA peak the whole path sustains"},
+        "pipeline": {"gemm_flops_per_step": flops_step, "achieved": round(flops_step / ms_step / 1e9, 3), "peak": step_peak,
+                     "unit": "TFLOP/s", "frac": round(flops_step / ms_step / 1e9 / step_peak, 4),
+                     "note": "all dense-layer flops of a step over the timed step itself (every kernel of the step included, batches on %d lanes)" % args.lanes + ": the fraction of the %s MFMA peak the whole path sustains" % ("f16 (the output layer is screened in it; its other layers are fp32)" if deferred else "fp32")},
         "kernels": {n: {k: (round(v, 5) if isinstance(v, float) else v) for k, v in kv.items()} for n, kv in kernels.items()},
         "cpu_baseline": cpu,
         "clock_settle_ms": SETTLE_SECONDS * 1e3,
@@ -522,9 +524,8 @@ def knn_bench(args, pkg, lib):
     ms_step = (time.perf_counter() - t0) * 1e3 / args.steps
     step(el)
     flops = 2.0 * Q * D * (rows - pad)
-    roofline = {"kernel": "fc_gemm_kernel (knn scores)", "bound": "mfma", "achieved": round(flops / el[0] / 1e9, 3), "peak": FP32_MFMA_PEAK_TF,
-                "unit": "TFLOP/s", "frac": round(flops / el[0] / 1e9 / FP32_MFMA_PEAK_TF, 4), "traffic": (lambda t: (t["read"] + t["write"]) if t else None)(
-                    measured_traffic(p.name).get("fc_gemm_kernel (knn scores)")), "avg_launch_ms": round(el[0], 4),
+    roofline = {"kernel": "f16 screening + fp32 scores of the candidates (knn)", "bound": "mfma", "achieved": round(flops / el[0] / 1e9, 3), "peak": F16_MFMA_PEAK_TF,
+                "unit": "TFLOP/s", "frac": round(flops / el[0] / 1e9 / F16_MFMA_PEAK_TF, 4), "traffic": None, "avg_launch_ms": round(el[0], 4),
                 "topk_ms": round(el[1], 4),
                 "path": {0: "blocks", 1: "candidate lists", 2: "candidate lists, redone block by block"}[lib.dsx_knn_last_search_path()]}
     # the same search with fp16 storage of items and queries (the reference's DataType::FP16): reported beside the fp32 figure
