@@ -7,7 +7,8 @@
 //
 // Error of a screened sum s' = sum x'_i w'_i against the fp32 sum s of the same row and column, x', w' rounded to f16 (unit
 // roundoff u = 2^-11, 2^-25 absolute below the normal range), fp32 accumulation:
-//   |s' - s| <= (2u + u^2) |x| |w| + 2^-25 sqrt(d) (|x| + |w|) + (3 d + 16) 2^-24 |x| |w|      (Cauchy-Schwarz; |.| = 2-norm)
+//   |s' - s| <= (2u + u^2) |x| |w| + 2^-25 sqrt(d) (|x| + |w|) + d 2^-50 + (3 d + 16) 2^-24 |x| |w|      (Cauchy-Schwarz; |.| = 2-norm)
+// (d 2^-50: both operands' absolute roundings together, all there is to go by where every component is near 2^-25)
 // The matrix instructions keep subnormal operands.  Norms above 65,504 (a component might overflow) set a flag instead.
 //
 //   ITEM_NORM = false (nearest neighbours): |w| is taken at its largest over all columns; the search reads the flag and, where lists
@@ -151,7 +152,7 @@ __global__ __launch_bounds__(256) void screen_rows_kernel(ScreenRowsArgs a)
     const float most = __uint_as_float(a.stats[0]), bias = ITEM_NORM ? __uint_as_float(a.stats[1]) : 0.0f;
     float eps = 2.9802322e-8f * 1.01f * sqrtf((float)a.dim + 4.0f) * (norm + most);
     if constexpr (ITEM_NORM) eps += ((float)a.dim + 64.0f) * 2.3841858e-7f * bias + 1e-6f * bias + 1e-7f;
-    else eps += screen_relative(a.dim) * norm * most;
+    else eps += screen_relative(a.dim) * norm * most + (float)a.dim * 8.8817842e-16f * 1.01f;   // (a layer's 1e-7 covers the last term)
     a.eps[row] = eps;
     // (a NaN in the row: its scores are NaN everywhere, there is nothing to miss)
     const bool bad = norm > kF16Max || most > kF16Max || bias > kF16Max;

@@ -75,6 +75,24 @@ def test_operands_that_f16_holds_badly(pkg, dsx, rng, form):
     check_against_float64(s / scale, i, full / scale, k, dim * 2.0 ** -24)
 
 
+@pytest.mark.parametrize("dim", [32, 128, 1024])
+def test_components_at_half_the_smallest_subnormal(pkg, dsx, rng, dim):
+    """Components a little above 2^-25 round up to 2^-24 in both operands: a screened sum is four times the score, and below any bound
+    that leaves out the product of the two roundings.  The best items lie behind the first block."""
+    n, queries, k = 66000, 512, 20
+    print("[case] screened knn tiny components dim=%d" % dim, flush=True)
+    c = rng.uniform(1.05, 1.2, n).astype(np.float32)
+    c[60000:60000 + 3 * k] = np.float32(1.0001) + np.arange(3 * k, dtype=np.float32) * np.float32(5e-4)
+    items = np.repeat(-c[:, None] * np.float32(2.0 ** -25), dim, axis=1)
+    q = np.full((queries, dim), 1.0001 * 2.0 ** -25, dtype=np.float32)
+    s, i = search(pkg, dsx, items, q, k)
+    full = np.repeat(q[:1].astype(np.float64) @ items.astype(np.float64).T, queries, axis=0)
+    unit = dim * (1.0001 * 2.0 ** -25) ** 2
+    # every score a sum of dim equal products: dim roundings of 2^-24 of it at most, and neighbours lie 5e-4 apart
+    check_against_float64(s / unit, i, full / unit, k, dim * 2.0 ** -24 * 1.2)
+    assert (i == 60000 + np.arange(k)).all()
+
+
 # activations with and without a flat part; columns whose norms span four orders; a bias; a filter; both sides of the padding
 @pytest.mark.parametrize("batch,kdim,n,k,act,biased,filtered", [(4096, 32, 16384, 10, 0, True, True), (2200, 60, 17003, 100, 3, True, False),
                                                                 (2050, 64, 20000, 256, 2, False, True), (520, 508, 70001, 20, 1, True, True)])
