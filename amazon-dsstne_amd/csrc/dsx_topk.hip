@@ -855,7 +855,7 @@ __global__ __launch_bounds__(kTopkThreads, 4) void topk_block_kernel(TopKArgs a)
     __shared__ uint64_t sStage[kTopkWaves][List::kStageWords];
     __shared__ uint32_t sMax[R * kTopkThreads];
     __shared__ uint32_t sTaint[FILTERED ? kTopkThreads : 1];   // bit u: the lane's group u holds a listed column
-    __shared__ uint32_t sBound, sReach, sStaged;
+    __shared__ uint32_t sBound, sNeed, sReach, sStaged;
     extern __shared__ uint32_t sBitmap[];
     const uint32_t b = blockIdx.x, seg = blockIdx.y;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
@@ -937,14 +937,17 @@ __global__ __launch_bounds__(kTopkThreads, 4) void topk_block_kernel(TopKArgs a)
             for (int n = 0; n < 4 * R; n++) all[n] = sMax[n * kWave + lane];
             t = wave_kth_key<4 * R>(all, a.k);
         }
-        if (lane == 0) sBound = t;
+        if (lane == 0) {
+            sBound = t;
+            // a bound from the row's other columns (fewer than k words may pass it); read once: other workgroups of the row raise it
+            // meanwhile, and the counts below are taken by all wavefronts against one bound
+            sNeed = a.row_bound ? max(t, a.row_bound[b]) : t;
+        }
     }
     __syncthreads();
-    uint32_t t = sBound;
-    const uint32_t none = score_key(-__builtin_inff());
-    bool failed = t <= none;   // fewer than k maxima
-    if (FILTERED && t <= score_key(0.0f)) failed = true;   // listed columns score 0 and may belong in the result
-    if (a.row_bound) t = max(t, a.row_bound[b]);           // (a bound from earlier columns of the row: fewer than k words may pass)
+    const uint32_t own = sBound, t = sNeed;
+    bool failed = own <= score_key(-__builtin_inff());       // fewer than k maxima
+    if (FILTERED && own <= score_key(0.0f)) failed = true;   // listed columns score 0 and may belong in the result
     // Saturated activations have thousands of scores at exactly 1.0.  Among equal scores the lower column wins: when k of the
     // segment's first 1,024 columns reach the bound, later ones have to lie above it.
     const float bound = key_score(t);

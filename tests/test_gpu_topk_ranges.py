@@ -131,6 +131,18 @@ def test_knn_few_queries(pkg, dsx, orc, rng, items, queries, dim, k):
     assert np.array_equal(got_s, ref_s) and np.array_equal(got_i, ref_i)
 
 
+@pytest.mark.parametrize("items,queries,k", [(200000, 100, 200), (200000, 100, 129), (150001, 65, 100), (270011, 130, 256)])
+def test_knn_segments_of_a_row_that_share_its_bound(pkg, dsx, orc, rng, items, queries, k):
+    """Several workgroups per row raise one bound while their siblings read it, and thousands of items tie at every score: the order
+    among them (lower item first) may not depend on who reads when."""
+    print("[case] shared row bound items=%d queries=%d k=%d" % (items, queries, k), flush=True)
+    dim = 8
+    it = rng.integers(-1, 2, size=(items, dim)).astype(np.float32)
+    q = rng.integers(-1, 2, size=(queries, dim)).astype(np.float32)
+    got_s, got_i, ref_s, ref_i, _ = knn_case(pkg, dsx, orc, it, q, k)
+    assert np.array_equal(got_s, ref_s) and np.array_equal(got_i, ref_i)
+
+
 @pytest.mark.parametrize("items,most,fewer", [(500, 129, (128, 127, 64, 3)), (5000, 65, (64, 33, 1)), (20000, 43, (42, 7))])
 @pytest.mark.parametrize("storage", ["fp32", "fp16", "split"])
 def test_knn_workspace_of_a_batch_holds_smaller_ones(pkg, dsx, orc, rng, items, most, fewer, storage):
