@@ -7,6 +7,7 @@
 // 64 lanes of an MFMA operand read 2 x 32 consecutive floats.  Workgroup ids are remapped so that the workgroups that land
 // on one XCD (id mod 8) sweep all row tiles of a few column tiles: a W tile is then fetched by one L2 only.
 #include <type_traits>
+#include <algorithm>
 #include "dsx_device.h"
 #include "dsx_internal.h"
 
@@ -627,13 +628,14 @@ template <int MI, int NI, int BK> static void launch_fc_shape(FcArgs& a, int xv,
 
 int fc_run(const float* X, uint32_t ldx, const float* W, uint32_t ldw, int transposed, const float* bias, float* Z, uint32_t ldz,
            uint32_t batch, uint32_t k, uint32_t n, int accumulate, uint32_t activation, const dsx_act_params* params, float* seg_max,
-           uint32_t* seg_width, void* out_planes)
+           uint32_t* seg_width, void* out_planes, const FcOrder& order)
 {
     if (seg_width) *seg_width = 0;
-    const bool small = !transposed && !accumulate && ((uintptr_t)X % 16) == 0 && (ldx % 4) == 0 && (k == 128 || k == 256) &&
-                       (uint64_t)batch * n <= (1u << 20);   // the one-round-trip kernel's shapes
-    if (!(small && n < 4096) && fc_rows_takes(batch, k, n, ldx, ldw, transposed)) {
-        int rc = fc_rows_run(X, ldx, W, ldw, bias, Z, ldz, batch, k, n, accumulate, activation, params, seg_max, seg_width);
+    const uint32_t plan_n = std::max(n, order.plan_n);
+    const bool small = !order.as_candidates && !transposed && !accumulate && ((uintptr_t)X % 16) == 0 && (ldx % 4) == 0 && (k == 128 || k == 256) &&
+                       (uint64_t)batch * plan_n <= (1u << 20);   // the one-round-trip kernel's shapes
+    if (!order.as_candidates && !(small && plan_n < 4096) && fc_rows_takes(batch, k, plan_n, ldx, ldw, transposed)) {
+        int rc = fc_rows_run(X, ldx, W, ldw, bias, Z, ldz, batch, k, n, accumulate, activation, params, seg_max, seg_width, plan_n);
         if (rc == DSX_OK && out_planes) rc = fc_split_planes_run(Z, ldz, 1, batch, n, out_planes);
         return rc;
     }

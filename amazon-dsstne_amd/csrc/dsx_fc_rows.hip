@@ -281,9 +281,8 @@ constexpr uint32_t kRowsWide = 4096;   // from this width on a wavefront takes 1
 //   64 x 64 tiles are level or better (100 x 128 x 27,278: 19.1 / 17.1; 128 x 256 x 60,000: 48 / 42), and from 160 rows on always.
 //   narrow layers: while the 64 x 64 tiles leave more than half of the compute units without one (1 x 1,024 x 1,024: 8.0 / 32;
 //   256 x 1,024 x 1,024: 11 / 22; 256 x 300 x 300: 4.6 / 17); above that a tenth at most is to be had (512 x 1,024 x 1,024: 20.8 / 23,
-//   1,024 x 512 x 512: 12.1 / 12.7).  Sums of at most 32 products stay where they are: there is nothing to split (and the
-//   candidate searches get the same bits from a column whichever of their steps it falls into).  So do sums of more than 4,096:
-//   cut into sixteen they would be five times closer to the exact sums than those of the split-products mode, which is to be as
+//   1,024 x 512 x 512: 12.1 / 12.7).  Sums of at most 32 products stay where they are: there is nothing to split.  So do sums
+//   of more than 4,096: cut into sixteen they would be five times closer to the exact sums than those of the split-products mode, which is to be as
 //   close as this one.
 bool fc_rows_takes(uint32_t batch, uint32_t k, uint32_t n, uint32_t ldx, uint32_t ldw, int transposed)
 {
@@ -295,7 +294,7 @@ bool fc_rows_takes(uint32_t batch, uint32_t k, uint32_t n, uint32_t ldx, uint32_
 
 int fc_rows_run(const float* X, uint32_t ldx, const float* W, uint32_t ldw, const float* bias, float* Z, uint32_t ldz, uint32_t batch,
                 uint32_t k, uint32_t n, int accumulate, uint32_t activation, const dsx_act_params* params, float* seg_max,
-                uint32_t* seg_width)
+                uint32_t* seg_width, uint32_t plan_n)
 {
     FcRowsArgs a{};
     a.X = X; a.W = W; a.bias = bias; a.Z = Z;
@@ -307,7 +306,7 @@ int fc_rows_run(const float* X, uint32_t ldx, const float* W, uint32_t ldw, cons
     a.alpha = params ? params->alpha : 1.0f;
     a.lambda = params ? params->lambda : 1.0f;
     const uint64_t cus = (uint64_t)ctx().num_cus;
-    if (n >= kRowsWide) {
+    if (plan_n >= kRowsWide) {   // (how a sum is split depends on plan_n alone: column blocks of one product agree)
         if (seg_max && seg_width && !accumulate) {
             a.seg_max = seg_max;
             a.nseg = (n + 63) / 64;
@@ -316,7 +315,7 @@ int fc_rows_run(const float* X, uint32_t ldx, const float* W, uint32_t ldw, cons
         // Four wavefronts share a tile's k unless there are tiles enough to keep every SIMD busy without (8 x 256 x 500,000: 103 us
         // against 110; 8 x 512 x 27,278: 15.4 us with four, 16.1 with eight).  32 rows per wavefront where a second block would be
         // mostly padding.
-        const bool split = k > 32 && (n + 127) / 128 < 8 * cus;
+        const bool split = k > 32 && (plan_n + 127) / 128 < 8 * cus;
         if (((batch - 1) / 32) % 2 == 0) {
             if (split) launch_fc_rows<4, 1, 4>(a);
             else launch_fc_rows<4, 1, 1>(a);
@@ -327,7 +326,7 @@ int fc_rows_run(const float* X, uint32_t ldx, const float* W, uint32_t ldw, cons
     } else {
         // as many wavefronts per tile as the number of tiles asks for (us with 4, 8, 16: 200 x 512 x 2,000 12.4, 12.7, 13.2;
         // 64 x 1,024 x 1,024 -, 10.8, 11.1; 100 x 300 x 1,000 5.4, 4.9, 4.6; 1 x 1,024 x 1,024 -, 8.4, 8.0)
-        const uint64_t tiles = ((uint64_t)(batch + 31) / 32) * ((n + 31) / 32);
+        const uint64_t tiles = ((uint64_t)(batch + 31) / 32) * ((plan_n + 31) / 32);
         if (tiles >= 128) launch_fc_rows<1, 1, 4>(a);
         else if (tiles >= 64) launch_fc_rows<1, 1, 8>(a);
         else launch_fc_rows<1, 1, 16>(a);

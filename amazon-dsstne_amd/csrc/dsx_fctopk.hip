@@ -217,8 +217,10 @@ static int fc_topk_common(const float* X, uint32_t ldx, const float* W, const fl
 
     // first block: the layer as a matrix, then the scanning top-K (filtered: indexes beyond the block are ignored)
     const uint32_t wrows = split_rows_padded(n);
+    FcOrder order;
+    order.as_candidates = ranges && !screened;
     int rc = x_planes ? fc_split_run(x_planes, w_planes, wrows, 0, bias, w.block_scores, ld0, batch, kdim, n0, 0, activation, params, nullptr, nullptr)
-                      : fc_run(X, ldx, W, n, 0, bias, w.block_scores, ld0, batch, kdim, n0, 0, activation, params);
+                      : fc_run(X, ldx, W, n, 0, bias, w.block_scores, ld0, batch, kdim, n0, 0, activation, params, nullptr, nullptr, nullptr, order);
     if (rc) return rc;
     if (!ranges)
         return topk_run(w.block_scores, ld0, n0, batch, k, keys, values, position, index, filter_start, filter_end, filter_index, nullptr, 0,

@@ -109,15 +109,22 @@ int topk_guided_launch(const float* in, uint32_t pitch, uint32_t width, uint32_t
 // Workgroups per row that topk_run takes on its own (forced_segments = 0).
 uint32_t topk_segments(uint32_t batch, uint32_t width, bool filtered);
 int topk_merge(const uint64_t* partial, uint32_t slots, uint32_t k, float* keys, uint32_t* values, uint32_t batch);
+// What the sums of an fc_run have to agree with, bit for bit, so that equal columns score the same wherever they lie.  plan_n: the
+// other column blocks of the same product, of this width each (this one may be narrower).  as_candidates: the candidate modes below,
+// which add the products in ascending order of k (with a bias they start from it and not from 0).
+struct FcOrder {
+    uint32_t plan_n = 0;
+    bool as_candidates = false;
+};
 // GEMM building block shared with the KNN search (dsx_fc.hip): Z = X.W (+bias, activation), see dsx_fc_forward.
 int fc_run(const float* X, uint32_t ldx, const float* W, uint32_t ldw, int transposed, const float* bias, float* Z, uint32_t ldz,
            uint32_t batch, uint32_t k, uint32_t n, int accumulate, uint32_t activation, const dsx_act_params* params,
-           float* seg_max = nullptr, uint32_t* seg_width = nullptr, void* out_planes = nullptr);
+           float* seg_max = nullptr, uint32_t* seg_width = nullptr, void* out_planes = nullptr, const FcOrder& order = FcOrder());
 // The same for few rows or few output tiles (dsx_fc_rows.hip): whether that kernel is the one for a shape, and the launch.
 bool fc_rows_takes(uint32_t batch, uint32_t k, uint32_t n, uint32_t ldx, uint32_t ldw, int transposed);
 int fc_rows_run(const float* X, uint32_t ldx, const float* W, uint32_t ldw, const float* bias, float* Z, uint32_t ldz, uint32_t batch,
                 uint32_t k, uint32_t n, int accumulate, uint32_t activation, const dsx_act_params* params, float* seg_max,
-                uint32_t* seg_width);
+                uint32_t* seg_width, uint32_t plan_n);
 // Candidate mode of the same kernel (exact KNN): scores are compared with the rows' bounds and the survivors appended to
 // per-row lists as packed words (CandArgs); nothing else is written.  knn_refresh folds a row's candidates into its best
 // list.  The caller guarantees 16-byte aligned operands with pitches that are multiples of four floats.

@@ -134,14 +134,16 @@ struct KnnOperands {
     const void* queries16 = nullptr;
     uint32_t rows_padded = 0, dim = 0, ld16 = 0;
 
-    int into_matrix(uint32_t c0, uint32_t ncols, uint32_t num_queries, float* Z, uint32_t ldz, float* seg_max = nullptr,
+    // order: what the fp32 sums have to agree with (the other column blocks, or the candidate ranges behind this one)
+    int into_matrix(uint32_t c0, uint32_t ncols, uint32_t num_queries, float* Z, uint32_t ldz, const FcOrder& order, float* seg_max = nullptr,
                     uint32_t* seg_width = nullptr) const
     {
         if (f16) return knn_f16_scores_run(queries16, items16 + (uint64_t)c0 * ld16 * 2, ld16, num_queries, ncols, Z, ldz, nullptr);
         if (split)
             return fc_split_run(query_planes, item_planes, split_rows_padded(rows_padded), c0, nullptr, Z, ldz, num_queries, dim, ncols, 0,
                                 DSX_ACT_LINEAR, nullptr, nullptr, nullptr);
-        return fc_run(queries, dim, items + c0, rows_padded, 0, nullptr, Z, ldz, num_queries, dim, ncols, 0, DSX_ACT_LINEAR, nullptr, seg_max, seg_width);
+        return fc_run(queries, dim, items + c0, rows_padded, 0, nullptr, Z, ldz, num_queries, dim, ncols, 0, DSX_ACT_LINEAR, nullptr, seg_max, seg_width,
+                      nullptr, order);
     }
     // *chunks_used: how many (row, chunk) lists of seg the range filled besides the shared lists (0: none)
     int into_candidates(uint32_t c0, uint32_t ncols, uint32_t num_queries, const CandArgs& cand, uint64_t* seg, uint32_t* seg_count,
@@ -202,6 +204,8 @@ static int knn_search_blocks(const KnnWorkspace& w, const KnnOperands& op, uint3
     hipStream_t s = ctx().stream;
     const uint32_t cb = knn_block_columns(op.rows_padded, num_queries);
     const uint32_t blocks = (M + cb - 1) / cb;
+    FcOrder order;
+    order.plan_n = blocks > 1 ? cb : 0;
     const uint32_t lists_per_block = knn_block_lists(num_queries, cb, k);
     const uint32_t lists = (blocks - 1) * lists_per_block + knn_block_lists(num_queries, M - (blocks - 1) * cb, k);
     hipLaunchKernelGGL(knn_clear_kernel, dim3((num_queries + 255) / 256), dim3(256), 0, s, w.row_bound, num_queries);
@@ -211,7 +215,7 @@ static int knn_search_blocks(const KnnWorkspace& w, const KnnOperands& op, uint3
         t.start(s);
         uint32_t seg_width = 0;
         const bool guided = knn_block_guided(num_queries, ncols, k);
-        int rc = op.into_matrix(c0, ncols, num_queries, w.block_scores, cb, guided ? w.seg_max : nullptr, guided ? &seg_width : nullptr);
+        int rc = op.into_matrix(c0, ncols, num_queries, w.block_scores, cb, order, guided ? w.seg_max : nullptr, guided ? &seg_width : nullptr);
         if (rc) return rc;
         t.stop(s, t.gemm);
         t.start(s);
@@ -249,7 +253,9 @@ static int knn_search_candidates(const KnnWorkspace& w, const KnnOperands& op, u
     int rc = DSX_OK;
     if (screened) rc = screen_prepare(w.screen, op.queries, op.dim, num_queries, op.items, op.rows_padded, nullptr, M, op.dim, false, w.overflow, nullptr);
     if (rc) return rc;
-    rc = op.into_matrix(0, done, num_queries, w.block_scores, cb);
+    FcOrder order;
+    order.as_candidates = !screened;
+    rc = op.into_matrix(0, done, num_queries, w.block_scores, cb, order);
     if (rc) return rc;
     t.stop(s, t.gemm);
     t.start(s);
