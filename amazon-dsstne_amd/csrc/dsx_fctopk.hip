@@ -239,9 +239,12 @@ static int fc_topk_common(const float* X, uint32_t ldx, const float* W, const fl
     // A bound taken over `done` columns lets about k * width / done of the next `width` columns pass: ranges grow by a factor that
     // keeps that near an eighth of a list (the sample's own items, which score high and pass as well, come on top).
     const uint32_t growth = std::max(4u, cap / (8 * k));
-    uint32_t done = n0;
+    // Screened, the first block's scores give the bounds and nothing else: what passes is scored by one kernel wherever it lies (equal
+    // columns are to tie, and its sums have not that block's order), so the first range starts at column 0.
+    uint32_t done = screened ? 0 : n0;
     while (done < n) {
-        uint32_t ncols = (uint32_t)std::min<uint64_t>((uint64_t)n - done, (uint64_t)done * growth / 128 * 128);
+        const bool first = done == 0;
+        uint32_t ncols = (uint32_t)std::min<uint64_t>((uint64_t)n - done, first ? n0 + (uint64_t)n0 * growth / 128 * 128 : (uint64_t)done * growth / 128 * 128);
         if (n - done - ncols < 128) ncols = n - done;   // no sliver of a last range
         CandArgs cand{};
         cand.row_bound = w.row_bound;
@@ -254,7 +257,7 @@ static int fc_topk_common(const float* X, uint32_t ldx, const float* W, const fl
         cand.slope = params ? params->slope : 0.01f;
         cand.alpha = params ? params->alpha : 1.0f;
         cand.lambda = params ? params->lambda : 1.0f;
-        if (screened) rc = screen_candidates(w.screen, X, ldx, batch, kdim, true, bias, ncols, cand, false);
+        if (screened) rc = screen_candidates(w.screen, X, ldx, batch, kdim, true, bias, ncols, cand, false, first);
         else rc = x_planes ? fc_split_candidates_run(x_planes, w_planes, wrows, done, batch, kdim, ncols, cand, true, bias ? bias + done : nullptr)
                            : fc_layer_candidates_run(X, ldx, W + done, n, bias ? bias + done : nullptr, batch, kdim, ncols, cand);
         if (rc) return rc;
@@ -267,7 +270,7 @@ static int fc_topk_common(const float* X, uint32_t ldx, const float* W, const fl
             r.keys = keys;
             r.values = values;
         }
-        r.X = X; r.W = W; r.bias = bias; r.ldx = ldx; r.ldw = n; r.kdim = kdim; r.n = n; r.first_columns = n0;
+        r.X = X; r.W = W; r.bias = bias; r.ldx = ldx; r.ldw = n; r.kdim = kdim; r.n = n; r.first_columns = screened ? 0 : n0; r.fresh = first;
         r.act = activation; r.slope = cand.slope; r.alpha = cand.alpha; r.lambda = cand.lambda;
         rc = layer_refresh_run(r, batch);
         if (rc) return rc;

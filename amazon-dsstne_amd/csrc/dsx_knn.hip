@@ -263,19 +263,24 @@ static int knn_search_candidates(const KnnWorkspace& w, const KnnOperands& op, u
                   1, w.row_bound);
     if (rc) return rc;
     t.stop(s, t.topk);
+    // Screened, the block's scores give the bounds and nothing else: what passes is scored by one kernel wherever it lies (equal items
+    // are to tie, and its sums have not this block's order), so the first range starts at column 0.
+    const uint32_t seen = done;
+    if (screened) done = 0;
     while (done < M) {
+        const bool first = screened && done == 0;
         // a multiple of the tile width keeps every range's first column 16-byte aligned
-        const uint32_t ncols = (uint32_t)std::min<uint64_t>((uint64_t)M - done, (uint64_t)done * 4 / 128 * 128);
+        const uint32_t ncols = (uint32_t)std::min<uint64_t>((uint64_t)M - done, first ? (uint64_t)seen * 5 / 128 * 128 : (uint64_t)done * 4 / 128 * 128);
         t.start(s);
         const CandArgs cand{w.row_bound, w.cand, w.cand_count, kCandCap, done, w.overflow};
         uint32_t chunks = 0;
-        rc = screened ? screen_candidates(w.screen, op.queries, op.dim, num_queries, op.dim, false, nullptr, ncols, cand, true)
+        rc = screened ? screen_candidates(w.screen, op.queries, op.dim, num_queries, op.dim, false, nullptr, ncols, cand, true, first)
                       : op.into_candidates(done, ncols, num_queries, cand, w.seg, w.seg_count, &chunks);
         if (rc) return rc;
         t.stop(s, t.gemm);
         t.start(s);
         rc = knn_refresh(w.partial, w.cand, w.cand_count, kCandCap, k, w.row_bound, num_queries, chunks ? w.seg : nullptr, w.seg_count, chunks,
-                         chunks ? kCandCap / chunks : 0);
+                         chunks ? kCandCap / chunks : 0, first);
         if (rc) return rc;
         t.stop(s, t.topk);
         done += ncols;

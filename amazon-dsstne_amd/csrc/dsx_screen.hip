@@ -2,8 +2,9 @@
 //
 // A search keeps, per row, the columns whose fp32 score reaches the row's bound: a few hundred of a million.  The fp32 matrix
 // instructions form every product at 1/16 of the f16 ones' rate (157 TFLOP/s against 2.5 PFLOP/s), so here the columns are looked at
-// in f16 first, with a bound lowered by what the f16 operands can be wrong by, and what passes is scored in fp32.  Scores, bounds and
-// results are fp32 as before; the f16 products only decide what cannot be a result.
+// in f16 first, with a bound lowered by what the f16 operands can be wrong by, and what passes is scored in fp32.  Scores and
+// results are fp32 sums, all of them formed by screen_rescore_kernel in one order (equal columns tie, wherever they lie); the f16
+// products only decide what cannot be a result, and the first block's fp32 matrix only gives the first bounds.
 //
 // Error of a screened sum s' = sum x'_i w'_i against the fp32 sum s of the same row and column, x', w' rounded to f16 (unit
 // roundoff u = 2^-11, 2^-25 absolute below the normal range), fp32 accumulation:
@@ -121,6 +122,7 @@ struct ScreenRowsArgs {
     _Float16* out16;        // [batch rounded up to 256][ld], zero filled
     const uint32_t* stats;
     float* eps;             // [batch] what a bound is lowered by
+    float* slack;           // [batch] layers: and by how much more where it comes from another kernel's sums
     uint32_t* flag;         // one word (nearest neighbours) or one per row (layers): set where the error has no bound
     uint32_t* told;         // host-visible word set with it (may be NULL)
 };
@@ -154,6 +156,9 @@ __global__ __launch_bounds__(256) void screen_rows_kernel(ScreenRowsArgs a)
     if constexpr (ITEM_NORM) eps += ((float)a.dim + 64.0f) * 2.3841858e-7f * bias + 1e-6f * bias + 1e-7f;
     else eps += screen_relative(a.dim) * norm * most + (float)a.dim * 8.8817842e-16f * 1.01f;   // (a layer's 1e-7 covers the last term)
     a.eps[row] = eps;
+    // The k columns that set the first bound are scored again in another order: d + d / 16 + 5 roundings of 2^-24 of |x| |w| apart at most,
+    // four more of |x| |w| + |b| for the bias.  (Nearest neighbours: inside the 4 d + 64 of screen_relative.)
+    if constexpr (ITEM_NORM) a.slack[row] = ((1.25f * (float)a.dim + 16.0f) * 5.9604645e-8f * norm * most + 2.3841858e-7f * bias) * 1.01f;
     // (a NaN in the row: its scores are NaN everywhere, there is nothing to miss)
     const bool bad = norm > kF16Max || most > kF16Max || bias > kF16Max;
     if (bad) {
@@ -163,16 +168,18 @@ __global__ __launch_bounds__(256) void screen_rows_kernel(ScreenRowsArgs a)
 }
 
 // The bounds the screened sums are compared with: the rows' bounds, as pre-activation sums, less the error.
-__global__ __launch_bounds__(256) void screen_bounds_kernel(const uint32_t* row_bound, const float* eps, uint32_t batch, uint32_t act, float slope,
-                                                            float alpha, float lambda, uint32_t* admit)
+__global__ __launch_bounds__(256) void screen_bounds_kernel(const uint32_t* row_bound, const float* eps, const float* slack, uint32_t batch, uint32_t act,
+                                                            float slope, float alpha, float lambda, uint32_t* admit)
 {
     const uint32_t row = blockIdx.x * 256 + threadIdx.x;
     if (row >= batch) return;
     const uint32_t key = row_bound[row];
     const float z = preactivation_bound(key, act, slope, alpha, lambda);
-    const float b = z - eps[row] * 1.001f - fabsf(z) * 2.3841858e-7f;   // (the subtraction itself is rounded)
+    const float b = z - (eps[row] + (slack ? slack[row] : 0.0f)) * 1.001f - fabsf(z) * 2.3841858e-7f;   // (the subtraction itself is rounded)
+    // a ReLU's k-th score this close to 0 may come out as 0 in the other order, and everything below 0 then ties with it
+    const bool flat = slack && act == DSX_ACT_RELU && z <= slack[row];
     // no bound yet, or none that can be lowered: everything that is a number passes
-    admit[row] = (key == 0 || !(b >= -__builtin_inff())) ? 0u : score_key(b);
+    admit[row] = (key == 0 || flat || !(b >= -__builtin_inff())) ? 0u : score_key(b);
 }
 
 // Scores what passed in fp32: one workgroup per row, sixteen lanes per candidate.  The row's shared list is rewritten in place, the
@@ -283,6 +290,8 @@ ScreenWorkspace screen_layout(void* base, uint32_t batch, uint32_t dim, uint64_t
     p += align256(knn_f16_rows(batch) * screen_ld(dim, layer) * 2);
     w.eps = (float*)p;
     p += align256((size_t)batch * sizeof(float));
+    w.slack = (float*)p;
+    p += align256((size_t)batch * sizeof(float));
     w.admit = (uint32_t*)p;
     p += align256((size_t)batch * sizeof(uint32_t));
     w.stats = (uint32_t*)p;
@@ -313,7 +322,7 @@ int screen_prepare(const ScreenWorkspace& w, const float* X, uint32_t ldx, uint3
     DSX_LAUNCH_CHECK("screen_items_kernel");
     ScreenRowsArgs r{};
     r.X = X; r.ldx = ldx; r.batch = batch; r.dim = dim; r.ld = i.ld;
-    r.out16 = (_Float16*)w.queries16; r.stats = w.stats; r.eps = w.eps; r.flag = flag; r.told = told;
+    r.out16 = (_Float16*)w.queries16; r.stats = w.stats; r.eps = w.eps; r.slack = w.slack; r.flag = flag; r.told = told;
     const dim3 rgrid((uint32_t)(knn_f16_rows(batch) / 4));
     if (layer) hipLaunchKernelGGL((screen_rows_kernel<true>), rgrid, dim3(256), 0, s, r);
     else hipLaunchKernelGGL((screen_rows_kernel<false>), rgrid, dim3(256), 0, s, r);
@@ -322,12 +331,12 @@ int screen_prepare(const ScreenWorkspace& w, const float* X, uint32_t ldx, uint3
 }
 
 int screen_candidates(const ScreenWorkspace& w, const float* X, uint32_t ldx, uint32_t batch, uint32_t dim, bool layer, const float* bias,
-                      uint32_t ncols, const CandArgs& cand, bool report_overflow)
+                      uint32_t ncols, const CandArgs& cand, bool report_overflow, bool first)
 {
     hipStream_t s = ctx().stream;
     const uint32_t ld = screen_ld(dim, layer), act = layer ? cand.act : (uint32_t)DSX_ACT_LINEAR;
-    hipLaunchKernelGGL(screen_bounds_kernel, dim3((batch + 255) / 256), dim3(256), 0, s, cand.row_bound, w.eps, batch, act, cand.slope, cand.alpha,
-                       cand.lambda, w.admit);
+    hipLaunchKernelGGL(screen_bounds_kernel, dim3((batch + 255) / 256), dim3(256), 0, s, cand.row_bound, w.eps, layer && first ? w.slack : nullptr, batch, act,
+                       cand.slope, cand.alpha, cand.lambda, w.admit);
     DSX_LAUNCH_CHECK("screen_bounds_kernel");
     CandArgs screened = cand;
     screened.row_bound = w.admit;

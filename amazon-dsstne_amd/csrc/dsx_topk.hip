@@ -1590,12 +1590,12 @@ int topk_merge(const uint64_t* partial, uint32_t slots, uint32_t k, float* keys,
 
 // Exact KNN with candidate lists: merges a row's running best list (k packed words, best first) with the candidates the last
 // column range left behind, writes the best k back, raises the row's bound to their k-th key and empties the candidate
-// lists.  One wavefront per row.  The candidates are the row's shared list (cand, cand_count) and, after a sweep
+// lists.  fresh: the candidates are all there is (no best list yet; the bound becomes their k-th key).  One wavefront per row.  The candidates are the row's shared list (cand, cand_count) and, after a sweep
 // (knn_f16_sweep_kernel), its `chunks` private lists seg[row][chunk][seg_cap] with fill counts seg_count[row][64].
 template <int R>
 __global__ __launch_bounds__(kWave) void knn_refresh_kernel(uint64_t* best, const uint64_t* cand, uint32_t* cand_count, uint32_t cap,
                                                             uint32_t k, uint32_t* row_bound, const uint64_t* seg, uint32_t* seg_count,
-                                                            uint32_t chunks, uint32_t seg_cap)
+                                                            uint32_t chunks, uint32_t seg_cap, int fresh)
 {
     using List = WaveTopK<R>;
     __shared__ uint64_t sStage[List::kStageWords];
@@ -1607,7 +1607,7 @@ __global__ __launch_bounds__(kWave) void knn_refresh_kernel(uint64_t* best, cons
     uint64_t* mine = best + (uint64_t)b * k;
     for (uint32_t p0 = 0; p0 < k; p0 += kWave) {
         const uint32_t p = p0 + lane;
-        const uint64_t word = (p < k) ? mine[p] : 0ull;
+        const uint64_t word = (p < k && !fresh) ? mine[p] : 0ull;
         list.offer(word != 0, word);
     }
     const uint32_t n = min(cand_count[b], cap);
@@ -1654,26 +1654,26 @@ __global__ __launch_bounds__(kWave) void knn_refresh_kernel(uint64_t* best, cons
     for (int r = 0; r < R; r++) {
         const uint32_t p = r * kWave + lane;
         if (p < k) mine[p] = list.q[r];
-        if (p == k - 1 && list.q[r] != 0) row_bound[b] = max(row_bound[b], (uint32_t)(list.q[r] >> 32));
+        if (p == k - 1 && list.q[r] != 0) row_bound[b] = max(fresh ? 0u : row_bound[b], (uint32_t)(list.q[r] >> 32));
     }
     if (lane == 0) cand_count[b] = 0;
 }
 
 int knn_refresh(uint64_t* best, const uint64_t* cand, uint32_t* cand_count, uint32_t cap, uint32_t k, uint32_t* row_bound, uint32_t batch,
-                const uint64_t* seg, uint32_t* seg_count, uint32_t chunks, uint32_t seg_cap)
+                const uint64_t* seg, uint32_t* seg_count, uint32_t chunks, uint32_t seg_cap, bool fresh)
 {
     hipStream_t s = ctx().stream;
     if (seg && (chunks == 0 || chunks > (uint32_t)kWave || !seg_count))
         return set_error(DSX_EINVAL, "knn_refresh: %u chunks (1..64)", chunks);
     if (k <= 64)
         hipLaunchKernelGGL((knn_refresh_kernel<1>), dim3(batch), dim3(kWave), 0, s, best, cand, cand_count, cap, k, row_bound, seg, seg_count,
-                           chunks, seg_cap);
+                           chunks, seg_cap, fresh ? 1 : 0);
     else if (k <= 128)
         hipLaunchKernelGGL((knn_refresh_kernel<2>), dim3(batch), dim3(kWave), 0, s, best, cand, cand_count, cap, k, row_bound, seg, seg_count,
-                           chunks, seg_cap);
+                           chunks, seg_cap, fresh ? 1 : 0);
     else
         hipLaunchKernelGGL((knn_refresh_kernel<4>), dim3(batch), dim3(kWave), 0, s, best, cand, cand_count, cap, k, row_bound, seg, seg_count,
-                           chunks, seg_cap);
+                           chunks, seg_cap, fresh ? 1 : 0);
     DSX_LAUNCH_CHECK("knn_refresh_kernel");
     return DSX_OK;
 }
@@ -1711,6 +1711,7 @@ struct LayerRefreshArgs {
     const float* bias;
     uint32_t ldx, ldw, kdim, n;
     uint32_t first_columns;    // columns of the first block, whose listed columns the scanning top-K has dealt with
+    int fresh;                 // the candidates are all there is: no best list yet, row_bound is replaced and not raised
     uint32_t act;
     float slope, alpha, lambda;
 };
@@ -1835,7 +1836,7 @@ __global__ __launch_bounds__(kWave) void layer_refresh_kernel(LayerRefreshArgs a
     uint64_t* mine = a.best + (uint64_t)b * a.k;
     for (uint32_t p0 = 0; p0 < a.k; p0 += kWave) {
         const uint32_t p = p0 + lane;
-        const uint64_t word = (p < a.k) ? mine[p] : 0ull;
+        const uint64_t word = (p < a.k && !a.fresh) ? mine[p] : 0ull;
         list.offer(word != 0, word);
     }
     for (uint32_t p0 = 0; p0 < count; p0 += kWave) {
@@ -1891,7 +1892,7 @@ __global__ __launch_bounds__(kWave) void layer_refresh_kernel(LayerRefreshArgs a
     for (int r = 0; r < R; r++) {
         const uint32_t p = r * kWave + lane;
         if (p < a.k) mine[p] = list.q[r];
-        if (p == a.k - 1 && list.q[r] != 0) a.row_bound[b] = max(a.row_bound[b], (uint32_t)(list.q[r] >> 32));
+        if (p == a.k - 1 && list.q[r] != 0) a.row_bound[b] = max(a.fresh ? 0u : a.row_bound[b], (uint32_t)(list.q[r] >> 32));
     }
 }
 
@@ -1905,6 +1906,7 @@ int layer_refresh_run(const LayerRefresh& r, uint32_t batch)
     a.keys = r.keys; a.values = r.values;
     a.X = r.X; a.W = r.W; a.bias = r.bias; a.ldx = r.ldx; a.ldw = r.ldw; a.kdim = r.kdim; a.n = r.n;
     a.first_columns = r.first_columns;
+    a.fresh = r.fresh ? 1 : 0;
     a.act = r.act; a.slope = r.slope; a.alpha = r.alpha; a.lambda = r.lambda;
     hipStream_t s = ctx().stream;
     if (a.k <= 64) hipLaunchKernelGGL((layer_refresh_kernel<1>), dim3(batch), dim3(kWave), 0, s, a);

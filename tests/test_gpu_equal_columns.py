@@ -38,6 +38,17 @@ def check_twins(scores, idx, twin):
     assert pairs > 0
 
 
+# the first block of a screened search is 8,192 items; both sweeps (up to 256 components and more)
+@pytest.mark.parametrize("n,queries,dim,k", [(70000, 512, 64, 50), (90003, 600, 300, 100), (66000, 520, 100, 200)])
+def test_screened_search(pkg, dsx, rng, n, queries, dim, k):
+    print("[case] equal items screened n=%d queries=%d dim=%d k=%d" % (n, queries, dim, k), flush=True)
+    items, twin = with_twins(rng, n, dim, 8192, 8192, 3000)
+    q = rng.standard_normal((queries, dim), dtype=np.float32)
+    s, i = search(pkg, dsx, items, q, k)
+    assert dsx.dsx_knn_last_search_path() == 1
+    check_twins(s, i, twin)
+
+
 # blocks of 1,024 items, the last one narrow (dim no multiple of 4: block by block); first block, then candidate ranges
 @pytest.mark.parametrize("n,queries,dim,k,path", [(3 * 1024 + 100, 100, 130, 60, 0), (2 * 1024 + 40, 9, 70, 100, 0), (3 * 1024 + 8, 300, 258, 20, 0),
                                                   (20000, 70, 64, 100, 1), (9000, 100, 256, 50, 1)])
@@ -54,8 +65,9 @@ def test_search_in_blocks(pkg, dsx, rng, n, queries, dim, k, path):
     check_twins(s, i, twin)
 
 
-# fp32 ranges of the shapes whose first block other kernels would take
-@pytest.mark.parametrize("batch,kdim,n,k,act,first,screened", [(100, 64, 6001, 40, 3, 256, False), (60, 128, 9000, 30, 1, 512, False)])
+# screened with a bias; in fp32 ranges of the shapes whose first block other kernels would take
+@pytest.mark.parametrize("batch,kdim,n,k,act,first,screened", [(2048, 64, 20000, 40, 3, 0, True), (640, 260, 30000, 100, 0, 0, True),
+                                                               (100, 64, 6001, 40, 3, 256, False), (60, 128, 9000, 30, 1, 512, False)])
 def test_layer(pkg, dsx, rng, batch, kdim, n, k, act, first, screened):
     print("[case] equal columns batch=%d kdim=%d n=%d k=%d act=%d" % (batch, kdim, n, k, act), flush=True)
     block = first or 2048
