@@ -2011,7 +2011,14 @@ int topk_guided_run(const float* in, uint32_t width, uint32_t batch, uint32_t k,
                     uint32_t seg_width, uint32_t position, const uint32_t* index, const uint64_t* fstart, const uint64_t* fend,
                     const uint32_t* fidx, const float* fmul)
 {
-    if (!seg_max || seg_width != kGuidedSegWidth || !topk_guided_pays(batch, width, k))
+    bool guided = seg_max && seg_width == kGuidedSegWidth && topk_guided_pays(batch, width, k);
+    if (guided && width > kGuidedMaxSegs * kGuidedSegWidth) {
+        // (these rows are always cut, and a graph may keep no address of the library's scratch: the scan takes most of them whole)
+        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+        DSX_HIP(hipStreamIsCapturing(ctx().stream, &capturing));
+        guided = capturing == hipStreamCaptureStatusNone;
+    }
+    if (!guided)
         return topk_run(in, width, width, batch, k, keys, values, position, index, fstart, fend, fidx, fmul, 0, nullptr, 0, 0, 0);
     return topk_guided_launch(in, width, width, batch, k, keys, values, seg_max, position, index, fstart, fend, fidx, fmul, 0, nullptr, 0, 0,
                               nullptr);

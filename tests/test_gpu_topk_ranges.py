@@ -119,6 +119,35 @@ def test_guided_rows_under_capture(pkg, dsx, orc, rng):
     assert hip.hipGraphExecDestroy(instance) == 0 and hip.hipGraphDestroy(graph) == 0
 
 
+def test_guided_rows_wider_than_one_part_under_capture(pkg, dsx, rng):
+    """1,024 rows of more than 131,072 columns: one workgroup per row scans them, in a graph of one node without library scratch."""
+    batch, width, k = 1024, 131137, 10
+    hip = C.CDLL("libamdhip64.so")
+    dsx.dsx_stream.restype = C.c_void_p
+    stream = C.c_void_p(dsx.dsx_stream())
+    scores = np.tile(rng.standard_normal((16, width), dtype=np.float32), (batch // 16, 1))
+    scores[np.arange(batch), rng.integers(0, width, batch)] = np.float32(9.0)
+    d, dm = dev(pkg, scores), dev(pkg, segment_maxima(scores))
+    keys, vals = pkg.DeviceArray((batch, k), np.float32), pkg.DeviceArray((batch, k), np.uint32)
+    pkg.check(dsx.dsx_sync())
+    graph, instance = C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamBeginCapture(stream, 2) == 0                 # relaxed
+    rc = dsx.dsx_topk_guided(d.ptr, keys.ptr, vals.ptr, batch, width, k, dm.ptr, 64, 0, None, None, None, None, None)
+    assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
+    pkg.check(rc)
+    nodes = C.c_size_t(0)
+    assert hip.hipGraphGetNodes(graph, None, C.byref(nodes)) == 0 and nodes.value == 1
+    assert hip.hipGraphInstantiate(C.byref(instance), graph, None, None, 0) == 0
+    want = run_topk(pkg, dsx, scores, k)
+    for _ in range(2):
+        keys.upload(np.zeros((batch, k), np.float32))
+        pkg.check(dsx.dsx_sync())
+        assert hip.hipGraphLaunch(instance, stream) == 0
+        pkg.check(dsx.dsx_sync())
+        assert_topk_exact(keys.numpy(), vals.numpy(), *want)
+    assert hip.hipGraphExecDestroy(instance) == 0 and hip.hipGraphDestroy(graph) == 0
+
+
 @pytest.mark.parametrize("items,queries,dim,k", [(200003, 1, 40, 20), (150001, 4, 128, 10), (70000, 64, 33, 64), (70000, 65, 33, 64),
                                                  (40000, 7, 16, 256), (500, 3, 16, 100)])
 def test_knn_few_queries(pkg, dsx, orc, rng, items, queries, dim, k):
