@@ -103,6 +103,7 @@ SIGNATURES = {
     "dsx_fc_topk_flagged": [_int],
     "dsx_fc_topk_flagged_for": [_vp, _int],
     "dsx_testing_reset": [],
+    "dsx_testing_set_allocation_limit": [_sz],
     "dsx_testing_occupy": [_u32, _u32, _u32],
     "dsx_testing_set_fc_topk_first_columns": [_u32],
     "dsx_testing_set_fc_topk_candidate_capacity": [_u32],
@@ -116,10 +117,11 @@ SIGNATURES = {
 }
 SPECIAL_RESTYPES = {"dsx_last_error": C.c_char_p, "dsx_stream": C.c_void_p, "dsx_knn_workspace_bytes": C.c_size_t,
                     "dsx_knn_workspace_bytes_f16": C.c_size_t, "dsx_knn_f16_table_bytes": C.c_size_t, "dsx_fc_split_bytes": _u64,
-                    "dsx_knn_workspace_bytes_split": C.c_size_t}
+                    "dsx_knn_workspace_bytes_split": C.c_size_t, "dsx_knn_workspace_bytes_least": C.c_size_t}
 SPECIAL_ARGTYPES = {"dsx_last_error": [], "dsx_stream": [], "dsx_knn_workspace_bytes": [_u32, _u32, _u32, _u32],
                     "dsx_knn_workspace_bytes_f16": [_u32, _u32, _u32, _u32], "dsx_knn_f16_table_bytes": [_u32, _u32],
-                    "dsx_fc_split_bytes": [_u32, _u32], "dsx_knn_workspace_bytes_split": [_u32, _u32, _u32, _u32]}
+                    "dsx_fc_split_bytes": [_u32, _u32], "dsx_knn_workspace_bytes_split": [_u32, _u32, _u32, _u32],
+                    "dsx_knn_workspace_bytes_least": [_u32, _u32, _u32, _u32]}
 
 _lib = None
 

@@ -204,9 +204,8 @@ static int fc_topk_common(const float* X, uint32_t ldx, const float* W, const fl
     const bool ranges = n0 < n;
     bool screened = ranges && !x_planes && screen_takes(batch, kdim, n, true);
     LibScratch& ws = g_layer_ws_of[current_lane()];
-    int reserved = lib_scratch_reserve(ws, layer_layout(nullptr, batch, n0, k, cap, ranges, screened, kdim, n).bytes, "dsx_fc_topk workspace");
+    int reserved = lib_scratch_reserve(ws, layer_layout(nullptr, batch, n0, k, cap, ranges, screened, kdim, n).bytes, "dsx_fc_topk workspace", screened);
     if (reserved == DSX_ENOMEM && screened) {   // the 16-bit copies (up to 8 GiB) do not fit beside what is there: fp32 ranges need none
-        (void)hipGetLastError();
         screened = false;
         reserved = lib_scratch_reserve(ws, layer_layout(nullptr, batch, n0, k, cap, ranges, screened, kdim, n).bytes, "dsx_fc_topk workspace");
     }

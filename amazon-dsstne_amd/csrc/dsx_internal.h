@@ -16,6 +16,7 @@ struct TestKnobs {
     uint32_t fc_topk_candidate_capacity = 0;
     uint32_t knn_block_columns = 0;
     int knn_f16_sweep = 1;
+    size_t allocation_limit = 0;
 };
 
 struct Context {
@@ -41,8 +42,8 @@ struct LibScratch {
     bool listed = false;
 };
 // Makes s hold at least `bytes` (contents are not preserved when it grows; the selected lane is waited for before the old
-// block is freed).
-int lib_scratch_reserve(LibScratch& s, size_t bytes, const char* what);
+// block is freed).  optional: the caller can do with less; a block that memory is too short for then leaves the old one as it is.
+int lib_scratch_reserve(LibScratch& s, size_t bytes, const char* what, bool optional = false);
 // fn runs once in the last dsx_shutdown, before the library's memory is released (file-scope state of the other translation units).
 void at_shutdown(void (*fn)());
 int current_lane();   // 0 or 1: which of the two in-order streams ctx().stream is (scratch buffers are kept per lane)

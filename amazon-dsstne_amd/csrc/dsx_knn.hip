@@ -114,11 +114,11 @@ static KnnWorkspace knn_layout(void* base, uint32_t rows_padded, uint32_t num_qu
 // What a search of any number of queries up to num_queries needs: a workspace of a batch is used for smaller ones too, and fewer
 // queries may need more (5,000 rows, k = 100: 64 queries 3.634 MB, 65 queries 3.618, because 64 leave more lists per query).
 // About 40 ns per query count, once per table.
-static size_t knn_workspace_most(uint32_t rows_padded, uint32_t num_queries, uint32_t k, bool f16, uint32_t dim, bool split)
+static size_t knn_workspace_most(uint32_t rows_padded, uint32_t num_queries, uint32_t k, bool f16, uint32_t dim, bool split, bool screen = true)
 {
     size_t most = 0;
     for (uint64_t q = std::min(1u, num_queries); q <= num_queries; q++)
-        most = std::max(most, knn_layout(nullptr, rows_padded, (uint32_t)q, k, f16, dim, split).bytes);
+        most = std::max(most, knn_layout(nullptr, rows_padded, (uint32_t)q, k, f16, dim, split, screen).bytes);
     return most;
 }
 
@@ -322,6 +322,11 @@ size_t dsx_knn_workspace_bytes(uint32_t rows_padded, uint32_t dim, uint32_t num_
     return knn_workspace_most(rows_padded, num_queries, k, false, dim, false);
 }
 
+size_t dsx_knn_workspace_bytes_least(uint32_t rows_padded, uint32_t dim, uint32_t num_queries, uint32_t k)
+{
+    return knn_workspace_most(rows_padded, num_queries, k, false, dim, false, false);
+}
+
 size_t dsx_knn_workspace_bytes_f16(uint32_t rows_padded, uint32_t dim, uint32_t num_queries, uint32_t k)
 {
     return knn_workspace_most(rows_padded, num_queries, k, true, dim, false);
@@ -349,19 +354,19 @@ int dsx_knn_f16_convert_items(const float* items, uint32_t rows_padded, uint32_t
 static int knn_search_common(KnnOperands& op, uint32_t padding, uint32_t num_queries, uint32_t k, float* scores, uint32_t* indexes, void* workspace,
                              size_t workspace_bytes, float* elapsed_ms, bool aligned, const float* queries_f32)
 {
-    const size_t need = knn_layout(nullptr, op.rows_padded, num_queries, k, op.f16, op.dim, op.split).bytes;
-    bool screen = true;
+    const size_t full = knn_layout(nullptr, op.rows_padded, num_queries, k, op.f16, op.dim, op.split).bytes;
+    const size_t need = knn_layout(nullptr, op.rows_padded, num_queries, k, op.f16, op.dim, op.split, false).bytes;
+    bool screen = full != need;   // the screening's copies of the table (up to 8 GiB) where there is room for them: fp32 needs none
     if (workspace) {
         DSX_CHECK_ARG(workspace_bytes >= need, "dsx_knn_search: workspace of %zu bytes, %zu needed", workspace_bytes, need);
+        screen = screen && workspace_bytes >= full;
         DSX_CHECK_ARG(((uintptr_t)workspace % 256) == 0, "dsx_knn_search: workspace is not 256-byte aligned");
     } else {
         LibScratch& ws = g_knn_ws_of[current_lane()];
-        int reserved = lib_scratch_reserve(ws, need, "dsx_knn_search workspace");
-        if (reserved == DSX_ENOMEM) {   // the screening's copies of the table (up to 8 GiB) may be what does not fit: fp32 needs none
-            (void)hipGetLastError();
+        int reserved = screen ? lib_scratch_reserve(ws, full, "dsx_knn_search workspace", true) : DSX_ENOMEM;
+        if (reserved == DSX_ENOMEM) {
             screen = false;
-            reserved = lib_scratch_reserve(ws, knn_layout(nullptr, op.rows_padded, num_queries, k, op.f16, op.dim, op.split, screen).bytes,
-                                           "dsx_knn_search workspace");
+            reserved = lib_scratch_reserve(ws, need, "dsx_knn_search workspace");
         }
         if (reserved) return reserved;
         workspace = ws.ptr;

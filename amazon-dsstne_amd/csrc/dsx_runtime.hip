@@ -51,9 +51,16 @@ static std::map<void*, size_t> g_host_allocs;
 
 static std::vector<LibScratch*> g_lib_scratch;
 
-int lib_scratch_reserve(LibScratch& s, size_t bytes, const char* what)
+static bool over_limit(size_t bytes) { return ctx().knobs.allocation_limit != 0 && bytes > ctx().knobs.allocation_limit; }
+
+int lib_scratch_reserve(LibScratch& s, size_t bytes, const char* what, bool optional)
 {
-    if (bytes <= s.bytes) return DSX_OK;
+    if (bytes <= s.bytes && !over_limit(bytes)) return DSX_OK;
+    if (optional) {
+        size_t free_bytes = 0, total = 0;
+        DSX_HIP(hipMemGetInfo(&free_bytes, &total));
+        if (over_limit(bytes) || bytes > free_bytes + s.bytes) return set_error(DSX_ENOMEM, "%s: no room for %zu bytes", what, bytes);
+    }
     std::lock_guard<std::mutex> lock(g_alloc_mutex);
     if (s.ptr) {
         DSX_HIP(hipStreamSynchronize(ctx().stream));
@@ -62,8 +69,9 @@ int lib_scratch_reserve(LibScratch& s, size_t bytes, const char* what)
         s.ptr = nullptr;
         s.bytes = 0;
     }
-    hipError_t e = hipMalloc(&s.ptr, bytes);
+    hipError_t e = over_limit(bytes) ? hipErrorOutOfMemory : hipMalloc(&s.ptr, bytes);
     if (e != hipSuccess) {
+        (void)hipGetLastError();   // (the next launch is not the one that failed)
         s.ptr = nullptr;
         return set_error(DSX_ENOMEM, "%s: cannot allocate %zu bytes: %s", what, bytes, hipGetErrorString(e));
     }
@@ -305,6 +313,12 @@ int dsx_testing_occupy(uint32_t workgroups, uint32_t cycles, uint32_t vgprs)
     return DSX_OK;
 }
 
+int dsx_testing_set_allocation_limit(size_t bytes)
+{
+    ctx().knobs.allocation_limit = bytes;
+    return DSX_OK;
+}
+
 int dsx_testing_reset(void)
 {
     ctx().knobs = TestKnobs();
@@ -378,8 +392,11 @@ int dsx_malloc(void** p, size_t bytes)
     DSX_CHECK_ARG(p, "dsx_malloc: null result pointer");
     *p = nullptr;
     if (bytes == 0) bytes = 4;
-    hipError_t e = hipMalloc(p, bytes);
-    if (e != hipSuccess) return set_error(DSX_ENOMEM, "dsx_malloc: hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
+    hipError_t e = over_limit(bytes) ? hipErrorOutOfMemory : hipMalloc(p, bytes);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();   // (the next launch is not the one that failed)
+        return set_error(DSX_ENOMEM, "dsx_malloc: hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
+    }
     DSX_HIP(hipMemsetAsync(*p, 0, bytes, ctx().stream));
     if (int rc = lanes_join_after()) return rc;
     std::lock_guard<std::mutex> lock(g_alloc_mutex);

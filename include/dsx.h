@@ -344,6 +344,9 @@ int dsx_knn_search(const float* items, uint32_t rows_padded, uint32_t padding, u
                    uint32_t num_queries, uint32_t k, float* scores, uint32_t* indexes, void* workspace, size_t workspace_bytes,
                    float* elapsed_ms);
 size_t dsx_knn_workspace_bytes(uint32_t rows_padded, uint32_t dim, uint32_t num_queries, uint32_t k);
+/* dsx_knn_workspace_bytes holds, for 512 queries and more, two copies of the table (1.5 x its size, up to 8 GiB) that make the search
+ * faster (its candidates are screened in 16 bits); a workspace of at least this size but not that one is searched without them. */
+size_t dsx_knn_workspace_bytes_least(uint32_t rows_padded, uint32_t dim, uint32_t num_queries, uint32_t k);
 /* fp16 storage (astdl::knn::DataType::FP16).  The reference converts the column-major table once (KnnData::load,
  * knn/KnnData.cpp:209-216, kFloatToHalf of knn/MathUtil.cu:33-81: round to nearest even) and every query batch before the
  * GEMM (knn/KnnExactGpu.cu:108-116), multiplies fp16 operands and keeps fp32 scores.  Same arithmetic here; the fp16 table's

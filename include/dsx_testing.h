@@ -4,6 +4,7 @@
  * put every switch back to its default; like every call of the library they belong to the one thread that drives it. */
 #ifndef DSX_TESTING_H
 #define DSX_TESTING_H
+#include <stddef.h>
 #include <stdint.h>
 #ifdef __cplusplus
 extern "C" {
@@ -27,6 +28,9 @@ int dsx_testing_set_knn_f16_sweep(int mode);
  * registers per lane.  bench.py --interference uses it to separate what a kernel beside a dense layer costs that layer by
  * merely being resident from what its instructions and memory traffic cost. */
 int dsx_testing_occupy(uint32_t workgroups, uint32_t cycles, uint32_t vgprs);
+/* Largest single block of device memory that dsx_malloc and the library's own scratch may hold, in bytes (0, the default: what the
+ * device has): larger ones fail as if the memory were short. */
+int dsx_testing_set_allocation_limit(size_t bytes);
 /* Every switch back to its default. */
 int dsx_testing_reset(void);
 

@@ -135,3 +135,41 @@ def test_layer_above_the_range_is_recomputed(pkg, dsx, rng):
     check_against_float64(keys.numpy() / scale, vals.numpy(), y / scale, k, kdim * 2.0 ** -24)
     pkg.check(dsx.dsx_sync())
     assert dsx.dsx_fc_topk_flagged(1) == 1
+
+
+def test_without_room_for_the_copies_of_the_table(pkg, dsx, rng):
+    """A workspace, a library scratch or a KnnData without the 16-bit copies: the search runs in fp32."""
+    n, queries, dim, k = 70000, 520, 64, 20
+    items = rng.integers(-3, 4, size=(n, dim)).astype(np.float32)
+    q = rng.integers(-3, 4, size=(queries, dim)).astype(np.float32)
+    rs, ri = best(q @ items.T, k)
+    full, least = dsx.dsx_knn_workspace_bytes(n, dim, queries, k), dsx.dsx_knn_workspace_bytes_least(n, dim, queries, k)
+    assert full > least + n * dim * 4
+    dI, dQ = dev(pkg, np.ascontiguousarray(items.T)), dev(pkg, q)
+    scores, idx = pkg.DeviceArray((queries, k), np.float32), pkg.DeviceArray((queries, k), np.uint32)
+    room = pkg.DeviceArray((full,), np.uint8)
+
+    def run(workspace, size):
+        scores.upload(np.zeros((queries, k), np.float32))
+        rc = dsx.dsx_knn_search(dI.ptr, n, 0, dim, dQ.ptr, queries, k, scores.ptr, idx.ptr, workspace, size, None)
+        if rc == 0:
+            assert np.array_equal(scores.numpy(), rs) and np.array_equal(idx.numpy(), ri)
+        return rc
+
+    for size, path in ((full, 1), (full - 256, 0), (least, 0)):
+        assert run(room.ptr, size) == 0 and dsx.dsx_knn_last_search_path() == path
+    assert run(room.ptr, least - 256) == -1
+    import amazon_dsstne_amd.host_api as host_api
+    lib = host_api.load_host_library()
+    dsx.dsx_testing_set_allocation_limit(full - 256)
+    try:
+        for _ in range(2):
+            assert run(None, 0) == 0 and dsx.dsx_knn_last_search_path() == 0
+        knn = lib.dsstne_knn_create_typed(queries, k, b"fp32")
+        assert knn and lib.dsstne_knn_load(knn, items.ctypes.data, n, dim, None) == 0
+        s, i = np.empty((queries, k), np.float32), np.empty((queries, k), np.uint32)
+        assert lib.dsstne_knn_search(knn, k, q.ctypes.data, queries, s.ctypes.data, i.ctypes.data) == 0
+        lib.dsstne_knn_destroy(knn)
+        assert np.array_equal(s, rs) and np.array_equal(i, ri) and dsx.dsx_knn_last_search_path() == 0
+    finally:
+        dsx.dsx_testing_set_allocation_limit(0)
