@@ -66,14 +66,17 @@ static uint32_t layer_first_columns(uint32_t n, uint32_t k)
 struct LayerWorkspace {
     float* block_scores;   // [batch][ld0]
     uint64_t* best;        // [batch][k]
-    uint32_t* row_bound;   // [batch]   (row_bound, cand_count and row_flag are cleared together)
+    uint32_t* row_bound;   // [batch]   (row_bound, cand_count, row_flag, overflow and redo_done are cleared together)
     uint32_t* cand_count;  // [batch]
     uint32_t* row_flag;    // [batch]
     uint32_t* overflow;    // [64] unused flag word of the shared epilogue
-    uint64_t* cand;        // [batch][cap]
+    uint32_t* redo_done;   // [layer_redo_groups]
+    uint64_t* cand;        // [batch][cap]; after the last range: the lists of rows that are computed again
     ScreenWorkspace screen;   // where the ranges are screened in 16 bits
     size_t bytes;
 };
+
+static size_t layer_clear_words(uint32_t batch) { return (size_t)3 * batch + 64 + layer_redo_groups(batch); }
 
 static LayerWorkspace layer_layout(void* base, uint32_t batch, uint32_t n0, uint32_t k, uint32_t cap, bool ranges, bool screened,
                                    uint32_t kdim, uint32_t n)
@@ -89,9 +92,10 @@ static LayerWorkspace layer_layout(void* base, uint32_t batch, uint32_t n0, uint
     w.cand_count = w.row_bound + batch;
     w.row_flag = w.cand_count + batch;
     w.overflow = w.row_flag + batch;
-    p += align256(((size_t)3 * batch + 64) * sizeof(uint32_t));
+    w.redo_done = w.overflow + 64;
+    p += align256(layer_clear_words(batch) * sizeof(uint32_t));
     w.cand = (uint64_t*)p;
-    if (ranges) p += align256((size_t)batch * cap * sizeof(uint64_t));
+    if (ranges) p += align256(std::max<size_t>((size_t)batch * cap, layer_redo_words(batch, k)) * sizeof(uint64_t));
     w.screen = ScreenWorkspace{};
     if (screened) {
         w.screen = screen_layout(p, batch, kdim, n, true, kLayerCandCap);
@@ -224,7 +228,7 @@ static int fc_topk_common(const float* X, uint32_t ldx, const float* W, const fl
     if (!ranges)
         return topk_run(w.block_scores, ld0, n0, batch, k, keys, values, position, index, filter_start, filter_end, filter_index, nullptr, 0,
                         nullptr, 0, 0, 0);
-    const uint32_t clear_words = 3 * batch + 64;
+    const uint32_t clear_words = (uint32_t)layer_clear_words(batch);
     hipLaunchKernelGGL(layer_clear_kernel, dim3((clear_words + 255) / 256), dim3(256), 0, s, w.row_bound, clear_words);
     DSX_LAUNCH_CHECK("layer_clear_kernel");
     if (screened) {
@@ -269,12 +273,19 @@ static int fc_topk_common(const float* X, uint32_t ldx, const float* W, const fl
             r.keys = keys;
             r.values = values;
         }
-        r.X = X; r.W = W; r.bias = bias; r.ldx = ldx; r.ldw = n; r.kdim = kdim; r.n = n; r.first_columns = screened ? 0 : n0; r.fresh = first;
-        r.act = activation; r.slope = cand.slope; r.alpha = cand.alpha; r.lambda = cand.lambda;
+        r.n = n; r.first_columns = screened ? 0 : n0; r.fresh = first;
         rc = layer_refresh_run(r, batch);
         if (rc) return rc;
     }
-    return DSX_OK;
+    LayerRedo redo{};
+    redo.X = X; redo.W = W; redo.bias = bias; redo.ldx = ldx; redo.ldw = n; redo.kdim = kdim; redo.n = n; redo.k = k;
+    redo.act = activation;
+    redo.slope = params ? params->slope : 0.01f;
+    redo.alpha = params ? params->alpha : 1.0f;
+    redo.lambda = params ? params->lambda : 1.0f;
+    redo.position = position; redo.index = index; redo.fstart = filter_start; redo.fend = filter_end; redo.fidx = filter_index;
+    redo.row_flag = w.row_flag; redo.partial = w.cand; redo.done = w.redo_done; redo.keys = keys; redo.values = values;
+    return layer_redo_run(redo, batch);
 }
 
 extern "C" {

@@ -164,16 +164,34 @@ struct LayerRefresh {
     const uint32_t* fidx;
     float* keys;
     uint32_t* values;
+    uint32_t n;
+    uint32_t first_columns;   // width of the first block (scanned with the filter applied)
+    bool fresh;               // best holds nothing yet, and row_bound is replaced by the k-th of these candidates
+};
+int layer_refresh_run(const LayerRefresh& r, uint32_t batch);
+// The rows that row_flag marks, from X and W: their results go to keys / values.  partial: layer_redo_words words of scratch; done:
+// layer_redo_groups words, 0 before the call.
+struct LayerRedo {
     const float* X;
     const float* W;
     const float* bias;
-    uint32_t ldx, ldw, kdim, n;
-    uint32_t first_columns;   // width of the first block (scanned with the filter applied)
-    bool fresh;               // best holds nothing yet, and row_bound is replaced by the k-th of these candidates
+    uint32_t ldx, ldw, kdim, n, k;
     uint32_t act;
     float slope, alpha, lambda;
+    uint32_t position;
+    const uint32_t* index;
+    const uint64_t* fstart;
+    const uint64_t* fend;
+    const uint32_t* fidx;
+    const uint32_t* row_flag;
+    uint64_t* partial;
+    uint32_t* done;
+    float* keys;
+    uint32_t* values;
 };
-int layer_refresh_run(const LayerRefresh& r, uint32_t batch);
+uint64_t layer_redo_words(uint32_t batch, uint32_t k);
+uint32_t layer_redo_groups(uint32_t batch);
+int layer_redo_run(const LayerRedo& r, uint32_t batch);
 // fp16 storage of the KNN operands (dsx_knn_f16.hip): padded row-major layout, conversion, and the score kernel in store mode
 // (cand == NULL: Z[batch][ldz]) or candidate mode.
 uint32_t knn_f16_ld(uint32_t dim);

@@ -1683,10 +1683,8 @@ int knn_refresh(uint64_t* best, const uint64_t* cand, uint32_t* cand_count, uint
 // the layer's last column range appended, minus the columns the row's filter lists (multiplier 0: the sample's own items).
 // One wavefront per row.  The filter is applied by hashing the candidates' columns into an LDS table (at most half full,
 // linear probing), striking out every listed column found there, and then offering only the candidates still present.
-// A row whose candidate list filled up is flagged; the refresh after the last range recomputes flagged rows from scratch,
-// without any list that could fill up: act(bias + x . W) 256 columns at a time (lane = column, k in order), the listed columns
-// marked in a bitmap that covers 262,144 columns at a time.  Slow (the whole matrix is read for one row) and exact.
-constexpr uint32_t kLayerTableSlots = 8192;   // twice the candidate capacity the layer search uses; as a bitmap: 262,144 columns
+// A row whose candidate list filled up is flagged, and layer_redo_kernel computes flagged rows from scratch after the last range.
+constexpr uint32_t kLayerTableSlots = 8192;   // twice the candidate capacity the layer search uses
 constexpr uint32_t kLayerEmpty = 0xffffffffu, kLayerStruck = 0xfffffffeu;   // (no column has these numbers: widths stay below 2^32 - 2)
 
 struct LayerRefreshArgs {
@@ -1705,63 +1703,12 @@ struct LayerRefreshArgs {
     const uint32_t* fidx;      // NULL: no filter
     float* keys;               // final range only (else NULL): [batch][k] results
     uint32_t* values;
-    // the layer itself, for flagged rows (final range only)
-    const float* X;
-    const float* W;
-    const float* bias;
-    uint32_t ldx, ldw, kdim, n;
+    uint32_t n;                // columns of the layer
     uint32_t first_columns;    // columns of the first block, whose listed columns the scanning top-K has dealt with
     int fresh;                 // the candidates are all there is: no best list yet, row_bound is replaced and not raised
-    uint32_t act;
-    float slope, alpha, lambda;
 };
 
 __device__ __forceinline__ uint32_t layer_hash(uint32_t col, uint32_t shift) { return (col * 2654435761u) >> shift; }
-
-template <int R>
-__device__ __forceinline__ void layer_recompute_row(WaveTopK<R>& list, const LayerRefreshArgs& a, uint32_t b, uint32_t lane, uint64_t fs,
-                                                    uint64_t fe, uint32_t* sBits)
-{
-    constexpr uint32_t kSpan = kLayerTableSlots * 32;
-    const float* x = a.X + (uint64_t)b * a.ldx;
-    for (uint32_t C0 = 0; C0 < a.n; C0 += kSpan) {
-        for (uint32_t i = lane; i < kLayerTableSlots; i += kWave) sBits[i] = 0;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        for (uint64_t t = fs + lane; t < fe; t += kWave) {
-            const uint32_t c = a.fidx[t];
-            if (c >= C0 && c - C0 < kSpan) atomicOr(&sBits[(c - C0) >> 5], 1u << ((c - C0) & 31));
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        const uint32_t C1 = (a.n - C0 < kSpan) ? a.n : C0 + kSpan;
-        for (uint32_t c0 = C0; c0 < C1; c0 += 4 * kWave) {
-            float sum[4];
-            uint32_t col[4];
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                col[j] = c0 + j * kWave + lane;
-                sum[j] = (a.bias && col[j] < C1) ? a.bias[col[j]] : 0.0f;
-            }
-            for (uint32_t kk = 0; kk < a.kdim; kk++) {
-                const float xk = x[kk];
-                const float* w = a.W + (uint64_t)kk * a.ldw;
-#pragma unroll
-                for (int j = 0; j < 4; j++)
-                    if (col[j] < C1) sum[j] = fmaf(xk, w[col[j]], sum[j]);
-            }
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                float y = activate_rt(sum[j], a.act, a.slope, a.alpha, a.lambda);
-                const uint32_t off = col[j] - C0;
-                // a listed column keeps its place with score * 0 (utils/Filters.cpp:62), once however often it is listed
-                if (col[j] < C1 && ((sBits[off >> 5] >> (off & 31)) & 1u)) y *= 0.0f;
-                list.offer(col[j] < C1 && y == y, pack_score(y, col[j]));
-            }
-        }
-        __builtin_amdgcn_wave_barrier();
-    }
-}
 
 template <int R>
 __global__ __launch_bounds__(kWave) void layer_refresh_kernel(LayerRefreshArgs a)
@@ -1784,9 +1731,9 @@ __global__ __launch_bounds__(kWave) void layer_refresh_kernel(LayerRefreshArgs a
         }
     }
     const bool final_range = a.keys != nullptr;
-    if (flagged && !final_range) return;
+    if (flagged) return;
     uint64_t fs = 0, fe = 0;
-    if (a.fidx && (count > 0 || flagged || final_range)) {
+    if (a.fidx && (count > 0 || final_range)) {
         uint32_t r = a.position + b;
         if (a.index) r = a.index[r];
         fs = a.fstart[r];
@@ -1794,12 +1741,6 @@ __global__ __launch_bounds__(kWave) void layer_refresh_kernel(LayerRefreshArgs a
     }
     List list;
     list.init(sStage, lane, a.k);
-    if (flagged) {
-        layer_recompute_row<R>(list, a, b, lane, fs, fe, sTable);
-        list.finish();
-        write_final<R>(list.q, lane, a.k, 0, a.keys + (uint64_t)b * a.k, a.values + (uint64_t)b * a.k);
-        return;
-    }
     const uint64_t* src = a.cand + (uint64_t)b * a.cap;
     const bool filtering = fe > fs && count > 0;   // wave-uniform
     // table size: a power of two, at least twice the candidates
@@ -1862,7 +1803,7 @@ __global__ __launch_bounds__(kWave) void layer_refresh_kernel(LayerRefreshArgs a
     if (final_range) {
         // The listed columns beyond the first block were struck out above, but a listed column scores 0, not nothing
         // (utils/Filters.cpp:62 multiplies, kCalculateTopK then sees the zero): when the row's k-th score is not above 0, or the
-        // row has fewer than k scores, such a zero belongs in the result.  Those rows are computed again, column by column.
+        // row has fewer than k scores, such a zero belongs in the result.  Those rows are computed again (layer_redo_kernel).
         uint64_t kth = 0;
 #pragma unroll
         for (int r = 0; r < R; r++) {
@@ -1879,11 +1820,11 @@ __global__ __launch_bounds__(kWave) void layer_refresh_kernel(LayerRefreshArgs a
             zeros_matter = __ballot(beyond) != 0;
         }
         if (zeros_matter) {
-            if (lane == 0 && a.flagged_total) *(volatile uint32_t*)a.flagged_total = 1u;
-            __builtin_amdgcn_wave_barrier();
-            list.init(sStage, lane, a.k);
-            layer_recompute_row<R>(list, a, b, lane, fs, fe, sTable);
-            list.finish();
+            if (lane == 0) {
+                a.row_flag[b] = 1;
+                if (a.flagged_total) *(volatile uint32_t*)a.flagged_total = 1u;
+            }
+            return;
         }
         write_final<R>(list.q, lane, a.k, 0, a.keys + (uint64_t)b * a.k, a.values + (uint64_t)b * a.k);
         return;
@@ -1904,15 +1845,279 @@ int layer_refresh_run(const LayerRefresh& r, uint32_t batch)
     a.row_bound = r.row_bound; a.row_flag = r.row_flag; a.flagged_total = r.flagged_total;
     a.position = r.position; a.index = r.index; a.fstart = r.fstart; a.fend = r.fend; a.fidx = r.fidx;
     a.keys = r.keys; a.values = r.values;
-    a.X = r.X; a.W = r.W; a.bias = r.bias; a.ldx = r.ldx; a.ldw = r.ldw; a.kdim = r.kdim; a.n = r.n;
+    a.n = r.n;
     a.first_columns = r.first_columns;
     a.fresh = r.fresh ? 1 : 0;
-    a.act = r.act; a.slope = r.slope; a.alpha = r.alpha; a.lambda = r.lambda;
     hipStream_t s = ctx().stream;
     if (a.k <= 64) hipLaunchKernelGGL((layer_refresh_kernel<1>), dim3(batch), dim3(kWave), 0, s, a);
     else if (a.k <= 128) hipLaunchKernelGGL((layer_refresh_kernel<2>), dim3(batch), dim3(kWave), 0, s, a);
     else hipLaunchKernelGGL((layer_refresh_kernel<4>), dim3(batch), dim3(kWave), 0, s, a);
     DSX_LAUNCH_CHECK("layer_refresh_kernel");
+    return DSX_OK;
+}
+
+// Rows of a layer whose lists filled up (thousands of scores tied at the top), or whose result needs the zeros of listed columns: the
+// whole row once more, without any list that could fill up.  The flagged rows are gathered 32 at a time and the columns cut into as many
+// parts as keep the GPU busy; a workgroup walks its part in steps of 512 columns, 128 per wavefront, sums in ascending pairs of k
+// (bias last: as a stored layer), W from memory straight into registers one chunk of eight k ahead.  The scores go through LDS, 128
+// columns at a time, to the wavefront that keeps the row's list, which stages what beats the row's k-th word and merges when more than 32 words wait; the last
+// workgroup of 32 rows to finish merges their parts.  Bound by reading W once per 32 rows from the caches; where no row is flagged, by
+// the launch.
+// 4,096 x 1,024 x 27,278 saturated, every row flagged: 3.05 ms, 75 TFLOP/s, of a call of 16 (12.4 of them the sweep, all of whose
+// scores pass); a wavefront per row that read W for itself took 0.5 s.
+constexpr uint32_t kRedoGrid = 512;   // two workgroups per compute unit
+constexpr int kRedoBlocks = 4;        // blocks of 32 columns per wavefront and step
+constexpr uint32_t kRedoRows = 32, kRedoCols = 128, kRedoSpan = 1024, kRedoStage = kRedoCols + 32, kRedoParts = 128;
+
+struct LayerRedoArgs {
+    const float* X;
+    const float* W;
+    const float* bias;
+    uint32_t ldx, ldw, batch, kdim, n, k;
+    uint32_t act;
+    float slope, alpha, lambda;
+    uint32_t position;
+    const uint32_t* index;
+    const uint64_t* fstart;
+    const uint64_t* fend;
+    const uint32_t* fidx;       // NULL: no filter
+    const uint32_t* row_flag;   // [batch]
+    uint64_t* partial;          // [work items][kRedoRows][k]
+    uint32_t* done;             // [groups of kRedoRows] finished parts, 0 before the launch
+    float* keys;
+    uint32_t* values;
+};
+
+template <int R>
+__global__ __launch_bounds__(256, 2) void layer_redo_kernel(LayerRedoArgs a)
+{
+    using List = WaveTopK<R>;
+    __shared__ float sScore[kRedoRows][kRedoCols + 4];
+    __shared__ uint64_t sStage[kRedoRows][kRedoStage];
+    __shared__ uint64_t sThr[kRedoRows];                    // the row's k-th word so far
+    __shared__ uint32_t sCount[kRedoRows], sMerged[kRedoRows];   // its staged words, whether it has a list yet
+    __shared__ uint32_t sBits[kRedoRows][kRedoSpan / 32];   // listed columns of the span
+    __shared__ uint32_t sRows[kRedoRows], sWave[4], sAny, sLast;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+    const uint32_t l32 = lane & 31, lhi = lane >> 5;
+    if (threadIdx.x == 0) sAny = 0;
+    __syncthreads();
+    uint32_t mine = 0;
+    for (uint32_t b = threadIdx.x; b < a.batch; b += 256) mine += a.row_flag[b] != 0 ? 1u : 0u;
+    if (mine != 0) atomicAdd(&sAny, mine);
+    __syncthreads();
+    const uint32_t flagged = sAny;
+    if (flagged == 0) return;   // the same for the whole grid
+    const uint32_t groups = (flagged + kRedoRows - 1) / kRedoRows, spans = (a.n + kRedoSpan - 1) / kRedoSpan;
+    const uint32_t most = max(1u, min(kRedoParts, gridDim.x / groups)), per = (spans + most - 1) / most, parts = (spans + per - 1) / per;
+
+    for (uint32_t item = blockIdx.x; item < groups * parts; item += gridDim.x) {
+        const uint32_t group = item / parts, part = item % parts;
+        const uint32_t rows = min(flagged - group * kRedoRows, kRedoRows);
+        // the rows themselves: the flagged ones in ascending order, from the (32 group)-th on
+        uint32_t before = 0;
+        for (uint32_t b0 = 0; b0 < a.batch && before < (group + 1) * kRedoRows; b0 += 256) {
+            const bool f = b0 + threadIdx.x < a.batch && a.row_flag[b0 + threadIdx.x] != 0;
+            const uint64_t m = __ballot(f);
+            __syncthreads();   // (sWave and sRows have been read)
+            if (lane == 0) sWave[wave] = (uint32_t)__popcll(m);
+            __syncthreads();
+            uint32_t at = before;
+            for (uint32_t w = 0; w < 4; w++) {
+                if (w < wave) at += sWave[w];
+                before += sWave[w];
+            }
+            at += __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+            if (f && at / kRedoRows == group) sRows[at % kRedoRows] = b0 + threadIdx.x;
+        }
+        if (threadIdx.x < kRedoRows) {
+            sThr[threadIdx.x] = 0;
+            sCount[threadIdx.x] = sMerged[threadIdx.x] = 0;
+        }
+        __syncthreads();
+        const float* x = a.X + (uint64_t)sRows[min(l32, rows - 1)] * a.ldx;   // (lanes beyond the rows repeat the last one)
+        uint64_t* lists = a.partial + (uint64_t)item * kRedoRows * a.k;
+        // (a row's staged words, their number, its k-th word and its list belong to one wavefront)
+        auto merge = [&](uint32_t r, uint32_t staged) {
+            const bool has = sMerged[r] != 0;
+            List list;
+            list.init(sStage[r], lane, a.k);
+            uint64_t* mem = lists + (uint64_t)r * a.k;
+#pragma unroll
+            for (int q = 0; q < R; q++) {
+                const uint32_t p = q * kWave + lane;
+                if (has && p < a.k) list.q[q] = mem[p];
+            }
+            list.count = staged;
+            list.finish();
+#pragma unroll
+            for (int q = 0; q < R; q++) {
+                const uint32_t p = q * kWave + lane;
+                if (p < a.k) mem[p] = list.q[q];
+            }
+            if (lane == 0) {
+                sThr[r] = list.thr;
+                sMerged[r] = 1;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        };
+        const uint32_t end = min(a.n, (part + 1) * per * kRedoSpan);
+        for (uint32_t span = part * per * kRedoSpan; span < end; span += kRedoSpan) {
+            if (a.fidx) {   // (the bits of the span before were last read before the barrier at the end of its last step)
+                for (uint32_t i = threadIdx.x; i < kRedoRows * kRedoSpan / 32; i += 256) (&sBits[0][0])[i] = 0;
+                __syncthreads();
+                for (uint32_t r = wave; r < rows; r += 4) {
+                    uint32_t f = a.position + sRows[r];
+                    if (a.index) f = a.index[f];
+                    const uint64_t fe = a.fend[f];
+                    for (uint64_t t = a.fstart[f] + lane; t < fe; t += kWave) {
+                        const uint32_t c = a.fidx[t];
+                        if (c >= span && c - span < kRedoSpan) atomicOr(&sBits[r][(c - span) >> 5], 1u << ((c - span) & 31));
+                    }
+                }
+                // (the barrier behind the first step's scores comes before they are read)
+            }
+            const uint32_t span_end = min(end, span + kRedoSpan);
+            for (uint32_t step = span; step < span_end; step += kRedoBlocks * kRedoCols) {
+                // block j of a wavefront: columns step + 128 j + 32 wave + l32
+                const float* w = a.W + (uint64_t)lhi * a.ldw;
+                uint32_t wcol[kRedoBlocks];
+#pragma unroll
+                for (int j = 0; j < kRedoBlocks; j++) wcol[j] = min(step + kRedoCols * j + 32 * wave + l32, a.n - 1);
+                struct Stage {
+                    float x[8], w[4][kRedoBlocks];
+                };
+                auto load = [&](Stage& s, uint32_t k0) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int t = 0; t < 4; t++)
+#pragma unroll
+                        for (int j = 0; j < kRedoBlocks; j++) s.w[t][j] = w[(uint64_t)(k0 + 2 * t) * a.ldw + wcol[j]];
+#pragma unroll
+                    for (int e = 0; e < 8; e += 4) {
+                        const float4u v = *reinterpret_cast<const float4u*>(x + k0 + e);
+                        s.x[e] = v.x; s.x[e + 1] = v.y; s.x[e + 2] = v.z; s.x[e + 3] = v.w;
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                };
+                floatx16 acc[kRedoBlocks];
+#pragma unroll
+                for (int j = 0; j < kRedoBlocks; j++)
+#pragma unroll
+                    for (int v = 0; v < 16; v++) acc[j][v] = 0.0f;
+                auto multiply = [&](const Stage& s) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int t = 0; t < 4; t++) {
+                        const float xv = lhi ? s.x[2 * t + 1] : s.x[2 * t];
+#pragma unroll
+                        for (int j = 0; j < kRedoBlocks; j++) acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(xv, s.w[t][j], acc[j], 0, 0, 0);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                };
+                const uint32_t chunks = a.kdim / 8, rest = a.kdim - chunks * 8;
+                if (chunks != 0) {
+                    const uint32_t last = (chunks - 1) * 8;
+                    Stage s0, s1;
+                    load(s0, 0);
+                    uint32_t k0 = 0, left = chunks;
+                    for (; left >= 2; left -= 2) {   // (the last chunk is requested again and not used)
+                        load(s1, k0 + 8);
+                        multiply(s0);
+                        load(s0, min(k0 + 16, last));
+                        multiply(s1);
+                        k0 += 16;
+                    }
+                    if (left) multiply(s0);
+                }
+                if (rest != 0) {
+                    Stage s;
+#pragma unroll
+                    for (int t = 0; t < 4; t++)
+#pragma unroll
+                        for (int j = 0; j < kRedoBlocks; j++) s.w[t][j] = (2 * t + lhi < rest) ? w[(uint64_t)(chunks * 8 + 2 * t) * a.ldw + wcol[j]] : 0.0f;
+#pragma unroll
+                    for (int e = 0; e < 8; e++) s.x[e] = ((uint32_t)e < rest) ? x[chunks * 8 + e] : 0.0f;
+                    multiply(s);
+                }
+#pragma unroll
+                for (int j = 0; j < kRedoBlocks; j++) {
+                    const uint32_t c0 = step + kRedoCols * j;
+                    if (c0 >= span_end) break;   // the same for the whole workgroup
+#pragma unroll
+                    for (int v = 0; v < 16; v++) sScore[8 * (v / 4) + 4 * lhi + v % 4][32 * wave + l32] = acc[j][v];
+                    __syncthreads();
+                    float bias[2];
+#pragma unroll
+                    for (int h = 0; h < 2; h++) bias[h] = (a.bias && c0 + h * kWave + lane < span_end) ? a.bias[c0 + h * kWave + lane] : 0.0f;
+#pragma unroll 1
+                    for (uint32_t r = wave; r < rows; r += 4) {
+                        const uint64_t thr = sThr[r];
+                        uint32_t count = sCount[r];   // wave-uniform
+#pragma unroll 1
+                        for (int h = 0; h < 2; h++) {
+                            const uint32_t c = c0 + h * kWave + lane;
+                            float y = activate_rt(sScore[r][h * kWave + lane] + (h ? bias[1] : bias[0]), a.act, a.slope, a.alpha, a.lambda);
+                            // a listed column keeps its place with score * 0 (utils/Filters.cpp:62), once however often it is listed
+                            if (a.fidx && ((sBits[r][(c - span) >> 5] >> (c & 31)) & 1u)) y *= 0.0f;
+                            const uint64_t word = pack_score(y, c);
+                            const bool cand = c < span_end && y == y && word > thr;
+                            const uint64_t m = __ballot(cand);
+                            if (cand) sStage[r][count + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))] = word;
+                            count += (uint32_t)__popcll(m);
+                        }
+                        if (count > kRedoStage - kRedoCols) {
+                            merge(r, count);
+                            count = 0;
+                        }
+                        if (lane == 0) sCount[r] = count;
+                    }
+                    __syncthreads();   // the scores have been read
+                }
+            }
+        }
+        for (uint32_t r = wave; r < rows; r += 4) merge(r, sCount[r]);
+        // The last part of the group to finish merges them all.  (Release: the lists are in memory before the count; acquire: they are
+        // read after it.  Workgroups of a group may run on different XCDs, whose L2s are not kept coherent.)
+        __threadfence();
+        __syncthreads();
+        if (threadIdx.x == 0) sLast = atomicAdd(&a.done[group], 1u) + 1 == parts ? 1u : 0u;
+        __syncthreads();
+        if (sLast != 0) {
+            __threadfence();
+            for (uint32_t r = wave; r < rows; r += 4) {
+                List list;
+                list.init(sStage[r], lane, a.k);
+                for (uint32_t s = 0; s < parts; s++) {
+                    const uint64_t* src = a.partial + ((uint64_t)(group * parts + s) * kRedoRows + r) * a.k;
+                    for (uint32_t p0 = 0; p0 < a.k; p0 += kWave) {
+                        const uint64_t word = (p0 + lane < a.k) ? src[p0 + lane] : 0ull;
+                        list.stage_only(word != 0, word);
+                        list.finish();   // (a staging row has room for 160 words)
+                    }
+                }
+                const uint64_t row = sRows[r];
+                write_final<R>(list.q, lane, a.k, 0, a.keys + row * a.k, a.values + row * a.k);
+            }
+        }
+        __syncthreads();   // (sRows is written again)
+    }
+}
+
+uint64_t layer_redo_words(uint32_t batch, uint32_t k) { return (uint64_t)std::max(kRedoGrid, (batch + kRedoRows - 1) / kRedoRows) * kRedoRows * k; }
+uint32_t layer_redo_groups(uint32_t batch) { return (batch + kRedoRows - 1) / kRedoRows; }
+
+int layer_redo_run(const LayerRedo& r, uint32_t batch)
+{
+    LayerRedoArgs a{};
+    a.X = r.X; a.W = r.W; a.bias = r.bias; a.ldx = r.ldx; a.ldw = r.ldw; a.batch = batch; a.kdim = r.kdim; a.n = r.n; a.k = r.k;
+    a.act = r.act; a.slope = r.slope; a.alpha = r.alpha; a.lambda = r.lambda;
+    a.position = r.position; a.index = r.index; a.fstart = r.fstart; a.fend = r.fend; a.fidx = r.fidx;
+    a.row_flag = r.row_flag; a.partial = r.partial; a.done = r.done; a.keys = r.keys; a.values = r.values;
+    hipStream_t s = ctx().stream;
+    if (a.k <= 64) hipLaunchKernelGGL((layer_redo_kernel<1>), dim3(kRedoGrid), dim3(256), 0, s, a);
+    else if (a.k <= 128) hipLaunchKernelGGL((layer_redo_kernel<2>), dim3(kRedoGrid), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((layer_redo_kernel<4>), dim3(kRedoGrid), dim3(256), 0, s, a);
+    DSX_LAUNCH_CHECK("layer_redo_kernel");
     return DSX_OK;
 }
 
