@@ -208,7 +208,7 @@ int knn_f16_candidates_run(const void* queries16, const void* items16, uint32_t 
                            uint64_t* seg, uint32_t* seg_count, uint32_t seg_words, int mode, uint32_t* chunks_used);
 // 16-bit screening of candidates for the fp32 searches (dsx_screen.hip): the table's two row-major copies (f16, fp32), the rows in f16
 // and the lists of a sweep.  screen_prepare lays them out (flag: one word, or one per row for layers, set where the error of a 16-bit
-// sum has no bound; told: a host-visible word set with it); screen_candidates screens ncols columns from cand.col_offset on and leaves
+// sum has no bound; told: a host-visible word set with it; first: the columns that give a layer its first bounds); screen_candidates screens ncols columns from cand.col_offset on and leaves
 // the fp32 scores of what passed in cand's lists.  All results come from there, so that equal columns have equal scores: `first` marks
 // the range whose bounds were taken from another kernel's sums (it starts at column 0).
 struct ScreenWorkspace {
@@ -227,7 +227,7 @@ struct ScreenWorkspace {
 bool screen_takes(uint32_t batch, uint32_t dim, uint64_t n, bool layer);
 ScreenWorkspace screen_layout(void* base, uint32_t batch, uint32_t dim, uint64_t n, bool layer, uint32_t list_words);
 int screen_prepare(const ScreenWorkspace& w, const float* X, uint32_t ldx, uint32_t batch, const float* W, uint64_t ldw, const float* bias,
-                   uint64_t n, uint32_t dim, bool layer, uint32_t* flag, uint32_t* told);
+                   uint64_t n, uint32_t dim, bool layer, uint32_t first, uint32_t* flag, uint32_t* told);
 int screen_candidates(const ScreenWorkspace& w, const float* X, uint32_t ldx, uint32_t batch, uint32_t dim, bool layer, const float* bias,
                       uint32_t ncols, const CandArgs& cand, bool report_overflow, bool first);
 

@@ -251,7 +251,7 @@ static int knn_search_candidates(const KnnWorkspace& w, const KnnOperands& op, u
     if (!ctx().knobs.knn_block_columns) done = std::min<uint32_t>(done, screened ? 8192u : std::max<uint32_t>(1024, cb / 4 / 1024 * 1024));
     t.start(s);
     int rc = DSX_OK;
-    if (screened) rc = screen_prepare(w.screen, op.queries, op.dim, num_queries, op.items, op.rows_padded, nullptr, M, op.dim, false, w.overflow, nullptr);
+    if (screened) rc = screen_prepare(w.screen, op.queries, op.dim, num_queries, op.items, op.rows_padded, nullptr, M, op.dim, false, 0, w.overflow, nullptr);
     if (rc) return rc;
     FcOrder order;
     order.as_candidates = !screened;

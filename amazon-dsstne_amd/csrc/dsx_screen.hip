@@ -10,12 +10,14 @@
 // roundoff u = 2^-11, 2^-25 absolute below the normal range), fp32 accumulation:
 //   |s' - s| <= (2u + u^2) |x| |w| + 2^-25 sqrt(d) (|x| + |w|) + d 2^-50 + (3 d + 16) 2^-24 |x| |w|      (Cauchy-Schwarz; |.| = 2-norm)
 // (d 2^-50: both operands' absolute roundings together, all there is to go by where every component is near 2^-25)
-// The matrix instructions keep subnormal operands.  Norms above 65,504 (a component might overflow) set a flag instead.
+// The matrix instructions keep subnormal operands.  A row's norm above 65,504 (a component might overflow) sets a flag instead.
 //
-//   ITEM_NORM = false (nearest neighbours): |w| is taken at its largest over all columns; the search reads the flag and, where lists
-//     filled up for it, runs again without screening.
+//   ITEM_NORM = false (nearest neighbours): |w| is taken at its largest over all columns, and a norm above 65,504 sets the flag too; the
+//     search reads the flag and, where lists filled up for it, runs again without screening.
 //   ITEM_NORM = true (layers): one more component adds (2u + ...) |x| |w| of its own column to every sum, which makes the sums upper
-//     bounds of the scores whatever the spread of the columns' norms; three more components carry the bias in three f16 pieces.
+//     bounds of the scores whatever the spread of the columns' norms; three more components carry the bias in three f16 pieces, raised
+//     by what a sum with it can be wrong by.  Items are masked with biases of -1e9 or -inf: a bias below -60,000 is taken as that, which
+//     bounds the score from above all the same.  A column above 60,000 (bias or norm) gets a bias of +inf and always passes.
 //
 // Preparing a table of n columns of d components reads 4 and writes 6 bytes per element, on every call (nothing is kept that could
 // go stale).  4,096 queries x 1,000,000 x 128, top 100: search 8.9 ms in fp32 -> 2.9 (0.28 preparation, 1.3 f16 products at
@@ -28,7 +30,7 @@
 namespace dsx {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-constexpr float kF16Max = 65504.0f;
+constexpr float kF16Max = 65504.0f, kScreenMax = 60000.0f;
 constexpr int kScreenExtra = 4;   // components a layer adds: bias in three pieces, the error term
 
 uint32_t screen_ld(uint32_t dim, bool layer) { return knn_f16_ld(dim + (layer ? kScreenExtra : 0)); }
@@ -37,13 +39,14 @@ uint32_t screen_pitch32(uint32_t dim) { return (dim + 3) / 4 * 4; }
 // Relative part of the error, with room for the rounding of the norms themselves.
 __device__ __forceinline__ float screen_relative(uint32_t dim) { return 9.765625e-4f * 1.01f + (4.0f * (float)dim + 64.0f) * 5.9604645e-8f; }
 
-// stats: [0] largest norm of a column, [1] largest |bias| (bits of non-negative floats; NaN columns and biases have no part in it:
-// their scores are NaN on every path)
+// stats: [0] largest norm of a column, of a layer's first block's columns only (the bits of a non-negative float; NaN columns have no
+// part in it: their scores are NaN on every path)
 struct ScreenItemsArgs {
     const float* W;       // [dim][ldw]
     const float* bias;    // layers: [n], or NULL
     uint64_t ldw;
     uint32_t n, dim, ld, pitch32;
+    uint32_t first;       // columns that stats[0] is taken over
     _Float16* out16;      // [n rounded up to 256][ld], zero filled
     float* out32;         // [n][pitch32], zero filled beyond dim
     uint32_t* stats;
@@ -95,20 +98,25 @@ __global__ __launch_bounds__(256) void screen_items_kernel(ScreenItemsArgs a)
         for (int d = 1; d < 64; d *= 2) v = fmaxf(v, __shfl_xor(v, d));
         if (l == 0 && __float_as_uint(v) > *(volatile uint32_t*)to) atomicMax(to, __float_as_uint(v));
     };
-    if (q == 0) raise(&a.stats[0], norm);
+    if (q == 0) raise(&a.stats[0], col0 + l < a.first ? norm : 0.0f);
     if constexpr (ITEM_NORM) {
-        const float b = (a.bias && valid) ? a.bias[col0 + l] : 0.0f;
-        if (q == 1) raise(&a.stats[1], fabsf(b));
-        const _Float16 hi = (_Float16)b;
-        const float r1 = b - (float)hi;
+        const float given = (a.bias && valid) ? a.bias[col0 + l] : 0.0f;
+        const bool always = norm > kScreenMax || given > kScreenMax;
+        float b = fmaxf(given, -kScreenMax);
+        // upwards by: the roundings of a sum that holds it, and the absolute roundings of x against this column
+        b += fabsf(b) * (((float)a.dim + 64.0f) * 2.3841858e-7f + 1e-6f) + 2.9802322e-8f * 1.01f * sqrtf((float)a.dim + 4.0f) * norm;
+        const _Float16 hi = always ? (_Float16)__builtin_inff() : (_Float16)b;
+        const float r1 = always ? 0.0f : b - (float)hi;
         const _Float16 mid = (_Float16)r1, lo = (_Float16)(r1 - (float)mid);
-        const _Float16 error = (_Float16)(norm * 0.03125f * 1.002f + 1e-7f);   // rounded up: half an ulp is at most 2^-11
+        const _Float16 error = always ? (_Float16)0.0f : (_Float16)(norm * 0.03125f * 1.002f + 1e-7f);   // rounded up: half an ulp is at most 2^-11
+        if (always)   // (its components may be infinite in f16; what the loop above wrote was ordered before by the barrier)
+            for (uint32_t p = 8 * q; p < whole; p += 32) *reinterpret_cast<half8*>(a.out16 + (uint64_t)(col0 + l) * a.ld + p) = half8{};
         for (uint32_t p = whole + 8 * q; p < a.ld; p += 32) {
             half8 h;
 #pragma unroll
             for (int e = 0; e < 8; e++) {
                 const uint32_t d = p + e;
-                if (d < a.dim) h[e] = valid ? (_Float16)a.W[(uint64_t)d * a.ldw + col0 + l] : (_Float16)0.0f;
+                if (d < a.dim) h[e] = valid && !always ? (_Float16)a.W[(uint64_t)d * a.ldw + col0 + l] : (_Float16)0.0f;
                 else h[e] = d == a.dim ? hi : d == a.dim + 1 ? mid : d == a.dim + 2 ? lo : d == a.dim + 3 ? error : (_Float16)0.0f;
             }
             *reinterpret_cast<half8*>(a.out16 + (uint64_t)(col0 + l) * a.ld + p) = h;
@@ -151,16 +159,17 @@ __global__ __launch_bounds__(256) void screen_rows_kernel(ScreenRowsArgs a)
         a.out16[(uint64_t)row * a.ld + d] = (_Float16)x;
     }
     if (!valid || lane != 0) return;
-    const float most = __uint_as_float(a.stats[0]), bias = ITEM_NORM ? __uint_as_float(a.stats[1]) : 0.0f;
-    float eps = 2.9802322e-8f * 1.01f * sqrtf((float)a.dim + 4.0f) * (norm + most);
-    if constexpr (ITEM_NORM) eps += ((float)a.dim + 64.0f) * 2.3841858e-7f * bias + 1e-6f * bias + 1e-7f;
+    const float most = __uint_as_float(a.stats[0]);
+    float eps = 2.9802322e-8f * 1.01f * sqrtf((float)a.dim + 4.0f) * (ITEM_NORM ? norm : norm + most);
+    if constexpr (ITEM_NORM) eps += 1e-7f;   // (the bias: its last piece is good to 2^-25)
     else eps += screen_relative(a.dim) * norm * most + (float)a.dim * 8.8817842e-16f * 1.01f;   // (a layer's 1e-7 covers the last term)
     a.eps[row] = eps;
     // The k columns that set the first bound are scored again in another order: d + d / 16 + 5 roundings of 2^-24 of |x| |w| apart at most,
-    // four more of |x| |w| + |b| for the bias.  (Nearest neighbours: inside the 4 d + 64 of screen_relative.)
-    if constexpr (ITEM_NORM) a.slack[row] = ((1.25f * (float)a.dim + 16.0f) * 5.9604645e-8f * norm * most + 2.3841858e-7f * bias) * 1.01f;
+    // and for the bias 2^-22 of |b| <= |x| |w| + |z|, whose |z| part the bounds' kernel takes off (a column that lies above the bound
+    // keeps above it by less |z| than it has more).  (Nearest neighbours: inside the 4 d + 64 of screen_relative.)
+    if constexpr (ITEM_NORM) a.slack[row] = (1.25f * (float)a.dim + 24.0f) * 5.9604645e-8f * 1.01f * norm * most;
     // (a NaN in the row: its scores are NaN everywhere, there is nothing to miss)
-    const bool bad = norm > kF16Max || most > kF16Max || bias > kF16Max;
+    const bool bad = norm > kF16Max || (!ITEM_NORM && most > kF16Max);
     if (bad) {
         a.flag[ITEM_NORM ? row : 0] = 1;
         if (a.told) *(volatile uint32_t*)a.told = 1u;
@@ -308,12 +317,12 @@ ScreenWorkspace screen_layout(void* base, uint32_t batch, uint32_t dim, uint64_t
 __global__ void screen_clear_kernel(uint32_t* stats) { stats[threadIdx.x] = 0; }
 
 int screen_prepare(const ScreenWorkspace& w, const float* X, uint32_t ldx, uint32_t batch, const float* W, uint64_t ldw, const float* bias,
-                   uint64_t n, uint32_t dim, bool layer, uint32_t* flag, uint32_t* told)
+                   uint64_t n, uint32_t dim, bool layer, uint32_t first, uint32_t* flag, uint32_t* told)
 {
     hipStream_t s = ctx().stream;
     hipLaunchKernelGGL(screen_clear_kernel, dim3(1), dim3(64), 0, s, w.stats);
     ScreenItemsArgs i{};
-    i.W = W; i.bias = bias; i.ldw = ldw; i.n = (uint32_t)n; i.dim = dim;
+    i.W = W; i.bias = bias; i.ldw = ldw; i.n = (uint32_t)n; i.dim = dim; i.first = layer ? first : (uint32_t)n;
     i.ld = screen_ld(dim, layer); i.pitch32 = screen_pitch32(dim);
     i.out16 = (_Float16*)w.items16; i.out32 = w.rows32; i.stats = w.stats;
     const dim3 grid((uint32_t)(knn_f16_rows(n) / 64));

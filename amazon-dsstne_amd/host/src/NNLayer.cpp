@@ -178,9 +178,10 @@ void NNLayer::ForwardPropagateFullyConnected(uint32_t position, uint32_t batch, 
             if (_bDeferOutput && !bHeld && TopKFusionPays(batch, 1) && !w->_bTransposed && _vOutgoingLayer.empty() && _vOutgoingSkip.empty() &&
                 dsx_fc_topk_supported(src->_stride, src->GetUnitBuffer(), (uint32_t)_activation, &params, NULL)) {
                 if (dsx_fc_topk_flagged_for(wsrc->_pbWeight->_pDevData, 0)) {
-                    // rows whose survivor lists filled up had to be computed again: this data (thousands of scores tied at the
-                    // top of a row) is served better by the stored layer and the scanning top-K
-                    printf("NNLayer::ForwardPropagate: scores of layer %s tie in their thousands; its result is stored from now on.\n", _name.c_str());
+                    // rows whose survivor lists filled up (thousands of scores tied at the top), or whose inputs f16 cannot hold, had
+                    // to be computed again: such data is served better by the stored layer and the scanning top-K
+                    printf("NNLayer::ForwardPropagate: rows of layer %s had to be computed twice for their top-K; its result is stored from now on.\n",
+                           _name.c_str());
                     _bDeferOutput = false;
                 } else {
                     _deferred = true;

@@ -173,3 +173,30 @@ def test_without_room_for_the_copies_of_the_table(pkg, dsx, rng):
         assert np.array_equal(s, rs) and np.array_equal(i, ri) and dsx.dsx_knn_last_search_path() == 0
     finally:
         dsx.dsx_testing_set_allocation_limit(0)
+
+
+@pytest.mark.parametrize("act,mask", [(0, -1e9), (0, -np.inf), (3, -1e9), (1, -3e38), (2, -70000.0)])
+def test_masked_columns(pkg, dsx, rng, act, mask):
+    """Retired items are masked by their biases, new ones pushed: neither makes a row be computed again, and the others' bounds do not
+    depend on them.  A few columns (behind the first block) lie above f16's range themselves."""
+    batch, kdim, n, k = 1024, 128, 40000, 30
+    print("[case] masked columns act=%d mask=%g" % (act, mask), flush=True)
+    X = np.maximum(rng.standard_normal((batch, kdim), dtype=np.float32), 0)
+    W = rng.standard_normal((kdim, n), dtype=np.float32) * np.float32(0.05)
+    bias = (rng.standard_normal(n) * 0.3 - (0.5 if act == 2 else 2)).astype(np.float32)
+    bias[rng.random(n) < 0.3] = np.float32(mask)
+    bias[[3, 20000, 39999]] = np.float32(-65000.0)
+    if act < 2:
+        bias[[7, 30000]] = np.float32(1e6)
+        W[:, 25000] *= np.float32(1e7)
+    dX, dW, db = dev(pkg, X), dev(pkg, W), dev(pkg, bias)
+    keys, vals = pkg.DeviceArray((batch, k), np.float32), pkg.DeviceArray((batch, k), np.uint32)
+    dsx.dsx_fc_topk_flagged(1)
+    pkg.check(dsx.dsx_fc_topk(dX.ptr, kdim, dW.ptr, db.ptr, batch, kdim, n, act, None, k, keys.ptr, vals.ptr, 0, None, None, None, None))
+    pkg.check(dsx.dsx_sync())
+    assert dsx.dsx_fc_topk_flagged(1) == 0
+    with np.errstate(over="ignore"):
+        z = X.astype(np.float64) @ W.astype(np.float64) + bias
+        y = {0: lambda v: 1 / (1 + np.exp(-v)), 1: np.tanh, 2: lambda v: np.maximum(v, 0), 3: lambda v: v}[act](z)
+    # |x| |w| + |b| below 20 for the columns whose scores are not flat: kdim + 8 roundings of 2^-24 of it, 1e-6 for the activations
+    check_against_float64(keys.numpy(), vals.numpy(), y, k, (kdim + 8) * 20 * 2.0 ** -24 / 4 + 1e-6)
