@@ -103,7 +103,8 @@ static KnnWorkspace knn_layout(void* base, uint32_t rows_padded, uint32_t num_qu
     }
     if (split) p += align256((size_t)split_plane_bytes(num_queries, dim));
     w.screen = ScreenWorkspace{};
-    if (screen && !f16 && !split && screen_takes(num_queries, dim, rows_padded, false)) {
+    if (screen && !f16 && !split && screen_takes(num_queries, dim, rows_padded, false) &&
+        screen_search_pays(num_queries, dim, rows_padded, k, blocks == 1, 1.0f)) {
         w.screen = screen_layout(p, num_queries, dim, rows_padded, false, kCandCap);
         p += w.screen.bytes;
     }
@@ -305,6 +306,12 @@ extern "C" {
 int dsx_testing_set_knn_block_columns(uint32_t columns)
 {
     ctx().knobs.knn_block_columns = columns;
+    return DSX_OK;
+}
+
+int dsx_testing_set_knn_screen(int mode)
+{
+    ctx().knobs.knn_screen = mode;
     return DSX_OK;
 }
 

@@ -24,6 +24,7 @@
 // 0.8 PFLOP/s, 0.55 fp32 scores of 1,200 candidates per query); output layer 4,096 x 512 x 1,000,000, top 100: 31.4 ms -> 9.3 (1.3,
 // 6.3, 0.9).  What bounds it: the sweep of dsx_knn_f16.hip.
 #include <algorithm>
+#include <cmath>
 #include "dsx_device.h"
 #include "dsx_internal.h"
 
@@ -276,13 +277,37 @@ __global__ __launch_bounds__(256) void screen_rescore_kernel(ScreenRescoreArgs a
     if (threadIdx.x == 0) a.cand_count[b] = total;
 }
 
-// Where screening pays: the preparation costs what about 130 rows' fp32 products do, and the candidates' scores and the extra
-// launches about 150 us (us, screened / fp32: 512 x 64 x 300,000 top 10 362 / 298, 512 x 256 x 300,000 642 / 734, 1,024 x 512 x 60,000
-// 398 / 509, 4,096 x 128 x 60,000 413 / 716).  Limits: the row in LDS, and 8 GiB for the two copies of the table.
+// What can be screened, and for layers whether it pays: the preparation costs what about 130 rows' fp32 products do, and the
+// candidates' scores and the extra launches about 150 us (us, screened / fp32, top 10: 512 x 64 x 300,000 362 / 298, 512 x 256 x 300,000
+// 642 / 734, 1,024 x 512 x 60,000 398 / 509, 4,096 x 128 x 60,000 413 / 716).  Limits: the row in LDS, and 8 GiB for the two copies of
+// the table.
 bool screen_takes(uint32_t batch, uint32_t dim, uint64_t n, bool layer)
 {
     const uint64_t bytes = knn_f16_rows(n) * ((uint64_t)screen_ld(dim, layer) * 2 + (uint64_t)screen_pitch32(dim) * 4);
     return batch >= 512 && dim >= 32 && dim <= 4096 && (!layer || (uint64_t)batch * dim >= 131072) && n >= (layer ? 16384 : 65536) && bytes <= ((uint64_t)8 << 30);
+}
+
+// Nearest neighbours: whether screening is the faster way.  Both sides as fitted to 336 measured searches of normalised random vectors (us;
+// 512 to 4,096 queries, 32 to 1,024 components, 65,536 to 1,000,000 items, k 10 to 256): fp32 within 13 %, block by block or with
+// candidate lists; screened within 45 %, which is why it has to be ahead by a tenth.  None of the 336 is slower than without
+// screening, 1.4 % of the time they could take is left (512 x 32 x 65,536 top 256 486 screened / 140 fp32, 2,048 x 32 x 300,000 top
+// 100 821 / 681, 512 x 128 x 300,000 top 100 544 / 569, 2,048 x 128 x 150,000 top 10 385 / 755, 4,096 x 128 x 1,000,000 top 100 2,368 /
+// 8,789).
+// norm_ratio: the largest norm of an item over the average one.  A bound is lowered by 2^-10 of the largest, about
+// 2^-10 sqrt(dim) norm_ratio of the scores' spread; where the k best lie, about four of it out, that many more candidates pass:
+// exp(4 * 2^-10 sqrt(dim) norm_ratio) times as many.  A first range leaves 5 k of them; lists hold 4,096.
+bool screen_search_pays(uint32_t batch, uint32_t dim, uint64_t n, uint32_t k, bool blocks, float norm_ratio)
+{
+    const double q = batch, d = dim, ld = std::max(d, 64.0), m = (double)n;
+    const double more = std::exp(std::min(20.0, 4.0 * std::sqrt(d) * (double)norm_ratio / 1024.0));
+    if (5.0 * k * more > 3600.0) return false;
+    if (ctx().knobs.knn_screen) return true;
+    const double ranges = 1.0 + std::max(1.0, std::ceil(std::log(m / 40960.0) / std::log(5.0))), fold = std::log(m / 8192.0) / std::log(5.0);
+    const double fp32 = blocks ? 1.464e-8 * q * m * d + 1.656e-6 * q * m + 4.3e-5 * q * k + 0.265 * k
+                               : 120.0 + 1.447e-8 * q * m * d + 2.56e-7 * q * m + 2.37e-4 * q * k + 0.6 * k;
+    const double screened = 90.0 + 30.0 * ranges + 3.2e-6 * m * ld + 2e-9 * q * m * ld + 1e-7 * q * m +
+                            more * (q * k * fold * (4e-4 + 1.9e-6 * ld) + 0.5 * k * ranges);
+    return fp32 > 1.1 * screened;
 }
 
 static inline size_t align256(size_t x) { return (x + 255) / 256 * 256; }

@@ -11,6 +11,14 @@ from test_gpu_screen import search
 pytestmark = pytest.mark.gpu
 
 
+@pytest.fixture(autouse=True)
+def screened(dsx):
+    """Searches that are small for a test are screened too (by default only where that is expected to be faster)."""
+    dsx.dsx_testing_set_knn_screen(1)
+    yield
+    dsx.dsx_testing_set_knn_screen(0)
+
+
 def with_twins(rng, n, dim, front, back, pairs):
     """n normal rows, `pairs` of which are copied from the first `front` rows to somewhere behind row `back`, scaled so that many rows
     of the result hold them.  Returns the rows and twin[row] = the lower row of its pair (its own number: no pair)."""

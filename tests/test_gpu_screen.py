@@ -10,6 +10,14 @@ from test_oracle import random_csr
 pytestmark = pytest.mark.gpu
 
 
+@pytest.fixture(autouse=True)
+def screened(dsx):
+    """Searches that are small for a test are screened too (by default only where that is expected to be faster)."""
+    dsx.dsx_testing_set_knn_screen(1)
+    yield
+    dsx.dsx_testing_set_knn_screen(0)
+
+
 def search(pkg, dsx, items, queries, k):
     n, dim = items.shape
     rows = (n + 7) // 8 * 8
@@ -71,7 +79,14 @@ def test_operands_that_f16_holds_badly(pkg, dsx, rng, form):
     s, i = search(pkg, dsx, items, q, k)
     full = q.astype(np.float64) @ items.astype(np.float64).T
     # dim products, each rounding at most 2^-24 of |q| |w|: rows are compared in units of |q| max |w|
-    scale = np.linalg.norm(q.astype(np.float64), axis=1)[:, None] * np.nanmax(np.linalg.norm(items.astype(np.float64), axis=1))
+    norms = np.linalg.norm(items.astype(np.float64), axis=1)
+    length = np.linalg.norm(q.astype(np.float64), axis=1)[:, None]
+    if form == "one large item":       # (its own scores in units of its own norm, the others in units of theirs)
+        at, large = np.take_along_axis(full, i.astype(np.int64), axis=1), i == n // 2
+        assert large.sum() > queries // 4 and (np.abs(s - at) / (length * norms[n // 2]))[large].max() <= dim * 2.0 ** -24
+        s = np.where(large, at, s)
+        norms[n // 2] = 0.0
+    scale = length * np.nanmax(norms)
     check_against_float64(s / scale, i, full / scale, k, dim * 2.0 ** -24)
 
 
@@ -200,3 +215,14 @@ def test_masked_columns(pkg, dsx, rng, act, mask):
         y = {0: lambda v: 1 / (1 + np.exp(-v)), 1: np.tanh, 2: lambda v: np.maximum(v, 0), 3: lambda v: v}[act](z)
     # |x| |w| + |b| below 20 for the columns whose scores are not flat: kdim + 8 roundings of 2^-24 of it, 1e-6 for the activations
     check_against_float64(keys.numpy(), vals.numpy(), y, k, (kdim + 8) * 20 * 2.0 ** -24 / 4 + 1e-6)
+
+
+@pytest.mark.parametrize("n,queries,dim,k,path", [(65536, 512, 32, 10, 0), (150000, 1000, 128, 10, 1), (150000, 512, 64, 256, 0)])
+def test_searches_are_screened_where_that_is_faster(pkg, dsx, rng, n, queries, dim, k, path):
+    dsx.dsx_testing_set_knn_screen(0)
+    items = rng.integers(-3, 4, size=(n, dim)).astype(np.float32)
+    q = rng.integers(-3, 4, size=(queries, dim)).astype(np.float32)
+    s, i = search(pkg, dsx, items, q, k)
+    assert dsx.dsx_knn_last_search_path() == path
+    rs, ri = best(q @ items.T, k)
+    assert np.array_equal(s, rs) and np.array_equal(i, ri)
