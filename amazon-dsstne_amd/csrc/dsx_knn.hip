@@ -235,10 +235,40 @@ static int knn_search_blocks(const KnnWorkspace& w, const KnnOperands& op, uint3
     return rc;
 }
 
+// What the preparation of a screened search found, read back while the first block runs (pinned).
+struct KnnNotes {
+    float largest, sum;
+    uint32_t number, flag;
+};
+static KnnNotes* g_knn_notes = nullptr;
+static hipEvent_t g_knn_noted = nullptr;
+
+static void knn_notes_release()
+{
+    if (g_knn_notes) hipHostFree(g_knn_notes);
+    if (g_knn_noted) hipEventDestroy(g_knn_noted);
+    g_knn_notes = nullptr;
+    g_knn_noted = nullptr;
+}
+
+static int knn_notes_request(const KnnWorkspace& w, hipStream_t s)
+{
+    if (!g_knn_noted) {
+        at_shutdown(knn_notes_release);
+        if (!g_knn_notes) DSX_HIP(hipHostMalloc((void**)&g_knn_notes, sizeof(KnnNotes), hipHostMallocDefault));
+        DSX_HIP(hipEventCreateWithFlags(&g_knn_noted, hipEventDisableTiming));
+    }
+    DSX_HIP(hipMemcpyAsync(g_knn_notes, w.screen.stats, 3 * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+    DSX_HIP(hipMemcpyAsync(&g_knn_notes->flag, w.overflow, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+    DSX_HIP(hipEventRecord(g_knn_noted, s));
+    return DSX_OK;
+}
+
 // First block as above, the rest in candidate mode, screened in 16 bits where asked for (fp32 storage).  *overflowed tells the caller
-// to redo the search without screening, or block by block.
+// to redo the search without screening, or block by block; *unfit (screened only), that the preparation found the table or the queries
+// unfit for screening (norms beyond f16's range, or one so large that the others' bounds are worth nothing) and the search ended there.
 static int knn_search_candidates(const KnnWorkspace& w, const KnnOperands& op, uint32_t M, uint32_t num_queries, uint32_t k, float* scores,
-                                 uint32_t* indexes, KnnTimer& t, bool screened, bool* overflowed)
+                                 uint32_t* indexes, KnnTimer& t, bool screened, bool* overflowed, bool* unfit)
 {
     hipStream_t s = ctx().stream;
     const uint32_t cb = knn_block_columns(op.rows_padded, num_queries);
@@ -253,6 +283,7 @@ static int knn_search_candidates(const KnnWorkspace& w, const KnnOperands& op, u
     t.start(s);
     int rc = DSX_OK;
     if (screened) rc = screen_prepare(w.screen, op.queries, op.dim, num_queries, op.items, op.rows_padded, nullptr, M, op.dim, false, 0, w.overflow, nullptr);
+    if (rc == DSX_OK && screened) rc = knn_notes_request(w, s);
     if (rc) return rc;
     FcOrder order;
     order.as_candidates = !screened;
@@ -267,7 +298,14 @@ static int knn_search_candidates(const KnnWorkspace& w, const KnnOperands& op, u
     // Screened, the block's scores give the bounds and nothing else: what passes is scored by one kernel wherever it lies (equal items
     // are to tie, and its sums have not this block's order), so the first range starts at column 0.
     const uint32_t seen = done;
-    if (screened) done = 0;
+    if (screened) {
+        done = 0;
+        DSX_HIP(hipEventSynchronize(g_knn_noted));   // (the first block is still running)
+        const KnnNotes notes = *g_knn_notes;
+        const float average = notes.number != 0 ? notes.sum / (float)notes.number : 0.0f;
+        *unfit = notes.flag != 0 || (notes.largest > 0.0f && !screen_search_pays(num_queries, op.dim, M, k, M <= cb, notes.largest / average));
+        if (*unfit) return DSX_OK;
+    }
     while (done < M) {
         const bool first = screened && done == 0;
         // a multiple of the tile width keeps every range's first column 16-byte aligned
@@ -403,12 +441,14 @@ static int knn_search_common(KnnOperands& op, uint32_t padding, uint32_t num_que
     // (few queries against an fp32 table stay with the blocks, however many there are; a width set by the caller is kept)
     const bool few = knn_few_queries(num_queries) && !op.f16 && !op.split && !ctx().knobs.knn_block_columns;
     const bool may = aligned && !few && capturing == hipStreamCaptureStatusNone;
-    const bool screened = may && w.screen.bytes != 0 && !ctx().knobs.knn_block_columns;
-    const bool candidates = may && (screened || M > knn_block_columns(op.rows_padded, num_queries));
-    bool redo = !candidates;
-    if (rc == DSX_OK && screened) rc = knn_search_candidates(w, op, M, num_queries, k, scores, indexes, t, true, &redo);
-    if (rc == DSX_OK && candidates && (!screened || redo) && M > knn_block_columns(op.rows_padded, num_queries))
-        rc = knn_search_candidates(w, op, M, num_queries, k, scores, indexes, t, false, &redo);
+    const bool many = M > knn_block_columns(op.rows_padded, num_queries);
+    bool screened = may && w.screen.bytes != 0 && !ctx().knobs.knn_block_columns;
+    bool redo = true, unfit = false;
+    if (rc == DSX_OK && screened) rc = knn_search_candidates(w, op, M, num_queries, k, scores, indexes, t, true, &redo, &unfit);
+    if (unfit) screened = false;
+    const bool candidates = may && (screened || many);
+    if (rc == DSX_OK && candidates && (!screened || redo) && many)
+        rc = knn_search_candidates(w, op, M, num_queries, k, scores, indexes, t, false, &redo, nullptr);
     g_knn_last_path = !candidates ? DSX_KNN_PATH_BLOCKS : (redo ? DSX_KNN_PATH_CANDIDATES_REDONE : DSX_KNN_PATH_CANDIDATES);
     if (rc == DSX_OK && redo) rc = knn_search_blocks(w, op, M, num_queries, k, scores, indexes, t);
     if (elapsed_ms) {

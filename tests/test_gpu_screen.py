@@ -88,6 +88,8 @@ def test_operands_that_f16_holds_badly(pkg, dsx, rng, form):
         norms[n // 2] = 0.0
     scale = length * np.nanmax(norms)
     check_against_float64(s / scale, i, full / scale, k, dim * 2.0 ** -24)
+    # what f16 cannot hold, or what would let everything pass, is found before the sweep: block by block straight away
+    assert dsx.dsx_knn_last_search_path() == {"unit": 1, "subnormal": 1, "nan items": 1, "rising": 2}.get(form, 0)
 
 
 @pytest.mark.parametrize("dim", [32, 128, 1024])
