@@ -104,7 +104,7 @@ SIGNATURES = {
     "dsx_fc_topk_flagged_for": [_vp, _int],
     "dsx_testing_reset": [],
     "dsx_testing_set_allocation_limit": [_sz],
-    "dsx_testing_set_knn_screen": [_int],
+    "dsx_testing_set_screen": [_int],
     "dsx_testing_occupy": [_u32, _u32, _u32],
     "dsx_testing_set_fc_topk_first_columns": [_u32],
     "dsx_testing_set_fc_topk_candidate_capacity": [_u32],

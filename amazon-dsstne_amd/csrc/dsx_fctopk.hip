@@ -169,7 +169,7 @@ int dsx_fc_topk_pays(uint32_t batch, uint32_t k_dim, uint32_t n, uint32_t activa
 {
     if (n >= 131072) return batch > 64;
     const double products = (double)batch * k_dim * n;
-    return activation == DSX_ACT_SIGMOID && screen_takes(batch, k_dim, n, true) &&
+    return activation == DSX_ACT_SIGMOID && screen_takes(batch, k_dim, n, true) && screen_layer_pays(batch, k_dim, n, k) &&
            ((k <= 32 && batch >= 1536 && products >= 2e10) || (k <= 128 && batch >= 2048 && products >= 1e11));
 }
 
@@ -206,7 +206,7 @@ static int fc_topk_common(const float* X, uint32_t ldx, const float* W, const fl
     const uint32_t cap = ctx().knobs.fc_topk_candidate_capacity ? ctx().knobs.fc_topk_candidate_capacity : kLayerCandCap;   // tests lower it to reach the overflow path with small inputs
     const uint32_t n0 = layer_first_columns(n, k);
     const bool ranges = n0 < n;
-    bool screened = ranges && !x_planes && screen_takes(batch, kdim, n, true);
+    bool screened = ranges && !x_planes && screen_takes(batch, kdim, n, true) && screen_layer_pays(batch, kdim, n, k);
     LibScratch& ws = g_layer_ws_of[current_lane()];
     int reserved = lib_scratch_reserve(ws, layer_layout(nullptr, batch, n0, k, cap, ranges, screened, kdim, n).bytes, "dsx_fc_topk workspace", screened);
     if (reserved == DSX_ENOMEM && screened) {   // the 16-bit copies (up to 8 GiB) do not fit beside what is there: fp32 ranges need none

@@ -17,7 +17,7 @@ struct TestKnobs {
     uint32_t knn_block_columns = 0;
     int knn_f16_sweep = 1;
     size_t allocation_limit = 0;
-    int knn_screen = 0;
+    int screen = 0;
 };
 
 struct Context {
@@ -226,6 +226,7 @@ struct ScreenWorkspace {
     size_t bytes;
 };
 bool screen_takes(uint32_t batch, uint32_t dim, uint64_t n, bool layer);
+bool screen_layer_pays(uint32_t batch, uint32_t dim, uint64_t n, uint32_t k);
 bool screen_search_pays(uint32_t batch, uint32_t dim, uint64_t n, uint32_t k, bool blocks, float norm_ratio);
 ScreenWorkspace screen_layout(void* base, uint32_t batch, uint32_t dim, uint64_t n, bool layer, uint32_t list_words);
 int screen_prepare(const ScreenWorkspace& w, const float* X, uint32_t ldx, uint32_t batch, const float* W, uint64_t ldw, const float* bias,

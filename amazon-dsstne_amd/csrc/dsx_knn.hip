@@ -347,9 +347,10 @@ int dsx_testing_set_knn_block_columns(uint32_t columns)
     return DSX_OK;
 }
 
-int dsx_testing_set_knn_screen(int mode)
+int dsx_testing_set_screen(int mode)
 {
-    ctx().knobs.knn_screen = mode;
+    DSX_CHECK_ARG(mode >= 0 && mode <= 2, "dsx_testing_set_screen: mode %d (0 to 2)", mode);
+    ctx().knobs.screen = mode;
     return DSX_OK;
 }
 

@@ -289,12 +289,26 @@ __global__ __launch_bounds__(256) void screen_rescore_kernel(ScreenRescoreArgs a
     if (threadIdx.x == 0) a.cand_count[b] = total;
 }
 
-// What can be screened, and for layers whether it pays: the preparation costs what about 130 rows' fp32 products do, and the
-// candidates' scores and the extra launches about 150 us (us, screened / fp32, top 10: 512 x 64 x 300,000 362 / 298, 512 x 256 x 300,000
-// 642 / 734, 1,024 x 512 x 60,000 398 / 509, 4,096 x 128 x 60,000 413 / 716).  Limits: the row in LDS, and 8 GiB for the two copies of
-// the table.
+// The same for a layer in ranges (dsx_fc_topk), fitted to 320 layers of 512 to 4,096 rows, 64 to 1,024 components, 16,384 to 1,000,000
+// columns, k 10 to 256, without filters: fp32 within 23 %, screened within 31 %; none is slower than in fp32, 1.3 % are left (us,
+// screened / fp32: 512 x 256 x 16,384 top 10 105 / 80, 4,096 x 1,024 x 27,278 top 256 3,977 / 2,591, 512 x 256 x 131,072 top 100
+// 539 / 539, 1,000 x 256 x 131,072 top 100 658 / 831, 4,096 x 512 x 300,000 top 100 3,578 / 10,343).
+bool screen_layer_pays(uint32_t batch, uint32_t dim, uint64_t n, uint32_t k)
+{
+    if (ctx().knobs.screen == 1) return true;
+    const double q = batch, d = dim, ld = screen_ld(dim, true), m = (double)n;
+    const double growth = std::max(4u, 4096 / (8 * k)), fold = std::log(std::max(m / 2048.0, 1.0)) / std::log(growth + 1.0);   // as fc_topk_common's ranges
+    const double ranges = std::ceil(fold), candidates = k * growth * fold;
+    const double fp32 = 28.0 + 17.6 * ranges + 1.553e-8 * q * m * d + 2.61e-7 * q * m + 7.7e-5 * q * candidates + 0.49 * k * ranges;
+    const double screened = 13.0 + 35.0 * ranges + 3.8e-6 * m * ld + 1.39e-9 * q * m * ld + 6e-8 * q * m + q * candidates * (7.6e-5 + 3.1e-7 * ld) + 0.57 * k * ranges;
+    return fp32 > 1.1 * screened;
+}
+
+// What can be screened: the preparation costs what about 130 rows' fp32 products do.  Limits: the row in LDS, and 8 GiB for the two
+// copies of the table.
 bool screen_takes(uint32_t batch, uint32_t dim, uint64_t n, bool layer)
 {
+    if (ctx().knobs.screen == 2) return false;
     const uint64_t bytes = knn_f16_rows(n) * ((uint64_t)screen_ld(dim, layer) * 2 + (uint64_t)screen_pitch32(dim) * 4);
     return batch >= 512 && dim >= 32 && dim <= 4096 && (!layer || (uint64_t)batch * dim >= 131072) && n >= (layer ? 16384 : 65536) && bytes <= ((uint64_t)8 << 30);
 }
@@ -313,7 +327,7 @@ bool screen_search_pays(uint32_t batch, uint32_t dim, uint64_t n, uint32_t k, bo
     const double q = batch, d = dim, ld = std::max(d, 64.0), m = (double)n;
     const double more = std::exp(std::min(20.0, 4.0 * std::sqrt(d) * (double)norm_ratio / 1024.0));
     if (5.0 * k * more > 3600.0) return false;
-    if (ctx().knobs.knn_screen) return true;
+    if (ctx().knobs.screen == 1) return true;
     const double ranges = 1.0 + std::max(1.0, std::ceil(std::log(m / 40960.0) / std::log(5.0))), fold = std::log(m / 8192.0) / std::log(5.0);
     const double fp32 = blocks ? 1.464e-8 * q * m * d + 1.656e-6 * q * m + 4.3e-5 * q * k + 0.265 * k
                                : 120.0 + 1.447e-8 * q * m * d + 2.56e-7 * q * m + 2.37e-4 * q * k + 0.6 * k;

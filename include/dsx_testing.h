@@ -28,9 +28,10 @@ int dsx_testing_set_knn_f16_sweep(int mode);
  * registers per lane.  bench.py --interference uses it to separate what a kernel beside a dense layer costs that layer by
  * merely being resident from what its instructions and memory traffic cost. */
 int dsx_testing_occupy(uint32_t workgroups, uint32_t cycles, uint32_t vgprs);
-/* dsx_knn_search: 1 screens in 16 bits whatever can be (512 queries and 65,536 items and more), 0 (default) only where it is expected to
- * be the faster way.  Workspace sizes depend on it. */
-int dsx_testing_set_knn_screen(int mode);
+/* dsx_knn_search, dsx_fc_topk: candidates are screened in 16 bits where that is expected to be the faster way (0, default), never (2);
+ * 1: whatever can be (searches of 512 queries and 65,536 items, layers of 512 rows and 16,384 columns and more).  Workspace sizes
+ * depend on it. */
+int dsx_testing_set_screen(int mode);
 /* Largest single block of device memory that dsx_malloc and the library's own scratch may hold, in bytes (0, the default: what the
  * device has): larger ones fail as if the memory were short. */
 int dsx_testing_set_allocation_limit(size_t bytes);

@@ -14,9 +14,9 @@ pytestmark = pytest.mark.gpu
 @pytest.fixture(autouse=True)
 def screened(dsx):
     """Searches that are small for a test are screened too (by default only where that is expected to be faster)."""
-    dsx.dsx_testing_set_knn_screen(1)
+    dsx.dsx_testing_set_screen(1)
     yield
-    dsx.dsx_testing_set_knn_screen(0)
+    dsx.dsx_testing_set_screen(0)
 
 
 def with_twins(rng, n, dim, front, back, pairs):

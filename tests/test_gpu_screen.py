@@ -13,9 +13,9 @@ pytestmark = pytest.mark.gpu
 @pytest.fixture(autouse=True)
 def screened(dsx):
     """Searches that are small for a test are screened too (by default only where that is expected to be faster)."""
-    dsx.dsx_testing_set_knn_screen(1)
+    dsx.dsx_testing_set_screen(1)
     yield
-    dsx.dsx_testing_set_knn_screen(0)
+    dsx.dsx_testing_set_screen(0)
 
 
 def search(pkg, dsx, items, queries, k):
@@ -221,7 +221,7 @@ def test_masked_columns(pkg, dsx, rng, act, mask):
 
 @pytest.mark.parametrize("n,queries,dim,k,path", [(65536, 512, 32, 10, 0), (150000, 1000, 128, 10, 1), (150000, 512, 64, 256, 0)])
 def test_searches_are_screened_where_that_is_faster(pkg, dsx, rng, n, queries, dim, k, path):
-    dsx.dsx_testing_set_knn_screen(0)
+    dsx.dsx_testing_set_screen(0)
     items = rng.integers(-3, 4, size=(n, dim)).astype(np.float32)
     q = rng.integers(-3, 4, size=(queries, dim)).astype(np.float32)
     s, i = search(pkg, dsx, items, q, k)
