@@ -457,6 +457,8 @@ static int knn_search_common(KnnOperands& op, uint32_t padding, uint32_t num_que
         elapsed_ms[0] = t.gemm;
         elapsed_ms[1] = t.topk;
     }
+    // the results are complete when the call returns (the other ways have waited by now)
+    if (rc == DSX_OK && redo && !elapsed_ms && capturing == hipStreamCaptureStatusNone) DSX_HIP(hipStreamSynchronize(s));
     return rc;
 }
 

@@ -160,6 +160,19 @@ def test_knn_few_queries(pkg, dsx, orc, rng, items, queries, dim, k):
     assert np.array_equal(got_s, ref_s) and np.array_equal(got_i, ref_i)
 
 
+def test_knn_search_returns_with_its_results(pkg, dsx, rng):
+    """Block by block and without timers too: nothing is left on the stream when the call returns."""
+    items, queries, dim, k = 1000000, 4, 64, 10
+    hip = C.CDLL("libamdhip64.so")
+    dsx.dsx_stream.restype = C.c_void_p
+    stream = C.c_void_p(dsx.dsx_stream())
+    table, q = pkg.DeviceArray((dim, items), np.float32), dev(pkg, rng.standard_normal((queries, dim), dtype=np.float32))
+    scores, idx = pkg.DeviceArray((queries, k), np.float32), pkg.DeviceArray((queries, k), np.uint32)
+    for _ in range(3):
+        pkg.check(dsx.dsx_knn_search(table.ptr, items, 0, dim, q.ptr, queries, k, scores.ptr, idx.ptr, None, 0, None))
+        assert dsx.dsx_knn_last_search_path() == 0 and hip.hipStreamQuery(stream) == 0
+
+
 @pytest.mark.parametrize("items,queries,k", [(200000, 100, 200), (200000, 100, 129), (150001, 65, 100), (270011, 130, 256)])
 def test_knn_segments_of_a_row_that_share_its_bound(pkg, dsx, orc, rng, items, queries, k):
     """Several workgroups per row raise one bound while their siblings read it, and thousands of items tie at every score: the order
