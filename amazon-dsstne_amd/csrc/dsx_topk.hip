@@ -832,6 +832,9 @@ __device__ __forceinline__ void scan_segment(const TopKArgs& a, uint64_t (*sStag
     finish_row<R>(list, sStage, a, b, seg, wave, lane);
 }
 
+// Four workgroups per compute unit for every R.  (R = 4 filtered spills 12 bytes a lane at that and none at two workgroups, which are
+// slower where a batch fills the GPU: 1,024 x 60,000 k = 200 96 us against 131, 256 x 200,000 k = 256 111 against 147; 1,024 x
+// 200,000 k = 256 343 against 342.)
 template <int R, bool FILTERED>
 __global__ __launch_bounds__(kTopkThreads, 4) void topk_scan_kernel(TopKArgs a)
 {
@@ -1485,7 +1488,10 @@ template <int R, int G> static void launch_block(const TopKArgs& a, uint32_t bat
 template <int R> static int launch_scan(const TopKArgs& a, uint32_t batch, bool filtered, size_t bitmap_bytes)
 {
     dim3 grid(batch, a.segments);
-    // Segments that fit a workgroup's registers (multipliers other than 0 need the listed scores: the general scan).
+    // Segments that fit a workgroup's registers (multipliers other than 0 need the listed scores: the general scan).  A group of 1,024
+    // columns is four registers of a lane, of the 128 that four workgroups per compute unit leave, which is what ends the ladder: 27 or
+    // 28 groups fit for k <= 128, 29 spill scores (k > 128 spills 20 bytes a lane at 27; filtered forms keep 8 to 44 bytes of the
+    // fallback, which few rows reach, in scratch).  The rungs below spare narrower rows the registers and compares they do not need.
     const uint32_t columns = ((a.width / 4 + 1 + a.segments - 1) / a.segments) * 4 + 8;   // an upper bound of a segment's
     if (!a.fmul && columns <= 27 * 4 * kTopkThreads) {
         if (columns <= 2 * 4 * kTopkThreads) launch_block<R, 2>(a, batch, filtered, bitmap_bytes);
