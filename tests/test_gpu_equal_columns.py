@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.fixture(autouse=True)
-def screened(dsx):
+def everything_screened(dsx):
     """Searches that are small for a test are screened too (by default only where that is expected to be faster)."""
     dsx.dsx_testing_set_screen(1)
     yield
