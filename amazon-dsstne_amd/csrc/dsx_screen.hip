@@ -41,7 +41,7 @@ uint32_t screen_pitch32(uint32_t dim) { return (dim + 3) / 4 * 4; }
 __device__ __forceinline__ float screen_relative(uint32_t dim) { return 9.765625e-4f * 1.01f + (4.0f * (float)dim + 64.0f) * 5.9604645e-8f; }
 
 // stats: [0] largest norm of a column, of a layer's first block's columns only (the bits of a non-negative float; NaN columns have no
-// part in it: their scores are NaN on every path); [1] sum of the norms of one column in 64, [2] their number (nearest neighbours)
+// part in it: their scores are NaN on every path); [1] sum of the norms of one column in 256, [2] their number (nearest neighbours)
 struct ScreenItemsArgs {
     const float* W;       // [dim][ldw]
     const float* bias;    // layers: [n], or NULL
@@ -101,13 +101,13 @@ __global__ __launch_bounds__(256) void screen_items_kernel(ScreenItemsArgs a)
     };
     if (q == 0) raise(&a.stats[0], col0 + l < a.first ? norm : 0.0f);
     if constexpr (!ITEM_NORM) {
-        if (q == 1 && blockIdx.x % 64 == 0) {
+        if (q == 1 && blockIdx.x % 256 == 0) {
             float some = (valid && norm <= kF16Max) ? norm : 0.0f;
 #pragma unroll
             for (int d = 1; d < 64; d *= 2) some += __shfl_xor(some, d);
             const uint32_t number = (uint32_t)__popcll(__ballot(valid && norm <= kF16Max));
             if (l == 0) {
-                atomicAdd(reinterpret_cast<float*>(&a.stats[1]), some);
+                unsafeAtomicAdd(reinterpret_cast<float*>(&a.stats[1]), some);   // (the instruction; plain atomicAdd is a loop, 36 us of it here)
                 atomicAdd(&a.stats[2], number);
             }
         }

@@ -1866,14 +1866,14 @@ int layer_refresh_run(const LayerRefresh& r, uint32_t batch)
 // whole row once more, without any list that could fill up.  The flagged rows are gathered 32 at a time and the columns cut into as many
 // parts as keep the GPU busy; a workgroup walks its part in steps of 512 columns, 128 per wavefront, sums in ascending pairs of k
 // (bias last: as a stored layer), W from memory straight into registers one chunk of eight k ahead.  The scores go through LDS, 128
-// columns at a time, to the wavefront that keeps the row's list, which stages what beats the row's k-th word and merges when more than 32 words wait; the last
+// columns at a time, to the wavefront that keeps the row's list, which merges what beats the row's k-th word when more than 32 words wait; the last
 // workgroup of 32 rows to finish merges their parts.  Bound by reading W once per 32 rows from the caches; where no row is flagged, by
 // the launch.
 // 4,096 x 1,024 x 27,278 saturated, every row flagged: 3.05 ms, 75 TFLOP/s, of a call of 16 (12.4 of them the sweep, all of whose
 // scores pass); a wavefront per row that read W for itself took 0.5 s.
-constexpr uint32_t kRedoGrid = 512;   // two workgroups per compute unit
+constexpr uint32_t kRedoGrid = 256;   // (a grid that finds nothing to do takes its place beside another lane's GEMM first: 512 of 62 KiB of LDS 25 us, these of 34 KiB 6)
 constexpr int kRedoBlocks = 4;        // blocks of 32 columns per wavefront and step
-constexpr uint32_t kRedoRows = 32, kRedoCols = 128, kRedoSpan = 1024, kRedoStage = kRedoCols + 32, kRedoParts = 128;
+constexpr uint32_t kRedoRows = 32, kRedoCols = 128, kRedoSpan = 1024, kRedoWait = 32, kRedoParts = 128;
 
 struct LayerRedoArgs {
     const float* X;
@@ -1899,13 +1899,15 @@ __global__ __launch_bounds__(256, 2) void layer_redo_kernel(LayerRedoArgs a)
 {
     using List = WaveTopK<R>;
     __shared__ float sScore[kRedoRows][kRedoCols + 4];
-    __shared__ uint64_t sStage[kRedoRows][kRedoStage];
+    __shared__ uint64_t sWait[kRedoRows][kRedoWait];        // words of a row that wait to be merged
+    __shared__ uint64_t sStage[4][kRedoWait + kRedoCols];   // per wavefront: what is merged
     __shared__ uint64_t sThr[kRedoRows];                    // the row's k-th word so far
     __shared__ uint32_t sCount[kRedoRows], sMerged[kRedoRows];   // its staged words, whether it has a list yet
     __shared__ uint32_t sBits[kRedoRows][kRedoSpan / 32];   // listed columns of the span
     __shared__ uint32_t sRows[kRedoRows], sWave[4], sAny, sLast;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
     const uint32_t l32 = lane & 31, lhi = lane >> 5;
+    __builtin_amdgcn_s_setprio(3);
     if (threadIdx.x == 0) sAny = 0;
     __syncthreads();
     uint32_t mine = 0;
@@ -1943,11 +1945,11 @@ __global__ __launch_bounds__(256, 2) void layer_redo_kernel(LayerRedoArgs a)
         __syncthreads();
         const float* x = a.X + (uint64_t)sRows[min(l32, rows - 1)] * a.ldx;   // (lanes beyond the rows repeat the last one)
         uint64_t* lists = a.partial + (uint64_t)item * kRedoRows * a.k;
-        // (a row's staged words, their number, its k-th word and its list belong to one wavefront)
+        // (a row's waiting words, their number, its k-th word and its list belong to one wavefront)
         auto merge = [&](uint32_t r, uint32_t staged) {
             const bool has = sMerged[r] != 0;
             List list;
-            list.init(sStage[r], lane, a.k);
+            list.init(sStage[wave], lane, a.k);
             uint64_t* mem = lists + (uint64_t)r * a.k;
 #pragma unroll
             for (int q = 0; q < R; q++) {
@@ -2058,30 +2060,38 @@ __global__ __launch_bounds__(256, 2) void layer_redo_kernel(LayerRedoArgs a)
 #pragma unroll 1
                     for (uint32_t r = wave; r < rows; r += 4) {
                         const uint64_t thr = sThr[r];
-                        uint32_t count = sCount[r];   // wave-uniform
-#pragma unroll 1
+                        const uint32_t waiting = sCount[r];   // wave-uniform
+                        uint64_t word[2], m[2];
+#pragma unroll
                         for (int h = 0; h < 2; h++) {
                             const uint32_t c = c0 + h * kWave + lane;
-                            float y = activate_rt(sScore[r][h * kWave + lane] + (h ? bias[1] : bias[0]), a.act, a.slope, a.alpha, a.lambda);
+                            float y = activate_rt(sScore[r][h * kWave + lane] + bias[h], a.act, a.slope, a.alpha, a.lambda);
                             // a listed column keeps its place with score * 0 (utils/Filters.cpp:62), once however often it is listed
                             if (a.fidx && ((sBits[r][(c - span) >> 5] >> (c & 31)) & 1u)) y *= 0.0f;
-                            const uint64_t word = pack_score(y, c);
-                            const bool cand = c < span_end && y == y && word > thr;
-                            const uint64_t m = __ballot(cand);
-                            if (cand) sStage[r][count + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))] = word;
-                            count += (uint32_t)__popcll(m);
+                            word[h] = pack_score(y, c);
+                            m[h] = __ballot(c < span_end && y == y && word[h] > thr);
                         }
-                        if (count > kRedoStage - kRedoCols) {
-                            merge(r, count);
-                            count = 0;
-                        }
-                        if (lane == 0) sCount[r] = count;
+                        if ((m[0] | m[1]) == 0) continue;
+                        const uint32_t first = (uint32_t)__popcll(m[0]), count = waiting + first + (uint32_t)__popcll(m[1]);
+                        const bool full = count > kRedoWait;
+                        uint64_t* to = full ? sStage[wave] : sWait[r];
+                        if (full && lane < waiting) to[lane] = sWait[r][lane];
+#pragma unroll
+                        for (int h = 0; h < 2; h++)
+                            if ((m[h] >> lane) & 1ull)
+                                to[waiting + (h ? first : 0u) + __builtin_amdgcn_mbcnt_hi((uint32_t)(m[h] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m[h], 0u))] = word[h];
+                        if (full) merge(r, count);
+                        if (lane == 0) sCount[r] = full ? 0u : count;
                     }
                     __syncthreads();   // the scores have been read
                 }
             }
         }
-        for (uint32_t r = wave; r < rows; r += 4) merge(r, sCount[r]);
+        for (uint32_t r = wave; r < rows; r += 4) {
+            const uint32_t waiting = sCount[r];
+            if (lane < waiting) sStage[wave][lane] = sWait[r][lane];
+            merge(r, waiting);
+        }
         // The last part of the group to finish merges them all.  (Release: the lists are in memory before the count; acquire: they are
         // read after it.  Workgroups of a group may run on different XCDs, whose L2s are not kept coherent.)
         __threadfence();
@@ -2092,13 +2102,13 @@ __global__ __launch_bounds__(256, 2) void layer_redo_kernel(LayerRedoArgs a)
             __threadfence();
             for (uint32_t r = wave; r < rows; r += 4) {
                 List list;
-                list.init(sStage[r], lane, a.k);
+                list.init(sStage[wave], lane, a.k);
                 for (uint32_t s = 0; s < parts; s++) {
                     const uint64_t* src = a.partial + ((uint64_t)(group * parts + s) * kRedoRows + r) * a.k;
                     for (uint32_t p0 = 0; p0 < a.k; p0 += kWave) {
                         const uint64_t word = (p0 + lane < a.k) ? src[p0 + lane] : 0ull;
                         list.stage_only(word != 0, word);
-                        list.finish();   // (a staging row has room for 160 words)
+                        list.finish();
                     }
                 }
                 const uint64_t row = sRows[r];
