@@ -319,7 +319,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
                             } else {   // this (row, chunk) list is full: the row's shared list
                                 const uint32_t p2 = atomicAdd(&a.cand.cand_count[r], 1u);
                                 if (p2 < a.cand.cand_cap) a.cand.cand[(uint64_t)r * a.cand.cand_cap + p2] = word;
-                                else *a.cand.overflow = 1u;
+                                else {   // the row is done otherwise: nothing more of it is wanted (4,096 x 1,024 x 27,278 with every
+                                         // score passing: 4.7 ms, 12.4 with all the appends that no list takes)
+                                    *a.cand.overflow = 1u;
+                                    row_state(rl)[1] = __float_as_uint(__builtin_inff());
+                                }
                             }
                         }
                     }
@@ -457,7 +461,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                     } else {   // this list is full: the query's shared list
                         const uint32_t p2 = atomicAdd(&a.cand.cand_count[q[h]], 1u);
                         if (p2 < a.cand.cand_cap) a.cand.cand[(uint64_t)q[h] * a.cand.cand_cap + p2] = word;
-                        else *a.cand.overflow = 1u;
+                        else {
+                            *a.cand.overflow = 1u;
+                            bound[h] = __builtin_inff();   // (the row is done otherwise: nothing more of it is wanted)
+                        }
                     }
                     fill[h]++;
                 }

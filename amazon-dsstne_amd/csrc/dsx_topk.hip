@@ -1869,7 +1869,7 @@ int layer_refresh_run(const LayerRefresh& r, uint32_t batch)
 // columns at a time, to the wavefront that keeps the row's list, which merges what beats the row's k-th word when more than 32 words wait; the last
 // workgroup of 32 rows to finish merges their parts.  Bound by reading W once per 32 rows from the caches; where no row is flagged, by
 // the launch.
-// 4,096 x 1,024 x 27,278 saturated, every row flagged: 3.05 ms, 75 TFLOP/s, of a call of 16 (12.4 of them the sweep, all of whose
+// 4,096 x 1,024 x 27,278 saturated, every row flagged: 2.8 ms, 80 TFLOP/s, of a call of 8 (4.7 of them the sweep, all of whose
 // scores pass); a wavefront per row that read W for itself took 0.5 s.
 constexpr uint32_t kRedoGrid = 256;   // (a grid that finds nothing to do takes its place beside another lane's GEMM first: 512 of 62 KiB of LDS 25 us, these of 34 KiB 6)
 constexpr int kRedoBlocks = 4;        // blocks of 32 columns per wavefront and step
