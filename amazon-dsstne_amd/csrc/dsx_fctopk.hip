@@ -232,7 +232,7 @@ static int fc_topk_common(const float* X, uint32_t ldx, const float* W, const fl
     hipLaunchKernelGGL(layer_clear_kernel, dim3((clear_words + 255) / 256), dim3(256), 0, s, w.row_bound, clear_words);
     DSX_LAUNCH_CHECK("layer_clear_kernel");
     if (screened) {
-        rc = screen_prepare(w.screen, X, ldx, batch, W, n, bias, n, kdim, true, n0, w.row_flag, flag_word);
+        rc = screen_prepare(w.screen, X, ldx, batch, W, n, bias, n, kdim, true, n0, w.row_flag, flag_word, nullptr);
         if (rc) return rc;
     }
     rc = topk_run(w.block_scores, ld0, n0, batch, k, nullptr, nullptr, position, index, filter_start, filter_end, filter_index, nullptr, 0,

@@ -225,12 +225,17 @@ struct ScreenWorkspace {
     uint32_t list_words;
     size_t bytes;
 };
+// Nearest neighbours, in pinned memory: the largest norm of the table, a sample of the norms and how many they are, and (told) the flag.
+struct ScreenNotes {
+    float largest, sum;
+    uint32_t number, flag;
+};
 bool screen_takes(uint32_t batch, uint32_t dim, uint64_t n, bool layer);
 bool screen_layer_pays(uint32_t batch, uint32_t dim, uint64_t n, uint32_t k);
 bool screen_search_pays(uint32_t batch, uint32_t dim, uint64_t n, uint32_t k, bool blocks, float norm_ratio);
 ScreenWorkspace screen_layout(void* base, uint32_t batch, uint32_t dim, uint64_t n, bool layer, uint32_t list_words);
 int screen_prepare(const ScreenWorkspace& w, const float* X, uint32_t ldx, uint32_t batch, const float* W, uint64_t ldw, const float* bias,
-                   uint64_t n, uint32_t dim, bool layer, uint32_t first, uint32_t* flag, uint32_t* told);
+                   uint64_t n, uint32_t dim, bool layer, uint32_t first, uint32_t* flag, uint32_t* told, ScreenNotes* notes);
 int screen_candidates(const ScreenWorkspace& w, const float* X, uint32_t ldx, uint32_t batch, uint32_t dim, bool layer, const float* bias,
                       uint32_t ncols, const CandArgs& cand, bool report_overflow, bool first);
 

@@ -235,12 +235,8 @@ static int knn_search_blocks(const KnnWorkspace& w, const KnnOperands& op, uint3
     return rc;
 }
 
-// What the preparation of a screened search found, read back while the first block runs (pinned).
-struct KnnNotes {
-    float largest, sum;
-    uint32_t number, flag;
-};
-static KnnNotes* g_knn_notes = nullptr;
+// What the preparation of a screened search finds, stored by it in pinned memory and read while the first block runs.
+static ScreenNotes* g_knn_notes = nullptr;
 static hipEvent_t g_knn_noted = nullptr;
 
 static void knn_notes_release()
@@ -251,16 +247,14 @@ static void knn_notes_release()
     g_knn_noted = nullptr;
 }
 
-static int knn_notes_request(const KnnWorkspace& w, hipStream_t s)
+static int knn_notes_ready()
 {
     if (!g_knn_noted) {
         at_shutdown(knn_notes_release);
-        if (!g_knn_notes) DSX_HIP(hipHostMalloc((void**)&g_knn_notes, sizeof(KnnNotes), hipHostMallocDefault));
+        if (!g_knn_notes) DSX_HIP(hipHostMalloc((void**)&g_knn_notes, sizeof(ScreenNotes), hipHostMallocMapped));
         DSX_HIP(hipEventCreateWithFlags(&g_knn_noted, hipEventDisableTiming));
     }
-    DSX_HIP(hipMemcpyAsync(g_knn_notes, w.screen.stats, 3 * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    DSX_HIP(hipMemcpyAsync(&g_knn_notes->flag, w.overflow, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-    DSX_HIP(hipEventRecord(g_knn_noted, s));
+    *g_knn_notes = ScreenNotes{};   // (a search is over when its call returns: nothing writes to them now)
     return DSX_OK;
 }
 
@@ -282,9 +276,13 @@ static int knn_search_candidates(const KnnWorkspace& w, const KnnOperands& op, u
     if (!ctx().knobs.knn_block_columns) done = std::min<uint32_t>(done, screened ? 8192u : std::max<uint32_t>(1024, cb / 4 / 1024 * 1024));
     t.start(s);
     int rc = DSX_OK;
-    if (screened) rc = screen_prepare(w.screen, op.queries, op.dim, num_queries, op.items, op.rows_padded, nullptr, M, op.dim, false, 0, w.overflow, nullptr);
-    if (rc == DSX_OK && screened) rc = knn_notes_request(w, s);
-    if (rc) return rc;
+    if (screened) {
+        if ((rc = knn_notes_ready())) return rc;
+        rc = screen_prepare(w.screen, op.queries, op.dim, num_queries, op.items, op.rows_padded, nullptr, M, op.dim, false, 0, w.overflow,
+                            &g_knn_notes->flag, g_knn_notes);
+        if (rc) return rc;
+        DSX_HIP(hipEventRecord(g_knn_noted, s));
+    }
     FcOrder order;
     order.as_candidates = !screened;
     rc = op.into_matrix(0, done, num_queries, w.block_scores, cb, order);
@@ -300,8 +298,12 @@ static int knn_search_candidates(const KnnWorkspace& w, const KnnOperands& op, u
     const uint32_t seen = done;
     if (screened) {
         done = 0;
-        DSX_HIP(hipEventSynchronize(g_knn_noted));   // (the first block is still running)
-        const KnnNotes notes = *g_knn_notes;
+        // (asked again and again: the first block runs for another 100 us, and a wait that sleeps wakes up later than that)
+        hipError_t noted;
+        while ((noted = hipEventQuery(g_knn_noted)) == hipErrorNotReady) {}
+        (void)hipGetLastError();   // (not ready is not an error of the next launch)
+        DSX_HIP(noted);
+        const ScreenNotes notes = *g_knn_notes;
         const float average = notes.number != 0 ? notes.sum / (float)notes.number : 0.0f;
         *unfit = notes.flag != 0 || (notes.largest > 0.0f && !screen_search_pays(num_queries, op.dim, M, k, M <= cb, notes.largest / average));
         if (*unfit) return DSX_OK;

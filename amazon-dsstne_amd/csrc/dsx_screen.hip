@@ -146,6 +146,7 @@ struct ScreenRowsArgs {
     float* slack;           // [batch] layers: and by how much more where it comes from another kernel's sums
     uint32_t* flag;         // one word (nearest neighbours) or one per row (layers): set where the error has no bound
     uint32_t* told;         // host-visible word set with it (may be NULL)
+    ScreenNotes* notes;     // host-visible: what the table's columns are like (nearest neighbours)
 };
 
 // One wavefront per row.
@@ -172,6 +173,11 @@ __global__ __launch_bounds__(256) void screen_rows_kernel(ScreenRowsArgs a)
         a.out16[(uint64_t)row * a.ld + d] = (_Float16)x;
     }
     if (!valid || lane != 0) return;
+    if (!ITEM_NORM && row == 0 && a.notes) {
+        a.notes->largest = __uint_as_float(a.stats[0]);
+        a.notes->sum = __uint_as_float(a.stats[1]);
+        a.notes->number = a.stats[2];
+    }
     const float most = __uint_as_float(a.stats[0]);
     float eps = 2.9802322e-8f * 1.01f * sqrtf((float)a.dim + 4.0f) * (ITEM_NORM ? norm : norm + most);
     if constexpr (ITEM_NORM) eps += 1e-7f;   // (the bias: its last piece is good to 2^-25)
@@ -368,7 +374,7 @@ ScreenWorkspace screen_layout(void* base, uint32_t batch, uint32_t dim, uint64_t
 __global__ void screen_clear_kernel(uint32_t* stats) { stats[threadIdx.x] = 0; }
 
 int screen_prepare(const ScreenWorkspace& w, const float* X, uint32_t ldx, uint32_t batch, const float* W, uint64_t ldw, const float* bias,
-                   uint64_t n, uint32_t dim, bool layer, uint32_t first, uint32_t* flag, uint32_t* told)
+                   uint64_t n, uint32_t dim, bool layer, uint32_t first, uint32_t* flag, uint32_t* told, ScreenNotes* notes)
 {
     hipStream_t s = ctx().stream;
     hipLaunchKernelGGL(screen_clear_kernel, dim3(1), dim3(64), 0, s, w.stats);
@@ -382,7 +388,7 @@ int screen_prepare(const ScreenWorkspace& w, const float* X, uint32_t ldx, uint3
     DSX_LAUNCH_CHECK("screen_items_kernel");
     ScreenRowsArgs r{};
     r.X = X; r.ldx = ldx; r.batch = batch; r.dim = dim; r.ld = i.ld;
-    r.out16 = (_Float16*)w.queries16; r.stats = w.stats; r.eps = w.eps; r.slack = w.slack; r.flag = flag; r.told = told;
+    r.out16 = (_Float16*)w.queries16; r.stats = w.stats; r.eps = w.eps; r.slack = w.slack; r.flag = flag; r.told = told; r.notes = notes;
     const dim3 rgrid((uint32_t)(knn_f16_rows(batch) / 4));
     if (layer) hipLaunchKernelGGL((screen_rows_kernel<true>), rgrid, dim3(256), 0, s, r);
     else hipLaunchKernelGGL((screen_rows_kernel<false>), rgrid, dim3(256), 0, s, r);
