@@ -30,7 +30,7 @@ F16_MFMA_PEAK_TF = 2500.0        # dense f16 MFMA, the same
 
 # HBM bytes per launch, measured: profiles/pmc_hbm_traffic.json holds, per workload and kernel, what rocprofv3 --pmc FETCH_SIZE and
 # WRITE_SIZE read (KiB per dispatch) and the calibration factors from a plain 256 MiB device-to-device copy in the same runs; the
-# summary beside it (profiles/pmc_cfg2_hbm_traffic.md) is made from the same file and gives the commands.
+# summary beside it (profiles/pmc_hbm_traffic.md) is made from the same file and gives the commands.
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "pmc_hbm_traffic.json")
 BATCHES = 8                  # distinct batches resident in HBM that the timed loop cycles over
 WINDOWS = 5                  # timed windows of --steps steps each; the median is reported
@@ -235,7 +235,8 @@ def network_bench(args, pkg, lib):
     ms_one_lane = float(np.median(timed_windows(step, net.sync, args.steps, 3)))
     net.set_lanes(args.lanes)
     # ... and with the output layer stored by PredictBatch as the reference does, instead of computed together with the top-K
-    # (NNNetwork::SetDeferredOutput; only layers of 131,072 units or more are deferred, so this differs for config 4 alone)
+    # (NNNetwork::SetDeferredOutput; dsx_fc_topk_pays says which layers are deferred.  Config 4 differs; config 3's layer is deferred for
+    # its first batch only, whose scores tie in their thousands)
     net.set_deferred_output(False)
     settle(pkg, lib, step)
     ms_stored = float(np.median(timed_windows(step, net.sync, args.steps, 3)))
@@ -490,7 +491,7 @@ def network_bench(args, pkg, lib):
         "one_lane": {"ms_per_step": round(ms_one_lane, 5), "value": rate(ms_one_lane), "unit": "samples/s",
                      "note": "NNNetwork::SetLanes(1): one set of buffers, one stream, batches strictly one after the other"},
         "stored_output": {"ms_per_step": round(ms_stored, 5), "value": rate(ms_stored), "unit": "samples/s",
-                          "note": "NNNetwork::SetDeferredOutput(false): PredictBatch stores the output layer, the top-K reads it back (the same as the default below 131,072 output units)"},
+                          "note": "NNNetwork::SetDeferredOutput(false): PredictBatch stores the output layer, the top-K reads it back (the same as the default where dsx_fc_topk does not pay)"},
         "split_products": {"ms_per_step": round(ms_split, 5), "value": rate(ms_split), "unit": "samples/s",
                            "dtype": "f32 products as six bf16 x bf16 MFMA terms, f32 sums",
                            "note": "NNNetwork::SetSplitProducts(true), off by default: dense layers of at least two 128 x 128 tiles per compute unit run fc_gemm_split_kernel (a deferred output layer: dsx_fc_topk_split); results within the same tolerance of the oracle, as close to fp64 as the fp32 kernel's"},
@@ -528,8 +529,10 @@ def knn_bench(args, pkg, lib):
     ms_step = (time.perf_counter() - t0) * 1e3 / args.steps
     step(el)
     flops = 2.0 * Q * D * (rows - pad)
-    roofline = {"kernel": "f16 screening + fp32 scores of the candidates (knn)", "bound": "mfma", "achieved": round(flops / el[0] / 1e9, 3), "peak": F16_MFMA_PEAK_TF,
-                "unit": "TFLOP/s", "frac": round(flops / el[0] / 1e9 / F16_MFMA_PEAK_TF, 4), "traffic": None, "avg_launch_ms": round(el[0], 4),
+    name = "f16 screening + fp32 scores of the candidates (knn)"
+    moved = measured_traffic(p.name).get(name)
+    roofline = {"kernel": name, "bound": "mfma", "achieved": round(flops / el[0] / 1e9, 3), "peak": F16_MFMA_PEAK_TF,
+                "unit": "TFLOP/s", "frac": round(flops / el[0] / 1e9 / F16_MFMA_PEAK_TF, 4), "traffic": moved["read"] + moved["write"] if moved else None, "avg_launch_ms": round(el[0], 4),
                 "topk_ms": round(el[1], 4),
                 "path": {0: "blocks", 1: "candidate lists", 2: "candidate lists, redone block by block"}[lib.dsx_knn_last_search_path()]}
     # the same search with fp16 storage of items and queries (the reference's DataType::FP16): reported beside the fp32 figure
