@@ -303,7 +303,7 @@ bool screen_layer_pays(uint32_t batch, uint32_t dim, uint64_t n, uint32_t k)
 {
     if (ctx().knobs.screen == 1) return true;
     const double q = batch, d = dim, ld = screen_ld(dim, true), m = (double)n;
-    const double growth = std::max(4u, 4096 / (8 * k)), fold = std::log(std::max(m / 2048.0, 1.0)) / std::log(growth + 1.0);   // as fc_topk_common's ranges
+    const double growth = std::max(4u, 512 / std::max(1u, k)), fold = std::log(std::max(m / 2048.0, 1.0)) / std::log(growth + 1.0);   // as fc_topk_common's ranges
     const double ranges = std::ceil(fold), candidates = k * growth * fold;
     const double fp32 = 28.0 + 17.6 * ranges + 1.553e-8 * q * m * d + 2.61e-7 * q * m + 7.7e-5 * q * candidates + 0.49 * k * ranges;
     const double screened = 13.0 + 35.0 * ranges + 3.8e-6 * m * ld + 1.39e-9 * q * m * ld + 6e-8 * q * m + q * candidates * (7.6e-5 + 3.1e-7 * ld) + 0.57 * k * ranges;

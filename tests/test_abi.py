@@ -59,3 +59,14 @@ def test_missing_library_raises(pkg, monkeypatch):
     monkeypatch.setattr(pkg, "LIB_PATH", "/nonexistent/libdsx_hip.so")
     with pytest.raises(pkg.DsxError):
         pkg.load_library()
+
+
+def test_dsx_fc_topk_pays_answers_for_any_arguments(pkg):
+    """The layer asks before it looks at its arguments: no shape and no k may end the process."""
+    lib = pkg.load_library()
+    for batch in (0, 1, 64, 65, 4096):
+        for kdim in (0, 1, 1024, 100000):
+            for n in (0, 1, 2048, 27278, 131072, 4000000000):
+                for k in (0, 1, 10, 256, 100000):
+                    assert lib.dsx_fc_topk_pays(batch, kdim, n, 0, k) in (0, 1)
+    assert lib.dsx_fc_topk_pays(4096, 1024, 27278, 0, 10) == 1 and lib.dsx_fc_topk_pays(4096, 1024, 27278, 0, 256) == 0
