@@ -309,7 +309,7 @@ int dsx_topk_guided(const float* in, float* keys, uint32_t* values, uint32_t bat
  * Results are exact under the same total order as dsx_topk (score descending, column ascending); a score here and the same
  * score from dsx_fc_forward may differ in the last place (the bias enters the sum first instead of last).  A row whose
  * survivor list fills up (thousands of scores tied at the top), or whose k-th score is not above 0 while its filter lists columns
- * beyond the first block, is computed again on the device (all such rows together, at about half the speed of the stored layer);
+ * beyond the first block (any columns, where the layer is screened in 16 bits), is computed again on the device (all such rows together, at about half the speed of the stored layer);
  * dsx_fc_topk_flagged tells a caller that this has happened, so that it can go back to dsx_fc_forward + dsx_topk_filtered.
  * Returns DSX_EUNSUPPORTED (dsx_fc_topk_supported() == 0) unless the activation is non-decreasing (sigmoid, tanh, ReLU, leaky
  * ReLU with a positive slope, linear) and X is 16-byte aligned with ldx a multiple of 4. */
