@@ -1,0 +1,469 @@
+// dsx_f16.hip — f16 products of a few hundred to a few thousand rows ("queries") with a long table of items, on the matrix cores.
+//
+// Operands are row-major halves, a row's components contiguous: queries [rows rounded up to 256][ld], items [items rounded up to
+// 256][ld], ld a multiple of 64, zero filled.  Products are exact in fp32, sums are fp32, added in ascending k: the same bits as
+// knn_f16_kernel's.  Three uses (MODE):
+//   kF16Scores   sums compared with the queries' bounds, survivors to lists (exact nearest neighbours, fp16 storage and screening)
+//   kF16Layer    sums that start from the items' biases, raised by the error they can have (dsx_screen.hip), against the bounds
+//   kF16Store    sums that start from the biases stored as halves, rounded up
+//
+// A wavefront owns 128 items x 64 queries: four row operands and two column operands per 16 components feed eight matrix
+// instructions, 48 LDS cycles for 64 cycles of each SIMD's matrix core (a 64 x 64 tile needs as many LDS cycles as there are).
+// WI x WQ wavefronts make a workgroup; with 2 x 4 it has 256 x 256 tiles, one workgroup per compute unit.  Operands go from memory
+// straight to LDS (no registers, no LDS store instructions), 32 components a stage, STAGES stages in a ring: while stage s is
+// multiplied, s + 1 is there (its first operands are read in s's last step, so that no barrier leaves the matrix cores idle) and the
+// ones behind it are on their way, across the border from one tile to the next.  A stage's rows are 64 bytes; the 16-byte piece c of
+// row r lies at place c ^ (r / 2 % 4) of its row (the lanes ask memory for their pieces in that order), which spreads the eight
+// rows of a read over all banks.
+// A workgroup keeps its queries and sweeps a chunk of the item tiles.  The items are the row operand: a lane's sixteen results of a block
+// are sixteen items of ONE query, so a block without survivors costs ten three-way maxima and one compare.  A lane with survivors puts
+// its sixteen results in the wavefront's queue in LDS; when that is full, all lanes go through it, four results of two entries each, and
+// survivors go to lists owned by one (query, chunk, wavefront row) with the fill counts in LDS.  (Looked through on the spot, result by
+// result, a block with two survivors took some 700 cycles of a wavefront: 245,760 items x 128 x 4,096 queries with 500 survivors each
+// 541 us, 430 so, 275 without survivors.)
+// 4,096 queries x 1,000,000 items: 1.09 PFLOP/s with 512 components (a large product of the matrix library reaches 1.16 on this part),
+// 0.90 with 128, where the compares are a third of the issued instructions.  knn_f16_kernel's 128 x 128 tiles reached 0.72 with 576.
+#include <algorithm>
+#include "dsx_screen.h"
+
+namespace dsx {
+
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
+
+constexpr int kF16Xcds = 8;
+constexpr uint32_t kF16Step = 32;   // components a stage
+
+struct F16SweepArgs {
+    const _Float16* Q;
+    const _Float16* I;      // of the range's first item
+    uint32_t ld;            // halves per row
+    uint32_t batch, n;      // valid queries, valid items of this range
+    uint32_t tiles_q, tiles_i, chunks, tiles_per_chunk;
+    uint32_t group;         // query tiles that sit on one XCD together
+    uint64_t* seg;          // [query][chunks * WI][seg_cap]
+    uint32_t* seg_count;    // [query][kF16ListStride]
+    uint32_t seg_cap;
+    CandArgs cand;          // bounds, column offset, and the shared lists a full list spills into
+    const float* norm;      // layers: norms of the range's items
+    const float* bias;      // layers: [n], or NULL
+    const float* e1;        // layers: [batch] error of a query's sum per unit of an item's norm
+    float bias_raise;       // layers: what a bias is raised by, per unit of it
+    _Float16* Z;            // kF16Store: [batch][ldz]
+    uint64_t ldz;
+    const float* scale;     // kF16Store: [batch] what a query's sums are multiplied by (a power of two)
+};
+
+constexpr uint32_t kF16Queue = 32;   // entries of a wavefront's queue
+
+template <int WI, int WQ, int STAGES> constexpr uint32_t f16_sweep_lds(int mode)
+{
+    return STAGES * (128 * WI + 64 * WQ) * 64 + (mode != kF16Scores ? 2 * (128 + 4) * WI * 4 : 0) +
+           (mode != kF16Store ? WI * WQ * (kF16Queue * 80 + 64 * 4) : 0);
+}
+
+template <int WI, int WQ, int STAGES, int MODE>
+__global__ __launch_bounds__(64 * WI * WQ) __attribute__((amdgpu_waves_per_eu(2, 2))) void f16_sweep_kernel(F16SweepArgs a)
+{
+    constexpr uint32_t WAVES = WI * WQ, BI = 128 * WI, BQ = 64 * WQ, STAGE = (BI + BQ) * 64;
+    constexpr uint32_t PI = BI / 16 / WAVES, PQ = BQ / 16 / WAVES;   // 1 KiB pieces (16 rows) of a stage per wavefront
+    static_assert(PI * WAVES * 16 == BI && PQ * WAVES * 16 == BQ, "whole pieces");
+    extern __shared__ __attribute__((aligned(16))) unsigned char f16_lds[];
+    // layers, two tiles each: what the items' sums start from, and the largest norm of 32 items
+    float* sStart = reinterpret_cast<float*>(f16_lds + STAGES * STAGE);
+    float* sMost = sStart + 2 * BI;
+    // the wavefronts' queues (sixteen results; then the bound, e1, the largest norm, the item and the query) and their lists' fill counts
+    unsigned char* after = f16_lds + STAGES * STAGE + (MODE != kF16Scores ? 2 * (128 + 4) * WI * 4 : 0);
+    float (*sResult)[16] = reinterpret_cast<float (*)[16]>(after) + (threadIdx.x >> 6) * kF16Queue;
+    uint4* sEntry = reinterpret_cast<uint4*>(after + WAVES * kF16Queue * 64) + (threadIdx.x >> 6) * kF16Queue;
+    uint32_t* sFill = reinterpret_cast<uint32_t*>(after + WAVES * kF16Queue * 80) + (threadIdx.x & ~63u);
+
+    const uint32_t total = a.tiles_q * a.chunks;
+    uint32_t wg = blockIdx.x;
+    {
+        const uint32_t per_xcd = (total + kF16Xcds - 1) / kF16Xcds;
+        const uint32_t xcd = wg % kF16Xcds, local = wg / kF16Xcds;
+        wg = xcd * per_xcd + local;
+        if (local >= per_xcd || wg >= total) return;
+    }
+    // groups of query tiles one after the other, all chunks of a group together
+    const uint32_t block = wg / (a.group * a.chunks), in_block = wg - block * a.group * a.chunks;
+    const uint32_t members = min(a.group, a.tiles_q - block * a.group);
+    const uint32_t tq = block * a.group + in_block % members, chunk = in_block / members;
+    const uint32_t row0 = tq * BQ;
+    const uint32_t t0 = chunk * a.tiles_per_chunk, t1 = min(t0 + a.tiles_per_chunk, a.tiles_i);
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t wi = wave / WQ, wq = wave % WQ, l32 = lane & 31, lhi = lane >> 5;
+
+    uint32_t q[2];
+    const uint32_t list = chunk * WI + wi;
+    float bound[2];
+#pragma unroll
+    for (int j = 0; j < 2; j++) q[j] = row0 + wq * 64 + j * 32 + l32;
+    if constexpr (MODE != kF16Store) {
+        if (t0 >= t1) {   // more chunks than tiles: empty lists (the same for the whole workgroup)
+            const uint32_t r = row0 + wq * 64 + lane;
+            if (r < a.batch) a.seg_count[(uint64_t)r * kF16ListStride + list] = 0;
+            return;
+        }
+        sFill[lane] = 0;   // (the wavefront's own)
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            bound[j] = __uint_as_float(0x7fc00000u);   // queries beyond the batch: NaN, which nothing reaches
+            if (q[j] < a.batch) {
+                const uint32_t key = a.cand.row_bound[q[j]];
+                bound[j] = key ? key_score(key) : -__builtin_inff();   // key 0: no bound yet, every number passes
+            }
+        }
+    } else if (t0 >= t1) return;
+
+    // What an item's sum starts from (its bias, raised by the roundings of a sum that holds it; an item of infinite norm always passes)
+    // and its norm: of tile t's items, a lane each, asked for a tile ahead.
+    float e1[2] = {0.0f, 0.0f};
+    float start_next = 0.0f, norm_next = 0.0f;
+    auto ask = [&](uint32_t t) __attribute__((always_inline)) {
+        const uint32_t c = t * BI + tid;
+        start_next = -__builtin_inff();
+        norm_next = 0.0f;
+        if (tid >= BI || t >= t1 || c >= a.n) return;
+        const float b = a.bias ? a.bias[c] : 0.0f, norm = a.norm[c];
+        start_next = (norm == __builtin_inff() && b == b) ? norm : b == -__builtin_inff() ? b : b + fabsf(b) * a.bias_raise;
+        norm_next = (norm == __builtin_inff()) ? 0.0f : norm;
+    };
+    auto put = [&](uint32_t t) __attribute__((always_inline)) {
+        if (tid >= BI) return;   // (whole wavefronts)
+        sStart[(t & 1) * BI + tid] = start_next;
+        if constexpr (MODE == kF16Layer) {
+            float m = norm_next;
+#pragma unroll
+            for (int d = 1; d < 32; d *= 2) m = fmaxf(m, __shfl_xor(m, d));
+            if (l32 == 0) sMost[(t & 1) * (BI / 32) + tid / 32] = m;
+        }
+    };
+    if constexpr (MODE != kF16Scores) {
+        if constexpr (MODE == kF16Layer) {
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+                if (q[j] < a.batch) e1[j] = a.e1[q[j]];
+        }
+        ask(t0);
+        put(t0);
+        ask(t0 + 1);
+    }
+
+    // Operands on their way: the stage of cursor (dt, dk) goes into ring place dp.  The cursor stops at the last stage (what is asked for
+    // beyond it is that stage again, and never used).
+    const uint32_t nk = a.ld / kF16Step;
+    const uint32_t voff = ((lane >> 2) * a.ld + (((lane & 3) ^ ((lane >> 3) & 3)) * 8)) * 2;   // this lane's bytes into a piece
+    const uint64_t piece_bytes = (uint64_t)a.ld * 32;   // 16 rows
+    const char* gI = reinterpret_cast<const char*>(a.I) + ((uint64_t)t0 * BI / 16 + wave * PI) * piece_bytes + voff;
+    const char* gQ = reinterpret_cast<const char*>(a.Q) + ((uint64_t)row0 / 16 + wave * PQ) * piece_bytes + voff;
+    uint32_t dt = t0, dk = 0, dp = 0;
+    auto request = [&]() __attribute__((always_inline)) {
+        typedef const __attribute__((address_space(1))) void* Src;
+        typedef __attribute__((address_space(3))) void* Dst;
+        unsigned char* place = f16_lds + dp * STAGE;
+#pragma unroll
+        for (uint32_t p = 0; p < PI; p++)
+            __builtin_amdgcn_global_load_lds((Src)(gI + p * piece_bytes), (Dst)(place + (wave * PI + p) * 1024), 16, 0, 0);
+#pragma unroll
+        for (uint32_t p = 0; p < PQ; p++)
+            __builtin_amdgcn_global_load_lds((Src)(gQ + p * piece_bytes), (Dst)(place + BI * 64 + (wave * PQ + p) * 1024), 16, 0, 0);
+        dp = (dp + 1 == STAGES) ? 0 : dp + 1;
+        if (dk + 1 < nk) {
+            dk++;
+            gI += kF16Step * 2;
+            gQ += kF16Step * 2;
+        } else if (dt + 1 < t1) {
+            dt++;
+            dk = 0;
+            gI += (uint64_t)BI * a.ld * 2 - (nk - 1) * kF16Step * 2;
+            gQ -= (nk - 1) * kF16Step * 2;
+        }
+    };
+    constexpr int PER = PI + PQ;
+    // waits until at most `stages` of the stages asked for last are outstanding, then for the other wavefronts
+#define F16_WAIT(STAGES_LEFT)                                                                    \
+    do {                                                                                         \
+        if constexpr ((STAGES_LEFT) * PER == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); \
+        else if constexpr ((STAGES_LEFT) * PER == 4) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");  \
+        else if constexpr ((STAGES_LEFT) * PER == 6) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");  \
+        else if constexpr ((STAGES_LEFT) * PER == 8) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");  \
+        else if constexpr ((STAGES_LEFT) * PER == 12) asm volatile("s_waitcnt vmcnt(12)" ::: "memory"); \
+        else static_assert((STAGES_LEFT) * PER == 0, "a count for this many requests");          \
+        __builtin_amdgcn_s_barrier();                                                            \
+        asm volatile("" ::: "memory");                                                           \
+    } while (0)
+
+    const uint32_t swz = (lhi ^ ((l32 >> 1) & 3)) * 16;
+    const uint32_t offI = (wi * 128 + l32) * 64 + swz, offQ = BI * 64 + (wq * 64 + l32) * 64 + swz;
+    half8 fi[2][4], fq[2][2];
+    auto fetch = [&](int set, uint32_t place, int ks) __attribute__((always_inline)) {
+        const unsigned char* pi = f16_lds + place * STAGE + (ks ? (offI ^ 32u) : offI);
+        const unsigned char* pq = f16_lds + place * STAGE + (ks ? (offQ ^ 32u) : offQ);
+#pragma unroll
+        for (int i = 0; i < 4; i++) fi[set][i] = *reinterpret_cast<const half8*>(pi + i * 2048);
+#pragma unroll
+        for (int j = 0; j < 2; j++) fq[set][j] = *reinterpret_cast<const half8*>(pq + j * 2048);
+    };
+    floatx16 acc[4][2];
+    // (a multiplication first, whose wait is then for the reads of the step before and not for the first of these; then the next
+    // step's six reads among the others)
+    auto order = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < 6; r++) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+    };
+    auto multiply = [&](int set) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fi[set][i], fq[set][j], acc[i][j], 0, 0, 0);
+    };
+
+    uint32_t queued = 0;   // wave-uniform
+    auto settle = [&]() __attribute__((always_inline)) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        // (both halves of the queue at once: their reads, and their counts, are waited for together)
+        constexpr int H = kF16Queue / 16;
+        float x[H][4];
+        uint32_t ql[H], col0[H], at[H], passes[H];
+#pragma unroll
+        for (int h = 0; h < H; h++) {
+            const uint32_t p = h * 16 + lane / 4;
+            const float4 v = *reinterpret_cast<const float4*>(&sResult[p][lane % 4 * 4]);
+            const uint4 w = sEntry[p];
+            x[h][0] = v.x; x[h][1] = v.y; x[h][2] = v.z; x[h][3] = v.w;
+            ql[h] = MODE == kF16Layer ? w.w % 64 : w.y % 64;
+            col0[h] = (MODE == kF16Layer ? w.w / 64 * 4 : w.w) + lane % 4 * 8;
+            passes[h] = 0;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float raised = MODE == kF16Layer ? fmaf(__uint_as_float(w.y), __uint_as_float(w.z), x[h][e]) : x[h][e];
+                if (raised >= __uint_as_float(w.x) && col0[h] + e < a.n) passes[h] |= 1u << e;   // (items beyond the range are zero padding)
+            }
+            if (p >= queued) passes[h] = 0;
+        }
+#pragma unroll
+        for (int h = 0; h < H; h++)
+            if (passes[h] != 0) at[h] = atomicAdd(&sFill[ql[h]], (uint32_t)__popc(passes[h])) & 0x7fffffffu;
+#pragma unroll
+        for (int h = 0; h < H; h++) {
+            if (passes[h] == 0) continue;
+            const uint32_t r = row0 + wq * 64 + ql[h];
+            uint64_t* mine = a.seg + ((uint64_t)r * (a.chunks * WI) + list) * a.seg_cap;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                if (!((passes[h] >> e) & 1)) continue;
+                const uint64_t word = ((uint64_t)score_key(x[h][e]) << 32) | (uint32_t)~(a.cand.col_offset + col0[h] + e);
+                if (at[h] < a.seg_cap) mine[at[h]] = word;
+                else {   // this list is full: the query's shared list
+                    const uint32_t s = atomicAdd(&a.cand.cand_count[r], 1u);
+                    if (s < a.cand.cand_cap) a.cand.cand[(uint64_t)r * a.cand.cand_cap + s] = word;
+                    else {
+                        *a.cand.overflow = 1u;
+                        atomicOr(&sFill[ql[h]], 0x80000000u);   // (the row is done otherwise: nothing more of it is wanted)
+                    }
+                }
+                at[h]++;
+            }
+        }
+        queued = 0;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+            if (sFill[j * 32 + l32] & 0x80000000u) bound[j] = __uint_as_float(0x7fc00000u);
+    };
+    // most: largest norm of the block's items, which stands for theirs here: what passes is listed as it is, and raised by its own
+    // norm where the lists are read.  (No item's raised sum is above its sum raised by most: the multiply-add rounds monotonically.)
+    auto compare = [&](const floatx16& s, int j, uint32_t item0, float most) __attribute__((always_inline)) {
+        float top = fmaxf(fmaxf(s[0], s[1]), s[2]);
+#pragma unroll
+        for (int v = 3; v < 15; v += 2) top = fmaxf(fmaxf(top, s[v]), s[v + 1]);
+        top = fmaxf(top, s[15]);
+        if constexpr (MODE == kF16Layer) top = fmaf(e1[j], most, top);
+        uint64_t hot = __builtin_amdgcn_ballot_w64(top >= bound[j]);
+        while (hot != 0) {
+            if (queued == kF16Queue) settle();
+            // the lowest lanes, as many as there is room for
+            const uint32_t place = queued + __builtin_amdgcn_mbcnt_hi((uint32_t)(hot >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)hot, 0u));
+            const bool mine = ((hot >> lane) & 1) != 0 && place < kF16Queue;
+            if (mine) {
+#pragma unroll
+                for (int g = 0; g < 4; g++) *reinterpret_cast<float4*>(&sResult[place][4 * g]) = make_float4(s[4 * g], s[4 * g + 1], s[4 * g + 2], s[4 * g + 3]);
+                if constexpr (MODE == kF16Layer)   // (fewer than 2^28 items: their table would not fit otherwise; item0 is a multiple of 4)
+                    sEntry[place] = make_uint4(__float_as_uint(bound[j]), __float_as_uint(e1[j]), __float_as_uint(most), item0 * 16 + j * 32 + l32);
+                else sEntry[place] = make_uint4(__float_as_uint(bound[j]), j * 32 + l32, 0, item0);
+            }
+            const uint64_t taken = __builtin_amdgcn_ballot_w64(mine);
+            queued += (uint32_t)__builtin_popcountll(taken);
+            hot &= ~taken;
+        }
+    };
+
+#pragma unroll
+    for (int s = 0; s < STAGES - 1; s++) request();
+    F16_WAIT(STAGES - 2);   // stage 0 is there
+    fetch(0, 0, 0);
+    uint32_t cp = 0;   // ring place of the stage that is multiplied
+    auto stage = [&]() __attribute__((always_inline)) {
+        F16_WAIT(STAGES - 3);   // the next stage is there, and every wavefront is done with the one before this
+        request();
+        const uint32_t np = (cp + 1 == STAGES) ? 0 : cp + 1;
+        fetch(1, cp, 1);
+        multiply(0);
+        order();
+        fetch(0, np, 0);
+        multiply(1);
+        order();
+        cp = np;
+    };
+    for (uint32_t t = t0; t < t1; t++) {
+        if constexpr (MODE == kF16Scores) {
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+#pragma unroll
+                    for (int v = 0; v < 16; v++) acc[i][j][v] = 0.0f;
+        } else {
+            const float* from = sStart + (t & 1) * BI + wi * 128 + 4 * lhi;
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    const float4 s = *reinterpret_cast<const float4*>(from + i * 32 + 8 * g);
+#pragma unroll
+                    for (int j = 0; j < 2; j++) {
+                        acc[i][j][4 * g] = s.x; acc[i][j][4 * g + 1] = s.y; acc[i][j][4 * g + 2] = s.z; acc[i][j][4 * g + 3] = s.w;
+                    }
+                }
+        }
+        __builtin_amdgcn_s_setprio(1);
+        stage();
+        if constexpr (MODE != kF16Scores) {
+            // (every wavefront has read this tile's starts and is done with the tile before, whose places take the next tile's, which
+            // the barriers of the stages behind this make visible)
+            put(t + 1);
+            ask(t + 2);
+        }
+        for (uint32_t kt = 1; kt < nk; kt++) stage();
+        __builtin_amdgcn_s_setprio(0);
+        if constexpr (MODE != kF16Store) {
+            const uint32_t item0 = t * BI + wi * 128 + 4 * lhi;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float most = MODE == kF16Layer ? sMost[(t & 1) * (BI / 32) + wi * 4 + i] : 0.0f;
+#pragma unroll
+                for (int j = 0; j < 2; j++) compare(acc[i][j], j, item0 + i * 32, most);
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                if (q[j] >= a.batch) continue;
+                const float scale = a.scale[q[j]];
+                // (both halves of a lane pair take the same branch: they hold the same query)
+                _Float16* dst = a.Z + (uint64_t)q[j] * a.ldz + (uint64_t)t * BI + wi * 128 + lhi * 16;
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    uint32_t w[4][2];
+#pragma unroll
+                    for (int g = 0; g < 4; g++)
+#pragma unroll
+                        for (int p = 0; p < 2; p++) {
+                            typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+                            const float x = acc[i][j][4 * g + 2 * p] * scale, y = acc[i][j][4 * g + 2 * p + 1] * scale;
+                            // raised by half a unit in the last place and a subnormal's, and no lower than the lowest half: what
+                            // rounds to nearest then lies above
+                            half2v h;
+                            h[0] = (_Float16)fmaxf(fmaf(fabsf(x), 4.932e-4f, x) + 6.0e-8f, -65504.0f);
+                            h[1] = (_Float16)fmaxf(fmaf(fabsf(y), 4.932e-4f, y) + 6.0e-8f, -65504.0f);
+                            w[g][p] = __builtin_bit_cast(uint32_t, h);
+                        }
+                    // a lane holds items 8 g + 4 lhi + 0..3: after the exchange the lower half's lanes hold items 0..15, the others 16..31
+#pragma unroll
+                    for (int g = 0; g < 2; g++) {
+                        u32x4v out;
+#pragma unroll
+                        for (int p = 0; p < 2; p++) {
+                            const auto r = __builtin_amdgcn_permlane32_swap(w[g][p], w[g + 2][p], false, false);
+                            out[p] = r[0];
+                            out[2 + p] = r[1];
+                        }
+                        *reinterpret_cast<u32x4v*>(dst + i * 32 + g * 8) = out;
+                    }
+                }
+            }
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (what was asked for beyond the end must not arrive in another workgroup's LDS)
+    if constexpr (MODE != kF16Store) {
+        settle();
+        const uint32_t r = row0 + wq * 64 + lane;
+        if (r < a.batch) a.seg_count[(uint64_t)r * kF16ListStride + list] = min(sFill[lane] & 0x7fffffffu, a.seg_cap);
+    }
+#undef F16_WAIT
+}
+
+template <int WI, int WQ, int STAGES, int MODE> static int launch_f16_sweep(F16SweepArgs& a)
+{
+    constexpr uint32_t lds = f16_sweep_lds<WI, WQ, STAGES>(MODE);
+    static bool sized[64] = {};   // per device: the kernel's LDS limit is raised once
+    const int dev = ctx().device;
+    if (dev < 0 || dev >= 64 || !sized[dev]) {
+        DSX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&f16_sweep_kernel<WI, WQ, STAGES, MODE>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        if (dev >= 0 && dev < 64) sized[dev] = true;
+    }
+    const uint32_t total = a.tiles_q * a.chunks, grid = (total + kF16Xcds - 1) / kF16Xcds * kF16Xcds;
+    hipLaunchKernelGGL((f16_sweep_kernel<WI, WQ, STAGES, MODE>), dim3(grid), dim3(64 * WI * WQ), lds, ctx().stream, a);
+    DSX_LAUNCH_CHECK("f16_sweep_kernel");
+    return DSX_OK;
+}
+
+static F16SweepArgs f16_args(const F16Job& j)
+{
+    F16SweepArgs a{};
+    a.Q = (const _Float16*)j.Q; a.I = (const _Float16*)j.items;
+    a.ld = j.ld; a.batch = j.batch; a.n = j.n;
+    a.norm = j.norm; a.bias = j.bias; a.e1 = j.e1; a.bias_raise = j.bias_raise;
+    a.cand = j.cand;
+    a.Z = (_Float16*)j.Z; a.ldz = j.ldz; a.scale = j.scale;
+    a.tiles_q = (j.batch + 255) / 256;
+    return a;
+}
+
+// Eight query tiles to an XCD: with 512 components their operands are half of its L2 (4, 8 and 16 are level within 2 %).
+constexpr uint32_t kF16Group = 8;
+
+int f16_sweep_run(const F16Job& j, bool layer, uint32_t* lists)
+{
+    F16SweepArgs a = f16_args(j);
+    a.tiles_i = (j.n + 255) / 256;
+    a.chunks = std::max(1u, std::min(std::min(kF16ListStride / 2, a.tiles_i), ((uint32_t)ctx().num_cus + a.tiles_q - 1) / a.tiles_q));
+    a.tiles_per_chunk = (a.tiles_i + a.chunks - 1) / a.chunks;
+    a.group = std::min(a.tiles_q, kF16Group);
+    *lists = a.chunks * 2;
+    a.seg = j.seg; a.seg_count = j.seg_count; a.seg_cap = j.seg_words / *lists;
+    return layer ? launch_f16_sweep<2, 4, 4, kF16Layer>(a) : launch_f16_sweep<2, 4, 4, kF16Scores>(a);
+}
+
+int f16_store_run(const F16Job& j)
+{
+    F16SweepArgs a = f16_args(j);
+    // 128 x 256 tiles, four wavefronts, where 256 x 256 ones leave half the GPU without work (256 x 1,024 x 27,278: 28 us against 35)
+    const uint32_t big = (j.n + 255) / 256;
+    const bool small = a.tiles_q * big < (uint32_t)ctx().num_cus;
+    a.tiles_i = small ? (j.n + 127) / 128 : big;
+    a.chunks = std::min(a.tiles_i, std::max(1u, (uint32_t)ctx().num_cus / a.tiles_q));
+    a.tiles_per_chunk = (a.tiles_i + a.chunks - 1) / a.chunks;
+    a.chunks = (a.tiles_i + a.tiles_per_chunk - 1) / a.tiles_per_chunk;
+    a.group = std::min(a.tiles_q, kF16Group);
+    return small ? launch_f16_sweep<1, 4, 4, kF16Store>(a) : launch_f16_sweep<2, 4, 4, kF16Store>(a);
+}
+
+}  // namespace dsx

@@ -12,8 +12,7 @@
 // of "score >= current k-th score" (preactivation_bound in dsx_device.h), lists are merged under the total order (score
 // descending, column ascending), and a row whose list fills up is recomputed from scratch on the device.
 #include <algorithm>
-#include "dsx_device.h"
-#include "dsx_internal.h"
+#include "dsx_screen.h"
 
 namespace dsx {
 
@@ -72,22 +71,24 @@ struct LayerWorkspace {
     uint32_t* overflow;    // [64] unused flag word of the shared epilogue
     uint32_t* redo_done;   // [layer_redo_groups]
     uint64_t* cand;        // [batch][cap]; after the last range: the lists of rows that are computed again
-    ScreenWorkspace screen;   // where the ranges are screened in 16 bits
+    ScreenTable table;     // where the layer is screened in 16 bits: the table, if the caller keeps none, and what the call works in
+    ScreenWorkspace screen;
     size_t bytes;
 };
 
 static size_t layer_clear_words(uint32_t batch) { return (size_t)3 * batch + 64 + layer_redo_groups(batch); }
 
-static LayerWorkspace layer_layout(void* base, uint32_t batch, uint32_t n0, uint32_t k, uint32_t cap, bool ranges, bool screened,
+// screened: 0 no, 1 yes, 2 yes and the caller has the table
+static LayerWorkspace layer_layout(void* base, uint32_t batch, uint32_t n0, uint32_t k, uint32_t cap, bool ranges, int screened,
                                    uint32_t kdim, uint32_t n)
 {
     LayerWorkspace w;
     char* p = (char*)base;
     const uint32_t ld0 = (n0 + 3) / 4 * 4;
     w.block_scores = (float*)p;
-    p += align256((size_t)batch * ld0 * sizeof(float));
+    if (!screened) p += align256((size_t)batch * ld0 * sizeof(float));
     w.best = (uint64_t*)p;
-    p += align256((size_t)batch * k * sizeof(uint64_t));
+    if (!screened) p += align256((size_t)batch * k * sizeof(uint64_t));
     w.row_bound = (uint32_t*)p;
     w.cand_count = w.row_bound + batch;
     w.row_flag = w.cand_count + batch;
@@ -96,10 +97,15 @@ static LayerWorkspace layer_layout(void* base, uint32_t batch, uint32_t n0, uint
     p += align256(layer_clear_words(batch) * sizeof(uint32_t));
     w.cand = (uint64_t*)p;
     if (ranges) p += align256(std::max<size_t>((size_t)batch * cap, layer_redo_words(batch, k)) * sizeof(uint64_t));
+    w.table = ScreenTable{};
     w.screen = ScreenWorkspace{};
     if (screened) {
-        w.screen = screen_layout(p, batch, kdim, n, true, kLayerCandCap);
+        w.screen = screen_layout(p, batch, kdim, n);
         p += w.screen.bytes;
+    }
+    if (screened == 1) {
+        w.table = screen_table(p, kdim, n);
+        p += w.table.bytes;
     }
     w.bytes = (size_t)(p - (char*)base);
     return w;
@@ -173,6 +179,12 @@ int dsx_fc_topk_pays(uint32_t batch, uint32_t k_dim, uint32_t n, uint32_t activa
            ((k <= 32 && batch >= 1536 && products >= 2e10) || (k <= 128 && batch >= 2048 && products >= 1e11));
 }
 
+int dsx_fc_topk_screened_pays(uint32_t batch, uint32_t k_dim, uint32_t n, uint32_t activation, uint32_t k)
+{
+    (void)k;
+    return batch > 0 && k_dim >= 32 && k_dim <= 4096 && n >= 8192 && activation == DSX_ACT_SIGMOID;
+}
+
 int dsx_fc_topk_supported(uint32_t ldx, const float* X, uint32_t activation, const dsx_act_params* params, const float* filter_mul)
 {
     return layer_activation_supported(activation, params) && filter_mul == nullptr && ((uintptr_t)X % 16) == 0 && (ldx % 4) == 0;
@@ -185,7 +197,7 @@ int dsx_fc_topk_supported(uint32_t ldx, const float* X, uint32_t activation, con
 static int fc_topk_common(const float* X, uint32_t ldx, const float* W, const float* bias, uint32_t batch, uint32_t kdim, uint32_t n,
                           uint32_t activation, const dsx_act_params* params, uint32_t k, float* keys, uint32_t* values, uint32_t position,
                           const uint32_t* index, const uint64_t* filter_start, const uint64_t* filter_end, const uint32_t* filter_index,
-                          const void* x_planes, const void* w_planes)
+                          const void* x_planes, const void* w_planes, const void* table)
 {
     DSX_REQUIRE_INIT();
     DSX_CHECK_ARG(X && W && keys && values, "dsx_fc_topk: null device pointer");
@@ -206,35 +218,56 @@ static int fc_topk_common(const float* X, uint32_t ldx, const float* W, const fl
     const uint32_t cap = ctx().knobs.fc_topk_candidate_capacity ? ctx().knobs.fc_topk_candidate_capacity : kLayerCandCap;   // tests lower it to reach the overflow path with small inputs
     const uint32_t n0 = layer_first_columns(n, k);
     const bool ranges = n0 < n;
-    bool screened = ranges && !x_planes && screen_takes(batch, kdim, n, true) && screen_layer_pays(batch, kdim, n, k);
+    int screened = x_planes ? 0 : table ? 2 : (ranges && screen_takes(batch, kdim, n, true) && screen_layer_pays(batch, kdim, n, k)) ? 1 : 0;
     LibScratch& ws = g_layer_ws_of[current_lane()];
-    int reserved = lib_scratch_reserve(ws, layer_layout(nullptr, batch, n0, k, cap, ranges, screened, kdim, n).bytes, "dsx_fc_topk workspace", screened);
-    if (reserved == DSX_ENOMEM && screened) {   // the 16-bit copies (up to 8 GiB) do not fit beside what is there: fp32 ranges need none
-        screened = false;
+    int reserved = lib_scratch_reserve(ws, layer_layout(nullptr, batch, n0, k, cap, ranges || screened, screened, kdim, n).bytes, "dsx_fc_topk workspace", screened);
+    if (reserved == DSX_ENOMEM && screened) {   // the 16-bit copies (up to 8 GiB) or the sums do not fit beside what is there: fp32 ranges need none
+        screened = 0;
         reserved = lib_scratch_reserve(ws, layer_layout(nullptr, batch, n0, k, cap, ranges, screened, kdim, n).bytes, "dsx_fc_topk workspace");
     }
     if (reserved) return reserved;
-    const LayerWorkspace w = layer_layout(ws.ptr, batch, n0, k, cap, ranges, screened, kdim, n);
+    const LayerWorkspace w = layer_layout(ws.ptr, batch, n0, k, cap, ranges || screened, screened, kdim, n);
+    LayerRedo redo{};
+    redo.X = X; redo.W = W; redo.bias = bias; redo.ldx = ldx; redo.ldw = n; redo.kdim = kdim; redo.n = n; redo.k = k;
+    redo.act = activation;
+    redo.slope = params ? params->slope : 0.01f;
+    redo.alpha = params ? params->alpha : 1.0f;
+    redo.lambda = params ? params->lambda : 1.0f;
+    redo.position = position; redo.index = index; redo.fstart = filter_start; redo.fend = filter_end; redo.fidx = filter_index;
+    redo.row_flag = w.row_flag; redo.partial = w.cand; redo.done = w.redo_done; redo.keys = keys; redo.values = values;
+    const uint32_t clear_words = (uint32_t)layer_clear_words(batch);
+    if (screened) {
+        hipLaunchKernelGGL(layer_clear_kernel, dim3((clear_words + 255) / 256), dim3(256), 0, ctx().stream, w.row_bound, clear_words);
+        DSX_LAUNCH_CHECK("layer_clear_kernel");
+        const ScreenTable t = table ? screen_table(const_cast<void*>(table), kdim, n) : w.table;
+        int rc = table ? DSX_OK : screen_build(t, W, n, n, kdim);
+        if (rc) return rc;
+        ScreenJob j{};
+        j.X = X; j.ldx = ldx; j.batch = batch; j.dim = kdim; j.n = n; j.k = k;
+        j.bias = bias; j.act = activation; j.slope = redo.slope; j.alpha = redo.alpha; j.lambda = redo.lambda;
+        j.position = position; j.index = index; j.fstart = filter_start; j.fend = filter_end; j.fidx = filter_index;
+        j.keys = keys; j.values = values;
+        j.row_flag = w.row_flag; j.told = flag_word;
+        j.cand = w.cand; j.cand_count = w.cand_count; j.cap = cap; j.overflow = w.overflow;
+        if ((rc = screen_rows(j, t, w.screen, nullptr))) return rc;
+        if ((rc = screen_run(j, t, w.screen))) return rc;
+        return layer_redo_run(redo, batch);
+    }
     const uint32_t ld0 = (n0 + 3) / 4 * 4;
     hipStream_t s = ctx().stream;
 
     // first block: the layer as a matrix, then the scanning top-K (filtered: indexes beyond the block are ignored)
     const uint32_t wrows = split_rows_padded(n);
     FcOrder order;
-    order.as_candidates = ranges && !screened;
+    order.as_candidates = ranges;
     int rc = x_planes ? fc_split_run(x_planes, w_planes, wrows, 0, bias, w.block_scores, ld0, batch, kdim, n0, 0, activation, params, nullptr, nullptr)
                       : fc_run(X, ldx, W, n, 0, bias, w.block_scores, ld0, batch, kdim, n0, 0, activation, params, nullptr, nullptr, nullptr, order);
     if (rc) return rc;
     if (!ranges)
         return topk_run(w.block_scores, ld0, n0, batch, k, keys, values, position, index, filter_start, filter_end, filter_index, nullptr, 0,
                         nullptr, 0, 0, 0);
-    const uint32_t clear_words = (uint32_t)layer_clear_words(batch);
     hipLaunchKernelGGL(layer_clear_kernel, dim3((clear_words + 255) / 256), dim3(256), 0, s, w.row_bound, clear_words);
     DSX_LAUNCH_CHECK("layer_clear_kernel");
-    if (screened) {
-        rc = screen_prepare(w.screen, X, ldx, batch, W, n, bias, n, kdim, true, n0, w.row_flag, flag_word, nullptr);
-        if (rc) return rc;
-    }
     rc = topk_run(w.block_scores, ld0, n0, batch, k, nullptr, nullptr, position, index, filter_start, filter_end, filter_index, nullptr, 0,
                   w.best, 1, 0, 1, w.row_bound);
     if (rc) return rc;
@@ -242,12 +275,9 @@ static int fc_topk_common(const float* X, uint32_t ldx, const float* W, const fl
     // A bound taken over `done` columns lets about k * width / done of the next `width` columns pass: ranges grow by a factor that
     // keeps that near an eighth of a list (the sample's own items, which score high and pass as well, come on top).
     const uint32_t growth = std::max(4u, cap / (8 * k));
-    // Screened, the first block's scores give the bounds and nothing else: what passes is scored by one kernel wherever it lies (equal
-    // columns are to tie, and its sums have not that block's order), so the first range starts at column 0.
-    uint32_t done = screened ? 0 : n0;
+    uint32_t done = n0;
     while (done < n) {
-        const bool first = done == 0;
-        uint32_t ncols = (uint32_t)std::min<uint64_t>((uint64_t)n - done, first ? n0 + (uint64_t)n0 * growth / 128 * 128 : (uint64_t)done * growth / 128 * 128);
+        uint32_t ncols = (uint32_t)std::min<uint64_t>((uint64_t)n - done, (uint64_t)done * growth / 128 * 128);
         if (n - done - ncols < 128) ncols = n - done;   // no sliver of a last range
         CandArgs cand{};
         cand.row_bound = w.row_bound;
@@ -260,9 +290,8 @@ static int fc_topk_common(const float* X, uint32_t ldx, const float* W, const fl
         cand.slope = params ? params->slope : 0.01f;
         cand.alpha = params ? params->alpha : 1.0f;
         cand.lambda = params ? params->lambda : 1.0f;
-        if (screened) rc = screen_candidates(w.screen, X, ldx, batch, kdim, true, bias, ncols, cand, false, first);
-        else rc = x_planes ? fc_split_candidates_run(x_planes, w_planes, wrows, done, batch, kdim, ncols, cand, true, bias ? bias + done : nullptr)
-                           : fc_layer_candidates_run(X, ldx, W + done, n, bias ? bias + done : nullptr, batch, kdim, ncols, cand);
+        rc = x_planes ? fc_split_candidates_run(x_planes, w_planes, wrows, done, batch, kdim, ncols, cand, true, bias ? bias + done : nullptr)
+                      : fc_layer_candidates_run(X, ldx, W + done, n, bias ? bias + done : nullptr, batch, kdim, ncols, cand);
         if (rc) return rc;
         done += ncols;
         LayerRefresh r{};
@@ -273,18 +302,10 @@ static int fc_topk_common(const float* X, uint32_t ldx, const float* W, const fl
             r.keys = keys;
             r.values = values;
         }
-        r.n = n; r.first_columns = screened ? 0 : n0; r.fresh = first;
+        r.n = n; r.first_columns = n0;
         rc = layer_refresh_run(r, batch);
         if (rc) return rc;
     }
-    LayerRedo redo{};
-    redo.X = X; redo.W = W; redo.bias = bias; redo.ldx = ldx; redo.ldw = n; redo.kdim = kdim; redo.n = n; redo.k = k;
-    redo.act = activation;
-    redo.slope = params ? params->slope : 0.01f;
-    redo.alpha = params ? params->alpha : 1.0f;
-    redo.lambda = params ? params->lambda : 1.0f;
-    redo.position = position; redo.index = index; redo.fstart = filter_start; redo.fend = filter_end; redo.fidx = filter_index;
-    redo.row_flag = w.row_flag; redo.partial = w.cand; redo.done = w.redo_done; redo.keys = keys; redo.values = values;
     return layer_redo_run(redo, batch);
 }
 
@@ -295,7 +316,32 @@ int dsx_fc_topk(const float* X, uint32_t ldx, const float* W, const float* bias,
                 const uint32_t* index, const uint64_t* filter_start, const uint64_t* filter_end, const uint32_t* filter_index)
 {
     return fc_topk_common(X, ldx, W, bias, batch, kdim, n, activation, params, k, keys, values, position, index, filter_start, filter_end,
-                          filter_index, nullptr, nullptr);
+                          filter_index, nullptr, nullptr, nullptr);
+}
+
+uint64_t dsx_screen_table_bytes(uint32_t n, uint32_t kdim)
+{
+    return screen_table(nullptr, kdim, n).bytes;
+}
+
+int dsx_screen_table_build(const float* W, uint32_t ldw, uint32_t n, uint32_t kdim, void* table)
+{
+    DSX_REQUIRE_INIT();
+    DSX_CHECK_ARG(W && table, "dsx_screen_table_build: null device pointer");
+    DSX_CHECK_ARG(((uintptr_t)table % 256) == 0, "dsx_screen_table_build: the table is not 256-byte aligned");
+    DSX_CHECK_ARG(n > 0 && kdim > 0 && kdim <= 4096 && ldw >= n, "dsx_screen_table_build: n = %u, k = %u, ldw = %u", n, kdim, ldw);
+    return screen_build(screen_table(table, kdim, n), W, ldw, n, kdim);
+}
+
+int dsx_fc_topk_screened(const float* X, uint32_t ldx, const float* W, const void* table, const float* bias, uint32_t batch, uint32_t kdim,
+                         uint32_t n, uint32_t activation, const dsx_act_params* params, uint32_t k, float* keys, uint32_t* values,
+                         uint32_t position, const uint32_t* index, const uint64_t* filter_start, const uint64_t* filter_end,
+                         const uint32_t* filter_index)
+{
+    DSX_CHECK_ARG(table && ((uintptr_t)table % 256) == 0, "dsx_fc_topk_screened: the table is missing or not 256-byte aligned");
+    DSX_CHECK_ARG(kdim <= 4096, "dsx_fc_topk_screened: k = %u (4,096 at most)", kdim);
+    return fc_topk_common(X, ldx, W, bias, batch, kdim, n, activation, params, k, keys, values, position, index, filter_start, filter_end,
+                          filter_index, nullptr, nullptr, table);
 }
 
 int dsx_fc_topk_split(const float* X, uint32_t ldx, const float* W, const void* x_planes, const void* w_planes, const float* bias,
@@ -306,7 +352,7 @@ int dsx_fc_topk_split(const float* X, uint32_t ldx, const float* W, const void* 
     DSX_CHECK_ARG(x_planes && w_planes, "dsx_fc_topk_split: null planes");
     DSX_CHECK_ARG(((uintptr_t)x_planes % 16) == 0 && ((uintptr_t)w_planes % 16) == 0, "dsx_fc_topk_split: planes must be 16-byte aligned");
     return fc_topk_common(X, ldx, W, bias, batch, kdim, n, activation, params, k, keys, values, position, index, filter_start, filter_end,
-                          filter_index, x_planes, w_planes);
+                          filter_index, x_planes, w_planes, nullptr);
 }
 
 }  // extern "C"

@@ -167,7 +167,6 @@ struct LayerRefresh {
     uint32_t* values;
     uint32_t n;
     uint32_t first_columns;   // width of the first block (scanned with the filter applied)
-    bool fresh;               // best holds nothing yet, and row_bound is replaced by the k-th of these candidates
 };
 int layer_refresh_run(const LayerRefresh& r, uint32_t batch);
 // The rows that row_flag marks, from X and W: their results go to keys / values.  partial: layer_redo_words words of scratch; done:
@@ -201,42 +200,11 @@ int knn_to_f16(const float* src, bool colmajor, uint64_t src_ld, uint32_t rows_v
 int knn_f16_scores_run(const void* queries16, const void* items16, uint32_t ld, uint32_t batch, uint32_t n, float* Z, uint32_t ldz,
                        const CandArgs* cand);
 int knn_refresh(uint64_t* best, const uint64_t* cand, uint32_t* cand_count, uint32_t cap, uint32_t k, uint32_t* row_bound, uint32_t batch,
-                const uint64_t* seg = nullptr, uint32_t* seg_count = nullptr, uint32_t chunks = 0, uint32_t seg_cap = 0, bool fresh = false);
+                const uint64_t* seg = nullptr, uint32_t* seg_count = nullptr, uint32_t lists = 0, uint32_t seg_cap = 0);
 // fp16 storage, candidate mode of a column range: one workgroup per tile, or (long ranges) workgroups that sweep a chunk of the
-// range each and keep (row, chunk) lists of their own (seg [queries][chunks][seg_words / chunks], seg_count [queries][64]); full
-// lists spill into cand's shared ones.  mode: see dsx_testing_set_knn_f16_sweep.  *chunks_used is what knn_refresh needs to know.
+// range each and keep lists of their own (seg [queries][lists][seg_words / lists], seg_count [queries][kF16ListStride]); full
+// lists spill into cand's shared ones.  mode: see dsx_testing_set_knn_f16_sweep.  *lists_used is what knn_refresh needs to know.
 int knn_f16_candidates_run(const void* queries16, const void* items16, uint32_t ld, uint32_t batch, uint32_t n, const CandArgs& cand,
-                           uint64_t* seg, uint32_t* seg_count, uint32_t seg_words, int mode, uint32_t* chunks_used);
-// 16-bit screening of candidates for the fp32 searches (dsx_screen.hip): the table's two row-major copies (f16, fp32), the rows in f16
-// and the lists of a sweep.  screen_prepare lays them out (flag: one word, or one per row for layers, set where the error of a 16-bit
-// sum has no bound; told: a host-visible word set with it; first: the columns that give a layer its first bounds); screen_candidates screens ncols columns from cand.col_offset on and leaves
-// the fp32 scores of what passed in cand's lists.  All results come from there, so that equal columns have equal scores: `first` marks
-// the range whose bounds were taken from another kernel's sums (it starts at column 0).
-struct ScreenWorkspace {
-    void* items16;
-    float* rows32;
-    void* queries16;
-    float* eps;
-    float* slack;
-    uint32_t* admit;
-    uint32_t* stats;
-    uint64_t* seg;
-    uint32_t* seg_count;
-    uint32_t list_words;
-    size_t bytes;
-};
-// Nearest neighbours, in pinned memory: the largest norm of the table, a sample of the norms and how many they are, and (told) the flag.
-struct ScreenNotes {
-    float largest, sum;
-    uint32_t number, flag;
-};
-bool screen_takes(uint32_t batch, uint32_t dim, uint64_t n, bool layer);
-bool screen_layer_pays(uint32_t batch, uint32_t dim, uint64_t n, uint32_t k);
-bool screen_search_pays(uint32_t batch, uint32_t dim, uint64_t n, uint32_t k, bool blocks, float norm_ratio);
-ScreenWorkspace screen_layout(void* base, uint32_t batch, uint32_t dim, uint64_t n, bool layer, uint32_t list_words);
-int screen_prepare(const ScreenWorkspace& w, const float* X, uint32_t ldx, uint32_t batch, const float* W, uint64_t ldw, const float* bias,
-                   uint64_t n, uint32_t dim, bool layer, uint32_t first, uint32_t* flag, uint32_t* told, ScreenNotes* notes);
-int screen_candidates(const ScreenWorkspace& w, const float* X, uint32_t ldx, uint32_t batch, uint32_t dim, bool layer, const float* bias,
-                      uint32_t ncols, const CandArgs& cand, bool report_overflow, bool first);
+                           uint64_t* seg, uint32_t* seg_count, uint32_t seg_words, int mode, uint32_t* lists_used);
 
 }  // namespace dsx

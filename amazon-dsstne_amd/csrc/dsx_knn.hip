@@ -12,10 +12,10 @@
 // the library's would have to be allocated inside the capture) and for operands that are not 16-byte aligned.  With fp16 storage (dsx_knn_search_f16) the scores come from the f16 MFMA kernel of dsx_knn_f16.hip instead, through
 // the same three steps.
 #include <algorithm>
+#include <cstring>
 #include <vector>
 #include <hip/hip_runtime.h>
-#include "dsx_device.h"
-#include "dsx_internal.h"
+#include "dsx_screen.h"
 
 namespace dsx {
 
@@ -53,9 +53,11 @@ struct KnnWorkspace {
     uint32_t* overflow;     // [1] (+ padding)
     uint64_t* cand;         // [queries][kCandCap]
     void* queries16;        // fp16 storage: the query batch, [queries rounded up to 256][ld] halves; split products: its bf16 planes
-    uint64_t* seg;          // fp16 storage only: [queries][chunks][kCandCap / chunks], the lists of a sweep (knn_f16_sweep_run)
-    uint32_t* seg_count;    // fp16 storage only: [queries][64]
-    ScreenWorkspace screen; // fp32 storage, where screen_takes says so
+    uint64_t* seg;          // fp16 storage only: [queries][lists][kCandCap / lists], the lists of a sweep in f16
+    uint32_t* seg_count;    // fp16 storage only: [queries][kF16ListStride]
+    ScreenTable table;      // fp32 storage, where screen_takes says so: at the workspace's start, whatever the number of queries
+    ScreenWorkspace screen;
+    uint32_t* row_flag;     // [queries] screened: rows without a result
     size_t bytes;
 };
 
@@ -70,13 +72,25 @@ static uint32_t knn_block_lists(uint32_t num_queries, uint32_t ncols, uint32_t k
     return knn_block_guided(num_queries, ncols, k) ? topk_guided_parts(ncols, num_queries) : topk_segments(num_queries, ncols, false);
 }
 
+static bool knn_screens(uint32_t rows_padded, uint32_t num_queries, uint32_t k, uint32_t dim)
+{
+    return screen_takes(num_queries, dim, rows_padded, false) &&
+           screen_search_pays(num_queries, dim, rows_padded, k, rows_padded <= knn_block_columns(rows_padded, num_queries), 1.0f);
+}
+
 static KnnWorkspace knn_layout(void* base, uint32_t rows_padded, uint32_t num_queries, uint32_t k, bool f16 = false, uint32_t dim = 0,
-                               bool split = false, bool screen = true)
+                               bool split = false, bool screen = true, bool table = false)
 {
     const uint32_t cb = knn_block_columns(rows_padded, num_queries);
     const uint32_t blocks = (rows_padded + cb - 1) / cb;
     KnnWorkspace w;
     char* p = (char*)base;
+    screen = screen && !f16 && !split && knn_screens(rows_padded, num_queries, k, dim);
+    w.table = ScreenTable{};
+    if (screen || table) {
+        w.table = screen_table(p, dim, rows_padded);
+        p += w.table.bytes;
+    }
     w.block_scores = (float*)p;
     p += align256((size_t)num_queries * cb * sizeof(float));
     w.seg_max = knn_few_queries(num_queries) ? (float*)p : nullptr;
@@ -85,10 +99,11 @@ static KnnWorkspace knn_layout(void* base, uint32_t rows_padded, uint32_t num_qu
     // (a last block narrower than the others may be cut into more parts than they are, but not into more than fill half the GPU)
     const uint32_t lists = std::max(knn_block_lists(num_queries, cb, k), std::max(topk_segments(num_queries, cb, false), (uint32_t)ctx().num_cus / (2 * std::max(1u, num_queries)) + 2));
     p += align256((size_t)num_queries * blocks * lists * k * sizeof(uint64_t));
-    w.row_bound = (uint32_t*)p;             // row_bound, cand_count and overflow are cleared together
+    w.row_bound = (uint32_t*)p;             // row_bound, cand_count, row_flag and overflow are cleared together
     w.cand_count = w.row_bound + num_queries;
-    w.overflow = w.cand_count + num_queries;
-    p += align256(((size_t)2 * num_queries + 64) * sizeof(uint32_t));
+    w.row_flag = w.cand_count + num_queries;
+    w.overflow = w.row_flag + num_queries;
+    p += align256(((size_t)3 * num_queries + 64) * sizeof(uint32_t));
     w.cand = (uint64_t*)p;
     p += align256((size_t)num_queries * kCandCap * sizeof(uint64_t));
     w.queries16 = p;
@@ -99,13 +114,12 @@ static KnnWorkspace knn_layout(void* base, uint32_t rows_padded, uint32_t num_qu
         w.seg = (uint64_t*)p;
         p += align256((size_t)num_queries * kCandCap * sizeof(uint64_t));
         w.seg_count = (uint32_t*)p;
-        p += align256((size_t)num_queries * 64 * sizeof(uint32_t));
+        p += align256((size_t)num_queries * kF16ListStride * sizeof(uint32_t));
     }
     if (split) p += align256((size_t)split_plane_bytes(num_queries, dim));
     w.screen = ScreenWorkspace{};
-    if (screen && !f16 && !split && screen_takes(num_queries, dim, rows_padded, false) &&
-        screen_search_pays(num_queries, dim, rows_padded, k, blocks == 1, 1.0f)) {
-        w.screen = screen_layout(p, num_queries, dim, rows_padded, false, kCandCap);
+    if (screen) {
+        w.screen = screen_layout(p, num_queries, dim, rows_padded);
         p += w.screen.bytes;
     }
     w.bytes = (size_t)(p - (char*)base);
@@ -114,13 +128,20 @@ static KnnWorkspace knn_layout(void* base, uint32_t rows_padded, uint32_t num_qu
 
 // What a search of any number of queries up to num_queries needs: a workspace of a batch is used for smaller ones too, and fewer
 // queries may need more (5,000 rows, k = 100: 64 queries 3.634 MB, 65 queries 3.618, because 64 leave more lists per query).
-// About 40 ns per query count, once per table.
-static size_t knn_workspace_most(uint32_t rows_padded, uint32_t num_queries, uint32_t k, bool f16, uint32_t dim, bool split, bool screen = true)
+// About 40 ns per query count, once per table.  *table: whether that includes the table of a screened search (which then lies at the start of
+// it for every number of queries).
+static size_t knn_workspace_most(uint32_t rows_padded, uint32_t num_queries, uint32_t k, bool f16, uint32_t dim, bool split, bool screen = true,
+                                 bool* table = nullptr)
 {
     size_t most = 0;
-    for (uint64_t q = std::min(1u, num_queries); q <= num_queries; q++)
-        most = std::max(most, knn_layout(nullptr, rows_padded, (uint32_t)q, k, f16, dim, split, screen).bytes);
-    return most;
+    bool any = false;
+    for (uint64_t q = std::min(1u, num_queries); q <= num_queries; q++) {
+        const KnnWorkspace w = knn_layout(nullptr, rows_padded, (uint32_t)q, k, f16, dim, split, screen);
+        most = std::max(most, w.bytes - w.table.bytes);
+        any = any || w.table.bytes != 0;
+    }
+    if (table) *table = any;
+    return most + (any ? screen_table(nullptr, dim, rows_padded).bytes : 0);
 }
 
 // Where the scores of a column range come from: the fp32 table through fc_gemm_kernel, or the fp16 table through knn_f16_kernel.
@@ -235,7 +256,7 @@ static int knn_search_blocks(const KnnWorkspace& w, const KnnOperands& op, uint3
     return rc;
 }
 
-// What the preparation of a screened search finds, stored by it in pinned memory and read while the first block runs.
+// What the preparation of a screened search finds, stored by it in pinned memory and read before the search goes on.
 static ScreenNotes* g_knn_notes = nullptr;
 static hipEvent_t g_knn_noted = nullptr;
 
@@ -245,6 +266,14 @@ static void knn_notes_release()
     if (g_knn_noted) hipEventDestroy(g_knn_noted);
     g_knn_notes = nullptr;
     g_knn_noted = nullptr;
+}
+
+// Whether what the preparation found speaks against screening.
+static bool knn_unfit(const ScreenNotes& notes, uint32_t num_queries, uint32_t dim, uint32_t M, uint32_t k)
+{
+    const float average = notes.number != 0 ? notes.sum / (float)notes.number : 0.0f;
+    return notes.flag != 0 || notes.largest > 65504.0f ||
+           (notes.largest > 0.0f && !screen_search_pays(num_queries, dim, M, k, M <= knn_block_columns(M, num_queries), notes.largest / average));
 }
 
 static int knn_notes_ready()
@@ -258,34 +287,22 @@ static int knn_notes_ready()
     return DSX_OK;
 }
 
-// First block as above, the rest in candidate mode, screened in 16 bits where asked for (fp32 storage).  *overflowed tells the caller
-// to redo the search without screening, or block by block; *unfit (screened only), that the preparation found the table or the queries
-// unfit for screening (norms beyond f16's range, or one so large that the others' bounds are worth nothing) and the search ended there.
+// First block as above, the rest in candidate mode.  *overflowed tells the caller to redo the search block by block.
 static int knn_search_candidates(const KnnWorkspace& w, const KnnOperands& op, uint32_t M, uint32_t num_queries, uint32_t k, float* scores,
-                                 uint32_t* indexes, KnnTimer& t, bool screened, bool* overflowed, bool* unfit)
+                                 uint32_t* indexes, KnnTimer& t, bool* overflowed)
 {
     hipStream_t s = ctx().stream;
     const uint32_t cb = knn_block_columns(op.rows_padded, num_queries);
-    const uint32_t clear_words = 2 * num_queries + 64;
+    const uint32_t clear_words = 3 * num_queries + 64;
     hipLaunchKernelGGL(knn_clear_kernel, dim3((clear_words + 255) / 256), dim3(256), 0, s, w.row_bound, clear_words);
-    if (w.seg_count) hipLaunchKernelGGL(knn_clear_kernel, dim3((num_queries * 64 + 255) / 256), dim3(256), 0, s, w.seg_count, num_queries * 64);
     // The first block only has to give every query a usable bound; a quarter of a column block does (measured on 2 M items x 4,096
     // queries: 8 K to 32 K columns are level, the full 64 K cost 0.1 ms more in stores and scan).  A width set by the caller is kept.
     uint32_t done = std::min(cb, M);
-    // (screened, later columns cost a tenth of the first block's: 8 K)
-    if (!ctx().knobs.knn_block_columns) done = std::min<uint32_t>(done, screened ? 8192u : std::max<uint32_t>(1024, cb / 4 / 1024 * 1024));
+    if (!ctx().knobs.knn_block_columns) done = std::min<uint32_t>(done, std::max<uint32_t>(1024, cb / 4 / 1024 * 1024));
     t.start(s);
-    int rc = DSX_OK;
-    if (screened) {
-        if ((rc = knn_notes_ready())) return rc;
-        rc = screen_prepare(w.screen, op.queries, op.dim, num_queries, op.items, op.rows_padded, nullptr, M, op.dim, false, 0, w.overflow,
-                            &g_knn_notes->flag, g_knn_notes);
-        if (rc) return rc;
-        DSX_HIP(hipEventRecord(g_knn_noted, s));
-    }
     FcOrder order;
-    order.as_candidates = !screened;
-    rc = op.into_matrix(0, done, num_queries, w.block_scores, cb, order);
+    order.as_candidates = true;
+    int rc = op.into_matrix(0, done, num_queries, w.block_scores, cb, order);
     if (rc) return rc;
     t.stop(s, t.gemm);
     t.start(s);
@@ -293,35 +310,18 @@ static int knn_search_candidates(const KnnWorkspace& w, const KnnOperands& op, u
                   1, w.row_bound);
     if (rc) return rc;
     t.stop(s, t.topk);
-    // Screened, the block's scores give the bounds and nothing else: what passes is scored by one kernel wherever it lies (equal items
-    // are to tie, and its sums have not this block's order), so the first range starts at column 0.
-    const uint32_t seen = done;
-    if (screened) {
-        done = 0;
-        // (asked again and again: the first block runs for another 100 us, and a wait that sleeps wakes up later than that)
-        hipError_t noted;
-        while ((noted = hipEventQuery(g_knn_noted)) == hipErrorNotReady) {}
-        (void)hipGetLastError();   // (not ready is not an error of the next launch)
-        DSX_HIP(noted);
-        const ScreenNotes notes = *g_knn_notes;
-        const float average = notes.number != 0 ? notes.sum / (float)notes.number : 0.0f;
-        *unfit = notes.flag != 0 || (notes.largest > 0.0f && !screen_search_pays(num_queries, op.dim, M, k, M <= cb, notes.largest / average));
-        if (*unfit) return DSX_OK;
-    }
     while (done < M) {
-        const bool first = screened && done == 0;
-        // a multiple of the tile width keeps every range's first column 16-byte aligned
-        const uint32_t ncols = (uint32_t)std::min<uint64_t>((uint64_t)M - done, first ? (uint64_t)seen * 5 / 128 * 128 : (uint64_t)done * 4 / 128 * 128);
+        // a multiple of the tile width keeps every range's first column 16-byte aligned (done is a multiple of 1,024)
+        const uint32_t ncols = (uint32_t)std::min<uint64_t>((uint64_t)M - done, (uint64_t)done * 4);
         t.start(s);
         const CandArgs cand{w.row_bound, w.cand, w.cand_count, kCandCap, done, w.overflow};
-        uint32_t chunks = 0;
-        rc = screened ? screen_candidates(w.screen, op.queries, op.dim, num_queries, op.dim, false, nullptr, ncols, cand, true, first)
-                      : op.into_candidates(done, ncols, num_queries, cand, w.seg, w.seg_count, &chunks);
+        uint32_t lists = 0;
+        rc = op.into_candidates(done, ncols, num_queries, cand, w.seg, w.seg_count, &lists);
         if (rc) return rc;
         t.stop(s, t.gemm);
         t.start(s);
-        rc = knn_refresh(w.partial, w.cand, w.cand_count, kCandCap, k, w.row_bound, num_queries, chunks ? w.seg : nullptr, w.seg_count, chunks,
-                         chunks ? kCandCap / chunks : 0, first);
+        rc = knn_refresh(w.partial, w.cand, w.cand_count, kCandCap, k, w.row_bound, num_queries, lists ? w.seg : nullptr, w.seg_count, lists,
+                         lists ? kCandCap / lists : 0);
         if (rc) return rc;
         t.stop(s, t.topk);
         done += ncols;
@@ -330,6 +330,46 @@ static int knn_search_candidates(const KnnWorkspace& w, const KnnOperands& op, u
     rc = topk_merge(w.partial, 1, k, scores, indexes, num_queries);
     if (rc) return rc;
     t.stop(s, t.topk);
+    uint32_t flag = 0;
+    DSX_HIP(hipMemcpyAsync(&flag, w.overflow, sizeof(flag), hipMemcpyDeviceToHost, s));
+    DSX_HIP(hipStreamSynchronize(s));
+    *overflowed = flag != 0;
+    return DSX_OK;
+}
+
+// Screened in 16 bits (fp32 storage).  built: the workspace's table is there already (dsx_knn_prepare), and what it is like has been
+// looked at.  *overflowed tells the caller to redo the search without screening; *unfit, that the table or the queries were found unfit
+// for it first (norms beyond f16's range, or one so large that the others' bounds would be worth little).
+static int knn_search_screened(const KnnWorkspace& w, const KnnOperands& op, uint32_t M, uint32_t num_queries, uint32_t k, float* scores,
+                               uint32_t* indexes, KnnTimer& t, bool built, bool* overflowed, bool* unfit)
+{
+    hipStream_t s = ctx().stream;
+    const uint32_t clear_words = 3 * num_queries + 64;
+    hipLaunchKernelGGL(knn_clear_kernel, dim3((clear_words + 255) / 256), dim3(256), 0, s, w.row_bound, clear_words);
+    ScreenJob j{};
+    j.X = op.queries; j.ldx = op.dim; j.batch = num_queries; j.dim = op.dim; j.n = M; j.k = k;
+    j.act = DSX_ACT_LINEAR;
+    j.keys = scores; j.values = indexes;
+    j.row_flag = w.row_flag; j.told = w.overflow;
+    j.cand = w.cand; j.cand_count = w.cand_count; j.cap = kCandCap; j.overflow = w.overflow;
+    t.start(s);
+    int rc = DSX_OK;
+    if (!built) {
+        if ((rc = knn_notes_ready())) return rc;
+        if ((rc = screen_build(w.table, op.items, op.rows_padded, M, op.dim))) return rc;
+    }
+    if ((rc = screen_rows(j, w.table, w.screen, built ? nullptr : g_knn_notes))) return rc;
+    if (!built) {
+        DSX_HIP(hipEventRecord(g_knn_noted, s));
+        hipError_t noted;   // (asked again and again: a wait that sleeps wakes up late)
+        while ((noted = hipEventQuery(g_knn_noted)) == hipErrorNotReady) {}
+        (void)hipGetLastError();   // (not ready is not an error of the next launch)
+        DSX_HIP(noted);
+        *unfit = knn_unfit(*g_knn_notes, num_queries, op.dim, M, k);
+        if (*unfit) return DSX_OK;
+    }
+    if ((rc = screen_run(j, w.table, w.screen))) return rc;
+    t.stop(s, t.gemm);
     uint32_t flag = 0;
     DSX_HIP(hipMemcpyAsync(&flag, w.overflow, sizeof(flag), hipMemcpyDeviceToHost, s));
     DSX_HIP(hipStreamSynchronize(s));
@@ -400,10 +440,10 @@ int dsx_knn_f16_convert_items(const float* items, uint32_t rows_padded, uint32_t
 
 // Both precisions: workspace, the two paths, timing.
 static int knn_search_common(KnnOperands& op, uint32_t padding, uint32_t num_queries, uint32_t k, float* scores, uint32_t* indexes, void* workspace,
-                             size_t workspace_bytes, float* elapsed_ms, bool aligned, const float* queries_f32)
+                             size_t workspace_bytes, float* elapsed_ms, bool aligned, const float* queries_f32, bool built = false)
 {
-    const size_t full = knn_layout(nullptr, op.rows_padded, num_queries, k, op.f16, op.dim, op.split).bytes;
-    const size_t need = knn_layout(nullptr, op.rows_padded, num_queries, k, op.f16, op.dim, op.split, false).bytes;
+    const size_t full = knn_layout(nullptr, op.rows_padded, num_queries, k, op.f16, op.dim, op.split, true, built).bytes;
+    const size_t need = knn_layout(nullptr, op.rows_padded, num_queries, k, op.f16, op.dim, op.split, false, built).bytes;
     bool screen = full != need;   // the screening's copies of the table (up to 8 GiB) where there is room for them: fp32 needs none
     if (workspace) {
         DSX_CHECK_ARG(workspace_bytes >= need, "dsx_knn_search: workspace of %zu bytes, %zu needed", workspace_bytes, need);
@@ -419,7 +459,7 @@ static int knn_search_common(KnnOperands& op, uint32_t padding, uint32_t num_que
         if (reserved) return reserved;
         workspace = ws.ptr;
     }
-    const KnnWorkspace w = knn_layout(workspace, op.rows_padded, num_queries, k, op.f16, op.dim, op.split, screen);
+    const KnnWorkspace w = knn_layout(workspace, op.rows_padded, num_queries, k, op.f16, op.dim, op.split, screen, built);
     const uint32_t M = op.rows_padded - padding;
     hipStream_t s = ctx().stream;
     KnnTimer t;
@@ -447,11 +487,11 @@ static int knn_search_common(KnnOperands& op, uint32_t padding, uint32_t num_que
     const bool many = M > knn_block_columns(op.rows_padded, num_queries);
     bool screened = may && w.screen.bytes != 0 && !ctx().knobs.knn_block_columns;
     bool redo = true, unfit = false;
-    if (rc == DSX_OK && screened) rc = knn_search_candidates(w, op, M, num_queries, k, scores, indexes, t, true, &redo, &unfit);
+    if (rc == DSX_OK && screened) rc = knn_search_screened(w, op, M, num_queries, k, scores, indexes, t, built, &redo, &unfit);
     if (unfit) screened = false;
     const bool candidates = may && (screened || many);
     if (rc == DSX_OK && candidates && (!screened || redo) && many)
-        rc = knn_search_candidates(w, op, M, num_queries, k, scores, indexes, t, false, &redo, nullptr);
+        rc = knn_search_candidates(w, op, M, num_queries, k, scores, indexes, t, &redo);
     g_knn_last_path = !candidates ? DSX_KNN_PATH_BLOCKS : (redo ? DSX_KNN_PATH_CANDIDATES_REDONE : DSX_KNN_PATH_CANDIDATES);
     if (rc == DSX_OK && redo) rc = knn_search_blocks(w, op, M, num_queries, k, scores, indexes, t);
     if (elapsed_ms) {
@@ -464,11 +504,9 @@ static int knn_search_common(KnnOperands& op, uint32_t padding, uint32_t num_que
     return rc;
 }
 
-extern "C" {
-
-int dsx_knn_search(const float* items, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,
-                   uint32_t num_queries, uint32_t k, float* scores, uint32_t* indexes, void* workspace, size_t workspace_bytes,
-                   float* elapsed_ms)
+static int knn_search_fp32(const float* items, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,
+                           uint32_t num_queries, uint32_t k, float* scores, uint32_t* indexes, void* workspace, size_t workspace_bytes,
+                           float* elapsed_ms, bool built)
 {
     DSX_REQUIRE_INIT();
     DSX_CHECK_ARG(items && queries && scores && indexes, "dsx_knn_search: null device pointer");
@@ -482,7 +520,51 @@ int dsx_knn_search(const float* items, uint32_t rows_padded, uint32_t padding, u
     op.rows_padded = rows_padded;
     op.dim = dim;
     const bool aligned = ((uintptr_t)items % 16) == 0 && ((uintptr_t)queries % 16) == 0 && (rows_padded % 4) == 0 && (dim % 4) == 0;
-    return knn_search_common(op, padding, num_queries, k, scores, indexes, workspace, workspace_bytes, elapsed_ms, aligned, nullptr);
+    return knn_search_common(op, padding, num_queries, k, scores, indexes, workspace, workspace_bytes, elapsed_ms, aligned, nullptr, built);
+}
+
+extern "C" {
+
+int dsx_knn_search(const float* items, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,
+                   uint32_t num_queries, uint32_t k, float* scores, uint32_t* indexes, void* workspace, size_t workspace_bytes,
+                   float* elapsed_ms)
+{
+    return knn_search_fp32(items, rows_padded, padding, dim, queries, num_queries, k, scores, indexes, workspace, workspace_bytes, elapsed_ms, false);
+}
+
+int dsx_knn_prepare(const float* items, uint32_t rows_padded, uint32_t padding, uint32_t dim, uint32_t num_queries, uint32_t k, void* workspace,
+                    size_t workspace_bytes, int* prepared)
+{
+    DSX_REQUIRE_INIT();
+    DSX_CHECK_ARG(items && workspace && prepared, "dsx_knn_prepare: null pointer");
+    DSX_CHECK_ARG(padding < rows_padded && dim > 0 && num_queries > 0 && k >= 1 && k <= 256, "dsx_knn_prepare: rows_padded %u, padding %u, dim %u, %u queries, k = %u",
+                  rows_padded, padding, dim, num_queries, k);
+    DSX_CHECK_ARG(((uintptr_t)workspace % 256) == 0, "dsx_knn_prepare: workspace is not 256-byte aligned");
+    *prepared = 0;
+    bool table = false;
+    const size_t full = knn_workspace_most(rows_padded, num_queries, k, false, dim, false, true, &table);
+    const bool aligned = ((uintptr_t)items % 16) == 0 && (rows_padded % 4) == 0 && (dim % 4) == 0;
+    if (!table || !aligned || workspace_bytes < full) return DSX_OK;
+    const uint32_t M = rows_padded - padding;
+    const ScreenTable t = screen_table(workspace, dim, rows_padded);
+    if (int rc = screen_build(t, items, rows_padded, M, dim)) return rc;
+    uint32_t stats[3];
+    DSX_HIP(hipMemcpyAsync(stats, t.stats, sizeof(stats), hipMemcpyDeviceToHost, ctx().stream));
+    DSX_HIP(hipStreamSynchronize(ctx().stream));
+    ScreenNotes notes{};
+    std::memcpy(&notes.largest, &stats[0], sizeof(float));
+    std::memcpy(&notes.sum, &stats[1], sizeof(float));
+    notes.number = stats[2];
+    *prepared = !knn_unfit(notes, num_queries, dim, M, k);
+    return DSX_OK;
+}
+
+int dsx_knn_search_prepared(const float* items, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,
+                            uint32_t num_queries, uint32_t k, float* scores, uint32_t* indexes, void* workspace, size_t workspace_bytes,
+                            float* elapsed_ms)
+{
+    DSX_CHECK_ARG(workspace, "dsx_knn_search_prepared: null workspace");
+    return knn_search_fp32(items, rows_padded, padding, dim, queries, num_queries, k, scores, indexes, workspace, workspace_bytes, elapsed_ms, true);
 }
 
 int dsx_knn_search_split(const void* item_planes, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,

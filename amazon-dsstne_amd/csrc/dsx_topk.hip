@@ -20,8 +20,7 @@
 //   * rows split over several segments write packed partial lists that a second small kernel merges.
 #include <algorithm>
 #include <type_traits>
-#include "dsx_device.h"
-#include "dsx_internal.h"
+#include "dsx_screen.h"
 
 namespace dsx {
 
@@ -1596,16 +1595,16 @@ int topk_merge(const uint64_t* partial, uint32_t slots, uint32_t k, float* keys,
 
 // Exact KNN with candidate lists: merges a row's running best list (k packed words, best first) with the candidates the last
 // column range left behind, writes the best k back, raises the row's bound to their k-th key and empties the candidate
-// lists.  fresh: the candidates are all there is (no best list yet; the bound becomes their k-th key).  One wavefront per row.  The candidates are the row's shared list (cand, cand_count) and, after a sweep
-// (knn_f16_sweep_kernel), its `chunks` private lists seg[row][chunk][seg_cap] with fill counts seg_count[row][64].
+// lists.  One wavefront per row.  The candidates are the row's shared list (cand, cand_count) and, after a sweep in f16, its `lists`
+// private ones, seg[row][list][seg_cap] with fill counts seg_count[row][kF16ListStride].
 template <int R>
 __global__ __launch_bounds__(kWave) void knn_refresh_kernel(uint64_t* best, const uint64_t* cand, uint32_t* cand_count, uint32_t cap,
                                                             uint32_t k, uint32_t* row_bound, const uint64_t* seg, uint32_t* seg_count,
-                                                            uint32_t chunks, uint32_t seg_cap, int fresh)
+                                                            uint32_t lists, uint32_t seg_cap)
 {
     using List = WaveTopK<R>;
     __shared__ uint64_t sStage[List::kStageWords];
-    __shared__ uint32_t sStart[kWave + 1];
+    __shared__ uint32_t sStart[kF16ListStride + 1];
     const uint32_t b = blockIdx.x;
     const uint32_t lane = threadIdx.x;
     List list;
@@ -1613,7 +1612,7 @@ __global__ __launch_bounds__(kWave) void knn_refresh_kernel(uint64_t* best, cons
     uint64_t* mine = best + (uint64_t)b * k;
     for (uint32_t p0 = 0; p0 < k; p0 += kWave) {
         const uint32_t p = p0 + lane;
-        const uint64_t word = (p < k && !fresh) ? mine[p] : 0ull;
+        const uint64_t word = (p < k) ? mine[p] : 0ull;
         list.offer(word != 0, word);
     }
     const uint32_t n = min(cand_count[b], cap);
@@ -1624,62 +1623,64 @@ __global__ __launch_bounds__(kWave) void knn_refresh_kernel(uint64_t* best, cons
         list.offer(word != 0, word);
     }
     if (seg) {
-        // entry e of the chunks' lists laid end to end: lane c holds where chunk c starts
-        uint32_t* counts = seg_count + (uint64_t)b * kWave;
-        const uint32_t mine_count = (lane < chunks) ? min(counts[lane], seg_cap) : 0u;
-        uint32_t incl = mine_count;
-#pragma unroll
-        for (int d = 1; d < kWave; d *= 2) {
-            const uint32_t below = __shfl_up(incl, d);
-            if (lane >= (uint32_t)d) incl += below;
-        }
+        // entry e of the lists laid end to end: sStart[l] is where list l starts
+        const uint32_t* counts = seg_count + (uint64_t)b * kF16ListStride;
+        uint32_t before = 0;
         if (lane == 0) sStart[0] = 0;
-        sStart[lane + 1] = incl;
+        for (uint32_t l0 = 0; l0 < kF16ListStride; l0 += kWave) {
+            uint32_t incl = (l0 + lane < lists) ? min(counts[l0 + lane], seg_cap) : 0u;
+#pragma unroll
+            for (int d = 1; d < kWave; d *= 2) {
+                const uint32_t below = __shfl_up(incl, d);
+                if (lane >= (uint32_t)d) incl += below;
+            }
+            sStart[l0 + lane + 1] = before + incl;
+            before += __shfl(incl, kWave - 1);
+        }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        const uint32_t total = sStart[kWave];
-        const uint64_t* lists = seg + (uint64_t)b * chunks * seg_cap;
+        const uint32_t total = sStart[kF16ListStride];
+        const uint64_t* from = seg + (uint64_t)b * lists * seg_cap;
         for (uint32_t e0 = 0; e0 < total; e0 += kWave) {
             const uint32_t e = e0 + lane;
             uint64_t word = 0;
             if (e < total) {
-                uint32_t lo = 0, hi = kWave;   // the last chunk that starts at or before e (empty chunks start where the next one does)
+                uint32_t lo = 0, hi = kF16ListStride;   // the last list that starts at or before e (empty ones start where the next one does)
                 while (hi - lo > 1) {
                     const uint32_t mid = (lo + hi) / 2;
                     if (sStart[mid] <= e) lo = mid;
                     else hi = mid;
                 }
-                word = lists[(uint64_t)lo * seg_cap + (e - sStart[lo])];
+                word = from[(uint64_t)lo * seg_cap + (e - sStart[lo])];
             }
             list.offer(word != 0, word);
         }
-        if (lane < chunks) counts[lane] = 0;
     }
     list.finish();
 #pragma unroll
     for (int r = 0; r < R; r++) {
         const uint32_t p = r * kWave + lane;
         if (p < k) mine[p] = list.q[r];
-        if (p == k - 1 && list.q[r] != 0) row_bound[b] = max(fresh ? 0u : row_bound[b], (uint32_t)(list.q[r] >> 32));
+        if (p == k - 1 && list.q[r] != 0) row_bound[b] = max(row_bound[b], (uint32_t)(list.q[r] >> 32));
     }
     if (lane == 0) cand_count[b] = 0;
 }
 
 int knn_refresh(uint64_t* best, const uint64_t* cand, uint32_t* cand_count, uint32_t cap, uint32_t k, uint32_t* row_bound, uint32_t batch,
-                const uint64_t* seg, uint32_t* seg_count, uint32_t chunks, uint32_t seg_cap, bool fresh)
+                const uint64_t* seg, uint32_t* seg_count, uint32_t lists, uint32_t seg_cap)
 {
     hipStream_t s = ctx().stream;
-    if (seg && (chunks == 0 || chunks > (uint32_t)kWave || !seg_count))
-        return set_error(DSX_EINVAL, "knn_refresh: %u chunks (1..64)", chunks);
+    if (seg && (lists == 0 || lists > kF16ListStride || !seg_count))
+        return set_error(DSX_EINVAL, "knn_refresh: %u lists (1..%u)", lists, kF16ListStride);
     if (k <= 64)
         hipLaunchKernelGGL((knn_refresh_kernel<1>), dim3(batch), dim3(kWave), 0, s, best, cand, cand_count, cap, k, row_bound, seg, seg_count,
-                           chunks, seg_cap, fresh ? 1 : 0);
+                           lists, seg_cap);
     else if (k <= 128)
         hipLaunchKernelGGL((knn_refresh_kernel<2>), dim3(batch), dim3(kWave), 0, s, best, cand, cand_count, cap, k, row_bound, seg, seg_count,
-                           chunks, seg_cap, fresh ? 1 : 0);
+                           lists, seg_cap);
     else
         hipLaunchKernelGGL((knn_refresh_kernel<4>), dim3(batch), dim3(kWave), 0, s, best, cand, cand_count, cap, k, row_bound, seg, seg_count,
-                           chunks, seg_cap, fresh ? 1 : 0);
+                           lists, seg_cap);
     DSX_LAUNCH_CHECK("knn_refresh_kernel");
     return DSX_OK;
 }
@@ -1711,7 +1712,6 @@ struct LayerRefreshArgs {
     uint32_t* values;
     uint32_t n;                // columns of the layer
     uint32_t first_columns;    // columns of the first block, whose listed columns the scanning top-K has dealt with
-    int fresh;                 // the candidates are all there is: no best list yet, row_bound is replaced and not raised
 };
 
 __device__ __forceinline__ uint32_t layer_hash(uint32_t col, uint32_t shift) { return (col * 2654435761u) >> shift; }
@@ -1783,7 +1783,7 @@ __global__ __launch_bounds__(kWave) void layer_refresh_kernel(LayerRefreshArgs a
     uint64_t* mine = a.best + (uint64_t)b * a.k;
     for (uint32_t p0 = 0; p0 < a.k; p0 += kWave) {
         const uint32_t p = p0 + lane;
-        const uint64_t word = (p < a.k && !a.fresh) ? mine[p] : 0ull;
+        const uint64_t word = (p < a.k) ? mine[p] : 0ull;
         list.offer(word != 0, word);
     }
     for (uint32_t p0 = 0; p0 < count; p0 += kWave) {
@@ -1839,7 +1839,7 @@ __global__ __launch_bounds__(kWave) void layer_refresh_kernel(LayerRefreshArgs a
     for (int r = 0; r < R; r++) {
         const uint32_t p = r * kWave + lane;
         if (p < a.k) mine[p] = list.q[r];
-        if (p == a.k - 1 && list.q[r] != 0) a.row_bound[b] = max(a.fresh ? 0u : a.row_bound[b], (uint32_t)(list.q[r] >> 32));
+        if (p == a.k - 1 && list.q[r] != 0) a.row_bound[b] = max(a.row_bound[b], (uint32_t)(list.q[r] >> 32));
     }
 }
 
@@ -1853,7 +1853,6 @@ int layer_refresh_run(const LayerRefresh& r, uint32_t batch)
     a.keys = r.keys; a.values = r.values;
     a.n = r.n;
     a.first_columns = r.first_columns;
-    a.fresh = r.fresh ? 1 : 0;
     hipStream_t s = ctx().stream;
     if (a.k <= 64) hipLaunchKernelGGL((layer_refresh_kernel<1>), dim3(batch), dim3(kWave), 0, s, a);
     else if (a.k <= 128) hipLaunchKernelGGL((layer_refresh_kernel<2>), dim3(batch), dim3(kWave), 0, s, a);

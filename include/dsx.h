@@ -322,6 +322,18 @@ int dsx_fc_topk_split(const float* X, uint32_t ldx, const float* W, const void* 
                       uint32_t batch, uint32_t k_dim, uint32_t n, uint32_t activation, const dsx_act_params* params, uint32_t k, float* keys,
                       uint32_t* values, uint32_t position, const uint32_t* index, const uint64_t* filter_start, const uint64_t* filter_end,
                       const uint32_t* filter_index);
+/* dsx_fc_topk for a caller that keeps the weights' table of the 16-bit screening (two row-major copies of W, 6 bytes per element, and the
+ * columns' norms): dsx_screen_table_build fills dsx_screen_table_bytes(n, k_dim) bytes at `table` (device, 256-byte aligned) from W
+ * [k_dim][ldw] on the selected lane's stream; it has to be built again when W changes.  k_dim is 4,096 at most.  The call computes no
+ * other results than dsx_fc_topk with its own table does; W is read for rows that have to be computed again.
+ * dsx_fc_topk_screened_pays: 1 where this is the fastest way to the top-K of an output layer. */
+uint64_t dsx_screen_table_bytes(uint32_t n, uint32_t k_dim);
+int dsx_screen_table_build(const float* W, uint32_t ldw, uint32_t n, uint32_t k_dim, void* table);
+int dsx_fc_topk_screened(const float* X, uint32_t ldx, const float* W, const void* table, const float* bias, uint32_t batch, uint32_t k_dim,
+                         uint32_t n, uint32_t activation, const dsx_act_params* params, uint32_t k, float* keys, uint32_t* values,
+                         uint32_t position, const uint32_t* index, const uint64_t* filter_start, const uint64_t* filter_end,
+                         const uint32_t* filter_index);
+int dsx_fc_topk_screened_pays(uint32_t batch, uint32_t k_dim, uint32_t n, uint32_t activation, uint32_t k);
 /* 1 where dsx_fc_topk is the faster way to the top-K, 0 where dsx_fc_forward_segmax + dsx_topk_guided are. */
 int dsx_fc_topk_pays(uint32_t batch, uint32_t k_dim, uint32_t n, uint32_t activation, uint32_t k);
 int dsx_fc_topk_supported(uint32_t ldx, const float* X, uint32_t activation, const dsx_act_params* params, const float* filter_mul);
@@ -347,6 +359,15 @@ size_t dsx_knn_workspace_bytes(uint32_t rows_padded, uint32_t dim, uint32_t num_
 /* dsx_knn_workspace_bytes holds, for 512 queries and more, two copies of the table (1.5 x its size, up to 8 GiB) that make the search
  * faster (its candidates are screened in 16 bits); a workspace of at least this size but not that one is searched without them. */
 size_t dsx_knn_workspace_bytes_least(uint32_t rows_padded, uint32_t dim, uint32_t num_queries, uint32_t k);
+/* Fills the two copies once, for a caller that searches one table many times: workspace holds dsx_knn_workspace_bytes(rows_padded, dim,
+ * num_queries, k) bytes (256-byte aligned).  *prepared: whether it did (the table may not be worth it, or unfit for it).  A prepared
+ * workspace goes with dsx_knn_search_prepared and searches of up to num_queries queries and the same items and k; nothing else may use
+ * it.  Waits for the device. */
+int dsx_knn_prepare(const float* items, uint32_t rows_padded, uint32_t padding, uint32_t dim, uint32_t num_queries, uint32_t k, void* workspace,
+                    size_t workspace_bytes, int* prepared);
+int dsx_knn_search_prepared(const float* items, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,
+                            uint32_t num_queries, uint32_t k, float* scores, uint32_t* indexes, void* workspace, size_t workspace_bytes,
+                            float* elapsed_ms);
 /* fp16 storage (astdl::knn::DataType::FP16).  The reference converts the column-major table once (KnnData::load,
  * knn/KnnData.cpp:209-216, kFloatToHalf of knn/MathUtil.cu:33-81: round to nearest even) and every query batch before the
  * GEMM (knn/KnnExactGpu.cu:108-116), multiplies fp16 operands and keeps fp32 scores.  Same arithmetic here; the fp16 table's
