@@ -211,6 +211,18 @@ void NNLayer::ForwardPropagateFullyConnected(uint32_t position, uint32_t batch, 
         return;
     }
 
+    // Softmax behind one dense source: the sums with their biases in one kernel, then the row operation.
+    if (nIn == 1 && _vIncomingSkip.empty() && !_vIncomingLayer[0]->_bFastSparse) {
+        NNLayer* src = _vIncomingLayer[0];
+        NNWeight* w = _vIncomingWeight[0];
+        NNWeight* wsrc = w->_bShared ? w->_pSharedWeight : w;
+        dsxFatal(dsx_fc_forward(src->GetUnitBuffer(), src->_stride, wsrc->_pbWeight->_pDevData, w->_bTransposed ? 1 : 0, w->_pbBias->_pDevData,
+                                pUnit, _stride, batch, src->_stride, _localStride, 0, DSX_ACT_LINEAR, &params),
+                 "NNLayer::ForwardPropagate: GEMM failure");
+        CalculateActivation(batch);
+        return;
+    }
+
     // General case, in the reference's order: bias sum, one product per source accumulated into z, skips, activation.
     NNFloat* bias[4] = {NULL, NULL, NULL, NULL};
     for (size_t i = 0; i < nIn; i++) bias[i] = _vIncomingWeight[i]->_pbBias->_pDevData;
