@@ -98,6 +98,9 @@ SIGNATURES = {
     "dsx_topk_guided": [_vp, _vp, _vp, _u32, _u32, _u32, _vp, _u32, _u32, _vp, _vp, _vp, _vp, _vp],
     "dsx_fc_topk": [_vp, _u32, _vp, _vp, _u32, _u32, _u32, _u32, C.POINTER(ActParams), _u32, _vp, _vp, _u32, _vp, _vp, _vp, _vp],
     "dsx_fc_topk_split": [_vp, _u32, _vp, _vp, _vp, _vp, _u32, _u32, _u32, _u32, C.POINTER(ActParams), _u32, _vp, _vp, _u32, _vp, _vp, _vp, _vp],
+    "dsx_screen_table_build": [_vp, _u32, _u32, _u32, _vp],
+    "dsx_fc_topk_screened": [_vp, _u32, _vp, _vp, _vp, _u32, _u32, _u32, _u32, C.POINTER(ActParams), _u32, _vp, _vp, _u32, _vp, _vp, _vp, _vp],
+    "dsx_fc_topk_screened_pays": [_u32, _u32, _u32, _u32, _u32],
     "dsx_fc_topk_pays": [_u32, _u32, _u32, _u32, _u32],
     "dsx_fc_topk_supported": [_u32, _vp, _u32, C.POINTER(ActParams), _vp],
     "dsx_fc_topk_flagged": [_int],
@@ -113,16 +116,20 @@ SIGNATURES = {
     "dsx_knn_f16_convert_items": [_vp, _u32, _u32, _u32, _vp],
     "dsx_knn_search_f16": [_vp, _u32, _u32, _u32, _vp, _u32, _u32, _vp, _vp, _vp, _sz, C.POINTER(_f32)],
     "dsx_knn_search_split": [_vp, _u32, _u32, _u32, _vp, _u32, _u32, _vp, _vp, _vp, _sz, C.POINTER(_f32)],
+    "dsx_knn_prepare": [_vp, _u32, _u32, _u32, _u32, _u32, _vp, _sz, C.POINTER(_int)],
+    "dsx_knn_search_host": [_int, _vp, _u32, _u32, _u32, _vp, _u32, _u32, _vp, _vp, _vp, _vp, _vp, _sz, C.POINTER(_f32)],
     "dsx_knn_last_search_path": [],
     "dsx_testing_set_knn_f16_sweep": [_int],
 }
 SPECIAL_RESTYPES = {"dsx_last_error": C.c_char_p, "dsx_stream": C.c_void_p, "dsx_knn_workspace_bytes": C.c_size_t,
                     "dsx_knn_workspace_bytes_f16": C.c_size_t, "dsx_knn_f16_table_bytes": C.c_size_t, "dsx_fc_split_bytes": _u64,
-                    "dsx_knn_workspace_bytes_split": C.c_size_t, "dsx_knn_workspace_bytes_least": C.c_size_t}
+                    "dsx_knn_workspace_bytes_split": C.c_size_t, "dsx_knn_workspace_bytes_least": C.c_size_t,
+                    "dsx_knn_workspace_bytes_prepared": C.c_size_t, "dsx_screen_table_bytes": _u64}
 SPECIAL_ARGTYPES = {"dsx_last_error": [], "dsx_stream": [], "dsx_knn_workspace_bytes": [_u32, _u32, _u32, _u32],
                     "dsx_knn_workspace_bytes_f16": [_u32, _u32, _u32, _u32], "dsx_knn_f16_table_bytes": [_u32, _u32],
                     "dsx_fc_split_bytes": [_u32, _u32], "dsx_knn_workspace_bytes_split": [_u32, _u32, _u32, _u32],
-                    "dsx_knn_workspace_bytes_least": [_u32, _u32, _u32, _u32]}
+                    "dsx_knn_workspace_bytes_least": [_u32, _u32, _u32, _u32],
+                    "dsx_knn_workspace_bytes_prepared": [_u32, _u32, _u32, _u32], "dsx_screen_table_bytes": [_u32, _u32]}
 
 _lib = None
 

@@ -5,7 +5,7 @@
 // knn_f16_kernel's.  Three uses (MODE):
 //   kF16Scores   sums compared with the queries' bounds, survivors to lists (exact nearest neighbours, fp16 storage and screening)
 //   kF16Layer    sums that start from the items' biases, raised by the error they can have (dsx_screen.hip), against the bounds
-//   kF16Store    sums that start from the biases stored as halves, rounded up
+//   kF16Store    sums that start from the biases stored as halves, rounded up, and the largest of every 32 of them
 //
 // A wavefront owns 128 items x 64 queries: four row operands and two column operands per 16 components feed eight matrix
 // instructions, 48 LDS cycles for 64 cycles of each SIMD's matrix core (a 64 x 64 tile needs as many LDS cycles as there are).
@@ -51,6 +51,7 @@ struct F16SweepArgs {
     float bias_raise;       // layers: what a bias is raised by, per unit of it
     _Float16* Z;            // kF16Store: [batch][ldz]
     uint64_t ldz;
+    _Float16* M;            // kF16Store: [batch][ldz / 32] the largest of every 32 of them
     const float* scale;     // kF16Store: [batch] what a query's sums are multiplied by (a power of two)
 };
 
@@ -58,22 +59,22 @@ constexpr uint32_t kF16Queue = 32;   // entries of a wavefront's queue
 
 template <int WI, int WQ, int STAGES> constexpr uint32_t f16_sweep_lds(int mode)
 {
-    return STAGES * (128 * WI + 64 * WQ) * 64 + (mode != kF16Scores ? 2 * (128 + 4) * WI * 4 : 0) +
+    return STAGES * (128 * WI + 64 * WQ) * 64 + (mode != kF16Scores ? 4 * (128 + 4) * WI * 4 : 0) +
            (mode != kF16Store ? WI * WQ * (kF16Queue * 80 + 64 * 4) : 0);
 }
 
 template <int WI, int WQ, int STAGES, int MODE>
-__global__ __launch_bounds__(64 * WI * WQ) __attribute__((amdgpu_waves_per_eu(2, 2))) void f16_sweep_kernel(F16SweepArgs a)
+__global__ __launch_bounds__(64 * WI * WQ) __attribute__((amdgpu_waves_per_eu(WI * WQ == 8 ? 2 : 1, 2))) void f16_sweep_kernel(F16SweepArgs a)
 {
     constexpr uint32_t WAVES = WI * WQ, BI = 128 * WI, BQ = 64 * WQ, STAGE = (BI + BQ) * 64;
     constexpr uint32_t PI = BI / 16 / WAVES, PQ = BQ / 16 / WAVES;   // 1 KiB pieces (16 rows) of a stage per wavefront
     static_assert(PI * WAVES * 16 == BI && PQ * WAVES * 16 == BQ, "whole pieces");
     extern __shared__ __attribute__((aligned(16))) unsigned char f16_lds[];
-    // layers, two tiles each: what the items' sums start from, and the largest norm of 32 items
+    // layers, four tiles each: what the items' sums start from, and the largest norm of 32 items
     float* sStart = reinterpret_cast<float*>(f16_lds + STAGES * STAGE);
-    float* sMost = sStart + 2 * BI;
+    float* sMost = sStart + 4 * BI;
     // the wavefronts' queues (sixteen results; then the bound, e1, the largest norm, the item and the query) and their lists' fill counts
-    unsigned char* after = f16_lds + STAGES * STAGE + (MODE != kF16Scores ? 2 * (128 + 4) * WI * 4 : 0);
+    unsigned char* after = f16_lds + STAGES * STAGE + (MODE != kF16Scores ? 4 * (128 + 4) * WI * 4 : 0);
     float (*sResult)[16] = reinterpret_cast<float (*)[16]>(after) + (threadIdx.x >> 6) * kF16Queue;
     uint4* sEntry = reinterpret_cast<uint4*>(after + WAVES * kF16Queue * 64) + (threadIdx.x >> 6) * kF16Queue;
     uint32_t* sFill = reinterpret_cast<uint32_t*>(after + WAVES * kF16Queue * 80) + (threadIdx.x & ~63u);
@@ -118,26 +119,34 @@ __global__ __launch_bounds__(64 * WI * WQ) __attribute__((amdgpu_waves_per_eu(2,
     } else if (t0 >= t1) return;
 
     // What an item's sum starts from (its bias, raised by the roundings of a sum that holds it; an item of infinite norm always passes)
-    // and its norm: of tile t's items, a lane each, asked for a tile ahead.
+    // and its norm, asked for a tile ahead.
     float e1[2] = {0.0f, 0.0f};
-    float start_next = 0.0f, norm_next = 0.0f;
+    constexpr uint32_t OWN = (BI + 64 * WAVES - 1) / (64 * WAVES);   // items of a tile per lane
+    float start_next[OWN], norm_next[OWN];
     auto ask = [&](uint32_t t) __attribute__((always_inline)) {
-        const uint32_t c = t * BI + tid;
-        start_next = -__builtin_inff();
-        norm_next = 0.0f;
-        if (tid >= BI || t >= t1 || c >= a.n) return;
-        const float b = a.bias ? a.bias[c] : 0.0f, norm = a.norm[c];
-        start_next = (norm == __builtin_inff() && b == b) ? norm : b == -__builtin_inff() ? b : b + fabsf(b) * a.bias_raise;
-        norm_next = (norm == __builtin_inff()) ? 0.0f : norm;
+#pragma unroll
+        for (uint32_t o = 0; o < OWN; o++) {
+            const uint32_t i = o * 64 * WAVES + tid, c = t * BI + i;
+            start_next[o] = -__builtin_inff();
+            norm_next[o] = 0.0f;
+            if (i >= BI || t >= t1 || c >= a.n) continue;
+            const float b = a.bias ? a.bias[c] : 0.0f, norm = a.norm[c];
+            start_next[o] = (norm == __builtin_inff() && b == b) ? norm : b == -__builtin_inff() ? b : b + fabsf(b) * a.bias_raise;
+            norm_next[o] = (norm == __builtin_inff()) ? 0.0f : norm;
+        }
     };
     auto put = [&](uint32_t t) __attribute__((always_inline)) {
-        if (tid >= BI) return;   // (whole wavefronts)
-        sStart[(t & 1) * BI + tid] = start_next;
-        if constexpr (MODE == kF16Layer) {
-            float m = norm_next;
 #pragma unroll
-            for (int d = 1; d < 32; d *= 2) m = fmaxf(m, __shfl_xor(m, d));
-            if (l32 == 0) sMost[(t & 1) * (BI / 32) + tid / 32] = m;
+        for (uint32_t o = 0; o < OWN; o++) {
+            const uint32_t i = o * 64 * WAVES + tid;
+            if (i >= BI) continue;   // (whole wavefronts)
+            sStart[(t & 3) * BI + i] = start_next[o];
+            if constexpr (MODE == kF16Layer) {
+                float m = norm_next[o];
+#pragma unroll
+                for (int d = 1; d < 32; d *= 2) m = fmaxf(m, __shfl_xor(m, d));
+                if (l32 == 0) sMost[(t & 3) * (BI / 32) + i / 32] = m;
+            }
         }
     };
     if constexpr (MODE != kF16Scores) {
@@ -149,6 +158,9 @@ __global__ __launch_bounds__(64 * WI * WQ) __attribute__((amdgpu_waves_per_eu(2,
         ask(t0);
         put(t0);
         ask(t0 + 1);
+        put(t0 + 1);
+        ask(t0 + 2);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (before the barrier below)
     }
 
     // Operands on their way: the stage of cursor (dt, dk) goes into ring place dp.  The cursor stops at the last stage (what is asked for
@@ -190,6 +202,8 @@ __global__ __launch_bounds__(64 * WI * WQ) __attribute__((amdgpu_waves_per_eu(2,
         else if constexpr ((STAGES_LEFT) * PER == 6) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");  \
         else if constexpr ((STAGES_LEFT) * PER == 8) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");  \
         else if constexpr ((STAGES_LEFT) * PER == 12) asm volatile("s_waitcnt vmcnt(12)" ::: "memory"); \
+        else if constexpr ((STAGES_LEFT) * PER == 30) asm volatile("s_waitcnt vmcnt(30)" ::: "memory"); \
+        else if constexpr ((STAGES_LEFT) * PER == 40) asm volatile("s_waitcnt vmcnt(40)" ::: "memory"); \
         else static_assert((STAGES_LEFT) * PER == 0, "a count for this many requests");          \
         __builtin_amdgcn_s_barrier();                                                            \
         asm volatile("" ::: "memory");                                                           \
@@ -332,7 +346,7 @@ __global__ __launch_bounds__(64 * WI * WQ) __attribute__((amdgpu_waves_per_eu(2,
 #pragma unroll
                     for (int v = 0; v < 16; v++) acc[i][j][v] = 0.0f;
         } else {
-            const float* from = sStart + (t & 1) * BI + wi * 128 + 4 * lhi;
+            const float* from = sStart + (t & 3) * BI + wi * 128 + 4 * lhi;
 #pragma unroll
             for (int i = 0; i < 4; i++)
 #pragma unroll
@@ -346,19 +360,21 @@ __global__ __launch_bounds__(64 * WI * WQ) __attribute__((amdgpu_waves_per_eu(2,
         }
         __builtin_amdgcn_s_setprio(1);
         stage();
+        stage();   // (ld is a multiple of 64: two stages at least)
         if constexpr (MODE != kF16Scores) {
-            // (every wavefront has read this tile's starts and is done with the tile before, whose places take the next tile's, which
-            // the barriers of the stages behind this make visible)
-            put(t + 1);
-            ask(t + 2);
+            // Two tiles ahead, into the places of the tile before last: a whole tile's barriers and waits lie before they are read.  The
+            // wait for what was asked for is then for requests that three stages follow (after one stage it emptied the ring once a tile:
+            // 4 x 128 x 1,000,000 77 us, 73.5 so).
+            put(t + 2);
+            ask(t + 3);
         }
-        for (uint32_t kt = 1; kt < nk; kt++) stage();
+        for (uint32_t kt = 2; kt < nk; kt++) stage();
         __builtin_amdgcn_s_setprio(0);
         if constexpr (MODE != kF16Store) {
             const uint32_t item0 = t * BI + wi * 128 + 4 * lhi;
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const float most = MODE == kF16Layer ? sMost[(t & 1) * (BI / 32) + wi * 4 + i] : 0.0f;
+                const float most = MODE == kF16Layer ? sMost[(t & 3) * (BI / 32) + wi * 4 + i] : 0.0f;
 #pragma unroll
                 for (int j = 0; j < 2; j++) compare(acc[i][j], j, item0 + i * 32, most);
             }
@@ -369,6 +385,29 @@ __global__ __launch_bounds__(64 * WI * WQ) __attribute__((amdgpu_waves_per_eu(2,
                 const float scale = a.scale[q[j]];
                 // (both halves of a lane pair take the same branch: they hold the same query)
                 _Float16* dst = a.Z + (uint64_t)q[j] * a.ldz + (uint64_t)t * BI + wi * 128 + lhi * 16;
+                typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+                // raised by half a unit in the last place and a subnormal's, and no lower than the lowest half: what rounds to nearest then
+                // lies above
+                auto up = [&](float v) __attribute__((always_inline)) -> _Float16 {
+                    const float x = v * scale;
+                    return (_Float16)fmaxf(fmaf(fabsf(x), 4.932e-4f, x) + 6.0e-8f, -65504.0f);
+                };
+                half2v most[2];
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const floatx16& v = acc[i][j];
+                    float top = fmaxf(fmaxf(v[0], v[1]), v[2]);
+#pragma unroll
+                    for (int e = 3; e < 15; e += 2) top = fmaxf(fmaxf(top, v[e]), v[e + 1]);
+                    top = fmaxf(top, v[15]);
+                    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(top), __float_as_uint(top), false, false);
+                    most[i / 2][i % 2] = up(fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])));
+                }
+                if (lhi == 0) {
+                    typedef uint32_t u32x2v __attribute__((ext_vector_type(2)));
+                    u32x2v w = {__builtin_bit_cast(uint32_t, most[0]), __builtin_bit_cast(uint32_t, most[1])};
+                    *reinterpret_cast<u32x2v*>(a.M + (uint64_t)q[j] * (a.ldz / 32) + t * (BI / 32) + wi * 4) = w;
+                }
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     uint32_t w[4][2];
@@ -376,13 +415,7 @@ __global__ __launch_bounds__(64 * WI * WQ) __attribute__((amdgpu_waves_per_eu(2,
                     for (int g = 0; g < 4; g++)
 #pragma unroll
                         for (int p = 0; p < 2; p++) {
-                            typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-                            const float x = acc[i][j][4 * g + 2 * p] * scale, y = acc[i][j][4 * g + 2 * p + 1] * scale;
-                            // raised by half a unit in the last place and a subnormal's, and no lower than the lowest half: what
-                            // rounds to nearest then lies above
-                            half2v h;
-                            h[0] = (_Float16)fmaxf(fmaf(fabsf(x), 4.932e-4f, x) + 6.0e-8f, -65504.0f);
-                            h[1] = (_Float16)fmaxf(fmaf(fabsf(y), 4.932e-4f, y) + 6.0e-8f, -65504.0f);
+                            const half2v h = {up(acc[i][j][4 * g + 2 * p]), up(acc[i][j][4 * g + 2 * p + 1])};
                             w[g][p] = __builtin_bit_cast(uint32_t, h);
                         }
                     // a lane holds items 8 g + 4 lhi + 0..3: after the exchange the lower half's lanes hold items 0..15, the others 16..31
@@ -432,8 +465,8 @@ static F16SweepArgs f16_args(const F16Job& j)
     a.ld = j.ld; a.batch = j.batch; a.n = j.n;
     a.norm = j.norm; a.bias = j.bias; a.e1 = j.e1; a.bias_raise = j.bias_raise;
     a.cand = j.cand;
-    a.Z = (_Float16*)j.Z; a.ldz = j.ldz; a.scale = j.scale;
-    a.tiles_q = (j.batch + 255) / 256;
+    a.Z = (_Float16*)j.Z; a.M = (_Float16*)j.M; a.ldz = j.ldz; a.scale = j.scale;
+    a.tiles_q = (j.batch + 255) / 256;   // (one where tiles are lower)
     return a;
 }
 
@@ -455,15 +488,23 @@ int f16_sweep_run(const F16Job& j, bool layer, uint32_t* lists)
 int f16_store_run(const F16Job& j)
 {
     F16SweepArgs a = f16_args(j);
-    // 128 x 256 tiles, four wavefronts, where 256 x 256 ones leave half the GPU without work (256 x 1,024 x 27,278: 28 us against 35)
-    const uint32_t big = (j.n + 255) / 256;
-    const bool small = a.tiles_q * big < (uint32_t)ctx().num_cus;
-    a.tiles_i = small ? (j.n + 127) / 128 : big;
+    // Few rows are bound by reading the items: as many of them in flight as LDS holds, and no matrix work for rows that are not there
+    // (8 x 256 x 500,000: 56 us, 4.5 TB/s; 4 x 128 x 1,000,000: 73.5, as half as many stages lie between two tiles' stores; a copy
+    // reaches 5.1 TB/s.  Seven stages in flight instead of six: 59 and 77).  128 items x 256 rows where 256 x 256 tiles leave half
+    // the GPU without work (256 x 1,024 x 27,278: 28 us against 35).
+    const int shape = j.batch <= 64 ? 0 : j.batch <= 128 ? 1 : a.tiles_q * ((j.n + 255) / 256) < (uint32_t)ctx().num_cus ? 2 : 3;
+    const uint32_t items = shape == 2 ? 128 : 256;
+    a.tiles_i = (j.n + items - 1) / items;
     a.chunks = std::min(a.tiles_i, std::max(1u, (uint32_t)ctx().num_cus / a.tiles_q));
     a.tiles_per_chunk = (a.tiles_i + a.chunks - 1) / a.chunks;
     a.chunks = (a.tiles_i + a.tiles_per_chunk - 1) / a.tiles_per_chunk;
     a.group = std::min(a.tiles_q, kF16Group);
-    return small ? launch_f16_sweep<1, 4, 4, kF16Store>(a) : launch_f16_sweep<2, 4, 4, kF16Store>(a);
+    switch (shape) {
+    case 0: return launch_f16_sweep<2, 1, 6, kF16Store>(a);
+    case 1: return launch_f16_sweep<2, 2, 4, kF16Store>(a);
+    case 2: return launch_f16_sweep<1, 4, 4, kF16Store>(a);
+    default: return launch_f16_sweep<2, 4, 4, kF16Store>(a);
+    }
 }
 
 }  // namespace dsx

@@ -100,7 +100,7 @@ static LayerWorkspace layer_layout(void* base, uint32_t batch, uint32_t n0, uint
     w.table = ScreenTable{};
     w.screen = ScreenWorkspace{};
     if (screened) {
-        w.screen = screen_layout(p, batch, kdim, n);
+        w.screen = screen_layout(p, batch, kdim, n, k);
         p += w.screen.bytes;
     }
     if (screened == 1) {
@@ -179,10 +179,27 @@ int dsx_fc_topk_pays(uint32_t batch, uint32_t k_dim, uint32_t n, uint32_t activa
            ((k <= 32 && batch >= 1536 && products >= 2e10) || (k <= 128 && batch >= 2048 && products >= 1e11));
 }
 
+// Where the line lies (us a batch; the layer stored and its guided top-K, or ranges in fp32 / screened by a kept table; filter of 144
+// columns a row, nets of one hidden layer, four batches after each other or, up to 128 rows of top 20, one by itself):
+//   More than 128 rows: 169 nets of 64 to 1,024 hidden units, 8,192 to 100,000 columns, 512 to 4,096 rows, top 10 and top 100, fitted:
+//   what is gained grows with the columns' scores that are not stored as floats (0.6 us a million) and with the products (2.5 us
+//   a thousand million); what it costs is three more launches and, for large k, candidates of long rows.  512 x 64 x 8,192 top 100 40 / 48 and top
+//   10 27 / 30, 512 x 128 x 8,192 top 10 32 / 32, 512 x 64 x 16,384 top 100 57 / 51, 512 x 512 x 8,192 top 100 76 / 65, 1,024 x 128 x
+//   27,278 top 10 98 / 51, 4,096 x 64 x 8,192 top 10 95 / 85, 1,024 x 1,024 x 60,000 top 10 979 / 220.
+//   65 to 128 rows: where the layer is wide.  128 x 1,024 x 8,192 91 / 110, 128 x 64 x 27,278 59 / 68, 128 x 256 x 27,278 83 / 81, 128 x
+//   1,024 x 27,278 141 / 94, 128 x 64 x 100,000 77 / 70, 128 x 256 x 500,000 461 / 170.
+//   Up to 64 rows: both read the weights once, and half as many bytes of them only pay where they come from memory and there are tiles for
+//   the whole GPU.  32 x 1,024 x 27,278 73 / 83, 1 x 64 x 100,000 55 / 55, 8 x 64 x 500,000 81 / 85, 8 x 256 x 100,000 73 / 65, 8 x
+//   256 x 500,000 154 / 114, 8 x 1,024 x 100,000 145 / 98.
+// Sigmoids only, as above, but for layers that are never stored; with few rows the rest of the weights' cost would be paid again for one.
 int dsx_fc_topk_screened_pays(uint32_t batch, uint32_t k_dim, uint32_t n, uint32_t activation, uint32_t k)
 {
-    (void)k;
-    return batch > 0 && k_dim >= 32 && k_dim <= 4096 && n >= 8192 && activation == DSX_ACT_SIGMOID;
+    if (batch == 0 || k > 256 || n < 64 * k || n < 8192 || n >= 1u << 28 || k_dim < 32 || k_dim > 4096) return 0;
+    if (activation != DSX_ACT_SIGMOID && (n < 131072 || batch <= 64)) return 0;
+    const double q = batch, d = k_dim, m = n;
+    if (batch <= 64) return n >= 65536 && k_dim >= 128 && m * d >= 2.5e7;
+    if (batch <= 128) return n >= 24576 && m * d >= 6e6;
+    return q * m * (6e-7 + 2.5e-9 * d) > 6.0 + 0.013 * k;
 }
 
 int dsx_fc_topk_supported(uint32_t ldx, const float* X, uint32_t activation, const dsx_act_params* params, const float* filter_mul)
@@ -235,10 +252,7 @@ static int fc_topk_common(const float* X, uint32_t ldx, const float* W, const fl
     redo.lambda = params ? params->lambda : 1.0f;
     redo.position = position; redo.index = index; redo.fstart = filter_start; redo.fend = filter_end; redo.fidx = filter_index;
     redo.row_flag = w.row_flag; redo.partial = w.cand; redo.done = w.redo_done; redo.keys = keys; redo.values = values;
-    const uint32_t clear_words = (uint32_t)layer_clear_words(batch);
     if (screened) {
-        hipLaunchKernelGGL(layer_clear_kernel, dim3((clear_words + 255) / 256), dim3(256), 0, ctx().stream, w.row_bound, clear_words);
-        DSX_LAUNCH_CHECK("layer_clear_kernel");
         const ScreenTable t = table ? screen_table(const_cast<void*>(table), kdim, n) : w.table;
         int rc = table ? DSX_OK : screen_build(t, W, n, n, kdim);
         if (rc) return rc;
@@ -249,6 +263,7 @@ static int fc_topk_common(const float* X, uint32_t ldx, const float* W, const fl
         j.keys = keys; j.values = values;
         j.row_flag = w.row_flag; j.told = flag_word;
         j.cand = w.cand; j.cand_count = w.cand_count; j.cap = cap; j.overflow = w.overflow;
+        j.clear = w.overflow; j.clear_words = 64 + layer_redo_groups(batch);   // (overflow and redo_done)
         if ((rc = screen_rows(j, t, w.screen, nullptr))) return rc;
         if ((rc = screen_run(j, t, w.screen))) return rc;
         return layer_redo_run(redo, batch);
@@ -266,6 +281,7 @@ static int fc_topk_common(const float* X, uint32_t ldx, const float* W, const fl
     if (!ranges)
         return topk_run(w.block_scores, ld0, n0, batch, k, keys, values, position, index, filter_start, filter_end, filter_index, nullptr, 0,
                         nullptr, 0, 0, 0);
+    const uint32_t clear_words = (uint32_t)layer_clear_words(batch);
     hipLaunchKernelGGL(layer_clear_kernel, dim3((clear_words + 255) / 256), dim3(256), 0, s, w.row_bound, clear_words);
     DSX_LAUNCH_CHECK("layer_clear_kernel");
     rc = topk_run(w.block_scores, ld0, n0, batch, k, nullptr, nullptr, position, index, filter_start, filter_end, filter_index, nullptr, 0,
@@ -329,7 +345,7 @@ int dsx_screen_table_build(const float* W, uint32_t ldw, uint32_t n, uint32_t kd
     DSX_REQUIRE_INIT();
     DSX_CHECK_ARG(W && table, "dsx_screen_table_build: null device pointer");
     DSX_CHECK_ARG(((uintptr_t)table % 256) == 0, "dsx_screen_table_build: the table is not 256-byte aligned");
-    DSX_CHECK_ARG(n > 0 && kdim > 0 && kdim <= 4096 && ldw >= n, "dsx_screen_table_build: n = %u, k = %u, ldw = %u", n, kdim, ldw);
+    DSX_CHECK_ARG(n > 0 && n < 1u << 28 && kdim > 0 && kdim <= 4096 && ldw >= n, "dsx_screen_table_build: n = %u, k = %u, ldw = %u", n, kdim, ldw);
     return screen_build(screen_table(table, kdim, n), W, ldw, n, kdim);
 }
 
@@ -339,7 +355,7 @@ int dsx_fc_topk_screened(const float* X, uint32_t ldx, const float* W, const voi
                          const uint32_t* filter_index)
 {
     DSX_CHECK_ARG(table && ((uintptr_t)table % 256) == 0, "dsx_fc_topk_screened: the table is missing or not 256-byte aligned");
-    DSX_CHECK_ARG(kdim <= 4096, "dsx_fc_topk_screened: k = %u (4,096 at most)", kdim);
+    DSX_CHECK_ARG(kdim <= 4096 && n < 1u << 28, "dsx_fc_topk_screened: k = %u (4,096 at most), n = %u (below 2^28)", kdim, n);
     return fc_topk_common(X, ldx, W, bias, batch, kdim, n, activation, params, k, keys, values, position, index, filter_start, filter_end,
                           filter_index, nullptr, nullptr, table);
 }

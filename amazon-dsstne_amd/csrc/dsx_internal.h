@@ -110,7 +110,9 @@ int topk_guided_launch(const float* in, uint32_t pitch, uint32_t width, uint32_t
                        uint32_t partial_slot0, uint32_t* row_bound);
 // Workgroups per row that topk_run takes on its own (forced_segments = 0).
 uint32_t topk_segments(uint32_t batch, uint32_t width, bool filtered);
-int topk_merge(const uint64_t* partial, uint32_t slots, uint32_t k, float* keys, uint32_t* values, uint32_t batch);
+// keys2 / values2: the results once more, in host memory that the device can write (or NULL).
+int topk_merge(const uint64_t* partial, uint32_t slots, uint32_t k, float* keys, uint32_t* values, uint32_t batch, float* keys2 = nullptr,
+               uint32_t* values2 = nullptr);
 // What the sums of an fc_run have to agree with, bit for bit, so that equal columns score the same wherever they lie.  plan_n: the
 // other column blocks of the same product, of this width each (this one may be narrower).  as_candidates: the candidate modes below,
 // which add the products in ascending order of k (with a bias they start from it and not from 0).

@@ -85,7 +85,7 @@ static KnnWorkspace knn_layout(void* base, uint32_t rows_padded, uint32_t num_qu
     const uint32_t blocks = (rows_padded + cb - 1) / cb;
     KnnWorkspace w;
     char* p = (char*)base;
-    screen = screen && !f16 && !split && knn_screens(rows_padded, num_queries, k, dim);
+    screen = screen && !f16 && !split && (table || knn_screens(rows_padded, num_queries, k, dim));
     w.table = ScreenTable{};
     if (screen || table) {
         w.table = screen_table(p, dim, rows_padded);
@@ -119,7 +119,7 @@ static KnnWorkspace knn_layout(void* base, uint32_t rows_padded, uint32_t num_qu
     if (split) p += align256((size_t)split_plane_bytes(num_queries, dim));
     w.screen = ScreenWorkspace{};
     if (screen) {
-        w.screen = screen_layout(p, num_queries, dim, rows_padded);
+        w.screen = screen_layout(p, num_queries, dim, rows_padded, k);
         p += w.screen.bytes;
     }
     w.bytes = (size_t)(p - (char*)base);
@@ -128,20 +128,13 @@ static KnnWorkspace knn_layout(void* base, uint32_t rows_padded, uint32_t num_qu
 
 // What a search of any number of queries up to num_queries needs: a workspace of a batch is used for smaller ones too, and fewer
 // queries may need more (5,000 rows, k = 100: 64 queries 3.634 MB, 65 queries 3.618, because 64 leave more lists per query).
-// About 40 ns per query count, once per table.  *table: whether that includes the table of a screened search (which then lies at the start of
-// it for every number of queries).
-static size_t knn_workspace_most(uint32_t rows_padded, uint32_t num_queries, uint32_t k, bool f16, uint32_t dim, bool split, bool screen = true,
-                                 bool* table = nullptr)
+// About 40 ns per query count, once per table.
+static size_t knn_workspace_most(uint32_t rows_padded, uint32_t num_queries, uint32_t k, bool f16, uint32_t dim, bool split, bool screen = true)
 {
     size_t most = 0;
-    bool any = false;
-    for (uint64_t q = std::min(1u, num_queries); q <= num_queries; q++) {
-        const KnnWorkspace w = knn_layout(nullptr, rows_padded, (uint32_t)q, k, f16, dim, split, screen);
-        most = std::max(most, w.bytes - w.table.bytes);
-        any = any || w.table.bytes != 0;
-    }
-    if (table) *table = any;
-    return most + (any ? screen_table(nullptr, dim, rows_padded).bytes : 0);
+    for (uint64_t q = std::min(1u, num_queries); q <= num_queries; q++)
+        most = std::max(most, knn_layout(nullptr, rows_padded, (uint32_t)q, k, f16, dim, split, screen).bytes);
+    return most;
 }
 
 // Where the scores of a column range come from: the fp32 table through fc_gemm_kernel, or the fp16 table through knn_f16_kernel.
@@ -219,9 +212,16 @@ struct KnnTimer {
     }
 };
 
+// Where the results go; host_*: once more, into host memory that the device can write (or NULL).
+struct KnnResults {
+    float* scores;
+    uint32_t* indexes;
+    float* host_scores;
+    uint32_t* host_indexes;
+};
+
 // Block by block through the scratch score matrix; exact for any input, no host read-back.
-static int knn_search_blocks(const KnnWorkspace& w, const KnnOperands& op, uint32_t M, uint32_t num_queries, uint32_t k, float* scores,
-                             uint32_t* indexes, KnnTimer& t)
+static int knn_search_blocks(const KnnWorkspace& w, const KnnOperands& op, uint32_t M, uint32_t num_queries, uint32_t k, const KnnResults& out, KnnTimer& t)
 {
     hipStream_t s = ctx().stream;
     const uint32_t cb = knn_block_columns(op.rows_padded, num_queries);
@@ -251,7 +251,7 @@ static int knn_search_blocks(const KnnWorkspace& w, const KnnOperands& op, uint3
         t.stop(s, t.topk);
     }
     t.start(s);
-    int rc = topk_merge(w.partial, lists, k, scores, indexes, num_queries);
+    int rc = topk_merge(w.partial, lists, k, out.scores, out.indexes, num_queries, out.host_scores, out.host_indexes);
     t.stop(s, t.topk);
     return rc;
 }
@@ -288,8 +288,8 @@ static int knn_notes_ready()
 }
 
 // First block as above, the rest in candidate mode.  *overflowed tells the caller to redo the search block by block.
-static int knn_search_candidates(const KnnWorkspace& w, const KnnOperands& op, uint32_t M, uint32_t num_queries, uint32_t k, float* scores,
-                                 uint32_t* indexes, KnnTimer& t, bool* overflowed)
+static int knn_search_candidates(const KnnWorkspace& w, const KnnOperands& op, uint32_t M, uint32_t num_queries, uint32_t k, const KnnResults& out,
+                                 KnnTimer& t, bool* overflowed)
 {
     hipStream_t s = ctx().stream;
     const uint32_t cb = knn_block_columns(op.rows_padded, num_queries);
@@ -327,7 +327,7 @@ static int knn_search_candidates(const KnnWorkspace& w, const KnnOperands& op, u
         done += ncols;
     }
     t.start(s);
-    rc = topk_merge(w.partial, 1, k, scores, indexes, num_queries);
+    rc = topk_merge(w.partial, 1, k, out.scores, out.indexes, num_queries, out.host_scores, out.host_indexes);
     if (rc) return rc;
     t.stop(s, t.topk);
     uint32_t flag = 0;
@@ -340,22 +340,21 @@ static int knn_search_candidates(const KnnWorkspace& w, const KnnOperands& op, u
 // Screened in 16 bits (fp32 storage).  built: the workspace's table is there already (dsx_knn_prepare), and what it is like has been
 // looked at.  *overflowed tells the caller to redo the search without screening; *unfit, that the table or the queries were found unfit
 // for it first (norms beyond f16's range, or one so large that the others' bounds would be worth little).
-static int knn_search_screened(const KnnWorkspace& w, const KnnOperands& op, uint32_t M, uint32_t num_queries, uint32_t k, float* scores,
-                               uint32_t* indexes, KnnTimer& t, bool built, bool* overflowed, bool* unfit)
+static int knn_search_screened(const KnnWorkspace& w, const KnnOperands& op, uint32_t M, uint32_t num_queries, uint32_t k, const KnnResults& out,
+                               KnnTimer& t, bool built, bool* overflowed, bool* unfit)
 {
     hipStream_t s = ctx().stream;
-    const uint32_t clear_words = 3 * num_queries + 64;
-    hipLaunchKernelGGL(knn_clear_kernel, dim3((clear_words + 255) / 256), dim3(256), 0, s, w.row_bound, clear_words);
+    int rc = knn_notes_ready();
+    if (rc) return rc;
     ScreenJob j{};
     j.X = op.queries; j.ldx = op.dim; j.batch = num_queries; j.dim = op.dim; j.n = M; j.k = k;
     j.act = DSX_ACT_LINEAR;
-    j.keys = scores; j.values = indexes;
-    j.row_flag = w.row_flag; j.told = w.overflow;
+    j.keys = out.scores; j.values = out.indexes; j.keys2 = out.host_scores; j.values2 = out.host_indexes;
+    j.row_flag = w.row_flag; j.told = &g_knn_notes->flag;
     j.cand = w.cand; j.cand_count = w.cand_count; j.cap = kCandCap; j.overflow = w.overflow;
+    j.clear = w.overflow; j.clear_words = 64;
     t.start(s);
-    int rc = DSX_OK;
     if (!built) {
-        if ((rc = knn_notes_ready())) return rc;
         if ((rc = screen_build(w.table, op.items, op.rows_padded, M, op.dim))) return rc;
     }
     if ((rc = screen_rows(j, w.table, w.screen, built ? nullptr : g_knn_notes))) return rc;
@@ -370,10 +369,8 @@ static int knn_search_screened(const KnnWorkspace& w, const KnnOperands& op, uin
     }
     if ((rc = screen_run(j, w.table, w.screen))) return rc;
     t.stop(s, t.gemm);
-    uint32_t flag = 0;
-    DSX_HIP(hipMemcpyAsync(&flag, w.overflow, sizeof(flag), hipMemcpyDeviceToHost, s));
     DSX_HIP(hipStreamSynchronize(s));
-    *overflowed = flag != 0;
+    *overflowed = *(volatile uint32_t*)&g_knn_notes->flag != 0;
     return DSX_OK;
 }
 
@@ -415,6 +412,22 @@ size_t dsx_knn_workspace_bytes_least(uint32_t rows_padded, uint32_t dim, uint32_
     return knn_workspace_most(rows_padded, num_queries, k, false, dim, false, false);
 }
 
+// A table that is kept pays for itself wherever a search is more than launches: few queries are bound by reading it, and its halves are
+// half of what fp32 would read (4 queries x 1,000,000 x 128: 191 us a search, 125 so; 4,096 queries 2,936, 2,000 so).
+static bool knn_prepares(uint32_t rows_padded, uint32_t dim, uint32_t num_queries, uint32_t k)
+{
+    return num_queries > 0 && ctx().knobs.screen != 2 && dim >= 32 && dim <= 4096 && rows_padded >= 65536 && (uint64_t)rows_padded * dim >= 50000000ull &&
+           screen_table(nullptr, dim, rows_padded).bytes <= ((uint64_t)8 << 30) && k <= 256;
+}
+
+size_t dsx_knn_workspace_bytes_prepared(uint32_t rows_padded, uint32_t dim, uint32_t num_queries, uint32_t k)
+{
+    if (!knn_prepares(rows_padded, dim, num_queries, k)) return dsx_knn_workspace_bytes(rows_padded, dim, num_queries, k);
+    size_t most = 0;
+    for (uint64_t q = 1; q <= num_queries; q++) most = std::max(most, knn_layout(nullptr, rows_padded, (uint32_t)q, k, false, dim, false, true, true).bytes);
+    return most;
+}
+
 size_t dsx_knn_workspace_bytes_f16(uint32_t rows_padded, uint32_t dim, uint32_t num_queries, uint32_t k)
 {
     return knn_workspace_most(rows_padded, num_queries, k, true, dim, false);
@@ -439,7 +452,7 @@ int dsx_knn_f16_convert_items(const float* items, uint32_t rows_padded, uint32_t
 }  // extern "C"
 
 // Both precisions: workspace, the two paths, timing.
-static int knn_search_common(KnnOperands& op, uint32_t padding, uint32_t num_queries, uint32_t k, float* scores, uint32_t* indexes, void* workspace,
+static int knn_search_common(KnnOperands& op, uint32_t padding, uint32_t num_queries, uint32_t k, const KnnResults& out, void* workspace,
                              size_t workspace_bytes, float* elapsed_ms, bool aligned, const float* queries_f32, bool built = false)
 {
     const size_t full = knn_layout(nullptr, op.rows_padded, num_queries, k, op.f16, op.dim, op.split, true, built).bytes;
@@ -483,17 +496,17 @@ static int knn_search_common(KnnOperands& op, uint32_t padding, uint32_t num_que
     hipStreamIsCapturing(s, &capturing);
     // (few queries against an fp32 table stay with the blocks, however many there are; a width set by the caller is kept)
     const bool few = knn_few_queries(num_queries) && !op.f16 && !op.split && !ctx().knobs.knn_block_columns;
-    const bool may = aligned && !few && capturing == hipStreamCaptureStatusNone;
+    const bool may = aligned && (!few || built) && capturing == hipStreamCaptureStatusNone;
     const bool many = M > knn_block_columns(op.rows_padded, num_queries);
     bool screened = may && w.screen.bytes != 0 && !ctx().knobs.knn_block_columns;
     bool redo = true, unfit = false;
-    if (rc == DSX_OK && screened) rc = knn_search_screened(w, op, M, num_queries, k, scores, indexes, t, built, &redo, &unfit);
+    if (rc == DSX_OK && screened) rc = knn_search_screened(w, op, M, num_queries, k, out, t, built, &redo, &unfit);
     if (unfit) screened = false;
     const bool candidates = may && (screened || many);
     if (rc == DSX_OK && candidates && (!screened || redo) && many)
-        rc = knn_search_candidates(w, op, M, num_queries, k, scores, indexes, t, &redo);
+        rc = knn_search_candidates(w, op, M, num_queries, k, out, t, &redo);
     g_knn_last_path = !candidates ? DSX_KNN_PATH_BLOCKS : (redo ? DSX_KNN_PATH_CANDIDATES_REDONE : DSX_KNN_PATH_CANDIDATES);
-    if (rc == DSX_OK && redo) rc = knn_search_blocks(w, op, M, num_queries, k, scores, indexes, t);
+    if (rc == DSX_OK && redo) rc = knn_search_blocks(w, op, M, num_queries, k, out, t);
     if (elapsed_ms) {
         t.finish();
         elapsed_ms[0] = t.gemm;
@@ -505,11 +518,10 @@ static int knn_search_common(KnnOperands& op, uint32_t padding, uint32_t num_que
 }
 
 static int knn_search_fp32(const float* items, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,
-                           uint32_t num_queries, uint32_t k, float* scores, uint32_t* indexes, void* workspace, size_t workspace_bytes,
-                           float* elapsed_ms, bool built)
+                           uint32_t num_queries, uint32_t k, const KnnResults& out, void* workspace, size_t workspace_bytes, float* elapsed_ms, bool built)
 {
     DSX_REQUIRE_INIT();
-    DSX_CHECK_ARG(items && queries && scores && indexes, "dsx_knn_search: null device pointer");
+    DSX_CHECK_ARG(items && queries && out.scores && out.indexes, "dsx_knn_search: null device pointer");
     DSX_CHECK_ARG(padding < rows_padded, "dsx_knn_search: padding %u leaves no item of %u", padding, rows_padded);
     DSX_CHECK_ARG(dim > 0, "dsx_knn_search: dim is 0");
     DSX_CHECK_ARG(k >= 1 && k <= 256, "dsx_knn_search: k = %u is outside 1..256", k);
@@ -520,59 +532,14 @@ static int knn_search_fp32(const float* items, uint32_t rows_padded, uint32_t pa
     op.rows_padded = rows_padded;
     op.dim = dim;
     const bool aligned = ((uintptr_t)items % 16) == 0 && ((uintptr_t)queries % 16) == 0 && (rows_padded % 4) == 0 && (dim % 4) == 0;
-    return knn_search_common(op, padding, num_queries, k, scores, indexes, workspace, workspace_bytes, elapsed_ms, aligned, nullptr, built);
+    return knn_search_common(op, padding, num_queries, k, out, workspace, workspace_bytes, elapsed_ms, aligned, nullptr, built);
 }
 
-extern "C" {
-
-int dsx_knn_search(const float* items, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,
-                   uint32_t num_queries, uint32_t k, float* scores, uint32_t* indexes, void* workspace, size_t workspace_bytes,
-                   float* elapsed_ms)
-{
-    return knn_search_fp32(items, rows_padded, padding, dim, queries, num_queries, k, scores, indexes, workspace, workspace_bytes, elapsed_ms, false);
-}
-
-int dsx_knn_prepare(const float* items, uint32_t rows_padded, uint32_t padding, uint32_t dim, uint32_t num_queries, uint32_t k, void* workspace,
-                    size_t workspace_bytes, int* prepared)
+static int knn_search_split(const void* item_planes, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,
+                            uint32_t num_queries, uint32_t k, const KnnResults& out, void* workspace, size_t workspace_bytes, float* elapsed_ms)
 {
     DSX_REQUIRE_INIT();
-    DSX_CHECK_ARG(items && workspace && prepared, "dsx_knn_prepare: null pointer");
-    DSX_CHECK_ARG(padding < rows_padded && dim > 0 && num_queries > 0 && k >= 1 && k <= 256, "dsx_knn_prepare: rows_padded %u, padding %u, dim %u, %u queries, k = %u",
-                  rows_padded, padding, dim, num_queries, k);
-    DSX_CHECK_ARG(((uintptr_t)workspace % 256) == 0, "dsx_knn_prepare: workspace is not 256-byte aligned");
-    *prepared = 0;
-    bool table = false;
-    const size_t full = knn_workspace_most(rows_padded, num_queries, k, false, dim, false, true, &table);
-    const bool aligned = ((uintptr_t)items % 16) == 0 && (rows_padded % 4) == 0 && (dim % 4) == 0;
-    if (!table || !aligned || workspace_bytes < full) return DSX_OK;
-    const uint32_t M = rows_padded - padding;
-    const ScreenTable t = screen_table(workspace, dim, rows_padded);
-    if (int rc = screen_build(t, items, rows_padded, M, dim)) return rc;
-    uint32_t stats[3];
-    DSX_HIP(hipMemcpyAsync(stats, t.stats, sizeof(stats), hipMemcpyDeviceToHost, ctx().stream));
-    DSX_HIP(hipStreamSynchronize(ctx().stream));
-    ScreenNotes notes{};
-    std::memcpy(&notes.largest, &stats[0], sizeof(float));
-    std::memcpy(&notes.sum, &stats[1], sizeof(float));
-    notes.number = stats[2];
-    *prepared = !knn_unfit(notes, num_queries, dim, M, k);
-    return DSX_OK;
-}
-
-int dsx_knn_search_prepared(const float* items, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,
-                            uint32_t num_queries, uint32_t k, float* scores, uint32_t* indexes, void* workspace, size_t workspace_bytes,
-                            float* elapsed_ms)
-{
-    DSX_CHECK_ARG(workspace, "dsx_knn_search_prepared: null workspace");
-    return knn_search_fp32(items, rows_padded, padding, dim, queries, num_queries, k, scores, indexes, workspace, workspace_bytes, elapsed_ms, true);
-}
-
-int dsx_knn_search_split(const void* item_planes, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,
-                         uint32_t num_queries, uint32_t k, float* scores, uint32_t* indexes, void* workspace, size_t workspace_bytes,
-                         float* elapsed_ms)
-{
-    DSX_REQUIRE_INIT();
-    DSX_CHECK_ARG(item_planes && queries && scores && indexes, "dsx_knn_search_split: null device pointer");
+    DSX_CHECK_ARG(item_planes && queries && out.scores && out.indexes, "dsx_knn_search_split: null device pointer");
     DSX_CHECK_ARG(((uintptr_t)item_planes % 16) == 0, "dsx_knn_search_split: the item planes are not 16-byte aligned");
     DSX_CHECK_ARG(padding < rows_padded, "dsx_knn_search_split: padding %u leaves no item of %u", padding, rows_padded);
     DSX_CHECK_ARG(dim > 0, "dsx_knn_search_split: dim is 0");
@@ -584,15 +551,14 @@ int dsx_knn_search_split(const void* item_planes, uint32_t rows_padded, uint32_t
     op.item_planes = item_planes;
     op.rows_padded = rows_padded;
     op.dim = dim;
-    return knn_search_common(op, padding, num_queries, k, scores, indexes, workspace, workspace_bytes, elapsed_ms, true, queries);
+    return knn_search_common(op, padding, num_queries, k, out, workspace, workspace_bytes, elapsed_ms, true, queries);
 }
 
-int dsx_knn_search_f16(const void* items_f16, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,
-                       uint32_t num_queries, uint32_t k, float* scores, uint32_t* indexes, void* workspace, size_t workspace_bytes,
-                       float* elapsed_ms)
+static int knn_search_f16(const void* items_f16, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,
+                          uint32_t num_queries, uint32_t k, const KnnResults& out, void* workspace, size_t workspace_bytes, float* elapsed_ms)
 {
     DSX_REQUIRE_INIT();
-    DSX_CHECK_ARG(items_f16 && queries && scores && indexes, "dsx_knn_search_f16: null device pointer");
+    DSX_CHECK_ARG(items_f16 && queries && out.scores && out.indexes, "dsx_knn_search_f16: null device pointer");
     DSX_CHECK_ARG(((uintptr_t)items_f16 % 16) == 0, "dsx_knn_search_f16: the fp16 table is not 16-byte aligned");
     DSX_CHECK_ARG(padding < rows_padded, "dsx_knn_search_f16: padding %u leaves no item of %u", padding, rows_padded);
     DSX_CHECK_ARG(dim > 0, "dsx_knn_search_f16: dim is 0");
@@ -604,7 +570,79 @@ int dsx_knn_search_f16(const void* items_f16, uint32_t rows_padded, uint32_t pad
     op.rows_padded = rows_padded;
     op.dim = dim;
     op.ld16 = knn_f16_ld(dim);
-    return knn_search_common(op, padding, num_queries, k, scores, indexes, workspace, workspace_bytes, elapsed_ms, true, queries);
+    return knn_search_common(op, padding, num_queries, k, out, workspace, workspace_bytes, elapsed_ms, true, queries);
+}
+
+extern "C" {
+
+int dsx_knn_search(const float* items, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,
+                   uint32_t num_queries, uint32_t k, float* scores, uint32_t* indexes, void* workspace, size_t workspace_bytes,
+                   float* elapsed_ms)
+{
+    return knn_search_fp32(items, rows_padded, padding, dim, queries, num_queries, k, KnnResults{scores, indexes, nullptr, nullptr}, workspace,
+                           workspace_bytes, elapsed_ms, false);
+}
+
+int dsx_knn_search_split(const void* item_planes, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,
+                         uint32_t num_queries, uint32_t k, float* scores, uint32_t* indexes, void* workspace, size_t workspace_bytes,
+                         float* elapsed_ms)
+{
+    return knn_search_split(item_planes, rows_padded, padding, dim, queries, num_queries, k, KnnResults{scores, indexes, nullptr, nullptr}, workspace,
+                            workspace_bytes, elapsed_ms);
+}
+
+int dsx_knn_search_f16(const void* items_f16, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,
+                       uint32_t num_queries, uint32_t k, float* scores, uint32_t* indexes, void* workspace, size_t workspace_bytes,
+                       float* elapsed_ms)
+{
+    return knn_search_f16(items_f16, rows_padded, padding, dim, queries, num_queries, k, KnnResults{scores, indexes, nullptr, nullptr}, workspace,
+                          workspace_bytes, elapsed_ms);
+}
+
+int dsx_knn_prepare(const float* items, uint32_t rows_padded, uint32_t padding, uint32_t dim, uint32_t num_queries, uint32_t k, void* workspace,
+                    size_t workspace_bytes, int* prepared)
+{
+    DSX_REQUIRE_INIT();
+    DSX_CHECK_ARG(items && workspace && prepared, "dsx_knn_prepare: null pointer");
+    DSX_CHECK_ARG(padding < rows_padded && dim > 0 && num_queries > 0 && k >= 1 && k <= 256, "dsx_knn_prepare: rows_padded %u, padding %u, dim %u, %u queries, k = %u",
+                  rows_padded, padding, dim, num_queries, k);
+    DSX_CHECK_ARG(((uintptr_t)workspace % 256) == 0, "dsx_knn_prepare: workspace is not 256-byte aligned");
+    *prepared = 0;
+    const bool aligned = ((uintptr_t)items % 16) == 0 && (rows_padded % 4) == 0 && (dim % 4) == 0;
+    if (!knn_prepares(rows_padded, dim, num_queries, k) || !aligned || workspace_bytes < dsx_knn_workspace_bytes_prepared(rows_padded, dim, num_queries, k)) return DSX_OK;
+    const uint32_t M = rows_padded - padding;
+    const ScreenTable t = screen_table(workspace, dim, rows_padded);
+    if (int rc = screen_build(t, items, rows_padded, M, dim)) return rc;
+    uint32_t stats[3];
+    DSX_HIP(hipMemcpyAsync(stats, t.stats, sizeof(stats), hipMemcpyDeviceToHost, ctx().stream));
+    DSX_HIP(hipStreamSynchronize(ctx().stream));
+    ScreenNotes notes{};
+    std::memcpy(&notes.largest, &stats[0], sizeof(float));
+    std::memcpy(&notes.sum, &stats[1], sizeof(float));
+    notes.number = stats[2];
+    // as where a search makes its own copies: no norm beyond f16's range, and none so far above the others that its share of the error
+    // (of the columns next to it, which are judged by the largest of 32 or 64) would let everything pass
+    const float average = notes.number != 0 ? notes.sum / (float)notes.number : 0.0f;
+    *prepared = notes.largest <= 65504.0f && notes.largest <= 64.0f * average;
+    return DSX_OK;
+}
+
+int dsx_knn_search_host(int storage, const void* items, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,
+                        uint32_t num_queries, uint32_t k, float* scores, uint32_t* indexes, float* host_scores, uint32_t* host_indexes,
+                        void* workspace, size_t workspace_bytes, float* elapsed_ms)
+{
+    DSX_CHECK_ARG((host_scores == nullptr) == (host_indexes == nullptr), "dsx_knn_search_host: host_scores and host_indexes go together");
+    DSX_CHECK_ARG(storage != DSX_KNN_FP32_PREPARED || workspace, "dsx_knn_search_host: no prepared workspace");
+    const KnnResults out{scores, indexes, host_scores, host_indexes};
+    switch (storage) {
+    case DSX_KNN_FP32:
+    case DSX_KNN_FP32_PREPARED:
+        return knn_search_fp32((const float*)items, rows_padded, padding, dim, queries, num_queries, k, out, workspace, workspace_bytes, elapsed_ms,
+                               storage == DSX_KNN_FP32_PREPARED);
+    case DSX_KNN_FP16: return knn_search_f16(items, rows_padded, padding, dim, queries, num_queries, k, out, workspace, workspace_bytes, elapsed_ms);
+    case DSX_KNN_SPLIT: return knn_search_split(items, rows_padded, padding, dim, queries, num_queries, k, out, workspace, workspace_bytes, elapsed_ms);
+    default: return set_error(DSX_EINVAL, "dsx_knn_search_host: storage %d", storage);
+    }
 }
 
 }  // extern "C"

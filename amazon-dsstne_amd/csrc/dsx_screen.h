@@ -21,6 +21,7 @@ struct F16Job {
     uint32_t* seg_count;      // [batch][kF16ListStride]
     uint32_t seg_words;
     void* Z;                  // stored sums: halves, [batch][ldz], ldz a multiple of 256
+    void* M;                  // the largest of every 32 of them, [batch][ldz / 32]
     uint64_t ldz;
     const float* scale;       // [batch] what a row's sums are multiplied by before they are stored
 };
@@ -47,6 +48,7 @@ struct ScreenWorkspace {
     float* e0;
     float* scale;
     void* sums;
+    void* most;
     uint32_t* admit;
     uint64_t* keep;
     uint32_t* keep_count;
@@ -54,7 +56,7 @@ struct ScreenWorkspace {
     uint32_t* seg_count;
     size_t bytes;
 };
-ScreenWorkspace screen_layout(void* base, uint32_t batch, uint32_t dim, uint64_t n);
+ScreenWorkspace screen_layout(void* base, uint32_t batch, uint32_t dim, uint64_t n, uint32_t k);
 
 // Nearest neighbours, in pinned memory: the largest norm of the table, a sample of the norms and how many they are; whether a row
 // cannot be screened.
@@ -76,12 +78,16 @@ struct ScreenJob {
     const uint32_t* fidx;     // NULL: no filter
     float* keys;              // [batch][k]
     uint32_t* values;
-    uint32_t* row_flag;       // [batch], 0 before: set for rows without a result (the caller computes them again)
+    float* keys2;             // the same once more, in host memory that the device can write (or NULL)
+    uint32_t* values2;
+    uint32_t* row_flag;       // [batch] set for rows without a result (the caller computes them again), 0 for the others
     uint32_t* told;           // word that is set to 1 with the first of them (may be host memory; may be NULL)
     uint64_t* cand;           // [batch][cap]
-    uint32_t* cand_count;     // [batch], 0 before
+    uint32_t* cand_count;     // [batch]
     uint32_t cap;
     uint32_t* overflow;       // scratch word
+    uint32_t* clear;          // [clear_words] set to 0 on the way
+    uint32_t clear_words;
 };
 // The rows in f16 (and notes of the table and the rows, NULL: none), then the search itself.
 int screen_rows(const ScreenJob& j, const ScreenTable& t, const ScreenWorkspace& w, ScreenNotes* notes);

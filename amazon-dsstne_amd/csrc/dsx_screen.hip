@@ -7,8 +7,9 @@
 //
 // Error of a screened sum s' = sum x'_i w'_i against the fp32 sum s of the same row and column, x', w' rounded to f16 (unit
 // roundoff u = 2^-11, 2^-25 absolute below the normal range), fp32 accumulation:
-//   |s' - s| <= (2u + u^2) |x| |w| + 2^-25 sqrt(d) (|x| + |w|) + d 2^-50 + (3 d + 16) 2^-24 |x| |w|      (Cauchy-Schwarz; |.| = 2-norm)
-// (d 2^-50: both operands' absolute roundings together, all there is to go by where every component is near 2^-25)
+//   |s' - s| <= (2u + u^2) |x| |w| + 2^-25 sqrt(d) (|x| + |w|) + d 2^-50 + (1.1 d + 16) 2^-24 |x| |w|      (Cauchy-Schwarz; |.| = 2-norm)
+// (d 2^-50: both operands' absolute roundings together, all there is to go by where every component is near 2^-25; the last term: d
+// roundings of the matrix instructions' sums and d / 16 + 5 of screen_finish's)
 // With the column's norm |w| kept in the table and e1, e0 per row, that is e1 |w| + e0.  A sum starts from its column's bias, raised by
 // b_raise |b| for the roundings of a sum that holds it; z is that sum plus e1 |w|.  z + e0 is never below the score, whatever the
 // spread of the norms, and the score lies above z - width(z, |w|) (screen_width).  So:
@@ -22,6 +23,7 @@
 // where they are formed, in ranges that grow by a factor, after each of which the lists are cut back to what can still be a result.
 // Candidates of earlier ranges are not scored until the last one is through: what is scored in fp32 is about 1.2 k columns a row.
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include "dsx_screen.h"
 
@@ -34,15 +36,14 @@ constexpr float kF16Max = 65504.0f, kScreenMax = 60000.0f;
 constexpr uint32_t kPickWords = 2048;    // candidates of a row (part) that its workgroup holds
 constexpr uint32_t kKeepWords = 1024;    // candidates of a row that outlive a column range
 constexpr uint32_t kListWords = 4096;    // words of all of a row's lists of one column range
-constexpr uint32_t kPickGroups = 14;     // groups of 2,048 columns that a workgroup of 256 lanes holds in registers
-constexpr uint32_t kPickColumns = kPickGroups * 2048;
+constexpr uint32_t kPickBlocks = 2048;   // blocks of 32 columns that a workgroup reads
 
 uint32_t screen_ld(uint32_t dim) { return knn_f16_ld(dim); }
 uint32_t screen_pitch32(uint32_t dim) { return (dim + 3) / 4 * 4; }
 
 // Relative part of the error, with room for the rounding of the norms themselves; what a bias is raised by, per unit.
-__host__ __device__ __forceinline__ float screen_relative(uint32_t dim) { return 9.765625e-4f * 1.01f + (4.0f * (float)dim + 64.0f) * 5.9604645e-8f; }
-__host__ __device__ __forceinline__ float screen_bias_raise(uint32_t dim) { return ((float)dim + 64.0f) * 1.2e-7f; }
+__host__ __device__ __forceinline__ float screen_relative(uint32_t dim) { return 9.765625e-4f * 1.01f + (1.25f * (float)dim + 64.0f) * 5.9604645e-8f; }
+__host__ __device__ __forceinline__ float screen_bias_raise(uint32_t dim) { return ((float)dim + 64.0f) * 6.6e-8f; }
 
 // stats (nearest neighbours): [0] largest norm of a column (the bits of a non-negative float; NaN columns have no part in it: their
 // scores are NaN on every path); [1] sum of the norms of one column in 256, [2] their number
@@ -132,8 +133,11 @@ struct ScreenRowsArgs {
     float* e0;              // [batch]
     float* scale;           // [batch]
     int scaled;             // the scale follows the norms (else 1)
-    uint32_t* row_flag;     // [batch] set where the error has no bound
+    uint32_t* row_flag;     // [batch] set where the error has no bound, else cleared
     uint32_t* told;         // host-visible word set with it (may be NULL)
+    uint32_t* cand_count;   // [batch] cleared, and so is
+    uint32_t* clear;        // [clear_words]
+    uint32_t clear_words;
     const uint32_t* stats;
     ScreenNotes* notes;     // host-visible: what the table's columns and the rows are like (nearest neighbours)
 };
@@ -157,7 +161,11 @@ __global__ __launch_bounds__(256) void screen_rows_kernel(ScreenRowsArgs a)
         const float x = (valid && !bad && d < a.dim) ? a.X[(uint64_t)row * a.ldx + d] : 0.0f;
         a.out16[(uint64_t)row * a.ld + d] = (_Float16)x;
     }
+    if (blockIdx.x == 0)
+        for (uint32_t i = threadIdx.x; i < a.clear_words; i += 256) a.clear[i] = 0;
     if (!valid || lane != 0) return;
+    a.cand_count[row] = 0;
+    a.row_flag[row] = bad ? 1u : 0u;
     if (row == 0 && a.notes) {
         a.notes->largest = __uint_as_float(a.stats[0]);
         a.notes->sum = __uint_as_float(a.stats[1]);
@@ -174,10 +182,7 @@ __global__ __launch_bounds__(256) void screen_rows_kernel(ScreenRowsArgs a)
         if (most > 1e-30f && most < 1e30f) scale = ldexpf(1.0f, 10 - ilogbf(most));
     }
     a.scale[row] = scale;
-    if (bad) {
-        a.row_flag[row] = 1;
-        if (a.told) *(volatile uint32_t*)a.told = 1u;
-    }
+    if (bad && a.told) *(volatile uint32_t*)a.told = 1u;
 }
 
 // What the two kernels below have in common.
@@ -209,13 +214,12 @@ struct ScreenFoldArgs {
     uint64_t* cand;          // [batch][cap]
     uint32_t* cand_count;
     uint32_t cap;
-    int fresh;               // fold: nothing is kept from earlier ranges
     // pick
     const _Float16* Z;
+    const _Float16* M;
     uint64_t ldz;
     const float* scale;
     uint32_t stored;         // columns of Z
-    uint32_t parts, part_columns;
     // final
     const float* X;
     uint32_t ldx, dim, pitch32;
@@ -223,6 +227,8 @@ struct ScreenFoldArgs {
     const float* bias;
     float* keys;
     uint32_t* values;
+    float* keys2;
+    uint32_t* values2;
 };
 
 // A score lies above z less this.  (z: rounded up when it was stored as a half, which width_z and the last term cover; half_step: 1 /
@@ -258,81 +264,89 @@ __device__ __forceinline__ void screen_flag(const ScreenFoldArgs& a, uint32_t b)
 
 // The row's candidates sList[0 .. count) scored in fp32 and its k best written.  Sixteen lanes per candidate; the order of a sum depends on
 // nothing but its length.  Every lane of the workgroup calls this.
-__device__ __forceinline__ void screen_finish(const ScreenFoldArgs& a, uint32_t b, uint64_t* sList, uint32_t count, float* sX, uint64_t fs, uint64_t fe)
+// first: the caller's component threadIdx.x of the row; listed: whether the row has a listed column (the same for the workgroup).
+template <int T>
+__device__ __forceinline__ void screen_finish(const ScreenFoldArgs& a, uint32_t b, uint64_t* sList, uint32_t count, float* sX, float first, bool listed)
 {
-    __shared__ uint32_t sValid, sListed;
-    __shared__ uint64_t sKth;
+    __shared__ uint64_t sBest[256];   // by rank (k is 256 at most)
     const uint32_t dpad = (a.dim + 63) / 64 * 64;
-    for (uint32_t d = threadIdx.x; d < dpad; d += 256) sX[d] = (d < a.dim) ? a.X[(uint64_t)b * a.ldx + d] : 0.0f;
-    if (threadIdx.x == 0) {
-        sValid = sListed = 0;
-        sKth = 0;
-    }
+    if (threadIdx.x < dpad) sX[threadIdx.x] = first;
+    for (uint32_t d = T + threadIdx.x; d < dpad; d += T) sX[d] = (d < a.dim) ? a.X[(uint64_t)b * a.ldx + d] : 0.0f;
+    if (threadIdx.x < 256) sBest[threadIdx.x] = 0;
     __syncthreads();
+    // (four candidates of a group of lanes at a time: their rows are waited for together)
+    constexpr int U = 4;
     const uint32_t sub = threadIdx.x % 16;
-    for (uint32_t e0 = 0; e0 < count; e0 += 16) {
-        const uint32_t e = e0 + threadIdx.x / 16;
-        const uint32_t col = ~(uint32_t)sList[min(e, count - 1)];
-        float sum = 0.0f;
-        if (e < count) {
-            const float* w = a.rows32 + (uint64_t)col * a.pitch32;
-#pragma unroll 4
-            for (uint32_t d = 4 * sub; d < a.pitch32; d += 64) {
-                const float4 v = *reinterpret_cast<const float4*>(w + d), x = *reinterpret_cast<const float4*>(sX + d);
-                sum = fmaf(x.x, v.x, sum);
-                sum = fmaf(x.y, v.y, sum);
-                sum = fmaf(x.z, v.z, sum);
-                sum = fmaf(x.w, v.w, sum);
-            }
+    for (uint32_t e0 = threadIdx.x / 16; e0 < count; e0 += T / 16 * U) {
+        uint32_t col[U];
+        float sum[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            col[u] = ~(uint32_t)sList[min(e0 + T / 16 * u, count - 1)];
+            sum[u] = 0.0f;
+        }
+#pragma unroll 2
+        for (uint32_t d = 4 * sub; d < a.pitch32; d += 64) {
+            const float4 x = *reinterpret_cast<const float4*>(sX + d);
+            float4 v[U];
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                if (u == 0 || e0 + T / 16 * u < count) v[u] = *reinterpret_cast<const float4*>(a.rows32 + (uint64_t)col[u] * a.pitch32 + d);
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                if (u == 0 || e0 + T / 16 * u < count) {
+                    sum[u] = fmaf(x.x, v[u].x, sum[u]);
+                    sum[u] = fmaf(x.y, v[u].y, sum[u]);
+                    sum[u] = fmaf(x.z, v[u].z, sum[u]);
+                    sum[u] = fmaf(x.w, v[u].w, sum[u]);
+                }
         }
 #pragma unroll
-        for (int d = 1; d < 16; d *= 2) sum += __shfl_xor(sum, d);
-        if (sub == 0 && e < count) {
-            const float y = activate_rt(sum + (a.bias ? a.bias[col] : 0.0f), a.act, a.slope, a.alpha, a.lambda);
-            sList[e] = (y == y) ? ((uint64_t)score_key(y) << 32) | (uint32_t)~col : 0ull;
+        for (int u = 0; u < U; u++) {
+#pragma unroll
+            for (int d = 1; d < 16; d *= 2) sum[u] += __shfl_xor(sum[u], d);
+            if (sub == 0 && e0 + T / 16 * u < count) {
+                const float y = activate_rt(sum[u] + (a.bias ? a.bias[col[u]] : 0.0f), a.act, a.slope, a.alpha, a.lambda);
+                sList[e0 + T / 16 * u] = (y == y) ? ((uint64_t)score_key(y) << 32) | (uint32_t)~col[u] : 0ull;
+            }
         }
     }
     __syncthreads();
-    float* keys = a.keys + (uint64_t)b * a.k;
-    uint32_t* values = a.values + (uint64_t)b * a.k;
-    for (uint32_t i = threadIdx.x; i < count; i += 256) {
+    for (uint32_t i = threadIdx.x; i < count; i += T) {
         const uint64_t w = sList[i];
         if (w == 0) continue;
         uint32_t rank = 0;
         for (uint32_t j = 0; j < count; j++) rank += sList[j] > w;
-        atomicAdd(&sValid, 1u);
-        if (rank == a.k - 1) sKth = w;
-        if (rank < a.k) {
-            keys[rank] = key_score((uint32_t)(w >> 32));
-            values[rank] = ~(uint32_t)w;
+        if (rank < a.k) sBest[rank] = w;
+    }
+    __syncthreads();
+    if (threadIdx.x < a.k) {
+        const uint64_t w = sBest[threadIdx.x], at = (uint64_t)b * a.k + threadIdx.x;
+        const float key = w != 0 ? key_score((uint32_t)(w >> 32)) : -kMaxValue;   // engine/kernels.cu:3221-3224: unfilled slots
+        const uint32_t col = w != 0 ? ~(uint32_t)w : 0u;
+        a.keys[at] = key;
+        a.values[at] = col;
+        if (a.keys2) {
+            a.keys2[at] = key;
+            a.values2[at] = col;
         }
     }
     // A listed column scores 0, not nothing (utils/Filters.cpp:62 multiplies, kCalculateTopK then sees the zero): when the row's k-th
     // score is not above 0, or the row has fewer than k scores, such a zero belongs in the result, and the row is computed again.
-    if (fe > fs) {
-        bool listed = false;
-        for (uint64_t t = fs + threadIdx.x; t < fe; t += 256) listed |= a.fidx[t] < a.n;
-        if (__ballot(listed) != 0 && threadIdx.x % kWave == 0) atomicOr(&sListed, 1u);
-    }
-    __syncthreads();
-    for (uint32_t p = sValid + threadIdx.x; p < a.k; p += 256) {   // engine/kernels.cu:3221-3224: unfilled slots
-        keys[p] = -kMaxValue;
-        values[p] = 0;
-    }
-    if (threadIdx.x == 0 && sListed != 0 && (sKth == 0 || (uint32_t)(sKth >> 32) <= score_key(0.0f))) screen_flag(a, b);
+    if (threadIdx.x == 0 && listed && (uint32_t)(sBest[a.k - 1] >> 32) <= score_key(0.0f)) screen_flag(a, b);
 }
 
 // A lower bound of the k-th largest of the workgroup's keys (0: dead ones, not counted), exact in its upper 24 bits; 0 where there are
-// fewer than k.  Radix select, a byte at a time.  total: keys beyond that many are 0.  s: 258 words.
-template <int N> __device__ __forceinline__ uint32_t block_kth_key(const uint32_t (&key)[N], uint32_t total, uint32_t k, uint32_t* s)
+// fewer than k.  Radix select, a byte at a time.  T: lanes; total: keys beyond that many are 0.  s: 258 words.
+template <int N, int T = 256> __device__ __forceinline__ uint32_t block_kth_key(const uint32_t (&key)[N], uint32_t total, uint32_t k, uint32_t* s)
 {
     uint32_t prefix = 0, need = k;
     for (int shift = 24; shift >= 8; shift -= 8) {
-        s[threadIdx.x] = 0;
+        if (threadIdx.x < 256) s[threadIdx.x] = 0;
         __syncthreads();
 #pragma unroll
         for (int u = 0; u < N; u++)
-            if (u * 256 < total && key[u] != 0 && (shift == 24 || (key[u] >> (shift + 8)) == (prefix >> (shift + 8)))) atomicAdd(&s[(key[u] >> shift) & 255], 1u);
+            if (u * T < total && key[u] != 0 && (shift == 24 || (key[u] >> (shift + 8)) == (prefix >> (shift + 8)))) atomicAdd(&s[(key[u] >> shift) & 255], 1u);
         __syncthreads();
         if (threadIdx.x < kWave) {
             const uint32_t lane = threadIdx.x;
@@ -392,28 +406,32 @@ template <int N> __device__ __forceinline__ uint32_t screen_wave_kth(const uint3
     return t;
 }
 
-enum { kPickFinal, kPickKeep, kPickList };
+enum { kPickFinal, kPickKeep };
 
-// Sums stored as halves: what reaches the bound, of a row or a part of one.  Everything is requested at once and held in registers; the
-// bound is the k-th of R maxima per lane (over groups of eight columns that hold no listed one, each less its width).
-template <int R, int G, int MODE>
-__global__ __launch_bounds__(256, 4) void screen_pick_kernel(ScreenFoldArgs a)
+// Sums stored as halves: what reaches the bound.  The maxima of the row's blocks of 32 columns say which blocks can hold a result: the k-th
+// of R maxima per lane (over blocks without a listed column, each less its width) bounds the k-th score, and only blocks whose largest
+// sum reaches the bound are read.  Bound by latency: two round trips, a key search and, in the form that ends with the results, one
+// round trip for the candidates' rows.  T lanes, E blocks each.  1,024 rows x 27,278 top 10, 144 listed columns each: 15.4 us; with all
+// of the row in registers and the maxima taken from there, 27.6.
+template <int T, int R, int E, int MODE>
+__global__ __launch_bounds__(T, T == 256 ? 5 : 4) void screen_pick_kernel(ScreenFoldArgs a)
 {
     __builtin_amdgcn_s_setprio(3);   // short kernels issue ahead of a GEMM's wavefronts that share their SIMD
     __shared__ uint64_t sList[kPickWords];
-    __shared__ uint32_t sMax[R * 256];
-    __shared__ uint32_t sCount;
+    __shared__ uint32_t sMax[R * T];
+    __shared__ uint16_t sBlock[kPickBlocks];
+    __shared__ uint32_t sHist[MODE == kPickFinal ? 258 : 1];
+    __shared__ uint32_t sCount, sBlocks, sClean, sListed;
     __shared__ float sCut;
-    extern __shared__ __attribute__((aligned(16))) uint32_t sDyn[];   // bitmap of the part's listed columns; afterwards the row (kPickFinal)
-    const uint32_t b = blockIdx.x, part = blockIdx.y, lane = threadIdx.x % kWave;
-    const uint32_t lo = part * a.part_columns, hi = min(a.stored, lo + a.part_columns);
+    extern __shared__ __attribute__((aligned(16))) uint32_t sDyn[];   // bitmap of the listed columns, a word a block; afterwards the row (kPickFinal)
+    constexpr int C = E < 8 ? E : 8;
+    static_assert(E * T <= 65536 && E % C == 0, "block numbers are 16 bits wide");
+    const uint32_t b = blockIdx.x, lane = threadIdx.x % kWave;
+    const uint32_t blocks = (a.stored + 31) / 32;
     if (a.row_flag[b] != 0) {
-        if (threadIdx.x == 0) {
-            if constexpr (MODE == kPickKeep) {
-                a.admit[b] = 0xffffffffu;
-                a.keep_count[b] = 0;
-            }
-            if constexpr (MODE == kPickList) a.seg_count[(uint64_t)b * kF16ListStride + part] = 0;
+        if (MODE == kPickKeep && threadIdx.x == 0) {
+            a.admit[b] = 0xffffffffu;
+            a.keep_count[b] = 0;
         }
         return;
     }
@@ -424,128 +442,172 @@ __global__ __launch_bounds__(256, 4) void screen_pick_kernel(ScreenFoldArgs a)
         fs = a.fstart[r];
         fe = a.fend[r];
     }
-    half8 z[G];
-    float norms[G];   // largest of the 64 columns that the group lies in
-    const _Float16* src = a.Z + (uint64_t)b * a.ldz + lo;
+    const _Float16* src = a.Z + (uint64_t)b * a.ldz;
+    const _Float16* maxima = a.M + (uint64_t)b * (a.ldz / 32);
+    // blocks' maxima, and the largest norms of the 64 columns that they lie in: held, or asked for again, C blocks at a time
+    _Float16 most[C];
+    float norms[C];
+    auto ask = [&](int from) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < G; u++) {
-        const uint32_t c = (u * 256 + threadIdx.x) * 8;
-        if (lo + c < hi) z[u] = *reinterpret_cast<const half8*>(src + c);   // (rows of Z are padded to whole tiles)
-        else
-#pragma unroll
-            for (int e = 0; e < 8; e++) z[u][e] = (_Float16)(-65504.0f);
-    }
-#pragma unroll
-    for (int u = 0; u < G; u++) {
-        const uint32_t c = lo + (u * 256 + threadIdx.x) * 8;
-        norms[u] = a.seg_norm[(c < hi ? c : lo) / 64];
-    }
-    const uint32_t words = (hi - lo + 31) / 32;
+        for (int e = 0; e < C; e++) {
+            const uint32_t i = min((from + e) * T + threadIdx.x, blocks - 1);
+            most[e] = maxima[i];
+            norms[e] = a.seg_norm[i / 2];
+        }
+    };
+    if constexpr (C == E) ask(0);
+    float first = 0.0f;
+    if (MODE == kPickFinal && threadIdx.x < a.dim) first = a.X[(uint64_t)b * a.ldx + threadIdx.x];
     if (fe > fs)
-        for (uint32_t i = threadIdx.x; i < words; i += 256) sDyn[i] = 0;
-    if (threadIdx.x == 0) sCount = 0;
+        for (uint32_t i = threadIdx.x; i < blocks; i += T) sDyn[i] = 0;
+    if (threadIdx.x == 0) sCount = sBlocks = sClean = sListed = 0;
     const float e1 = a.e1[b], e0 = a.e0[b], step = 1.0f / a.scale[b];   // (a power of two)
     __syncthreads();
     if (fe > fs) {
-        for (uint64_t t = fs + threadIdx.x; t < fe; t += 256) {
+        bool any = false;
+        for (uint64_t t = fs + threadIdx.x; t < fe; t += T) {
             const uint32_t c = a.fidx[t];
-            if (c >= lo && c < hi) atomicOr(&sDyn[(c - lo) >> 5], 1u << ((c - lo) & 31));
+            if (c < a.stored) atomicOr(&sDyn[c >> 5], 1u << (c & 31));
+            any |= c < a.n;
         }
+        if (MODE == kPickFinal && __ballot(any) != 0 && lane == 0) atomicOr(&sListed, 1u);
         __syncthreads();
-        // a group of eight columns is a byte of the bitmap: listed ones have no part in the bound
-#pragma unroll
-        for (int u = 0; u < G; u++) {
-            const uint32_t c = (u * 256 + threadIdx.x) * 8;
-            const uint32_t listed = (lo + c < hi) ? reinterpret_cast<const unsigned char*>(sDyn)[c / 8] : 0u;
-            if (__ballot(listed != 0) == 0) continue;
-#pragma unroll
-            for (int e = 0; e < 8; e++)
-                if ((listed >> e) & 1) z[u][e] = (_Float16)(-65504.0f);
-        }
+        // A block with a listed column has no part in the bound, unless too few others are left: then its other columns are looked at.
+        uint32_t clean = 0;
+#pragma unroll 4
+        for (int e = 0; e < E; e++) clean += (uint32_t)__popcll(__ballot(e * T + threadIdx.x < blocks && sDyn[min(e * T + threadIdx.x, blocks - 1)] == 0));
+        if (lane == 0) atomicAdd(&sClean, clean);
+        __syncthreads();
     }
-    auto largest = [&](int u) __attribute__((always_inline)) -> float {
-        const half2v x = __builtin_elementwise_max(__builtin_elementwise_max(half2v{z[u][0], z[u][1]}, half2v{z[u][2], z[u][3]}),
-                                                   __builtin_elementwise_max(half2v{z[u][4], z[u][5]}, half2v{z[u][6], z[u][7]}));
-        return (float)__builtin_elementwise_max(x[0], x[1]);
-    };
+    const bool exact = fe > fs && sClean < min(4 * a.k, blocks);   // the same for the whole workgroup
     {
         float low[R];
 #pragma unroll
         for (int i = 0; i < R; i++) low[i] = -__builtin_inff();
+#pragma unroll 1
+        for (int from = 0; from < E; from += C) {
+            if (from * T >= blocks) break;
+            if constexpr (C != E) ask(from);
 #pragma unroll
-        for (int u = 0; u < G; u++) {
-            const float m = largest(u), raised = fmaf(m, step, e1 * norms[u]);
-            // (what does not fit a half says nothing: rounded up to infinity, or held at the lowest half, as the places beyond the end are)
-            const float l = (m < 65504.0f && m > -65504.0f) ? raised - screen_width(a, raised, norms[u], e1, e0, step) : -__builtin_inff();
-            low[u % R] = fmaxf(low[u % R], l);
+            for (int u = 0; u < C; u++) {
+                const uint32_t i = (from + u) * T + threadIdx.x, listed = (fe > fs && i < blocks) ? sDyn[i] : 0u;
+                float m = (float)most[u];
+                if (listed != 0) {
+                    m = -65504.0f;
+                    if (exact)
+                        for (uint32_t c = 0; c < 32; c += 8) {
+                            const half8 z = *reinterpret_cast<const half8*>(src + (uint64_t)i * 32 + c);
+#pragma unroll
+                            for (int x = 0; x < 8; x++)
+                                if (!((listed >> (c + x)) & 1u)) m = fmaxf(m, (float)z[x]);
+                        }
+                }
+                const float norm = norms[u], raised = fmaf(m, step, e1 * norm);
+                // (what does not fit a half says nothing: rounded up to infinity, or held at the lowest half)
+                if (i < blocks && m < 65504.0f && m > -65504.0f) low[u % R] = fmaxf(low[u % R], raised - screen_width(a, raised, norm, e1, e0, step));
+            }
         }
 #pragma unroll
-        for (int i = 0; i < R; i++) sMax[i * 256 + threadIdx.x] = score_key(low[i]);
+        for (int i = 0; i < R; i++) sMax[i * T + threadIdx.x] = score_key(low[i]);
     }
     __syncthreads();
     // (one wavefront searches, a different one from row to row, so that the four SIMDs of a compute unit share the searches)
     if (__builtin_amdgcn_readfirstlane(threadIdx.x / kWave) == ((b >> 8) & 3u)) {
-        uint32_t all[4 * R];
+        constexpr int K = R * T / kWave;
+        uint32_t all[K];
 #pragma unroll
-        for (int i = 0; i < 4 * R; i++) all[i] = sMax[i * kWave + lane];
-        const uint32_t t = screen_wave_kth<4 * R>(all, a.k);
+        for (int i = 0; i < K; i++) all[i] = sMax[i * kWave + lane];
+        const uint32_t t = screen_wave_kth<K>(all, a.k);
         if (lane == 0) sCut = screen_cut(a, t > score_key(-__builtin_inff()) ? key_score(t) : -__builtin_inff(), e0);
     }
     __syncthreads();
     const float cut = sCut;
+#pragma unroll 1
+    for (int from = 0; from < E; from += C) {
+        if (from * T >= blocks) break;
+        if constexpr (C != E) ask(from);
 #pragma unroll
-    for (int u = 0; u < G; u++) {
-        uint32_t at0 = lo + (u * 256 + threadIdx.x) * 8;
-        asm volatile("" : "+v"(at0));   // (the norm is read again, from the cache, and not kept)
-        const float raise = e1 * a.seg_norm[(at0 < hi ? at0 : lo) / 64];
-        if (__ballot(fmaf(largest(u), step, raise) >= cut) == 0) continue;
+        for (int u = 0; u < C; u++) {
+            const uint32_t i = (from + u) * T + threadIdx.x;
+            const bool hot = i < blocks && fmaf((float)most[u], step, e1 * norms[u]) >= cut;
+            const uint64_t m = __ballot(hot);
+            if (m == 0) continue;
+            uint32_t at = 0;
+            if (lane == 0) at = atomicAdd(&sBlocks, (uint32_t)__popcll(m));
+            at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at) + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+            if (hot && at < kPickBlocks) sBlock[at] = (uint16_t)i;
+        }
+    }
+    __syncthreads();
+    const uint32_t hot_blocks = sBlocks;
+    const bool many = hot_blocks > kPickBlocks;   // (thousands of tied scores: the row is given up below)
+    // four lanes a block, eight columns each
+    for (uint32_t p0 = 0; p0 < hot_blocks && !many; p0 += T / 4) {
+        const uint32_t p = p0 + threadIdx.x / 4;
+        const uint32_t block = sBlock[min(p, hot_blocks - 1)], c0 = block * 32 + threadIdx.x % 4 * 8;
+        half8 z = {};
+        if (p < hot_blocks) z = *reinterpret_cast<const half8*>(src + c0);   // (rows of Z are padded to whole tiles)
+        const float raise = e1 * a.seg_norm[block / 2];
+        uint32_t listed = (fe > fs) ? sDyn[block] >> (threadIdx.x % 4 * 8) : 0u;
+        if (p >= hot_blocks) listed = 0xffu;
 #pragma unroll
         for (int e = 0; e < 8; e++) {
-            const uint32_t c = (u * 256 + threadIdx.x) * 8 + e;
-            uint32_t bits = __builtin_bit_cast(u32x4s, z[u])[e / 2];
-            asm volatile("" : "+v"(bits));   // (unpacked here, where one is needed, and not for all groups at once)
-            const half2v two = __builtin_bit_cast(half2v, bits);
-            const float h = (float)two[e & 1];
-            bool ok = fmaf(h, step, raise) >= cut && lo + c < hi;
-            if (ok && fe > fs) ok = !((sDyn[c >> 5] >> (c & 31)) & 1u);
+            const float h = (float)z[e];
+            const bool ok = fmaf(h, step, raise) >= cut && c0 + e < a.stored && !((listed >> e) & 1u);
             const uint64_t m = __ballot(ok);
             if (m == 0) continue;
             uint32_t at = 0;
             if (lane == 0) at = atomicAdd(&sCount, (uint32_t)__popcll(m));
             at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at) + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-            if (ok && at < kPickWords) sList[at] = ((uint64_t)score_key(h * step) << 32) | (uint32_t)~(lo + c);   // (not raised: screen_raised)
+            if (ok && at < kPickWords) sList[at] = ((uint64_t)score_key(h * step) << 32) | (uint32_t)~(c0 + e);   // (not raised: screen_raised)
         }
     }
     __syncthreads();
     const uint32_t count = sCount;
-    if (count > (MODE == kPickKeep ? kKeepWords : kPickWords)) {   // the same for the whole workgroup
+    if (many || count > (MODE == kPickKeep ? kKeepWords : kPickWords)) {   // the same for the whole workgroup
         if (threadIdx.x == 0) {
             screen_flag(a, b);
             if constexpr (MODE == kPickKeep) a.keep_count[b] = 0;
-            if constexpr (MODE == kPickList) a.seg_count[(uint64_t)b * kF16ListStride + part] = 0;
         }
         return;
     }
-    if constexpr (MODE == kPickKeep)
-        for (uint32_t i = threadIdx.x; i < count; i += 256) sList[i] = screen_raised(a, sList[i], e1);   // (a lane reads below what it writes here)
-    if constexpr (MODE == kPickFinal) {
-        screen_finish(a, b, sList, count, reinterpret_cast<float*>(sDyn), fs, fe);
-    } else if constexpr (MODE == kPickKeep) {
-        for (uint32_t i = threadIdx.x; i < count; i += 256) a.keep[(uint64_t)b * kKeepWords + i] = sList[i];
+    if constexpr (MODE == kPickKeep) {
+        for (uint32_t i = threadIdx.x; i < count; i += T) a.keep[(uint64_t)b * kKeepWords + i] = screen_raised(a, sList[i], e1);
         if (threadIdx.x == 0) {
             a.keep_count[b] = count;
             a.admit[b] = score_key(cut);
         }
     } else {
-        uint64_t* mine = a.seg + ((uint64_t)b * a.lists + part) * a.seg_cap;
-        for (uint32_t i = threadIdx.x; i < count; i += 256) {
-            if (i < a.seg_cap) mine[i] = sList[i];
-            else {   // the row's shared list
-                const uint32_t p = atomicAdd(&a.cand_count[b], 1u);
-                if (p < a.cap) a.cand[(uint64_t)b * a.cap + p] = sList[i];
+        // With many candidates of long rows, the k-th of the candidates' own bounds (by column and not by block) first: a third of them go.
+        uint32_t left = count;
+        if (a.k > 32 && a.dim >= 256 && count > a.k) {   // the same for the whole workgroup
+            constexpr int W = kPickWords / T;
+            uint64_t word[W];
+            uint32_t low[W];
+#pragma unroll
+            for (int u = 0; u < W; u++) {
+                const uint32_t i = u * T + threadIdx.x;
+                word[u] = 0;
+                low[u] = 0;
+                if (i >= count) continue;
+                word[u] = screen_raised(a, sList[i], e1);
+                const float z = key_score((uint32_t)(word[u] >> 32)), l = z - screen_width(a, z, a.norm[~(uint32_t)word[u]], e1, e0, step);
+                low[u] = (l > -__builtin_inff()) ? score_key(l) : 0u;
             }
+            const uint32_t t = block_kth_key<W, T>(low, count, a.k, sHist);
+            if (threadIdx.x == 0) {
+                sCut = screen_cut(a, t != 0 ? key_score(t) : -__builtin_inff(), e0);
+                sCount = 0;
+            }
+            __syncthreads();
+            const float closer = sCut;
+#pragma unroll
+            for (int u = 0; u < W; u++)
+                if (word[u] != 0 && key_score((uint32_t)(word[u] >> 32)) >= closer) sList[atomicAdd(&sCount, 1u)] = word[u];
+            __syncthreads();
+            left = sCount;
         }
-        if (threadIdx.x == 0) a.seg_count[(uint64_t)b * kF16ListStride + part] = min(count, a.seg_cap);
+        screen_finish<T>(a, b, sList, left, reinterpret_cast<float*>(sDyn), first, sListed != 0);
     }
 }
 
@@ -570,7 +632,7 @@ __global__ __launch_bounds__(256, 4) void screen_fold_kernel(ScreenFoldArgs a)
     const uint32_t shared = a.cand_count[b];
     const bool flagged = a.row_flag[b] != 0;
     uint32_t incl = (threadIdx.x < a.lists) ? min(a.seg_count[(uint64_t)b * kF16ListStride + threadIdx.x], a.seg_cap) : 0u;
-    const uint32_t kept = a.fresh ? 0u : a.keep_count[b];
+    const uint32_t kept = a.keep_count[b];
     const float e1 = a.e1[b], e0 = a.e0[b], step = 1.0f / a.scale[b];
     uint64_t fs = 0, fe = 0;
     if (a.fidx) {
@@ -645,7 +707,7 @@ __global__ __launch_bounds__(256, 4) void screen_fold_kernel(ScreenFoldArgs a)
 #pragma unroll
             for (int u = 0; u < NW; u++) {
                 const uint32_t i = u * 256 + threadIdx.x;
-                if (first) key[u] = low[u] = 0;
+                if (first) key[u] = low[u] = col[u] = 0;
                 if (u * 256 >= here || i >= here || (!first && key[u] == 0)) continue;
                 const uint32_t e = pos + (i - carried);
                 const bool new_word = i >= carried && e >= kept;
@@ -705,7 +767,11 @@ __global__ __launch_bounds__(256, 4) void screen_fold_kernel(ScreenFoldArgs a)
     }
     const uint32_t count = carried;
     if constexpr (FINAL) {
-        screen_finish(a, b, left, count, reinterpret_cast<float*>(sDyn), fs, fe);
+        float x = 0.0f;
+        if (threadIdx.x < a.dim) x = a.X[(uint64_t)b * a.ldx + threadIdx.x];
+        bool any = false;
+        for (uint64_t t = fs + threadIdx.x; t < fe; t += 256) any |= a.fidx[t] < a.n;
+        screen_finish<256>(a, b, left, count, reinterpret_cast<float*>(sDyn), x, __syncthreads_or(any) != 0);
     } else {
         for (uint32_t i = threadIdx.x; i < count; i += 256) a.keep[(uint64_t)b * kKeepWords + i] = left[i];
         if (threadIdx.x == 0) {
@@ -765,26 +831,20 @@ bool screen_search_pays(uint32_t batch, uint32_t dim, uint64_t n, uint32_t k, bo
 static inline size_t align256(size_t x) { return (x + 255) / 256 * 256; }
 
 // Whether all columns' sums are stored.  (They are compared with bounds only where a bound keeps most columns out, and where there
-// are rows for the whole GPU: a workgroup of that kind has 256 rows, and 64 share a row's columns at most.)
+// are rows for the whole GPU: a workgroup of that kind has 256 rows, and 64 share a row's columns at most.)  A workgroup reads the maxima of
+// 131,072 columns; few rows have one of four times as many wavefronts each, which takes the bitmap of a million columns' filter.
 static bool screen_stored(uint32_t batch, uint64_t n)
 {
     if (ctx().knobs.fc_topk_first_columns) return false;
-    return (n <= 131072 || (batch <= 512 && n <= 64 * kPickColumns)) && (uint64_t)batch * n <= ((uint64_t)1 << 30);
+    return (n <= 131072 || (batch <= 512 && n <= 1048576)) && (uint64_t)batch * n <= ((uint64_t)1 << 30);
 }
 
-static uint32_t screen_first_columns(uint32_t n)
+static uint32_t screen_first_columns(uint32_t n, uint32_t k)
 {
-    uint32_t c = ctx().knobs.fc_topk_first_columns ? ctx().knobs.fc_topk_first_columns : 8192;
-    c = std::max(256u, std::min(c, kPickColumns)) / 256 * 256;
+    // (two blocks of maxima for each of the k best: with fewer the bound is far below the k-th score; sixteen chunks of whole tiles)
+    uint32_t c = ctx().knobs.fc_topk_first_columns ? ctx().knobs.fc_topk_first_columns : (std::max(8192u, 64 * k) + 4095) / 4096 * 4096;
+    c = std::max(256u, std::min(c, 32768u)) / 256 * 256;
     return std::min(c, n);
-}
-
-// Workgroups per row of the stored sums.
-static uint32_t screen_parts(uint32_t batch, uint32_t n)
-{
-    const uint32_t least = (n + kPickColumns - 1) / kPickColumns;
-    const uint32_t wanted = std::min((2 * (uint32_t)ctx().num_cus + batch - 1) / batch, std::max(1u, n / 8192));
-    return std::min(64u, std::max(least, wanted));
 }
 
 ScreenTable screen_table(void* base, uint32_t dim, uint64_t n)
@@ -806,11 +866,11 @@ ScreenTable screen_table(void* base, uint32_t dim, uint64_t n)
     return t;
 }
 
-ScreenWorkspace screen_layout(void* base, uint32_t batch, uint32_t dim, uint64_t n)
+ScreenWorkspace screen_layout(void* base, uint32_t batch, uint32_t dim, uint64_t n, uint32_t k)
 {
     ScreenWorkspace w;
     char* p = (char*)base;
-    const uint64_t columns = screen_stored(batch, n) ? n : screen_first_columns((uint32_t)n);
+    const uint64_t columns = screen_stored(batch, n) ? n : screen_first_columns((uint32_t)n, k);
     w.rows16 = p;
     p += align256(knn_f16_rows(batch) * screen_ld(dim) * 2);
     w.e1 = (float*)p;
@@ -821,6 +881,8 @@ ScreenWorkspace screen_layout(void* base, uint32_t batch, uint32_t dim, uint64_t
     p += align256((size_t)batch * sizeof(float));
     w.sums = p;
     p += align256(batch * ((columns + 255) / 256 * 256) * 2);
+    w.most = p;
+    p += align256(batch * ((columns + 255) / 256 * 8) * 2);
     w.admit = (uint32_t*)p;
     p += align256((size_t)batch * sizeof(uint32_t));
     w.keep = (uint64_t*)p;
@@ -855,32 +917,41 @@ int screen_rows(const ScreenJob& j, const ScreenTable& t, const ScreenWorkspace&
     ScreenRowsArgs r{};
     r.X = j.X; r.ldx = j.ldx; r.batch = j.batch; r.dim = j.dim; r.ld = screen_ld(j.dim);
     r.out16 = (_Float16*)w.rows16; r.e1 = w.e1; r.e0 = w.e0; r.scale = w.scale; r.scaled = j.bias == nullptr; r.row_flag = j.row_flag; r.told = notes ? &notes->flag : j.told;
+    r.cand_count = j.cand_count; r.clear = j.clear; r.clear_words = j.clear_words;
     r.stats = t.stats; r.notes = notes;
     hipLaunchKernelGGL(screen_rows_kernel, dim3((uint32_t)(knn_f16_rows(j.batch) / 4)), dim3(256), 0, ctx().stream, r);
     DSX_LAUNCH_CHECK("screen_rows_kernel");
     return DSX_OK;
 }
 
-template <int R, int G> static int launch_pick_mode(const ScreenFoldArgs& a, int mode, size_t lds)
+template <int T, int R, int E, int MODE> static int launch_pick_as(const ScreenFoldArgs& a, size_t lds)
 {
-    const dim3 grid(a.batch, a.parts);
-    hipStream_t s = ctx().stream;
-    switch (mode) {
-    case kPickFinal: hipLaunchKernelGGL((screen_pick_kernel<R, G, kPickFinal>), grid, dim3(256), lds, s, a); break;
-    case kPickKeep: hipLaunchKernelGGL((screen_pick_kernel<R, G, kPickKeep>), grid, dim3(256), lds, s, a); break;
-    default: hipLaunchKernelGGL((screen_pick_kernel<R, G, kPickList>), grid, dim3(256), lds, s, a); break;
+    // More LDS than a kernel gets unasked, for the bitmap of 262,144 columns and more.  Asked for once per device, as much as there can
+    // be: threads that come here together ask for the same.
+    if (lds > 65536 - 32768) {
+        static std::atomic<bool> asked[64] = {};
+        const int dev = ctx().device;
+        if (dev < 0 || dev >= 64 || !asked[dev].load(std::memory_order_acquire)) {
+            DSX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&screen_pick_kernel<T, R, E, MODE>), hipFuncAttributeMaxDynamicSharedMemorySize, 131072));
+            if (dev >= 0 && dev < 64) asked[dev].store(true, std::memory_order_release);
+        }
     }
+    hipLaunchKernelGGL((screen_pick_kernel<T, R, E, MODE>), dim3(a.batch), dim3(T), lds, ctx().stream, a);
     DSX_LAUNCH_CHECK("screen_pick_kernel");
     return DSX_OK;
 }
 
-static int launch_pick(const ScreenFoldArgs& a, int mode)
+static int launch_pick(const ScreenFoldArgs& a, bool keep)
 {
-    const size_t bitmap = a.fidx ? ((size_t)a.part_columns + 31) / 32 * 4 : 0, row = mode == kPickFinal ? (size_t)(a.dim + 63) / 64 * 256 : 0;
+    const size_t bitmap = a.fidx ? ((size_t)a.stored + 31) / 32 * 4 : 0, row = keep ? 0 : (size_t)(a.dim + 63) / 64 * 256;
     const size_t lds = std::max<size_t>(16, std::max(bitmap, row));
     // (maxima: a lane's only one for small k, four where more than one of the k best are likely to share a lane)
-    if (a.part_columns <= 8192) return a.k <= 32 ? launch_pick_mode<1, 4>(a, mode, lds) : launch_pick_mode<4, 4>(a, mode, lds);
-    return a.k <= 32 ? launch_pick_mode<1, kPickGroups>(a, mode, lds) : launch_pick_mode<4, kPickGroups>(a, mode, lds);
+    const bool one = a.k <= 32;
+    if (keep) return one ? launch_pick_as<256, 1, 4, kPickKeep>(a, lds) : launch_pick_as<256, 4, 4, kPickKeep>(a, lds);
+    if (a.batch > 64 && a.stored <= 32768) return one ? launch_pick_as<256, 1, 4, kPickFinal>(a, lds) : launch_pick_as<256, 4, 4, kPickFinal>(a, lds);
+    if (a.batch > 512) return one ? launch_pick_as<256, 1, 16, kPickFinal>(a, lds) : launch_pick_as<256, 4, 16, kPickFinal>(a, lds);
+    if (a.stored <= 131072) return launch_pick_as<1024, 1, 4, kPickFinal>(a, lds);
+    return launch_pick_as<1024, 1, 32, kPickFinal>(a, lds);
 }
 
 int screen_run(const ScreenJob& j, const ScreenTable& t, const ScreenWorkspace& w)
@@ -888,11 +959,11 @@ int screen_run(const ScreenJob& j, const ScreenTable& t, const ScreenWorkspace& 
     hipStream_t s = ctx().stream;
     const uint32_t ld = screen_ld(j.dim), n = j.n;
     const bool stored = screen_stored(j.batch, n);
-    const uint32_t n0 = stored ? n : screen_first_columns(n);
+    const uint32_t n0 = stored ? n : screen_first_columns(n, j.k);
     F16Job f{};
     f.Q = w.rows16; f.items = t.items16; f.ld = ld; f.batch = j.batch; f.n = n0;
     f.norm = t.norm; f.bias = j.bias; f.e1 = w.e1; f.bias_raise = screen_bias_raise(j.dim);
-    f.Z = w.sums; f.ldz = (n0 + 255) / 256 * 256; f.scale = w.scale;
+    f.Z = w.sums; f.M = w.most; f.ldz = (n0 + 255) / 256 * 256; f.scale = w.scale;
     int rc = f16_store_run(f);
     if (rc) return rc;
     ScreenFoldArgs a{};
@@ -906,28 +977,15 @@ int screen_run(const ScreenJob& j, const ScreenTable& t, const ScreenWorkspace& 
     a.keep = w.keep; a.keep_count = w.keep_count; a.admit = w.admit;
     a.seg = w.seg; a.seg_count = w.seg_count;
     a.cand = j.cand; a.cand_count = j.cand_count; a.cap = j.cap;
-    a.Z = (const _Float16*)w.sums; a.ldz = f.ldz; a.scale = w.scale; a.stored = n0;
+    a.Z = (const _Float16*)w.sums; a.M = (const _Float16*)w.most; a.ldz = f.ldz; a.scale = w.scale; a.stored = n0;
     a.X = j.X; a.ldx = j.ldx; a.dim = j.dim; a.pitch32 = screen_pitch32(j.dim); a.rows32 = t.rows32; a.bias = j.bias;
-    a.keys = j.keys; a.values = j.values;
+    a.keys = j.keys; a.values = j.values; a.keys2 = j.keys2; a.values2 = j.values2;
     a.width_z = 2.1f * f.bias_raise + 1.0e-3f;   // (rounding up to a half: 9.9e-4 of it at most)
-    a.parts = stored ? screen_parts(j.batch, n) : 1;
-    a.part_columns = ((n0 + a.parts - 1) / a.parts + 63) / 64 * 64;
-    a.parts = (n0 + a.part_columns - 1) / a.part_columns;
-    a.lists = a.parts; a.seg_cap = kListWords / a.parts;
-    const bool whole = stored && a.parts == 1;
-    if ((rc = launch_pick(a, whole ? kPickFinal : stored ? kPickList : kPickKeep))) return rc;
-    if (whole) return DSX_OK;
+    if ((rc = launch_pick(a, !stored)) || stored) return rc;
     const size_t row_lds = (size_t)(j.dim + 63) / 64 * 256;
-    if (stored) {
-        a.fresh = 1;
-        hipLaunchKernelGGL((screen_fold_kernel<true>), dim3(j.batch), dim3(256), row_lds, s, a);
-        DSX_LAUNCH_CHECK("screen_fold_kernel");
-        return DSX_OK;
-    }
     // A bound taken over `done` columns lets about k * width / done of the next `width` columns pass: ranges grow by a factor that
     // keeps that near an eighth of the lists (the sample's own items, which score high and pass as well, come on top).
     const uint32_t growth = std::max(4u, j.cap / (8 * j.k));
-    a.fresh = 0;
     for (uint32_t done = n0; done < n;) {
         uint32_t ncols = (uint32_t)std::min<uint64_t>((uint64_t)n - done, (uint64_t)done * growth);
         if (n - done - ncols < 256) ncols = n - done;   // no sliver of a last range

@@ -307,6 +307,8 @@ struct TopKArgs {
     // results: either final (keys/values, pitch k) or packed partial lists
     float* keys;
     uint32_t* values;
+    float* keys2;               // the final results once more (pinned host memory), or NULL
+    uint32_t* values2;
     uint64_t* partial;          // [batch][partial_slots][k]
     uint32_t partial_slots;
     uint32_t partial_slot0;     // this launch writes slots partial_slot0 + segment
@@ -381,6 +383,10 @@ __device__ __forceinline__ void finish_row(WaveTopK<R>& list, uint64_t (*sStage)
         } else {
             keys[p] = key;
             values[p] = col;
+            if (a.keys2) {
+                a.keys2[(uint64_t)b * a.k + p] = key;
+                a.values2[(uint64_t)b * a.k + p] = col;
+            }
         }
     };
 
@@ -1403,7 +1409,7 @@ __global__ __launch_bounds__(kTopkThreads, R <= 2 ? 4 : 2) void topk_guided_kern
 // against one wavefront that sorts and merges 64 words at a time.)
 template <int R>
 __global__ __launch_bounds__(kTopkThreads) void topk_merge_kernel(const uint64_t* partial, uint32_t slots, uint32_t k, float* keys,
-                                                                  uint32_t* values)
+                                                                  uint32_t* values, float* keys2, uint32_t* values2)
 {
     __builtin_amdgcn_s_setprio(3);   // short kernels issue ahead of a GEMM's wavefronts that share their SIMD
     using List = WaveTopK<R>;
@@ -1415,6 +1421,8 @@ __global__ __launch_bounds__(kTopkThreads) void topk_merge_kernel(const uint64_t
     a.k = k;
     a.keys = keys;
     a.values = values;
+    a.keys2 = keys2;
+    a.values2 = values2;
     if (slots == 1) {   // already in order
         for (uint32_t p = threadIdx.x; p < k; p += kTopkThreads) {
             float key = -kMaxValue;
@@ -1422,6 +1430,10 @@ __global__ __launch_bounds__(kTopkThreads) void topk_merge_kernel(const uint64_t
             if (src[p] != 0) unpack_score(src[p], key, col);
             keys[(uint64_t)b * k + p] = key;
             values[(uint64_t)b * k + p] = col;
+            if (keys2) {
+                keys2[(uint64_t)b * k + p] = key;
+                values2[(uint64_t)b * k + p] = col;
+            }
         }
         return;
     }
@@ -1508,9 +1520,10 @@ template <int R> static int launch_scan(const TopKArgs& a, uint32_t batch, bool 
     return DSX_OK;
 }
 
-template <int R> static int launch_merge(const uint64_t* partial, uint32_t slots, uint32_t k, float* keys, uint32_t* values, uint32_t batch)
+template <int R> static int launch_merge(const uint64_t* partial, uint32_t slots, uint32_t k, float* keys, uint32_t* values, uint32_t batch, float* keys2,
+                                         uint32_t* values2)
 {
-    hipLaunchKernelGGL((topk_merge_kernel<R>), dim3(batch), dim3(kTopkThreads), 0, ctx().stream, partial, slots, k, keys, values);
+    hipLaunchKernelGGL((topk_merge_kernel<R>), dim3(batch), dim3(kTopkThreads), 0, ctx().stream, partial, slots, k, keys, values, keys2, values2);
     DSX_LAUNCH_CHECK("topk_merge_kernel");
     return DSX_OK;
 }
@@ -1529,8 +1542,6 @@ uint32_t topk_segments(uint32_t batch, uint32_t width, bool filtered)
     }
     return std::max(1u, s);
 }
-
-int topk_merge(const uint64_t* partial, uint32_t slots, uint32_t k, float* keys, uint32_t* values, uint32_t batch);
 
 int topk_run(const float* in, uint32_t pitch, uint32_t width, uint32_t batch, uint32_t k, float* keys, uint32_t* values,
              uint32_t position, const uint32_t* index, const uint64_t* fstart, const uint64_t* fend, const uint32_t* fidx,
@@ -1586,11 +1597,11 @@ int topk_run(const float* in, uint32_t pitch, uint32_t width, uint32_t batch, ui
     return DSX_OK;
 }
 
-int topk_merge(const uint64_t* partial, uint32_t slots, uint32_t k, float* keys, uint32_t* values, uint32_t batch)
+int topk_merge(const uint64_t* partial, uint32_t slots, uint32_t k, float* keys, uint32_t* values, uint32_t batch, float* keys2, uint32_t* values2)
 {
-    if (k <= 64) return launch_merge<1>(partial, slots, k, keys, values, batch);
-    if (k <= 128) return launch_merge<2>(partial, slots, k, keys, values, batch);
-    return launch_merge<4>(partial, slots, k, keys, values, batch);
+    if (k <= 64) return launch_merge<1>(partial, slots, k, keys, values, batch, keys2, values2);
+    if (k <= 128) return launch_merge<2>(partial, slots, k, keys, values, batch, keys2, values2);
+    return launch_merge<4>(partial, slots, k, keys, values, batch, keys2, values2);
 }
 
 // Exact KNN with candidate lists: merges a row's running best list (k packed words, best first) with the candidates the last

@@ -359,15 +359,22 @@ size_t dsx_knn_workspace_bytes(uint32_t rows_padded, uint32_t dim, uint32_t num_
 /* dsx_knn_workspace_bytes holds, for 512 queries and more, two copies of the table (1.5 x its size, up to 8 GiB) that make the search
  * faster (its candidates are screened in 16 bits); a workspace of at least this size but not that one is searched without them. */
 size_t dsx_knn_workspace_bytes_least(uint32_t rows_padded, uint32_t dim, uint32_t num_queries, uint32_t k);
-/* Fills the two copies once, for a caller that searches one table many times: workspace holds dsx_knn_workspace_bytes(rows_padded, dim,
- * num_queries, k) bytes (256-byte aligned).  *prepared: whether it did (the table may not be worth it, or unfit for it).  A prepared
- * workspace goes with dsx_knn_search_prepared and searches of up to num_queries queries and the same items and k; nothing else may use
- * it.  Waits for the device. */
+/* Fills the two copies once, for a caller that searches one table many times: workspace holds
+ * dsx_knn_workspace_bytes_prepared(rows_padded, dim, num_queries, k) bytes (256-byte aligned).  *prepared: whether it did (the
+ * table may not be worth it, or unfit for it).  A prepared workspace goes with dsx_knn_search_host(DSX_KNN_FP32_PREPARED, ...) and searches of up to num_queries queries with the same items and
+ * k; it has to be prepared again when the items change, and nothing else may use it.  Waits for the device. */
+size_t dsx_knn_workspace_bytes_prepared(uint32_t rows_padded, uint32_t dim, uint32_t num_queries, uint32_t k);
 int dsx_knn_prepare(const float* items, uint32_t rows_padded, uint32_t padding, uint32_t dim, uint32_t num_queries, uint32_t k, void* workspace,
                     size_t workspace_bytes, int* prepared);
-int dsx_knn_search_prepared(const float* items, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,
-                            uint32_t num_queries, uint32_t k, float* scores, uint32_t* indexes, void* workspace, size_t workspace_bytes,
-                            float* elapsed_ms);
+/* dsx_knn_search, _f16 or _split (storage; items and workspace as these take them) whose last kernel writes the results into host memory
+ * too (dsx_malloc_host; both NULL: device only). */
+#define DSX_KNN_FP32 0
+#define DSX_KNN_FP16 1
+#define DSX_KNN_SPLIT 2
+#define DSX_KNN_FP32_PREPARED 3
+int dsx_knn_search_host(int storage, const void* items, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,
+                        uint32_t num_queries, uint32_t k, float* scores, uint32_t* indexes, float* host_scores, uint32_t* host_indexes,
+                        void* workspace, size_t workspace_bytes, float* elapsed_ms);
 /* fp16 storage (astdl::knn::DataType::FP16).  The reference converts the column-major table once (KnnData::load,
  * knn/KnnData.cpp:209-216, kFloatToHalf of knn/MathUtil.cu:33-81: round to nearest even) and every query batch before the
  * GEMM (knn/KnnExactGpu.cu:108-116), multiplies fp16 operands and keeps fp32 scores.  Same arithmetic here; the fp16 table's
