@@ -94,6 +94,10 @@ private:
     void* SplitInputBuffer();         // this lane's buffer for them, allocated on first use
     // Whether the deferred layer and a top-K of k entries are computed in one call (or the layer is stored first).
     bool TopKFusionPays(uint32_t batch, uint32_t k);
+    // The weights' table, where the layer and a top-K of k entries are fastest screened by it (else NULL).
+    const void* TopKScreenTable(uint32_t batch, uint32_t k);
+    // Whether the deferred layer's top-K has been computed; a narrower layer whose units are asked for all the same is stored from then on.
+    bool _bToppedDeferred = false;
     bool UseSplitProducts(uint32_t batch) const
     {
         if (!_bSplitProducts || _vIncomingLayer.empty()) return false;
@@ -107,6 +111,7 @@ private:
     bool _deferred = false;
     uint32_t _deferredBatch = 0;
     void Materialise();
+    void MaterialiseForCaller();
     bool _bHandedOut = false;     // NNNetwork::GetUnitBuffer was called for this layer: its units may change at any time
     void SettleConsumers();       // before this layer's units change: computes deferred layers that are fed by them
     void SwitchLane(uint32_t lane)

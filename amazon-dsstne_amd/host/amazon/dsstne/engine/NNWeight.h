@@ -49,7 +49,13 @@ private:
     unique_ptr<GpuBuffer<uint32_t>> _pbSplit[2];
     bool _bSplitValid[2] = {false, false};
     const void* SplitPlanes(bool bTransposed, uint32_t k, uint32_t n);
-    void InvalidateSplit() { _bSplitValid[0] = _bSplitValid[1] = false; }
+    // The table of the 16-bit screening (dsx_screen_table_build) of a matrix stored [k][n], for output layers that are computed with
+    // their top-K; kept like the planes.  NULL: there is no room for it (half of what is free), or the caller may change the matrix
+    // (_bHandedOut).
+    void* _pScreen = NULL;
+    bool _bScreenValid = false;
+    const void* ScreenTable(uint32_t k, uint32_t n);
+    void InvalidateSplit() { _bSplitValid[0] = _bSplitValid[1] = _bScreenValid = false; }
 
     NNWeight(NNLayer& inputLayer, NNLayer& outputLayer, bool bShared = false, bool bTransposed = false, bool bLocked = false,
              NNFloat maxNorm = 0.0f);

@@ -163,10 +163,23 @@ Matrix loadDataOnHost(DataReader* dataReader)
     return matrix;
 }
 
+// Result buffers: pinned host memory, which the search's last kernel writes (two copies and their waits less).
+static Matrix allocateResults(uint32_t numRows, int numColumns, size_t elementSize)
+{
+    void* data = nullptr;
+    check(dsx_malloc_host(&data, (size_t)numRows * numColumns * elementSize), "allocateResults");
+    return Matrix(data, numRows, numColumns, elementSize, MemoryType::Host);
+}
+
+static void freeResults(const Matrix& matrix)
+{
+    if (matrix.data != nullptr && dsx_is_initialized()) check(dsx_free(matrix.data), "freeResults");
+}
+
 KnnData::KnnData(int numGpus, int batchSize, int maxK, DataType dataType)
     : numGpus(numGpus), batchSize(batchSize), maxK(maxK), dCollectionPartitions(numGpus), dInputBatches(numGpus), dResultScores(numGpus),
       dResultIndexes(numGpus), hResultScores(numGpus), hResultIndexes(numGpus), hKeys(numGpus), dWorkspaces(numGpus),
-      collectionRowsPadded(numGpus), elapsedSgemm(numGpus), elapsedTopK(numGpus), dataType(dataType)
+      collectionRowsPadded(numGpus), workspacePrepared(numGpus), elapsedSgemm(numGpus), elapsedTopK(numGpus), dataType(dataType)
 {
     if (numGpus != 1) {
         std::stringstream msg;
@@ -202,8 +215,8 @@ void KnnData::load(int device, DataReader* dataReader)
     freeMatrix(dInputBatches[device]);
     freeMatrix(dResultScores[device]);
     freeMatrix(dResultIndexes[device]);
-    freeMatrix(hResultScores[device]);
-    freeMatrix(hResultIndexes[device]);
+    freeResults(hResultScores[device]);
+    freeResults(hResultIndexes[device]);
     freeMatrix(dWorkspaces[device]);
     if (dataType == DataType::FP16) {
         // knn/KnnData.cpp:209-216: the table is kept as halves (round to nearest even); the fp32 copy only lives until it is
@@ -236,11 +249,11 @@ void KnnData::load(int device, DataReader* dataReader)
     dInputBatches[device] = allocateMatrixOnDevice(batchSize, columns, sizeof(float));
     dResultScores[device] = allocateMatrixOnDevice(batchSize, maxK, sizeof(float));
     dResultIndexes[device] = allocateMatrixOnDevice(batchSize, maxK, sizeof(uint32_t));
-    hResultScores[device] = allocateMatrixOnHost(batchSize, maxK, sizeof(float));
-    hResultIndexes[device] = allocateMatrixOnHost(batchSize, maxK, sizeof(uint32_t));
+    hResultScores[device] = allocateResults(batchSize, maxK, sizeof(float));
+    hResultIndexes[device] = allocateResults(batchSize, maxK, sizeof(uint32_t));
     const size_t ws = dataType == DataType::FP16        ? dsx_knn_workspace_bytes_f16(rows, columns, batchSize, maxK)
                       : dataType == DataType::FP32Split ? dsx_knn_workspace_bytes_split(rows, columns, batchSize, maxK)
-                                                        : dsx_knn_workspace_bytes(rows, columns, batchSize, maxK);
+                                                        : dsx_knn_workspace_bytes_prepared(rows, columns, batchSize, maxK);
     // the fp32 search is faster with copies of the table (up to 8 GiB), and needs none: no more than half of what is free goes to them
     const size_t least = dataType == DataType::FP32 ? dsx_knn_workspace_bytes_least(rows, columns, batchSize, maxK) : ws;
     dsx_device_info info;
@@ -254,7 +267,12 @@ void KnnData::load(int device, DataReader* dataReader)
     }
     check(rc, "KnnData::load");
     dWorkspaces[device] = Matrix(workspace, 1, 1, wsTaken, MemoryType::Device);
-    check(dsx_get_device_info(&info), "KnnData::load");
+    int prepared = 0;
+    if (dataType == DataType::FP32 && wsTaken == ws)
+        check(dsx_knn_prepare((const float*)dCollectionPartitions[device].data, rows, rows - actualRows, (uint32_t)columns, (uint32_t)batchSize,
+                              (uint32_t)maxK, workspace, ws, &prepared),
+              "KnnData::load");
+    workspacePrepared[device] = prepared != 0;
     check(dsx_get_device_info(&info), "KnnData::load");
     fprintf(stderr, "INFO: loaded %u (%u padded) rows and %d columns into device %d. Used: %zu MB, Free: %zu MB, Total: %zu MB\n", actualRows,
             rows, columns, device, (info.hbm_bytes - info.hbm_free_bytes) >> 20, info.hbm_free_bytes >> 20, info.hbm_bytes >> 20);
@@ -292,8 +310,8 @@ KnnData::~KnnData()
     for (auto& m : dInputBatches) freeMatrix(m);
     for (auto& m : dResultScores) freeMatrix(m);
     for (auto& m : dResultIndexes) freeMatrix(m);
-    for (auto& m : hResultScores) freeMatrix(m);
-    for (auto& m : hResultIndexes) freeMatrix(m);
+    for (auto& m : hResultScores) freeResults(m);
+    for (auto& m : hResultIndexes) freeResults(m);
     for (auto& m : dWorkspaces) freeMatrix(m);
 }
 
@@ -319,33 +337,21 @@ void KnnExactGpu::searchDevice(int k, const float* inputs, int size)
     const int device = 0;
     Matrix& items = data->dCollectionPartitions[device];
     Matrix& dIn = data->dInputBatches[device];
-    float* dScores = (float*)data->dResultScores[device].data;
-    uint32_t* dIndexes = (uint32_t*)data->dResultIndexes[device].data;
-    float* hScores = (float*)data->hResultScores[device].data;
-    uint32_t* hIndexes = (uint32_t*)data->hResultIndexes[device].data;
     const int D = items.numColumns;
 
     check(dsx_memcpy_h2d(dIn.data, inputs, (size_t)size * D * sizeof(float)), "KnnExactGpu::search");
     float elapsed[2] = {0, 0};
-    if (data->dataType == DataType::FP16)
-        check(dsx_knn_search_f16(items.data, items.numRows, data->collectionRowsPadded[device], (uint32_t)D, (const float*)dIn.data,
-                                 (uint32_t)size, (uint32_t)maxK, dScores, dIndexes, data->dWorkspaces[device].data,
-                                 data->dWorkspaces[device].elementSize, elapsed),
-              "KnnExactGpu::search");
-    else if (data->dataType == DataType::FP32Split)
-        check(dsx_knn_search_split(items.data, items.numRows, data->collectionRowsPadded[device], (uint32_t)D, (const float*)dIn.data,
-                                   (uint32_t)size, (uint32_t)maxK, dScores, dIndexes, data->dWorkspaces[device].data,
-                                   data->dWorkspaces[device].elementSize, elapsed),
-              "KnnExactGpu::search");
-    else
-        check(dsx_knn_search((const float*)items.data, items.numRows, data->collectionRowsPadded[device], (uint32_t)D, (const float*)dIn.data,
-                             (uint32_t)size, (uint32_t)maxK, dScores, dIndexes, data->dWorkspaces[device].data,
-                             data->dWorkspaces[device].elementSize, elapsed),
-              "KnnExactGpu::search");
+    const int storage = data->dataType == DataType::FP16        ? DSX_KNN_FP16
+                        : data->dataType == DataType::FP32Split ? DSX_KNN_SPLIT
+                        : data->workspacePrepared[device]       ? DSX_KNN_FP32_PREPARED
+                                                                : DSX_KNN_FP32;
+    check(dsx_knn_search_host(storage, items.data, items.numRows, data->collectionRowsPadded[device], (uint32_t)D, (const float*)dIn.data,
+                              (uint32_t)size, (uint32_t)maxK, (float*)data->dResultScores[device].data, (uint32_t*)data->dResultIndexes[device].data,
+                              (float*)data->hResultScores[device].data, (uint32_t*)data->hResultIndexes[device].data,
+                              data->dWorkspaces[device].data, data->dWorkspaces[device].elementSize, elapsed),
+          "KnnExactGpu::search");
     data->elapsedSgemm[device] = elapsed[0];
     data->elapsedTopK[device] = elapsed[1];
-    check(dsx_memcpy_d2h(hScores, dScores, (size_t)size * maxK * sizeof(float)), "KnnExactGpu::search");
-    check(dsx_memcpy_d2h(hIndexes, dIndexes, (size_t)size * maxK * sizeof(uint32_t)), "KnnExactGpu::search");
 }
 
 void KnnExactGpu::search(int k, const float* inputs, int size, std::string* keys, float* scores)

@@ -141,8 +141,18 @@ static const uint32_t kSegMaxMinWidth = 8192;
 // 16 GB of stores and loads go away.
 static const uint32_t kDeferMinWidth = 131072;
 
+const void* NNLayer::TopKScreenTable(uint32_t batch, uint32_t k)
+{
+    NNLayer* src = _vIncomingLayer[0];
+    NNWeight* w = _vIncomingWeight[0];
+    NNWeight* wsrc = w->_bShared ? w->_pSharedWeight : w;
+    if (w->_bTransposed || UseSplitProducts(batch) || !dsx_fc_topk_screened_pays(batch, src->_stride, _localStride, (uint32_t)_activation, k)) return NULL;
+    return wsrc->ScreenTable(src->_stride, _localStride);
+}
+
 bool NNLayer::TopKFusionPays(uint32_t batch, uint32_t k)
 {
+    if (TopKScreenTable(batch, k)) return true;
     if (_localStride < kDeferMinWidth && UseSplitProducts(batch)) return false;
     return dsx_fc_topk_pays(batch, _vIncomingLayer[0]->_stride, _localStride, (uint32_t)_activation, k) != 0;
 }
@@ -185,6 +195,7 @@ void NNLayer::ForwardPropagateFullyConnected(uint32_t position, uint32_t batch, 
                     _bDeferOutput = false;
                 } else {
                     _deferred = true;
+                    _bToppedDeferred = false;
                     _deferredBatch = batch;
                     return;
                 }
@@ -262,6 +273,13 @@ void NNLayer::Materialise()
              "NNLayer::ForwardPropagate: GEMM failure");
 }
 
+// Units that are asked for although their top-K has been computed: a narrower layer is better stored in the first place then.
+void NNLayer::MaterialiseForCaller()
+{
+    if (_bToppedDeferred && _localStride < kDeferMinWidth) _bDeferOutput = false;
+    Materialise();
+}
+
 void NNLayer::SettleConsumers()
 {
     for (auto l : _vOutgoingLayer)
@@ -323,7 +341,7 @@ bool NNLayer::GetUnits(vector<NNFloat>& vUnit)
         printf("NNLayer::GetUnits: Unit data not yet allocated.\n");
         return false;
     }
-    if (_deferred) Materialise();
+    if (_deferred) MaterialiseForCaller();
     // the whole [batch][stride] buffer comes back (the reference sizes the vector to one row only and then overruns it)
     if (vUnit.size() < _pbUnit->_length) vUnit.resize(_pbUnit->_length);
     _pbUnit->Download(vUnit.data());
@@ -340,7 +358,7 @@ bool NNLayer::GetUnits(NNFloat* pUnit)
         printf("NNLayer::GetUnits: Download pointer invalid.\n");
         return false;
     }
-    if (_deferred) Materialise();
+    if (_deferred) MaterialiseForCaller();
     _pbUnit->Download(pUnit);
     return true;
 }

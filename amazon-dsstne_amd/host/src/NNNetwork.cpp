@@ -328,6 +328,14 @@ void NNNetwork::LayerWithTopK(NNLayer* pLayer, uint32_t k, uint32_t batch, const
                  "NNNetwork::CalculateTopK: output layer with top-K");
         return;
     }
+    pLayer->_bToppedDeferred = true;
+    if (const void* pTable = pLayer->TopKScreenTable(batch, k)) {
+        dsxFatal(dsx_fc_topk_screened(src->GetUnitBuffer(), src->_stride, wsrc->_pbWeight->_pDevData, pTable, w->_pbBias->_pDevData, batch,
+                                      src->_stride, pLayer->_localStride, (uint32_t)pLayer->_activation, &params, k, pKey, pValue, _position,
+                                      pIndex, pFilterStart, pFilterEnd, pFilterIndex),
+                 "NNNetwork::CalculateTopK: output layer with top-K");
+        return;
+    }
     dsxFatal(dsx_fc_topk(src->GetUnitBuffer(), src->_stride, wsrc->_pbWeight->_pDevData, w->_pbBias->_pDevData, batch, src->_stride,
                          pLayer->_localStride, (uint32_t)pLayer->_activation, &params, k, pKey, pValue, _position, pIndex, pFilterStart,
                          pFilterEnd, pFilterIndex),
@@ -541,7 +549,7 @@ NNFloat* NNNetwork::GetUnitBuffer(const string& layer)
         printf("NNNetwork::GetUnitBuffer: Unknown layer %s.\n", layer.c_str());
         return NULL;
     }
-    if (itr->second->_deferred) itr->second->Materialise();
+    if (itr->second->_deferred) itr->second->MaterialiseForCaller();
     itr->second->SettleConsumers();
     itr->second->_bHandedOut = true;
     // the caller gets a writable device pointer: the segment maxima of the batch may not describe the units any longer

@@ -44,7 +44,10 @@ NNWeight::NNWeight(NNLayer& inputLayer, NNLayer& outputLayer, bool bShared, bool
     _pbBias.reset(new GpuBuffer<NNFloat>(_localBiasSize));
 }
 
-NNWeight::~NNWeight() {}
+NNWeight::~NNWeight()
+{
+    if (_pScreen && dsx_is_initialized()) dsx_free(_pScreen);
+}
 
 namespace {
 // Counter-based stream: value i of a connection depends only on the process seed, the two layer names and i, so a
@@ -196,6 +199,26 @@ const void* NNWeight::SplitPlanes(bool bTransposed, uint32_t k, uint32_t n)
         _bSplitValid[o] = true;
     }
     return _pbSplit[o]->_pDevData;
+}
+
+const void* NNWeight::ScreenTable(uint32_t k, uint32_t n)
+{
+    if (_bHandedOut) return NULL;
+    if (!_bScreenValid) {
+        if (!_pScreen) {
+            const uint64_t bytes = dsx_screen_table_bytes(n, k);
+            dsx_device_info info;
+            dsxFatal(dsx_get_device_info(&info), "NNWeight::ScreenTable");
+            if (bytes > info.hbm_free_bytes / 2 || dsx_malloc(&_pScreen, bytes) != DSX_OK) {
+                _pScreen = NULL;
+                return NULL;
+            }
+        }
+        dsxFatal(dsx_screen_table_build(_pbWeight->_pDevData, n, n, k, _pScreen), "NNWeight::ScreenTable");
+        dsxFatal(dsx_sync(), "NNWeight::ScreenTable");
+        _bScreenValid = true;
+    }
+    return _pScreen;
 }
 
 bool NNWeight::SetBiases(const vector<NNFloat>& vBias)
