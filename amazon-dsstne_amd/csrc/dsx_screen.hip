@@ -142,25 +142,47 @@ struct ScreenRowsArgs {
     ScreenNotes* notes;     // host-visible: what the table's columns and the rows are like (nearest neighbours)
 };
 
-// One wavefront per row.
+// One wavefront per row, which holds up to 1,024 components of it between the two passes.  Bound by latency, one round trip so (256 x 1,024:
+// 9.7 us when a lane read its components one by one, twice; 4.5 so; 4,096 x 1,024 28 / 14 beside other kernels).  X is 16-byte aligned and its pitch a multiple of 4.
 __global__ __launch_bounds__(256) void screen_rows_kernel(ScreenRowsArgs a)
 {
     const uint32_t row = blockIdx.x * 4 + threadIdx.x / kWave, lane = threadIdx.x % kWave;
     const bool valid = row < a.batch;
-    float sum = 0.0f;
-    if (valid)
-        for (uint32_t d = lane; d < a.dim; d += kWave) {
-            const float x = a.X[(uint64_t)row * a.ldx + d];
-            sum += x * x;
+    const float* x = a.X + (uint64_t)row * a.ldx;
+    auto part = [&](uint32_t d) __attribute__((always_inline)) -> float4 {
+        float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (valid && d < a.dim) {
+            v = *reinterpret_cast<const float4*>(x + d);
+            if (d + 1 >= a.dim) v.y = 0.0f;
+            if (d + 2 >= a.dim) v.z = 0.0f;
+            if (d + 3 >= a.dim) v.w = 0.0f;
         }
+        return v;
+    };
+    constexpr int G = 4;
+    float4 held[G];
+#pragma unroll
+    for (int g = 0; g < G; g++) held[g] = part(g * 4 * kWave + 4 * lane);
+    float sum = 0.0f;
+    auto add = [&](const float4& v) __attribute__((always_inline)) { sum += (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w); };
+#pragma unroll
+    for (int g = 0; g < G; g++) add(held[g]);
+#pragma unroll 4
+    for (uint32_t d = G * 4 * kWave + 4 * lane; d < a.dim; d += 4 * kWave) add(part(d));
 #pragma unroll
     for (int d = 1; d < kWave; d *= 2) sum += __shfl_xor(sum, d);
     const float norm = sqrtf(sum);
     const bool bad = norm > kF16Max;   // (a NaN in the row: its scores are NaN everywhere, there is nothing to miss)
-    for (uint32_t d = lane; d < a.ld; d += kWave) {
-        const float x = (valid && !bad && d < a.dim) ? a.X[(uint64_t)row * a.ldx + d] : 0.0f;
-        a.out16[(uint64_t)row * a.ld + d] = (_Float16)x;
-    }
+    auto put = [&](uint32_t d, const float4& v) __attribute__((always_inline)) {
+        typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+        half4 h = {};
+        if (!bad) h = half4{(_Float16)v.x, (_Float16)v.y, (_Float16)v.z, (_Float16)v.w};
+        if (d < a.ld) *reinterpret_cast<half4*>(a.out16 + (uint64_t)row * a.ld + d) = h;
+    };
+#pragma unroll
+    for (int g = 0; g < G; g++) put(g * 4 * kWave + 4 * lane, held[g]);
+#pragma unroll 4
+    for (uint32_t d = G * 4 * kWave + 4 * lane; d < a.ld; d += 4 * kWave) put(d, part(d));
     if (blockIdx.x == 0)
         for (uint32_t i = threadIdx.x; i < a.clear_words; i += 256) a.clear[i] = 0;
     if (!valid || lane != 0) return;
@@ -945,10 +967,13 @@ static int launch_pick(const ScreenFoldArgs& a, bool keep)
 {
     const size_t bitmap = a.fidx ? ((size_t)a.stored + 31) / 32 * 4 : 0, row = keep ? 0 : (size_t)(a.dim + 63) / 64 * 256;
     const size_t lds = std::max<size_t>(16, std::max(bitmap, row));
-    // (maxima: a lane's only one for small k, four where more than one of the k best are likely to share a lane)
+    // Maxima: a lane's only one for small k, four where more than one of the k best are likely to share a lane.  Sixteen wavefronts a row
+    // where there is a compute unit for each: with four, what is in flight of the candidates' rows does not cover the latency
+    // (256 x 1,024 x 27,278 top 100: 47.7 us / 31.1); with more rows than that four of them pass through at a time (512 x 128 x 27,278 top 10, four
+    // batches: 153 us / 214 with sixteen).
     const bool one = a.k <= 32;
     if (keep) return one ? launch_pick_as<256, 1, 4, kPickKeep>(a, lds) : launch_pick_as<256, 4, 4, kPickKeep>(a, lds);
-    if (a.batch > 64 && a.stored <= 32768) return one ? launch_pick_as<256, 1, 4, kPickFinal>(a, lds) : launch_pick_as<256, 4, 4, kPickFinal>(a, lds);
+    if (a.batch > (uint32_t)ctx().num_cus && a.stored <= 32768) return one ? launch_pick_as<256, 1, 4, kPickFinal>(a, lds) : launch_pick_as<256, 4, 4, kPickFinal>(a, lds);
     if (a.batch > 512) return one ? launch_pick_as<256, 1, 16, kPickFinal>(a, lds) : launch_pick_as<256, 4, 16, kPickFinal>(a, lds);
     if (a.stored <= 131072) return launch_pick_as<1024, 1, 4, kPickFinal>(a, lds);
     return launch_pick_as<1024, 1, 32, kPickFinal>(a, lds);
