@@ -206,6 +206,8 @@ int knn_refresh(uint64_t* best, const uint64_t* cand, uint32_t* cand_count, uint
 // fp16 storage, candidate mode of a column range: one workgroup per tile, or (long ranges) workgroups that sweep a chunk of the
 // range each and keep lists of their own (seg [queries][lists][seg_words / lists], seg_count [queries][kF16ListStride]); full
 // lists spill into cand's shared ones.  mode: see dsx_testing_set_knn_f16_sweep.  *lists_used is what knn_refresh needs to know.
+int knn_f16_wide_run(const void* queries16, const void* items16, uint32_t ld, uint32_t batch, uint32_t n, const CandArgs& cand, uint64_t* seg,
+                     uint32_t* seg_count, uint32_t seg_words, bool every, uint32_t* lists_used);
 int knn_f16_candidates_run(const void* queries16, const void* items16, uint32_t ld, uint32_t batch, uint32_t n, const CandArgs& cand,
                            uint64_t* seg, uint32_t* seg_count, uint32_t seg_words, int mode, uint32_t* lists_used);
 

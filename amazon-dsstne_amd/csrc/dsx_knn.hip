@@ -341,7 +341,7 @@ static int knn_search_candidates(const KnnWorkspace& w, const KnnOperands& op, u
 // looked at.  *overflowed tells the caller to redo the search without screening; *unfit, that the table or the queries were found unfit
 // for it first (norms beyond f16's range, or one so large that the others' bounds would be worth little).
 static int knn_search_screened(const KnnWorkspace& w, const KnnOperands& op, uint32_t M, uint32_t num_queries, uint32_t k, const KnnResults& out,
-                               KnnTimer& t, bool built, bool* overflowed, bool* unfit)
+                               KnnTimer& t, bool built, bool even, bool* overflowed, bool* unfit)
 {
     hipStream_t s = ctx().stream;
     int rc = knn_notes_ready();
@@ -349,6 +349,7 @@ static int knn_search_screened(const KnnWorkspace& w, const KnnOperands& op, uin
     ScreenJob j{};
     j.X = op.queries; j.ldx = op.dim; j.batch = num_queries; j.dim = op.dim; j.n = M; j.k = k;
     j.act = DSX_ACT_LINEAR;
+    j.even = even;
     j.keys = out.scores; j.values = out.indexes; j.keys2 = out.host_scores; j.values2 = out.host_indexes;
     j.row_flag = w.row_flag; j.told = &g_knn_notes->flag;
     j.cand = w.cand; j.cand_count = w.cand_count; j.cap = kCandCap; j.overflow = w.overflow;
@@ -366,6 +367,7 @@ static int knn_search_screened(const KnnWorkspace& w, const KnnOperands& op, uin
         DSX_HIP(noted);
         *unfit = knn_unfit(*g_knn_notes, num_queries, op.dim, M, k);
         if (*unfit) return DSX_OK;
+        j.even = g_knn_notes->number != 0 && screen_even(g_knn_notes->largest, g_knn_notes->sum / (float)g_knn_notes->number);
     }
     if ((rc = screen_run(j, w.table, w.screen))) return rc;
     t.stop(s, t.gemm);
@@ -453,7 +455,7 @@ int dsx_knn_f16_convert_items(const float* items, uint32_t rows_padded, uint32_t
 
 // Both precisions: workspace, the two paths, timing.
 static int knn_search_common(KnnOperands& op, uint32_t padding, uint32_t num_queries, uint32_t k, const KnnResults& out, void* workspace,
-                             size_t workspace_bytes, float* elapsed_ms, bool aligned, const float* queries_f32, bool built = false)
+                             size_t workspace_bytes, float* elapsed_ms, bool aligned, const float* queries_f32, bool built = false, bool even = false)
 {
     const size_t full = knn_layout(nullptr, op.rows_padded, num_queries, k, op.f16, op.dim, op.split, true, built).bytes;
     const size_t need = knn_layout(nullptr, op.rows_padded, num_queries, k, op.f16, op.dim, op.split, false, built).bytes;
@@ -500,7 +502,7 @@ static int knn_search_common(KnnOperands& op, uint32_t padding, uint32_t num_que
     const bool many = M > knn_block_columns(op.rows_padded, num_queries);
     bool screened = may && w.screen.bytes != 0 && !ctx().knobs.knn_block_columns;
     bool redo = true, unfit = false;
-    if (rc == DSX_OK && screened) rc = knn_search_screened(w, op, M, num_queries, k, out, t, built, &redo, &unfit);
+    if (rc == DSX_OK && screened) rc = knn_search_screened(w, op, M, num_queries, k, out, t, built, even, &redo, &unfit);
     if (unfit) screened = false;
     const bool candidates = may && (screened || many);
     if (rc == DSX_OK && candidates && (!screened || redo) && many)
@@ -518,7 +520,7 @@ static int knn_search_common(KnnOperands& op, uint32_t padding, uint32_t num_que
 }
 
 static int knn_search_fp32(const float* items, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,
-                           uint32_t num_queries, uint32_t k, const KnnResults& out, void* workspace, size_t workspace_bytes, float* elapsed_ms, bool built)
+                           uint32_t num_queries, uint32_t k, const KnnResults& out, void* workspace, size_t workspace_bytes, float* elapsed_ms, bool built, bool even)
 {
     DSX_REQUIRE_INIT();
     DSX_CHECK_ARG(items && queries && out.scores && out.indexes, "dsx_knn_search: null device pointer");
@@ -532,7 +534,7 @@ static int knn_search_fp32(const float* items, uint32_t rows_padded, uint32_t pa
     op.rows_padded = rows_padded;
     op.dim = dim;
     const bool aligned = ((uintptr_t)items % 16) == 0 && ((uintptr_t)queries % 16) == 0 && (rows_padded % 4) == 0 && (dim % 4) == 0;
-    return knn_search_common(op, padding, num_queries, k, out, workspace, workspace_bytes, elapsed_ms, aligned, nullptr, built);
+    return knn_search_common(op, padding, num_queries, k, out, workspace, workspace_bytes, elapsed_ms, aligned, nullptr, built, even);
 }
 
 static int knn_search_split(const void* item_planes, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,
@@ -580,7 +582,7 @@ int dsx_knn_search(const float* items, uint32_t rows_padded, uint32_t padding, u
                    float* elapsed_ms)
 {
     return knn_search_fp32(items, rows_padded, padding, dim, queries, num_queries, k, KnnResults{scores, indexes, nullptr, nullptr}, workspace,
-                           workspace_bytes, elapsed_ms, false);
+                           workspace_bytes, elapsed_ms, false, false);
 }
 
 int dsx_knn_search_split(const void* item_planes, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,
@@ -623,7 +625,7 @@ int dsx_knn_prepare(const float* items, uint32_t rows_padded, uint32_t padding, 
     // as where a search makes its own copies: no norm beyond f16's range, and none so far above the others that its share of the error
     // (of the columns next to it, which are judged by the largest of 32 or 64) would let everything pass
     const float average = notes.number != 0 ? notes.sum / (float)notes.number : 0.0f;
-    *prepared = notes.largest <= 65504.0f && notes.largest <= 64.0f * average;
+    if (notes.largest <= 65504.0f && notes.largest <= 64.0f * average) *prepared = screen_even(notes.largest, average) ? DSX_KNN_FP32_PREPARED_EVEN : DSX_KNN_FP32_PREPARED;
     return DSX_OK;
 }
 
@@ -632,13 +634,15 @@ int dsx_knn_search_host(int storage, const void* items, uint32_t rows_padded, ui
                         void* workspace, size_t workspace_bytes, float* elapsed_ms)
 {
     DSX_CHECK_ARG((host_scores == nullptr) == (host_indexes == nullptr), "dsx_knn_search_host: host_scores and host_indexes go together");
-    DSX_CHECK_ARG(storage != DSX_KNN_FP32_PREPARED || workspace, "dsx_knn_search_host: no prepared workspace");
+    const bool built = storage == DSX_KNN_FP32_PREPARED || storage == DSX_KNN_FP32_PREPARED_EVEN;
+    DSX_CHECK_ARG(!built || workspace, "dsx_knn_search_host: no prepared workspace");
     const KnnResults out{scores, indexes, host_scores, host_indexes};
     switch (storage) {
     case DSX_KNN_FP32:
     case DSX_KNN_FP32_PREPARED:
+    case DSX_KNN_FP32_PREPARED_EVEN:
         return knn_search_fp32((const float*)items, rows_padded, padding, dim, queries, num_queries, k, out, workspace, workspace_bytes, elapsed_ms,
-                               storage == DSX_KNN_FP32_PREPARED);
+                               built, storage == DSX_KNN_FP32_PREPARED_EVEN);
     case DSX_KNN_FP16: return knn_search_f16(items, rows_padded, padding, dim, queries, num_queries, k, out, workspace, workspace_bytes, elapsed_ms);
     case DSX_KNN_SPLIT: return knn_search_split(items, rows_padded, padding, dim, queries, num_queries, k, out, workspace, workspace_bytes, elapsed_ms);
     default: return set_error(DSX_EINVAL, "dsx_knn_search_host: storage %d", storage);

@@ -427,6 +427,42 @@ int knn_f16_scores_run(const void* queries16, const void* items16, uint32_t ld, 
     return DSX_OK;
 }
 
+// knn_f16_wide_kernel over a range, where it has workgroups for (half of) the CUs and enough items per chunk (every: wherever every chunk
+// gets a stage).  *lists_used: a row's lists, 0 where nothing was started.
+int knn_f16_wide_run(const void* queries16, const void* items16, uint32_t ld, uint32_t batch, uint32_t n, const CandArgs& cand, uint64_t* seg,
+                     uint32_t* seg_count, uint32_t seg_words, bool every, uint32_t* lists_used)
+{
+    *lists_used = 0;
+    if (ld > 256) return DSX_OK;
+    // queries in registers: 512 per workgroup, stages of 64 items, one workgroup per CU
+    const uint32_t cus = (uint32_t)ctx().num_cus, tiles_q = (batch + 511) / 512, stages = (n + kWideStageItems - 1) / kWideStageItems;
+    const uint32_t chunks = std::min<uint32_t>(kF16ListStride / 2, (cus + tiles_q - 1) / tiles_q);   // two lists per (query, chunk)
+    if (every ? stages < chunks : (2 * tiles_q * chunks < cus || stages < 8 * chunks)) return DSX_OK;
+    KnnF16SweepArgs a{};
+    a.A = (const _Float16*)queries16;
+    a.B = (const _Float16*)items16;
+    a.ld = ld;
+    a.batch = batch;
+    a.n = n;
+    a.seg = seg;
+    a.seg_count = seg_count;
+    a.cand = cand;
+    a.tiles_m = tiles_q;
+    a.tiles_n = stages;
+    a.chunks = chunks;
+    a.tiles_per_chunk = (stages + chunks - 1) / chunks;
+    a.seg_cap = seg_words / (2 * chunks);
+    const uint32_t total = tiles_q * chunks;
+    const uint32_t grid = ((total + kF16Xcds - 1) / kF16Xcds) * kF16Xcds;
+    *lists_used = 2 * chunks;
+    switch (ld) {
+    case 64: return launch_wide<4>(a, grid);
+    case 128: return launch_wide<8>(a, grid);
+    case 192: return launch_wide<12>(a, grid);
+    default: return launch_wide<16>(a, grid);
+    }
+}
+
 // Candidate mode of a column range of n items for `batch` queries.  mode 0: one workgroup per tile (knn_f16_kernel); 1: a
 // sweep when it has workgroups for (half of) the CUs and enough items per chunk — knn_f16_wide_kernel for vectors of at most 256
 // components, f16_sweep_kernel (dsx_f16.hip) otherwise; 2: f16_sweep_kernel whenever every chunk gets a tile, 3: knn_f16_wide_kernel
@@ -437,35 +473,9 @@ int knn_f16_candidates_run(const void* queries16, const void* items16, uint32_t 
 {
     *lists_used = 0;
     const uint32_t cus = (uint32_t)ctx().num_cus;
-    KnnF16SweepArgs a{};
-    a.A = (const _Float16*)queries16;
-    a.B = (const _Float16*)items16;
-    a.ld = ld;
-    a.batch = batch;
-    a.n = n;
-    a.seg = seg;
-    a.seg_count = seg_count;
-    a.cand = cand;
-    if (seg && seg_count && ld <= 256 && (mode == 1 || mode == 3)) {
-        // queries in registers: 512 per workgroup, stages of 64 items, one workgroup per CU
-        const uint32_t tiles_q = (batch + 511) / 512, stages = (n + kWideStageItems - 1) / kWideStageItems;
-        const uint32_t chunks = std::min<uint32_t>(kF16ListStride / 2, (cus + tiles_q - 1) / tiles_q);   // two lists per (query, chunk)
-        if (mode == 3 ? stages >= chunks : (2 * tiles_q * chunks >= cus && stages >= 8 * chunks)) {
-            a.tiles_m = tiles_q;
-            a.tiles_n = stages;
-            a.chunks = chunks;
-            a.tiles_per_chunk = (stages + chunks - 1) / chunks;
-            a.seg_cap = seg_words / (2 * chunks);
-            const uint32_t total = tiles_q * chunks;
-            const uint32_t grid = ((total + kF16Xcds - 1) / kF16Xcds) * kF16Xcds;
-            *lists_used = 2 * chunks;
-            switch (ld) {
-            case 64: return launch_wide<4>(a, grid);
-            case 128: return launch_wide<8>(a, grid);
-            case 192: return launch_wide<12>(a, grid);
-            default: return launch_wide<16>(a, grid);
-            }
-        }
+    if (seg && seg_count && (mode == 1 || mode == 3)) {
+        const int rc = knn_f16_wide_run(queries16, items16, ld, batch, n, cand, seg, seg_count, seg_words, mode == 3, lists_used);
+        if (rc || *lists_used) return rc;
     }
     const uint32_t tiles_q = (batch + 255) / 256, tiles_i = (n + 255) / 256, chunks = std::min<uint32_t>(kF16ListStride / 2, (cus + tiles_q - 1) / tiles_q);
     const bool sweep = seg && seg_count && (mode == 2 || mode == 3 ? tiles_i >= chunks : (mode == 1 && 2 * tiles_q * chunks >= cus && tiles_i >= 2 * chunks));

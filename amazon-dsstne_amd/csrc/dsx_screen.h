@@ -88,10 +88,15 @@ struct ScreenJob {
     uint32_t* overflow;       // scratch word
     uint32_t* clear;          // [clear_words] set to 0 on the way
     uint32_t clear_words;
+    bool even;                // no bias, no column that always passes, and norms close together (screen_even)
 };
 // The rows in f16 (and notes of the table and the rows, NULL: none), then the search itself.
 int screen_rows(const ScreenJob& j, const ScreenTable& t, const ScreenWorkspace& w, ScreenNotes* notes);
 int screen_run(const ScreenJob& j, const ScreenTable& t, const ScreenWorkspace& w);
+
+// Whether the bounds may be lowered by the error that the largest norm has, instead of raising every sum by its own: what passes beyond that
+// is a factor of exp(4 * 2^-10 sqrt(dim) (largest / average - 1)) at most, 1.07 for 256 components.
+inline bool screen_even(float largest, float average) { return largest < 60000.0f && largest <= 2.0f * average; }
 
 bool screen_takes(uint32_t batch, uint32_t dim, uint64_t n, bool layer);
 bool screen_layer_pays(uint32_t batch, uint32_t dim, uint64_t n, uint32_t k);

@@ -216,6 +216,7 @@ struct ScreenFoldArgs {
     float width_z;           // and per unit of |z|
     const float* norm;       // by column
     const float* seg_norm;
+    const float* largest;    // norm whose error the ranges' bounds are lowered by (NULL: the sums are raised)
     uint32_t act;
     float slope, alpha, lambda;
     uint32_t* row_flag;
@@ -430,6 +431,14 @@ template <int N> __device__ __forceinline__ uint32_t screen_wave_kth(const uint3
 
 enum { kPickFinal, kPickKeep };
 
+// What a range's sums are compared with.
+__device__ __forceinline__ uint32_t screen_admit(const ScreenFoldArgs& a, float cut, float e1)
+{
+    if (!a.largest) return score_key(cut);
+    const float lowered = fmaf(-e1, *a.largest, cut);
+    return score_key(lowered - (fabsf(lowered) + fabsf(cut)) * 2.4e-7f);   // (below what the roundings of the raised sum reach)
+}
+
 // Sums stored as halves: what reaches the bound.  The maxima of the row's blocks of 32 columns say which blocks can hold a result: the k-th
 // of R maxima per lane (over blocks without a listed column, each less its width) bounds the k-th score, and only blocks whose largest
 // sum reaches the bound are read.  Bound by latency: two round trips, a key search and, in the form that ends with the results, one
@@ -597,7 +606,7 @@ __global__ __launch_bounds__(T, T == 256 ? 5 : 4) void screen_pick_kernel(Screen
         for (uint32_t i = threadIdx.x; i < count; i += T) a.keep[(uint64_t)b * kKeepWords + i] = screen_raised(a, sList[i], e1);
         if (threadIdx.x == 0) {
             a.keep_count[b] = count;
-            a.admit[b] = score_key(cut);
+            a.admit[b] = screen_admit(a, cut, e1);
         }
     } else {
         // With many candidates of long rows, the k-th of the candidates' own bounds (by column and not by block) first: a third of them go.
@@ -798,7 +807,7 @@ __global__ __launch_bounds__(256, 4) void screen_fold_kernel(ScreenFoldArgs a)
         for (uint32_t i = threadIdx.x; i < count; i += 256) a.keep[(uint64_t)b * kKeepWords + i] = left[i];
         if (threadIdx.x == 0) {
             a.keep_count[b] = count;
-            a.admit[b] = score_key(sCut);
+            a.admit[b] = screen_admit(a, sCut, e1);
         }
     }
 }
@@ -996,6 +1005,7 @@ int screen_run(const ScreenJob& j, const ScreenTable& t, const ScreenWorkspace& 
     a.e1 = w.e1; a.e0 = w.e0;
     a.width_bias = 2.3f * screen_bias_raise(j.dim) / (screen_relative(j.dim) + screen_bias_raise(j.dim));
     a.norm = t.norm; a.seg_norm = t.seg_norm;
+    a.largest = j.even ? reinterpret_cast<const float*>(t.stats) : nullptr;
     a.act = j.act; a.slope = j.slope; a.alpha = j.alpha; a.lambda = j.lambda;
     a.row_flag = j.row_flag; a.told = j.told;
     a.position = j.position; a.index = j.index; a.fstart = j.fstart; a.fend = j.fend; a.fidx = j.fidx;
@@ -1020,7 +1030,11 @@ int screen_run(const ScreenJob& j, const ScreenTable& t, const ScreenWorkspace& 
         f.n = ncols;
         f.cand = CandArgs{w.admit, j.cand, j.cand_count, j.cap, done, j.overflow};
         f.seg = w.seg; f.seg_count = w.seg_count; f.seg_words = kListWords;
-        if ((rc = f16_sweep_run(f, true, &a.lists))) return rc;
+        // Vectors that fit a wavefront's registers go through the kernel that keeps the queries there, which raises no sums (1,000,000 x
+        // 128 x 4,096 queries, top 100: 1,461 us in three ranges, 1,361 so).
+        a.lists = 0;
+        if (j.even && (rc = knn_f16_wide_run(f.Q, f.items, ld, j.batch, ncols, f.cand, f.seg, f.seg_count, f.seg_words, false, &a.lists))) return rc;
+        if (!a.lists && (rc = f16_sweep_run(f, true, &a.lists))) return rc;
         a.seg_cap = kListWords / a.lists;
         done += ncols;
         // (the sums of the first block, rounded up to halves, are among what is kept: their width is the others' from here on)

@@ -52,9 +52,9 @@ struct KnnData {
     std::vector<std::vector<std::string>> hKeys;
     std::vector<Matrix> dWorkspaces;             // score blocks + partial lists of the search (instead of a full product matrix)
     std::vector<uint32_t> collectionRowsPadded;  // pad rows per device (rows are padded to a multiple of 8)
-    // FP32: the workspace holds copies of the table that load made (dsx_knn_prepare); a program that writes to dCollectionPartitions
+    // FP32: not 0 if the workspace holds copies of the table that load made (dsx_knn_prepare: with which storage); a program that writes to dCollectionPartitions
     // itself sets this to 0, and searches make their own
-    std::vector<char> workspacePrepared;
+    std::vector<int> workspacePrepared;
     std::vector<float> elapsedSgemm;             // milliseconds of the last search, per device
     std::vector<float> elapsedTopK;
     const DataType dataType;

@@ -272,7 +272,7 @@ void KnnData::load(int device, DataReader* dataReader)
         check(dsx_knn_prepare((const float*)dCollectionPartitions[device].data, rows, rows - actualRows, (uint32_t)columns, (uint32_t)batchSize,
                               (uint32_t)maxK, workspace, ws, &prepared),
               "KnnData::load");
-    workspacePrepared[device] = prepared != 0;
+    workspacePrepared[device] = prepared;
     check(dsx_get_device_info(&info), "KnnData::load");
     fprintf(stderr, "INFO: loaded %u (%u padded) rows and %d columns into device %d. Used: %zu MB, Free: %zu MB, Total: %zu MB\n", actualRows,
             rows, columns, device, (info.hbm_bytes - info.hbm_free_bytes) >> 20, info.hbm_free_bytes >> 20, info.hbm_bytes >> 20);
@@ -343,7 +343,7 @@ void KnnExactGpu::searchDevice(int k, const float* inputs, int size)
     float elapsed[2] = {0, 0};
     const int storage = data->dataType == DataType::FP16        ? DSX_KNN_FP16
                         : data->dataType == DataType::FP32Split ? DSX_KNN_SPLIT
-                        : data->workspacePrepared[device]       ? DSX_KNN_FP32_PREPARED
+                        : data->workspacePrepared[device]       ? data->workspacePrepared[device]
                                                                 : DSX_KNN_FP32;
     check(dsx_knn_search_host(storage, items.data, items.numRows, data->collectionRowsPadded[device], (uint32_t)D, (const float*)dIn.data,
                               (uint32_t)size, (uint32_t)maxK, (float*)data->dResultScores[device].data, (uint32_t*)data->dResultIndexes[device].data,

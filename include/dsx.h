@@ -360,9 +360,9 @@ size_t dsx_knn_workspace_bytes(uint32_t rows_padded, uint32_t dim, uint32_t num_
  * faster (its candidates are screened in 16 bits); a workspace of at least this size but not that one is searched without them. */
 size_t dsx_knn_workspace_bytes_least(uint32_t rows_padded, uint32_t dim, uint32_t num_queries, uint32_t k);
 /* Fills the two copies once, for a caller that searches one table many times: workspace holds
- * dsx_knn_workspace_bytes_prepared(rows_padded, dim, num_queries, k) bytes (256-byte aligned).  *prepared: whether it did (the
- * table may not be worth it, or unfit for it).  A prepared workspace goes with dsx_knn_search_host(DSX_KNN_FP32_PREPARED, ...) and searches of up to num_queries queries with the same items and
- * k; it has to be prepared again when the items change, and nothing else may use it.  Waits for the device. */
+ * dsx_knn_workspace_bytes_prepared(rows_padded, dim, num_queries, k) bytes (256-byte aligned).  *prepared: 0 (the table is
+ * not worth it, or unfit for it) or the storage, DSX_KNN_FP32_PREPARED or _EVEN, with which dsx_knn_search_host takes the workspace, in
+ * searches of up to num_queries queries with the same items and k; it has to be prepared again when the items change, and nothing else may use it.  Waits for the device. */
 size_t dsx_knn_workspace_bytes_prepared(uint32_t rows_padded, uint32_t dim, uint32_t num_queries, uint32_t k);
 int dsx_knn_prepare(const float* items, uint32_t rows_padded, uint32_t padding, uint32_t dim, uint32_t num_queries, uint32_t k, void* workspace,
                     size_t workspace_bytes, int* prepared);
@@ -372,6 +372,7 @@ int dsx_knn_prepare(const float* items, uint32_t rows_padded, uint32_t padding, 
 #define DSX_KNN_FP16 1
 #define DSX_KNN_SPLIT 2
 #define DSX_KNN_FP32_PREPARED 3
+#define DSX_KNN_FP32_PREPARED_EVEN 4   /* the items' norms lie close together */
 int dsx_knn_search_host(int storage, const void* items, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,
                         uint32_t num_queries, uint32_t k, float* scores, uint32_t* indexes, float* host_scores, uint32_t* host_indexes,
                         void* workspace, size_t workspace_bytes, float* elapsed_ms);

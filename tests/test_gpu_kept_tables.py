@@ -68,7 +68,7 @@ def test_prepared_search(pkg, dsx, rng, n, dim, most, k):
     room = pkg.DeviceArray((dsx.dsx_knn_workspace_bytes_prepared(rows, dim, most, k),), np.uint8)
     prepared = C.c_int(-1)
     pkg.check(dsx.dsx_knn_prepare(dI.ptr, rows, rows - n, dim, most, k, room.ptr, room.nbytes, C.byref(prepared)))
-    assert prepared.value == 1
+    assert prepared.value == 4
     rs, ri = best(q @ items.T, k)
     scores, idx = pkg.DeviceArray((most, k), np.float32), pkg.DeviceArray((most, k), np.uint32)
     host = C.c_void_p()
@@ -76,7 +76,7 @@ def test_prepared_search(pkg, dsx, rng, n, dim, most, k):
     try:
         for queries in sorted({1, min(most, 64), most}):
             C.memset(host, 0, 8 * most * k)
-            pkg.check(dsx.dsx_knn_search_host(3, dI.ptr, rows, rows - n, dim, dQ.ptr, queries, k, scores.ptr, idx.ptr, host.value,
+            pkg.check(dsx.dsx_knn_search_host(prepared.value, dI.ptr, rows, rows - n, dim, dQ.ptr, queries, k, scores.ptr, idx.ptr, host.value,
                                               host.value + 4 * most * k, room.ptr, room.nbytes, None))
             words = np.ctypeslib.as_array(C.cast(host, C.POINTER(C.c_uint32)), (2, most * k)).copy()
             hs, hi = words[0].view(np.float32).reshape(most, k)[:queries], words[1].reshape(most, k)[:queries]
