@@ -499,13 +499,15 @@ static int knn_search_common(KnnOperands& op, uint32_t padding, uint32_t num_que
     // (few queries against an fp32 table stay with the blocks, however many there are; a width set by the caller is kept)
     const bool few = knn_few_queries(num_queries) && !op.f16 && !op.split && !ctx().knobs.knn_block_columns;
     const bool may = aligned && (!few || built) && capturing == hipStreamCaptureStatusNone;
+    // (screened searches need no alignment: vectors of 215 components, say, whose fp32 products would be formed block by block)
+    const bool may_screen = (!few || built) && capturing == hipStreamCaptureStatusNone;
     const bool many = M > knn_block_columns(op.rows_padded, num_queries);
-    bool screened = may && w.screen.bytes != 0 && !ctx().knobs.knn_block_columns;
+    bool screened = may_screen && w.screen.bytes != 0 && !ctx().knobs.knn_block_columns;
     bool redo = true, unfit = false;
     if (rc == DSX_OK && screened) rc = knn_search_screened(w, op, M, num_queries, k, out, t, built, even, &redo, &unfit);
     if (unfit) screened = false;
-    const bool candidates = may && (screened || many);
-    if (rc == DSX_OK && candidates && (!screened || redo) && many)
+    const bool candidates = screened || (may && many);
+    if (rc == DSX_OK && may && (!screened || redo) && many)
         rc = knn_search_candidates(w, op, M, num_queries, k, out, t, &redo);
     g_knn_last_path = !candidates ? DSX_KNN_PATH_BLOCKS : (redo ? DSX_KNN_PATH_CANDIDATES_REDONE : DSX_KNN_PATH_CANDIDATES);
     if (rc == DSX_OK && redo) rc = knn_search_blocks(w, op, M, num_queries, k, out, t);
@@ -610,8 +612,7 @@ int dsx_knn_prepare(const float* items, uint32_t rows_padded, uint32_t padding, 
                   rows_padded, padding, dim, num_queries, k);
     DSX_CHECK_ARG(((uintptr_t)workspace % 256) == 0, "dsx_knn_prepare: workspace is not 256-byte aligned");
     *prepared = 0;
-    const bool aligned = ((uintptr_t)items % 16) == 0 && (rows_padded % 4) == 0 && (dim % 4) == 0;
-    if (!knn_prepares(rows_padded, dim, num_queries, k) || !aligned || workspace_bytes < dsx_knn_workspace_bytes_prepared(rows_padded, dim, num_queries, k)) return DSX_OK;
+    if (!knn_prepares(rows_padded, dim, num_queries, k) || workspace_bytes < dsx_knn_workspace_bytes_prepared(rows_padded, dim, num_queries, k)) return DSX_OK;
     const uint32_t M = rows_padded - padding;
     const ScreenTable t = screen_table(workspace, dim, rows_padded);
     if (int rc = screen_build(t, items, rows_padded, M, dim)) return rc;

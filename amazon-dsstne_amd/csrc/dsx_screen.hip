@@ -128,6 +128,7 @@ __global__ __launch_bounds__(256) void screen_items_kernel(ScreenItemsArgs a)
 struct ScreenRowsArgs {
     const float* X;
     uint32_t ldx, batch, dim, ld;
+    int whole;              // X is 16-byte aligned and its pitch a multiple of 4
     _Float16* out16;        // [batch rounded up to 256][ld], zero filled
     float* e1;              // [batch]
     float* e0;              // [batch]
@@ -143,7 +144,7 @@ struct ScreenRowsArgs {
 };
 
 // One wavefront per row, which holds up to 1,024 components of it between the two passes.  Bound by latency, one round trip so (256 x 1,024:
-// 9.7 us when a lane read its components one by one, twice; 4.5 so; 4,096 x 1,024 28 / 14 beside other kernels).  X is 16-byte aligned and its pitch a multiple of 4.
+// 9.7 us when a lane read its components one by one, twice; 4.5 so; 4,096 x 1,024 28 / 14 beside other kernels).
 __global__ __launch_bounds__(256) void screen_rows_kernel(ScreenRowsArgs a)
 {
     const uint32_t row = blockIdx.x * 4 + threadIdx.x / kWave, lane = threadIdx.x % kWave;
@@ -151,11 +152,17 @@ __global__ __launch_bounds__(256) void screen_rows_kernel(ScreenRowsArgs a)
     const float* x = a.X + (uint64_t)row * a.ldx;
     auto part = [&](uint32_t d) __attribute__((always_inline)) -> float4 {
         float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (valid && d < a.dim) {
+        if (!valid || d >= a.dim) return v;
+        if (a.whole) {
             v = *reinterpret_cast<const float4*>(x + d);
             if (d + 1 >= a.dim) v.y = 0.0f;
             if (d + 2 >= a.dim) v.z = 0.0f;
             if (d + 3 >= a.dim) v.w = 0.0f;
+        } else {
+            v.x = x[d];
+            if (d + 1 < a.dim) v.y = x[d + 1];
+            if (d + 2 < a.dim) v.z = x[d + 2];
+            if (d + 3 < a.dim) v.w = x[d + 3];
         }
         return v;
     };
@@ -946,6 +953,7 @@ int screen_build(const ScreenTable& t, const float* W, uint64_t ldw, uint64_t n,
 int screen_rows(const ScreenJob& j, const ScreenTable& t, const ScreenWorkspace& w, ScreenNotes* notes)
 {
     ScreenRowsArgs r{};
+    r.whole = (uintptr_t)j.X % 16 == 0 && j.ldx % 4 == 0;
     r.X = j.X; r.ldx = j.ldx; r.batch = j.batch; r.dim = j.dim; r.ld = screen_ld(j.dim);
     r.out16 = (_Float16*)w.rows16; r.e1 = w.e1; r.e0 = w.e0; r.scale = w.scale; r.scaled = j.bias == nullptr; r.row_flag = j.row_flag; r.told = notes ? &notes->flag : j.told;
     r.cand_count = j.cand_count; r.clear = j.clear; r.clear_words = j.clear_words;
