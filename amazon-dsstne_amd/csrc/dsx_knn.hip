@@ -369,8 +369,13 @@ static int knn_search_screened(const KnnWorkspace& w, const KnnOperands& op, uin
         if (*unfit) return DSX_OK;
         j.even = g_knn_notes->number != 0 && screen_even(g_knn_notes->largest, g_knn_notes->sum / (float)g_knn_notes->number);
     }
+    // (candidates are cut back between the ranges too: what is counted as top-K is the kernel that scores and sorts what is left)
+    if (t.on) {
+        j.before_last = [](void* p) { static_cast<KnnTimer*>(p)->stop(ctx().stream, static_cast<KnnTimer*>(p)->gemm); };
+        j.before_last_arg = &t;
+    }
     if ((rc = screen_run(j, w.table, w.screen))) return rc;
-    t.stop(s, t.gemm);
+    t.stop(s, t.topk);
     DSX_HIP(hipStreamSynchronize(s));
     *overflowed = *(volatile uint32_t*)&g_knn_notes->flag != 0;
     return DSX_OK;
@@ -414,11 +419,14 @@ size_t dsx_knn_workspace_bytes_least(uint32_t rows_padded, uint32_t dim, uint32_
     return knn_workspace_most(rows_padded, num_queries, k, false, dim, false, false);
 }
 
-// A table that is kept pays for itself wherever a search is more than launches: few queries are bound by reading it, and its halves are
-// half of what fp32 would read (4 queries x 1,000,000 x 128: 191 us a search, 125 so; 4,096 queries 2,936, 2,000 so).
+// Where a kept table is used: everywhere but for tables so small that k blocks of 32 items are a large part of them, vectors whose halves are
+// mostly padding, and tables of more than 8 GiB.  us a search, in fp32 / so (both with their results written
+// to host memory): 1 query, 8,192 x 256 top 10 46 / 43, 70,000 x 256 61 / 51, 400,000 x 256 141 / 83; 32 queries, 20,000 x 16 top 100 54 / 44; 128
+// queries, 70,000 x 64 top 10 74 / 53; 512 queries, 8,192 x 64 top 100 138 / 127, 400,000 x 64 643 / 239; 4,096 queries, 8,192 x 16 top 10
+// 228 / 205, 70,000 x 256 1,658 / 563.  None of 88 is slower but few short queries of a long table (knn_search_common).
 static bool knn_prepares(uint32_t rows_padded, uint32_t dim, uint32_t num_queries, uint32_t k)
 {
-    return num_queries > 0 && ctx().knobs.screen != 2 && dim >= 32 && dim <= 4096 && rows_padded >= 65536 && (uint64_t)rows_padded * dim >= 50000000ull &&
+    return num_queries > 0 && ctx().knobs.screen != 2 && dim >= 16 && dim <= 4096 && rows_padded >= 8192 && rows_padded >= 64 * k &&
            screen_table(nullptr, dim, rows_padded).bytes <= ((uint64_t)8 << 30) && k <= 256;
 }
 
@@ -500,7 +508,8 @@ static int knn_search_common(KnnOperands& op, uint32_t padding, uint32_t num_que
     const bool few = knn_few_queries(num_queries) && !op.f16 && !op.split && !ctx().knobs.knn_block_columns;
     const bool may = aligned && (!few || built) && capturing == hipStreamCaptureStatusNone;
     // (screened searches need no alignment: vectors of 215 components, say, whose fp32 products would be formed block by block)
-    const bool may_screen = (!few || built) && capturing == hipStreamCaptureStatusNone;
+    const bool narrow = built && op.dim < 32 && op.rows_padded > 131072 && knn_few_queries(num_queries);   // (16 x 400,000, 32 queries: 65 us / 69)
+    const bool may_screen = (!few || built) && !narrow && capturing == hipStreamCaptureStatusNone;
     const bool many = M > knn_block_columns(op.rows_padded, num_queries);
     bool screened = may_screen && w.screen.bytes != 0 && !ctx().knobs.knn_block_columns;
     bool redo = true, unfit = false;

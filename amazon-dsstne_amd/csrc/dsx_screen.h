@@ -88,6 +88,8 @@ struct ScreenJob {
     uint32_t* overflow;       // scratch word
     uint32_t* clear;          // [clear_words] set to 0 on the way
     uint32_t clear_words;
+    void (*before_last)(void*);   // called before the kernel that ends with the results is launched (NULL: not)
+    void* before_last_arg;
     bool even;                // no bias, no column that always passes, and norms close together (screen_even)
 };
 // The rows in f16 (and notes of the table and the rows, NULL: none), then the search itself.

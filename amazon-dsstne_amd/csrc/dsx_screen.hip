@@ -1024,6 +1024,7 @@ int screen_run(const ScreenJob& j, const ScreenTable& t, const ScreenWorkspace& 
     a.X = j.X; a.ldx = j.ldx; a.dim = j.dim; a.pitch32 = screen_pitch32(j.dim); a.rows32 = t.rows32; a.bias = j.bias;
     a.keys = j.keys; a.values = j.values; a.keys2 = j.keys2; a.values2 = j.values2;
     a.width_z = 2.1f * f.bias_raise + 1.0e-3f;   // (rounding up to a half: 9.9e-4 of it at most)
+    if (stored && j.before_last) j.before_last(j.before_last_arg);
     if ((rc = launch_pick(a, !stored)) || stored) return rc;
     const size_t row_lds = (size_t)(j.dim + 63) / 64 * 256;
     // A bound taken over `done` columns lets about k * width / done of the next `width` columns pass: ranges grow by a factor that
@@ -1045,6 +1046,7 @@ int screen_run(const ScreenJob& j, const ScreenTable& t, const ScreenWorkspace& 
         if (!a.lists && (rc = f16_sweep_run(f, true, &a.lists))) return rc;
         a.seg_cap = kListWords / a.lists;
         done += ncols;
+        if (done >= n && j.before_last) j.before_last(j.before_last_arg);
         // (the sums of the first block, rounded up to halves, are among what is kept: their width is the others' from here on)
         if (done < n) hipLaunchKernelGGL((screen_fold_kernel<false>), dim3(j.batch), dim3(256), 0, s, a);
         else hipLaunchKernelGGL((screen_fold_kernel<true>), dim3(j.batch), dim3(256), row_lds, s, a);

@@ -55,7 +55,8 @@ def test_layer(pkg, dsx, rng, batch, kdim, n, k, filtered):
     assert not differ[want_keys != 0].any()
 
 
-@pytest.mark.parametrize("n,dim,most,k", [(65601, 768, 520, 100), (400003, 128, 4, 10), (270001, 187, 513, 33)])
+@pytest.mark.parametrize("n,dim,most,k", [(65601, 768, 520, 100), (400003, 128, 4, 10), (270001, 187, 513, 33),
+                                               (8192, 16, 70, 128), (8193, 19, 1, 1)])
 def test_prepared_search(pkg, dsx, rng, n, dim, most, k):
     """Few queries, many, and the results in host memory."""
     print("[case] prepared search n=%d dim=%d queries=%d k=%d" % (n, dim, most, k), flush=True)
