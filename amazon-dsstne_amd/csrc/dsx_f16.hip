@@ -22,7 +22,7 @@
 // result, a block with two survivors took some 700 cycles of a wavefront: 245,760 items x 128 x 4,096 queries with 500 survivors each
 // 541 us, 430 so, 275 without survivors.)
 // 4,096 queries x 1,000,000 items: 1.09 PFLOP/s with 512 components (a large product of the matrix library reaches 1.16 on this part),
-// 0.90 with 128, where the compares are a third of the issued instructions.  knn_f16_kernel's 128 x 128 tiles reached 0.72 with 576.
+// 0.90 with 128, where the compares are a third of the issued instructions.  (128 x 128 tiles through registers: 0.72 with 576.)
 #include <algorithm>
 #include "dsx_screen.h"
 

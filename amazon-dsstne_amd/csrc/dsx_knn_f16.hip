@@ -434,7 +434,7 @@ int knn_f16_wide_run(const void* queries16, const void* items16, uint32_t ld, ui
 {
     *lists_used = 0;
     if (ld > 256) return DSX_OK;
-    // queries in registers: 512 per workgroup, stages of 64 items, one workgroup per CU
+    // queries in registers: 512 per workgroup, stages of 128 items, one workgroup per CU
     const uint32_t cus = (uint32_t)ctx().num_cus, tiles_q = (batch + 511) / 512, stages = (n + kWideStageItems - 1) / kWideStageItems;
     const uint32_t chunks = std::min<uint32_t>(kF16ListStride / 2, (cus + tiles_q - 1) / tiles_q);   // two lists per (query, chunk)
     if (every ? stages < chunks : (2 * tiles_q * chunks < cus || stages < 8 * chunks)) return DSX_OK;

@@ -18,9 +18,10 @@
 // Exceptions: a column whose norm is above 60,000 gets zeros and an infinite start (it always passes); a row above 65,504 is flagged,
 // as is one whose lists fill up (thousands of scores tied at the top): its caller computes it again in fp32.
 //
-// Two ways (screen_stored).  Few columns, or few rows: the sums are stored as halves, rounded up, and a workgroup per row (or part of
-// one) takes what reaches the bound from there.  Many of both: only a first block's are; the rest are compared with the rows' bounds
-// where they are formed, in ranges that grow by a factor, after each of which the lists are cut back to what can still be a result.
+// Two ways (screen_stored).  Few columns, or few rows: the sums are stored as halves, rounded up, and a workgroup per row takes what
+// reaches the bound from there.  Many of both: only a first block's are; the rest are compared with the rows' bounds where they are
+// formed (raised by their errors, or against bounds lowered by the largest: screen_even), in ranges that grow by a factor, after
+// each of which the lists are cut back to what can still be a result.
 // Candidates of earlier ranges are not scored until the last one is through: what is scored in fp32 is about 1.2 k columns a row.
 #include <algorithm>
 #include <atomic>

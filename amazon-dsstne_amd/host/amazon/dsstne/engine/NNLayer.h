@@ -95,6 +95,7 @@ private:
     // Whether the deferred layer and a top-K of k entries are computed in one call (or the layer is stored first).
     bool TopKFusionPays(uint32_t batch, uint32_t k);
     // The weights' table, where the layer and a top-K of k entries are fastest screened by it (else NULL).
+    bool TopKScreenPays(uint32_t batch, uint32_t k);
     const void* TopKScreenTable(uint32_t batch, uint32_t k);
     // Whether the deferred layer's top-K has been computed; a narrower layer whose units are asked for all the same is stored from then on.
     bool _bToppedDeferred = false;

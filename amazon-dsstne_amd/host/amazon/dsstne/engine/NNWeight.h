@@ -53,7 +53,7 @@ private:
     // their top-K; kept like the planes.  NULL: there is no room for it (half of what is free), or the caller may change the matrix
     // (_bHandedOut).
     void* _pScreen = NULL;
-    bool _bScreenValid = false;
+    bool _bScreenValid = false, _bScreenRefused = false;
     const void* ScreenTable(uint32_t k, uint32_t n);
     void InvalidateSplit() { _bSplitValid[0] = _bSplitValid[1] = _bScreenValid = false; }
 

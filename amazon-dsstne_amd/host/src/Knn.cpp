@@ -168,6 +168,7 @@ static Matrix allocateResults(uint32_t numRows, int numColumns, size_t elementSi
 {
     void* data = nullptr;
     check(dsx_malloc_host(&data, (size_t)numRows * numColumns * elementSize), "allocateResults");
+    std::memset(data, 0, (size_t)numRows * numColumns * elementSize);   // (pages that nobody has touched fault one by one in the first search)
     return Matrix(data, numRows, numColumns, elementSize, MemoryType::Host);
 }
 

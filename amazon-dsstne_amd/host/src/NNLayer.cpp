@@ -141,13 +141,16 @@ static const uint32_t kSegMaxMinWidth = 8192;
 // 16 GB of stores and loads go away.
 static const uint32_t kDeferMinWidth = 131072;
 
+bool NNLayer::TopKScreenPays(uint32_t batch, uint32_t k)
+{
+    NNWeight* w = _vIncomingWeight[0];
+    return !w->_bTransposed && !UseSplitProducts(batch) && dsx_fc_topk_screened_pays(batch, _vIncomingLayer[0]->_stride, _localStride, (uint32_t)_activation, k) != 0;
+}
+
 const void* NNLayer::TopKScreenTable(uint32_t batch, uint32_t k)
 {
-    NNLayer* src = _vIncomingLayer[0];
     NNWeight* w = _vIncomingWeight[0];
-    NNWeight* wsrc = w->_bShared ? w->_pSharedWeight : w;
-    if (w->_bTransposed || UseSplitProducts(batch) || !dsx_fc_topk_screened_pays(batch, src->_stride, _localStride, (uint32_t)_activation, k)) return NULL;
-    return wsrc->ScreenTable(src->_stride, _localStride);
+    return TopKScreenPays(batch, k) ? (w->_bShared ? w->_pSharedWeight : w)->ScreenTable(_vIncomingLayer[0]->_stride, _localStride) : NULL;
 }
 
 bool NNLayer::TopKFusionPays(uint32_t batch, uint32_t k)
@@ -185,7 +188,7 @@ void NNLayer::ForwardPropagateFullyConnected(uint32_t position, uint32_t batch, 
             // without the layer's result ever being stored.  The layer is computed when somebody asks for it.
             // (a narrower one is not put off while a caller holds a pointer through which its operands may change meanwhile)
             const bool bHeld = _localStride < kDeferMinWidth && (src->_bHandedOut || wsrc->_bHandedOut);
-            if (_bDeferOutput && !bHeld && TopKFusionPays(batch, 1) && !w->_bTransposed && _vOutgoingLayer.empty() && _vOutgoingSkip.empty() &&
+            if (_bDeferOutput && !bHeld && (TopKScreenPays(batch, 1) || TopKFusionPays(batch, 1)) && !w->_bTransposed && _vOutgoingLayer.empty() && _vOutgoingSkip.empty() &&
                 dsx_fc_topk_supported(src->_stride, src->GetUnitBuffer(), (uint32_t)_activation, &params, NULL)) {
                 if (dsx_fc_topk_flagged_for(wsrc->_pbWeight->_pDevData, 0)) {
                     // rows whose survivor lists filled up (thousands of scores tied at the top), or whose inputs f16 cannot hold, had

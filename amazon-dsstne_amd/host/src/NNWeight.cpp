@@ -203,7 +203,7 @@ const void* NNWeight::SplitPlanes(bool bTransposed, uint32_t k, uint32_t n)
 
 const void* NNWeight::ScreenTable(uint32_t k, uint32_t n)
 {
-    if (_bHandedOut) return NULL;
+    if (_bHandedOut || _bScreenRefused) return NULL;
     if (!_bScreenValid) {
         if (!_pScreen) {
             const uint64_t bytes = dsx_screen_table_bytes(n, k);
@@ -211,6 +211,7 @@ const void* NNWeight::ScreenTable(uint32_t k, uint32_t n)
             dsxFatal(dsx_get_device_info(&info), "NNWeight::ScreenTable");
             if (bytes > info.hbm_free_bytes / 2 || dsx_malloc(&_pScreen, bytes) != DSX_OK) {
                 _pScreen = NULL;
+                _bScreenRefused = true;   // (asked once: every top-K comes here)
                 return NULL;
             }
         }
