@@ -372,25 +372,32 @@ def network_bench(args, pkg, lib):
             g.update({"achieved": (moved["read"] + moved["write"]) / ms / 1e6, "peak": HBM_PEAK_GBS, "unit": "GB/s"})
             g["frac"] = g["achieved"] / g["peak"]
         kernels["topk_guided_kernel"] = g
-    deferred = bool(lib.dsx_fc_topk_pays(B, p.widths[last], N, p.acts[last], K))      # as NNLayer decides
+    # as NNLayer decides: with a kept table of the weights, or without
+    kept = bool(lib.dsx_fc_topk_screened_pays(B, p.widths[last], N, p.acts[last], K))
+    deferred = kept or bool(lib.dsx_fc_topk_pays(B, p.widths[last], N, p.acts[last], K))
+    fused_name = "%s (output layer + filtered top-K, nothing stored)" % ("dsx_fc_topk_screened" if kept else "dsx_fc_topk")
     if deferred:
+        if kept:
+            table = pkg.DeviceArray((lib.dsx_screen_table_bytes(N, p.widths[last]),), np.uint8)
+            pkg.check(lib.dsx_screen_table_build(ptr(pipe.W[last]), N, N, p.widths[last], table.ptr))
         keys = pkg.DeviceArray((B, K), np.float32)
         vals = pkg.DeviceArray((B, K), np.uint32)
 
         def k_fused():
-            pkg.check(lib.dsx_fc_topk(ptr(pipe.units[last - 1]), p.widths[last], ptr(pipe.W[last]), ptr(pipe.b[last]), B, p.widths[last], N,
-                                      p.acts[last], params, K, keys.ptr, vals.ptr, 0, ptr(pipe.index), ptr(pipe.start), ptr(pipe.end),
-                                      ptr(pipe.sidx)))
+            of, tail = (ptr(pipe.units[last - 1]), p.widths[last], ptr(pipe.W[last])), (
+                ptr(pipe.b[last]), B, p.widths[last], N, p.acts[last], params, K, keys.ptr, vals.ptr, 0, ptr(pipe.index), ptr(pipe.start),
+                ptr(pipe.end), ptr(pipe.sidx))
+            pkg.check(lib.dsx_fc_topk_screened(*of, table.ptr, *tail) if kept else lib.dsx_fc_topk(*of, *tail))
         k_fused()
         pkg.check(lib.dsx_sync())
         deferred = not lib.dsx_fc_topk_flagged_for(ptr(pipe.W[last]), 0)   # scores that tie in their thousands: the network stores the layer from then on
     if deferred:
         flops = 2.0 * B * p.widths[last] * N
         ms = time_launches(pkg, lib, k_fused, max(5, reps // 4))
-        kernels["dsx_fc_topk (output layer + filtered top-K, nothing stored)"] = {
+        kernels[fused_name] = {
             "bound": "mfma", "ms": ms, "achieved": flops / ms / 1e9, "peak": F16_MFMA_PEAK_TF, "unit": "TFLOP/s",
             "algorithmic_flops": flops, "frac": flops / ms / 1e9 / F16_MFMA_PEAK_TF,
-            "note": "what the timed step runs for this layer: first column block stored and scanned, the rest screened in f16 and what passes scored in fp32; priced against the f16 peak"}
+            "note": "what the timed step runs for this layer: all columns screened in f16, what can be a result scored in fp32; priced against the f16 peak"}
 
     # The output layer's kernel of the split-products mode (off by default, so never the dominant kernel of `roofline`): priced as the
     # bf16 matrix work it executes, six products per fp32 product, against the bf16 peak.
