@@ -1041,9 +1041,8 @@ __global__ __launch_bounds__(1024) void softmax_kernel(float* z, uint32_t stride
         for (int o = 32; o > 0; o >>= 1) v = op(v, __shfl_xor(v, o, kWave));
         if (lane == 0) sRed[which][wave] = v;
         __syncthreads();
-        float r = sRed[which][0];
-#pragma unroll
-        for (int w = 1; w < 1024 / kWave; w++) r = op(r, sRed[which][w]);
+        float r = sRed[which][lane % (1024 / kWave)];
+        for (int o = 1024 / kWave / 2; o > 0; o >>= 1) r = op(r, __shfl_xor(r, o, kWave));   // (by halves: fewer roundings than in turn)
         return r;
     };
     if constexpr (HELD) {
@@ -1067,10 +1066,12 @@ __global__ __launch_bounds__(1024) void softmax_kernel(float* z, uint32_t stride
         for (int g = 0; g < G; g++) {
             const uint32_t j = (g * 1024 + threadIdx.x) * 4;
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                x[g][e] = __expf(x[g][e] - m);
-                if (j + e < stride) s += x[g][e];
-            }
+            for (int e = 0; e < 4; e++) x[g][e] = __expf(x[g][e] - m);
+            if (j + 4 <= stride) s += (x[g][0] + x[g][1]) + (x[g][2] + x[g][3]);
+            else
+#pragma unroll
+                for (int e = 0; e < 3; e++)
+                    if (j + e < stride) s += x[g][e];
         }
     } else
         for (uint32_t j = threadIdx.x; j < stride; j += 1024) s += __expf(row[j] - m);
