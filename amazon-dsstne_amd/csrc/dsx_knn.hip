@@ -9,7 +9,8 @@
 // score, say) raises a flag that the host reads at the end, and the search is then redone block by block — GEMM into the
 // scratch matrix, scanning top-K into packed partial lists with the running bound, one merge — which is also the path
 // taken while the stream is being captured into a graph (no host read-back there; the caller then passes its own workspace,
-// the library's would have to be allocated inside the capture) and for operands that are not 16-byte aligned.  With fp16 storage (dsx_knn_search_f16) the scores come from the f16 MFMA kernel of dsx_knn_f16.hip instead, through
+// the library's would have to be allocated inside the capture) and for operands that are not 16-byte aligned, unless they are screened
+// (dsx_screen.hip).  With fp16 storage (dsx_knn_search_f16) the scores come from the f16 MFMA kernel of dsx_knn_f16.hip instead, through
 // the same three steps.
 #include <algorithm>
 #include <cstring>
