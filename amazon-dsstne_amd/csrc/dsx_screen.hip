@@ -909,7 +909,9 @@ ScreenWorkspace screen_layout(void* base, uint32_t batch, uint32_t dim, uint64_t
 {
     ScreenWorkspace w;
     char* p = (char*)base;
-    const uint64_t columns = screen_stored(batch, n) ? n : screen_first_columns((uint32_t)n, k);
+    // (decided here for every search in this workspace, which may be of fewer columns: pad rows of an item table)
+    w.stored = screen_stored(batch, n);
+    const uint64_t columns = w.columns = w.stored ? (uint32_t)n : screen_first_columns((uint32_t)n, k);
     w.rows16 = p;
     p += align256(knn_f16_rows(batch) * screen_ld(dim) * 2);
     w.e1 = (float*)p;
@@ -1001,8 +1003,8 @@ int screen_run(const ScreenJob& j, const ScreenTable& t, const ScreenWorkspace& 
 {
     hipStream_t s = ctx().stream;
     const uint32_t ld = screen_ld(j.dim), n = j.n;
-    const bool stored = screen_stored(j.batch, n);
-    const uint32_t n0 = stored ? n : screen_first_columns(n, j.k);
+    const bool stored = w.stored;
+    const uint32_t n0 = std::min(w.columns, n);
     F16Job f{};
     f.Q = w.rows16; f.items = t.items16; f.ld = ld; f.batch = j.batch; f.n = n0;
     f.norm = t.norm; f.bias = j.bias; f.e1 = w.e1; f.bias_raise = screen_bias_raise(j.dim);
@@ -1057,3 +1059,19 @@ int screen_run(const ScreenJob& j, const ScreenTable& t, const ScreenWorkspace& 
 }
 
 }  // namespace dsx
+
+using namespace dsx;
+
+extern "C" int dsx_testing_screen_columns(uint32_t batch, uint32_t dim, uint32_t rows_padded, uint32_t padding, uint32_t k, uint64_t* room, uint64_t* stored,
+                                          int* ranges)
+{
+    DSX_CHECK_ARG(room && stored && ranges, "dsx_testing_screen_columns: null pointer");
+    DSX_CHECK_ARG(batch > 0 && dim > 0 && padding < rows_padded && k >= 1, "dsx_testing_screen_columns: batch %u, dim %u, rows_padded %u, padding %u, k = %u", batch,
+                  dim, rows_padded, padding, k);
+    const ScreenWorkspace w = screen_layout(nullptr, batch, dim, rows_padded, k);
+    const uint32_t n0 = std::min(w.columns, rows_padded - padding);   // as screen_run
+    *room = (uint64_t)((char*)w.most - (char*)w.sums) / 2 / batch;
+    *stored = (n0 + 255) / 256 * 256;
+    *ranges = !w.stored;
+    return DSX_OK;
+}

@@ -32,6 +32,11 @@ int dsx_testing_occupy(uint32_t workgroups, uint32_t cycles, uint32_t vgprs);
  * 1: whatever can be (searches of 512 queries and 65,536 items, layers of 512 rows and 16,384 columns and more).  Workspace sizes
  * depend on it. */
 int dsx_testing_set_screen(int mode);
+/* What a screened search of `batch` rows among rows_padded - padding columns (of rows_padded, which its workspace is laid out for) does:
+ * columns of sums that there is room for per row, columns that are stored (whole tiles), and whether the others are gone through in ranges
+ * (0: the results come from the stored ones).  Runs on the host alone, without dsx_init. */
+int dsx_testing_screen_columns(uint32_t batch, uint32_t dim, uint32_t rows_padded, uint32_t padding, uint32_t k, uint64_t* room, uint64_t* stored,
+                               int* ranges);
 /* Largest single block of device memory that dsx_malloc and the library's own scratch may hold, in bytes (0, the default: what the
  * device has): larger ones fail as if the memory were short. */
 int dsx_testing_set_allocation_limit(size_t bytes);

@@ -118,3 +118,31 @@ def test_results_in_host_memory(pkg, dsx, rng, storage, n, queries, k):
         assert np.array_equal(scores.numpy(), rs) and np.array_equal(idx.numpy(), ri)
     finally:
         dsx.dsx_free(host)
+
+
+# tables whose pad rows lie across a width, or a product with the queries, at which whole rows stop being stored: laid out for the one side, searched
+# on the other
+@pytest.mark.parametrize("rows,padding,queries,k", [(131080, 8, 600, 10), (140000, 12000, 513, 33), (1048584, 16, 3, 20), (129400, 100, 8300, 10)])
+def test_pad_rows_across_a_limit(pkg, dsx, rng, rows, padding, queries, k):
+    print("[case] pad rows rows=%d padding=%d queries=%d k=%d" % (rows, padding, queries, k), flush=True)
+    dim, n = 32, rows - padding
+    items = rng.integers(-3, 4, size=(n, dim)).astype(np.float32)
+    q = rng.integers(-3, 4, size=(queries, dim)).astype(np.float32)
+    cm = np.full((dim, rows), 1e30, dtype=np.float32)
+    cm[:, :n] = items.T
+    dI, dQ = dev(pkg, cm), dev(pkg, q)
+    room = pkg.DeviceArray((dsx.dsx_knn_workspace_bytes_prepared(rows, dim, queries, k),), np.uint8)
+    prepared = C.c_int(-1)
+    pkg.check(dsx.dsx_knn_prepare(dI.ptr, rows, padding, dim, queries, k, room.ptr, room.nbytes, C.byref(prepared)))
+    assert prepared.value == 4
+    scores, idx = pkg.DeviceArray((queries, k), np.float32), pkg.DeviceArray((queries, k), np.uint32)
+    rows_looked_at = np.unique(np.concatenate([np.arange(min(queries, 40)), rng.integers(0, queries, 200), [queries - 1]]))
+    rs, ri = best(q[rows_looked_at] @ items.T, k)
+    # the kept table, a table made in the call, and the library's own workspace
+    for storage, space in ((prepared.value, room), (0, room), (0, None)):
+        scores.upload(np.zeros((queries, k), np.float32))
+        pkg.check(dsx.dsx_knn_search_host(storage, dI.ptr, rows, padding, dim, dQ.ptr, queries, k, scores.ptr, idx.ptr, None, None,
+                                          space.ptr if space else None, space.nbytes if space else 0, None))
+        assert np.array_equal(scores.numpy()[rows_looked_at], rs) and np.array_equal(idx.numpy()[rows_looked_at], ri)
+        if storage == prepared.value:   # (the other ways write over the table)
+            assert dsx.dsx_knn_last_search_path() == 1

@@ -1,0 +1,32 @@
+"""Where a screened search stores its sums and what it does with the columns behind them: decided on the host, from the workspace that was laid
+out (no GPU)."""
+import ctypes as C
+import itertools
+
+import pytest
+
+
+def plan(lib, pkg, batch, rows, padding, k, dim=32):
+    room, stored, ranges = C.c_uint64(), C.c_uint64(), C.c_int()
+    pkg.check(lib.dsx_testing_screen_columns(batch, dim, rows, padding, k, C.byref(room), C.byref(stored), C.byref(ranges)))
+    return room.value, stored.value, ranges.value
+
+
+def around(x):
+    return [x - 257, x - 8, x - 1, x, x + 1, x + 8, x + 300]
+
+
+# the widths and products at which whole rows stop being stored
+SHAPES = [(b, r) for b, r in itertools.chain(((b, r) for b in (1, 64, 512, 513, 1000, 4096) for edge in (8192, 131072, 1048576) for r in around(edge)),
+                                             ((b, r) for b in (2000, 10000, 65600, 120000, 131073) for r in around((1 << 30) // b)))]
+
+
+@pytest.mark.parametrize("k", [1, 100, 256])
+def test_what_is_stored_fits_what_was_laid_out(pkg, k):
+    lib = pkg.load_library()
+    for batch, rows in SHAPES:
+        for padding in (0, 1, 4, 7, 8, 300, rows // 2, rows - 1):
+            if padding >= rows:
+                continue
+            room, stored, ranges = plan(lib, pkg, batch, rows, padding, k)
+            assert stored <= (room + 255) // 256 * 256 and stored <= room, (batch, rows, padding, k)
