@@ -41,10 +41,9 @@ struct ScreenTable {
 ScreenTable screen_table(void* base, uint32_t dim, uint64_t n);
 int screen_build(const ScreenTable& t, const float* W, uint64_t ldw, uint64_t n, uint32_t dim);
 
-// What a call works in.  stored, columns: whether all columns' sums are stored, and how many columns there is room for at most (the first block's
-// otherwise); screen_run goes by these and not by its own number of columns.
+// What a call works in.  columns: how many columns' sums there is room for, all of them or a first block's; screen_run goes by that and not by its
+// own number of columns.
 struct ScreenWorkspace {
-    bool stored;
     uint32_t columns;
     void* rows16;
     float* e1;

@@ -910,8 +910,7 @@ ScreenWorkspace screen_layout(void* base, uint32_t batch, uint32_t dim, uint64_t
     ScreenWorkspace w;
     char* p = (char*)base;
     // (decided here for every search in this workspace, which may be of fewer columns: pad rows of an item table)
-    w.stored = screen_stored(batch, n);
-    const uint64_t columns = w.columns = w.stored ? (uint32_t)n : screen_first_columns((uint32_t)n, k);
+    const uint64_t columns = w.columns = screen_stored(batch, n) ? (uint32_t)n : screen_first_columns((uint32_t)n, k);
     w.rows16 = p;
     p += align256(knn_f16_rows(batch) * screen_ld(dim) * 2);
     w.e1 = (float*)p;
@@ -1003,8 +1002,9 @@ int screen_run(const ScreenJob& j, const ScreenTable& t, const ScreenWorkspace& 
 {
     hipStream_t s = ctx().stream;
     const uint32_t ld = screen_ld(j.dim), n = j.n;
-    const bool stored = w.stored;
+    // (a first block that is everything, of a narrow table and more than 2^30 sums, is a search of stored sums too: there is no range to end with)
     const uint32_t n0 = std::min(w.columns, n);
+    const bool stored = n0 == n;
     F16Job f{};
     f.Q = w.rows16; f.items = t.items16; f.ld = ld; f.batch = j.batch; f.n = n0;
     f.norm = t.norm; f.bias = j.bias; f.e1 = w.e1; f.bias_raise = screen_bias_raise(j.dim);
@@ -1072,6 +1072,6 @@ extern "C" int dsx_testing_screen_columns(uint32_t batch, uint32_t dim, uint32_t
     const uint32_t n0 = std::min(w.columns, rows_padded - padding);   // as screen_run
     *room = (uint64_t)((char*)w.most - (char*)w.sums) / 2 / batch;
     *stored = (n0 + 255) / 256 * 256;
-    *ranges = !w.stored;
+    *ranges = n0 < rows_padded - padding;
     return DSX_OK;
 }

@@ -146,3 +146,39 @@ def test_pad_rows_across_a_limit(pkg, dsx, rng, rows, padding, queries, k):
         assert np.array_equal(scores.numpy()[rows_looked_at], rs) and np.array_equal(idx.numpy()[rows_looked_at], ri)
         if storage == prepared.value:   # (the other ways write over the table)
             assert dsx.dsx_knn_last_search_path() == 1
+
+
+# more than 2^30 sums of a table no wider than a first block, which is all there is then
+def test_large_batches_of_narrow_tables(pkg, dsx, rng):
+    queries, n, dim, k = 66000, 16380, 16, 256
+    print("[case] prepared search n=%d dim=%d queries=%d k=%d" % (n, dim, queries, k), flush=True)
+    items = rng.integers(-3, 4, size=(n, dim)).astype(np.float32)
+    q = rng.integers(-3, 4, size=(queries, dim)).astype(np.float32)
+    rows, looked_at = n + 4, np.unique(np.concatenate([np.arange(20), rng.integers(0, queries, 200), np.arange(queries - 20, queries)]))
+    cm = np.full((dim, rows), 1e30, dtype=np.float32)
+    cm[:, :n] = items.T
+    dI, dQ = dev(pkg, cm), dev(pkg, q)
+    room = pkg.DeviceArray((dsx.dsx_knn_workspace_bytes_prepared(rows, dim, queries, k),), np.uint8)
+    prepared = C.c_int(-1)
+    pkg.check(dsx.dsx_knn_prepare(dI.ptr, rows, 4, dim, queries, k, room.ptr, room.nbytes, C.byref(prepared)))
+    scores, idx = dev(pkg, np.zeros((queries, k), np.float32)), pkg.DeviceArray((queries, k), np.uint32)
+    pkg.check(dsx.dsx_knn_search_host(prepared.value, dI.ptr, rows, 4, dim, dQ.ptr, queries, k, scores.ptr, idx.ptr, None, None, room.ptr, room.nbytes, None))
+    rs, ri = best(q[looked_at] @ items.T, k)
+    assert np.array_equal(scores.numpy()[looked_at], rs) and np.array_equal(idx.numpy()[looked_at], ri)
+
+    print("[case] kept table layer batch=%d kdim=%d n=%d k=%d" % (queries, dim, n, k), flush=True)
+    room.free()
+    start, end, fidx = random_csr(rng, queries, n, 100)
+    W, bias = np.ascontiguousarray(items.T), rng.integers(30, 41, size=n).astype(np.float32)
+    dW, db, ds, de, dx = (dev(pkg, a) for a in (W, bias, start, end, fidx))
+    table = pkg.DeviceArray((dsx.dsx_screen_table_bytes(n, dim),), np.uint8)
+    pkg.check(dsx.dsx_screen_table_build(dW.ptr, n, n, dim, table.ptr))
+    scores.upload(np.zeros((queries, k), np.float32))
+    pkg.check(dsx.dsx_fc_topk_screened(dQ.ptr, dim, dW.ptr, table.ptr, db.ptr, queries, dim, n, 3, None, k, scores.ptr, idx.ptr, 0, None, ds.ptr,
+                                       de.ptr, dx.ptr))
+    y = q[looked_at] @ W + bias
+    for at, b in enumerate(looked_at):
+        y[at, fidx[int(start[b]):int(end[b])]] = 0
+    rs, ri = best(y, k)
+    assert np.array_equal(scores.numpy()[looked_at], rs)
+    assert not (idx.numpy()[looked_at] != ri)[rs != 0].any()

@@ -30,3 +30,14 @@ def test_what_is_stored_fits_what_was_laid_out(pkg, k):
                 continue
             room, stored, ranges = plan(lib, pkg, batch, rows, padding, k)
             assert stored <= (room + 255) // 256 * 256 and stored <= room, (batch, rows, padding, k)
+
+
+@pytest.mark.parametrize("k", [1, 100, 150, 256])
+def test_every_search_ends_with_its_results(pkg, k):
+    """Results come from the stored sums, or from the last of the ranges behind them: where the first block is everything there are none."""
+    lib = pkg.load_library()
+    for batch, rows in SHAPES + [(120000, 10000), (70000, 16384), (66000, 16380), (140000, 8192), (33000, 32768)]:
+        for padding in (0, 7, 300, rows // 2, rows - 1):
+            if padding < rows:
+                room, stored, ranges = plan(lib, pkg, batch, rows, padding, k)
+                assert ranges == (stored < rows - padding), (batch, rows, padding, k)
