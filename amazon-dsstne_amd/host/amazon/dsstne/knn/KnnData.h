@@ -38,22 +38,52 @@ struct Matrix {
 
 Matrix loadDataOnHost(DataReader* dataReader);
 
+// Matrices of which something else is kept (copies of the table, in the workspace), to be used like the vector of them that they are. A program
+// that has asked for one may write to it, or put another in its place, at any time from then on: handedOut says so, and what is kept is not
+// relied on any more.
+class WatchedMatrices {
+public:
+    explicit WatchedMatrices(size_t count) : all(count) {}
+    operator std::vector<Matrix>&() const { return handOut(); }
+    WatchedMatrices& operator=(const std::vector<Matrix>& other) { handOut() = other; return *this; }
+    Matrix& operator[](size_t i) const { return handOut()[i]; }
+    Matrix& at(size_t i) const { return handOut().at(i); }
+    Matrix& front() const { return handOut().front(); }
+    Matrix& back() const { return handOut().back(); }
+    Matrix* data() const { return handOut().data(); }
+    std::vector<Matrix>::iterator begin() const { return handOut().begin(); }
+    std::vector<Matrix>::iterator end() const { return handOut().end(); }
+    size_t size() const { return all.size(); }
+    bool empty() const { return all.empty(); }
+
+private:
+    friend struct KnnData;
+    friend class KnnExactGpu;
+    std::vector<Matrix>& handOut() const
+    {
+        handedOut = true;
+        return all;
+    }
+    mutable std::vector<Matrix> all;
+    mutable bool handedOut = false;
+};
+
 struct KnnData {
     const int numGpus;
     const int batchSize;
     const int maxK;
 
-    std::vector<Matrix> dCollectionPartitions;   // column major
+    WatchedMatrices dCollectionPartitions;       // column major
     std::vector<Matrix> dInputBatches;
     std::vector<Matrix> dResultScores;
     std::vector<Matrix> dResultIndexes;
     std::vector<Matrix> hResultScores;
     std::vector<Matrix> hResultIndexes;
     std::vector<std::vector<std::string>> hKeys;
-    std::vector<Matrix> dWorkspaces;             // score blocks + partial lists of the search (instead of a full product matrix)
+    WatchedMatrices dWorkspaces;                 // score blocks + partial lists of the search (instead of a full product matrix)
     std::vector<uint32_t> collectionRowsPadded;  // pad rows per device (rows are padded to a multiple of 8)
-    // FP32: not 0 if the workspace holds copies of the table that load made (dsx_knn_prepare: with which storage); a program that writes to dCollectionPartitions
-    // itself sets this to 0, and searches make their own
+    // FP32: not 0 if the workspace holds copies of the table that load made (dsx_knn_prepare: with which storage); searches use them unless the program
+    // has asked for the table or the workspace itself, and as long as this is not set to 0
     std::vector<int> workspacePrepared;
     std::vector<float> elapsedSgemm;             // milliseconds of the last search, per device
     std::vector<float> elapsedTopK;

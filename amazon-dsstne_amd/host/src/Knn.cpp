@@ -193,7 +193,7 @@ KnnData::KnnData(int numGpus, int batchSize, int maxK, DataType dataType)
             getDataTypeString(dataType).c_str());
 }
 
-int KnnData::getFeatureSize() const { return dCollectionPartitions[0].numColumns; }
+int KnnData::getFeatureSize() const { return dCollectionPartitions.all[0].numColumns; }
 
 void KnnData::load(int device, DataReader* dataReader)
 {
@@ -212,13 +212,13 @@ void KnnData::load(int device, DataReader* dataReader)
         hKeys[device].push_back(key);
         for (int j = 0; j < columns; ++j) hTmpData[(size_t)j * rows + rowNum] = vec[j];   // column major
     }
-    freeMatrix(dCollectionPartitions[device]);
+    freeMatrix(dCollectionPartitions.all[device]);
     freeMatrix(dInputBatches[device]);
     freeMatrix(dResultScores[device]);
     freeMatrix(dResultIndexes[device]);
     freeResults(hResultScores[device]);
     freeResults(hResultIndexes[device]);
-    freeMatrix(dWorkspaces[device]);
+    freeMatrix(dWorkspaces.all[device]);
     if (dataType == DataType::FP16) {
         // knn/KnnData.cpp:209-216: the table is kept as halves (round to nearest even); the fp32 copy only lives until it is
         // converted.  The fp16 table has this library's padded item-major layout, so its Matrix describes the logical shape
@@ -227,7 +227,7 @@ void KnnData::load(int device, DataReader* dataReader)
         check(dsx_memcpy_h2d(dTmp.data, hTmpData, hTmp.getSizeInBytes()), "KnnData::load");
         void* table = nullptr;
         check(dsx_malloc(&table, dsx_knn_f16_table_bytes(rows, (uint32_t)columns)), "KnnData::load");
-        dCollectionPartitions[device] = Matrix(table, rows, columns, 2, MemoryType::Device);
+        dCollectionPartitions.all[device] = Matrix(table, rows, columns, 2, MemoryType::Device);
         check(dsx_knn_f16_convert_items((const float*)dTmp.data, rows, rows - actualRows, (uint32_t)columns, table), "KnnData::load");
         check(dsx_sync(), "KnnData::load");
         freeMatrix(dTmp);
@@ -238,13 +238,13 @@ void KnnData::load(int device, DataReader* dataReader)
         check(dsx_memcpy_h2d(dTmp.data, hTmpData, hTmp.getSizeInBytes()), "KnnData::load");
         void* planes = nullptr;
         check(dsx_malloc(&planes, dsx_fc_split_bytes(rows, (uint32_t)columns)), "KnnData::load");
-        dCollectionPartitions[device] = Matrix(planes, rows, columns, 6, MemoryType::Device);
+        dCollectionPartitions.all[device] = Matrix(planes, rows, columns, 6, MemoryType::Device);
         check(dsx_fc_split((const float*)dTmp.data, rows, 1, rows, (uint32_t)columns, planes), "KnnData::load");
         check(dsx_sync(), "KnnData::load");
         freeMatrix(dTmp);
     } else {
-        dCollectionPartitions[device] = allocateMatrixOnDevice(rows, columns, sizeof(float));
-        check(dsx_memcpy_h2d(dCollectionPartitions[device].data, hTmpData, hTmp.getSizeInBytes()), "KnnData::load");
+        dCollectionPartitions.all[device] = allocateMatrixOnDevice(rows, columns, sizeof(float));
+        check(dsx_memcpy_h2d(dCollectionPartitions.all[device].data, hTmpData, hTmp.getSizeInBytes()), "KnnData::load");
     }
     freeMatrix(hTmp);
     dInputBatches[device] = allocateMatrixOnDevice(batchSize, columns, sizeof(float));
@@ -267,10 +267,10 @@ void KnnData::load(int device, DataReader* dataReader)
         rc = dsx_malloc(&workspace, least);
     }
     check(rc, "KnnData::load");
-    dWorkspaces[device] = Matrix(workspace, 1, 1, wsTaken, MemoryType::Device);
+    dWorkspaces.all[device] = Matrix(workspace, 1, 1, wsTaken, MemoryType::Device);
     int prepared = 0;
     if (dataType == DataType::FP32 && wsTaken == ws)
-        check(dsx_knn_prepare((const float*)dCollectionPartitions[device].data, rows, rows - actualRows, (uint32_t)columns, (uint32_t)batchSize,
+        check(dsx_knn_prepare((const float*)dCollectionPartitions.all[device].data, rows, rows - actualRows, (uint32_t)columns, (uint32_t)batchSize,
                               (uint32_t)maxK, workspace, ws, &prepared),
               "KnnData::load");
     workspacePrepared[device] = prepared;
@@ -307,13 +307,13 @@ void KnnData::load(const std::map<int, std::string>& deviceToFile, char keyValDe
 
 KnnData::~KnnData()
 {
-    for (auto& m : dCollectionPartitions) freeMatrix(m);
+    for (auto& m : dCollectionPartitions.all) freeMatrix(m);
     for (auto& m : dInputBatches) freeMatrix(m);
     for (auto& m : dResultScores) freeMatrix(m);
     for (auto& m : dResultIndexes) freeMatrix(m);
     for (auto& m : hResultScores) freeResults(m);
     for (auto& m : hResultIndexes) freeResults(m);
-    for (auto& m : dWorkspaces) freeMatrix(m);
+    for (auto& m : dWorkspaces.all) freeMatrix(m);
 }
 
 Knn::Knn(KnnData* data) : data(data) {}
@@ -336,20 +336,21 @@ void KnnExactGpu::searchDevice(int k, const float* inputs, int size)
         throw std::invalid_argument(msg.str());
     }
     const int device = 0;
-    Matrix& items = data->dCollectionPartitions[device];
+    Matrix& items = data->dCollectionPartitions.all[device];
     Matrix& dIn = data->dInputBatches[device];
     const int D = items.numColumns;
 
     check(dsx_memcpy_h2d(dIn.data, inputs, (size_t)size * D * sizeof(float)), "KnnExactGpu::search");
     float elapsed[2] = {0, 0};
+    const bool kept = data->workspacePrepared[device] != 0 && !data->dCollectionPartitions.handedOut && !data->dWorkspaces.handedOut;
     const int storage = data->dataType == DataType::FP16        ? DSX_KNN_FP16
                         : data->dataType == DataType::FP32Split ? DSX_KNN_SPLIT
-                        : data->workspacePrepared[device]       ? data->workspacePrepared[device]
+                        : kept                                  ? data->workspacePrepared[device]
                                                                 : DSX_KNN_FP32;
     check(dsx_knn_search_host(storage, items.data, items.numRows, data->collectionRowsPadded[device], (uint32_t)D, (const float*)dIn.data,
                               (uint32_t)size, (uint32_t)maxK, (float*)data->dResultScores[device].data, (uint32_t*)data->dResultIndexes[device].data,
                               (float*)data->hResultScores[device].data, (uint32_t*)data->hResultIndexes[device].data,
-                              data->dWorkspaces[device].data, data->dWorkspaces[device].elementSize, elapsed),
+                              data->dWorkspaces.all[device].data, data->dWorkspaces.all[device].elementSize, elapsed),
           "KnnExactGpu::search");
     data->elapsedSgemm[device] = elapsed[0];
     data->elapsedTopK[device] = elapsed[1];
