@@ -186,9 +186,11 @@ void NNLayer::ForwardPropagateFullyConnected(uint32_t position, uint32_t batch, 
         } else if (_kind == Output && _localStride >= kSegMaxMinWidth) {
             // Wide output layer that feeds no other layer: what usually follows is a top-K, which can run together with the layer
             // without the layer's result ever being stored.  The layer is computed when somebody asks for it.
-            // (a narrower one is not put off while a caller holds a pointer through which its operands may change meanwhile)
-            const bool bHeld = _localStride < kDeferMinWidth && (src->_bHandedOut || wsrc->_bHandedOut);
-            if (_bDeferOutput && !bHeld && (TopKScreenPays(batch, 1) || TopKFusionPays(batch, 1)) && !w->_bTransposed && _vOutgoingLayer.empty() && _vOutgoingSkip.empty() &&
+            // (while a caller holds a pointer through which its operands may change meanwhile only a wide one of many rows is put off)
+            const bool bHeld = src->_bHandedOut || wsrc->_bHandedOut;
+            const bool bPays = bHeld ? _localStride >= kDeferMinWidth && dsx_fc_topk_pays(batch, src->_stride, _localStride, (uint32_t)_activation, 1) != 0
+                                     : TopKScreenPays(batch, 1) || TopKFusionPays(batch, 1);
+            if (_bDeferOutput && bPays && !w->_bTransposed && _vOutgoingLayer.empty() && _vOutgoingSkip.empty() &&
                 dsx_fc_topk_supported(src->_stride, src->GetUnitBuffer(), (uint32_t)_activation, &params, NULL)) {
                 if (dsx_fc_topk_flagged_for(wsrc->_pbWeight->_pDevData, 0)) {
                     // rows whose survivor lists filled up (thousands of scores tied at the top), or whose inputs f16 cannot hold, had

@@ -1,4 +1,5 @@
 """Kept tables behind the C++ classes: what a program does between two searches or two top-Ks."""
+import numpy as np
 import pytest
 
 from test_host_gpu import run_exe
@@ -9,3 +10,35 @@ pytestmark = pytest.mark.gpu
 def test_knn_matrices_that_a_program_works_on_itself():
     rc, out = run_exe("test_knn_gpu")
     assert rc == 0 and "0 failed" in out, out[-3000:]
+
+
+def network(synth, host_api, items, hidden, batch, batches=1, k=20):
+    p = synth.autoencoder("kept-%d" % items, 5, items, [hidden], batch, k, batches=batches, zipf_s=1.0, nnz_mean=20, nnz_sigma=0.5, nnz_clip=(1, 200))
+    return p, host_api.Network(p, max_k=k)
+
+
+@pytest.mark.parametrize("items,hidden,batch", [(140000, 256, 8), (27278, 64, 300)])
+def test_units_written_through_a_pointer_after_the_prediction(pkg, dsx, synth, items, hidden, batch):
+    """A program that holds the hidden layer's buffer may write to it at any time after a prediction: the output layer is of the units that were
+    there then."""
+    from amazon_dsstne_amd import host_api
+    p, net = network(synth, host_api, items, hidden, batch)
+    try:
+        net.bind_input()
+        net.set_deferred_output(False)
+        net.predict_batch(0)
+        net.topk(p.k)
+        want, _ = net.get_topk(p.batch)
+        net.set_deferred_output(True)
+        net.set_lanes(1)
+        net.predict_batch(0)
+        ptr = net.unit_buffer("Hidden1")
+        net.predict_batch(0)
+        ones = np.ones((p.batch, hidden), np.float32)
+        pkg.check(dsx.dsx_memcpy_h2d(ptr, ones.ctypes.data, ones.nbytes))
+        net.topk(p.k)
+        got, _ = net.get_topk(p.batch)
+        # sums of up to 256 products below 1 in another order: 1e-5 is far above their roundings
+        assert np.abs(got - want).max() < 1e-5
+    finally:
+        net.close()
