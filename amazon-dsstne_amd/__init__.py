@@ -56,6 +56,7 @@ SIGNATURES = {
     "dsx_malloc_host": [C.POINTER(_vp), _sz],
     "dsx_free": [_vp],
     "dsx_free_host": [_vp],
+    "dsx_host_is_pinned": [_vp, _sz],
     "dsx_memset": [_vp, _int, _sz],
     "dsx_memcpy_h2d": [_vp, _vp, _sz],
     "dsx_memcpy_d2h": [_vp, _vp, _sz],

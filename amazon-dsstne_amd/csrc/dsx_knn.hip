@@ -645,6 +645,9 @@ int dsx_knn_search_host(int storage, const void* items, uint32_t rows_padded, ui
                         void* workspace, size_t workspace_bytes, float* elapsed_ms)
 {
     DSX_CHECK_ARG((host_scores == nullptr) == (host_indexes == nullptr), "dsx_knn_search_host: host_scores and host_indexes go together");
+    const size_t host_bytes = (size_t)num_queries * k * sizeof(float);
+    DSX_CHECK_ARG(!host_scores || host_bytes == 0 || (dsx_host_is_pinned(host_scores, host_bytes) && dsx_host_is_pinned(host_indexes, host_bytes)),
+                  "dsx_knn_search_host: the device cannot write to the host memory for %u x %u results", num_queries, k);
     const bool built = storage == DSX_KNN_FP32_PREPARED || storage == DSX_KNN_FP32_PREPARED_EVEN;
     DSX_CHECK_ARG(!built || workspace, "dsx_knn_search_host: no prepared workspace");
     const KnnResults out{scores, indexes, host_scores, host_indexes};

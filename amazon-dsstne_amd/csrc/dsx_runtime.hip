@@ -461,6 +461,26 @@ int dsx_free(void* p)
 
 int dsx_free_host(void* p) { return dsx_free(p); }
 
+int dsx_host_is_pinned(const void* p, size_t bytes)
+{
+    if (!ctx().initialized || !p) return 0;
+    {
+        std::lock_guard<std::mutex> lock(g_alloc_mutex);
+        auto after = g_host_allocs.upper_bound(const_cast<void*>(p));
+        if (after != g_host_allocs.begin()) {
+            const auto& block = *std::prev(after);
+            const size_t offset = (size_t)((const char*)p - (const char*)block.first);
+            if (offset <= block.second && bytes <= block.second - offset) return 1;
+        }
+    }
+    hipPointerAttribute_t attributes;
+    if (hipPointerGetAttributes(&attributes, p) != hipSuccess) {
+        (void)hipGetLastError();   // (memory that HIP does not know is no error of the next launch)
+        return 0;
+    }
+    return attributes.type == hipMemoryTypeHost || attributes.type == hipMemoryTypeManaged;
+}
+
 int dsx_memset(void* p, int value, size_t bytes)
 {
     DSX_REQUIRE_INIT();

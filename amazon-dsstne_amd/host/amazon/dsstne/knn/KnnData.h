@@ -95,6 +95,11 @@ struct KnnData {
     void load(const std::map<int, std::string>& deviceToFile, char keyValDelim, char vecDelim);
     int getFeatureSize() const;
     ~KnnData();
+
+private:
+    // the pinned memory that load put into hResultScores and hResultIndexes
+    void* pinnedScores = nullptr;
+    void* pinnedIndexes = nullptr;
 };
 
 Matrix allocateMatrixOnHost(uint32_t numRows, int numColumns, size_t elementSize);

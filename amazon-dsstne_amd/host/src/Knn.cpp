@@ -147,7 +147,7 @@ void freeMatrix(const Matrix& matrix)
     if (matrix.data == nullptr) return;
     if (matrix.memoryType == MemoryType::Device) {
         if (dsx_is_initialized()) check(dsx_free(matrix.data), "freeMatrix");
-    } else {
+    } else if (!dsx_is_initialized() || dsx_free_host(matrix.data) != DSX_OK) {   // (pinned memory, or not from there)
         free(matrix.data);
     }
 }
@@ -163,7 +163,8 @@ Matrix loadDataOnHost(DataReader* dataReader)
     return matrix;
 }
 
-// Result buffers: pinned host memory, which the search's last kernel writes (two copies and their waits less).
+// Result buffers: pinned host memory, which the search's last kernel writes (two copies and their waits less).  A program may put matrices of its
+// own in their place.
 static Matrix allocateResults(uint32_t numRows, int numColumns, size_t elementSize)
 {
     void* data = nullptr;
@@ -172,9 +173,10 @@ static Matrix allocateResults(uint32_t numRows, int numColumns, size_t elementSi
     return Matrix(data, numRows, numColumns, elementSize, MemoryType::Host);
 }
 
-static void freeResults(const Matrix& matrix)
+// made: what allocateResults gave.  (Its memory went with the device if that has been shut down.)
+static void freeResults(const Matrix& matrix, const void* made)
 {
-    if (matrix.data != nullptr && dsx_is_initialized()) check(dsx_free(matrix.data), "freeResults");
+    if (matrix.data != made || dsx_is_initialized()) freeMatrix(matrix);
 }
 
 KnnData::KnnData(int numGpus, int batchSize, int maxK, DataType dataType)
@@ -216,8 +218,8 @@ void KnnData::load(int device, DataReader* dataReader)
     freeMatrix(dInputBatches[device]);
     freeMatrix(dResultScores[device]);
     freeMatrix(dResultIndexes[device]);
-    freeResults(hResultScores[device]);
-    freeResults(hResultIndexes[device]);
+    freeResults(hResultScores[device], pinnedScores);
+    freeResults(hResultIndexes[device], pinnedIndexes);
     freeMatrix(dWorkspaces.all[device]);
     if (dataType == DataType::FP16) {
         // knn/KnnData.cpp:209-216: the table is kept as halves (round to nearest even); the fp32 copy only lives until it is
@@ -252,6 +254,8 @@ void KnnData::load(int device, DataReader* dataReader)
     dResultIndexes[device] = allocateMatrixOnDevice(batchSize, maxK, sizeof(uint32_t));
     hResultScores[device] = allocateResults(batchSize, maxK, sizeof(float));
     hResultIndexes[device] = allocateResults(batchSize, maxK, sizeof(uint32_t));
+    pinnedScores = hResultScores[device].data;
+    pinnedIndexes = hResultIndexes[device].data;
     const size_t ws = dataType == DataType::FP16        ? dsx_knn_workspace_bytes_f16(rows, columns, batchSize, maxK)
                       : dataType == DataType::FP32Split ? dsx_knn_workspace_bytes_split(rows, columns, batchSize, maxK)
                                                         : dsx_knn_workspace_bytes_prepared(rows, columns, batchSize, maxK);
@@ -311,8 +315,8 @@ KnnData::~KnnData()
     for (auto& m : dInputBatches) freeMatrix(m);
     for (auto& m : dResultScores) freeMatrix(m);
     for (auto& m : dResultIndexes) freeMatrix(m);
-    for (auto& m : hResultScores) freeResults(m);
-    for (auto& m : hResultIndexes) freeResults(m);
+    for (auto& m : hResultScores) freeResults(m, pinnedScores);
+    for (auto& m : hResultIndexes) freeResults(m, pinnedIndexes);
     for (auto& m : dWorkspaces.all) freeMatrix(m);
 }
 
@@ -347,13 +351,19 @@ void KnnExactGpu::searchDevice(int k, const float* inputs, int size)
                         : data->dataType == DataType::FP32Split ? DSX_KNN_SPLIT
                         : kept                                  ? data->workspacePrepared[device]
                                                                 : DSX_KNN_FP32;
+    void *dScores = data->dResultScores[device].data, *dIndexes = data->dResultIndexes[device].data;
+    void *hScores = data->hResultScores[device].data, *hIndexes = data->hResultIndexes[device].data;
+    const size_t bytes = (size_t)size * maxK * sizeof(float);   // of the scores, and of the indexes
+    const bool pinned = dsx_host_is_pinned(hScores, bytes) && dsx_host_is_pinned(hIndexes, bytes);
     check(dsx_knn_search_host(storage, items.data, items.numRows, data->collectionRowsPadded[device], (uint32_t)D, (const float*)dIn.data,
-                              (uint32_t)size, (uint32_t)maxK, (float*)data->dResultScores[device].data, (uint32_t*)data->dResultIndexes[device].data,
-                              (float*)data->hResultScores[device].data, (uint32_t*)data->hResultIndexes[device].data,
-                              data->dWorkspaces.all[device].data, data->dWorkspaces.all[device].elementSize, elapsed),
+                              (uint32_t)size, (uint32_t)maxK, (float*)dScores, (uint32_t*)dIndexes, pinned ? (float*)hScores : nullptr,
+                              pinned ? (uint32_t*)hIndexes : nullptr, data->dWorkspaces.all[device].data, data->dWorkspaces.all[device].elementSize, elapsed),
           "KnnExactGpu::search");
     data->elapsedSgemm[device] = elapsed[0];
     data->elapsedTopK[device] = elapsed[1];
+    if (pinned) return;
+    check(dsx_memcpy_d2h(hScores, dScores, bytes), "KnnExactGpu::search");
+    check(dsx_memcpy_d2h(hIndexes, dIndexes, bytes), "KnnExactGpu::search");
 }
 
 void KnnExactGpu::search(int k, const float* inputs, int size, std::string* keys, float* scores)

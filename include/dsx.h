@@ -113,6 +113,8 @@ int dsx_malloc_managed(void** ptr, size_t bytes);
 int dsx_malloc_host(void** host_ptr, size_t bytes);
 int dsx_free(void* device_ptr);
 int dsx_free_host(void* host_ptr);
+/* 1 if the device can write to these bytes of host memory: dsx_malloc_host's, dsx_malloc_managed's, or pinned by another call of HIP. */
+int dsx_host_is_pinned(const void* host_ptr, size_t bytes);
 int dsx_memset(void* device_ptr, int value, size_t bytes);
 /* GpuBuffer::Upload.  host_src may be reused as soon as the call returns; the copy itself is ordered on the library's stream
  * before everything queued later (uploads of up to 4 MiB are staged in pinned memory and not waited for). */
@@ -367,7 +369,7 @@ size_t dsx_knn_workspace_bytes_prepared(uint32_t rows_padded, uint32_t dim, uint
 int dsx_knn_prepare(const float* items, uint32_t rows_padded, uint32_t padding, uint32_t dim, uint32_t num_queries, uint32_t k, void* workspace,
                     size_t workspace_bytes, int* prepared);
 /* dsx_knn_search, _f16 or _split (storage; items and workspace as these take them) whose last kernel writes the results into host memory
- * too (dsx_malloc_host; both NULL: device only). */
+ * too (dsx_host_is_pinned; other memory is refused; both NULL: device only). */
 #define DSX_KNN_FP32 0
 #define DSX_KNN_FP16 1
 #define DSX_KNN_SPLIT 2

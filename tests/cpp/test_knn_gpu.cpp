@@ -95,5 +95,35 @@ int main()
         CHECK_EQ(dsx_memcpy_h2d(spaces[0].data, numbersToo.data(), numbersToo.size() * sizeof(float)), DSX_OK);
         CHECK(finds(data, items, queries));
     }
+    printf("result buffers of the program's own\n");
+    fflush(stdout);
+    {
+        KnnData data(1, BATCH, K, DataType::FP32);
+        ArrayDataReader reader(items.data(), ROWS, DIM);
+        data.load(0, &reader);
+        freeMatrix(data.hResultScores[0]);
+        data.hResultScores[0] = allocateMatrixOnHost(BATCH, K, sizeof(float));
+        CHECK_EQ(dsx_host_is_pinned(data.hResultScores[0].data, BATCH * K * sizeof(float)), 0);
+        CHECK(finds(data, items, queries));
+        Matrix before = data.hResultIndexes[0];
+        CHECK_EQ(dsx_host_is_pinned(before.data, BATCH * K * sizeof(float)), 1);
+        data.hResultIndexes[0] = allocateMatrixOnHost(BATCH, K, sizeof(uint32_t));
+        CHECK(finds(data, items, queries));
+        CHECK_EQ(((uint32_t*)data.hResultIndexes[0].data)[BATCH * K - 1] < ROWS, true);
+        // the call itself refuses what the device cannot write to
+        CHECK_EQ(dsx_knn_search_host(DSX_KNN_FP32, data.dCollectionPartitions[0].data, padded, padded - ROWS, DIM, (const float*)data.dInputBatches[0].data, BATCH, K,
+                                     (float*)data.dResultScores[0].data, (uint32_t*)data.dResultIndexes[0].data, (float*)data.hResultScores[0].data,
+                                     (uint32_t*)data.hResultIndexes[0].data, nullptr, 0, nullptr),
+                 DSX_EINVAL);
+        freeMatrix(before);
+    }
+    printf("tables that outlive the device\n");
+    fflush(stdout);
+    {
+        KnnData data(1, BATCH, K, DataType::FP32);
+        ArrayDataReader reader(items.data(), ROWS, DIM);
+        data.load(0, &reader);
+        while (dsx_is_initialized()) dsx_shutdown();
+    }
     return finish("test_knn_gpu");
 }
