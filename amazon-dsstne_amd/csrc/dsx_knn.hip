@@ -184,6 +184,7 @@ struct KnnTimer {
     int mark(hipStream_t s)
     {
         hipEvent_t e = nullptr;
+        if (ctx().knobs.knn_no_events) return set_error(DSX_EHIP, "KnnTimer: no events");
         DSX_HIP(hipEventCreate(&e));
         marks.push_back(e);
         DSX_HIP(hipEventRecord(e, s));
@@ -401,6 +402,12 @@ int dsx_testing_set_screen(int mode)
     return DSX_OK;
 }
 
+int dsx_testing_set_knn_no_events(int none)
+{
+    ctx().knobs.knn_no_events = none;
+    return DSX_OK;
+}
+
 int dsx_knn_last_search_path(void) { return g_knn_last_path; }
 
 int dsx_testing_set_knn_f16_sweep(int mode)
@@ -526,8 +533,8 @@ static int knn_search_common(KnnOperands& op, uint32_t padding, uint32_t num_que
         elapsed_ms[0] = t.gemm;
         elapsed_ms[1] = t.topk;
     }
-    // the results are complete when the call returns (the other ways have waited by now)
-    if (rc == DSX_OK && redo && !elapsed_ms && capturing == hipStreamCaptureStatusNone) DSX_HIP(hipStreamSynchronize(s));
+    // the results are complete when the call returns (the other ways have waited by now, and nothing is left to wait for where the times were taken)
+    if (rc == DSX_OK && redo && capturing == hipStreamCaptureStatusNone) DSX_HIP(hipStreamSynchronize(s));
     return rc;
 }
 

@@ -182,3 +182,30 @@ def test_large_batches_of_narrow_tables(pkg, dsx, rng):
     rs, ri = best(y, k)
     assert np.array_equal(scores.numpy()[looked_at], rs)
     assert not (idx.numpy()[looked_at] != ri)[rs != 0].any()
+
+
+def test_results_are_complete_without_events(pkg, dsx, rng):
+    """The call returns with its results in host memory whether or not its stages can be timed."""
+    n, dim, queries, k = 60000, 256, 2048, 100
+    items = rng.integers(-3, 4, size=(n, dim)).astype(np.float32)
+    q = rng.integers(-3, 4, size=(queries, dim)).astype(np.float32)
+    dI, dQ = dev(pkg, np.ascontiguousarray(items.T)), dev(pkg, q)
+    scores, idx = pkg.DeviceArray((queries, k), np.float32), pkg.DeviceArray((queries, k), np.uint32)
+    host, elapsed = C.c_void_p(), (C.c_float * 2)()
+    pkg.check(dsx.dsx_malloc_host(C.byref(host), 8 * queries * k))
+    pkg.check(dsx.dsx_testing_set_screen(2))
+    try:
+        for none in (0, 1):
+            pkg.check(dsx.dsx_testing_set_knn_no_events(none))
+            C.memset(host, 0, 8 * queries * k)
+            pkg.check(dsx.dsx_knn_search_host(0, dI.ptr, n, 0, dim, dQ.ptr, queries, k, scores.ptr, idx.ptr, host.value, host.value + 4 * queries * k, None,
+                                              0, elapsed))
+            words = np.ctypeslib.as_array(C.cast(host, C.POINTER(C.c_uint32)), (2, queries, k)).copy()
+            assert dsx.dsx_knn_last_search_path() == 0
+            assert np.array_equal(words[0].view(np.float32), scores.numpy()) and np.array_equal(words[1], idx.numpy()), "events: %d" % (1 - none)
+        looked_at = rng.integers(0, queries, 50)
+        rs, ri = best(q[looked_at] @ items.T, k)
+        assert np.array_equal(words[0].view(np.float32)[looked_at], rs) and np.array_equal(words[1][looked_at], ri)
+    finally:
+        dsx.dsx_testing_reset()
+        dsx.dsx_free(host)
