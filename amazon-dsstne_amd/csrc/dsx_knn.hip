@@ -625,8 +625,7 @@ int dsx_knn_prepare(const float* items, uint32_t rows_padded, uint32_t padding, 
 {
     DSX_REQUIRE_INIT();
     DSX_CHECK_ARG(items && workspace && prepared, "dsx_knn_prepare: null pointer");
-    DSX_CHECK_ARG(padding < rows_padded && dim > 0 && num_queries > 0 && k >= 1 && k <= 256, "dsx_knn_prepare: rows_padded %u, padding %u, dim %u, %u queries, k = %u",
-                  rows_padded, padding, dim, num_queries, k);
+    DSX_CHECK_ARG(padding < rows_padded && k >= 1 && k <= 256, "dsx_knn_prepare: rows_padded %u, padding %u, k = %u", rows_padded, padding, k);
     DSX_CHECK_ARG(((uintptr_t)workspace % 256) == 0, "dsx_knn_prepare: workspace is not 256-byte aligned");
     *prepared = 0;
     if (!knn_prepares(rows_padded, dim, num_queries, k) || workspace_bytes < dsx_knn_workspace_bytes_prepared(rows_padded, dim, num_queries, k)) return DSX_OK;

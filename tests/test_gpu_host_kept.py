@@ -42,3 +42,15 @@ def test_units_written_through_a_pointer_after_the_prediction(pkg, dsx, synth, i
         assert np.abs(got - want).max() < 1e-5
     finally:
         net.close()
+
+
+def test_vectors_without_components(pkg, dsx):
+    """Loading takes what it took before there were kept tables."""
+    from amazon_dsstne_amd import host_api
+    lib = host_api.load_host_library()
+    items = np.ones((9000, 32), np.float32)
+    knn = lib.dsstne_knn_create(4, 5)
+    try:
+        assert lib.dsstne_knn_load(knn, items.ctypes.data, 9000, 0, None) == 0, lib.dsstne_last_error()
+    finally:
+        lib.dsstne_knn_destroy(knn)
