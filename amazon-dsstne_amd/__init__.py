@@ -122,6 +122,7 @@ SIGNATURES = {
     "dsx_knn_prepare": [_vp, _u32, _u32, _u32, _u32, _u32, _vp, _sz, C.POINTER(_int)],
     "dsx_knn_search_host": [_int, _vp, _u32, _u32, _u32, _vp, _u32, _u32, _vp, _vp, _vp, _vp, _vp, _sz, C.POINTER(_f32)],
     "dsx_knn_last_search_path": [],
+    "dsx_knn_last_search_repeated": [],
     "dsx_testing_set_knn_f16_sweep": [_int],
 }
 SPECIAL_RESTYPES = {"dsx_last_error": C.c_char_p, "dsx_stream": C.c_void_p, "dsx_knn_workspace_bytes": C.c_size_t,

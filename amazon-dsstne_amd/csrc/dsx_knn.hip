@@ -23,6 +23,7 @@ namespace dsx {
 static LibScratch g_knn_ws_of[DSX_MAX_LANES];   // per lane
 
 static int g_knn_last_path = 0;            // how the last search ran: DSX_KNN_PATH_*
+static bool g_knn_last_repeated = false;   // it was screened for nothing
 
 static uint32_t knn_block_columns(uint32_t rows_padded, uint32_t num_queries)
 {
@@ -410,6 +411,8 @@ int dsx_testing_set_knn_no_events(int none)
 
 int dsx_knn_last_search_path(void) { return g_knn_last_path; }
 
+int dsx_knn_last_search_repeated(void) { return g_knn_last_repeated ? 1 : 0; }
+
 int dsx_testing_set_knn_f16_sweep(int mode)
 {
     DSX_CHECK_ARG(mode >= 0 && mode <= 3, "dsx_testing_set_knn_f16_sweep: mode %d (0 to 3)", mode);
@@ -469,12 +472,14 @@ int dsx_knn_f16_convert_items(const float* items, uint32_t rows_padded, uint32_t
 
 }  // extern "C"
 
-// Both precisions: workspace, the two paths, timing.
+// Both precisions: workspace, the two paths, timing.  screening: whether candidates may be screened; table: the workspace holds a prepared table, which
+// screening uses and everything else leaves as it is.
 static int knn_search_common(KnnOperands& op, uint32_t padding, uint32_t num_queries, uint32_t k, const KnnResults& out, void* workspace,
-                             size_t workspace_bytes, float* elapsed_ms, bool aligned, const float* queries_f32, bool built = false, bool even = false)
+                             size_t workspace_bytes, float* elapsed_ms, bool aligned, const float* queries_f32, bool screening = false, bool table = false, bool even = false)
 {
-    const size_t full = knn_layout(nullptr, op.rows_padded, num_queries, k, op.f16, op.dim, op.split, true, built).bytes;
-    const size_t need = knn_layout(nullptr, op.rows_padded, num_queries, k, op.f16, op.dim, op.split, false, built).bytes;
+    const bool built = screening && table;
+    const size_t full = knn_layout(nullptr, op.rows_padded, num_queries, k, op.f16, op.dim, op.split, screening, table).bytes;
+    const size_t need = knn_layout(nullptr, op.rows_padded, num_queries, k, op.f16, op.dim, op.split, false, table).bytes;
     bool screen = full != need;   // the screening's copies of the table (up to 8 GiB) where there is room for them: fp32 needs none
     if (workspace) {
         DSX_CHECK_ARG(workspace_bytes >= need, "dsx_knn_search: workspace of %zu bytes, %zu needed", workspace_bytes, need);
@@ -490,7 +495,7 @@ static int knn_search_common(KnnOperands& op, uint32_t padding, uint32_t num_que
         if (reserved) return reserved;
         workspace = ws.ptr;
     }
-    const KnnWorkspace w = knn_layout(workspace, op.rows_padded, num_queries, k, op.f16, op.dim, op.split, screen, built);
+    const KnnWorkspace w = knn_layout(workspace, op.rows_padded, num_queries, k, op.f16, op.dim, op.split, screen, table);
     const uint32_t M = op.rows_padded - padding;
     hipStream_t s = ctx().stream;
     KnnTimer t;
@@ -523,6 +528,7 @@ static int knn_search_common(KnnOperands& op, uint32_t padding, uint32_t num_que
     bool redo = true, unfit = false;
     if (rc == DSX_OK && screened) rc = knn_search_screened(w, op, M, num_queries, k, out, t, built, even, &redo, &unfit);
     if (unfit) screened = false;
+    g_knn_last_repeated = screened && redo;
     const bool candidates = screened || (may && many);
     if (rc == DSX_OK && may && (!screened || redo) && many)
         rc = knn_search_candidates(w, op, M, num_queries, k, out, t, &redo);
@@ -539,7 +545,8 @@ static int knn_search_common(KnnOperands& op, uint32_t padding, uint32_t num_que
 }
 
 static int knn_search_fp32(const float* items, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,
-                           uint32_t num_queries, uint32_t k, const KnnResults& out, void* workspace, size_t workspace_bytes, float* elapsed_ms, bool built, bool even)
+                           uint32_t num_queries, uint32_t k, const KnnResults& out, void* workspace, size_t workspace_bytes, float* elapsed_ms,
+                           bool screening, bool table, bool even)
 {
     DSX_REQUIRE_INIT();
     DSX_CHECK_ARG(items && queries && out.scores && out.indexes, "dsx_knn_search: null device pointer");
@@ -553,7 +560,7 @@ static int knn_search_fp32(const float* items, uint32_t rows_padded, uint32_t pa
     op.rows_padded = rows_padded;
     op.dim = dim;
     const bool aligned = ((uintptr_t)items % 16) == 0 && ((uintptr_t)queries % 16) == 0 && (rows_padded % 4) == 0 && (dim % 4) == 0;
-    return knn_search_common(op, padding, num_queries, k, out, workspace, workspace_bytes, elapsed_ms, aligned, nullptr, built, even);
+    return knn_search_common(op, padding, num_queries, k, out, workspace, workspace_bytes, elapsed_ms, aligned, nullptr, screening, table, even);
 }
 
 static int knn_search_split(const void* item_planes, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,
@@ -601,7 +608,7 @@ int dsx_knn_search(const float* items, uint32_t rows_padded, uint32_t padding, u
                    float* elapsed_ms)
 {
     return knn_search_fp32(items, rows_padded, padding, dim, queries, num_queries, k, KnnResults{scores, indexes, nullptr, nullptr}, workspace,
-                           workspace_bytes, elapsed_ms, false, false);
+                           workspace_bytes, elapsed_ms, true, false, false);
 }
 
 int dsx_knn_search_split(const void* item_planes, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,
@@ -654,15 +661,16 @@ int dsx_knn_search_host(int storage, const void* items, uint32_t rows_padded, ui
     const size_t host_bytes = (size_t)num_queries * k * sizeof(float);
     DSX_CHECK_ARG(!host_scores || host_bytes == 0 || (dsx_host_is_pinned(host_scores, host_bytes) && dsx_host_is_pinned(host_indexes, host_bytes)),
                   "dsx_knn_search_host: the device cannot write to the host memory for %u x %u results", num_queries, k);
-    const bool built = storage == DSX_KNN_FP32_PREPARED || storage == DSX_KNN_FP32_PREPARED_EVEN;
-    DSX_CHECK_ARG(!built || workspace, "dsx_knn_search_host: no prepared workspace");
+    const bool table = storage == DSX_KNN_FP32_PREPARED || storage == DSX_KNN_FP32_PREPARED_EVEN || storage == DSX_KNN_FP32_PREPARED_UNSCREENED;
+    DSX_CHECK_ARG(!table || workspace, "dsx_knn_search_host: no prepared workspace");
     const KnnResults out{scores, indexes, host_scores, host_indexes};
     switch (storage) {
     case DSX_KNN_FP32:
+    case DSX_KNN_FP32_PREPARED_UNSCREENED:
     case DSX_KNN_FP32_PREPARED:
     case DSX_KNN_FP32_PREPARED_EVEN:
         return knn_search_fp32((const float*)items, rows_padded, padding, dim, queries, num_queries, k, out, workspace, workspace_bytes, elapsed_ms,
-                               built, storage == DSX_KNN_FP32_PREPARED_EVEN);
+                               storage != DSX_KNN_FP32_PREPARED_UNSCREENED, table, storage == DSX_KNN_FP32_PREPARED_EVEN);
     case DSX_KNN_FP16: return knn_search_f16(items, rows_padded, padding, dim, queries, num_queries, k, out, workspace, workspace_bytes, elapsed_ms);
     case DSX_KNN_SPLIT: return knn_search_split(items, rows_padded, padding, dim, queries, num_queries, k, out, workspace, workspace_bytes, elapsed_ms);
     default: return set_error(DSX_EINVAL, "dsx_knn_search_host: storage %d", storage);

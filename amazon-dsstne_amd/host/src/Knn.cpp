@@ -256,6 +256,7 @@ void KnnData::load(int device, DataReader* dataReader)
     hResultIndexes[device] = allocateResults(batchSize, maxK, sizeof(uint32_t));
     pinnedScores = hResultScores[device].data;
     pinnedIndexes = hResultIndexes[device].data;
+    unscreened = unscreenedNext = 0;
     const size_t ws = dataType == DataType::FP16        ? dsx_knn_workspace_bytes_f16(rows, columns, batchSize, maxK)
                       : dataType == DataType::FP32Split ? dsx_knn_workspace_bytes_split(rows, columns, batchSize, maxK)
                                                         : dsx_knn_workspace_bytes_prepared(rows, columns, batchSize, maxK);
@@ -349,6 +350,7 @@ void KnnExactGpu::searchDevice(int k, const float* inputs, int size)
     const bool kept = data->workspacePrepared[device] != 0 && !data->dCollectionPartitions.handedOut && !data->dWorkspaces.handedOut;
     const int storage = data->dataType == DataType::FP16        ? DSX_KNN_FP16
                         : data->dataType == DataType::FP32Split ? DSX_KNN_SPLIT
+                        : kept && data->unscreened != 0         ? DSX_KNN_FP32_PREPARED_UNSCREENED
                         : kept                                  ? data->workspacePrepared[device]
                                                                 : DSX_KNN_FP32;
     void *dScores = data->dResultScores[device].data, *dIndexes = data->dResultIndexes[device].data;
@@ -361,6 +363,12 @@ void KnnExactGpu::searchDevice(int k, const float* inputs, int size)
           "KnnExactGpu::search");
     data->elapsedSgemm[device] = elapsed[0];
     data->elapsedTopK[device] = elapsed[1];
+    if (kept && data->unscreened != 0)
+        data->unscreened--;
+    else if (kept) {
+        data->unscreenedNext = dsx_knn_last_search_repeated() ? std::min(64u, std::max(1u, 2 * data->unscreenedNext)) : data->unscreenedNext / 2;
+        if (dsx_knn_last_search_repeated()) data->unscreened = data->unscreenedNext;
+    }
     if (pinned) return;
     check(dsx_memcpy_d2h(hScores, dScores, bytes), "KnnExactGpu::search");
     check(dsx_memcpy_d2h(hIndexes, dIndexes, bytes), "KnnExactGpu::search");

@@ -375,6 +375,7 @@ int dsx_knn_prepare(const float* items, uint32_t rows_padded, uint32_t padding, 
 #define DSX_KNN_SPLIT 2
 #define DSX_KNN_FP32_PREPARED 3
 #define DSX_KNN_FP32_PREPARED_EVEN 4   /* the items' norms lie close together */
+#define DSX_KNN_FP32_PREPARED_UNSCREENED 5   /* a prepared workspace, whose copies are left alone: searched without screening */
 int dsx_knn_search_host(int storage, const void* items, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,
                         uint32_t num_queries, uint32_t k, float* scores, uint32_t* indexes, float* host_scores, uint32_t* host_indexes,
                         void* workspace, size_t workspace_bytes, float* elapsed_ms);
@@ -405,6 +406,9 @@ size_t dsx_knn_workspace_bytes_split(uint32_t rows_padded, uint32_t dim, uint32_
 #define DSX_KNN_PATH_CANDIDATES 1         /* first block as above, then candidate lists */
 #define DSX_KNN_PATH_CANDIDATES_REDONE 2  /* a candidate list filled up: repeated block by block */
 int dsx_knn_last_search_path(void);
+/* 1 if the last search was screened in 16 bits and found rows that cannot be (thousands of ties, norms beyond f16's range), so that it was repeated
+ * without: a caller with more such queries is better off with DSX_KNN_FP32_PREPARED_UNSCREENED. */
+int dsx_knn_last_search_repeated(void);
 /* dsx_knn_search_f16 scores the column ranges after the first block one workgroup per tile, or, when a range has enough item
  * tiles, with workgroups that keep their queries and walk a chunk of the range each (private candidate lists, no atomics on
  * device memory): the queries in registers when the vectors have at most 256 components, 128 queries per workgroup staged

@@ -54,3 +54,38 @@ def test_vectors_without_components(pkg, dsx):
         assert lib.dsstne_knn_load(knn, items.ctypes.data, 9000, 0, None) == 0, lib.dsstne_last_error()
     finally:
         lib.dsstne_knn_destroy(knn)
+
+
+@pytest.mark.parametrize("n,batch", [(20000, 32), (500000, 600)])
+def test_tables_full_of_ties_stop_being_screened(pkg, dsx, rng, n, batch):
+    """10,000 copies of one item: every search that wants it would be screened and done again.  Few are; other queries are screened as before."""
+    from amazon_dsstne_amd import host_api
+    lib = host_api.load_host_library()
+    dim, k = 32, 10
+    items = rng.integers(-3, 4, size=(n, dim)).astype(np.float32)
+    items[5000:15000] = 3.0
+    tied = np.ones((batch, dim), np.float32)
+    apart = np.repeat(items[:1], batch, axis=0) * 2
+    knn = lib.dsstne_knn_create(batch, k)
+    try:
+        assert lib.dsstne_knn_load(knn, items.ctypes.data, n, dim, None) == 0
+        scores, idx = np.empty((batch, k), np.float32), np.empty((batch, k), np.uint32)
+        best = {id(q): np.argsort(-(items @ q[0]), kind="stable")[:k] for q in (tied, apart)}
+
+        def search(q):
+            """Whether it was screened for nothing, and whether it was not screened at all."""
+            assert lib.dsstne_knn_search(knn, k, q.ctypes.data, batch, scores.ctypes.data, idx.ctypes.data) == 0
+            order = best[id(q)]
+            assert np.array_equal(idx, np.repeat(order[None], batch, axis=0)) and np.array_equal(scores[0], items[order] @ q[0])
+            return dsx.dsx_knn_last_search_repeated()
+
+        assert search(apart) == 0
+        assert sum(search(tied) for _ in range(200)) <= 9
+        # one in a batch is enough
+        assert sum(search(apart) for _ in range(70)) == 0
+        mixed = apart.copy()
+        mixed[batch - 1] = 1.0
+        assert lib.dsstne_knn_search(knn, k, mixed.ctypes.data, batch, scores.ctypes.data, idx.ctypes.data) == 0
+        assert dsx.dsx_knn_last_search_repeated() == 1 and np.array_equal(idx[batch - 1], best[id(tied)]) and np.array_equal(idx[0], best[id(apart)])
+    finally:
+        lib.dsstne_knn_destroy(knn)
