@@ -97,6 +97,9 @@ private:
     // The weights' table, where the layer and a top-K of k entries are fastest screened by it (else NULL).
     bool TopKScreenPays(uint32_t batch, uint32_t k);
     const void* TopKScreenTable(uint32_t batch, uint32_t k);
+    void PrepareTopK(uint32_t batch, uint32_t k);
+    // Whether the layer may be put off for its top-K at all, whatever is the faster way.
+    bool MayDefer();
     // Whether the deferred layer's top-K has been computed; a narrower layer whose units are asked for all the same is stored from then on.
     bool _bToppedDeferred = false;
     bool UseSplitProducts(uint32_t batch) const

@@ -83,6 +83,9 @@ public:
     // but together with the CalculateTopK / CalculateFilteredTopK that follows, without storing its result; GetUnitBuffer and
     // GetUnits compute it on demand.  SetDeferredOutput(false) makes PredictBatch store every layer, as the reference does.
     bool SetDeferredOutput(bool bDefer);
+    // No counterpart in the reference.  Says that top-Ks of up to k entries of the output layers are to come: what a layer's top-K is fastest with and
+    // its weights alone decide (NNWeight::ScreenTable) is made now, and not by the first of them.
+    void PrepareTopK(uint32_t k);
     // No counterpart in the reference.  SetSplitProducts(true): dense layers wide enough for the tiled kernel (at least two
     // 128 x 128 tiles per compute unit) form every fp32 product from six bf16 matrix instructions (dsx_fc_forward_split): sums as
     // close to the exact ones as fp32 multiplication gives, not bit-identical to it, about 1.5 times as fast; the weights of those

@@ -35,6 +35,7 @@ DsstneContext::DsstneContext(const string& networkFilename, uint32_t batchSize, 
             }
         }
     }
+    if (maxK != ALL) network->PrepareTopK((uint32_t)maxK);
 }
 
 // The buffers of the batch predicted last (the network's current lane).

@@ -153,6 +153,22 @@ const void* NNLayer::TopKScreenTable(uint32_t batch, uint32_t k)
     return TopKScreenPays(batch, k) ? (w->_bShared ? w->_pSharedWeight : w)->ScreenTable(_vIncomingLayer[0]->_stride, _localStride) : NULL;
 }
 
+bool NNLayer::MayDefer()
+{
+    if (!_bDeferOutput || _kind != Output || _vIncomingLayer.size() != 1 || !_vIncomingSkip.empty() || !_vOutgoingLayer.empty() || !_vOutgoingSkip.empty() ||
+        _vIncomingWeight[0]->_bTransposed)
+        return false;
+    const dsx_act_params params = {_RELUSlope, _ELUAlpha, _SELULambda};
+    NNLayer* src = _vIncomingLayer[0];
+    return dsx_fc_topk_supported(src->_stride, src->_pbUnit ? src->GetUnitBuffer() : NULL, (uint32_t)_activation, &params, NULL) != 0;
+}
+
+// (an input layer may turn out to be sparse once its data is there: its output layer is then no dense one)
+void NNLayer::PrepareTopK(uint32_t batch, uint32_t k)
+{
+    if (_localStride >= kSegMaxMinWidth && MayDefer() && _vIncomingLayer[0]->_kind != Input) TopKScreenTable(batch, k);
+}
+
 bool NNLayer::TopKFusionPays(uint32_t batch, uint32_t k)
 {
     if (TopKScreenTable(batch, k)) return true;
@@ -190,8 +206,7 @@ void NNLayer::ForwardPropagateFullyConnected(uint32_t position, uint32_t batch, 
             const bool bHeld = src->_bHandedOut || wsrc->_bHandedOut;
             const bool bPays = bHeld ? _localStride >= kDeferMinWidth && dsx_fc_topk_pays(batch, src->_stride, _localStride, (uint32_t)_activation, 1) != 0
                                      : TopKScreenPays(batch, 1) || TopKFusionPays(batch, 1);
-            if (_bDeferOutput && bPays && !w->_bTransposed && _vOutgoingLayer.empty() && _vOutgoingSkip.empty() &&
-                dsx_fc_topk_supported(src->_stride, src->GetUnitBuffer(), (uint32_t)_activation, &params, NULL)) {
+            if (bPays && MayDefer()) {
                 if (dsx_fc_topk_flagged_for(wsrc->_pbWeight->_pDevData, 0)) {
                     // rows whose survivor lists filled up (thousands of scores tied at the top), or whose inputs f16 cannot hold, had
                     // to be computed again: such data is served better by the stored layer and the scanning top-K

@@ -361,6 +361,11 @@ bool NNNetwork::SetSplitProducts(bool bSplit)
     return true;
 }
 
+void NNNetwork::PrepareTopK(uint32_t k)
+{
+    for (auto l : _vOutputLayer) l->PrepareTopK(_batch, k);
+}
+
 bool NNNetwork::SetDeferredOutput(bool bDefer)
 {
     for (auto l : _vLayer) {

@@ -56,6 +56,7 @@ static NNDataSetBase* makeSparse(const char* name, uint32_t width, uint32_t exam
 static void makeResultBuffers(dsstne_context* c)
 {
     if (c->maxK <= 0) return;
+    c->network->PrepareTopK((uint32_t)c->maxK);
     vector<const NNLayer*> outs;
     for (auto it = c->network->GetLayers(NNLayer::Kind::Output, outs); it != outs.end(); ++it) {
         for (int lane = 0; lane < DSX_MAX_LANES; lane++) {

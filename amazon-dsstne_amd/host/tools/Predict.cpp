@@ -116,6 +116,7 @@ int main(int argc, char** argv)
         cout << "Error: the network has no layer " << recsGenLayerLabel << endl;
         return 1;
     }
+    pNetwork->PrepareTopK(std::min(topK * NNRecsGenerator::TOPK_SCALAR, 256u));
     NNRecsGenerator* nnRecsGenerator =
         new NNRecsGenerator(pNetwork->GetBatch(), topK, (unsigned int)pNetwork->GetBufferSize(recsGenLayerLabel), recsGenLayerLabel, scoreFormat);
     const auto recsGenerationStart = chrono::steady_clock::now();

@@ -1,4 +1,6 @@
 """Kept tables behind the C++ classes: what a program does between two searches or two top-Ks."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -89,3 +91,24 @@ def test_tables_full_of_ties_stop_being_screened(pkg, dsx, rng, n, batch):
         assert dsx.dsx_knn_last_search_repeated() == 1 and np.array_equal(idx[batch - 1], best[id(tied)]) and np.array_equal(idx[0], best[id(apart)])
     finally:
         lib.dsstne_knn_destroy(knn)
+
+
+def memory(dsx):
+    gpu, cpu = C.c_int(), C.c_int()
+    assert dsx.dsx_get_memory_usage(C.byref(gpu), C.byref(cpu)) == 0
+    return gpu.value << 10
+
+
+def test_the_first_top_k_makes_no_table(pkg, dsx, synth):
+    """The weights' table is there once the input is bound, and not made in the middle of a request."""
+    from amazon_dsstne_amd import host_api
+    p, net = network(synth, host_api, 140000, 256, 8)
+    try:
+        net.bind_input()
+        net.predict_batch(0)
+        before = memory(dsx)
+        net.topk(p.k)
+        net.get_topk(p.batch)
+        assert memory(dsx) - before < 100 << 20      # the table: 217 MB
+    finally:
+        net.close()
