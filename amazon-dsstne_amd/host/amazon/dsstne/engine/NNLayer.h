@@ -92,11 +92,12 @@ private:
     unique_ptr<GpuBuffer<uint32_t>> _pbSplitInput;
     bool _bSplitInputFresh = false;   // the layer before this one wrote the planes of the current batch itself (dsx_fc_forward_planes)
     void* SplitInputBuffer();         // this lane's buffer for them, allocated on first use
-    // Whether the deferred layer and a top-K of k entries are computed in one call (or the layer is stored first).
-    bool TopKFusionPays(uint32_t batch, uint32_t k);
-    // The weights' table, where the layer and a top-K of k entries are fastest screened by it (else NULL).
+    // Whether the deferred layer and a top-K of k entries are computed in one call (or the layer is stored first), and the table it is screened by.
+    // Asked once per top-K.
+    bool TopKFusionPays(uint32_t batch, uint32_t k, const void** ppTable = NULL);
+    // The weights' table, where the layer and a top-K of k entries are fastest screened by it (else NULL; bMake: see NNWeight::ScreenTable).
     bool TopKScreenPays(uint32_t batch, uint32_t k);
-    const void* TopKScreenTable(uint32_t batch, uint32_t k);
+    const void* TopKScreenTable(uint32_t batch, uint32_t k, bool bMake);
     void PrepareTopK(uint32_t batch, uint32_t k);
     // Whether the layer may be put off for its top-K at all, whatever is the faster way.
     bool MayDefer();

@@ -50,12 +50,17 @@ private:
     bool _bSplitValid[2] = {false, false};
     const void* SplitPlanes(bool bTransposed, uint32_t k, uint32_t n);
     // The table of the 16-bit screening (dsx_screen_table_build) of a matrix stored [k][n], for output layers that are computed with
-    // their top-K; kept like the planes.  NULL: there is no room for it (half of what is free), or the caller may change the matrix
-    // (_bHandedOut).
+    // their top-K; kept like the planes.  NULL: there is no room for it (half of what is free), the caller may change the matrix
+    // (_bHandedOut), or it is not there and not made: bMake makes it, and so does the ninth call that would use it since the matrix changed.
     void* _pScreen = NULL;
     bool _bScreenValid = false, _bScreenRefused = false;
-    const void* ScreenTable(uint32_t k, uint32_t n);
-    void InvalidateSplit() { _bSplitValid[0] = _bSplitValid[1] = _bScreenValid = false; }
+    uint32_t _screenAsked = 0;
+    const void* ScreenTable(uint32_t k, uint32_t n, bool bMake);
+    void InvalidateSplit()
+    {
+        _bSplitValid[0] = _bSplitValid[1] = _bScreenValid = false;
+        _screenAsked = 0;
+    }
 
     NNWeight(NNLayer& inputLayer, NNLayer& outputLayer, bool bShared = false, bool bTransposed = false, bool bLocked = false,
              NNFloat maxNorm = 0.0f);

@@ -147,10 +147,10 @@ bool NNLayer::TopKScreenPays(uint32_t batch, uint32_t k)
     return !w->_bTransposed && !UseSplitProducts(batch) && dsx_fc_topk_screened_pays(batch, _vIncomingLayer[0]->_stride, _localStride, (uint32_t)_activation, k) != 0;
 }
 
-const void* NNLayer::TopKScreenTable(uint32_t batch, uint32_t k)
+const void* NNLayer::TopKScreenTable(uint32_t batch, uint32_t k, bool bMake)
 {
     NNWeight* w = _vIncomingWeight[0];
-    return TopKScreenPays(batch, k) ? (w->_bShared ? w->_pSharedWeight : w)->ScreenTable(_vIncomingLayer[0]->_stride, _localStride) : NULL;
+    return TopKScreenPays(batch, k) ? (w->_bShared ? w->_pSharedWeight : w)->ScreenTable(_vIncomingLayer[0]->_stride, _localStride, bMake) : NULL;
 }
 
 bool NNLayer::MayDefer()
@@ -166,12 +166,14 @@ bool NNLayer::MayDefer()
 // (an input layer may turn out to be sparse once its data is there: its output layer is then no dense one)
 void NNLayer::PrepareTopK(uint32_t batch, uint32_t k)
 {
-    if (_localStride >= kSegMaxMinWidth && MayDefer() && _vIncomingLayer[0]->_kind != Input) TopKScreenTable(batch, k);
+    if (_localStride >= kSegMaxMinWidth && MayDefer() && _vIncomingLayer[0]->_kind != Input) TopKScreenTable(batch, k, true);
 }
 
-bool NNLayer::TopKFusionPays(uint32_t batch, uint32_t k)
+bool NNLayer::TopKFusionPays(uint32_t batch, uint32_t k, const void** ppTable)
 {
-    if (TopKScreenTable(batch, k)) return true;
+    const void* pTable = TopKScreenTable(batch, k, false);
+    if (ppTable) *ppTable = pTable;
+    if (pTable) return true;
     if (_localStride < kDeferMinWidth && UseSplitProducts(batch)) return false;
     return dsx_fc_topk_pays(batch, _vIncomingLayer[0]->_stride, _localStride, (uint32_t)_activation, k) != 0;
 }

@@ -311,8 +311,8 @@ bool NNNetwork::SetLanes(uint32_t lanes)
     return true;
 }
 
-// The deferred output layer and its top-K in one call; the layer's result is not stored.
-void NNNetwork::LayerWithTopK(NNLayer* pLayer, uint32_t k, uint32_t batch, const uint32_t* pIndex, const uint64_t* pFilterStart,
+// The deferred output layer and its top-K in one call; the layer's result is not stored.  pTable: what TopKFusionPays gave.
+void NNNetwork::LayerWithTopK(NNLayer* pLayer, const void* pTable, uint32_t k, uint32_t batch, const uint32_t* pIndex, const uint64_t* pFilterStart,
                               const uint64_t* pFilterEnd, const uint32_t* pFilterIndex, NNFloat* pKey, uint32_t* pValue)
 {
     NNLayer* src = pLayer->_vIncomingLayer[0];
@@ -329,7 +329,7 @@ void NNNetwork::LayerWithTopK(NNLayer* pLayer, uint32_t k, uint32_t batch, const
         return;
     }
     pLayer->_bToppedDeferred = true;
-    if (const void* pTable = pLayer->TopKScreenTable(batch, k)) {
+    if (pTable) {
         dsxFatal(dsx_fc_topk_screened(src->GetUnitBuffer(), src->_stride, wsrc->_pbWeight->_pDevData, pTable, w->_pbBias->_pDevData, batch,
                                       src->_stride, pLayer->_localStride, (uint32_t)pLayer->_activation, &params, k, pKey, pValue, _position,
                                       pIndex, pFilterStart, pFilterEnd, pFilterIndex),
@@ -397,9 +397,10 @@ void NNNetwork::CalculateTopK(const string& layer, uint32_t k, GpuBuffer<NNFloat
     }
     uint32_t batch = _batch;
     if (_position + batch > _examples) batch = _examples - _position;
-    if (pLayer->_deferred && !pLayer->TopKFusionPays(batch, k)) pLayer->Materialise();
+    const void* pTable = NULL;
+    if (pLayer->_deferred && !pLayer->TopKFusionPays(batch, k, &pTable)) pLayer->Materialise();
     if (pLayer->_deferred)
-        LayerWithTopK(pLayer, k, batch, NULL, NULL, NULL, NULL, pbKey->_pDevData, pbValue->_pDevData);
+        LayerWithTopK(pLayer, pTable, k, batch, NULL, NULL, NULL, NULL, pbKey->_pDevData, pbValue->_pDevData);
     else if (pLayer->_segWidth != 0 && pLayer->_pbSegMax)
         dsxFatal(dsx_topk_guided(pLayer->_pbUnit->_pDevData, pbKey->_pDevData, pbValue->_pDevData, batch, pLayer->_localStride, k,
                                  pLayer->_pbSegMax->_pDevData, pLayer->_segWidth, 0, NULL, NULL, NULL, NULL, NULL),
@@ -440,8 +441,9 @@ void NNNetwork::CalculateFilteredTopK(const string& layer, uint32_t k, NNDataSet
     pFilter->NoteSparseRead();
     const uint32_t* pIndex = (pFilter->_attributes & NNDataSetEnums::Indexed) ? pFilter->_pbIndex->_pDevData : NULL;
     if (pLayer->_deferred) {
-        if (pMul == NULL && pLayer->TopKFusionPays(batch, k)) {
-            LayerWithTopK(pLayer, k, batch, pIndex, pFilter->_pbSparseStart->_pDevData, pFilter->_pbSparseEnd->_pDevData,
+        const void* pTable = NULL;
+        if (pMul == NULL && pLayer->TopKFusionPays(batch, k, &pTable)) {
+            LayerWithTopK(pLayer, pTable, k, batch, pIndex, pFilter->_pbSparseStart->_pDevData, pFilter->_pbSparseEnd->_pDevData,
                           pFilter->_pbSparseIndex->_pDevData, pbKey->_pDevData, pbValue->_pDevData);
             return;
         }
@@ -471,8 +473,9 @@ void NNNetwork::CalculateFilteredTopK(const string& layer, uint32_t k, const uin
     uint32_t batch = _batch;
     if (_position + batch > _examples) batch = _examples - _position;
     if (pLayer->_deferred) {
-        if (pFilterMul == NULL && pLayer->TopKFusionPays(batch, k)) {
-            LayerWithTopK(pLayer, k, batch, NULL, pFilterStart, pFilterEnd, pFilterIndex, pKey, pValue);
+        const void* pTable = NULL;
+        if (pFilterMul == NULL && pLayer->TopKFusionPays(batch, k, &pTable)) {
+            LayerWithTopK(pLayer, pTable, k, batch, NULL, pFilterStart, pFilterEnd, pFilterIndex, pKey, pValue);
             return;
         }
         pLayer->Materialise();

@@ -112,3 +112,36 @@ def test_the_first_top_k_makes_no_table(pkg, dsx, synth):
         assert memory(dsx) - before < 100 << 20      # the table: 217 MB
     finally:
         net.close()
+
+
+@pytest.mark.parametrize("items,hidden,batch", [(140000, 256, 8), (27278, 128, 300)])
+def test_weights_set_between_two_top_ks(pkg, dsx, synth, items, hidden, batch):
+    """Every top-K is of the weights there are, whatever table is kept; and a table of new weights is made when they have stayed for a few of them,
+    the top-Ks before being those of the stored layer, bit for bit."""
+    from amazon_dsstne_amd import host_api
+    p, net = network(synth, host_api, items, hidden, batch)
+    stored = host_api.Network(p, max_k=p.k)
+    rng = np.random.default_rng(8)
+
+    def topk(n):
+        n.predict_batch(0)
+        n.topk(p.k)
+        return n.get_topk(p.batch)[0]
+    try:
+        net.bind_input()
+        stored.bind_input()
+        stored.set_deferred_output(False)
+        for change in range(4):
+            if change:
+                w = rng.permutation(p.weights[1])
+                net.set_weights("Hidden1", "Output", weights=w)
+                stored.set_weights("Hidden1", "Output", weights=w)
+            want = topk(stored)
+            got = [topk(net) for _ in range(12 if change < 3 else 2)]
+            # sums of up to 256 products below 1 in another order: 1e-5 is far above their roundings
+            assert max(np.abs(g - want).max() for g in got) < 1e-5
+            assert np.array_equal(got[0], want) == (change > 0)
+            assert not (change < 3 and np.array_equal(got[-1], want))
+    finally:
+        stored.close()
+        net.close()
