@@ -117,6 +117,7 @@ private:
     uint32_t _deferredBatch = 0;
     void Materialise();
     void MaterialiseForCaller();
+    void StoreFromNowOn();   // and the table that its top-Ks were screened by is given back
     bool _bHandedOut = false;     // NNNetwork::GetUnitBuffer was called for this layer: its units may change at any time
     void SettleConsumers();       // before this layer's units change: computes deferred layers that are fed by them
     void SwitchLane(uint32_t lane)

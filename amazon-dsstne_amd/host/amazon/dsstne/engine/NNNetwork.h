@@ -53,6 +53,8 @@ private:
     void LoadBatch();
     void RefreshState();
     void ClearUpdates() {}
+    uint32_t _topKPrepared = 0;   // PrepareTopK
+    void ReviseScreenTables();
     void LayerWithTopK(NNLayer* pLayer, const void* pTable, uint32_t k, uint32_t batch, const uint32_t* pIndex, const uint64_t* pFilterStart,
                        const uint64_t* pFilterEnd, const uint32_t* pFilterIndex, NNFloat* pKey, uint32_t* pValue);
 

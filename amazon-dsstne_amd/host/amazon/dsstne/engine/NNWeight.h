@@ -56,6 +56,7 @@ private:
     bool _bScreenValid = false, _bScreenRefused = false;
     uint32_t _screenAsked = 0;
     const void* ScreenTable(uint32_t k, uint32_t n, bool bMake);
+    void ReleaseScreenTable();
     void InvalidateSplit()
     {
         _bSplitValid[0] = _bSplitValid[1] = _bScreenValid = false;

@@ -214,7 +214,7 @@ void NNLayer::ForwardPropagateFullyConnected(uint32_t position, uint32_t batch, 
                     // to be computed again: such data is served better by the stored layer and the scanning top-K
                     printf("NNLayer::ForwardPropagate: rows of layer %s had to be computed twice for their top-K; its result is stored from now on.\n",
                            _name.c_str());
-                    _bDeferOutput = false;
+                    StoreFromNowOn();
                 } else {
                     _deferred = true;
                     _bToppedDeferred = false;
@@ -298,8 +298,14 @@ void NNLayer::Materialise()
 // Units that are asked for although their top-K has been computed: a narrower layer is better stored in the first place then.
 void NNLayer::MaterialiseForCaller()
 {
-    if (_bToppedDeferred && _localStride < kDeferMinWidth) _bDeferOutput = false;
+    if (_bToppedDeferred && _localStride < kDeferMinWidth) StoreFromNowOn();
     Materialise();
+}
+
+void NNLayer::StoreFromNowOn()
+{
+    _bDeferOutput = false;
+    for (auto w : _vIncomingWeight) (w->_bShared ? w->_pSharedWeight : w)->ReleaseScreenTable();
 }
 
 void NNLayer::SettleConsumers()

@@ -358,12 +358,23 @@ bool NNNetwork::SetSplitProducts(bool bSplit)
             w->_pbSplit[1].reset();
         }
     }
+    ReviseScreenTables();
     return true;
 }
 
 void NNNetwork::PrepareTopK(uint32_t k)
 {
+    _topKPrepared = k;
     for (auto l : _vOutputLayer) l->PrepareTopK(_batch, k);
+}
+
+// After a switch of how layers are computed: the tables that are not used any more go, and those that were asked for beforehand come back.
+void NNNetwork::ReviseScreenTables()
+{
+    for (auto l : _vOutputLayer)
+        if (!l->_bDeferOutput || l->UseSplitProducts(_batch))
+            for (auto w : l->_vIncomingWeight) (w->_bShared ? w->_pSharedWeight : w)->ReleaseScreenTable();
+    if (_topKPrepared != 0) PrepareTopK(_topKPrepared);
 }
 
 bool NNNetwork::SetDeferredOutput(bool bDefer)
@@ -372,6 +383,7 @@ bool NNNetwork::SetDeferredOutput(bool bDefer)
         if (!bDefer && l->_deferred) l->Materialise();
         l->_bDeferOutput = bDefer;
     }
+    ReviseScreenTables();
     return true;
 }
 

@@ -44,10 +44,7 @@ NNWeight::NNWeight(NNLayer& inputLayer, NNLayer& outputLayer, bool bShared, bool
     _pbBias.reset(new GpuBuffer<NNFloat>(_localBiasSize));
 }
 
-NNWeight::~NNWeight()
-{
-    if (_pScreen && dsx_is_initialized()) dsx_free(_pScreen);
-}
+NNWeight::~NNWeight() { ReleaseScreenTable(); }
 
 namespace {
 // Counter-based stream: value i of a connection depends only on the process seed, the two layer names and i, so a
@@ -144,6 +141,7 @@ NNFloat* NNWeight::GetWeightBuffer()
     if (!_pbWeight) return NULL;
     SettleUnits();
     _bHandedOut = true;
+    ReleaseScreenTable();
     return _pbWeight->_pDevData;
 }
 
@@ -228,6 +226,18 @@ const void* NNWeight::ScreenTable(uint32_t k, uint32_t n, bool bMake)
         _bScreenValid = true;
     }
     return _pScreen;
+}
+
+// For weights that are not screened any more.  (Batches of any lane may still be reading the table.)
+void NNWeight::ReleaseScreenTable()
+{
+    if (_pScreen && dsx_is_initialized()) {
+        dsxFatal(dsx_sync(), "NNWeight::ReleaseScreenTable");
+        dsxFatal(dsx_free(_pScreen), "NNWeight::ReleaseScreenTable");
+    }
+    _pScreen = NULL;
+    _bScreenValid = false;
+    _screenAsked = 0;
 }
 
 bool NNWeight::SetBiases(const vector<NNFloat>& vBias)

@@ -145,3 +145,29 @@ def test_weights_set_between_two_top_ks(pkg, dsx, synth, items, hidden, batch):
     finally:
         stored.close()
         net.close()
+
+
+@pytest.mark.parametrize("change", ["split products", "stored output"])
+def test_a_table_that_is_not_used_is_given_back(pkg, dsx, synth, change):
+    from amazon_dsstne_amd import host_api
+    p, net = network(synth, host_api, 140000, 256, 8)
+    try:
+        net.bind_input()
+        net.predict_batch(0)
+        net.topk(p.k)
+        net.get_topk(p.batch)
+        before = memory(dsx)
+        want = net.get_topk(p.batch)
+        if change == "split products":
+            net.set_split_products(True)
+        else:
+            net.set_deferred_output(False)
+        assert before - memory(dsx) > 200 << 20
+        net.set_split_products(False)
+        net.set_deferred_output(True)
+        assert before - memory(dsx) < 10 << 20       # (it is used again)
+        net.predict_batch(0)
+        net.topk(p.k)
+        assert all(np.array_equal(a, b) for a, b in zip(want, net.get_topk(p.batch)))
+    finally:
+        net.close()
