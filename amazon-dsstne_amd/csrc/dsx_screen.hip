@@ -871,11 +871,15 @@ static inline size_t align256(size_t x) { return (x + 255) / 256 * 256; }
 
 // Whether all columns' sums are stored.  (They are compared with bounds only where a bound keeps most columns out, and where there
 // are rows for the whole GPU: a workgroup of that kind has 256 rows, and 64 share a row's columns at most.)  A workgroup reads the maxima of
-// 131,072 columns; few rows have one of four times as many wavefronts each, which takes the bitmap of a million columns' filter.
+// 131,072 columns; few rows have one of four times as many wavefronts each, which takes the bitmap of a million columns' filter.  More than 2^28
+// sums are not stored: writing them takes what it takes, ranges leave most of them in registers (us, stored / in ranges, top 10, kept tables: 4,096 x
+// 128 x 131,072 551 / 280, 512 x 64 x 1,000,000 445 / 295, 4,096 x 512 x 100,000 719 / 546; top 100 4,096 x 32 x 100,000 366 / 382, the only kind that
+// loses, of 720 searches and layers).  Below, top 10 gains in ranges too from 2^26 sums on (2,048 x 128 x 100,000 193 / 151) and top 100 loses (256 x
+// 128 x 1,000,000 272 / 414).
 static bool screen_stored(uint32_t batch, uint64_t n)
 {
     if (ctx().knobs.fc_topk_first_columns) return false;
-    return (n <= 131072 || (batch <= 512 && n <= 1048576)) && (uint64_t)batch * n <= ((uint64_t)1 << 30);
+    return (n <= 131072 || (batch <= 512 && n <= 1048576)) && (uint64_t)batch * n <= ((uint64_t)1 << 28);
 }
 
 static uint32_t screen_first_columns(uint32_t n, uint32_t k)
@@ -1002,7 +1006,7 @@ int screen_run(const ScreenJob& j, const ScreenTable& t, const ScreenWorkspace& 
 {
     hipStream_t s = ctx().stream;
     const uint32_t ld = screen_ld(j.dim), n = j.n;
-    // (a first block that is everything, of a narrow table and more than 2^30 sums, is a search of stored sums too: there is no range to end with)
+    // (a first block that is everything, of a narrow table and many rows, is a search of stored sums too: there is no range to end with)
     const uint32_t n0 = std::min(w.columns, n);
     const bool stored = n0 == n;
     F16Job f{};

@@ -122,7 +122,7 @@ def test_results_in_host_memory(pkg, dsx, rng, storage, n, queries, k):
 
 # tables whose pad rows lie across a width, or a product with the queries, at which whole rows stop being stored: laid out for the one side, searched
 # on the other
-@pytest.mark.parametrize("rows,padding,queries,k", [(131080, 8, 600, 10), (140000, 12000, 513, 33), (1048584, 16, 3, 20), (129400, 100, 8300, 10)])
+@pytest.mark.parametrize("rows,padding,queries,k", [(131080, 8, 600, 10), (140000, 12000, 513, 33), (1048584, 16, 3, 20), (32400, 100, 8300, 10)])
 def test_pad_rows_across_a_limit(pkg, dsx, rng, rows, padding, queries, k):
     print("[case] pad rows rows=%d padding=%d queries=%d k=%d" % (rows, padding, queries, k), flush=True)
     dim, n = 32, rows - padding
@@ -148,7 +148,7 @@ def test_pad_rows_across_a_limit(pkg, dsx, rng, rows, padding, queries, k):
             assert dsx.dsx_knn_last_search_path() == 1
 
 
-# more than 2^30 sums of a table no wider than a first block, which is all there is then
+# more sums than are stored of whole tables, of a table no wider than a first block, which is all there is then
 def test_large_batches_of_narrow_tables(pkg, dsx, rng):
     queries, n, dim, k = 66000, 16380, 16, 256
     print("[case] prepared search n=%d dim=%d queries=%d k=%d" % (n, dim, queries, k), flush=True)

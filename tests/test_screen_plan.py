@@ -18,7 +18,7 @@ def around(x):
 
 # the widths and products at which whole rows stop being stored
 SHAPES = [(b, r) for b, r in itertools.chain(((b, r) for b in (1, 64, 512, 513, 1000, 4096) for edge in (8192, 131072, 1048576) for r in around(edge)),
-                                             ((b, r) for b in (2000, 10000, 65600, 120000, 131073) for r in around((1 << 30) // b)))]
+                                             ((b, r) for b in (2000, 10000, 65600, 120000, 131073) for sums in (28, 30) for r in around((1 << sums) // b)))]
 
 
 @pytest.mark.parametrize("k", [1, 100, 256])
@@ -41,3 +41,11 @@ def test_every_search_ends_with_its_results(pkg, k):
             if padding < rows:
                 room, stored, ranges = plan(lib, pkg, batch, rows, padding, k)
                 assert ranges == (stored < rows - padding), (batch, rows, padding, k)
+
+
+def test_where_sums_are_stored(pkg):
+    """Up to 2^28 of them; beyond, ranges are the faster way."""
+    lib = pkg.load_library()
+    for batch, n, ranges in ((1024, 27278, 0), (4096, 65536, 0), (4, 1000000, 0), (256, 1048576, 0), (4096, 65537, 1), (4096, 131072, 1), (512, 1000000, 1),
+                             (4096, 1000000, 1), (2049, 131072, 1), (2048, 131072, 0)):
+        assert plan(lib, pkg, batch, n, 0, 10)[2] == ranges, (batch, n)
