@@ -1035,8 +1035,10 @@ int screen_run(const ScreenJob& j, const ScreenTable& t, const ScreenWorkspace& 
     if ((rc = launch_pick(a, !stored)) || stored) return rc;
     const size_t row_lds = (size_t)(j.dim + 63) / 64 * 256;
     // A bound taken over `done` columns lets about k * width / done of the next `width` columns pass: ranges grow by a factor that
-    // keeps that near an eighth of the lists (the sample's own items, which score high and pass as well, come on top).
-    const uint32_t growth = std::max(4u, j.cap / (8 * j.k));
+    // keeps that near an eighth of the lists (the sample's own items, which score high and pass as well, come on top).  Where the queries are kept in
+    // registers (below) a survivor costs more than in the other sweep, which queues them: twelve times at most there (top 10, us, 51 times / 12: 4,096 x
+    // 32 x 1,000,000 984 / 834, 4,096 x 64 x 300,000 522 / 445, 512 x 128 x 1,000,000 648 / 558; 4 to 16 times are level).
+    const uint32_t growth = std::max(4u, std::min(j.cap / (8 * j.k), j.even && ld <= 256 ? 12u : 0xffffffffu));
     for (uint32_t done = n0; done < n;) {
         uint32_t ncols = (uint32_t)std::min<uint64_t>((uint64_t)n - done, (uint64_t)done * growth);
         if (n - done - ncols < 256) ncols = n - done;   // no sliver of a last range
