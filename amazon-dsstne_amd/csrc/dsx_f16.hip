@@ -12,7 +12,10 @@
 // WI x WQ wavefronts make a workgroup; with 2 x 4 it has 256 x 256 tiles, one workgroup per compute unit.  Operands go from memory
 // straight to LDS (no registers, no LDS store instructions), 32 components a stage, STAGES stages in a ring: while stage s is
 // multiplied, s + 1 is there (its first operands are read in s's last step, so that no barrier leaves the matrix cores idle) and the
-// ones behind it are on their way, across the border from one tile to the next.  A stage's rows are 64 bytes; the 16-byte piece c of
+// ones behind it are on their way; what is asked for next crosses the border from one tile to the next.  What does not run on across it in the
+// forms for layers and stored sums: memory answers in order and a wait for any other load is a wait for the stages before it, so ask's loads (of which
+// it makes the sums' starts on the spot) and the storing form's scales empty the ring; its compiled loop has seven or eight waits for everything, a
+// large part of the time where a tile is four stages (128 components).  A stage's rows are 64 bytes; the 16-byte piece c of
 // row r lies at place c ^ (r / 2 % 4) of its row (the lanes ask memory for their pieces in that order).  LDS is not what bounds the kernel:
 // with r / 4 % 4 the counters' bank conflicts go from 45 % of its cycles to 1 %, and the times stay (4,411 us against 4,350 for 4,096 x
 // 512 x 1,000,000 with its candidates, 796 against 805 for 6,000 x 1,024 x 27,278; two runs of one side differ by as much).
@@ -363,9 +366,8 @@ __global__ __launch_bounds__(64 * WI * WQ) __attribute__((amdgpu_waves_per_eu(WI
         stage();
         stage();   // (ld is a multiple of 64: two stages at least)
         if constexpr (MODE != kF16Scores) {
-            // Two tiles ahead, into the places of the tile before last: a whole tile's barriers and waits lie before they are read.  The
-            // wait for what was asked for is then for requests that three stages follow (after one stage it emptied the ring once a tile:
-            // 4 x 128 x 1,000,000 77 us, 73.5 so).
+            // Two tiles ahead, into the places of the tile before last: a whole tile's barriers and waits lie before they are read.  (After the
+            // tile's second stage: 4 x 128 x 1,000,000 73.5 us; after its first 77.)
             put(t + 2);
             ask(t + 3);
         }
