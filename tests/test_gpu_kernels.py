@@ -812,7 +812,7 @@ def knn_case_f16(pkg, dsx, orc, items_m, queries_m, k):
     return scores.numpy(), idx.numpy(), ref_s, ref_i, it16, q16, table
 
 
-# sweep 0: one workgroup per tile of scores; 2: column ranges with at least a tile per chunk go through knn_f16_sweep_kernel
+# sweep 0: one workgroup per tile of scores; 2: column ranges with at least a tile per chunk go through f16_sweep_kernel
 # (with these few queries that is 64 chunks per row tile, so ranges from 8,192 columns on); 3: through knn_f16_wide_kernel
 # (queries in registers; ranges from 4,096 columns on; 192 components is the one register layout the other cases leave out)
 @pytest.mark.parametrize("sweep", [0, 2, 3])
