@@ -163,19 +163,20 @@ int dsx_fc_topk_flagged_for(const float* W, int reset)
     return seen;
 }
 
-// Where the line lies (us, layer stored and guided top-K / this call, filter of 144 columns a row):
+// Where the line lies (us, layer stored and guided top-K / this call, filter of 144 columns a row that score high):
 //   From 131,072 columns on always, but for batches of up to 64: those are bound by reading the layer's weights once; storing their
-//   scores and maxima adds little to that, and this call's tiles of 128 rows a lot (8 x 256 x 500,000, top 50: 135 / 440).
-//   Narrower layers where the ranges are screened in 16 bits and that is most of the work: 4,096 x 1,024 x 27,278 top 10 2,011 / 920,
-//   1,904 rows 913 / 517, 2,048 x 512 x 27,278 490 / 281, 4,096 x 128 x 60,000 716 / 413; 1,024 x 1,024 x 27,278 468 / 370, but with
-//   own items that score high (trained networks) the candidates double.  Candidates grow with k: top 100 2,084 / 1,852, 4,096 x 512 x
-//   60,000 2,056 / 1,465, but 2,048 x 512 x 27,278 515 / 593.  Sigmoids only: their scores are above 0, so that no row has to be
-//   computed again for a listed column's zero.
+//   scores and maxima adds little to that, and this call's tiles of 128 rows a lot (8 x 256 x 500,000, top 50: 135 / 440).  It is the memory that the
+//   scores would take as much as the time: 512 x 256 x 131,072 top 10 347 / 229, but layers too small to be screened take longer (512 x 64 x 131,072
+//   top 10 147 / 347).
+//   Narrower layers where they are screened, and large: 4,096 x 1,024 x 27,278 top 10 1,861 / 524, 2,048 x 512 x 27,278 529 / 187, 4,096 x 128 x
+//   60,000 734 / 305; top 100 4,096 x 1,024 x 27,278 1,927 / 718, 4,096 x 512 x 60,000 2,108 / 654.  (Smaller ones gain too, 1,024 x 1,024 x 27,278 530 / 262,
+//   but pay for the table with every batch; with a kept one the line is the one below.)  Sigmoids only: their scores are above 0, so that no row has
+//   to be computed again for a listed column's zero.
 int dsx_fc_topk_pays(uint32_t batch, uint32_t k_dim, uint32_t n, uint32_t activation, uint32_t k)
 {
     if (n >= 131072) return batch > 64;
     const double products = (double)batch * k_dim * n;
-    return activation == DSX_ACT_SIGMOID && screen_takes(batch, k_dim, n, true) && screen_layer_pays(batch, k_dim, n, k) &&
+    return activation == DSX_ACT_SIGMOID && screen_takes(batch, k_dim, n, true) &&
            ((k <= 32 && batch >= 1536 && products >= 2e10) || (k <= 128 && batch >= 2048 && products >= 1e11));
 }
 
@@ -235,7 +236,7 @@ static int fc_topk_common(const float* X, uint32_t ldx, const float* W, const fl
     const uint32_t cap = ctx().knobs.fc_topk_candidate_capacity ? ctx().knobs.fc_topk_candidate_capacity : kLayerCandCap;   // tests lower it to reach the overflow path with small inputs
     const uint32_t n0 = layer_first_columns(n, k);
     const bool ranges = n0 < n;
-    int screened = x_planes ? 0 : table ? 2 : (ranges && screen_takes(batch, kdim, n, true) && screen_layer_pays(batch, kdim, n, k)) ? 1 : 0;
+    int screened = x_planes ? 0 : table ? 2 : (ranges && screen_takes(batch, kdim, n, true)) ? 1 : 0;
     LibScratch& ws = g_layer_ws_of[current_lane()];
     int reserved = lib_scratch_reserve(ws, layer_layout(nullptr, batch, n0, k, cap, ranges || screened, screened, kdim, n).bytes, "dsx_fc_topk workspace", screened);
     if (reserved == DSX_ENOMEM && screened) {   // the 16-bit copies (up to 8 GiB) or the sums do not fit beside what is there: fp32 ranges need none

@@ -76,8 +76,7 @@ static uint32_t knn_block_lists(uint32_t num_queries, uint32_t ncols, uint32_t k
 
 static bool knn_screens(uint32_t rows_padded, uint32_t num_queries, uint32_t k, uint32_t dim)
 {
-    return screen_takes(num_queries, dim, rows_padded, false) &&
-           screen_search_pays(num_queries, dim, rows_padded, k, rows_padded <= knn_block_columns(rows_padded, num_queries), 1.0f);
+    return screen_takes(num_queries, dim, rows_padded, false) && screen_search_pays(num_queries, dim, rows_padded, k);
 }
 
 static KnnWorkspace knn_layout(void* base, uint32_t rows_padded, uint32_t num_queries, uint32_t k, bool f16 = false, uint32_t dim = 0,
@@ -272,11 +271,9 @@ static void knn_notes_release()
 }
 
 // Whether what the preparation found speaks against screening.
-static bool knn_unfit(const ScreenNotes& notes, uint32_t num_queries, uint32_t dim, uint32_t M, uint32_t k)
+static bool knn_unfit(const ScreenNotes& notes)
 {
-    const float average = notes.number != 0 ? notes.sum / (float)notes.number : 0.0f;
-    return notes.flag != 0 || notes.largest > 65504.0f ||
-           (notes.largest > 0.0f && !screen_search_pays(num_queries, dim, M, k, M <= knn_block_columns(M, num_queries), notes.largest / average));
+    return notes.flag != 0 || !screen_fits(notes.largest, notes.number != 0 ? notes.sum / (float)notes.number : 0.0f);
 }
 
 static int knn_notes_ready()
@@ -368,7 +365,7 @@ static int knn_search_screened(const KnnWorkspace& w, const KnnOperands& op, uin
         while ((noted = hipEventQuery(g_knn_noted)) == hipErrorNotReady) {}
         (void)hipGetLastError();   // (not ready is not an error of the next launch)
         DSX_HIP(noted);
-        *unfit = knn_unfit(*g_knn_notes, num_queries, op.dim, M, k);
+        *unfit = knn_unfit(*g_knn_notes);
         if (*unfit) return DSX_OK;
         j.even = g_knn_notes->number != 0 && screen_even(g_knn_notes->largest, g_knn_notes->sum / (float)g_knn_notes->number);
     }
@@ -646,10 +643,9 @@ int dsx_knn_prepare(const float* items, uint32_t rows_padded, uint32_t padding, 
     std::memcpy(&notes.largest, &stats[0], sizeof(float));
     std::memcpy(&notes.sum, &stats[1], sizeof(float));
     notes.number = stats[2];
-    // as where a search makes its own copies: no norm beyond f16's range, and none so far above the others that its share of the error
-    // (of the columns next to it, which are judged by the largest of 32 or 64) would let everything pass
+    // as where a search makes its own copies
     const float average = notes.number != 0 ? notes.sum / (float)notes.number : 0.0f;
-    if (notes.largest <= 65504.0f && notes.largest <= 64.0f * average) *prepared = screen_even(notes.largest, average) ? DSX_KNN_FP32_PREPARED_EVEN : DSX_KNN_FP32_PREPARED;
+    if (screen_fits(notes.largest, average)) *prepared = screen_even(notes.largest, average) ? DSX_KNN_FP32_PREPARED_EVEN : DSX_KNN_FP32_PREPARED;
     return DSX_OK;
 }
 

@@ -102,8 +102,11 @@ int screen_run(const ScreenJob& j, const ScreenTable& t, const ScreenWorkspace& 
 // is a factor of exp(4 * 2^-10 sqrt(dim) (largest / average - 1)) at most, 1.07 for 256 components.
 inline bool screen_even(float largest, float average) { return largest < 60000.0f && largest <= 2.0f * average; }
 
+// Whether an item table is fit for screening: no norm beyond f16's range, and none so far above the others that its share of the error (of the
+// columns next to it, which are judged by the largest of 32 or 64) would let everything pass.
+inline bool screen_fits(float largest, float average) { return largest <= 65504.0f && largest <= 64.0f * average; }
+
 bool screen_takes(uint32_t batch, uint32_t dim, uint64_t n, bool layer);
-bool screen_layer_pays(uint32_t batch, uint32_t dim, uint64_t n, uint32_t k);
-bool screen_search_pays(uint32_t batch, uint32_t dim, uint64_t n, uint32_t k, bool blocks, float norm_ratio);
+bool screen_search_pays(uint32_t batch, uint32_t dim, uint64_t n, uint32_t k);
 
 }  // namespace dsx

@@ -820,23 +820,11 @@ __global__ __launch_bounds__(256, 4) void screen_fold_kernel(ScreenFoldArgs a)
     }
 }
 
-// The same for a layer in ranges (dsx_fc_topk), fitted to 320 layers of 512 to 4,096 rows, 64 to 1,024 components, 16,384 to 1,000,000
-// columns, k 10 to 256, without filters: fp32 within 23 %, screened within 31 %; none is slower than in fp32, 1.3 % are left (us,
-// screened / fp32: 512 x 256 x 16,384 top 10 105 / 80, 4,096 x 1,024 x 27,278 top 256 3,977 / 2,591, 512 x 256 x 131,072 top 100
-// 539 / 539, 1,000 x 256 x 131,072 top 100 658 / 831, 4,096 x 512 x 300,000 top 100 3,578 / 10,343).
-bool screen_layer_pays(uint32_t batch, uint32_t dim, uint64_t n, uint32_t k)
-{
-    if (ctx().knobs.screen == 1) return true;
-    const double q = batch, d = dim, ld = screen_ld(dim), m = (double)n;
-    const double growth = std::max(4u, 512 / std::max(1u, k)), fold = std::log(std::max(m / 2048.0, 1.0)) / std::log(growth + 1.0);   // as fc_topk_common's ranges
-    const double ranges = std::ceil(fold), candidates = k * growth * fold;
-    const double fp32 = 28.0 + 17.6 * ranges + 1.553e-8 * q * m * d + 2.61e-7 * q * m + 7.7e-5 * q * candidates + 0.49 * k * ranges;
-    const double screened = 13.0 + 35.0 * ranges + 3.8e-6 * m * ld + 1.39e-9 * q * m * ld + 6e-8 * q * m + q * candidates * (7.6e-5 + 3.1e-7 * ld) + 0.57 * k * ranges;
-    return fp32 > 1.1 * screened;
-}
-
-// What can be screened: the preparation costs what about 130 rows' fp32 products do.  Limits: the row in LDS, and 8 GiB for the two
-// copies of the table.
+// What can be screened with copies of the table made in the call: the preparation costs what about 130 rows' fp32 products do.  Limits: the row in LDS,
+// and 8 GiB for the two copies.  A layer that is taken is faster so than in fp32 ranges: 714 calls of dsx_fc_topk, 512 to 4,096 rows, 64 to 1,024
+// components, 16,384 to 1,000,000 columns, k 10 to 256, with and without a filter, take 0.16 to 0.81 of the time (us, fp32 / screened: 512 x 1,024 x
+// 40,000 top 10 397 / 310, 512 x 256 x 16,384 top 10 87 / 67, 1,024 x 128 x 65,536 top 100 363 / 133, 4,096 x 1,024 x 27,278 top 256 2,552 / 920,
+// 4,096 x 512 x 1,000,000 top 10 31,177 / 5,081).
 bool screen_takes(uint32_t batch, uint32_t dim, uint64_t n, bool layer)
 {
     if (ctx().knobs.screen == 2) return false;
@@ -844,27 +832,17 @@ bool screen_takes(uint32_t batch, uint32_t dim, uint64_t n, bool layer)
     return batch >= 512 && dim >= 32 && dim <= 4096 && (!layer || (uint64_t)batch * dim >= 131072) && n >= (layer ? 16384 : 65536) && bytes <= ((uint64_t)8 << 30);
 }
 
-// Nearest neighbours: whether screening is the faster way.  Both sides as fitted to 336 measured searches of normalised random vectors (us;
-// 512 to 4,096 queries, 32 to 1,024 components, 65,536 to 1,000,000 items, k 10 to 256): fp32 within 13 %, block by block or with
-// candidate lists; screened within 45 %, which is why it has to be ahead by a tenth.  None of the 336 is slower than without
-// screening, 1.4 % of the time they could take is left (512 x 32 x 65,536 top 256 486 screened / 140 fp32, 2,048 x 32 x 300,000 top
-// 100 821 / 681, 512 x 128 x 300,000 top 100 544 / 569, 2,048 x 128 x 150,000 top 10 385 / 755, 4,096 x 128 x 1,000,000 top 100 2,368 /
-// 8,789).
-// norm_ratio: the largest norm of an item over the average one.  A bound is lowered by 2^-10 of the largest, about
-// 2^-10 sqrt(dim) norm_ratio of the scores' spread; where the k best lie, about four of it out, that many more candidates pass:
-// exp(4 * 2^-10 sqrt(dim) norm_ratio) times as many.  A first range leaves 5 k of them; lists hold 4,096.
-bool screen_search_pays(uint32_t batch, uint32_t dim, uint64_t n, uint32_t k, bool blocks, float norm_ratio)
+// Nearest neighbours: whether screening is the faster way, the copies' making included.  Fitted to 752 searches of 512 to 4,096 queries, 32 to 1,024
+// components, 65,536 to 1,000,000 items, k 1 to 256: none is slower, 0.3 % of the time they could take is left (us, fp32 / screened: 512 x 32 x 65,536
+// top 10 79 / 98, 512 x 64 x 65,536 top 10 90 / 105, 512 x 32 x 131,072 top 10 145 / 129, 512 x 128 x 65,536 top 10 129 / 104, 1,024 x 32 x 65,536 top
+// 10 151 / 103, 512 x 32 x 140,000 top 10 149 / 144, 2,048 x 128 x 150,000 top 10 767 / 260, 4,096 x 128 x 1,000,000 top 100 8,788 / 1,915).  These were
+// random vectors: beyond 131,072 items, where columns may go through lists, the line is held back for large k (512 x 32 x 140,000 top 256 225 / 160),
+// whose lists fill first where neighbours lie closer together.
+// So it is for norms that differ: 360 searches of tables with a lognormal spread (0.5) or an item 3 or 50 times as long as the others take 0.28 of the
+// time that fp32 does in all.
+bool screen_search_pays(uint32_t batch, uint32_t dim, uint64_t n, uint32_t k)
 {
-    const double q = batch, d = dim, ld = std::max(d, 64.0), m = (double)n;
-    const double more = std::exp(std::min(20.0, 4.0 * std::sqrt(d) * (double)norm_ratio / 1024.0));
-    if (5.0 * k * more > 3600.0) return false;
-    if (ctx().knobs.screen == 1) return true;
-    const double ranges = 1.0 + std::max(1.0, std::ceil(std::log(m / 40960.0) / std::log(5.0))), fold = std::log(m / 8192.0) / std::log(5.0);
-    const double fp32 = blocks ? 1.464e-8 * q * m * d + 1.656e-6 * q * m + 4.3e-5 * q * k + 0.265 * k
-                               : 120.0 + 1.447e-8 * q * m * d + 2.56e-7 * q * m + 2.37e-4 * q * k + 0.6 * k;
-    const double screened = 90.0 + 30.0 * ranges + 3.2e-6 * m * ld + 2e-9 * q * m * ld + 1e-7 * q * m +
-                            more * (q * k * fold * (4e-4 + 1.9e-6 * ld) + 0.5 * k * ranges);
-    return fp32 > 1.1 * screened;
+    return ctx().knobs.screen == 1 || (double)batch * (dim + 32 + (n <= 131072 ? 0.25 : -0.125) * k) * (double)n >= 5.2e9;
 }
 
 static inline size_t align256(size_t x) { return (x + 255) / 256 * 256; }

@@ -92,6 +92,27 @@ def test_operands_that_f16_holds_badly(pkg, dsx, rng, form):
     assert dsx.dsx_knn_last_search_path() == {"unit": 1, "subnormal": 1, "nan items": 1, "rising": 2}.get(form, 0)
 
 
+# both sides of the line for small searches and of the limit for long items; sums stored and in ranges; a spread that raised bounds pay for most (k
+# large, vectors long)
+@pytest.mark.parametrize("n,queries,dim,k,longest,path", [(65536, 512, 32, 10, 1, 0), (66001, 513, 120, 10, 1, 1), (70001, 1000, 700, 256, 12, 1),
+                                                          (70001, 600, 128, 256, 55, 1), (70001, 600, 128, 256, 90, 0), (140001, 560, 900, 256, 55, 1)])
+def test_where_searches_are_screened(pkg, dsx, rng, n, queries, dim, k, longest, path):
+    print("[case] screened knn by rule n=%d queries=%d dim=%d k=%d longest=%d" % (n, queries, dim, k, longest), flush=True)
+    dsx.dsx_testing_set_screen(0)
+    items = rng.standard_normal((n, dim), dtype=np.float32)
+    items /= np.linalg.norm(items, axis=1, keepdims=True)
+    if longest > 1:
+        items *= np.exp(rng.normal(0, 0.3, n)).astype(np.float32)[:, None]
+        items[n // 3] *= np.float32(longest) * np.linalg.norm(items, axis=1).mean() / np.linalg.norm(items[n // 3])
+    q = rng.standard_normal((queries, dim), dtype=np.float32)
+    s, i = search(pkg, dsx, items, q, k)
+    assert dsx.dsx_knn_last_search_path() == path and dsx.dsx_knn_last_search_repeated() == 0
+    some = np.unique(np.concatenate([[0, queries - 1], rng.integers(0, queries, 40)]))
+    full = q[some].astype(np.float64) @ items.astype(np.float64).T
+    scale = np.linalg.norm(q[some].astype(np.float64), axis=1)[:, None] * np.linalg.norm(items.astype(np.float64), axis=1).max()
+    check_against_float64(s[some] / scale, i[some], full / scale, k, dim * 2.0 ** -24)
+
+
 @pytest.mark.parametrize("dim", [32, 128, 1024])
 def test_components_at_half_the_smallest_subnormal(pkg, dsx, rng, dim):
     """Components a little above 2^-25 round up to 2^-24 in both operands: a screened sum is four times the score, and below any bound
