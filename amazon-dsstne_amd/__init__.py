@@ -101,6 +101,7 @@ SIGNATURES = {
     "dsx_fc_topk_split": [_vp, _u32, _vp, _vp, _vp, _vp, _u32, _u32, _u32, _u32, C.POINTER(ActParams), _u32, _vp, _vp, _u32, _vp, _vp, _vp, _vp],
     "dsx_screen_table_build": [_vp, _u32, _u32, _u32, _vp],
     "dsx_fc_topk_screened": [_vp, _u32, _vp, _vp, _vp, _u32, _u32, _u32, _u32, C.POINTER(ActParams), _u32, _vp, _vp, _u32, _vp, _vp, _vp, _vp],
+    "dsx_fc_topk_screened_reserve": [_int, _u32, _u32, _u32, _u32],
     "dsx_fc_topk_screened_pays": [_u32, _u32, _u32, _u32, _u32],
     "dsx_fc_topk_pays": [_u32, _u32, _u32, _u32, _u32],
     "dsx_fc_topk_supported": [_u32, _vp, _u32, C.POINTER(ActParams), _vp],

@@ -210,6 +210,15 @@ int dsx_fc_topk_supported(uint32_t ldx, const float* X, uint32_t activation, con
 
 }  // extern "C"
 
+static int layer_flags_ready()
+{
+    if (g_layer_flagged) return DSX_OK;
+    DSX_HIP(hipHostMalloc((void**)&g_layer_flagged, kFlagWords * sizeof(uint32_t), hipHostMallocMapped));
+    for (int i = 0; i < kFlagWords; i++) g_layer_flagged[i] = 0;
+    at_shutdown(layer_flags_release);
+    return DSX_OK;
+}
+
 // x_planes / w_planes (both or neither): the operands as dsx_fc_split leaves them; the products then come from the split-product
 // kernel.  X and W are needed either way (rows whose lists fill up are recomputed from them, in fp32).
 static int fc_topk_common(const float* X, uint32_t ldx, const float* W, const float* bias, uint32_t batch, uint32_t kdim, uint32_t n,
@@ -227,11 +236,7 @@ static int fc_topk_common(const float* X, uint32_t ldx, const float* W, const fl
                          "linear are), or X is not 16-byte aligned with a pitch that is a multiple of 4: use dsx_fc_forward + dsx_topk_filtered",
                          activation);
     if (batch == 0) return DSX_OK;
-    if (!g_layer_flagged) {
-        DSX_HIP(hipHostMalloc((void**)&g_layer_flagged, kFlagWords * sizeof(uint32_t), hipHostMallocMapped));
-        for (int i = 0; i < kFlagWords; i++) g_layer_flagged[i] = 0;
-        at_shutdown(layer_flags_release);
-    }
+    if (int rc = layer_flags_ready()) return rc;
     uint32_t* const flag_word = g_layer_flagged + layer_flag_slot(W, true);
     const uint32_t cap = ctx().knobs.fc_topk_candidate_capacity ? ctx().knobs.fc_topk_candidate_capacity : kLayerCandCap;   // tests lower it to reach the overflow path with small inputs
     const uint32_t n0 = layer_first_columns(n, k);
@@ -348,6 +353,21 @@ int dsx_screen_table_build(const float* W, uint32_t ldw, uint32_t n, uint32_t kd
     DSX_CHECK_ARG(((uintptr_t)table % 256) == 0, "dsx_screen_table_build: the table is not 256-byte aligned");
     DSX_CHECK_ARG(n > 0 && n < 1u << 28 && kdim > 0 && kdim <= 4096 && ldw >= n, "dsx_screen_table_build: n = %u, k = %u, ldw = %u", n, kdim, ldw);
     return screen_build(screen_table(table, kdim, n), W, ldw, n, kdim);
+}
+
+int dsx_fc_topk_screened_reserve(int lane, uint32_t batch, uint32_t kdim, uint32_t n, uint32_t k)
+{
+    DSX_REQUIRE_INIT();
+    DSX_CHECK_ARG(lane >= 0 && lane < DSX_MAX_LANES, "dsx_fc_topk_screened_reserve: lane %d (0..%d)", lane, DSX_MAX_LANES - 1);
+    DSX_CHECK_ARG(batch > 0 && kdim > 0 && kdim <= 4096 && n > 0 && n < 1u << 28 && k >= 1 && k <= 256, "dsx_fc_topk_screened_reserve: batch %u, k_dim %u, n %u, k %u",
+                  batch, kdim, n, k);
+    if (int rc = layer_flags_ready()) return rc;
+    const uint32_t cap = ctx().knobs.fc_topk_candidate_capacity ? ctx().knobs.fc_topk_candidate_capacity : kLayerCandCap;
+    LibScratch& ws = g_layer_ws_of[lane];
+    const size_t bytes = layer_layout(nullptr, batch, layer_first_columns(n, k), k, cap, true, 2, kdim, n).bytes;
+    if (ws.ptr && bytes > ws.bytes)
+        if (int rc = dsx_sync()) return rc;   // (the lane need not be the selected one, which is what growing waits for)
+    return lib_scratch_reserve(ws, bytes, "dsx_fc_topk workspace", true);
 }
 
 int dsx_fc_topk_screened(const float* X, uint32_t ldx, const float* W, const void* table, const float* bias, uint32_t batch, uint32_t kdim,

@@ -163,10 +163,12 @@ bool NNLayer::MayDefer()
     return dsx_fc_topk_supported(src->_stride, src->_pbUnit ? src->GetUnitBuffer() : NULL, (uint32_t)_activation, &params, NULL) != 0;
 }
 
-// (an input layer may turn out to be sparse once its data is there: its output layer is then no dense one)
+// The table and the scratch memory.  (An input layer may turn out to be sparse once its data is there: its output layer is then no dense one)
 void NNLayer::PrepareTopK(uint32_t batch, uint32_t k)
 {
-    if (_localStride >= kSegMaxMinWidth && MayDefer() && _vIncomingLayer[0]->_kind != Input) TopKScreenTable(batch, k, true);
+    if (_localStride < kSegMaxMinWidth || !MayDefer() || _vIncomingLayer[0]->_kind == Input || !TopKScreenTable(batch, k, true)) return;
+    for (uint32_t lane = 0; lane < _lanes; lane++)   // (no room for the scratch now: the top-K may have it, or does without)
+        if (dsx_fc_topk_screened_reserve((int)lane, batch, _vIncomingLayer[0]->_stride, _localStride, k) != DSX_OK) return;
 }
 
 bool NNLayer::TopKFusionPays(uint32_t batch, uint32_t k, const void** ppTable)

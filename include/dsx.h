@@ -335,6 +335,8 @@ int dsx_fc_topk_screened(const float* X, uint32_t ldx, const float* W, const voi
                          uint32_t n, uint32_t activation, const dsx_act_params* params, uint32_t k, float* keys, uint32_t* values,
                          uint32_t position, const uint32_t* index, const uint64_t* filter_start, const uint64_t* filter_end,
                          const uint32_t* filter_index);
+/* The scratch memory of a dsx_fc_topk_screened call of these sizes on that lane, allocated now and not by the call. */
+int dsx_fc_topk_screened_reserve(int lane, uint32_t batch, uint32_t k_dim, uint32_t n, uint32_t k);
 int dsx_fc_topk_screened_pays(uint32_t batch, uint32_t k_dim, uint32_t n, uint32_t activation, uint32_t k);
 /* 1 where dsx_fc_topk is the faster way to the top-K, 0 where dsx_fc_forward_segmax + dsx_topk_guided are. */
 int dsx_fc_topk_pays(uint32_t batch, uint32_t k_dim, uint32_t n, uint32_t activation, uint32_t k);

@@ -100,7 +100,7 @@ def memory(dsx):
 
 
 def test_the_first_top_k_makes_no_table(pkg, dsx, synth):
-    """The weights' table is there once the input is bound, and not made in the middle of a request."""
+    """The weights' table is there once the input is bound, and not made in the middle of a request; nor is the scratch memory allocated there."""
     from amazon_dsstne_amd import host_api
     p, net = network(synth, host_api, 140000, 256, 8)
     try:
@@ -110,6 +110,10 @@ def test_the_first_top_k_makes_no_table(pkg, dsx, synth):
         net.topk(p.k)
         net.get_topk(p.batch)
         assert memory(dsx) - before < 100 << 20      # the table: 217 MB
+        net.predict_batch(0)                         # (the other lane)
+        net.topk(p.k)
+        net.get_topk(p.batch)
+        assert memory(dsx) == before
     finally:
         net.close()
 
