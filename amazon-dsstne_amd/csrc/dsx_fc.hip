@@ -1023,32 +1023,37 @@ __global__ __launch_bounds__(256) void activation_kernel(float* z, uint64_t size
     for (; pos < size; pos += step) z[pos] = activate_rt(z[pos], act, slope, alpha, lambda);
 }
 
-// Row softmax (engine/kActivation.cu:155-236): a = min(1, exp(x - max) / sum exp(x - max)); one workgroup of sixteen wavefronts per row.
-// Bound by one compute unit's share of the caches' bandwidth: a row of up to 32,768 units is read once, held in registers and
-// written once (64 x 27,278: 57.5 us in three passes by four wavefronts, 7.4 so); wider rows are read three times.
+// Row softmax (engine/kActivation.cu:155-236): a = min(1, exp(x - max) / sum exp(x - max)).  T lanes per row (one wavefront: four rows a workgroup),
+// G groups of 4 T units held in registers: the row is read once and written once; G = 0: rows too wide for that are read three times.
+// Many rows are bound by memory, few by a compute unit's share of the caches' bandwidth, narrow ones by what a workgroup costs, so T and G are the
+// smallest that hold the row (us, three passes by four wavefronts / sixteen wavefronts with G = 8 whatever the width / so: 16,384 x 100
+// 17 / 296 / 6, 4,096 x 1,000 11.4 / 76 / 5.8, 4,096 x 5,000 51 / 81 / 26, 16,384 x 8,192 431 / 349 / 199, 64 x 27,278 42 / 6.9 / 6.9).
 typedef float float4a4 __attribute__((ext_vector_type(4), aligned(4)));   // 128-bit accesses of any row
-template <bool HELD>
-__global__ __launch_bounds__(1024) void softmax_kernel(float* z, uint32_t stride)
+template <int T, int G>
+__global__ __launch_bounds__(T < 256 ? 256 : T) void softmax_kernel(float* z, uint32_t batch, uint32_t stride)
 {
-    constexpr int G = 8;
-    __shared__ float sRed[2][1024 / kWave];
-    float* row = z + (uint64_t)blockIdx.x * stride;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int ROWS = T < 256 ? 256 / T : 1, WAVES = T / kWave;
+    __shared__ float sRed[2][WAVES];
+    const uint32_t b = blockIdx.x * ROWS + threadIdx.x / T, t = threadIdx.x % T;
+    if (ROWS > 1 && b >= batch) return;   // (whole wavefronts, which wait for no other)
+    float* row = z + (uint64_t)b * stride;
+    const int lane = threadIdx.x & 63, wave = t >> 6;
     const float low = -__builtin_inff();
     float m = low, s = 0.0f;
-    float4a4 x[HELD ? G : 1];
+    float4a4 x[G > 0 ? G : 1];
     auto reduce = [&](float v, int which, auto op) __attribute__((always_inline)) -> float {
         for (int o = 32; o > 0; o >>= 1) v = op(v, __shfl_xor(v, o, kWave));
+        if constexpr (WAVES == 1) return v;
         if (lane == 0) sRed[which][wave] = v;
         __syncthreads();
-        float r = sRed[which][lane % (1024 / kWave)];
-        for (int o = 1024 / kWave / 2; o > 0; o >>= 1) r = op(r, __shfl_xor(r, o, kWave));   // (by halves: fewer roundings than in turn)
+        float r = sRed[which][lane % WAVES];
+        for (int o = WAVES / 2; o > 0; o >>= 1) r = op(r, __shfl_xor(r, o, kWave));   // (by halves: fewer roundings than in turn)
         return r;
     };
-    if constexpr (HELD) {
+    if constexpr (G > 0) {
 #pragma unroll
         for (int g = 0; g < G; g++) {
-            const uint32_t j = (g * 1024 + threadIdx.x) * 4;
+            const uint32_t j = (g * T + t) * 4;
             x[g] = float4a4{low, low, low, low};
             if (j + 4 <= stride) x[g] = *reinterpret_cast<const float4a4*>(row + j);
             else
@@ -1059,12 +1064,12 @@ __global__ __launch_bounds__(1024) void softmax_kernel(float* z, uint32_t stride
             for (int e = 0; e < 4; e++) m = fmaxf(m, x[g][e]);
         }
     } else
-        for (uint32_t j = threadIdx.x; j < stride; j += 1024) m = fmaxf(m, row[j]);
+        for (uint32_t j = t; j < stride; j += T) m = fmaxf(m, row[j]);
     m = reduce(m, 0, [](float a, float b) { return fmaxf(a, b); });
-    if constexpr (HELD) {
+    if constexpr (G > 0) {
 #pragma unroll
         for (int g = 0; g < G; g++) {
-            const uint32_t j = (g * 1024 + threadIdx.x) * 4;
+            const uint32_t j = (g * T + t) * 4;
 #pragma unroll
             for (int e = 0; e < 4; e++) x[g][e] = __expf(x[g][e] - m);
             if (j + 4 <= stride) s += (x[g][0] + x[g][1]) + (x[g][2] + x[g][3]);
@@ -1074,13 +1079,13 @@ __global__ __launch_bounds__(1024) void softmax_kernel(float* z, uint32_t stride
                     if (j + e < stride) s += x[g][e];
         }
     } else
-        for (uint32_t j = threadIdx.x; j < stride; j += 1024) s += __expf(row[j] - m);
+        for (uint32_t j = t; j < stride; j += T) s += __expf(row[j] - m);
     s = reduce(s, 1, [](float a, float b) { return a + b; });
     const float inv = 1.0f / s;
-    if constexpr (HELD) {
+    if constexpr (G > 0) {
 #pragma unroll
         for (int g = 0; g < G; g++) {
-            const uint32_t j = (g * 1024 + threadIdx.x) * 4;
+            const uint32_t j = (g * T + t) * 4;
 #pragma unroll
             for (int e = 0; e < 4; e++) x[g][e] = fminf(1.0f, x[g][e] * inv);
             if (j + 4 <= stride) *reinterpret_cast<float4a4*>(row + j) = x[g];
@@ -1090,7 +1095,28 @@ __global__ __launch_bounds__(1024) void softmax_kernel(float* z, uint32_t stride
                     if (j + e < stride) row[j + e] = x[g][e];
         }
     } else
-        for (uint32_t j = threadIdx.x; j < stride; j += 1024) row[j] = fminf(1.0f, __expf(row[j] - m) * inv);
+        for (uint32_t j = t; j < stride; j += T) row[j] = fminf(1.0f, __expf(row[j] - m) * inv);
+}
+
+template <int T, int G> static int launch_softmax(float* z, uint32_t batch, uint32_t stride)
+{
+    constexpr uint32_t rows = T < 256 ? 256 / T : 1;
+    hipLaunchKernelGGL((softmax_kernel<T, G>), dim3((batch + rows - 1) / rows), dim3(T < 256 ? 256 : T), 0, ctx().stream, z, batch, stride);
+    DSX_LAUNCH_CHECK("softmax_kernel");
+    return DSX_OK;
+}
+
+static int softmax_run(float* z, uint32_t batch, uint32_t stride)
+{
+    if (stride <= 256) return launch_softmax<64, 1>(z, batch, stride);
+    if (stride <= 512) return launch_softmax<64, 2>(z, batch, stride);
+    if (stride <= 1024) return launch_softmax<64, 4>(z, batch, stride);
+    if (stride <= 2048) return launch_softmax<64, 8>(z, batch, stride);
+    if (stride <= 4096) return launch_softmax<256, 4>(z, batch, stride);
+    if (stride <= 8192) return launch_softmax<256, 8>(z, batch, stride);
+    if (stride <= 16384) return launch_softmax<1024, 4>(z, batch, stride);
+    if (stride <= 32768) return launch_softmax<1024, 8>(z, batch, stride);
+    return launch_softmax<1024, 0>(z, batch, stride);
 }
 
 }  // namespace dsx
@@ -1178,12 +1204,7 @@ int dsx_activation(float* unit, uint32_t batch, uint32_t stride, uint32_t activa
     DSX_REQUIRE_INIT();
     DSX_CHECK_ARG(unit && stride > 0, "dsx_activation: null unit or zero stride");
     if (batch == 0) return DSX_OK;
-    if (activation == DSX_ACT_SOFTMAX) {
-        if (stride <= 32768) hipLaunchKernelGGL((softmax_kernel<true>), dim3(batch), dim3(1024), 0, ctx().stream, unit, stride);
-        else hipLaunchKernelGGL((softmax_kernel<false>), dim3(batch), dim3(1024), 0, ctx().stream, unit, stride);
-        DSX_LAUNCH_CHECK("softmax_kernel");
-        return DSX_OK;
-    }
+    if (activation == DSX_ACT_SOFTMAX) return softmax_run(unit, batch, stride);
     switch (activation) {
     case DSX_ACT_SIGMOID:
     case DSX_ACT_TANH:
