@@ -480,7 +480,8 @@ int f16_sweep_run(const F16Job& j, bool layer, uint32_t* lists)
 {
     F16SweepArgs a = f16_args(j);
     a.tiles_i = (j.n + 255) / 256;
-    a.chunks = std::max(1u, std::min(std::min(kF16ListStride / 2, a.tiles_i), ((uint32_t)ctx().num_cus + a.tiles_q - 1) / a.tiles_q));
+    // (one workgroup per compute unit and no more than there are: two too many take as long again)
+    a.chunks = std::min(std::min(kF16ListStride / 2, a.tiles_i), std::max(1u, (uint32_t)ctx().num_cus / a.tiles_q));
     a.tiles_per_chunk = (a.tiles_i + a.chunks - 1) / a.chunks;
     a.group = std::min(a.tiles_q, kF16Group);
     *lists = a.chunks * 2;

@@ -436,8 +436,9 @@ int knn_f16_wide_run(const void* queries16, const void* items16, uint32_t ld, ui
     if (ld > 256) return DSX_OK;
     // queries in registers: 512 per workgroup, stages of 128 items, one workgroup per CU
     const uint32_t cus = (uint32_t)ctx().num_cus, tiles_q = (batch + 511) / 512, stages = (n + kWideStageItems - 1) / kWideStageItems;
-    const uint32_t chunks = std::min<uint32_t>(kF16ListStride / 2, (cus + tiles_q - 1) / tiles_q);   // two lists per (query, chunk)
-    if (every ? stages < chunks : (2 * tiles_q * chunks < cus || stages < 8 * chunks)) return DSX_OK;
+    // (two lists per (query, chunk); eight stages a chunk and more; no more workgroups than there are compute units: two too many take as long again)
+    const uint32_t chunks = std::min(std::min<uint32_t>(kF16ListStride / 2, std::max(1u, cus / tiles_q)), every ? 0xffffffffu : stages / 8);
+    if (every ? stages < chunks : 2 * tiles_q * chunks < cus) return DSX_OK;
     KnnF16SweepArgs a{};
     a.A = (const _Float16*)queries16;
     a.B = (const _Float16*)items16;
@@ -477,7 +478,7 @@ int knn_f16_candidates_run(const void* queries16, const void* items16, uint32_t 
         const int rc = knn_f16_wide_run(queries16, items16, ld, batch, n, cand, seg, seg_count, seg_words, mode == 3, lists_used);
         if (rc || *lists_used) return rc;
     }
-    const uint32_t tiles_q = (batch + 255) / 256, tiles_i = (n + 255) / 256, chunks = std::min<uint32_t>(kF16ListStride / 2, (cus + tiles_q - 1) / tiles_q);
+    const uint32_t tiles_q = (batch + 255) / 256, tiles_i = (n + 255) / 256, chunks = std::min<uint32_t>(kF16ListStride / 2, std::max(1u, cus / tiles_q));
     const bool sweep = seg && seg_count && (mode == 2 || mode == 3 ? tiles_i >= chunks : (mode == 1 && 2 * tiles_q * chunks >= cus && tiles_i >= 2 * chunks));
     if (!sweep) return knn_f16_scores_run(queries16, items16, ld, batch, n, nullptr, 0, &cand);
     F16Job f{};

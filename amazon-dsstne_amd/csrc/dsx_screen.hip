@@ -851,13 +851,17 @@ static inline size_t align256(size_t x) { return (x + 255) / 256 * 256; }
 // are rows for the whole GPU: a workgroup of that kind has 256 rows, and 64 share a row's columns at most.)  A workgroup reads the maxima of
 // 131,072 columns; few rows have one of four times as many wavefronts each, which takes the bitmap of a million columns' filter.  More than 2^28
 // sums are not stored: writing them takes what it takes, ranges leave most of them in registers (us, stored / in ranges, top 10, kept tables: 4,096 x
-// 128 x 131,072 551 / 280, 512 x 64 x 1,000,000 445 / 295, 4,096 x 512 x 100,000 719 / 546; top 100 4,096 x 32 x 100,000 366 / 382, the only kind that
-// loses, of 720 searches and layers).  Below, top 10 gains in ranges too from 2^26 sums on (2,048 x 128 x 100,000 193 / 151) and top 100 loses (256 x
-// 128 x 1,000,000 272 / 414).
-static bool screen_stored(uint32_t batch, uint64_t n)
+// 128 x 131,072 551 / 280, 512 x 64 x 1,000,000 445 / 295, 4,096 x 512 x 100,000 719 / 546).  For small k, of which few pass a bound, ranges are ahead
+// from fewer sums on, if a first block is a small part of the columns (819 layers and as many searches of 2^24 to 2^28 sums measured both ways, k 1 to 64:
+// 1.7 and 1.3 % of the time they could take are left, 8 and 7 with 2^28 alone; none loses more than 3 %): 4,096 x 64 x 65,536 top 1 248 / 166, 1,024 x 128 x
+// 131,072 top 10 151 / 119, 512 x 128 x 131,072 top 1 108 / 93, but 4,096 x 64 x 32,768 top 1 124 / 140, 2,048 x 64 x 65,536 top 32 124 / 141,
+// 256 x 256 x 524,288 top 10 204 / 243, 256 x 128 x 1,000,000 top 100 272 / 414.
+static bool screen_stored(uint32_t batch, uint64_t n, uint32_t k)
 {
     if (ctx().knobs.fc_topk_first_columns) return false;
-    return (n <= 131072 || (batch <= 512 && n <= 1048576)) && (uint64_t)batch * n <= ((uint64_t)1 << 28);
+    const uint64_t sums = (uint64_t)batch * n;
+    if (batch > 256 && n >= 49152 + 512 * k && sums > ((uint64_t)1 << 26) + ((uint64_t)k << 22)) return false;
+    return (n <= 131072 || (batch <= 512 && n <= 1048576)) && sums <= ((uint64_t)1 << 28);
 }
 
 static uint32_t screen_first_columns(uint32_t n, uint32_t k)
@@ -892,7 +896,7 @@ ScreenWorkspace screen_layout(void* base, uint32_t batch, uint32_t dim, uint64_t
     ScreenWorkspace w;
     char* p = (char*)base;
     // (decided here for every search in this workspace, which may be of fewer columns: pad rows of an item table)
-    const uint64_t columns = w.columns = screen_stored(batch, n) ? (uint32_t)n : screen_first_columns((uint32_t)n, k);
+    const uint64_t columns = w.columns = screen_stored(batch, n, k) ? (uint32_t)n : screen_first_columns((uint32_t)n, k);
     w.rows16 = p;
     p += align256(knn_f16_rows(batch) * screen_ld(dim) * 2);
     w.e1 = (float*)p;

@@ -1638,7 +1638,7 @@ __global__ __launch_bounds__(kWave) void knn_refresh_kernel(uint64_t* best, cons
         const uint32_t* counts = seg_count + (uint64_t)b * kF16ListStride;
         uint32_t before = 0;
         if (lane == 0) sStart[0] = 0;
-        for (uint32_t l0 = 0; l0 < kF16ListStride; l0 += kWave) {
+        for (uint32_t l0 = 0; l0 < lists; l0 += kWave) {
             uint32_t incl = (l0 + lane < lists) ? min(counts[l0 + lane], seg_cap) : 0u;
 #pragma unroll
             for (int d = 1; d < kWave; d *= 2) {
@@ -1650,13 +1650,13 @@ __global__ __launch_bounds__(kWave) void knn_refresh_kernel(uint64_t* best, cons
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        const uint32_t total = sStart[kF16ListStride];
+        const uint32_t total = sStart[lists];
         const uint64_t* from = seg + (uint64_t)b * lists * seg_cap;
         for (uint32_t e0 = 0; e0 < total; e0 += kWave) {
             const uint32_t e = e0 + lane;
             uint64_t word = 0;
             if (e < total) {
-                uint32_t lo = 0, hi = kF16ListStride;   // the last list that starts at or before e (empty ones start where the next one does)
+                uint32_t lo = 0, hi = lists;   // the last list that starts at or before e (empty ones start where the next one does)
                 while (hi - lo > 1) {
                     const uint32_t mid = (lo + hi) / 2;
                     if (sStart[mid] <= e) lo = mid;
