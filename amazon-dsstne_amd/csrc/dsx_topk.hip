@@ -307,7 +307,7 @@ struct TopKArgs {
     // results: either final (keys/values, pitch k) or packed partial lists
     float* keys;
     uint32_t* values;
-    float* keys2;               // the final results once more (pinned host memory), or NULL
+    float* keys2;               // the final results once more (pinned host memory): finish_row<R, true>
     uint32_t* values2;
     uint64_t* partial;          // [batch][partial_slots][k]
     uint32_t partial_slots;
@@ -342,7 +342,7 @@ __device__ __forceinline__ void write_final(const uint64_t (&q)[R], uint32_t lan
 
 // End of a (row, segment): merges the lists of the four waves into wave 0 and writes the result (final pairs, or packed words
 // for the merge kernel).  Every lane of the workgroup must call it.
-template <int R>
+template <int R, bool TWICE = false>
 __device__ __forceinline__ void finish_row(WaveTopK<R>& list, uint64_t (*sStage)[WaveTopK<R>::kStageWords], const TopKArgs& a,
                                            uint32_t b, uint32_t seg, uint32_t wave, uint32_t lane)
 {
@@ -383,7 +383,7 @@ __device__ __forceinline__ void finish_row(WaveTopK<R>& list, uint64_t (*sStage)
         } else {
             keys[p] = key;
             values[p] = col;
-            if (a.keys2) {
+            if constexpr (TWICE) {
                 a.keys2[(uint64_t)b * a.k + p] = key;
                 a.values2[(uint64_t)b * a.k + p] = col;
             }
@@ -1407,7 +1407,9 @@ __global__ __launch_bounds__(kTopkThreads, R <= 2 ? 4 : 2) void topk_guided_kern
 // the lists' d-th words bounds the k-th word; with d about 2 k / slots that rank is in the middle of the lists, and what
 // passes is little more than k words, which finish_row puts in order by counting.  (61 lists of 50 words, one row: 27 -> 6 us
 // against one wavefront that sorts and merges 64 words at a time.)
-template <int R>
+// TWICE: the results go to keys2 and values2 too.  (With a test at run time instead the scans and merges of a search's top 100 took 2 to 3 us more,
+// 64 x 200 x 100,000 in halves 45.5 against 42.5.)
+template <int R, bool TWICE>
 __global__ __launch_bounds__(kTopkThreads) void topk_merge_kernel(const uint64_t* partial, uint32_t slots, uint32_t k, float* keys,
                                                                   uint32_t* values, float* keys2, uint32_t* values2)
 {
@@ -1430,7 +1432,7 @@ __global__ __launch_bounds__(kTopkThreads) void topk_merge_kernel(const uint64_t
             if (src[p] != 0) unpack_score(src[p], key, col);
             keys[(uint64_t)b * k + p] = key;
             values[(uint64_t)b * k + p] = col;
-            if (keys2) {
+            if constexpr (TWICE) {
                 keys2[(uint64_t)b * k + p] = key;
                 values2[(uint64_t)b * k + p] = col;
             }
@@ -1465,7 +1467,7 @@ __global__ __launch_bounds__(kTopkThreads) void topk_merge_kernel(const uint64_t
 #pragma unroll
         for (int u = 0; u < U; u++) word[u] = next[u];
     }
-    finish_row<R>(list, sStage, a, b, 0, wave, lane);
+    finish_row<R, TWICE>(list, sStage, a, b, 0, wave, lane);
 }
 
 // In-place payload gather for the key/value overloads: values[b][j] holds a column number on entry.
@@ -1523,7 +1525,8 @@ template <int R> static int launch_scan(const TopKArgs& a, uint32_t batch, bool 
 template <int R> static int launch_merge(const uint64_t* partial, uint32_t slots, uint32_t k, float* keys, uint32_t* values, uint32_t batch, float* keys2,
                                          uint32_t* values2)
 {
-    hipLaunchKernelGGL((topk_merge_kernel<R>), dim3(batch), dim3(kTopkThreads), 0, ctx().stream, partial, slots, k, keys, values, keys2, values2);
+    if (keys2) hipLaunchKernelGGL((topk_merge_kernel<R, true>), dim3(batch), dim3(kTopkThreads), 0, ctx().stream, partial, slots, k, keys, values, keys2, values2);
+    else hipLaunchKernelGGL((topk_merge_kernel<R, false>), dim3(batch), dim3(kTopkThreads), 0, ctx().stream, partial, slots, k, keys, values, keys2, values2);
     DSX_LAUNCH_CHECK("topk_merge_kernel");
     return DSX_OK;
 }
