@@ -99,6 +99,7 @@ private:
     bool TopKScreenPays(uint32_t batch, uint32_t k);
     const void* TopKScreenTable(uint32_t batch, uint32_t k, bool bMake);
     void PrepareTopK(uint32_t batch, uint32_t k);
+    void PrepareSplit(uint32_t batch);   // the weights' planes, where the layer's products are formed from them
     // Whether the layer may be put off for its top-K at all, whatever is the faster way.
     bool MayDefer();
     // Whether the deferred layer's top-K has been computed; a narrower layer whose units are asked for all the same is stored from then on.

@@ -171,6 +171,13 @@ void NNLayer::PrepareTopK(uint32_t batch, uint32_t k)
         if (dsx_fc_topk_screened_reserve((int)lane, batch, _vIncomingLayer[0]->_stride, _localStride, k) != DSX_OK) return;
 }
 
+void NNLayer::PrepareSplit(uint32_t batch)
+{
+    if (_vIncomingLayer.size() != 1 || !_vIncomingSkip.empty() || _activation == SoftMax || _vIncomingLayer[0]->_kind == Input || !UseSplitProducts(batch)) return;
+    NNWeight* w = _vIncomingWeight[0];
+    (w->_bShared ? w->_pSharedWeight : w)->SplitPlanes(w->_bTransposed, _vIncomingLayer[0]->_stride, _localStride);
+}
+
 bool NNLayer::TopKFusionPays(uint32_t batch, uint32_t k, const void** ppTable)
 {
     const void* pTable = TopKScreenTable(batch, k, false);

@@ -350,7 +350,7 @@ bool NNNetwork::SetSplitProducts(bool bSplit)
         l->_bSplitProducts = bSplit;
         l->_splitMinTiles = 2u * info.compute_units;
     }
-    // (also the way to say that weights were written through NNWeight::GetWeightBuffer: the planes are built again on next use)
+    // (also the way to say that weights were written through NNWeight::GetWeightBuffer: the planes are built again, where top-Ks were prepared for now, else on next use)
     for (auto w : _vWeight) {
         w->InvalidateSplit();
         if (!bSplit) {
@@ -368,13 +368,16 @@ void NNNetwork::PrepareTopK(uint32_t k)
     for (auto l : _vOutputLayer) l->PrepareTopK(_batch, k);
 }
 
-// After a switch of how layers are computed: the tables that are not used any more go, and those that were asked for beforehand come back.
+// After a switch of how layers are computed: the tables that are not used any more go, and those that were asked for beforehand come back, as do
+// the planes of split products (the first pass would allocate and fill them otherwise).
 void NNNetwork::ReviseScreenTables()
 {
     for (auto l : _vOutputLayer)
         if (!l->_bDeferOutput || l->UseSplitProducts(_batch))
             for (auto w : l->_vIncomingWeight) (w->_bShared ? w->_pSharedWeight : w)->ReleaseScreenTable();
-    if (_topKPrepared != 0) PrepareTopK(_topKPrepared);
+    if (_topKPrepared == 0) return;
+    PrepareTopK(_topKPrepared);
+    for (auto l : _vLayer) l->PrepareSplit(_batch);
 }
 
 bool NNNetwork::SetDeferredOutput(bool bDefer)
