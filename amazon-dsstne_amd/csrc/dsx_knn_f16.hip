@@ -436,9 +436,9 @@ int knn_f16_wide_run(const void* queries16, const void* items16, uint32_t ld, ui
     if (ld > 256) return DSX_OK;
     // queries in registers: 512 per workgroup, stages of 128 items, one workgroup per CU
     const uint32_t cus = (uint32_t)ctx().num_cus, tiles_q = (batch + 511) / 512, stages = (n + kWideStageItems - 1) / kWideStageItems;
-    // (two lists per (query, chunk); eight stages a chunk and more; no more workgroups than there are compute units: two too many take as long again)
-    const uint32_t chunks = std::min(std::min<uint32_t>(kF16ListStride / 2, std::max(1u, cus / tiles_q)), every ? 0xffffffffu : stages / 8);
-    if (every ? stages < chunks : 2 * tiles_q * chunks < cus) return DSX_OK;
+    // (two lists per (query, chunk); no more workgroups than there are compute units: two too many take as long again)
+    const uint32_t chunks = std::min<uint32_t>(kF16ListStride / 2, std::max(1u, cus / tiles_q));
+    if (every ? stages < chunks : (2 * tiles_q * chunks < cus || stages < 8 * chunks)) return DSX_OK;
     KnnF16SweepArgs a{};
     a.A = (const _Float16*)queries16;
     a.B = (const _Float16*)items16;

@@ -698,7 +698,7 @@ __global__ __launch_bounds__(256, 4) void screen_fold_kernel(ScreenFoldArgs a)
     if (threadIdx.x == 0) a.cand_count[b] = 0;
     if (flagged) return;
     const uint32_t in_lists = sStart[256], fresh_words = shared + in_lists, total = kept + fresh_words;
-    if (fresh_words > a.cap) {
+    if (shared > a.cap) {   // (the lists of a row's own hold as many again)
         if (threadIdx.x == 0) screen_flag(a, b);
         return;
     }
@@ -1016,13 +1016,15 @@ int screen_run(const ScreenJob& j, const ScreenTable& t, const ScreenWorkspace& 
     if (stored && j.before_last) j.before_last(j.before_last_arg);
     if ((rc = launch_pick(a, !stored)) || stored) return rc;
     const size_t row_lds = (size_t)(j.dim + 63) / 64 * 256;
-    // A bound taken over `done` columns lets about k * width / done of the next `width` columns pass: ranges grow by a factor that
-    // keeps that near an eighth of the lists (the sample's own items, which score high and pass as well, come on top).  Where the queries are kept in
-    // registers (below) a survivor costs more than in the other sweep, which queues them: twelve times at most there (top 10, us, 51 times / 12: 4,096 x
-    // 32 x 1,000,000 984 / 834, 4,096 x 64 x 300,000 522 / 445, 512 x 128 x 1,000,000 648 / 558; 4 to 16 times are level).
-    const uint32_t growth = std::max(4u, std::min(j.cap / (8 * j.k), j.even && ld <= 256 ? 12u : 0xffffffffu));
+    // A bound taken over `done` columns lets about k * width / done of the next `width` columns pass: ranges grow by a factor that keeps that near an
+    // eighth of the lists (the sample's own items, which score high and pass as well, come on top), by twelve times at most, but for a last
+    // range of up to twenty: survivors cost more than another range's launches then (top 10, us, 51 times / 12: searches 4,096 x 32 x 1,000,000 984 / 834,
+    // 512 x 128 x 1,000,000 648 / 558; top 1, one range of 16 times / two: layers 4,096 x 64 x 140,000 245 / 279), and where scores rise along the table, or a filter lists the
+    // best columns of the first block, lists do not fill up that do with 51 times (4,096 x 64 x 1,000,000 top 10, 144 such columns a row: 23.8 ms / 1.1;
+    // what it costs: 1,024 x 64 x 300,000 top 1 172 / 192).
+    const uint32_t growth = std::max(4u, std::min(j.cap / (8 * j.k), 12u)), last = std::max(4u, std::min(j.cap / (8 * j.k), 20u));
     for (uint32_t done = n0; done < n;) {
-        uint32_t ncols = (uint32_t)std::min<uint64_t>((uint64_t)n - done, (uint64_t)done * growth);
+        uint32_t ncols = (uint32_t)((uint64_t)done * last >= n - done ? n - done : (uint64_t)done * growth);
         if (n - done - ncols < 256) ncols = n - done;   // no sliver of a last range
         f.items = (const char*)t.items16 + (uint64_t)done * ld * 2;
         f.norm = t.norm + done;

@@ -147,3 +147,24 @@ def test_prepared_searches(pkg, dsx, rng, n, dim, queries, k, storage):
     scale = np.linalg.norm(q.astype(np.float64), axis=1)[:, None]
     # dim products, each rounding at most 2^-24 of |q| |w|, |w| at most 1
     check_against_float64(s / scale, i, full / scale, k, dim * 2.0 ** -24)
+
+
+def test_a_first_block_whose_best_columns_are_listed(pkg, dsx, rng):
+    """Every row's filter lists the 144 best of the first 8,192 columns: the bound that is left lets one column in fifty of the next range pass, which is
+    within what the lists hold."""
+    batch, n, kdim, k = 600, 600000, 32, 10
+    print("[case] kept table, listed first block batch=%d kdim=%d n=%d k=%d" % (batch, kdim, n, k), flush=True)
+    X = np.maximum(rng.standard_normal((batch, kdim), dtype=np.float32), 0)
+    W = rng.standard_normal((kdim, n), dtype=np.float32) * np.float32(1 / np.sqrt(kdim))
+    bias = (rng.standard_normal(n) * 0.5 - 4).astype(np.float32)
+    own = np.sort(np.argpartition(-(X @ W[:, :8192] + bias[:8192]), 144, axis=1)[:, :144], axis=1).astype(np.uint32)
+    start = np.arange(batch, dtype=np.uint64) * 144
+    dsx.dsx_fc_topk_flagged(1)
+    s, i = layer(pkg, dsx, X, W, bias, k, 0, (start, start + 144, own.reshape(-1)))
+    assert dsx.dsx_fc_topk_flagged(0) == 0
+    at_rows = some(rng, batch, 20)
+    y = 1 / (1 + np.exp(-(X[at_rows].astype(np.float64) @ W.astype(np.float64) + bias)))
+    for r, b in enumerate(at_rows):
+        y[r, own[b]] = 0
+    # sums of kdim products and the bias, |x| |w| + |b| below 40: as above; the slope is a quarter at most
+    check_against_float64(s[at_rows], i[at_rows], y, k, (kdim + 8) * 40 * 2.0 ** -24 / 8 + 1e-6)
