@@ -19,7 +19,7 @@ def around(x):
 # the widths and products at which whole rows stop being stored
 SHAPES = [(b, r) for b, r in itertools.chain(((b, r) for b in (1, 64, 512, 513, 1000, 4096) for edge in (8192, 131072, 1048576) for r in around(edge)),
                                              ((b, r) for b in (2000, 10000, 65600, 120000, 131073) for sums in (28, 30) for r in around((1 << sums) // b)),
-                                             ((b, 65536 + r) for b in (257, 1024, 1200) for r in (-8, -1, 0, 1, 8)),
+                                             ((b, 49152 + 512 * k + r) for b in (257, 1024, 1700, 4096) for k in (1, 100, 150) for r in (-8, -1, 0, 1, 8)),
                                              ((b, r) for b in (257, 513, 1023) for k in (1, 100, 150, 256) for r in around(((1 << 26) + (k << 22)) // b)))]
 
 
@@ -48,8 +48,8 @@ def test_every_search_ends_with_its_results(pkg, k):
 def test_where_sums_are_stored(pkg):
     """Up to 2^28 of them, for more than 256 rows of a wide table and small k up to fewer; beyond, ranges are the faster way."""
     lib = pkg.load_library()
-    for batch, n, k, ranges in ((1024, 27278, 10, 0), (4096, 65535, 10, 0), (4, 1000000, 10, 0), (256, 1048576, 10, 0), (4096, 65537, 10, 1), (4096, 131072, 10, 1),
+    for batch, n, k, ranges in ((1024, 27278, 10, 0), (4096, 54271, 10, 0), (4096, 54272, 10, 1), (4, 1000000, 10, 0), (256, 1048576, 10, 0), (4096, 65537, 10, 1), (4096, 131072, 10, 1),
                                 (512, 1000000, 10, 1), (4096, 1000000, 10, 1), (2049, 131072, 100, 1), (2048, 131072, 100, 0), (2048, 131072, 10, 1),
-                                (4096, 60000, 1, 0), (4096, 65536, 1, 1), (1024, 65536, 1, 0), (1024, 98304, 10, 0), (1024, 131072, 10, 1), (512, 400000, 1, 1),
+                                (4096, 49663, 1, 0), (4096, 49664, 1, 1), (1024, 65536, 1, 0), (1024, 98304, 10, 0), (1024, 131072, 10, 1), (512, 400000, 1, 1),
                                 (512, 262144, 32, 0), (512, 524288, 32, 1)):
         assert plan(lib, pkg, batch, n, 0, k)[2] == ranges, (batch, n, k)
