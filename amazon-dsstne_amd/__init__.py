@@ -111,6 +111,7 @@ SIGNATURES = {
     "dsx_testing_set_allocation_limit": [_sz],
     "dsx_testing_set_screen": [_int],
     "dsx_testing_screen_columns": [_u32, _u32, _u32, _u32, _u32, C.POINTER(_u64), C.POINTER(_u64), C.POINTER(_int)],
+    "dsx_testing_set_screen_bytes": [_int],
     "dsx_testing_set_knn_no_events": [_int],
     "dsx_testing_occupy": [_u32, _u32, _u32],
     "dsx_testing_set_fc_topk_first_columns": [_u32],

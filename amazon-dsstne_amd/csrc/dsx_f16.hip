@@ -2,10 +2,13 @@
 //
 // Operands are row-major halves, a row's components contiguous: queries [rows rounded up to 256][ld], items [items rounded up to
 // 256][ld], ld a multiple of 64, zero filled.  Products are exact in fp32, sums are fp32, added in ascending k: the same bits as
-// knn_f16_kernel's.  Three uses (MODE):
+// knn_f16_kernel's.  Uses (MODE):
 //   kF16Scores   sums compared with the queries' bounds, survivors to lists (exact nearest neighbours, fp16 storage and screening)
 //   kF16Layer    sums that start from the items' biases, raised by the error they can have (dsx_screen.hip), against the bounds
 //   kF16Store    sums that start from the biases stored as halves, rounded up, and the largest of every 32 of them
+//   kI8Scores    operands are bytes (rows of 2 ld of them, a unit per query and per 32 items), sums are whole numbers; of every 32 items a word is
+//                stored (i8_word): the largest sum, whose it is, and the second largest.  Nothing is compared and nothing listed.
+//   kI8Layer     the same with the items' starts added
 //
 // A wavefront owns 128 items x 64 queries: four row operands and two column operands per 16 components feed eight matrix
 // instructions, 48 LDS cycles for 64 cycles of each SIMD's matrix core (a 64 x 64 tile needs as many LDS cycles as there are).
@@ -28,6 +31,7 @@
 // 4,096 queries x 1,000,000 items: 1.09 PFLOP/s with 512 components (a large product of the matrix library reaches 1.16 on this part),
 // 0.90 with 128, where the compares are a third of the issued instructions.  (128 x 128 tiles through registers: 0.72 with 576.)
 #include <algorithm>
+#include <type_traits>
 #include "dsx_screen.h"
 
 namespace dsx {
@@ -56,16 +60,29 @@ struct F16SweepArgs {
     _Float16* Z;            // kF16Store: [batch][ldz]
     uint64_t ldz;
     _Float16* M;            // kF16Store: [batch][ldz / 32] the largest of every 32 of them
-    const float* scale;     // kF16Store: [batch] what a query's sums are multiplied by (a power of two)
+    const float* scale;     // kF16Store: [batch] what a query's sums are multiplied by (a power of two); kI8*: a query's unit
+    const float* unit;      // kI8*: units of the items' components, one for every 32 items
+    uint32_t* words;        // kI8*: [batch][ldw] a word for every 32 items (i8_word)
+    uint64_t ldw;
 };
 
 constexpr uint32_t kF16Queue = 32;   // entries of a wavefront's queue
 
+// Whether a mode's sums start from something, and whether they go to lists.
+constexpr bool f16_starts(int mode) { return mode != kF16Scores && mode != kI8Scores; }
+constexpr bool f16_lists(int mode) { return mode == kF16Scores || mode == kF16Layer; }
+
 template <int WI, int WQ, int STAGES> constexpr uint32_t f16_sweep_lds(int mode)
 {
-    return STAGES * (128 * WI + 64 * WQ) * 64 + (mode != kF16Scores ? 4 * (128 + 4) * WI * 4 : 0) +
-           (mode != kF16Store ? WI * WQ * (kF16Queue * 80 + 64 * 4) : 0);
+    return STAGES * (128 * WI + 64 * WQ) * 64 + (f16_starts(mode) ? 4 * (128 + 4) * WI * 4 : 0) +
+           (f16_lists(mode) ? WI * WQ * (kF16Queue * 80 + 64 * 4) : 0);
 }
+
+// The integer sums start from this: the bits of 1.5 * 2^23, whose last one is worth 1, so that the sums are floats as they are (and in the order
+// of floats): magnitudes below 2^22 (i8_unit).
+constexpr int32_t kI8Start = 0x4B400000;
+constexpr float kI8StartValue = 12582912.0f;
+constexpr float kI8Most = 3.3e38f;   // above every sum
 
 template <int WI, int WQ, int STAGES, int MODE>
 __global__ __launch_bounds__(64 * WI * WQ) __attribute__((amdgpu_waves_per_eu(WI * WQ == 8 ? 2 : 1, 2))) void f16_sweep_kernel(F16SweepArgs a)
@@ -77,8 +94,9 @@ __global__ __launch_bounds__(64 * WI * WQ) __attribute__((amdgpu_waves_per_eu(WI
     // layers, four tiles each: what the items' sums start from, and the largest norm of 32 items
     float* sStart = reinterpret_cast<float*>(f16_lds + STAGES * STAGE);
     float* sMost = sStart + 4 * BI;
+    constexpr bool EIGHT = MODE == kI8Scores || MODE == kI8Layer;
     // the wavefronts' queues (sixteen results; then the bound, e1, the largest norm, the item and the query) and their lists' fill counts
-    unsigned char* after = f16_lds + STAGES * STAGE + (MODE != kF16Scores ? 4 * (128 + 4) * WI * 4 : 0);
+    unsigned char* after = f16_lds + STAGES * STAGE + (f16_starts(MODE) ? 4 * (128 + 4) * WI * 4 : 0);
     float (*sResult)[16] = reinterpret_cast<float (*)[16]>(after) + (threadIdx.x >> 6) * kF16Queue;
     uint4* sEntry = reinterpret_cast<uint4*>(after + WAVES * kF16Queue * 64) + (threadIdx.x >> 6) * kF16Queue;
     uint32_t* sFill = reinterpret_cast<uint32_t*>(after + WAVES * kF16Queue * 80) + (threadIdx.x & ~63u);
@@ -105,7 +123,7 @@ __global__ __launch_bounds__(64 * WI * WQ) __attribute__((amdgpu_waves_per_eu(WI
     float bound[2];
 #pragma unroll
     for (int j = 0; j < 2; j++) q[j] = row0 + wq * 64 + j * 32 + l32;
-    if constexpr (MODE != kF16Store) {
+    if constexpr (f16_lists(MODE)) {
         if (t0 >= t1) {   // more chunks than tiles: empty lists (the same for the whole workgroup)
             const uint32_t r = row0 + wq * 64 + lane;
             if (r < a.batch) a.seg_count[(uint64_t)r * kF16ListStride + list] = 0;
@@ -133,9 +151,13 @@ __global__ __launch_bounds__(64 * WI * WQ) __attribute__((amdgpu_waves_per_eu(WI
             const uint32_t i = o * 64 * WAVES + tid, c = t * BI + i;
             start_next[o] = -__builtin_inff();
             norm_next[o] = 0.0f;
+            if constexpr (EIGHT) start_next[o] = -3e37f;
             if (i >= BI || t >= t1 || c >= a.n) continue;
             const float b = a.bias ? a.bias[c] : 0.0f, norm = a.norm[c];
-            start_next[o] = (norm == __builtin_inff() && b == b) ? norm : b == -__builtin_inff() ? b : b + fabsf(b) * a.bias_raise;
+            if constexpr (EIGHT)   // (finite, as its lowest bits are taken; an item or a bias that is no number: never)
+                start_next[o] = (b != b || norm != norm) ? -3e37f : (norm == __builtin_inff()) ? 3e37f : fminf(fmaxf(b + fabsf(b) * a.bias_raise, -3e37f), 3e37f);
+            else
+                start_next[o] = (norm == __builtin_inff() && b == b) ? norm : b == -__builtin_inff() ? b : b + fabsf(b) * a.bias_raise;
             norm_next[o] = (norm == __builtin_inff()) ? 0.0f : norm;
         }
     };
@@ -153,7 +175,7 @@ __global__ __launch_bounds__(64 * WI * WQ) __attribute__((amdgpu_waves_per_eu(WI
             }
         }
     };
-    if constexpr (MODE != kF16Scores) {
+    if constexpr (f16_starts(MODE)) {
         if constexpr (MODE == kF16Layer) {
 #pragma unroll
             for (int j = 0; j < 2; j++)
@@ -224,7 +246,10 @@ __global__ __launch_bounds__(64 * WI * WQ) __attribute__((amdgpu_waves_per_eu(WI
 #pragma unroll
         for (int j = 0; j < 2; j++) fq[set][j] = *reinterpret_cast<const half8*>(pq + j * 2048);
     };
-    floatx16 acc[4][2];
+    typedef int32_t intx16 __attribute__((ext_vector_type(16)));
+    typedef int32_t intx4 __attribute__((ext_vector_type(4)));
+    typedef std::conditional_t<EIGHT, intx16, floatx16> Acc;
+    Acc acc[4][2];
     // (a multiplication first, whose wait is then for the reads of the step before and not for the first of these; then the next
     // step's six reads among the others)
     auto order = [&]() __attribute__((always_inline)) {
@@ -239,8 +264,21 @@ __global__ __launch_bounds__(64 * WI * WQ) __attribute__((amdgpu_waves_per_eu(WI
 #pragma unroll
         for (int i = 0; i < 4; i++)
 #pragma unroll
-            for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fi[set][i], fq[set][j], acc[i][j], 0, 0, 0);
+            for (int j = 0; j < 2; j++) {
+                if constexpr (EIGHT)
+                    acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(__builtin_bit_cast(intx4, fi[set][i]), __builtin_bit_cast(intx4, fq[set][j]), acc[i][j], 0, 0, 0);
+                else
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fi[set][i], fq[set][j], acc[i][j], 0, 0, 0);
+            }
     };
+
+    float mine[2] = {0.0f, 0.0f};   // the queries' units
+    uint32_t word[2][2];
+    if constexpr (EIGHT) {
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+            if (q[j] < a.batch) mine[j] = a.scale[q[j]];
+    }
 
     uint32_t queued = 0;   // wave-uniform
     auto settle = [&]() __attribute__((always_inline)) {
@@ -342,13 +380,16 @@ __global__ __launch_bounds__(64 * WI * WQ) __attribute__((amdgpu_waves_per_eu(WI
         cp = np;
     };
     for (uint32_t t = t0; t < t1; t++) {
-        if constexpr (MODE == kF16Scores) {
+        if constexpr (MODE == kF16Scores || EIGHT) {
 #pragma unroll
             for (int i = 0; i < 4; i++)
 #pragma unroll
                 for (int j = 0; j < 2; j++)
 #pragma unroll
-                    for (int v = 0; v < 16; v++) acc[i][j][v] = 0.0f;
+                    for (int v = 0; v < 16; v++) {
+                        if constexpr (EIGHT) acc[i][j][v] = kI8Start;
+                        else acc[i][j][v] = 0.0f;
+                    }
         } else {
             const float* from = sStart + (t & 3) * BI + wi * 128 + 4 * lhi;
 #pragma unroll
@@ -365,7 +406,7 @@ __global__ __launch_bounds__(64 * WI * WQ) __attribute__((amdgpu_waves_per_eu(WI
         __builtin_amdgcn_s_setprio(1);
         stage();
         stage();   // (ld is a multiple of 64: two stages at least)
-        if constexpr (MODE != kF16Scores) {
+        if constexpr (f16_starts(MODE)) {
             // Two tiles ahead, into the places of the tile before last: a whole tile's barriers and waits lie before they are read.  (After the
             // tile's second stage: 4 x 128 x 1,000,000 73.5 us; after its first 77.)
             put(t + 2);
@@ -373,7 +414,70 @@ __global__ __launch_bounds__(64 * WI * WQ) __attribute__((amdgpu_waves_per_eu(WI
         }
         for (uint32_t kt = 2; kt < nk; kt++) stage();
         __builtin_amdgcn_s_setprio(0);
-        if constexpr (MODE != kF16Store) {
+        if constexpr (EIGHT) {
+            // The largest two of a block's 32 sums per query: a lane's sixteen first, each with its place in its lowest bits, then the two lanes of the
+            // query, two blocks at a time.  (med3 where a maximum would do: fmaxf costs an instruction more, which quiets a NaN; there is none.)
+            const __attribute__((address_space(4))) float* units = (const __attribute__((address_space(4))) float*)(a.unit + (uint64_t)t * (BI / 32) + wi * 4);
+            float unit[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) unit[i] = units[i];
+#pragma unroll
+            for (int half = 0; half < 2; half++) {   // blocks half and half + 2
+                float most[2][2], second[2][2];
+#pragma unroll
+                for (int x = 0; x < 2; x++) {
+                    const int i = half + 2 * x;
+                    float start[16];
+                    if constexpr (MODE == kI8Layer) {
+                        const float* from = sStart + (t & 3) * BI + wi * 128 + 4 * lhi + i * 32;
+#pragma unroll
+                        for (int g = 0; g < 4; g++) {
+                            const float4 s = *reinterpret_cast<const float4*>(from + 8 * g);
+                            start[4 * g] = s.x; start[4 * g + 1] = s.y; start[4 * g + 2] = s.z; start[4 * g + 3] = s.w;
+                        }
+                    }
+#pragma unroll
+                    for (int j = 0; j < 2; j++) {
+                        const float p = mine[j] * unit[i];
+                        float h[2] = {-kI8Most, -kI8Most}, l[2] = {-kI8Most, -kI8Most};
+#pragma unroll
+                        for (int v = 0; v < 16; v++) {
+                            int32_t bits = acc[i][j][v];
+                            if constexpr (MODE == kI8Layer) bits = __float_as_int(fmaf(__int_as_float(bits), p, start[v]));
+                            const float s = __int_as_float((bits & ~31) | (v / 4 * 8 + v % 4));
+                            l[v % 2] = __builtin_amdgcn_fmed3f(h[v % 2], l[v % 2], s);
+                            h[v % 2] = __builtin_amdgcn_fmed3f(h[v % 2], s, kI8Most);
+                        }
+                        most[x][j] = __builtin_amdgcn_fmed3f(h[0], h[1], kI8Most);
+                        second[x][j] = fmaxf(fmaxf(__builtin_amdgcn_fmed3f(h[0], h[1], -kI8Most), l[0]), l[1]);
+                    }
+                }
+                const float lower = unit[half], upper = unit[half + 2], own = lhi ? upper : lower;
+#pragma unroll
+                for (int j = 0; j < 2; j++) {
+                    // (after the exchange the lower half's lanes hold both halves' of block `half`, the others of block half + 2)
+                    const auto m = __builtin_amdgcn_permlane32_swap(__float_as_uint(most[0][j]), __float_as_uint(most[1][j]), false, false);
+                    const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(second[0][j]), __float_as_uint(second[1][j]), false, false);
+                    const float m0 = __uint_as_float(m[0]), m1 = __uint_as_float(m[1] | 4u);
+                    const float top = fmaxf(m0, m1), next = fmaxf(fmaxf(fminf(m0, m1), __uint_as_float(s[0])), __uint_as_float(s[1]));
+                    const float p = mine[j] * own;
+                    const auto value = [&](float v) __attribute__((always_inline)) -> uint32_t {
+                        const uint32_t bits = __float_as_uint(v);
+                        const float raised = __uint_as_float(v < 0.0f ? bits & ~31u : bits | 31u);   // (of those with these bits but the place's, the largest)
+                        const float x = MODE == kI8Layer ? raised - kI8StartValue * p : (raised - kI8StartValue) * p;
+                        const _Float16 up = (_Float16)fmaxf(fmaf(fabsf(x), 4.932e-4f, x) + 6.0e-8f, -65504.0f);
+                        return __builtin_bit_cast(uint16_t, up);
+                    };
+                    word[half][j] = i8_word(value(top), value(next), __float_as_uint(top) & 31u);
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                typedef uint32_t u32x2v __attribute__((ext_vector_type(2)));
+                const u32x2v w = {word[0][j], word[1][j]};
+                if (q[j] < a.batch) *reinterpret_cast<u32x2v*>(a.words + (uint64_t)q[j] * a.ldw + t * (BI / 32) + wi * 4 + 2 * lhi) = w;
+            }
+        } else if constexpr (MODE != kF16Store) {
             const uint32_t item0 = t * BI + wi * 128 + 4 * lhi;
 #pragma unroll
             for (int i = 0; i < 4; i++) {
@@ -438,7 +542,7 @@ __global__ __launch_bounds__(64 * WI * WQ) __attribute__((amdgpu_waves_per_eu(WI
         }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (what was asked for beyond the end must not arrive in another workgroup's LDS)
-    if constexpr (MODE != kF16Store) {
+    if constexpr (f16_lists(MODE)) {
         settle();
         const uint32_t r = row0 + wq * 64 + lane;
         if (r < a.batch) a.seg_count[(uint64_t)r * kF16ListStride + list] = min(sFill[lane] & 0x7fffffffu, a.seg_cap);
@@ -469,6 +573,7 @@ static F16SweepArgs f16_args(const F16Job& j)
     a.norm = j.norm; a.bias = j.bias; a.e1 = j.e1; a.bias_raise = j.bias_raise;
     a.cand = j.cand;
     a.Z = (_Float16*)j.Z; a.M = (_Float16*)j.M; a.ldz = j.ldz; a.scale = j.scale;
+    a.unit = j.unit; a.words = j.words; a.ldw = j.ldw;
     a.tiles_q = (j.batch + 255) / 256;   // (one where tiles are lower)
     return a;
 }
@@ -489,7 +594,7 @@ int f16_sweep_run(const F16Job& j, bool layer, uint32_t* lists)
     return layer ? launch_f16_sweep<2, 4, 4, kF16Layer>(a) : launch_f16_sweep<2, 4, 4, kF16Scores>(a);
 }
 
-int f16_store_run(const F16Job& j)
+template <int MODE> static int launch_f16_tiles(const F16Job& j)
 {
     F16SweepArgs a = f16_args(j);
     // Few rows are bound by reading the items: as many of them in flight as LDS holds, and no matrix work for rows that are not there
@@ -504,11 +609,15 @@ int f16_store_run(const F16Job& j)
     a.chunks = (a.tiles_i + a.tiles_per_chunk - 1) / a.tiles_per_chunk;
     a.group = std::min(a.tiles_q, kF16Group);
     switch (shape) {
-    case 0: return launch_f16_sweep<2, 1, 6, kF16Store>(a);
-    case 1: return launch_f16_sweep<2, 2, 4, kF16Store>(a);
-    case 2: return launch_f16_sweep<1, 4, 4, kF16Store>(a);
-    default: return launch_f16_sweep<2, 4, 4, kF16Store>(a);
+    case 0: return launch_f16_sweep<2, 1, 6, MODE>(a);
+    case 1: return launch_f16_sweep<2, 2, 4, MODE>(a);
+    case 2: return launch_f16_sweep<1, 4, 4, MODE>(a);
+    default: return launch_f16_sweep<2, 4, 4, MODE>(a);
     }
 }
+
+int f16_store_run(const F16Job& j) { return launch_f16_tiles<kF16Store>(j); }
+
+int i8_best_run(const F16Job& j, bool starts) { return starts ? launch_f16_tiles<kI8Layer>(j) : launch_f16_tiles<kI8Scores>(j); }
 
 }  // namespace dsx

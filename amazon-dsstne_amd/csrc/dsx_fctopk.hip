@@ -100,11 +100,11 @@ static LayerWorkspace layer_layout(void* base, uint32_t batch, uint32_t n0, uint
     w.table = ScreenTable{};
     w.screen = ScreenWorkspace{};
     if (screened) {
-        w.screen = screen_layout(p, batch, kdim, n, k);
+        w.screen = screen_layout(p, batch, kdim, n, k, screened == 2);
         p += w.screen.bytes;
     }
     if (screened == 1) {
-        w.table = screen_table(p, kdim, n);
+        w.table = screen_table(p, kdim, n, false);
         p += w.table.bytes;
     }
     w.bytes = (size_t)(p - (char*)base);
@@ -259,7 +259,7 @@ static int fc_topk_common(const float* X, uint32_t ldx, const float* W, const fl
     redo.position = position; redo.index = index; redo.fstart = filter_start; redo.fend = filter_end; redo.fidx = filter_index;
     redo.row_flag = w.row_flag; redo.partial = w.cand; redo.done = w.redo_done; redo.keys = keys; redo.values = values;
     if (screened) {
-        const ScreenTable t = table ? screen_table(const_cast<void*>(table), kdim, n) : w.table;
+        const ScreenTable t = table ? screen_table(const_cast<void*>(table), kdim, n, true) : w.table;
         int rc = table ? DSX_OK : screen_build(t, W, n, n, kdim);
         if (rc) return rc;
         ScreenJob j{};
@@ -343,7 +343,7 @@ int dsx_fc_topk(const float* X, uint32_t ldx, const float* W, const float* bias,
 
 uint64_t dsx_screen_table_bytes(uint32_t n, uint32_t kdim)
 {
-    return screen_table(nullptr, kdim, n).bytes;
+    return screen_table(nullptr, kdim, n, true).bytes;
 }
 
 int dsx_screen_table_build(const float* W, uint32_t ldw, uint32_t n, uint32_t kdim, void* table)
@@ -352,7 +352,7 @@ int dsx_screen_table_build(const float* W, uint32_t ldw, uint32_t n, uint32_t kd
     DSX_CHECK_ARG(W && table, "dsx_screen_table_build: null device pointer");
     DSX_CHECK_ARG(((uintptr_t)table % 256) == 0, "dsx_screen_table_build: the table is not 256-byte aligned");
     DSX_CHECK_ARG(n > 0 && n < 1u << 28 && kdim > 0 && kdim <= 4096 && ldw >= n, "dsx_screen_table_build: n = %u, k = %u, ldw = %u", n, kdim, ldw);
-    return screen_build(screen_table(table, kdim, n), W, ldw, n, kdim);
+    return screen_build(screen_table(table, kdim, n, true), W, ldw, n, kdim);
 }
 
 int dsx_fc_topk_screened_reserve(int lane, uint32_t batch, uint32_t kdim, uint32_t n, uint32_t k)

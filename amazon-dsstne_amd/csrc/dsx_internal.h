@@ -18,6 +18,7 @@ struct TestKnobs {
     int knn_f16_sweep = 1;
     size_t allocation_limit = 0;
     int screen = 0;
+    int screen_bytes = 0;
     int knn_no_events = 0;
 };
 

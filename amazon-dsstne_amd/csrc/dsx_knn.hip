@@ -89,7 +89,7 @@ static KnnWorkspace knn_layout(void* base, uint32_t rows_padded, uint32_t num_qu
     screen = screen && !f16 && !split && (table || knn_screens(rows_padded, num_queries, k, dim));
     w.table = ScreenTable{};
     if (screen || table) {
-        w.table = screen_table(p, dim, rows_padded);
+        w.table = screen_table(p, dim, rows_padded, table);
         p += w.table.bytes;
     }
     w.block_scores = (float*)p;
@@ -120,7 +120,7 @@ static KnnWorkspace knn_layout(void* base, uint32_t rows_padded, uint32_t num_qu
     if (split) p += align256((size_t)split_plane_bytes(num_queries, dim));
     w.screen = ScreenWorkspace{};
     if (screen) {
-        w.screen = screen_layout(p, num_queries, dim, rows_padded, k);
+        w.screen = screen_layout(p, num_queries, dim, rows_padded, k, table);
         p += w.screen.bytes;
     }
     w.bytes = (size_t)(p - (char*)base);
@@ -402,6 +402,13 @@ int dsx_testing_set_screen(int mode)
     return DSX_OK;
 }
 
+int dsx_testing_set_screen_bytes(int mode)
+{
+    DSX_CHECK_ARG(mode >= 0 && mode <= 2, "dsx_testing_set_screen_bytes: mode %d (0 to 2)", mode);
+    ctx().knobs.screen_bytes = mode;
+    return DSX_OK;
+}
+
 int dsx_testing_set_knn_no_events(int none)
 {
     ctx().knobs.knn_no_events = none;
@@ -437,7 +444,7 @@ size_t dsx_knn_workspace_bytes_least(uint32_t rows_padded, uint32_t dim, uint32_
 static bool knn_prepares(uint32_t rows_padded, uint32_t dim, uint32_t num_queries, uint32_t k)
 {
     return num_queries > 0 && ctx().knobs.screen != 2 && dim >= 16 && dim <= 4096 && rows_padded >= 8192 && rows_padded >= 64 * k &&
-           screen_table(nullptr, dim, rows_padded).bytes <= ((uint64_t)8 << 30) && k <= 256;
+           screen_table(nullptr, dim, rows_padded, false).bytes <= ((uint64_t)8 << 30) && k <= 256;
 }
 
 size_t dsx_knn_workspace_bytes_prepared(uint32_t rows_padded, uint32_t dim, uint32_t num_queries, uint32_t k)
@@ -638,7 +645,7 @@ int dsx_knn_prepare(const float* items, uint32_t rows_padded, uint32_t padding, 
     *prepared = 0;
     if (!knn_prepares(rows_padded, dim, num_queries, k) || workspace_bytes < dsx_knn_workspace_bytes_prepared(rows_padded, dim, num_queries, k)) return DSX_OK;
     const uint32_t M = rows_padded - padding;
-    const ScreenTable t = screen_table(workspace, dim, rows_padded);
+    const ScreenTable t = screen_table(workspace, dim, rows_padded, true);
     if (int rc = screen_build(t, items, rows_padded, M, dim)) return rc;
     uint32_t stats[3];
     DSX_HIP(hipMemcpyAsync(stats, t.stats, sizeof(stats), hipMemcpyDeviceToHost, ctx().stream));

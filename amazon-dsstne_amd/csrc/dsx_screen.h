@@ -6,7 +6,7 @@
 namespace dsx {
 
 // f16 products of a batch of rows with a range of items (dsx_f16.hip; layouts of knn_f16_ld / knn_f16_rows).
-constexpr int kF16Scores = 0, kF16Layer = 1, kF16Store = 2;
+constexpr int kF16Scores = 0, kF16Layer = 1, kF16Store = 2, kI8Scores = 3, kI8Layer = 4;
 constexpr uint32_t kF16ListStride = 256;   // seg_count's pitch: lists per row at most
 struct F16Job {
     const void* Q;
@@ -23,22 +23,40 @@ struct F16Job {
     void* Z;                  // stored sums: halves, [batch][ldz], ldz a multiple of 256
     void* M;                  // the largest of every 32 of them, [batch][ldz / 32]
     uint64_t ldz;
-    const float* scale;       // [batch] what a row's sums are multiplied by before they are stored
+    const float* scale;       // [batch] what a row's sums are multiplied by before they are stored; products of bytes: the rows' units
+    const float* unit;        // products of bytes: the items' units, one for every 32 of them
+    uint32_t* words;          // products of bytes: [batch][ldw], a word for every 32 items, ldw a multiple of 8
+    uint64_t ldw;
 };
 int f16_sweep_run(const F16Job& j, bool layer, uint32_t* lists);
 int f16_store_run(const F16Job& j);
+// Products of bytes (Q and items of ld / 2 pairs of bytes): a word for every 32 items and row.  starts: of the biases and the columns that always pass.
+int i8_best_run(const F16Job& j, bool starts);
 
-// The table of a screened search: two row-major copies (f16, fp32), the columns' norms and what they are like.  Laid out in
-// screen_table(...).bytes bytes at base, filled by screen_build from W [dim][ldw].
+// A row's word for 32 items: the largest of their sums as a half (upper 16 bits), the second largest as the upper 11 bits of a half, and in between
+// the lowest 5 bits the place of the largest.  Both are upper bounds: i8_first, i8_second.
+__device__ __forceinline__ uint32_t i8_word(uint32_t first, uint32_t second, uint32_t place) { return first << 16 | (second & 0xffe0u) | place; }
+__device__ __forceinline__ float i8_first(uint32_t word) { return (float)__builtin_bit_cast(_Float16, (uint16_t)(word >> 16)); }
+__device__ __forceinline__ float i8_second(uint32_t word)
+{
+    if ((word & 0x7c00u) == 0x7c00u) return (word & 0x8000u) ? -65504.0f : __builtin_inff();
+    return (float)__builtin_bit_cast(_Float16, (uint16_t)((word & 0x8000u) ? word & 0xffe0u : word | 31u));
+}
+
+// The table of a screened search: two row-major copies (f16, fp32), the columns' norms and what they are like; one that is kept holds a copy in bytes
+// as well.  Laid out in screen_table(...).bytes bytes at base, filled by screen_build from W [dim][ldw].
 struct ScreenTable {
     void* items16;
     float* rows32;
     float* norm;
     float* seg_norm;
     uint32_t* stats;
+    void* items8;             // NULL: no bytes
+    float* unit8;
+    float2* error8;
     size_t bytes;
 };
-ScreenTable screen_table(void* base, uint32_t dim, uint64_t n);
+ScreenTable screen_table(void* base, uint32_t dim, uint64_t n, bool kept);
 int screen_build(const ScreenTable& t, const float* W, uint64_t ldw, uint64_t n, uint32_t dim);
 
 // What a call works in.  columns: how many columns' sums there is room for, all of them or a first block's; screen_run goes by that and not by its
@@ -56,9 +74,15 @@ struct ScreenWorkspace {
     uint32_t* keep_count;
     uint64_t* seg;
     uint32_t* seg_count;
+    void* rows8;              // screened in bytes (only these are there then, else they are NULL)
+    float* unit8;
+    float4* error8;
+    uint32_t* words;
+    uint2* near;
+    uint2* near_found;
     size_t bytes;
 };
-ScreenWorkspace screen_layout(void* base, uint32_t batch, uint32_t dim, uint64_t n, uint32_t k);
+ScreenWorkspace screen_layout(void* base, uint32_t batch, uint32_t dim, uint64_t n, uint32_t k, bool kept);
 
 // Nearest neighbours, in pinned memory: the largest norm of the table, a sample of the norms and how many they are; whether a row
 // cannot be screened.

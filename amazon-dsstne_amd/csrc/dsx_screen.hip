@@ -23,9 +23,18 @@
 // formed (raised by their errors, or against bounds lowered by the largest: screen_even), in ranges that grow by a factor, after
 // each of which the lists are cut back to what can still be a result.
 // Candidates of earlier ranges are not scored until the last one is through: what is scored in fp32 is about 1.2 k columns a row.
+//
+// Searches with a table that is kept go in bytes where they would go in ranges (screen_in_bytes): the matrix instructions form products of bytes at twice
+// the rate of halves, and read half as much.  x' = u q, w' = v r with whole numbers q, r of 127 at most; u is a row's unit, v one of 32 columns.  With
+// what the bytes leave out, x = x' + x", w = w' + w", the sum of the products of the bytes is exact and
+//   |s' - s| <= |x"| |w| + |x'| |w"| + (0.1 d + 16) 2^-24 |x| |w| + 3 u v      (the last two: screen_score's roundings, and a start's)
+// which is some fifteen times what halves leave open.  So columns are not told apart by estimates of their scores on both sides: the columns of the k largest
+// sums are scored at once, and their k-th score is what the others' upper bounds are held against (i8_finish_kernel): 1.2 to 4 k columns a row are
+// scored.  No ranges, whose bounds and lists would take as long as the products do, and no lists that fill up.
 #include <algorithm>
 #include <atomic>
 #include <cmath>
+#include <type_traits>
 #include "dsx_screen.h"
 
 namespace dsx {
@@ -47,7 +56,7 @@ __host__ __device__ __forceinline__ float screen_relative(uint32_t dim) { return
 __host__ __device__ __forceinline__ float screen_bias_raise(uint32_t dim) { return ((float)dim + 64.0f) * 6.6e-8f; }
 
 // stats (nearest neighbours): [0] largest norm of a column (the bits of a non-negative float; NaN columns have no part in it: their
-// scores are NaN on every path); [1] sum of the norms of one column in 256, [2] their number
+// scores are NaN on every path); [1] sum of the norms of one column in 256, [2] their number; [4], [5] I8ItemsArgs::error_most
 struct ScreenItemsArgs {
     const float* W;       // [dim][ldw]
     uint64_t ldw;
@@ -215,7 +224,177 @@ __global__ __launch_bounds__(256) void screen_rows_kernel(ScreenRowsArgs a)
     if (bad && a.told) *(volatile uint32_t*)a.told = 1u;
 }
 
-// What the two kernels below have in common.
+// ---- bytes
+// The unit of a vector's bytes: 127 of it are the largest component, and the bytes' own norm stays below 2,000 and their roundings (2,032 with
+// 4,096 components), so that a sum of products of two vectors' bytes is below 2^22.
+__device__ __forceinline__ float i8_unit(float largest, float norm) { return fmaxf(largest * (1.0f / 127.0f) * 1.000001f, norm * (1.0f / 2000.0f)); }
+
+// Norms whose squares are too small to be summed count as what the largest component allows (also what bytes leave out: half a unit each, or
+// everything where the unit is too small to divide by).
+__device__ __forceinline__ float i8_norm(float norm, float largest, uint32_t dim) { return norm < 1e-15f ? largest * 1.01f * sqrtf((float)dim) : norm; }
+__device__ __forceinline__ float i8_left(float left, float unit, float largest, uint32_t dim)
+{
+    const float most = (unit > 1e-35f ? 0.5f * unit : largest) * sqrtf((float)dim);
+    return 1.01f * (unit < 1e-15f ? most : sqrtf(left));
+}
+
+struct I8ItemsArgs {
+    const float* rows32;    // [n][pitch32]
+    const float* norm;      // [n]
+    uint32_t n, dim, pitch32, ld8;
+    int8_t* items8;         // [n rounded up to 256][ld8], zero filled
+    float* unit;            // [n rounded up to 256 / 32]
+    float2* error;          // [n rounded up to 256 / 128] largest norm, and largest norm of what the bytes leave out, of 128 columns
+    uint32_t* error_most;   // the largest two of these (the bits of non-negative floats)
+};
+
+// A workgroup takes 128 columns, 32 after each other: their largest component, then their bytes; a wavefront eight columns.  Bound by memory (the second
+// reading comes from L2).
+__global__ __launch_bounds__(256) void i8_items_kernel(I8ItemsArgs a)
+{
+    __shared__ float sLargest[4], sNorm[4], sLeft[4];
+    const uint32_t lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    float norm_most = 0.0f, left_most = 0.0f;
+    for (uint32_t block = blockIdx.x * 4; block < blockIdx.x * 4 + 4; block++) {
+        const uint32_t c0 = block * 32 + wave * 8;
+        float largest = 0.0f, norms = 0.0f;
+        for (uint32_t c = c0; c < min(c0 + 8, a.n); c++) {
+            const float norm = a.norm[c];
+            if (!(norm < __builtin_inff())) continue;   // always passes, or never: no bytes
+            norms = fmaxf(norms, norm);
+            for (uint32_t d = 4 * lane; d < a.pitch32; d += 4 * kWave) {
+                const float4 v = *reinterpret_cast<const float4*>(a.rows32 + (uint64_t)c * a.pitch32 + d);
+                largest = fmaxf(fmaxf(largest, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
+            }
+        }
+#pragma unroll
+        for (int d = 1; d < kWave; d *= 2) largest = fmaxf(largest, __shfl_xor(largest, d));
+        if (lane == 0) {
+            sLargest[wave] = largest;
+            sNorm[wave] = norms;
+        }
+        __syncthreads();
+        const float norm32 = fmaxf(fmaxf(sNorm[0], sNorm[1]), fmaxf(sNorm[2], sNorm[3]));
+        const float largest32 = fmaxf(fmaxf(sLargest[0], sLargest[1]), fmaxf(sLargest[2], sLargest[3])), unit = i8_unit(largest32, norm32);
+        const float inverse = unit > 1e-35f ? 1.0f / unit : 0.0f;   // (all bytes 0: what they leave out is everything)
+        norm_most = fmaxf(norm_most, i8_norm(norm32, largest32, a.dim));
+        for (uint32_t c = c0; c < c0 + 8; c++) {
+            const bool some = c < a.n && a.norm[min(c, a.n - 1)] < __builtin_inff();
+            float left = 0.0f;
+            for (uint32_t d = 4 * lane; d < a.ld8; d += 4 * kWave) {
+                float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+                if (some && d < a.pitch32) *reinterpret_cast<float4*>(v) = *reinterpret_cast<const float4*>(a.rows32 + (uint64_t)c * a.pitch32 + d);
+                uint32_t bytes = 0;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const float b = fminf(fmaxf(rintf(v[e] * inverse), -127.0f), 127.0f), rest = fmaf(-b, unit, v[e]);
+                    bytes |= ((uint32_t)(int32_t)b & 255u) << (8 * e);
+                    left = fmaf(rest, rest, left);
+                }
+                *reinterpret_cast<uint32_t*>(a.items8 + (uint64_t)c * a.ld8 + d) = bytes;
+            }
+#pragma unroll
+            for (int d = 1; d < kWave; d *= 2) left += __shfl_xor(left, d);
+            // (three units of the sums' last place for the roundings of a sum that has started from something: i8_rows_kernel's |x| is 127 of its units at least)
+            left_most = fmaxf(left_most, i8_left(left, unit, largest32, a.dim) + unit * (4.0f / 127.0f) + 1e-30f);
+        }
+        if (threadIdx.x == 0) a.unit[block] = unit;
+        __syncthreads();
+    }
+    if (lane == 0) sLeft[wave] = left_most;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const float left = fmaxf(fmaxf(sLeft[0], sLeft[1]), fmaxf(sLeft[2], sLeft[3]));
+        a.error[blockIdx.x] = make_float2(norm_most, left);
+        if (__float_as_uint(norm_most) > *(volatile uint32_t*)&a.error_most[0]) atomicMax(&a.error_most[0], __float_as_uint(norm_most));
+        if (__float_as_uint(left) > *(volatile uint32_t*)&a.error_most[1]) atomicMax(&a.error_most[1], __float_as_uint(left));
+    }
+}
+
+struct I8RowsArgs {
+    const float* X;
+    uint32_t ldx, batch, dim, ld8;
+    int8_t* rows8;          // [batch rounded up to 256][ld8], zero filled
+    float* unit;            // [batch] times scale
+    float4* error;          // [batch] a column's sum is wrong by x times its norm, y times the norm of what its bytes leave out, and z at most; w: 1 / scale
+    const uint32_t* stats;  // (the table's) where sums are scaled before they are stored as halves, NULL: they are not
+    uint32_t* row_flag;     // as screen_rows_kernel
+    uint32_t* told;
+    uint32_t* clear;
+    uint32_t clear_words;
+};
+
+// One wavefront per row, which it reads twice.  Bound by latency.
+__global__ __launch_bounds__(256) void i8_rows_kernel(I8RowsArgs a)
+{
+    const uint32_t row = blockIdx.x * 4 + threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    const bool valid = row < a.batch;
+    const float* x = a.X + (uint64_t)row * a.ldx;
+    auto part = [&](uint32_t d, float (&v)[4]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[e] = (valid && d + e < a.dim) ? x[d + e] : 0.0f;
+    };
+    constexpr int G = 4;
+    float held[G][4];
+#pragma unroll
+    for (int g = 0; g < G; g++) part(4 * (g * kWave + lane), held[g]);
+    float sum = 0.0f, largest = 0.0f;
+    auto add = [&](const float (&v)[4]) __attribute__((always_inline)) {
+        sum += (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
+        largest = fmaxf(fmaxf(largest, fmaxf(fabsf(v[0]), fabsf(v[1]))), fmaxf(fabsf(v[2]), fabsf(v[3])));
+    };
+#pragma unroll
+    for (int g = 0; g < G; g++) add(held[g]);
+    for (uint32_t d = G * 4 * kWave + 4 * lane; d < a.dim; d += 4 * kWave) {
+        float v[4];
+        part(d, v);
+        add(v);
+    }
+#pragma unroll
+    for (int d = 1; d < kWave; d *= 2) {
+        sum += __shfl_xor(sum, d);
+        largest = fmaxf(largest, __shfl_xor(largest, d));
+    }
+    const float norm = sqrtf(sum);
+    const bool bad = norm > kF16Max;   // (a NaN in the row: its unit is one too, and the row has no results)
+    const float unit = (norm != norm) ? norm : bad ? 0.0f : i8_unit(largest, norm), inverse = unit > 1e-35f ? 1.0f / unit : 0.0f;
+    float left = 0.0f;
+    auto put = [&](uint32_t d, const float (&v)[4]) __attribute__((always_inline)) {
+        uint32_t bytes = 0;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const float b = inverse > 0.0f ? fminf(fmaxf(rintf(v[e] * inverse), -127.0f), 127.0f) : 0.0f, rest = fmaf(-b, unit, v[e]);
+            bytes |= ((uint32_t)(int32_t)b & 255u) << (8 * e);
+            left = fmaf(rest, rest, left);
+        }
+        if (d < a.ld8) *reinterpret_cast<uint32_t*>(a.rows8 + (uint64_t)row * a.ld8 + d) = bytes;
+    };
+#pragma unroll
+    for (int g = 0; g < G; g++) put(4 * (g * kWave + lane), held[g]);
+    for (uint32_t d = G * 4 * kWave + 4 * lane; d < a.ld8; d += 4 * kWave) {
+        float v[4];
+        part(d, v);
+        put(d, v);
+    }
+#pragma unroll
+    for (int d = 1; d < kWave; d *= 2) left += __shfl_xor(left, d);
+    if (blockIdx.x == 0)
+        for (uint32_t i = threadIdx.x; i < a.clear_words; i += 256) a.clear[i] = 0;
+    if (!valid || lane != 0) return;
+    a.row_flag[row] = bad ? 1u : 0u;
+    float scale = 1.0f;
+    if (a.stats) {
+        const float most = norm * __uint_as_float(a.stats[0]);
+        if (most > 1e-30f && most < 1e30f) scale = ldexpf(1.0f, 10 - ilogbf(most));
+    }
+    const float rest = i8_left(left, unit, largest, a.dim), length = i8_norm(norm, largest, a.dim);
+    a.unit[row] = unit * scale;
+    a.error[row] = make_float4(rest + ((1.25f * (float)a.dim + 64.0f) * 5.9604645e-8f + screen_bias_raise(a.dim)) * length + 1e-30f, (length + rest) * 1.01f + 1e-30f,
+                               1e-30f, 1.0f / scale);
+    if (bad && a.told) *(volatile uint32_t*)a.told = 1u;
+}
+
+// What the kernels below have in common.
 struct ScreenFoldArgs {
     uint32_t batch, k, n;
     const float* e1;
@@ -251,6 +430,13 @@ struct ScreenFoldArgs {
     uint64_t ldz;
     const float* scale;
     uint32_t stored;         // columns of Z
+    // in bytes
+    const uint32_t* words;   // [batch][ldw]
+    uint64_t ldw;
+    const float2* error_items;
+    const float4* error_rows;
+    const uint2* near;       // i8_near_kernel's
+    const uint2* near_found;
     // final
     const float* X;
     uint32_t ldx, dim, pitch32;
@@ -276,14 +462,19 @@ __device__ __forceinline__ uint64_t screen_raised(const ScreenFoldArgs& a, uint6
     return ((uint64_t)score_key(norm < __builtin_inff() ? fmaf(e1, norm, x) : __builtin_inff()) << 32) | (uint32_t)word;
 }
 
-// The sum z below which nothing can be a result when k columns score at least t (as a sum); -inf: anything can.
+// The sum z below which nothing can be a result when k columns have scores of at least this key.
+__device__ __forceinline__ float screen_cut_key(const ScreenFoldArgs& a, uint32_t key, float e0)
+{
+    const float z = preactivation_bound(key, a.act, a.slope, a.alpha, a.lambda);
+    const float cut = z - e0 * 1.001f - fabsf(z) * 2.3841858e-7f;   // (the subtraction itself is rounded)
+    return (cut == cut) ? cut : -__builtin_inff();
+}
+
+// The same when k columns score at least t (as a sum); -inf: anything can.
 __device__ __forceinline__ float screen_cut(const ScreenFoldArgs& a, float t, float e0)
 {
     if (!(t > -__builtin_inff())) return -__builtin_inff();
-    const float y = activate_rt(t, a.act, a.slope, a.alpha, a.lambda);
-    const float z = preactivation_bound(score_key(y), a.act, a.slope, a.alpha, a.lambda);
-    const float cut = z - e0 * 1.001f - fabsf(z) * 2.3841858e-7f;   // (the subtraction itself is rounded)
-    return (cut == cut) ? cut : -__builtin_inff();
+    return screen_cut_key(a, score_key(activate_rt(t, a.act, a.slope, a.alpha, a.lambda)), e0);
 }
 
 __device__ __forceinline__ void screen_flag(const ScreenFoldArgs& a, uint32_t b)
@@ -293,22 +484,22 @@ __device__ __forceinline__ void screen_flag(const ScreenFoldArgs& a, uint32_t b)
     if (a.admit) a.admit[b] = 0xffffffffu;   // a NaN: nothing more of the row is wanted
 }
 
-// The row's candidates sList[0 .. count) scored in fp32 and its k best written.  Sixteen lanes per candidate; the order of a sum depends on
-// nothing but its length.  Every lane of the workgroup calls this.
-// first: the caller's component threadIdx.x of the row; listed: whether the row has a listed column (the same for the workgroup).
-template <int T>
-__device__ __forceinline__ void screen_finish(const ScreenFoldArgs& a, uint32_t b, uint64_t* sList, uint32_t count, float* sX, float first, bool listed)
+// The row itself into LDS, zero filled to whole rounds of the loop below; first: the caller's component threadIdx.x of it.
+template <int T> __device__ __forceinline__ void screen_row(const ScreenFoldArgs& a, uint32_t b, float* sX, float first)
 {
-    __shared__ uint64_t sBest[256];   // by rank (k is 256 at most)
     const uint32_t dpad = (a.dim + 63) / 64 * 64;
     if (threadIdx.x < dpad) sX[threadIdx.x] = first;
     for (uint32_t d = T + threadIdx.x; d < dpad; d += T) sX[d] = (d < a.dim) ? a.X[(uint64_t)b * a.ldx + d] : 0.0f;
-    if (threadIdx.x < 256) sBest[threadIdx.x] = 0;
-    __syncthreads();
+}
+
+// The row's candidates sList[from .. count) scored in fp32: their words get the scores' keys, and become 0 where a score is no number.  Sixteen lanes per
+// candidate; the order of a sum depends on nothing but its length.  Every lane of the workgroup calls this.
+template <int T, int STEPS = 2> __device__ __forceinline__ void screen_score(const ScreenFoldArgs& a, uint64_t* sList, uint32_t from, uint32_t count, const float* sX)
+{
     // (four candidates of a group of lanes at a time: their rows are waited for together)
     constexpr int U = 4;
     const uint32_t sub = threadIdx.x % 16;
-    for (uint32_t e0 = threadIdx.x / 16; e0 < count; e0 += T / 16 * U) {
+    for (uint32_t e0 = from + threadIdx.x / 16; e0 < count; e0 += T / 16 * U) {
         uint32_t col[U];
         float sum[U];
 #pragma unroll
@@ -316,7 +507,7 @@ __device__ __forceinline__ void screen_finish(const ScreenFoldArgs& a, uint32_t 
             col[u] = ~(uint32_t)sList[min(e0 + T / 16 * u, count - 1)];
             sum[u] = 0.0f;
         }
-#pragma unroll 2
+#pragma unroll STEPS
         for (uint32_t d = 4 * sub; d < a.pitch32; d += 64) {
             const float4 x = *reinterpret_cast<const float4*>(sX + d);
             float4 v[U];
@@ -342,7 +533,12 @@ __device__ __forceinline__ void screen_finish(const ScreenFoldArgs& a, uint32_t 
             }
         }
     }
-    __syncthreads();
+}
+
+// The k best of the scored words sList[0 .. count) written.  sBest: 256 words, cleared before the caller's last barrier.
+template <int T>
+__device__ __forceinline__ void screen_results(const ScreenFoldArgs& a, uint32_t b, const uint64_t* sList, uint32_t count, uint64_t* sBest, bool listed)
+{
     for (uint32_t i = threadIdx.x; i < count; i += T) {
         const uint64_t w = sList[i];
         if (w == 0) continue;
@@ -365,6 +561,20 @@ __device__ __forceinline__ void screen_finish(const ScreenFoldArgs& a, uint32_t 
     // A listed column scores 0, not nothing (utils/Filters.cpp:62 multiplies, kCalculateTopK then sees the zero): when the row's k-th
     // score is not above 0, or the row has fewer than k scores, such a zero belongs in the result, and the row is computed again.
     if (threadIdx.x == 0 && listed && (uint32_t)(sBest[a.k - 1] >> 32) <= score_key(0.0f)) screen_flag(a, b);
+}
+
+// The row's candidates sList[0 .. count) scored and its k best written.  Every lane of the workgroup calls this.
+// first: the caller's component threadIdx.x of the row; listed: whether the row has a listed column (the same for the workgroup).
+template <int T>
+__device__ __forceinline__ void screen_finish(const ScreenFoldArgs& a, uint32_t b, uint64_t* sList, uint32_t count, float* sX, float first, bool listed)
+{
+    __shared__ uint64_t sBest[256];   // by rank (k is 256 at most)
+    screen_row<T>(a, b, sX, first);
+    if (threadIdx.x < 256) sBest[threadIdx.x] = 0;
+    __syncthreads();
+    screen_score<T>(a, sList, 0, count, sX);
+    __syncthreads();
+    screen_results<T>(a, b, sList, count, sBest, listed);
 }
 
 // A lower bound of the k-th largest of the workgroup's keys (0: dead ones, not counted), exact in its upper 24 bits; 0 where there are
@@ -418,12 +628,12 @@ template <int N, int T = 256> __device__ __forceinline__ uint32_t block_kth_key(
     return prefix;
 }
 
-// The k-th largest of 64 * N keys of a wavefront, exact in its upper 20 bits, 0 if there are fewer.  (As the top-K kernels' key search.)
-template <int N> __device__ __forceinline__ uint32_t screen_wave_kth(const uint32_t (&key)[N], uint32_t k)
+// The k-th largest of 64 * N keys of a wavefront, exact but for its LAST lowest bits, 0 if there are fewer.  (As the top-K kernels' key search.)
+template <int N, int LAST = 12> __device__ __forceinline__ uint32_t screen_wave_kth(const uint32_t (&key)[N], uint32_t k)
 {
     uint32_t t = 0;
 #pragma unroll 1
-    for (int bit = 30; bit >= 12; bit -= 2) {
+    for (int bit = 30; bit >= LAST; bit -= 2) {
         const uint32_t c1 = t | (1u << bit), c2 = t | (2u << bit), c3 = t | (3u << bit);
         uint32_t n1 = 0, n2 = 0, n3 = 0;
 #pragma unroll
@@ -820,6 +1030,360 @@ __global__ __launch_bounds__(256, 4) void screen_fold_kernel(ScreenFoldArgs a)
     }
 }
 
+constexpr uint32_t kBestWords = 2048;    // candidates of a row at a time
+constexpr uint32_t kBestMost = 16384;    // candidates of a row after which it is computed otherwise (thousands of scores tied at the top)
+constexpr uint32_t kBestColumns = 1u << 20;
+constexpr uint32_t kNearWords = 4096;    // words of a row that are listed
+
+// Sums of bytes: a word for every 32 columns says what the largest of their sums is at most, whose it is, and what the others are at most.  The columns
+// of the k largest words are scored first; then all columns whose words reach the k-th of those scores, and where the others of a block
+// reach it, all of the block.  So a row's bound is a score and not an estimate of one: e1 |w| + e2 |w's rest| is open on one side of it only.
+//
+// Two kernels.  i8_near_kernel reads a row's words, once, and lists those that can reach the bound whatever it will be: the k-th word less twice the
+// largest error.  i8_finish_kernel scores.  (In one kernel of sixteen wavefronts a row, 610 us for 4,096 rows of 1,000,000 columns, 100 results:
+// two rows to a compute unit, and all sixteen wavefronts went through the searches and lists of a few hundred words.)
+struct I8NearArgs {
+    uint32_t batch, k, n;
+    const uint32_t* words;
+    uint64_t ldw;
+    const float4* error_rows;
+    const float2* error_most;
+    const uint32_t* row_flag;
+    uint32_t position;
+    const uint32_t* index;
+    const uint64_t* fstart;
+    const uint64_t* fend;
+    const uint32_t* fidx;
+    uint2* near;             // [batch][kNearWords] block (kNearDead: its largest sum is a listed column's) and word, as an integer in the order of halves
+    uint2* near_found;       // [batch] how many there are, and the word that k columns reach
+};
+constexpr uint32_t kNearDead = 0x80000000u;
+constexpr int32_t kNoWord = INT32_MIN;
+
+// A word as an integer in the order of its first half, and back.
+__device__ __forceinline__ int32_t i8_sortable(int32_t word) { return word ^ ((word >> 31) & 0x7fff0000); }
+
+// A row per workgroup, 4 V words a lane.  Bound by reading them.
+template <int V, int T>
+__global__ __launch_bounds__(T, T == 1024 ? 8 : 4) void i8_near_kernel(I8NearArgs a)
+{
+    __builtin_amdgcn_s_setprio(3);
+    constexpr int B = V * T * 4 / 32, R = V == 1 ? 4 : V == 4 ? 2 : 1;   // words of a bitmap of blocks; keys a lane has in the search
+    __shared__ uint32_t sDead[B], sTop[R * T];
+    __shared__ uint32_t sNears, sKth;
+    const uint32_t b = blockIdx.x, tid = threadIdx.x;
+    if (a.row_flag[b] != 0) return;
+    const uint32_t blocks = (a.n + 31) / 32;
+    const uint32_t* words = a.words + (uint64_t)b * a.ldw;
+    int4 w[V];
+#pragma unroll
+    for (int v = 0; v < V; v++) {
+        const uint32_t at = min((v * T + tid) * 4, (uint32_t)a.ldw - 4);   // (ldw is a multiple of 8)
+        w[v] = *reinterpret_cast<const int4*>(words + at);
+    }
+    uint64_t fs = 0, fe = 0;
+    if (a.fidx) {
+        uint32_t r = a.position + b;
+        if (a.index) r = a.index[r];
+        fs = a.fstart[r];
+        fe = a.fend[r];
+    }
+    const float4 error = a.error_rows[b];
+    const float2 most = *a.error_most;
+    if (tid == 0) sNears = 0;
+    const bool some_dead = fe > fs || a.n % 32 != 0;   // the same for the workgroup
+    if (some_dead) {
+        for (uint32_t i = tid; i < B; i += T) sDead[i] = 0;
+        __syncthreads();
+        for (uint64_t t = fs + tid; t < fe; t += T) {
+            const uint32_t c = a.fidx[t];
+            if (c < a.n && (words[c >> 5] & 31u) == (c & 31u)) atomicOr(&sDead[c >> 10], 1u << ((c >> 5) & 31u));
+        }
+        // (the largest sum of the last block may be one of a column beyond it)
+        if (tid == 0 && a.n % 32 != 0 && (words[blocks - 1] & 31u) >= a.n % 32) atomicOr(&sDead[(blocks - 1) >> 5], 1u << ((blocks - 1) & 31u));
+        __syncthreads();
+    }
+    auto part = [&](int4& x, int c) __attribute__((always_inline)) -> int32_t& { return c == 0 ? x.x : c == 1 ? x.y : c == 2 ? x.z : x.w; };
+    int32_t top[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) top[r] = kNoWord;
+#pragma unroll
+    for (int v = 0; v < V; v++) {
+        const uint32_t q = v * T + tid;
+        const uint32_t dead = (some_dead && q * 4 < blocks) ? sDead[q / 8] >> (q % 8 * 4) : 0u;
+        const bool whole = (uint32_t)(v + 1) * T * 4 <= blocks;
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const int32_t x = (whole || q * 4 + c < blocks) ? i8_sortable(part(w[v], c)) : kNoWord;
+            part(w[v], c) = x;
+            top[c % R] = max(top[c % R], ((dead >> c) & 1u) ? kNoWord : x);
+        }
+    }
+    // One wavefront searches.  The k-th of the lanes' largest is a word that k columns reach, and seldom much below the k-th of all.
+#pragma unroll
+    for (int r = 0; r < R; r++) sTop[r * T + tid] = top[r] == kNoWord ? 0u : (uint32_t)top[r] ^ 0x80000000u;
+    __syncthreads();
+    if (__builtin_amdgcn_readfirstlane(tid / kWave) == (b >> 8) % (T / kWave)) {
+        constexpr int K = R * T / kWave;
+        uint32_t key[K];
+#pragma unroll
+        for (int i = 0; i < K; i++) key[i] = sTop[i * kWave + tid % kWave];
+        const uint32_t t = screen_wave_kth<K, 16>(key, a.k);
+        if (tid % kWave == 0) sKth = t;
+    }
+    __syncthreads();
+    const uint32_t kth = sKth;
+    const int32_t t0 = kth != 0 ? (int32_t)(kth ^ 0x80000000u) : kNoWord + 1;
+    // What can reach the bound: a score of the k is no further below its word than what a half is rounded up by and the error.
+    int32_t near = kNoWord + 1;
+    if (kth != 0) {
+        const float step = error.w, z = i8_first((uint32_t)i8_sortable(t0)) * step, wide = fmaf(error.x, most.x, error.y * most.y);
+        const float low = (z - fabsf(z) * 2.0e-3f - 2.1f * wide - 2.1f * error.z - 4e-7f * step) / step;
+        if (low > -65000.0f && z < 60000.0f * step) {
+            const uint32_t h = __builtin_bit_cast(uint16_t, (_Float16)(low - fabsf(low) * 1.0e-3f - 1.2e-7f));
+            near = i8_sortable((int32_t)(h << 16));
+        }
+    }
+    uint32_t mine = 0;
+#pragma unroll
+    for (int v = 0; v < V; v++)
+#pragma unroll
+        for (int c = 0; c < 4; c++) mine += part(w[v], c) >= near;
+    uint32_t at = mine;
+#pragma unroll
+    for (int d = 1; d < kWave; d *= 2) {
+        const uint32_t below = __shfl_up(at, d);
+        if (tid % kWave >= (uint32_t)d) at += below;
+    }
+    uint32_t base = 0;
+    if (tid % kWave == kWave - 1) base = atomicAdd(&sNears, at);
+    at += __shfl(base, kWave - 1) - mine;
+    uint2* out = a.near + (uint64_t)b * kNearWords;
+#pragma unroll
+    for (int v = 0; v < V; v++) {
+        const uint32_t q = v * T + tid;
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const int32_t x = part(w[v], c);
+            if (x >= near) {
+                const uint32_t dead = some_dead ? (sDead[q / 8] >> (q % 8 * 4 + c) & 1u) * kNearDead : 0u;
+                if (at < kNearWords) out[at] = make_uint2((q * 4 + c) | dead, (uint32_t)x);
+                at++;
+            }
+        }
+    }
+    __syncthreads();
+    if (tid == 0) a.near_found[b] = make_uint2(sNears, (uint32_t)t0);
+}
+
+// The k-th largest key of the list's first `count` words (256 * N at most), exact but for the lowest 8 bits; 0: fewer.  The wavefront that calls it.
+template <int N> __device__ __forceinline__ uint32_t list_kth(const uint64_t* sList, uint32_t count, uint32_t k)
+{
+    uint32_t key[N];
+#pragma unroll
+    for (int i = 0; i < N; i++) key[i] = (i * kWave + threadIdx.x < count) ? (uint32_t)(sList[i * kWave + threadIdx.x] >> 32) : 0u;
+    return screen_wave_kth<N, 8>(key, k);
+}
+
+// A row per workgroup; several of them to a compute unit hide each other's latency: candidates' rows, twice, and a search after each.  Nothing fills up:
+// what a round's list has no room for comes with the next one, against a bound that only rises.
+__global__ __launch_bounds__(256, 4) void i8_finish_kernel(ScreenFoldArgs a)
+{
+    __builtin_amdgcn_s_setprio(3);
+    constexpr int T = 256, B = kBestColumns / 32 / 32;
+    constexpr uint32_t kOpen = 32;               // blocks of which all columns are looked at, per round
+    __shared__ uint64_t sList[kBestWords];
+    __shared__ uint64_t sBest[256];
+    __shared__ uint32_t sDead[B], sHot[B], sMore[B];   // blocks whose largest sum is a listed column's (for `all`); is one to be scored; of which the others are
+    __shared__ uint32_t sHist[258];
+    __shared__ uint32_t sOpen[kOpen], sMask[kOpen];
+    __shared__ uint32_t sCount, sOpened, sKth;
+    extern __shared__ __attribute__((aligned(16))) uint32_t sDyn[];   // the row
+    float* sX = reinterpret_cast<float*>(sDyn);
+    const uint32_t b = blockIdx.x, tid = threadIdx.x;
+    if (a.row_flag[b] != 0) return;
+    const uint32_t blocks = (a.n + 31) / 32, bitmap = (blocks + 31) / 32;
+    const uint32_t* words = a.words + (uint64_t)b * a.ldw;
+    const uint2* near = a.near + (uint64_t)b * kNearWords;
+    const uint2 found = a.near_found[b];
+    uint64_t fs = 0, fe = 0;
+    if (a.fidx) {
+        uint32_t r = a.position + b;
+        if (a.index) r = a.index[r];
+        fs = a.fstart[r];
+        fe = a.fend[r];
+    }
+    const float4 error = a.error_rows[b];
+    const float e1 = error.x, e2 = error.y, e0 = error.z, step = error.w;
+    const float first = (tid < a.dim) ? a.X[(uint64_t)b * a.ldx + tid] : 0.0f;
+    for (uint32_t i = tid; i < bitmap; i += T) sHot[i] = sMore[i] = 0;
+    sBest[tid] = 0;
+    if (tid == 0) sCount = 0;
+    screen_row<T>(a, b, sX, first);
+    bool any = false;
+    for (uint64_t t = fs + tid; t < fe; t += T) any |= a.fidx[t] < a.n;
+    const bool listed = __syncthreads_or(any) != 0;
+    if (!(e1 == e1)) {   // a row that is no number has no scores
+        screen_results<T>(a, b, sList, 0, sBest, listed);
+        return;
+    }
+    const uint32_t nears = found.x;
+    const int32_t t0 = (int32_t)found.y;
+    const bool all = nears > kNearWords;   // (more than there was room for: the words are read again; the same for the whole workgroup, as are all of these)
+    if (all) {
+        for (uint32_t i = tid; i < bitmap; i += T) sDead[i] = 0;
+        __syncthreads();
+        for (uint64_t t = fs + tid; t < fe; t += T) {
+            const uint32_t c = a.fidx[t];
+            if (c < a.n && (words[c >> 5] & 31u) == (c & 31u)) atomicOr(&sDead[c >> 10], 1u << ((c >> 5) & 31u));
+        }
+        if (tid == 0 && a.n % 32 != 0 && (words[blocks - 1] & 31u) >= a.n % 32) atomicOr(&sDead[(blocks - 1) >> 5], 1u << ((blocks - 1) & 31u));
+        __syncthreads();
+    }
+    // Every block that can reach the bound, with its word in the order of integers (and its errors), eight a lane at a time: their loads are waited
+    // for together.
+    auto each = [&](auto errors, auto&& look) __attribute__((always_inline)) {
+        constexpr int G = 8;
+        const uint32_t total = all ? blocks : nears;
+        for (uint32_t base = tid; base < total; base += G * T) {
+            uint2 x[G];
+            float2 e[G];
+#pragma unroll
+            for (int g = 0; g < G; g++) {
+                const uint32_t i = base + g * T;
+                x[g] = make_uint2(0, (uint32_t)kNoWord);
+                if (g == 0 || i < total) x[g] = all ? make_uint2(i, words[i]) : near[i];
+            }
+            if constexpr (errors.value) {
+#pragma unroll
+                for (int g = 0; g < G; g++)
+                    if (g == 0 || base + g * T < total) e[g] = a.error_items[(x[g].x & ~kNearDead) / 4];
+            }
+#pragma unroll
+            for (int g = 0; g < G; g++) {
+                if (base + g * T >= total) break;
+                const uint32_t block = x[g].x & ~kNearDead;
+                look(block, all ? i8_sortable((int32_t)x[g].y) : (int32_t)x[g].y, all ? ((sDead[block >> 5] >> (block & 31u)) & 1u) != 0 : (x[g].x & kNearDead) != 0, e[g]);
+            }
+        }
+    };
+    each(std::false_type{}, [&](uint32_t block, int32_t x, bool dead, float2) {
+        if (x >= t0 && !dead) {
+            const uint32_t at = atomicAdd(&sCount, 1u);
+            if (at < kBestWords) sList[at] = (uint32_t)~(block * 32 + ((uint32_t)x & 31u));
+        }
+    });
+    __syncthreads();
+    uint32_t count = sCount, scored = count, kept = 0;
+    if (count > kBestWords) {
+        if (tid == 0) screen_flag(a, b);
+        return;
+    }
+    float cut = 0.0f;
+    bool begun = false;
+    constexpr int W = B / T;
+    uint32_t hot[W], more[W];
+    for (;;) {
+        // Scores of what is new, and what is left of the list: what is no worse than its k-th.
+        screen_score<T, 4>(a, sList, kept, count, sX);
+        __syncthreads();
+        constexpr int L = kBestWords / T;
+        uint64_t word[L];
+        uint32_t key[L];
+#pragma unroll
+        for (int u = 0; u < L; u++) {
+            word[u] = (u * T + tid < count) ? sList[u * T + tid] : 0ull;
+            key[u] = (uint32_t)(word[u] >> 32);
+        }
+        uint32_t t;
+        if (count <= 8 * kWave) {
+            if (tid < kWave) {
+                t = count <= 2 * kWave ? list_kth<2>(sList, count, a.k) : count <= 4 * kWave ? list_kth<4>(sList, count, a.k) : list_kth<8>(sList, count, a.k);
+                if (tid == 0) sKth = t;
+            }
+            __syncthreads();
+            t = sKth;
+        } else t = block_kth_key<L, T>(key, count, a.k, sHist);   // (its barriers: every lane has its words)
+        if (tid == 0) sCount = 0;
+        cut = (t != 0) ? screen_cut_key(a, t, e0) : -__builtin_inff();
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < L; u++)
+            if (word[u] != 0 && key[u] >= t) sList[atomicAdd(&sCount, 1u)] = word[u];
+        __syncthreads();
+        kept = sCount;
+        if (!begun) {
+            begun = true;
+            each(std::true_type{}, [&](uint32_t block, int32_t x, bool dead, float2 e) {
+                const float wide = fmaf(e1, e.x, e2 * e.y) * 1.000001f;
+                const uint32_t word = (uint32_t)i8_sortable(x);
+                if (!(fmaf(i8_first(word), step, wide) >= cut)) return;
+                if (x < t0 && !dead) atomicOr(&sHot[block >> 5], 1u << (block & 31u));
+                if (fmaf(i8_second(word), step, wide) >= cut) atomicOr(&sMore[block >> 5], 1u << (block & 31u));
+            });
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < W; u++) {
+                const uint32_t i = u * T + tid;
+                hot[u] = i < bitmap ? sHot[i] : 0u;
+                more[u] = i < bitmap ? sMore[i] : 0u;
+            }
+        }
+        uint32_t pending = 0;
+#pragma unroll
+        for (int u = 0; u < W; u++) pending |= hot[u] | more[u];
+        if (tid == 0) sOpened = 0;
+        if (!__syncthreads_or(pending != 0)) break;
+        if (scored > kBestMost || kept > kBestWords / 2) {
+            if (tid == 0) screen_flag(a, b);
+            return;
+        }
+#pragma unroll
+        for (int u = 0; u < W; u++)
+            while (hot[u] != 0) {
+                const uint32_t at = atomicAdd(&sCount, 1u);
+                if (at >= kBestWords) break;
+                const uint32_t block = (u * T + tid) * 32 + (uint32_t)__builtin_ctz(hot[u]);
+                sList[at] = (uint32_t)~(block * 32 + (words[block] & 31u));
+                hot[u] &= hot[u] - 1;
+            }
+        __syncthreads();
+        count = min(sCount, kBestWords);
+        __syncthreads();
+        if (count <= kBestWords - kOpen * 32) {
+#pragma unroll
+            for (int u = 0; u < W; u++)
+                while (more[u] != 0) {
+                    const uint32_t at = atomicAdd(&sOpened, 1u);
+                    if (at >= kOpen) break;
+                    const uint32_t block = (u * T + tid) * 32 + (uint32_t)__builtin_ctz(more[u]);
+                    sOpen[at] = block;
+                    sMask[at] = 1u << (words[block] & 31u);   // (scored, or not wanted)
+                    more[u] &= more[u] - 1;
+                }
+            __syncthreads();
+            const uint32_t opened = min(sOpened, kOpen);
+            if (opened != 0) {
+                for (uint64_t t = fs + tid; t < fe; t += T) {
+                    const uint32_t c = a.fidx[t];
+                    for (uint32_t o = 0; o < opened; o++)
+                        if (sOpen[o] == c >> 5) atomicOr(&sMask[o], 1u << (c & 31u));
+                }
+                __syncthreads();
+                for (uint32_t i = tid; i < opened * 32; i += T) {
+                    const uint32_t col = sOpen[i / 32] * 32 + i % 32;
+                    if (!((sMask[i / 32] >> (i % 32)) & 1u) && col < a.n) sList[atomicAdd(&sCount, 1u)] = (uint32_t)~col;
+                }
+                __syncthreads();
+                count = min(sCount, kBestWords);
+                __syncthreads();
+            }
+        }
+        scored += count - kept;
+    }
+    screen_results<T>(a, b, sList, kept, sBest, listed);
+}
+
 // What can be screened with copies of the table made in the call: the preparation costs what about 130 rows' fp32 products do.  Limits: the row in LDS,
 // and 8 GiB for the two copies.  A layer that is taken is faster so than in fp32 ranges: 714 calls of dsx_fc_topk, 512 to 4,096 rows, 64 to 1,024
 // components, 16,384 to 1,000,000 columns, k 10 to 256, with and without a filter, take 0.16 to 0.81 of the time (us, fp32 / screened: 512 x 1,024 x
@@ -872,7 +1436,19 @@ static uint32_t screen_first_columns(uint32_t n, uint32_t k)
     return std::min(c, n);
 }
 
-ScreenTable screen_table(void* base, uint32_t dim, uint64_t n)
+// Whether a search with a kept table goes in bytes: where it would go in ranges of halves, for as many columns as a row's words are looked at by one
+// workgroup (us, halves / bytes, a whole pass with its hidden layer, upload and results: 4,096 x 512 x 1,000,000 top 100 with a filter 4,219 / 3,000, searches of 4,096 x 128 x
+// 1,000,000 top 100 1,924 / 1,417).
+static bool screen_in_bytes(uint32_t batch, uint32_t dim, uint64_t n, uint32_t k)
+{
+    if (ctx().knobs.screen_bytes != 0) return ctx().knobs.screen_bytes == 1 && n <= kBestColumns && n >= 64 * (uint64_t)k;
+    if (ctx().knobs.fc_topk_first_columns || n > kBestColumns || n < 64 * (uint64_t)k) return false;
+    return !screen_stored(batch, n, k);
+}
+
+static uint32_t i8_ld(uint32_t dim) { return (dim + 127) / 128 * 128; }
+
+ScreenTable screen_table(void* base, uint32_t dim, uint64_t n, bool kept)
 {
     ScreenTable t;
     char* p = (char*)base;
@@ -887,14 +1463,42 @@ ScreenTable screen_table(void* base, uint32_t dim, uint64_t n)
     p += align256(rows / 64 * sizeof(float));
     t.stats = (uint32_t*)p;
     p += 256;
+    t.items8 = nullptr;
+    t.unit8 = nullptr;
+    t.error8 = nullptr;
+    if (kept && n <= kBestColumns) {
+        t.items8 = p;
+        p += align256(rows * i8_ld(dim));
+        t.unit8 = (float*)p;
+        p += align256(rows / 32 * sizeof(float));
+        t.error8 = (float2*)p;
+        p += align256(rows / 128 * sizeof(float2));
+    }
     t.bytes = (size_t)(p - (char*)base);
     return t;
 }
 
-ScreenWorkspace screen_layout(void* base, uint32_t batch, uint32_t dim, uint64_t n, uint32_t k)
+ScreenWorkspace screen_layout(void* base, uint32_t batch, uint32_t dim, uint64_t n, uint32_t k, bool kept)
 {
-    ScreenWorkspace w;
+    ScreenWorkspace w{};
     char* p = (char*)base;
+    if (kept && screen_in_bytes(batch, dim, n, k)) {
+        w.columns = (uint32_t)n;
+        w.rows8 = p;
+        p += align256(knn_f16_rows(batch) * i8_ld(dim));
+        w.unit8 = (float*)p;
+        p += align256((size_t)batch * sizeof(float));
+        w.error8 = (float4*)p;
+        p += align256((size_t)batch * sizeof(float4));
+        w.words = (uint32_t*)p;
+        p += align256(batch * ((n + 255) / 256 * 8) * sizeof(uint32_t));
+        w.near = (uint2*)p;
+        p += align256((size_t)batch * kNearWords * sizeof(uint2));
+        w.near_found = (uint2*)p;
+        p += align256((size_t)batch * sizeof(uint2));
+        w.bytes = (size_t)(p - (char*)base);
+        return w;
+    }
     // (decided here for every search in this workspace, which may be of fewer columns: pad rows of an item table)
     const uint64_t columns = w.columns = screen_stored(batch, n, k) ? (uint32_t)n : screen_first_columns((uint32_t)n, k);
     w.rows16 = p;
@@ -935,11 +1539,28 @@ int screen_build(const ScreenTable& t, const float* W, uint64_t ldw, uint64_t n,
     i.out16 = (_Float16*)t.items16; i.out32 = t.rows32; i.norm = t.norm; i.seg_norm = t.seg_norm; i.stats = t.stats;
     hipLaunchKernelGGL(screen_items_kernel, dim3((uint32_t)(knn_f16_rows(n) / 64)), dim3(256), 0, s, i);
     DSX_LAUNCH_CHECK("screen_items_kernel");
+    if (t.items8) {
+        I8ItemsArgs e{};
+        e.rows32 = t.rows32; e.norm = t.norm; e.n = (uint32_t)n; e.dim = dim; e.pitch32 = i.pitch32; e.ld8 = i8_ld(dim);
+        e.items8 = (int8_t*)t.items8; e.unit = t.unit8; e.error = t.error8; e.error_most = t.stats + 4;
+        hipLaunchKernelGGL(i8_items_kernel, dim3((uint32_t)(knn_f16_rows(n) / 128)), dim3(256), 0, s, e);
+        DSX_LAUNCH_CHECK("i8_items_kernel");
+    }
     return DSX_OK;
 }
 
 int screen_rows(const ScreenJob& j, const ScreenTable& t, const ScreenWorkspace& w, ScreenNotes* notes)
 {
+    if (w.words) {
+        I8RowsArgs r{};
+        r.X = j.X; r.ldx = j.ldx; r.batch = j.batch; r.dim = j.dim; r.ld8 = i8_ld(j.dim);
+        r.rows8 = (int8_t*)w.rows8; r.unit = w.unit8; r.error = w.error8;
+        r.stats = j.bias ? nullptr : t.stats;
+        r.row_flag = j.row_flag; r.told = j.told; r.clear = j.clear; r.clear_words = j.clear_words;
+        hipLaunchKernelGGL(i8_rows_kernel, dim3((uint32_t)(knn_f16_rows(j.batch) / 4)), dim3(256), 0, ctx().stream, r);
+        DSX_LAUNCH_CHECK("i8_rows_kernel");
+        return DSX_OK;
+    }
     ScreenRowsArgs r{};
     r.whole = (uintptr_t)j.X % 16 == 0 && j.ldx % 4 == 0;
     r.X = j.X; r.ldx = j.ldx; r.batch = j.batch; r.dim = j.dim; r.ld = screen_ld(j.dim);
@@ -984,8 +1605,46 @@ static int launch_pick(const ScreenFoldArgs& a, bool keep)
     return launch_pick_as<1024, 1, 32, kPickFinal>(a, lds);
 }
 
+// What a search in bytes and one in halves tell the kernels that end with results.
+static ScreenFoldArgs fold_args(const ScreenJob& j, const ScreenTable& t)
+{
+    ScreenFoldArgs a{};
+    a.batch = j.batch; a.k = j.k; a.n = j.n;
+    a.act = j.act; a.slope = j.slope; a.alpha = j.alpha; a.lambda = j.lambda;
+    a.row_flag = j.row_flag; a.told = j.told;
+    a.position = j.position; a.index = j.index; a.fstart = j.fstart; a.fend = j.fend; a.fidx = j.fidx;
+    a.X = j.X; a.ldx = j.ldx; a.dim = j.dim; a.pitch32 = screen_pitch32(j.dim); a.rows32 = t.rows32; a.bias = j.bias;
+    a.keys = j.keys; a.values = j.values; a.keys2 = j.keys2; a.values2 = j.values2;
+    return a;
+}
+
+static int screen_run_bytes(const ScreenJob& j, const ScreenTable& t, const ScreenWorkspace& w)
+{
+    F16Job f{};
+    f.Q = w.rows8; f.items = t.items8; f.ld = i8_ld(j.dim) / 2; f.batch = j.batch; f.n = j.n;
+    f.norm = t.norm; f.bias = j.bias; f.bias_raise = screen_bias_raise(j.dim);
+    f.scale = w.unit8; f.unit = t.unit8; f.words = w.words; f.ldw = ((uint64_t)j.n + 255) / 256 * 8;
+    if (int rc = i8_best_run(f, j.bias || !j.even)) return rc;
+    ScreenFoldArgs a = fold_args(j, t);
+    a.words = w.words; a.ldw = f.ldw; a.error_items = t.error8; a.error_rows = w.error8; a.near = w.near; a.near_found = w.near_found;
+    I8NearArgs e{};
+    e.batch = j.batch; e.k = j.k; e.n = j.n; e.words = w.words; e.ldw = f.ldw; e.error_rows = w.error8; e.error_most = reinterpret_cast<const float2*>(t.stats + 4);
+    e.row_flag = j.row_flag; e.position = j.position; e.index = j.index; e.fstart = j.fstart; e.fend = j.fend; e.fidx = j.fidx;
+    e.near = w.near; e.near_found = w.near_found;
+    if (j.n <= kBestColumns / 16) hipLaunchKernelGGL((i8_near_kernel<1, 512>), dim3(j.batch), dim3(512), 0, ctx().stream, e);
+    else if (j.n <= kBestColumns / 4) hipLaunchKernelGGL((i8_near_kernel<4, 512>), dim3(j.batch), dim3(512), 0, ctx().stream, e);
+    else hipLaunchKernelGGL((i8_near_kernel<8, 1024>), dim3(j.batch), dim3(1024), 0, ctx().stream, e);
+    DSX_LAUNCH_CHECK("i8_near_kernel");
+    const size_t row_lds = (size_t)(j.dim + 63) / 64 * 256;
+    if (j.before_last) j.before_last(j.before_last_arg);
+    hipLaunchKernelGGL(i8_finish_kernel, dim3(j.batch), dim3(256), row_lds, ctx().stream, a);
+    DSX_LAUNCH_CHECK("i8_finish_kernel");
+    return DSX_OK;
+}
+
 int screen_run(const ScreenJob& j, const ScreenTable& t, const ScreenWorkspace& w)
 {
+    if (w.words) return screen_run_bytes(j, t, w);
     hipStream_t s = ctx().stream;
     const uint32_t ld = screen_ld(j.dim), n = j.n;
     // (a first block that is everything, of a narrow table and many rows, is a search of stored sums too: there is no range to end with)
@@ -997,21 +1656,15 @@ int screen_run(const ScreenJob& j, const ScreenTable& t, const ScreenWorkspace& 
     f.Z = w.sums; f.M = w.most; f.ldz = (n0 + 255) / 256 * 256; f.scale = w.scale;
     int rc = f16_store_run(f);
     if (rc) return rc;
-    ScreenFoldArgs a{};
-    a.batch = j.batch; a.k = j.k; a.n = n;
+    ScreenFoldArgs a = fold_args(j, t);
     a.e1 = w.e1; a.e0 = w.e0;
     a.width_bias = 2.3f * screen_bias_raise(j.dim) / (screen_relative(j.dim) + screen_bias_raise(j.dim));
     a.norm = t.norm; a.seg_norm = t.seg_norm;
     a.largest = j.even ? reinterpret_cast<const float*>(t.stats) : nullptr;
-    a.act = j.act; a.slope = j.slope; a.alpha = j.alpha; a.lambda = j.lambda;
-    a.row_flag = j.row_flag; a.told = j.told;
-    a.position = j.position; a.index = j.index; a.fstart = j.fstart; a.fend = j.fend; a.fidx = j.fidx;
     a.keep = w.keep; a.keep_count = w.keep_count; a.admit = w.admit;
     a.seg = w.seg; a.seg_count = w.seg_count;
     a.cand = j.cand; a.cand_count = j.cand_count; a.cap = j.cap;
     a.Z = (const _Float16*)w.sums; a.M = (const _Float16*)w.most; a.ldz = f.ldz; a.scale = w.scale; a.stored = n0;
-    a.X = j.X; a.ldx = j.ldx; a.dim = j.dim; a.pitch32 = screen_pitch32(j.dim); a.rows32 = t.rows32; a.bias = j.bias;
-    a.keys = j.keys; a.values = j.values; a.keys2 = j.keys2; a.values2 = j.values2;
     a.width_z = 2.1f * f.bias_raise + 1.0e-3f;   // (rounding up to a half: 9.9e-4 of it at most)
     if (stored && j.before_last) j.before_last(j.before_last_arg);
     if ((rc = launch_pick(a, !stored)) || stored) return rc;
@@ -1058,7 +1711,7 @@ extern "C" int dsx_testing_screen_columns(uint32_t batch, uint32_t dim, uint32_t
     DSX_CHECK_ARG(room && stored && ranges, "dsx_testing_screen_columns: null pointer");
     DSX_CHECK_ARG(batch > 0 && dim > 0 && padding < rows_padded && k >= 1, "dsx_testing_screen_columns: batch %u, dim %u, rows_padded %u, padding %u, k = %u", batch,
                   dim, rows_padded, padding, k);
-    const ScreenWorkspace w = screen_layout(nullptr, batch, dim, rows_padded, k);
+    const ScreenWorkspace w = screen_layout(nullptr, batch, dim, rows_padded, k, false);
     const uint32_t n0 = std::min(w.columns, rows_padded - padding);   // as screen_run
     *room = (uint64_t)((char*)w.most - (char*)w.sums) / 2 / batch;
     *stored = (n0 + 255) / 256 * 256;
