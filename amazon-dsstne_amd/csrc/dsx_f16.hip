@@ -78,12 +78,6 @@ template <int WI, int WQ, int STAGES> constexpr uint32_t f16_sweep_lds(int mode)
            (f16_lists(mode) ? WI * WQ * (kF16Queue * 80 + 64 * 4) : 0);
 }
 
-// The integer sums start from this: the bits of 1.5 * 2^23, whose last one is worth 1, so that the sums are floats as they are (and in the order
-// of floats): magnitudes below 2^22 (i8_unit).
-constexpr int32_t kI8Start = 0x4B400000;
-constexpr float kI8StartValue = 12582912.0f;
-constexpr float kI8Most = 3.3e38f;   // above every sum
-
 template <int WI, int WQ, int STAGES, int MODE>
 __global__ __launch_bounds__(64 * WI * WQ) __attribute__((amdgpu_waves_per_eu(WI * WQ == 8 ? 2 : 1, 2))) void f16_sweep_kernel(F16SweepArgs a)
 {
@@ -154,8 +148,7 @@ __global__ __launch_bounds__(64 * WI * WQ) __attribute__((amdgpu_waves_per_eu(WI
             if constexpr (EIGHT) start_next[o] = -3e37f;
             if (i >= BI || t >= t1 || c >= a.n) continue;
             const float b = a.bias ? a.bias[c] : 0.0f, norm = a.norm[c];
-            if constexpr (EIGHT)   // (finite, as its lowest bits are taken; an item or a bias that is no number: never)
-                start_next[o] = (b != b || norm != norm) ? -3e37f : (norm == __builtin_inff()) ? 3e37f : fminf(fmaxf(b + fabsf(b) * a.bias_raise, -3e37f), 3e37f);
+            if constexpr (EIGHT) start_next[o] = i8_start(b, norm, a.bias_raise);
             else
                 start_next[o] = (norm == __builtin_inff() && b == b) ? norm : b == -__builtin_inff() ? b : b + fabsf(b) * a.bias_raise;
             norm_next[o] = (norm == __builtin_inff()) ? 0.0f : norm;
@@ -458,17 +451,7 @@ __global__ __launch_bounds__(64 * WI * WQ) __attribute__((amdgpu_waves_per_eu(WI
                     // (after the exchange the lower half's lanes hold both halves' of block `half`, the others of block half + 2)
                     const auto m = __builtin_amdgcn_permlane32_swap(__float_as_uint(most[0][j]), __float_as_uint(most[1][j]), false, false);
                     const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(second[0][j]), __float_as_uint(second[1][j]), false, false);
-                    const float m0 = __uint_as_float(m[0]), m1 = __uint_as_float(m[1] | 4u);
-                    const float top = fmaxf(m0, m1), next = fmaxf(fmaxf(fminf(m0, m1), __uint_as_float(s[0])), __uint_as_float(s[1]));
-                    const float p = mine[j] * own;
-                    const auto value = [&](float v) __attribute__((always_inline)) -> uint32_t {
-                        const uint32_t bits = __float_as_uint(v);
-                        const float raised = __uint_as_float(v < 0.0f ? bits & ~31u : bits | 31u);   // (of those with these bits but the place's, the largest)
-                        const float x = MODE == kI8Layer ? raised - kI8StartValue * p : (raised - kI8StartValue) * p;
-                        const _Float16 up = (_Float16)fmaxf(fmaf(fabsf(x), 4.932e-4f, x) + 6.0e-8f, -65504.0f);
-                        return __builtin_bit_cast(uint16_t, up);
-                    };
-                    word[half][j] = i8_word(value(top), value(next), __float_as_uint(top) & 31u);
+                    word[half][j] = i8_block_word<MODE == kI8Layer>(m[0], m[1], s[0], s[1], mine[j] * own);
                 }
             }
 #pragma unroll

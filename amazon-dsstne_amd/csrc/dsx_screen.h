@@ -32,10 +32,41 @@ int f16_sweep_run(const F16Job& j, bool layer, uint32_t* lists);
 int f16_store_run(const F16Job& j);
 // Products of bytes (Q and items of ld / 2 pairs of bytes): a word for every 32 items and row.  starts: of the biases and the columns that always pass.
 int i8_best_run(const F16Job& j, bool starts);
+// The same from vectors of 128, 256 or 512 bytes, for more than 256 rows (dsx_i8.hip).  side: for every 32 items what their sums start from, their unit, and
+// three words of nothing; kI8SideSlack bytes more than that are read.
+constexpr uint32_t kI8Side = 36, kI8SideSlack = 1024;
+bool i8_wide_takes(uint32_t ld8, uint32_t batch);
+int i8_wide_run(const F16Job& j, const float* side, bool starts);
+
+// The integer sums start from this: the bits of 1.5 * 2^23, whose last one is worth 1, so that the sums are floats as they are (and in the order
+// of floats): magnitudes below 2^22 (i8_unit).
+constexpr int32_t kI8Start = 0x4B400000;
+constexpr float kI8StartValue = 12582912.0f;
+constexpr float kI8Most = 3.3e38f;   // above every sum
+
+// What an item's sum starts from.  (Finite, as its lowest bits are taken; an item or a bias that is no number: never.)
+__device__ __forceinline__ float i8_start(float bias, float norm, float bias_raise)
+{
+    return (bias != bias || norm != norm) ? -3e37f : (norm == __builtin_inff()) ? 3e37f : fminf(fmaxf(bias + fabsf(bias) * bias_raise, -3e37f), 3e37f);
+}
 
 // A row's word for 32 items: the largest of their sums as a half (upper 16 bits), the second largest as the upper 11 bits of a half, and in between
 // the lowest 5 bits the place of the largest.  Both are upper bounds: i8_first, i8_second.
 __device__ __forceinline__ uint32_t i8_word(uint32_t first, uint32_t second, uint32_t place) { return first << 16 | (second & 0xffe0u) | place; }
+// Of a query's two lanes: the largest sums m0, m1 of 16 items each, their places in the lowest bits, and the second largest; p: the product of the units.
+template <bool STARTS> __device__ __forceinline__ uint32_t i8_block_word(uint32_t m0, uint32_t m1, uint32_t s0, uint32_t s1, float p)
+{
+    const float a = __uint_as_float(m0), b = __uint_as_float(m1 | 4u);
+    const float top = fmaxf(a, b), next = fmaxf(fmaxf(fminf(a, b), __uint_as_float(s0)), __uint_as_float(s1));
+    const auto value = [&](float v) __attribute__((always_inline)) -> uint32_t {
+        const uint32_t bits = __float_as_uint(v);
+        const float raised = __uint_as_float(v < 0.0f ? bits & ~31u : bits | 31u);   // (of those with these bits but the place's, the largest)
+        const float x = STARTS ? raised - kI8StartValue * p : (raised - kI8StartValue) * p;
+        const _Float16 up = (_Float16)fmaxf(fmaf(fabsf(x), 4.932e-4f, x) + 6.0e-8f, -65504.0f);
+        return __builtin_bit_cast(uint16_t, up);
+    };
+    return i8_word(value(top), value(next), __float_as_uint(top) & 31u);
+}
 __device__ __forceinline__ float i8_first(uint32_t word) { return (float)__builtin_bit_cast(_Float16, (uint16_t)(word >> 16)); }
 __device__ __forceinline__ float i8_second(uint32_t word)
 {
@@ -54,6 +85,7 @@ struct ScreenTable {
     void* items8;             // NULL: no bytes
     float* unit8;
     float2* error8;
+    float* side8;             // i8_wide_run's, without biases
     size_t bytes;
 };
 ScreenTable screen_table(void* base, uint32_t dim, uint64_t n, bool kept);
@@ -77,6 +109,7 @@ struct ScreenWorkspace {
     void* rows8;              // screened in bytes (only these are there then, else they are NULL)
     float* unit8;
     float4* error8;
+    float* side8;             // i8_wide_run's, with the call's biases
     uint32_t* words;
     uint2* near;
     uint2* near_found;

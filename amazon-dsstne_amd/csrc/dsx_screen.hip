@@ -244,6 +244,7 @@ struct I8ItemsArgs {
     uint32_t n, dim, pitch32, ld8;
     int8_t* items8;         // [n rounded up to 256][ld8], zero filled
     float* unit;            // [n rounded up to 256 / 32]
+    float* side;            // [n rounded up to 256 / 32][kI8Side]
     float2* error;          // [n rounded up to 256 / 128] largest norm, and largest norm of what the bytes leave out, of 128 columns
     uint32_t* error_most;   // the largest two of these (the bits of non-negative floats)
 };
@@ -299,6 +300,10 @@ __global__ __launch_bounds__(256) void i8_items_kernel(I8ItemsArgs a)
             left_most = fmaxf(left_most, i8_left(left, unit, largest32, a.dim) + unit * (4.0f / 127.0f) + 1e-30f);
         }
         if (threadIdx.x == 0) a.unit[block] = unit;
+        if (threadIdx.x < kI8Side) {
+            const uint32_t c = block * 32 + threadIdx.x;
+            a.side[(uint64_t)block * kI8Side + threadIdx.x] = threadIdx.x == 32 ? unit : (threadIdx.x > 32 || c >= a.n) ? -3e37f : i8_start(0.0f, a.norm[c], 0.0f);
+        }
         __syncthreads();
     }
     if (lane == 0) sLeft[wave] = left_most;
@@ -322,11 +327,24 @@ struct I8RowsArgs {
     uint32_t* told;
     uint32_t* clear;
     uint32_t clear_words;
+    const float* bias;      // with row_blocks: the side of i8_wide_run, made by the workgroups behind the rows' (NULL: not)
+    const float* norm;
+    float bias_raise;
+    uint32_t row_blocks, n;
+    const float* table_side;
+    float* side;
 };
 
 // One wavefront per row, which it reads twice.  Bound by latency.
 __global__ __launch_bounds__(256) void i8_rows_kernel(I8RowsArgs a)
 {
+    if (blockIdx.x >= a.row_blocks) {
+        for (uint64_t i = (uint64_t)(blockIdx.x - a.row_blocks) * 256 + threadIdx.x; i < ((uint64_t)a.n + 255) / 256 * 8 * kI8Side; i += (uint64_t)(gridDim.x - a.row_blocks) * 256) {
+            const uint32_t block = (uint32_t)(i / kI8Side), e = (uint32_t)(i % kI8Side), c = block * 32 + e;
+            a.side[i] = (e >= 32 || c >= a.n) ? a.table_side[i] : i8_start(a.bias[c], a.norm[c], a.bias_raise);
+        }
+        return;
+    }
     const uint32_t row = blockIdx.x * 4 + threadIdx.x / kWave, lane = threadIdx.x % kWave;
     const bool valid = row < a.batch;
     const float* x = a.X + (uint64_t)row * a.ldx;
@@ -1446,7 +1464,8 @@ static bool screen_in_bytes(uint32_t batch, uint32_t dim, uint64_t n, uint32_t k
     return !screen_stored(batch, n, k);
 }
 
-static uint32_t i8_ld(uint32_t dim) { return (dim + 127) / 128 * 128; }
+// (what i8_wide_kernel takes, or a whole number of f16_sweep_kernel's pairs of stages)
+static uint32_t i8_ld(uint32_t dim) { return dim > 256 && dim <= 512 ? 512 : (dim + 127) / 128 * 128; }
 
 ScreenTable screen_table(void* base, uint32_t dim, uint64_t n, bool kept)
 {
@@ -1466,6 +1485,7 @@ ScreenTable screen_table(void* base, uint32_t dim, uint64_t n, bool kept)
     t.items8 = nullptr;
     t.unit8 = nullptr;
     t.error8 = nullptr;
+    t.side8 = nullptr;
     if (kept && n <= kBestColumns) {
         t.items8 = p;
         p += align256(rows * i8_ld(dim));
@@ -1473,6 +1493,8 @@ ScreenTable screen_table(void* base, uint32_t dim, uint64_t n, bool kept)
         p += align256(rows / 32 * sizeof(float));
         t.error8 = (float2*)p;
         p += align256(rows / 128 * sizeof(float2));
+        t.side8 = (float*)p;
+        p += align256(rows / 32 * kI8Side * sizeof(float) + kI8SideSlack);
     }
     t.bytes = (size_t)(p - (char*)base);
     return t;
@@ -1490,6 +1512,8 @@ ScreenWorkspace screen_layout(void* base, uint32_t batch, uint32_t dim, uint64_t
         p += align256((size_t)batch * sizeof(float));
         w.error8 = (float4*)p;
         p += align256((size_t)batch * sizeof(float4));
+        w.side8 = (float*)p;
+        p += align256(knn_f16_rows(n) / 32 * kI8Side * sizeof(float) + kI8SideSlack);
         w.words = (uint32_t*)p;
         p += align256(batch * ((n + 255) / 256 * 8) * sizeof(uint32_t));
         w.near = (uint2*)p;
@@ -1542,7 +1566,7 @@ int screen_build(const ScreenTable& t, const float* W, uint64_t ldw, uint64_t n,
     if (t.items8) {
         I8ItemsArgs e{};
         e.rows32 = t.rows32; e.norm = t.norm; e.n = (uint32_t)n; e.dim = dim; e.pitch32 = i.pitch32; e.ld8 = i8_ld(dim);
-        e.items8 = (int8_t*)t.items8; e.unit = t.unit8; e.error = t.error8; e.error_most = t.stats + 4;
+        e.items8 = (int8_t*)t.items8; e.unit = t.unit8; e.side = t.side8; e.error = t.error8; e.error_most = t.stats + 4;
         hipLaunchKernelGGL(i8_items_kernel, dim3((uint32_t)(knn_f16_rows(n) / 128)), dim3(256), 0, s, e);
         DSX_LAUNCH_CHECK("i8_items_kernel");
     }
@@ -1557,7 +1581,13 @@ int screen_rows(const ScreenJob& j, const ScreenTable& t, const ScreenWorkspace&
         r.rows8 = (int8_t*)w.rows8; r.unit = w.unit8; r.error = w.error8;
         r.stats = j.bias ? nullptr : t.stats;
         r.row_flag = j.row_flag; r.told = j.told; r.clear = j.clear; r.clear_words = j.clear_words;
-        hipLaunchKernelGGL(i8_rows_kernel, dim3((uint32_t)(knn_f16_rows(j.batch) / 4)), dim3(256), 0, ctx().stream, r);
+        r.row_blocks = (uint32_t)(knn_f16_rows(j.batch) / 4);
+        uint32_t more = 0;
+        if (j.bias && i8_wide_takes(r.ld8, j.batch)) {
+            r.bias = j.bias; r.norm = t.norm; r.bias_raise = screen_bias_raise(j.dim); r.n = j.n; r.table_side = t.side8; r.side = w.side8;
+            more = std::min(1024u, (j.n + 1023) / 1024);
+        }
+        hipLaunchKernelGGL(i8_rows_kernel, dim3(r.row_blocks + more), dim3(256), 0, ctx().stream, r);
         DSX_LAUNCH_CHECK("i8_rows_kernel");
         return DSX_OK;
     }
@@ -1624,7 +1654,8 @@ static int screen_run_bytes(const ScreenJob& j, const ScreenTable& t, const Scre
     f.Q = w.rows8; f.items = t.items8; f.ld = i8_ld(j.dim) / 2; f.batch = j.batch; f.n = j.n;
     f.norm = t.norm; f.bias = j.bias; f.bias_raise = screen_bias_raise(j.dim);
     f.scale = w.unit8; f.unit = t.unit8; f.words = w.words; f.ldw = ((uint64_t)j.n + 255) / 256 * 8;
-    if (int rc = i8_best_run(f, j.bias || !j.even)) return rc;
+    const bool starts = j.bias || !j.even;
+    if (int rc = i8_wide_takes(f.ld * 2, j.batch) ? i8_wide_run(f, j.bias ? w.side8 : t.side8, starts) : i8_best_run(f, starts)) return rc;
     ScreenFoldArgs a = fold_args(j, t);
     a.words = w.words; a.ldw = f.ldw; a.error_items = t.error8; a.error_rows = w.error8; a.near = w.near; a.near_found = w.near_found;
     I8NearArgs e{};
