@@ -24,7 +24,7 @@
 // each of which the lists are cut back to what can still be a result.
 // Candidates of earlier ranges are not scored until the last one is through: what is scored in fp32 is about 1.2 k columns a row.
 //
-// Searches with a table that is kept go in bytes where they would go in ranges (screen_in_bytes): the matrix instructions form products of bytes at twice
+// Searches of long tables that are kept go in bytes (screen_in_bytes): the matrix instructions form products of bytes at twice
 // the rate of halves, and read half as much.  x' = u q, w' = v r with whole numbers q, r of 127 at most; u is a row's unit, v one of 32 columns.  With
 // what the bytes leave out, x = x' + x", w = w' + w", the sum of the products of the bytes is exact and
 //   |s' - s| <= |x"| |w| + |x'| |w"| + (0.1 d + 16) 2^-24 |x| |w| + 3 u v      (the last two: screen_score's roundings, and a start's)
@@ -1454,18 +1454,21 @@ static uint32_t screen_first_columns(uint32_t n, uint32_t k)
     return std::min(c, n);
 }
 
-// Whether a search with a kept table goes in bytes: where it would go in ranges of halves, for as many columns as a row's words are looked at by one
-// workgroup (us, halves / bytes, a whole pass with its hidden layer, upload and results: 4,096 x 512 x 1,000,000 top 100 with a filter 4,219 / 3,000, searches of 4,096 x 128 x
-// 1,000,000 top 100 1,924 / 1,417).
-static bool screen_in_bytes(uint32_t batch, uint32_t dim, uint64_t n, uint32_t k)
-{
-    if (ctx().knobs.screen_bytes != 0) return ctx().knobs.screen_bytes == 1 && n <= kBestColumns && n >= 64 * (uint64_t)k;
-    if (ctx().knobs.fc_topk_first_columns || n > kBestColumns || n < 64 * (uint64_t)k) return false;
-    return !screen_stored(batch, n, k);
-}
-
 // (what i8_wide_kernel takes, or a whole number of f16_sweep_kernel's pairs of stages)
 static uint32_t i8_ld(uint32_t dim) { return dim > 256 && dim <= 512 ? 512 : (dim + 127) / 128 * 128; }
+
+// Whether a search with a kept table goes in bytes: many products of a long table, whose bytes are not mostly padding.  539 searches and layers (8,192 to
+// 1,000,000 columns, 16 to 1,024 components, 1 to 4,096 rows, k 1 to 200) measured both ways, of which 2.5 % of the time they could take are left, 7 % with
+// halves alone; three are slower by more than 3 % (us, halves / bytes: 144 x 1,024 x 75,254 top 15 103 / 122).  4,096 x 512 x 1,000,000 top 100 with a filter 4,140 / 2,550,
+// 4,096 x 128 x 1,000,000 top 100 1,780 / 1,330, 256 x 128 x 1,000,000 top 100 304 / 169, 128 x 256 x 500,000 top 50 168 / 121, 2,659 x 480 x 54,259 top 10
+// 323 / 216, but 3,592 x 47 x 475,890 top 2 436 / 627, 4,096 x 128 x 27,278 top 10 159 / 182, 8 x 256 x 500,000 top 50 114 / 115.
+static bool screen_in_bytes(uint32_t batch, uint32_t dim, uint64_t n, uint32_t k)
+{
+    if (n > kBestColumns || n < 64 * (uint64_t)k || ctx().knobs.screen_bytes == 2) return false;
+    if (ctx().knobs.screen_bytes == 1) return true;
+    const uint32_t ld = screen_ld(dim);
+    return !ctx().knobs.fc_topk_first_columns && n >= std::max<uint64_t>(49152, 3000 * (uint64_t)k) && 3 * i8_ld(dim) <= 4 * ld && (double)batch * (double)n * ld >= 6e9;
+}
 
 ScreenTable screen_table(void* base, uint32_t dim, uint64_t n, bool kept)
 {
