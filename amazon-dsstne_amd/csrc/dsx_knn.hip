@@ -383,6 +383,49 @@ static int knn_search_screened(const KnnWorkspace& w, const KnnOperands& op, uin
     return DSX_OK;
 }
 
+// fp16 storage, screened in bytes: the workspace starts with the bytes (screen_table_halves); behind them lies what an unscreened search works in, or what
+// this one does, as they come after each other.  *overflowed as above.
+static int knn_search_halves(const ScreenTable& table, void* rest, const KnnOperands& op, const float* queries, uint32_t M, uint32_t num_queries, uint32_t k,
+                             const KnnResults& out, KnnTimer& t, bool* overflowed)
+{
+    hipStream_t s = ctx().stream;
+    int rc = knn_notes_ready();
+    if (rc) return rc;
+    const ScreenWorkspace w = screen_layout((char*)rest + align256((size_t)num_queries * sizeof(uint32_t)), num_queries, op.dim, op.rows_padded, k, true);
+    ScreenJob j{};
+    j.X = queries; j.ldx = op.dim; j.batch = num_queries; j.dim = op.dim; j.n = M; j.k = k;
+    j.act = DSX_ACT_LINEAR;
+    j.even = true;   // (every item is finite)
+    j.rows16 = op.items16;
+    j.keys = out.scores; j.values = out.indexes; j.keys2 = out.host_scores; j.values2 = out.host_indexes;
+    j.row_flag = (uint32_t*)rest; j.told = &g_knn_notes->flag;
+    t.start(s);
+    if ((rc = screen_rows(j, table, w, nullptr))) return rc;
+    if (t.on) {
+        j.before_last = [](void* p) { static_cast<KnnTimer*>(p)->stop(ctx().stream, static_cast<KnnTimer*>(p)->gemm); };
+        j.before_last_arg = &t;
+    }
+    if ((rc = screen_run(j, table, w))) return rc;
+    t.stop(s, t.topk);
+    DSX_HIP(hipStreamSynchronize(s));
+    *overflowed = *(volatile uint32_t*)&g_knn_notes->flag != 0;
+    return DSX_OK;
+}
+
+// Bytes of a workspace behind the bytes of the table, for this number of queries.
+static size_t knn_halves_rest(uint32_t rows_padded, uint32_t dim, uint32_t num_queries, uint32_t k)
+{
+    const size_t unscreened = knn_layout(nullptr, rows_padded, num_queries, k, true, dim, false).bytes;
+    if (!screen_in_bytes(num_queries, dim, rows_padded, k)) return unscreened;
+    return std::max(unscreened, align256((size_t)num_queries * sizeof(uint32_t)) + screen_layout(nullptr, num_queries, dim, rows_padded, k, true).bytes);
+}
+
+// Whether a table of halves is worth its bytes for some number of queries.
+static bool knn_prepares_halves(uint32_t rows_padded, uint32_t dim, uint32_t num_queries, uint32_t k)
+{
+    return num_queries > 0 && ctx().knobs.screen != 2 && dim >= 16 && dim <= 4096 && k >= 1 && k <= 256 && screen_in_bytes(num_queries, dim, rows_padded, k);
+}
+
 }  // namespace dsx
 
 using namespace dsx;
@@ -458,6 +501,14 @@ size_t dsx_knn_workspace_bytes_prepared(uint32_t rows_padded, uint32_t dim, uint
 size_t dsx_knn_workspace_bytes_f16(uint32_t rows_padded, uint32_t dim, uint32_t num_queries, uint32_t k)
 {
     return knn_workspace_most(rows_padded, num_queries, k, true, dim, false);
+}
+
+size_t dsx_knn_workspace_bytes_f16_prepared(uint32_t rows_padded, uint32_t dim, uint32_t num_queries, uint32_t k)
+{
+    if (!knn_prepares_halves(rows_padded, dim, num_queries, k)) return dsx_knn_workspace_bytes_f16(rows_padded, dim, num_queries, k);
+    size_t most = 0;
+    for (uint64_t q = 1; q <= num_queries; q++) most = std::max(most, knn_halves_rest(rows_padded, dim, (uint32_t)q, k));
+    return screen_table_halves(nullptr, dim, rows_padded).bytes + most;
 }
 
 size_t dsx_knn_workspace_bytes_split(uint32_t rows_padded, uint32_t dim, uint32_t num_queries, uint32_t k)
@@ -590,8 +641,10 @@ static int knn_search_split(const void* item_planes, uint32_t rows_padded, uint3
     return knn_search_common(op, padding, num_queries, k, out, workspace, workspace_bytes, elapsed_ms, true, queries);
 }
 
+// prepared: the workspace starts with the bytes of the table, which are used where that is faster (screening) and else left as they are.
 static int knn_search_f16(const void* items_f16, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,
-                          uint32_t num_queries, uint32_t k, const KnnResults& out, void* workspace, size_t workspace_bytes, float* elapsed_ms)
+                          uint32_t num_queries, uint32_t k, const KnnResults& out, void* workspace, size_t workspace_bytes, float* elapsed_ms,
+                          bool prepared = false, bool screening = false)
 {
     DSX_REQUIRE_INIT();
     DSX_CHECK_ARG(items_f16 && queries && out.scores && out.indexes, "dsx_knn_search_f16: null device pointer");
@@ -606,6 +659,35 @@ static int knn_search_f16(const void* items_f16, uint32_t rows_padded, uint32_t 
     op.rows_padded = rows_padded;
     op.dim = dim;
     op.ld16 = knn_f16_ld(dim);
+    if (prepared) {
+        const ScreenTable table = screen_table_halves(workspace, dim, rows_padded);
+        const size_t rest = knn_halves_rest(rows_padded, dim, num_queries, k);
+        DSX_CHECK_ARG(((uintptr_t)workspace % 256) == 0, "dsx_knn_search: workspace is not 256-byte aligned");
+        DSX_CHECK_ARG(workspace_bytes >= table.bytes + rest, "dsx_knn_search: workspace of %zu bytes, %zu needed", workspace_bytes, table.bytes + rest);
+        workspace = (char*)workspace + table.bytes;
+        workspace_bytes -= table.bytes;
+        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+        hipStreamIsCapturing(ctx().stream, &capturing);
+        if (screening && capturing == hipStreamCaptureStatusNone && !ctx().knobs.knn_block_columns && knn_prepares_halves(rows_padded, dim, num_queries, k)) {
+            KnnTimer t;
+            t.on = elapsed_ms != nullptr;
+            bool redo = true;
+            if (int rc = knn_search_halves(table, workspace, op, queries, rows_padded - padding, num_queries, k, out, t, &redo)) return rc;
+            if (!redo) {
+                g_knn_last_path = DSX_KNN_PATH_CANDIDATES;
+                g_knn_last_repeated = false;
+                if (elapsed_ms) {
+                    t.finish();
+                    elapsed_ms[0] = t.gemm;
+                    elapsed_ms[1] = t.topk;
+                }
+                return DSX_OK;
+            }
+            const int rc = knn_search_common(op, padding, num_queries, k, out, workspace, workspace_bytes, elapsed_ms, true, queries);
+            g_knn_last_repeated = true;
+            return rc;
+        }
+    }
     return knn_search_common(op, padding, num_queries, k, out, workspace, workspace_bytes, elapsed_ms, true, queries);
 }
 
@@ -660,6 +742,25 @@ int dsx_knn_prepare(const float* items, uint32_t rows_padded, uint32_t padding, 
     return DSX_OK;
 }
 
+int dsx_knn_prepare_f16(const void* items_f16, uint32_t rows_padded, uint32_t padding, uint32_t dim, uint32_t num_queries, uint32_t k, void* workspace,
+                        size_t workspace_bytes, int* prepared)
+{
+    DSX_REQUIRE_INIT();
+    DSX_CHECK_ARG(items_f16 && workspace && prepared, "dsx_knn_prepare_f16: null pointer");
+    DSX_CHECK_ARG(((uintptr_t)items_f16 % 16) == 0, "dsx_knn_prepare_f16: the fp16 table is not 16-byte aligned");
+    DSX_CHECK_ARG(padding < rows_padded && k >= 1 && k <= 256, "dsx_knn_prepare_f16: rows_padded %u, padding %u, k = %u", rows_padded, padding, k);
+    DSX_CHECK_ARG(((uintptr_t)workspace % 256) == 0, "dsx_knn_prepare_f16: workspace is not 256-byte aligned");
+    *prepared = 0;
+    if (!knn_prepares_halves(rows_padded, dim, num_queries, k) || workspace_bytes < dsx_knn_workspace_bytes_f16_prepared(rows_padded, dim, num_queries, k)) return DSX_OK;
+    const ScreenTable t = screen_table_halves(workspace, dim, rows_padded);
+    if (int rc = screen_build_halves(t, items_f16, rows_padded - padding, dim)) return rc;
+    uint32_t stats[8];
+    DSX_HIP(hipMemcpyAsync(stats, t.stats, sizeof(stats), hipMemcpyDeviceToHost, ctx().stream));
+    DSX_HIP(hipStreamSynchronize(ctx().stream));
+    if (stats[6] == 0) *prepared = DSX_KNN_FP16_PREPARED;
+    return DSX_OK;
+}
+
 int dsx_knn_search_host(int storage, const void* items, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,
                         uint32_t num_queries, uint32_t k, float* scores, uint32_t* indexes, float* host_scores, uint32_t* host_indexes,
                         void* workspace, size_t workspace_bytes, float* elapsed_ms)
@@ -670,6 +771,8 @@ int dsx_knn_search_host(int storage, const void* items, uint32_t rows_padded, ui
                   "dsx_knn_search_host: the device cannot write to the host memory for %u x %u results", num_queries, k);
     const bool table = storage == DSX_KNN_FP32_PREPARED || storage == DSX_KNN_FP32_PREPARED_EVEN || storage == DSX_KNN_FP32_PREPARED_UNSCREENED;
     DSX_CHECK_ARG(!table || workspace, "dsx_knn_search_host: no prepared workspace");
+    const bool bytes = storage == DSX_KNN_FP16_PREPARED || storage == DSX_KNN_FP16_PREPARED_UNSCREENED;
+    DSX_CHECK_ARG(!bytes || workspace, "dsx_knn_search_host: no prepared workspace");
     const KnnResults out{scores, indexes, host_scores, host_indexes};
     switch (storage) {
     case DSX_KNN_FP32:
@@ -679,6 +782,10 @@ int dsx_knn_search_host(int storage, const void* items, uint32_t rows_padded, ui
         return knn_search_fp32((const float*)items, rows_padded, padding, dim, queries, num_queries, k, out, workspace, workspace_bytes, elapsed_ms,
                                storage != DSX_KNN_FP32_PREPARED_UNSCREENED, table, storage == DSX_KNN_FP32_PREPARED_EVEN);
     case DSX_KNN_FP16: return knn_search_f16(items, rows_padded, padding, dim, queries, num_queries, k, out, workspace, workspace_bytes, elapsed_ms);
+    case DSX_KNN_FP16_PREPARED:
+    case DSX_KNN_FP16_PREPARED_UNSCREENED:
+        return knn_search_f16(items, rows_padded, padding, dim, queries, num_queries, k, out, workspace, workspace_bytes, elapsed_ms, true,
+                              storage == DSX_KNN_FP16_PREPARED);
     case DSX_KNN_SPLIT: return knn_search_split(items, rows_padded, padding, dim, queries, num_queries, k, out, workspace, workspace_bytes, elapsed_ms);
     default: return set_error(DSX_EINVAL, "dsx_knn_search_host: storage %d", storage);
     }

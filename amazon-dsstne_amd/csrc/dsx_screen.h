@@ -90,6 +90,10 @@ struct ScreenTable {
 };
 ScreenTable screen_table(void* base, uint32_t dim, uint64_t n, bool kept);
 int screen_build(const ScreenTable& t, const float* W, uint64_t ldw, uint64_t n, uint32_t dim);
+// The bytes alone, of a table that is kept as halves (items16 [n rounded up to 256][knn_f16_ld(dim)], which searches score from); [6] of stats is set if
+// it holds something that is no finite number, which such a search cannot take.
+ScreenTable screen_table_halves(void* base, uint32_t dim, uint64_t n);
+int screen_build_halves(const ScreenTable& t, const void* items16, uint64_t n, uint32_t dim);
 
 // What a call works in.  columns: how many columns' sums there is room for, all of them or a first block's; screen_run goes by that and not by its
 // own number of columns.
@@ -149,6 +153,7 @@ struct ScreenJob {
     uint32_t clear_words;
     void (*before_last)(void*);   // called before the kernel that ends with the results is launched (NULL: not)
     void* before_last_arg;
+    const void* rows16;       // the table as halves: scores are products of these and of the rows rounded to halves (NULL: of floats); for searches in bytes
     bool even;                // no bias, no column that always passes, and norms close together (screen_even)
 };
 // The rows in f16 (and notes of the table and the rows, NULL: none), then the search itself.
@@ -164,6 +169,7 @@ inline bool screen_even(float largest, float average) { return largest < 60000.0
 inline bool screen_fits(float largest, float average) { return largest <= 65504.0f && largest <= 64.0f * average; }
 
 bool screen_takes(uint32_t batch, uint32_t dim, uint64_t n, bool layer);
+bool screen_in_bytes(uint32_t batch, uint32_t dim, uint64_t n, uint32_t k);
 bool screen_search_pays(uint32_t batch, uint32_t dim, uint64_t n, uint32_t k);
 
 }  // namespace dsx

@@ -240,7 +240,10 @@ __device__ __forceinline__ float i8_left(float left, float unit, float largest, 
 
 struct I8ItemsArgs {
     const float* rows32;    // [n][pitch32]
-    const float* norm;      // [n]
+    const _Float16* rows16; // or [n rounded up to 256][ld16]
+    uint32_t ld16;
+    float* norm;            // [n]; from rows16 it is made here
+    uint32_t* stats;        // from rows16: [0] the largest norm, [6] whether there is one that is no finite number
     uint32_t n, dim, pitch32, ld8;
     int8_t* items8;         // [n rounded up to 256][ld8], zero filled
     float* unit;            // [n rounded up to 256 / 32]
@@ -251,22 +254,49 @@ struct I8ItemsArgs {
 
 // A workgroup takes 128 columns, 32 after each other: their largest component, then their bytes; a wavefront eight columns.  Bound by memory (the second
 // reading comes from L2).
+template <bool HALVES>
 __global__ __launch_bounds__(256) void i8_items_kernel(I8ItemsArgs a)
 {
     __shared__ float sLargest[4], sNorm[4], sLeft[4];
     const uint32_t lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
     float norm_most = 0.0f, left_most = 0.0f;
+    auto four = [&](uint32_t c, uint32_t d) __attribute__((always_inline)) -> float4 {
+        if constexpr (HALVES) {
+            typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+            if (d >= a.ld16) return make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            const half4 h = *reinterpret_cast<const half4*>(a.rows16 + (uint64_t)c * a.ld16 + d);
+            return make_float4((float)h[0], (float)h[1], (float)h[2], (float)h[3]);
+        } else {
+            if (d >= a.pitch32) return make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            return *reinterpret_cast<const float4*>(a.rows32 + (uint64_t)c * a.pitch32 + d);
+        }
+    };
     for (uint32_t block = blockIdx.x * 4; block < blockIdx.x * 4 + 4; block++) {
         const uint32_t c0 = block * 32 + wave * 8;
         float largest = 0.0f, norms = 0.0f;
         for (uint32_t c = c0; c < min(c0 + 8, a.n); c++) {
-            const float norm = a.norm[c];
-            if (!(norm < __builtin_inff())) continue;   // always passes, or never: no bytes
-            norms = fmaxf(norms, norm);
-            for (uint32_t d = 4 * lane; d < a.pitch32; d += 4 * kWave) {
-                const float4 v = *reinterpret_cast<const float4*>(a.rows32 + (uint64_t)c * a.pitch32 + d);
-                largest = fmaxf(fmaxf(largest, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
+            float norm, most = 0.0f, sum = 0.0f;
+            if constexpr (!HALVES) {
+                norm = a.norm[c];
+                if (!(norm < __builtin_inff())) continue;   // always passes, or never: no bytes
             }
+            for (uint32_t d = 4 * lane; d < a.ld8; d += 4 * kWave) {
+                const float4 v = four(c, d);
+                most = fmaxf(fmaxf(most, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
+                if constexpr (HALVES) sum += (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w);
+            }
+            if constexpr (HALVES) {
+#pragma unroll
+                for (int d = 1; d < kWave; d *= 2) sum += __shfl_xor(sum, d);
+                norm = sqrtf(sum);
+                if (lane == 0) {
+                    a.norm[c] = norm;
+                    if (!(norm < __builtin_inff())) a.stats[6] = 1u;
+                }
+                if (!(norm < __builtin_inff())) continue;
+            }
+            norms = fmaxf(norms, norm);
+            largest = fmaxf(largest, most);
         }
 #pragma unroll
         for (int d = 1; d < kWave; d *= 2) largest = fmaxf(largest, __shfl_xor(largest, d));
@@ -280,11 +310,11 @@ __global__ __launch_bounds__(256) void i8_items_kernel(I8ItemsArgs a)
         const float inverse = unit > 1e-35f ? 1.0f / unit : 0.0f;   // (all bytes 0: what they leave out is everything)
         norm_most = fmaxf(norm_most, i8_norm(norm32, largest32, a.dim));
         for (uint32_t c = c0; c < c0 + 8; c++) {
-            const bool some = c < a.n && a.norm[min(c, a.n - 1)] < __builtin_inff();
+            const bool some = c < a.n && a.norm[min(c, a.n - 1)] < __builtin_inff();   // (this wavefront's own, and behind a barrier)
             float left = 0.0f;
             for (uint32_t d = 4 * lane; d < a.ld8; d += 4 * kWave) {
                 float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-                if (some && d < a.pitch32) *reinterpret_cast<float4*>(v) = *reinterpret_cast<const float4*>(a.rows32 + (uint64_t)c * a.pitch32 + d);
+                if (some) *reinterpret_cast<float4*>(v) = four(c, d);
                 uint32_t bytes = 0;
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
@@ -311,6 +341,7 @@ __global__ __launch_bounds__(256) void i8_items_kernel(I8ItemsArgs a)
     if (threadIdx.x == 0) {
         const float left = fmaxf(fmaxf(sLeft[0], sLeft[1]), fmaxf(sLeft[2], sLeft[3]));
         a.error[blockIdx.x] = make_float2(norm_most, left);
+        if (HALVES && __float_as_uint(norm_most) > *(volatile uint32_t*)&a.stats[0]) atomicMax(&a.stats[0], __float_as_uint(norm_most));
         if (__float_as_uint(norm_most) > *(volatile uint32_t*)&a.error_most[0]) atomicMax(&a.error_most[0], __float_as_uint(norm_most));
         if (__float_as_uint(left) > *(volatile uint32_t*)&a.error_most[1]) atomicMax(&a.error_most[1], __float_as_uint(left));
     }
@@ -327,6 +358,7 @@ struct I8RowsArgs {
     uint32_t* told;
     uint32_t* clear;
     uint32_t clear_words;
+    int halves;             // the rows are rounded to halves first
     const float* bias;      // with row_blocks: the side of i8_wide_run, made by the workgroups behind the rows' (NULL: not)
     const float* norm;
     float bias_raise;
@@ -350,7 +382,10 @@ __global__ __launch_bounds__(256) void i8_rows_kernel(I8RowsArgs a)
     const float* x = a.X + (uint64_t)row * a.ldx;
     auto part = [&](uint32_t d, float (&v)[4]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int e = 0; e < 4; e++) v[e] = (valid && d + e < a.dim) ? x[d + e] : 0.0f;
+        for (int e = 0; e < 4; e++) {
+            v[e] = (valid && d + e < a.dim) ? x[d + e] : 0.0f;
+            if (a.halves) v[e] = (float)(_Float16)v[e];
+        }
     };
     constexpr int G = 4;
     float held[G][4];
@@ -453,6 +488,8 @@ struct ScreenFoldArgs {
     uint64_t ldw;
     const float2* error_items;
     const float4* error_rows;
+    const _Float16* rows16;  // scores are products of halves (else NULL)
+    uint32_t ld16;
     const uint2* near;       // i8_near_kernel's
     const uint2* near_found;
     // final
@@ -503,16 +540,17 @@ __device__ __forceinline__ void screen_flag(const ScreenFoldArgs& a, uint32_t b)
 }
 
 // The row itself into LDS, zero filled to whole rounds of the loop below; first: the caller's component threadIdx.x of it.
-template <int T> __device__ __forceinline__ void screen_row(const ScreenFoldArgs& a, uint32_t b, float* sX, float first)
+template <int T, bool HALVES = false> __device__ __forceinline__ void screen_row(const ScreenFoldArgs& a, uint32_t b, float* sX, float first)
 {
-    const uint32_t dpad = (a.dim + 63) / 64 * 64;
-    if (threadIdx.x < dpad) sX[threadIdx.x] = first;
-    for (uint32_t d = T + threadIdx.x; d < dpad; d += T) sX[d] = (d < a.dim) ? a.X[(uint64_t)b * a.ldx + d] : 0.0f;
+    const uint32_t dpad = HALVES ? (a.dim + 127) / 128 * 128 : (a.dim + 63) / 64 * 64;
+    auto as_kept = [](float x) { return HALVES ? (float)(_Float16)x : x; };
+    if (threadIdx.x < dpad) sX[threadIdx.x] = as_kept(first);
+    for (uint32_t d = T + threadIdx.x; d < dpad; d += T) sX[d] = (d < a.dim) ? as_kept(a.X[(uint64_t)b * a.ldx + d]) : 0.0f;
 }
 
 // The row's candidates sList[from .. count) scored in fp32: their words get the scores' keys, and become 0 where a score is no number.  Sixteen lanes per
 // candidate; the order of a sum depends on nothing but its length.  Every lane of the workgroup calls this.
-template <int T, int STEPS = 2> __device__ __forceinline__ void screen_score(const ScreenFoldArgs& a, uint64_t* sList, uint32_t from, uint32_t count, const float* sX)
+template <int T, int STEPS = 2, bool HALVES = false> __device__ __forceinline__ void screen_score(const ScreenFoldArgs& a, uint64_t* sList, uint32_t from, uint32_t count, const float* sX)
 {
     // (four candidates of a group of lanes at a time: their rows are waited for together)
     constexpr int U = 4;
@@ -525,6 +563,21 @@ template <int T, int STEPS = 2> __device__ __forceinline__ void screen_score(con
             col[u] = ~(uint32_t)sList[min(e0 + T / 16 * u, count - 1)];
             sum[u] = 0.0f;
         }
+        if constexpr (HALVES) {
+#pragma unroll STEPS
+            for (uint32_t d = 8 * sub; d < a.ld16; d += 128) {
+                half8 v[U];
+#pragma unroll
+                for (int u = 0; u < U; u++)
+                    if (u == 0 || e0 + T / 16 * u < count) v[u] = *reinterpret_cast<const half8*>(a.rows16 + (uint64_t)col[u] * a.ld16 + d);
+#pragma unroll
+                for (int u = 0; u < U; u++)
+                    if (u == 0 || e0 + T / 16 * u < count) {
+#pragma unroll
+                        for (int e = 0; e < 8; e++) sum[u] = fmaf(sX[d + e], (float)v[u][e], sum[u]);
+                    }
+            }
+        } else
 #pragma unroll STEPS
         for (uint32_t d = 4 * sub; d < a.pitch32; d += 64) {
             const float4 x = *reinterpret_cast<const float4*>(sX + d);
@@ -1205,6 +1258,7 @@ template <int N> __device__ __forceinline__ uint32_t list_kth(const uint64_t* sL
 
 // A row per workgroup; several of them to a compute unit hide each other's latency: candidates' rows, twice, and a search after each.  Nothing fills up:
 // what a round's list has no room for comes with the next one, against a bound that only rises.
+template <bool HALVES>
 __global__ __launch_bounds__(256, 4) void i8_finish_kernel(ScreenFoldArgs a)
 {
     __builtin_amdgcn_s_setprio(3);
@@ -1237,7 +1291,7 @@ __global__ __launch_bounds__(256, 4) void i8_finish_kernel(ScreenFoldArgs a)
     for (uint32_t i = tid; i < bitmap; i += T) sHot[i] = sMore[i] = 0;
     sBest[tid] = 0;
     if (tid == 0) sCount = 0;
-    screen_row<T>(a, b, sX, first);
+    screen_row<T, HALVES>(a, b, sX, first);
     bool any = false;
     for (uint64_t t = fs + tid; t < fe; t += T) any |= a.fidx[t] < a.n;
     const bool listed = __syncthreads_or(any) != 0;
@@ -1303,7 +1357,7 @@ __global__ __launch_bounds__(256, 4) void i8_finish_kernel(ScreenFoldArgs a)
     uint32_t hot[W], more[W];
     for (;;) {
         // Scores of what is new, and what is left of the list: what is no worse than its k-th.
-        screen_score<T, 4>(a, sList, kept, count, sX);
+        screen_score<T, HALVES ? 2 : 4, HALVES>(a, sList, kept, count, sX);
         __syncthreads();
         constexpr int L = kBestWords / T;
         uint64_t word[L];
@@ -1462,7 +1516,7 @@ static uint32_t i8_ld(uint32_t dim) { return dim > 256 && dim <= 512 ? 512 : (di
 // halves alone; three are slower by more than 3 % (us, halves / bytes: 144 x 1,024 x 75,254 top 15 103 / 122).  4,096 x 512 x 1,000,000 top 100 with a filter 4,140 / 2,550,
 // 4,096 x 128 x 1,000,000 top 100 1,780 / 1,330, 256 x 128 x 1,000,000 top 100 304 / 169, 128 x 256 x 500,000 top 50 168 / 121, 2,659 x 480 x 54,259 top 10
 // 323 / 216, but 3,592 x 47 x 475,890 top 2 436 / 627, 4,096 x 128 x 27,278 top 10 159 / 182, 8 x 256 x 500,000 top 50 114 / 115.
-static bool screen_in_bytes(uint32_t batch, uint32_t dim, uint64_t n, uint32_t k)
+bool screen_in_bytes(uint32_t batch, uint32_t dim, uint64_t n, uint32_t k)
 {
     if (n > kBestColumns || n < 64 * (uint64_t)k || ctx().knobs.screen_bytes == 2) return false;
     if (ctx().knobs.screen_bytes == 1) return true;
@@ -1499,6 +1553,27 @@ ScreenTable screen_table(void* base, uint32_t dim, uint64_t n, bool kept)
         t.side8 = (float*)p;
         p += align256(rows / 32 * kI8Side * sizeof(float) + kI8SideSlack);
     }
+    t.bytes = (size_t)(p - (char*)base);
+    return t;
+}
+
+ScreenTable screen_table_halves(void* base, uint32_t dim, uint64_t n)
+{
+    ScreenTable t{};
+    char* p = (char*)base;
+    const uint64_t rows = knn_f16_rows(n);
+    t.norm = (float*)p;
+    p += align256(rows * sizeof(float));
+    t.stats = (uint32_t*)p;
+    p += 256;
+    t.items8 = p;
+    p += align256(rows * i8_ld(dim));
+    t.unit8 = (float*)p;
+    p += align256(rows / 32 * sizeof(float));
+    t.error8 = (float2*)p;
+    p += align256(rows / 128 * sizeof(float2));
+    t.side8 = (float*)p;
+    p += align256(rows / 32 * kI8Side * sizeof(float) + kI8SideSlack);
     t.bytes = (size_t)(p - (char*)base);
     return t;
 }
@@ -1570,9 +1645,21 @@ int screen_build(const ScreenTable& t, const float* W, uint64_t ldw, uint64_t n,
         I8ItemsArgs e{};
         e.rows32 = t.rows32; e.norm = t.norm; e.n = (uint32_t)n; e.dim = dim; e.pitch32 = i.pitch32; e.ld8 = i8_ld(dim);
         e.items8 = (int8_t*)t.items8; e.unit = t.unit8; e.side = t.side8; e.error = t.error8; e.error_most = t.stats + 4;
-        hipLaunchKernelGGL(i8_items_kernel, dim3((uint32_t)(knn_f16_rows(n) / 128)), dim3(256), 0, s, e);
+        hipLaunchKernelGGL((i8_items_kernel<false>), dim3((uint32_t)(knn_f16_rows(n) / 128)), dim3(256), 0, s, e);
         DSX_LAUNCH_CHECK("i8_items_kernel");
     }
+    return DSX_OK;
+}
+
+int screen_build_halves(const ScreenTable& t, const void* items16, uint64_t n, uint32_t dim)
+{
+    hipStream_t s = ctx().stream;
+    hipLaunchKernelGGL(screen_clear_kernel, dim3(1), dim3(64), 0, s, t.stats);
+    I8ItemsArgs e{};
+    e.rows16 = (const _Float16*)items16; e.ld16 = knn_f16_ld(dim); e.norm = t.norm; e.stats = t.stats; e.n = (uint32_t)n; e.dim = dim; e.ld8 = i8_ld(dim);
+    e.items8 = (int8_t*)t.items8; e.unit = t.unit8; e.side = t.side8; e.error = t.error8; e.error_most = t.stats + 4;
+    hipLaunchKernelGGL((i8_items_kernel<true>), dim3((uint32_t)(knn_f16_rows(n) / 128)), dim3(256), 0, s, e);
+    DSX_LAUNCH_CHECK("i8_items_kernel");
     return DSX_OK;
 }
 
@@ -1581,6 +1668,7 @@ int screen_rows(const ScreenJob& j, const ScreenTable& t, const ScreenWorkspace&
     if (w.words) {
         I8RowsArgs r{};
         r.X = j.X; r.ldx = j.ldx; r.batch = j.batch; r.dim = j.dim; r.ld8 = i8_ld(j.dim);
+        r.halves = j.rows16 != nullptr;
         r.rows8 = (int8_t*)w.rows8; r.unit = w.unit8; r.error = w.error8;
         r.stats = j.bias ? nullptr : t.stats;
         r.row_flag = j.row_flag; r.told = j.told; r.clear = j.clear; r.clear_words = j.clear_words;
@@ -1669,9 +1757,13 @@ static int screen_run_bytes(const ScreenJob& j, const ScreenTable& t, const Scre
     else if (j.n <= kBestColumns / 4) hipLaunchKernelGGL((i8_near_kernel<4, 512>), dim3(j.batch), dim3(512), 0, ctx().stream, e);
     else hipLaunchKernelGGL((i8_near_kernel<8, 1024>), dim3(j.batch), dim3(1024), 0, ctx().stream, e);
     DSX_LAUNCH_CHECK("i8_near_kernel");
-    const size_t row_lds = (size_t)(j.dim + 63) / 64 * 256;
+    const size_t row_lds = (size_t)(j.dim + 127) / 128 * 512;
     if (j.before_last) j.before_last(j.before_last_arg);
-    hipLaunchKernelGGL(i8_finish_kernel, dim3(j.batch), dim3(256), row_lds, ctx().stream, a);
+    if (j.rows16) {
+        a.rows16 = (const _Float16*)j.rows16;
+        a.ld16 = knn_f16_ld(j.dim);
+        hipLaunchKernelGGL((i8_finish_kernel<true>), dim3(j.batch), dim3(256), row_lds, ctx().stream, a);
+    } else hipLaunchKernelGGL((i8_finish_kernel<false>), dim3(j.batch), dim3(256), row_lds, ctx().stream, a);
     DSX_LAUNCH_CHECK("i8_finish_kernel");
     return DSX_OK;
 }

@@ -257,16 +257,19 @@ void KnnData::load(int device, DataReader* dataReader)
     pinnedScores = hResultScores[device].data;
     pinnedIndexes = hResultIndexes[device].data;
     unscreened = unscreenedNext = 0;
-    const size_t ws = dataType == DataType::FP16        ? dsx_knn_workspace_bytes_f16(rows, columns, batchSize, maxK)
+    const size_t ws = dataType == DataType::FP16        ? dsx_knn_workspace_bytes_f16_prepared(rows, columns, batchSize, maxK)
                       : dataType == DataType::FP32Split ? dsx_knn_workspace_bytes_split(rows, columns, batchSize, maxK)
                                                         : dsx_knn_workspace_bytes_prepared(rows, columns, batchSize, maxK);
-    // the fp32 search is faster with copies of the table (up to 8 GiB), and needs none: no more than half of what is free goes to them
-    const size_t least = dataType == DataType::FP32 ? dsx_knn_workspace_bytes_least(rows, columns, batchSize, maxK) : ws;
+    // searches are faster with copies of the table (up to 9.5 GiB of an fp32 one, in bytes of an fp16 one), and need none: no more than half of what is
+    // free goes to them
+    const size_t least = dataType == DataType::FP32   ? dsx_knn_workspace_bytes_least(rows, columns, batchSize, maxK)
+                         : dataType == DataType::FP16 ? dsx_knn_workspace_bytes_f16(rows, columns, batchSize, maxK)
+                                                      : ws;
     dsx_device_info info;
     check(dsx_get_device_info(&info), "KnnData::load");
     void* workspace = nullptr;
     size_t wsTaken = ws;
-    int rc = (ws - least > info.hbm_free_bytes / 2) ? DSX_ENOMEM : dsx_malloc(&workspace, ws);
+    int rc = (ws > least && ws - least > info.hbm_free_bytes / 2) ? DSX_ENOMEM : dsx_malloc(&workspace, ws);
     if (rc == DSX_ENOMEM && least < ws) {
         wsTaken = least;
         rc = dsx_malloc(&workspace, least);
@@ -277,6 +280,10 @@ void KnnData::load(int device, DataReader* dataReader)
     if (dataType == DataType::FP32 && wsTaken == ws)
         check(dsx_knn_prepare((const float*)dCollectionPartitions.all[device].data, rows, rows - actualRows, (uint32_t)columns, (uint32_t)batchSize,
                               (uint32_t)maxK, workspace, ws, &prepared),
+              "KnnData::load");
+    else if (dataType == DataType::FP16 && wsTaken == ws)
+        check(dsx_knn_prepare_f16(dCollectionPartitions.all[device].data, rows, rows - actualRows, (uint32_t)columns, (uint32_t)batchSize, (uint32_t)maxK,
+                                  workspace, ws, &prepared),
               "KnnData::load");
     workspacePrepared[device] = prepared;
     check(dsx_get_device_info(&info), "KnnData::load");
@@ -348,11 +355,12 @@ void KnnExactGpu::searchDevice(int k, const float* inputs, int size)
     check(dsx_memcpy_h2d(dIn.data, inputs, (size_t)size * D * sizeof(float)), "KnnExactGpu::search");
     float elapsed[2] = {0, 0};
     const bool kept = data->workspacePrepared[device] != 0 && !data->dCollectionPartitions.handedOut && !data->dWorkspaces.handedOut;
-    const int storage = data->dataType == DataType::FP16        ? DSX_KNN_FP16
-                        : data->dataType == DataType::FP32Split ? DSX_KNN_SPLIT
-                        : kept && data->unscreened != 0         ? DSX_KNN_FP32_PREPARED_UNSCREENED
-                        : kept                                  ? data->workspacePrepared[device]
-                                                                : DSX_KNN_FP32;
+    const bool halves = data->dataType == DataType::FP16;
+    const int storage = data->dataType == DataType::FP32Split ? DSX_KNN_SPLIT
+                        : kept && data->unscreened != 0       ? (halves ? DSX_KNN_FP16_PREPARED_UNSCREENED : DSX_KNN_FP32_PREPARED_UNSCREENED)
+                        : kept                                ? data->workspacePrepared[device]
+                        : halves                              ? DSX_KNN_FP16
+                                                              : DSX_KNN_FP32;
     void *dScores = data->dResultScores[device].data, *dIndexes = data->dResultIndexes[device].data;
     void *hScores = data->hResultScores[device].data, *hIndexes = data->hResultIndexes[device].data;
     const size_t bytes = (size_t)size * maxK * sizeof(float);   // of the scores, and of the indexes

@@ -378,6 +378,8 @@ int dsx_knn_prepare(const float* items, uint32_t rows_padded, uint32_t padding, 
 #define DSX_KNN_FP32_PREPARED 3
 #define DSX_KNN_FP32_PREPARED_EVEN 4   /* the items' norms lie close together */
 #define DSX_KNN_FP32_PREPARED_UNSCREENED 5   /* a prepared workspace, whose copies are left alone: searched without screening */
+#define DSX_KNN_FP16_PREPARED 6              /* dsx_knn_prepare_f16 */
+#define DSX_KNN_FP16_PREPARED_UNSCREENED 7   /* the same, left alone */
 int dsx_knn_search_host(int storage, const void* items, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,
                         uint32_t num_queries, uint32_t k, float* scores, uint32_t* indexes, float* host_scores, uint32_t* host_indexes,
                         void* workspace, size_t workspace_bytes, float* elapsed_ms);
@@ -393,6 +395,12 @@ int dsx_knn_search_f16(const void* items_f16, uint32_t rows_padded, uint32_t pad
                        uint32_t num_queries, uint32_t k, float* scores, uint32_t* indexes, void* workspace, size_t workspace_bytes,
                        float* elapsed_ms);
 size_t dsx_knn_workspace_bytes_f16(uint32_t rows_padded, uint32_t dim, uint32_t num_queries, uint32_t k);
+/* No counterpart in the reference: a copy of the fp16 table in bytes (half its size), by which searches of many queries find what has to be scored; as
+ * dsx_knn_prepare, with dsx_knn_workspace_bytes_f16_prepared bytes and the storage DSX_KNN_FP16_PREPARED (*prepared, or 0).  The scores are the same products
+ * of halves with fp32 sums. */
+size_t dsx_knn_workspace_bytes_f16_prepared(uint32_t rows_padded, uint32_t dim, uint32_t num_queries, uint32_t k);
+int dsx_knn_prepare_f16(const void* items_f16, uint32_t rows_padded, uint32_t padding, uint32_t dim, uint32_t num_queries, uint32_t k, void* workspace,
+                        size_t workspace_bytes, int* prepared);
 
 /* dsx_knn_search with every fp32 product formed from bf16 matrix instructions (see dsx_fc_forward_split: as close to the exact
  * inner products as fp32 multiplication, not bit-identical to it; no counterpart in the reference).  item_planes: the table

@@ -145,3 +145,64 @@ def test_layer_of_floats(pkg, dsx, rng, form, act):
     else:
         assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
     if act == SIGMOID: assert got[2] == 0
+
+
+def search_halves(pkg, dsx, items, q, k, storage=None):
+    """fp16 storage with the table's bytes kept (storage: another one of the same workspace); scores, indexes, whether it was repeated."""
+    n, dim = items.shape
+    rows = (n + 7) // 8 * 8
+    pkg.check(dsx.dsx_testing_set_screen_bytes(1))
+    cm = np.full((dim, rows), 6e4, dtype=np.float32)      # pad rows: never looked at
+    cm[:, :n] = items.T
+    dI, dQ = dev(pkg, cm), dev(pkg, q)
+    table = pkg.DeviceArray((dsx.dsx_knn_f16_table_bytes(rows, dim),), np.uint8)
+    pkg.check(dsx.dsx_knn_f16_convert_items(dI.ptr, rows, rows - n, dim, table.ptr))
+    room = pkg.DeviceArray((dsx.dsx_knn_workspace_bytes_f16_prepared(rows, dim, len(q), k),), np.uint8)
+    prepared = C.c_int(-1)
+    pkg.check(dsx.dsx_knn_prepare_f16(table.ptr, rows, rows - n, dim, len(q), k, room.ptr, room.nbytes, C.byref(prepared)))
+    if prepared.value == 0: return None
+    assert prepared.value == 6
+    scores, idx = pkg.DeviceArray((len(q), k), np.float32), pkg.DeviceArray((len(q), k), np.uint32)
+    pkg.check(dsx.dsx_knn_search_host(storage or prepared.value, table.ptr, rows, rows - n, dim, dQ.ptr, len(q), k, scores.ptr, idx.ptr, None, None, room.ptr,
+                                      room.nbytes, None))
+    return scores.numpy(), idx.numpy(), dsx.dsx_knn_last_search_repeated()
+
+
+@pytest.mark.parametrize("n,dim,queries,k", [(8192, 16, 70, 128), (65601, 768, 520, 100), (400003, 128, 4, 10), (270001, 187, 513, 33), (30001, 300, 300, 256)])
+def test_search_of_whole_halves(pkg, dsx, rng, n, dim, queries, k):
+    print("[case] halves in bytes n=%d dim=%d queries=%d k=%d" % (n, dim, queries, k), flush=True)
+    items = rng.integers(-3, 4, size=(n, dim)).astype(np.float32)
+    q = rng.integers(-3, 4, size=(queries, dim)).astype(np.float32)
+    rs, ri = best(q @ items.T, k)
+    for storage in (6, 7):
+        scores, idx, _ = search_halves(pkg, dsx, items, q, k, storage)
+        assert np.array_equal(scores, rs) and np.array_equal(idx, ri)
+
+
+@pytest.mark.parametrize("form", ["normal", "lognormal", "one long", "constant", "infinite items", "infinite query", "tied"])
+def test_search_of_halves(pkg, dsx, rng, form):
+    n, dim, queries, k = 70001, 130, 300, 50
+    print("[case] halves in bytes, %s" % form, flush=True)
+    items = rng.normal(size=(n, dim)).astype(np.float32)
+    q = rng.normal(size=(queries, dim)).astype(np.float32)
+    if form == "lognormal": items *= rng.lognormal(0, 0.5, size=(n, 1)).astype(np.float32)
+    elif form == "one long": items[12345] *= 40
+    elif form == "constant": items = np.sign(items) * np.float32(0.7)
+    elif form == "infinite items": items[77, 5] = 1e6   # beyond the largest half
+    elif form == "infinite query": q[7, 3] = 1e6
+    elif form == "tied": items[:] = items[0]
+    got = search_halves(pkg, dsx, items, q, k)
+    if form == "infinite items":
+        assert got is None   # searched as before
+        return
+    want = search_halves(pkg, dsx, items, q, k, 7)
+    assert got[2] == (1 if form in ("infinite query", "tied") else 0)
+    if got[2]:   # the same search
+        assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+        return
+    # sums of exact products of halves in two orders: both within dim roundings of the exact sum
+    x, w = q.astype(np.float16).astype(np.float64), items.astype(np.float16).astype(np.float64)
+    bound = dim * 2.0 ** -24 * np.sqrt((x ** 2).sum(axis=1))[:, None] * np.sqrt((w ** 2).sum(axis=1)).max()
+    exact = np.einsum("qd,qkd->qk", x, w[got[1]])
+    assert (np.abs(got[0] - exact) <= bound).all()
+    assert (np.abs(got[0].astype(np.float64) - want[0]) <= 2 * bound).all()
