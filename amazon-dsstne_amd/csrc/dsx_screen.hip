@@ -1111,8 +1111,8 @@ constexpr uint32_t kNearWords = 4096;    // words of a row that are listed
 // reach it, all of the block.  So a row's bound is a score and not an estimate of one: e1 |w| + e2 |w's rest| is open on one side of it only.
 //
 // Two kernels.  i8_near_kernel reads a row's words, once, and lists those that can reach the bound whatever it will be: the k-th word less twice the
-// largest error.  i8_finish_kernel scores.  (In one kernel of sixteen wavefronts a row, 610 us for 4,096 rows of 1,000,000 columns, 100 results:
-// two rows to a compute unit, and all sixteen wavefronts went through the searches and lists of a few hundred words.)
+// largest error.  i8_finish_kernel scores.  (In one kernel of sixteen wavefronts a row, 604 us for 4,096 rows of 1,000,000 columns, 128 components and 100
+// results, 137 + 177 so: two rows to a compute unit, and all sixteen wavefronts went through the searches and lists of a few hundred words.)
 struct I8NearArgs {
     uint32_t batch, k, n;
     const uint32_t* words;
@@ -1134,24 +1134,22 @@ constexpr int32_t kNoWord = INT32_MIN;
 // A word as an integer in the order of its first half, and back.
 __device__ __forceinline__ int32_t i8_sortable(int32_t word) { return word ^ ((word >> 31) & 0x7fff0000); }
 
-// A row per workgroup, 4 V words a lane.  Bound by reading them.
-template <int V, int T>
-__global__ __launch_bounds__(T, T == 1024 ? 8 : 4) void i8_near_kernel(I8NearArgs a)
+// A row per workgroup, 4 V words a lane.  Bound by reading them: their first halves alone stay in registers, two in one, so that three or four rows
+// are on a compute unit; what is listed is read once more.  4,096 rows x 1,000,000 columns: 137 us, 3.7 TB/s (255 with whole words in registers, two rows to a compute
+// unit; 191 with four rows and 88 bytes of scratch a lane).
+template <int V>
+__global__ __launch_bounds__(512, V == 16 ? 6 : 8) void i8_near_kernel(I8NearArgs a)
 {
     __builtin_amdgcn_s_setprio(3);
-    constexpr int B = V * T * 4 / 32, R = V == 1 ? 4 : V == 4 ? 2 : 1;   // words of a bitmap of blocks; keys a lane has in the search
-    __shared__ uint32_t sDead[B], sTop[R * T];
+    constexpr int T = 512, B = V * T * 4 / 32, R = V == 1 ? 2 : 1;   // words of a bitmap of blocks; registers of keys that a lane has in the search
+    typedef int16_t short2v __attribute__((ext_vector_type(2)));
+    __shared__ uint32_t sDead[B], sTop[2 * R * T];
+    __shared__ uint16_t sNear[kNearWords];
     __shared__ uint32_t sNears, sKth;
     const uint32_t b = blockIdx.x, tid = threadIdx.x;
     if (a.row_flag[b] != 0) return;
     const uint32_t blocks = (a.n + 31) / 32;
     const uint32_t* words = a.words + (uint64_t)b * a.ldw;
-    int4 w[V];
-#pragma unroll
-    for (int v = 0; v < V; v++) {
-        const uint32_t at = min((v * T + tid) * 4, (uint32_t)a.ldw - 4);   // (ldw is a multiple of 8)
-        w[v] = *reinterpret_cast<const int4*>(words + at);
-    }
     uint64_t fs = 0, fe = 0;
     if (a.fidx) {
         uint32_t r = a.position + b;
@@ -1162,9 +1160,9 @@ __global__ __launch_bounds__(T, T == 1024 ? 8 : 4) void i8_near_kernel(I8NearArg
     const float4 error = a.error_rows[b];
     const float2 most = *a.error_most;
     if (tid == 0) sNears = 0;
-    const bool some_dead = fe > fs || a.n % 32 != 0;   // the same for the workgroup
+    const bool some_dead = fe > fs || a.n % 256 != 0;   // the same for the workgroup
     if (some_dead) {
-        for (uint32_t i = tid; i < B; i += T) sDead[i] = 0;
+        for (uint32_t i = tid; i < B; i += T) sDead[i] = (i + 1) * 32 <= blocks ? 0u : i * 32 >= blocks ? ~0u : ~0u << (blocks % 32);   // (no blocks)
         __syncthreads();
         for (uint64_t t = fs + tid; t < fe; t += T) {
             const uint32_t c = a.fidx[t];
@@ -1174,39 +1172,73 @@ __global__ __launch_bounds__(T, T == 1024 ? 8 : 4) void i8_near_kernel(I8NearArg
         if (tid == 0 && a.n % 32 != 0 && (words[blocks - 1] & 31u) >= a.n % 32) atomicOr(&sDead[(blocks - 1) >> 5], 1u << ((blocks - 1) & 31u));
         __syncthreads();
     }
-    auto part = [&](int4& x, int c) __attribute__((always_inline)) -> int32_t& { return c == 0 ? x.x : c == 1 ? x.y : c == 2 ? x.z : x.w; };
-    int32_t top[R];
+    // Halves in the order of integers of 16 bits, blocks 4 q and 4 q + 1 in one register, the next two in another; -32768: no words.
+    short2v held[2 * V];
+    constexpr int G = V < 4 ? V : 4;   // reads in flight
 #pragma unroll
-    for (int r = 0; r < R; r++) top[r] = kNoWord;
+    for (int g = 0; g < V; g += G) {
+        uint4 w[G];
 #pragma unroll
-    for (int v = 0; v < V; v++) {
-        const uint32_t q = v * T + tid;
-        const uint32_t dead = (some_dead && q * 4 < blocks) ? sDead[q / 8] >> (q % 8 * 4) : 0u;
-        const bool whole = (uint32_t)(v + 1) * T * 4 <= blocks;
+        for (int v = 0; v < G; v++) {
+            const uint32_t at = ((g + v) * T + tid) * 4;
+            w[v] = make_uint4(~0u, ~0u, ~0u, ~0u);   // (in that order the least half)
+            if (at < a.ldw) w[v] = *reinterpret_cast<const uint4*>(words + at);   // (ldw is a multiple of 8)
+        }
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-            const int32_t x = (whole || q * 4 + c < blocks) ? i8_sortable(part(w[v], c)) : kNoWord;
-            part(w[v], c) = x;
-            top[c % R] = max(top[c % R], ((dead >> c) & 1u) ? kNoWord : x);
+        for (int v = 0; v < G; v++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const short2v x = __builtin_bit_cast(short2v, h ? __builtin_amdgcn_perm(w[v].w, w[v].z, 0x07060302u) : __builtin_amdgcn_perm(w[v].y, w[v].x, 0x07060302u));
+                held[2 * (g + v) + h] = x ^ ((x >> (short2v){15, 15}) & (short2v){0x7fff, 0x7fff});
+            }
+        asm volatile("" ::: "memory");   // (no more reads in flight than that: the halves have the registers)
+    }
+    short2v top[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) top[r] = short2v{INT16_MIN, INT16_MIN};
+    if (!some_dead) {
+#pragma unroll
+        for (int e = 0; e < 2 * V; e++) top[e % R] = __builtin_elementwise_max(top[e % R], held[e]);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 2 * V; e++) {
+            const uint32_t q = e / 2 * T + tid, dead = sDead[q / 8] >> (q % 8 * 4 + e % 2 * 2);
+            short2v x = held[e];
+            if (dead & 1u) x[0] = INT16_MIN;
+            if (dead & 2u) x[1] = INT16_MIN;
+            top[e % R] = __builtin_elementwise_max(top[e % R], x);
         }
     }
     // One wavefront searches.  The k-th of the lanes' largest is a word that k columns reach, and seldom much below the k-th of all.
 #pragma unroll
-    for (int r = 0; r < R; r++) sTop[r * T + tid] = top[r] == kNoWord ? 0u : (uint32_t)top[r] ^ 0x80000000u;
+    for (int r = 0; r < R; r++) {
+        sTop[2 * r * T + tid] = ((uint32_t)(uint16_t)top[r][0] << 16) ^ 0x80000000u;
+        sTop[(2 * r + 1) * T + tid] = ((uint32_t)(uint16_t)top[r][1] << 16) ^ 0x80000000u;
+    }
     __syncthreads();
     if (__builtin_amdgcn_readfirstlane(tid / kWave) == (b >> 8) % (T / kWave)) {
-        constexpr int K = R * T / kWave;
-        uint32_t key[K];
-#pragma unroll
-        for (int i = 0; i < K; i++) key[i] = sTop[i * kWave + tid % kWave];
-        const uint32_t t = screen_wave_kth<K, 16>(key, a.k);
+        // (as screen_wave_kth, but for the keys, which stay in LDS)
+        uint32_t t = 0;
+#pragma unroll 1
+        for (int bit = 30; bit >= 16; bit -= 2) {
+            const uint32_t c1 = t | (1u << bit), c2 = t | (2u << bit), c3 = t | (3u << bit);
+            uint32_t n1 = 0, n2 = 0, n3 = 0;
+#pragma unroll 8
+            for (int i = 0; i < 2 * R * T / kWave; i++) {
+                const uint32_t key = sTop[i * kWave + tid % kWave];
+                n1 += (uint32_t)__popcll(__ballot(key >= c1));
+                n2 += (uint32_t)__popcll(__ballot(key >= c2));
+                n3 += (uint32_t)__popcll(__ballot(key >= c3));
+            }
+            t = (n3 >= a.k) ? c3 : (n2 >= a.k) ? c2 : (n1 >= a.k) ? c1 : t;
+        }
         if (tid % kWave == 0) sKth = t;
     }
     __syncthreads();
     const uint32_t kth = sKth;
     const int32_t t0 = kth != 0 ? (int32_t)(kth ^ 0x80000000u) : kNoWord + 1;
     // What can reach the bound: a score of the k is no further below its word than what a half is rounded up by and the error.
-    int32_t near = kNoWord + 1;
+    int32_t near = kNoWord + 0x10000;
     if (kth != 0) {
         const float step = error.w, z = i8_first((uint32_t)i8_sortable(t0)) * step, wide = fmaf(error.x, most.x, error.y * most.y);
         const float low = (z - fabsf(z) * 2.0e-3f - 2.1f * wide - 2.1f * error.z - 4e-7f * step) / step;
@@ -1215,11 +1247,13 @@ __global__ __launch_bounds__(T, T == 1024 ? 8 : 4) void i8_near_kernel(I8NearArg
             near = i8_sortable((int32_t)(h << 16));
         }
     }
+    auto listed = [&](int e) __attribute__((always_inline)) -> bool {   // the lane's e-th block (in registers)
+        const uint32_t two = __builtin_bit_cast(uint32_t, held[e / 2]);
+        return (int32_t)(e % 2 ? two & 0xffff0000u : two << 16) >= near;
+    };
     uint32_t mine = 0;
 #pragma unroll
-    for (int v = 0; v < V; v++)
-#pragma unroll
-        for (int c = 0; c < 4; c++) mine += part(w[v], c) >= near;
+    for (int e = 0; e < 4 * V; e++) mine += listed(e);
     uint32_t at = mine;
 #pragma unroll
     for (int d = 1; d < kWave; d *= 2) {
@@ -1229,22 +1263,22 @@ __global__ __launch_bounds__(T, T == 1024 ? 8 : 4) void i8_near_kernel(I8NearArg
     uint32_t base = 0;
     if (tid % kWave == kWave - 1) base = atomicAdd(&sNears, at);
     at += __shfl(base, kWave - 1) - mine;
-    uint2* out = a.near + (uint64_t)b * kNearWords;
+    asm volatile("" : "+v"(near));   // (compared again: the results of the comparisons above would not fit the scalar registers)
 #pragma unroll
-    for (int v = 0; v < V; v++) {
-        const uint32_t q = v * T + tid;
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            const int32_t x = part(w[v], c);
-            if (x >= near) {
-                const uint32_t dead = some_dead ? (sDead[q / 8] >> (q % 8 * 4 + c) & 1u) * kNearDead : 0u;
-                if (at < kNearWords) out[at] = make_uint2((q * 4 + c) | dead, (uint32_t)x);
-                at++;
-            }
+    for (int e = 0; e < 4 * V; e++)
+        if (listed(e)) {
+            if (at < kNearWords) sNear[at] = (uint16_t)((e / 4 * T + tid) * 4 + e % 4);
+            at++;
         }
-    }
     __syncthreads();
-    if (tid == 0) a.near_found[b] = make_uint2(sNears, (uint32_t)t0);
+    const uint32_t nears = sNears;
+    uint2* out = a.near + (uint64_t)b * kNearWords;
+    if (nears <= kNearWords)
+        for (uint32_t i = tid; i < nears; i += T) {
+            const uint32_t block = sNear[i], dead = some_dead ? (sDead[block >> 5] >> (block & 31u) & 1u) * kNearDead : 0u;
+            out[i] = make_uint2(block | dead, (uint32_t)i8_sortable((int32_t)words[block]));
+        }
+    if (tid == 0) a.near_found[b] = make_uint2(nears, (uint32_t)t0);
 }
 
 // The k-th largest key of the list's first `count` words (256 * N at most), exact but for the lowest 8 bits; 0: fewer.  The wavefront that calls it.
@@ -1753,9 +1787,9 @@ static int screen_run_bytes(const ScreenJob& j, const ScreenTable& t, const Scre
     e.batch = j.batch; e.k = j.k; e.n = j.n; e.words = w.words; e.ldw = f.ldw; e.error_rows = w.error8; e.error_most = reinterpret_cast<const float2*>(t.stats + 4);
     e.row_flag = j.row_flag; e.position = j.position; e.index = j.index; e.fstart = j.fstart; e.fend = j.fend; e.fidx = j.fidx;
     e.near = w.near; e.near_found = w.near_found;
-    if (j.n <= kBestColumns / 16) hipLaunchKernelGGL((i8_near_kernel<1, 512>), dim3(j.batch), dim3(512), 0, ctx().stream, e);
-    else if (j.n <= kBestColumns / 4) hipLaunchKernelGGL((i8_near_kernel<4, 512>), dim3(j.batch), dim3(512), 0, ctx().stream, e);
-    else hipLaunchKernelGGL((i8_near_kernel<8, 1024>), dim3(j.batch), dim3(1024), 0, ctx().stream, e);
+    if (j.n <= kBestColumns / 16) hipLaunchKernelGGL((i8_near_kernel<1>), dim3(j.batch), dim3(512), 0, ctx().stream, e);
+    else if (j.n <= kBestColumns / 4) hipLaunchKernelGGL((i8_near_kernel<4>), dim3(j.batch), dim3(512), 0, ctx().stream, e);
+    else hipLaunchKernelGGL((i8_near_kernel<16>), dim3(j.batch), dim3(512), 0, ctx().stream, e);
     DSX_LAUNCH_CHECK("i8_near_kernel");
     const size_t row_lds = (size_t)(j.dim + 127) / 128 * 512;
     if (j.before_last) j.before_last(j.before_last_arg);

@@ -93,7 +93,7 @@ def test_search_of_whole_numbers(pkg, dsx, rng, n, dim, queries, k):
     assert np.array_equal(scores, rs) and np.array_equal(idx, ri)
 
 
-@pytest.mark.parametrize("form", ["normal", "lognormal", "one long", "tiny", "constant", "sparse", "clusters", "zero and NaN queries", "NaN items"])
+@pytest.mark.parametrize("form", ["normal", "lognormal", "one long", "tiny", "constant", "sparse", "clusters", "wide cluster", "zero and NaN queries", "NaN items"])
 def test_search_of_floats(pkg, dsx, rng, form):
     n, dim, queries, k = 70001, 130, 300, 50
     print("[case] search in bytes, %s" % form, flush=True)
@@ -105,6 +105,9 @@ def test_search_of_floats(pkg, dsx, rng, form):
     elif form == "constant": items = np.sign(items) * np.float32(0.7)   # every component as large as the largest
     elif form == "sparse": items[rng.random(items.shape) < 0.95] = 0
     elif form == "clusters": items = items[rng.integers(0, 400, n)] + items * np.float32(0.01)   # some 175 near each neighbour
+    elif form == "wide cluster":   # more items within the error of the best than a row's list holds, or are scored in one round
+        items[::11] = 2 * items[0] + items[::11] * np.float32(0.01)
+        q = items[0] / 2 + q * np.float32(0.1)
     elif form == "zero and NaN queries": q[7] = 0; q[9, 3] = np.nan
     elif form == "NaN items": items[77, 5] = np.nan; items[78] = np.nan
     got, want = search(pkg, dsx, items, q, k), search(pkg, dsx, items, q, k, mode=2)
