@@ -93,9 +93,9 @@ def test_search_of_whole_numbers(pkg, dsx, rng, n, dim, queries, k):
     assert np.array_equal(scores, rs) and np.array_equal(idx, ri)
 
 
-@pytest.mark.parametrize("form", ["normal", "lognormal", "one long", "tiny", "constant", "sparse", "clusters", "wide cluster", "zero and NaN queries", "NaN items"])
+@pytest.mark.parametrize("form", ["normal", "lognormal", "one long", "tiny", "constant", "sparse", "clusters", "one in two blocks", "one place", "zero and NaN queries", "NaN items"])
 def test_search_of_floats(pkg, dsx, rng, form):
-    n, dim, queries, k = 70001, 130, 300, 50
+    n, dim, queries, k = 270001 if form == "one in two blocks" else 70001, 130, 300, 50
     print("[case] search in bytes, %s" % form, flush=True)
     items = rng.normal(size=(n, dim)).astype(np.float32)
     q = rng.normal(size=(queries, dim)).astype(np.float32)
@@ -105,8 +105,9 @@ def test_search_of_floats(pkg, dsx, rng, form):
     elif form == "constant": items = np.sign(items) * np.float32(0.7)   # every component as large as the largest
     elif form == "sparse": items[rng.random(items.shape) < 0.95] = 0
     elif form == "clusters": items = items[rng.integers(0, 400, n)] + items * np.float32(0.01)   # some 175 near each neighbour
-    elif form == "wide cluster":   # more items within the error of the best than a row's list holds, or are scored in one round
-        items[::11] = 2 * items[0] + items[::11] * np.float32(0.01)
+    elif form in ("one in two blocks", "one place"):   # as many within the error of the best that lists of words overflow, or several rounds of whole blocks
+        near = slice(0, n, 64) if form == "one in two blocks" else slice(100, 6100)
+        items[near] = 2 * items[0] + items[near] * np.float32(0.01)
         q = items[0] / 2 + q * np.float32(0.1)
     elif form == "zero and NaN queries": q[7] = 0; q[9, 3] = np.nan
     elif form == "NaN items": items[77, 5] = np.nan; items[78] = np.nan
