@@ -1137,17 +1137,16 @@ __device__ __forceinline__ int32_t i8_sortable(int32_t word) { return word ^ ((w
 // A row per workgroup, 4 V words a lane.  Bound by reading them: their first halves alone stay in registers, two in one, so that three or four rows
 // are on a compute unit; what is listed is read once more.  4,096 rows x 1,000,000 columns: 137 us, 3.7 TB/s (255 with whole words in registers, two rows to a compute
 // unit; 191 with four rows and 88 bytes of scratch a lane).
-template <int V>
-__global__ __launch_bounds__(512, V == 16 ? 6 : 8) void i8_near_kernel(I8NearArgs a)
+// V: reads a lane; R: registers of keys that a lane has in the search; ROOM: words that out has room for.  Returns how many there are, and the word that k
+// columns reach; any: whether this lane saw a listed column.
+template <int V, int T, int R, uint32_t ROOM> __device__ __forceinline__ uint2 i8_near(const I8NearArgs& a, uint32_t b, uint2* out, bool& any)
 {
-    __builtin_amdgcn_s_setprio(3);
-    constexpr int T = 512, B = V * T * 4 / 32, R = V == 1 ? 2 : 1;   // words of a bitmap of blocks; registers of keys that a lane has in the search
+    constexpr int B = V * T * 4 / 32;   // words of a bitmap of blocks
     typedef int16_t short2v __attribute__((ext_vector_type(2)));
     __shared__ uint32_t sDead[B], sTop[2 * R * T];
-    __shared__ uint16_t sNear[kNearWords];
+    __shared__ uint16_t sNear[ROOM];
     __shared__ uint32_t sNears, sKth;
-    const uint32_t b = blockIdx.x, tid = threadIdx.x;
-    if (a.row_flag[b] != 0) return;
+    const uint32_t tid = threadIdx.x;
     const uint32_t blocks = (a.n + 31) / 32;
     const uint32_t* words = a.words + (uint64_t)b * a.ldw;
     uint64_t fs = 0, fe = 0;
@@ -1166,6 +1165,7 @@ __global__ __launch_bounds__(512, V == 16 ? 6 : 8) void i8_near_kernel(I8NearArg
         __syncthreads();
         for (uint64_t t = fs + tid; t < fe; t += T) {
             const uint32_t c = a.fidx[t];
+            any |= c < a.n;
             if (c < a.n && (words[c >> 5] & 31u) == (c & 31u)) atomicOr(&sDead[c >> 10], 1u << ((c >> 5) & 31u));
         }
         // (the largest sum of the last block may be one of a column beyond it)
@@ -1267,18 +1267,28 @@ __global__ __launch_bounds__(512, V == 16 ? 6 : 8) void i8_near_kernel(I8NearArg
 #pragma unroll
     for (int e = 0; e < 4 * V; e++)
         if (listed(e)) {
-            if (at < kNearWords) sNear[at] = (uint16_t)((e / 4 * T + tid) * 4 + e % 4);
+            if (at < ROOM) sNear[at] = (uint16_t)((e / 4 * T + tid) * 4 + e % 4);
             at++;
         }
     __syncthreads();
     const uint32_t nears = sNears;
-    uint2* out = a.near + (uint64_t)b * kNearWords;
-    if (nears <= kNearWords)
+    if (nears <= ROOM)
         for (uint32_t i = tid; i < nears; i += T) {
             const uint32_t block = sNear[i], dead = some_dead ? (sDead[block >> 5] >> (block & 31u) & 1u) * kNearDead : 0u;
             out[i] = make_uint2(block | dead, (uint32_t)i8_sortable((int32_t)words[block]));
         }
-    if (tid == 0) a.near_found[b] = make_uint2(nears, (uint32_t)t0);
+    return make_uint2(nears, (uint32_t)t0);
+}
+
+template <int V>
+__global__ __launch_bounds__(512, V == 16 ? 6 : 8) void i8_near_kernel(I8NearArgs a)
+{
+    __builtin_amdgcn_s_setprio(3);
+    const uint32_t b = blockIdx.x;
+    if (a.row_flag[b] != 0) return;
+    bool any = false;
+    const uint2 found = i8_near<V, 512, 1, kNearWords>(a, b, a.near + (uint64_t)b * kNearWords, any);
+    if (threadIdx.x == 0) a.near_found[b] = found;
 }
 
 // The k-th largest key of the list's first `count` words (256 * N at most), exact but for the lowest 8 bits; 0: fewer.  The wavefront that calls it.
@@ -1292,11 +1302,14 @@ template <int N> __device__ __forceinline__ uint32_t list_kth(const uint64_t* sL
 
 // A row per workgroup; several of them to a compute unit hide each other's latency: candidates' rows, twice, and a search after each.  Nothing fills up:
 // what a round's list has no room for comes with the next one, against a bound that only rises.
-template <bool HALVES>
-__global__ __launch_bounds__(256, 4) void i8_finish_kernel(ScreenFoldArgs a)
+// NEAR: not 0 for up to 32,768 columns, whose words this workgroup looks through itself (NEAR registers of keys a lane): both kernels are bound by latency
+// then (4,096 and 1,904 rows x 1,024 x 27,278 top 10 with a filter, two batches: 806 us with two kernels, 727 so).
+template <bool HALVES, int NEAR>
+__global__ __launch_bounds__(256, 4) void i8_finish_kernel(ScreenFoldArgs a, I8NearArgs e)
 {
     __builtin_amdgcn_s_setprio(3);
-    constexpr int T = 256, B = kBestColumns / 32 / 32;
+    constexpr int T = 256, B = NEAR ? T * 4 / 32 : kBestColumns / 32 / 32;
+    __shared__ uint2 sNearWords[NEAR ? T * 4 : 1];
     constexpr uint32_t kOpen = 32;               // blocks of which all columns are looked at, per round
     __shared__ uint64_t sList[kBestWords];
     __shared__ uint64_t sBest[256];
@@ -1310,8 +1323,7 @@ __global__ __launch_bounds__(256, 4) void i8_finish_kernel(ScreenFoldArgs a)
     if (a.row_flag[b] != 0) return;
     const uint32_t blocks = (a.n + 31) / 32, bitmap = (blocks + 31) / 32;
     const uint32_t* words = a.words + (uint64_t)b * a.ldw;
-    const uint2* near = a.near + (uint64_t)b * kNearWords;
-    const uint2 found = a.near_found[b];
+    const uint2* near = NEAR ? sNearWords : a.near + (uint64_t)b * kNearWords;
     uint64_t fs = 0, fe = 0;
     if (a.fidx) {
         uint32_t r = a.position + b;
@@ -1327,7 +1339,12 @@ __global__ __launch_bounds__(256, 4) void i8_finish_kernel(ScreenFoldArgs a)
     if (tid == 0) sCount = 0;
     screen_row<T, HALVES>(a, b, sX, first);
     bool any = false;
-    for (uint64_t t = fs + tid; t < fe; t += T) any |= a.fidx[t] < a.n;
+    uint2 found;
+    if constexpr (NEAR != 0) found = i8_near<1, T, NEAR, T * 4>(e, b, sNearWords, any);
+    else {
+        found = a.near_found[b];
+        for (uint64_t t = fs + tid; t < fe; t += T) any |= a.fidx[t] < a.n;
+    }
     const bool listed = __syncthreads_or(any) != 0;
     if (!(e1 == e1)) {   // a row that is no number has no scores
         screen_results<T>(a, b, sList, 0, sBest, listed);
@@ -1335,7 +1352,7 @@ __global__ __launch_bounds__(256, 4) void i8_finish_kernel(ScreenFoldArgs a)
     }
     const uint32_t nears = found.x;
     const int32_t t0 = (int32_t)found.y;
-    const bool all = nears > kNearWords;   // (more than there was room for: the words are read again; the same for the whole workgroup, as are all of these)
+    const bool all = NEAR ? false : nears > kNearWords;   // (more than there was room for: the words are read again; the same for the whole workgroup, as are all of these)
     if (all) {
         for (uint32_t i = tid; i < bitmap; i += T) sDead[i] = 0;
         __syncthreads();
@@ -1387,7 +1404,7 @@ __global__ __launch_bounds__(256, 4) void i8_finish_kernel(ScreenFoldArgs a)
     }
     float cut = 0.0f;
     bool begun = false;
-    constexpr int W = B / T;
+    constexpr int W = (B + T - 1) / T;
     uint32_t hot[W], more[W];
     for (;;) {
         // Scores of what is new, and what is left of the list: what is no worse than its k-th.
@@ -1545,17 +1562,20 @@ static uint32_t screen_first_columns(uint32_t n, uint32_t k)
 // (what i8_wide_kernel takes, or a whole number of f16_sweep_kernel's pairs of stages)
 static uint32_t i8_ld(uint32_t dim) { return dim > 256 && dim <= 512 ? 512 : (dim + 127) / 128 * 128; }
 
-// Whether a search with a kept table goes in bytes: many products of a long table, whose bytes are not mostly padding.  539 searches and layers (8,192 to
-// 1,000,000 columns, 16 to 1,024 components, 1 to 4,096 rows, k 1 to 200) measured both ways, of which 2.5 % of the time they could take are left, 7 % with
-// halves alone; three are slower by more than 3 % (us, halves / bytes: 144 x 1,024 x 75,254 top 15 103 / 122).  4,096 x 512 x 1,000,000 top 100 with a filter 4,140 / 2,550,
-// 4,096 x 128 x 1,000,000 top 100 1,780 / 1,330, 256 x 128 x 1,000,000 top 100 304 / 169, 128 x 256 x 500,000 top 50 168 / 121, 2,659 x 480 x 54,259 top 10
-// 323 / 216, but 3,592 x 47 x 475,890 top 2 436 / 627, 4,096 x 128 x 27,278 top 10 159 / 182, 8 x 256 x 500,000 top 50 114 / 115.
+// Whether a search with a kept table goes in bytes: many products of a long table, whose bytes are not mostly padding, of which k columns are a small part (else
+// blocks with one candidate hold a second one, and all 32 columns are scored).  Fitted to 1,814 searches and layers (12,000 to 1,000,000 columns, 16 to
+// 1,024 components, 1 to 4,096 rows, k 1 to 200) measured both ways: 3.1 % of the time they could
+// take is left, 6.3 % with halves alone; nine are slower by more than 3 %, by 22 % at most (130 x 393 x 118,322 top 30 92 / 112).  us, halves / bytes, the whole call:
+// 4,096 x 512 x 1,000,000 top 100 with a filter 4,140 / 2,550, 4,096 x 128 x 1,000,000 top 100 1,780 / 1,240, 256 x 128 x 1,000,000 top 100 304 / 169, 128 x 256 x
+// 500,000 top 50 168 / 121, 4,096 x 1,024 x 27,278 top 10 and then 1,904 rows 790 / 727; but 4,096 x 32 x 1,000,000 top 10 738 / 975, 1,024 x 128 x 27,278 top 10 49 / 50,
+// 8 x 256 x 500,000 top 50 114 / 115, 256 x 1,024 x 27,278 top 100 87 / 276.
 bool screen_in_bytes(uint32_t batch, uint32_t dim, uint64_t n, uint32_t k)
 {
     if (n > kBestColumns || n < 64 * (uint64_t)k || ctx().knobs.screen_bytes == 2) return false;
     if (ctx().knobs.screen_bytes == 1) return true;
     const uint32_t ld = screen_ld(dim);
-    return !ctx().knobs.fc_topk_first_columns && n >= std::max<uint64_t>(49152, 3000 * (uint64_t)k) && 3 * i8_ld(dim) <= 4 * ld && (double)batch * (double)n * ld >= 6e9;
+    return !ctx().knobs.fc_topk_first_columns && n >= std::max<uint64_t>(20000, 2500 * (uint64_t)k) && 3 * i8_ld(dim) <= 4 * ld &&
+           (dim <= 512 || batch >= 1024) && (double)batch * (double)n * ld >= (n < 65536 ? 2e10 : 4e9);
 }
 
 ScreenTable screen_table(void* base, uint32_t dim, uint64_t n, bool kept)
@@ -1787,17 +1807,25 @@ static int screen_run_bytes(const ScreenJob& j, const ScreenTable& t, const Scre
     e.batch = j.batch; e.k = j.k; e.n = j.n; e.words = w.words; e.ldw = f.ldw; e.error_rows = w.error8; e.error_most = reinterpret_cast<const float2*>(t.stats + 4);
     e.row_flag = j.row_flag; e.position = j.position; e.index = j.index; e.fstart = j.fstart; e.fend = j.fend; e.fidx = j.fidx;
     e.near = w.near; e.near_found = w.near_found;
-    if (j.n <= kBestColumns / 16) hipLaunchKernelGGL((i8_near_kernel<1>), dim3(j.batch), dim3(512), 0, ctx().stream, e);
-    else if (j.n <= kBestColumns / 4) hipLaunchKernelGGL((i8_near_kernel<4>), dim3(j.batch), dim3(512), 0, ctx().stream, e);
-    else hipLaunchKernelGGL((i8_near_kernel<16>), dim3(j.batch), dim3(512), 0, ctx().stream, e);
-    DSX_LAUNCH_CHECK("i8_near_kernel");
     const size_t row_lds = (size_t)(j.dim + 127) / 128 * 512;
     if (j.before_last) j.before_last(j.before_last_arg);
+    const bool alone = j.n <= 32768;   // (no kernel of its own for the words)
+    if (!alone) {
+        if (j.n <= kBestColumns / 4) hipLaunchKernelGGL((i8_near_kernel<4>), dim3(j.batch), dim3(512), 0, ctx().stream, e);
+        else hipLaunchKernelGGL((i8_near_kernel<16>), dim3(j.batch), dim3(512), 0, ctx().stream, e);
+        DSX_LAUNCH_CHECK("i8_near_kernel");
+    }
+    auto finish = [&](auto halves) {
+        constexpr bool H = decltype(halves)::value;
+        if (!alone) hipLaunchKernelGGL((i8_finish_kernel<H, 0>), dim3(j.batch), dim3(256), row_lds, ctx().stream, a, e);
+        else if (j.k <= 32) hipLaunchKernelGGL((i8_finish_kernel<H, 1>), dim3(j.batch), dim3(256), row_lds, ctx().stream, a, e);
+        else hipLaunchKernelGGL((i8_finish_kernel<H, 2>), dim3(j.batch), dim3(256), row_lds, ctx().stream, a, e);
+    };
     if (j.rows16) {
         a.rows16 = (const _Float16*)j.rows16;
         a.ld16 = knn_f16_ld(j.dim);
-        hipLaunchKernelGGL((i8_finish_kernel<true>), dim3(j.batch), dim3(256), row_lds, ctx().stream, a);
-    } else hipLaunchKernelGGL((i8_finish_kernel<false>), dim3(j.batch), dim3(256), row_lds, ctx().stream, a);
+        finish(std::true_type{});
+    } else finish(std::false_type{});
     DSX_LAUNCH_CHECK("i8_finish_kernel");
     return DSX_OK;
 }
