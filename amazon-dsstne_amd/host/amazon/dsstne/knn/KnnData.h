@@ -82,7 +82,7 @@ struct KnnData {
     std::vector<std::vector<std::string>> hKeys;
     WatchedMatrices dWorkspaces;                 // score blocks + partial lists of the search (instead of a full product matrix)
     std::vector<uint32_t> collectionRowsPadded;  // pad rows per device (rows are padded to a multiple of 8)
-    // FP32: not 0 if the workspace holds copies of the table that load made (dsx_knn_prepare: with which storage); searches use them unless the program
+    // FP32, FP16: not 0 if the workspace holds copies of the table that load made (dsx_knn_prepare, _f16: with which storage); searches use them unless the program
     // has asked for the table or the workspace itself, and as long as this is not set to 0
     std::vector<int> workspacePrepared;
     std::vector<float> elapsedSgemm;             // milliseconds of the last search, per device
