@@ -364,7 +364,10 @@ int dsx_fc_topk_screened_reserve(int lane, uint32_t batch, uint32_t kdim, uint32
     if (int rc = layer_flags_ready()) return rc;
     const uint32_t cap = ctx().knobs.fc_topk_candidate_capacity ? ctx().knobs.fc_topk_candidate_capacity : kLayerCandCap;
     LibScratch& ws = g_layer_ws_of[lane];
-    const size_t bytes = layer_layout(nullptr, batch, layer_first_columns(n, k), k, cap, true, 2, kdim, n).bytes;
+    size_t bytes = layer_layout(nullptr, batch, layer_first_columns(n, k), k, cap, true, 2, kdim, n).bytes;
+    // (a shorter last batch may go in halves where full ones go in bytes, whose scratch is not always the larger)
+    if (screen_in_bytes(batch, kdim, n, k))
+        for (uint32_t b = 1; b < batch; b++) bytes = std::max(bytes, layer_layout(nullptr, b, layer_first_columns(n, k), k, cap, true, 2, kdim, n).bytes);
     if (ws.ptr && bytes > ws.bytes)
         if (int rc = dsx_sync()) return rc;   // (the lane need not be the selected one, which is what growing waits for)
     return lib_scratch_reserve(ws, bytes, "dsx_fc_topk workspace", true);

@@ -325,7 +325,7 @@ int dsx_fc_topk_split(const float* X, uint32_t ldx, const float* W, const void* 
                       uint32_t* values, uint32_t position, const uint32_t* index, const uint64_t* filter_start, const uint64_t* filter_end,
                       const uint32_t* filter_index);
 /* dsx_fc_topk for a caller that keeps the weights' table of the 16-bit screening (two row-major copies of W, 6 bytes per element, and the
- * columns' norms): dsx_screen_table_build fills dsx_screen_table_bytes(n, k_dim) bytes at `table` (device, 256-byte aligned) from W
+ * columns' norms, and a copy in bytes): dsx_screen_table_build fills dsx_screen_table_bytes(n, k_dim) bytes at `table` (device, 256-byte aligned) from W
  * [k_dim][ldw] on the selected lane's stream; it has to be built again when W changes.  k_dim is 4,096 at most.  The call computes no
  * other results than dsx_fc_topk with its own table does; W is read for rows that have to be computed again.
  * dsx_fc_topk_screened_pays: 1 where this is the fastest way to the top-K of an output layer. */
@@ -363,7 +363,7 @@ size_t dsx_knn_workspace_bytes(uint32_t rows_padded, uint32_t dim, uint32_t num_
 /* dsx_knn_workspace_bytes holds, for 512 queries and more, two copies of the table (1.5 x its size, up to 8 GiB) that make the search
  * faster (its candidates are screened in 16 bits); a workspace of at least this size but not that one is searched without them. */
 size_t dsx_knn_workspace_bytes_least(uint32_t rows_padded, uint32_t dim, uint32_t num_queries, uint32_t k);
-/* Fills the two copies once, for a caller that searches one table many times: workspace holds
+/* Fills the copies (and one in bytes, for long tables) once, for a caller that searches one table many times: workspace holds
  * dsx_knn_workspace_bytes_prepared(rows_padded, dim, num_queries, k) bytes (256-byte aligned).  *prepared: 0 (the table is
  * not worth it, or unfit for it) or the storage, DSX_KNN_FP32_PREPARED or _EVEN, with which dsx_knn_search_host takes the workspace, in
  * searches of up to num_queries queries with the same items and k; it has to be prepared again when the items change, and nothing else may use it.  Waits for the device. */
@@ -416,7 +416,7 @@ size_t dsx_knn_workspace_bytes_split(uint32_t rows_padded, uint32_t dim, uint32_
 #define DSX_KNN_PATH_CANDIDATES 1         /* first block as above, then candidate lists */
 #define DSX_KNN_PATH_CANDIDATES_REDONE 2  /* a candidate list filled up: repeated block by block */
 int dsx_knn_last_search_path(void);
-/* 1 if the last search was screened in 16 bits and found rows that cannot be (thousands of ties, norms beyond f16's range), so that it was repeated
+/* 1 if the last search was screened in 16 bits or in bytes and found rows that cannot be (thousands of ties, norms beyond f16's range), so that it was repeated
  * without: a caller with more such queries is better off with DSX_KNN_FP32_PREPARED_UNSCREENED. */
 int dsx_knn_last_search_repeated(void);
 /* dsx_knn_search_f16 scores the column ranges after the first block one workgroup per tile, or, when a range has enough item

@@ -210,3 +210,20 @@ def test_search_of_halves(pkg, dsx, rng, form):
     exact = np.einsum("qd,qkd->qk", x, w[got[1]])
     assert (np.abs(got[0] - exact) <= bound).all()
     assert (np.abs(got[0].astype(np.float64) - want[0]) <= 2 * bound).all()
+
+
+def test_scratch_of_shorter_batches(pkg, dsx, rng):
+    """What is reserved for batches that go in bytes holds shorter ones, which go in halves and need more."""
+    batch, short, kdim, n, k = 4096, 1023, 768, 131072, 50
+    print("[case] scratch of %d rows behind %d" % (short, batch), flush=True)
+    dX, dW = dev(pkg, rng.integers(-3, 4, size=(short, kdim)).astype(np.float32)), dev(pkg, rng.integers(-3, 4, size=(kdim, n)).astype(np.float32))
+    table = pkg.DeviceArray((dsx.dsx_screen_table_bytes(n, kdim),), np.uint8)
+    keys, vals = pkg.DeviceArray((short, k), np.float32), pkg.DeviceArray((short, k), np.uint32)
+    pkg.check(dsx.dsx_screen_table_build(dW.ptr, n, n, kdim, table.ptr))
+    pkg.check(dsx.dsx_fc_topk_screened_reserve(0, batch, kdim, n, k))
+    before, after = C.c_int(), C.c_int()
+    pkg.check(dsx.dsx_get_memory_usage(C.byref(before), None))
+    pkg.check(dsx.dsx_fc_topk_screened(dX.ptr, kdim, dW.ptr, table.ptr, None, short, kdim, n, LINEAR, None, k, keys.ptr, vals.ptr, 0, None, None, None, None))
+    pkg.check(dsx.dsx_get_memory_usage(C.byref(after), None))
+    assert after.value == before.value
+    keys.numpy()
