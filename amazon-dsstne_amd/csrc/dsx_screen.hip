@@ -28,7 +28,11 @@
 // the rate of halves, and read half as much.  x' = u q, w' = v r with whole numbers q, r of 127 at most; u is a row's unit, v one of 32 columns.  With
 // what the bytes leave out, x = x' + x", w = w' + w", the sum of the products of the bytes is exact and
 //   |s' - s| <= |x"| |w| + |x'| |w"| + (0.1 d + 16) 2^-24 |x| |w| + 3 u v      (the last two: screen_score's roundings, and a start's)
-// which is some fifteen times what halves leave open.  So columns are not told apart by estimates of their scores on both sides: the columns of the k largest
+// which is some fifteen times what halves leave open.  A word holds s' as an upper bound, and lies above it by
+//   |word - s'| <= 50 u v + 1e-3 |word|
+// at most: the lowest five bits of the float of 1.5 * 2^23 u v + s' say whose it is, and are taken for the largest they could be (33 units of its last place, a
+// rounding of the start and one of the product counted in: 49.5 u v + 4e-6 |s'|), and it is rounded up to a half.  Where both operands are nearly whole numbers
+// of their units that is more than the error.  So columns are not told apart by estimates of their scores on both sides: the columns of the k largest
 // sums are scored at once, and their k-th score is what the others' upper bounds are held against (i8_finish_kernel): 1.2 to 4 k columns a row are
 // scored.  No ranges, whose bounds and lists would take as long as the products do, and no lists that fill up.
 #include <algorithm>
@@ -56,7 +60,7 @@ __host__ __device__ __forceinline__ float screen_relative(uint32_t dim) { return
 __host__ __device__ __forceinline__ float screen_bias_raise(uint32_t dim) { return ((float)dim + 64.0f) * 6.6e-8f; }
 
 // stats (nearest neighbours): [0] largest norm of a column (the bits of a non-negative float; NaN columns have no part in it: their
-// scores are NaN on every path); [1] sum of the norms of one column in 256, [2] their number; [4], [5] I8ItemsArgs::error_most
+// scores are NaN on every path); [1] sum of the norms of one column in 256, [2] their number; [4], [5], [7] I8ItemsArgs::error_most
 struct ScreenItemsArgs {
     const float* W;       // [dim][ldw]
     uint64_t ldw;
@@ -249,7 +253,7 @@ struct I8ItemsArgs {
     float* unit;            // [n rounded up to 256 / 32]
     float* side;            // [n rounded up to 256 / 32][kI8Side]
     float2* error;          // [n rounded up to 256 / 128] largest norm, and largest norm of what the bytes leave out, of 128 columns
-    uint32_t* error_most;   // the largest two of these (the bits of non-negative floats)
+    uint32_t* error_most;   // the largest two of these, and ([3]) the largest unit (the bits of non-negative floats)
 };
 
 // A workgroup takes 128 columns, 32 after each other: their largest component, then their bytes; a wavefront eight columns.  Bound by memory (the second
@@ -259,7 +263,7 @@ __global__ __launch_bounds__(256) void i8_items_kernel(I8ItemsArgs a)
 {
     __shared__ float sLargest[4], sNorm[4], sLeft[4];
     const uint32_t lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-    float norm_most = 0.0f, left_most = 0.0f;
+    float norm_most = 0.0f, left_most = 0.0f, unit_most = 0.0f;
     auto four = [&](uint32_t c, uint32_t d) __attribute__((always_inline)) -> float4 {
         if constexpr (HALVES) {
             typedef _Float16 half4 __attribute__((ext_vector_type(4)));
@@ -309,6 +313,7 @@ __global__ __launch_bounds__(256) void i8_items_kernel(I8ItemsArgs a)
         const float largest32 = fmaxf(fmaxf(sLargest[0], sLargest[1]), fmaxf(sLargest[2], sLargest[3])), unit = i8_unit(largest32, norm32);
         const float inverse = unit > 1e-35f ? 1.0f / unit : 0.0f;   // (all bytes 0: what they leave out is everything)
         norm_most = fmaxf(norm_most, i8_norm(norm32, largest32, a.dim));
+        unit_most = fmaxf(unit_most, unit);
         for (uint32_t c = c0; c < c0 + 8; c++) {
             const bool some = c < a.n && a.norm[min(c, a.n - 1)] < __builtin_inff();   // (this wavefront's own, and behind a barrier)
             float left = 0.0f;
@@ -344,6 +349,7 @@ __global__ __launch_bounds__(256) void i8_items_kernel(I8ItemsArgs a)
         if (HALVES && __float_as_uint(norm_most) > *(volatile uint32_t*)&a.stats[0]) atomicMax(&a.stats[0], __float_as_uint(norm_most));
         if (__float_as_uint(norm_most) > *(volatile uint32_t*)&a.error_most[0]) atomicMax(&a.error_most[0], __float_as_uint(norm_most));
         if (__float_as_uint(left) > *(volatile uint32_t*)&a.error_most[1]) atomicMax(&a.error_most[1], __float_as_uint(left));
+        if (__float_as_uint(unit_most) > *(volatile uint32_t*)&a.error_most[3]) atomicMax(&a.error_most[3], __float_as_uint(unit_most));
     }
 }
 
@@ -1118,7 +1124,8 @@ struct I8NearArgs {
     const uint32_t* words;
     uint64_t ldw;
     const float4* error_rows;
-    const float2* error_most;
+    const float* unit;       // the rows', by the rows' scale
+    const float4* error_most;   // I8ItemsArgs::error_most
     const uint32_t* row_flag;
     uint32_t position;
     const uint32_t* index;
@@ -1157,7 +1164,7 @@ template <int V, int T, int R, uint32_t ROOM> __device__ __forceinline__ uint2 i
         fe = a.fend[r];
     }
     const float4 error = a.error_rows[b];
-    const float2 most = *a.error_most;
+    const float4 most = *a.error_most;
     if (tid == 0) sNears = 0;
     const bool some_dead = fe > fs || a.n % 256 != 0;   // the same for the workgroup
     if (some_dead) {
@@ -1237,11 +1244,13 @@ template <int V, int T, int R, uint32_t ROOM> __device__ __forceinline__ uint2 i
     __syncthreads();
     const uint32_t kth = sKth;
     const int32_t t0 = kth != 0 ? (int32_t)(kth ^ 0x80000000u) : kNoWord + 1;
-    // What can reach the bound: a score of the k is no further below its word than what a half is rounded up by and the error.
+    // What can reach the bound: a score of the k is no further below its word than what a half is rounded up by, what the place in the sum's lowest bits
+    // raised it by, and the error.
     int32_t near = kNoWord + 0x10000;
     if (kth != 0) {
         const float step = error.w, z = i8_first((uint32_t)i8_sortable(t0)) * step, wide = fmaf(error.x, most.x, error.y * most.y);
-        const float low = (z - fabsf(z) * 2.0e-3f - 2.1f * wide - 2.1f * error.z - 4e-7f * step) / step;
+        const float raised = 50.0f * (a.unit[b] * step) * most.w;
+        const float low = (z - fabsf(z) * 2.0e-3f - raised - 2.1f * wide - 2.1f * error.z - 4e-7f * step) / step;
         if (low > -65000.0f && z < 60000.0f * step) {
             const uint32_t h = __builtin_bit_cast(uint16_t, (_Float16)(low - fabsf(low) * 1.0e-3f - 1.2e-7f));
             near = i8_sortable((int32_t)(h << 16));
@@ -1804,7 +1813,8 @@ static int screen_run_bytes(const ScreenJob& j, const ScreenTable& t, const Scre
     ScreenFoldArgs a = fold_args(j, t);
     a.words = w.words; a.ldw = f.ldw; a.error_items = t.error8; a.error_rows = w.error8; a.near = w.near; a.near_found = w.near_found;
     I8NearArgs e{};
-    e.batch = j.batch; e.k = j.k; e.n = j.n; e.words = w.words; e.ldw = f.ldw; e.error_rows = w.error8; e.error_most = reinterpret_cast<const float2*>(t.stats + 4);
+    e.batch = j.batch; e.k = j.k; e.n = j.n; e.words = w.words; e.ldw = f.ldw; e.error_rows = w.error8; e.unit = w.unit8;
+    e.error_most = reinterpret_cast<const float4*>(t.stats + 4);
     e.row_flag = j.row_flag; e.position = j.position; e.index = j.index; e.fstart = j.fstart; e.fend = j.fend; e.fidx = j.fidx;
     e.near = w.near; e.near_found = w.near_found;
     const size_t row_lds = (size_t)(j.dim + 127) / 128 * 512;
