@@ -523,8 +523,8 @@ __device__ __forceinline__ uint64_t screen_raised(const ScreenFoldArgs& a, uint6
     return ((uint64_t)score_key(norm < __builtin_inff() ? fmaf(e1, norm, x) : __builtin_inff()) << 32) | (uint32_t)word;
 }
 
-// The sum z below which nothing can be a result when k columns have scores of at least this key.
-__device__ __forceinline__ float screen_cut_key(const ScreenFoldArgs& a, uint32_t key, float e0)
+// The sum z below which nothing can be a result when k columns have scores of at least this key.  (Args: what knows the activation)
+template <class Args> __device__ __forceinline__ float screen_cut_key(const Args& a, uint32_t key, float e0)
 {
     const float z = preactivation_bound(key, a.act, a.slope, a.alpha, a.lambda);
     const float cut = z - e0 * 1.001f - fabsf(z) * 2.3841858e-7f;   // (the subtraction itself is rounded)
@@ -532,7 +532,7 @@ __device__ __forceinline__ float screen_cut_key(const ScreenFoldArgs& a, uint32_
 }
 
 // The same when k columns score at least t (as a sum); -inf: anything can.
-__device__ __forceinline__ float screen_cut(const ScreenFoldArgs& a, float t, float e0)
+template <class Args> __device__ __forceinline__ float screen_cut(const Args& a, float t, float e0)
 {
     if (!(t > -__builtin_inff())) return -__builtin_inff();
     return screen_cut_key(a, score_key(activate_rt(t, a.act, a.slope, a.alpha, a.lambda)), e0);
@@ -1117,7 +1117,7 @@ constexpr uint32_t kNearWords = 4096;    // words of a row that are listed
 // reach it, all of the block.  So a row's bound is a score and not an estimate of one: e1 |w| + e2 |w's rest| is open on one side of it only.
 //
 // Two kernels.  i8_near_kernel reads a row's words, once, and lists those that can reach the bound whatever it will be: the k-th word less twice the
-// largest error.  i8_finish_kernel scores.  (In one kernel of sixteen wavefronts a row, 604 us for 4,096 rows of 1,000,000 columns, 128 components and 100
+// largest error, where the activation is not flat.  i8_finish_kernel scores.  (In one kernel of sixteen wavefronts a row, 604 us for 4,096 rows of 1,000,000 columns, 128 components and 100
 // results, 137 + 177 so: two rows to a compute unit, and all sixteen wavefronts went through the searches and lists of a few hundred words.)
 struct I8NearArgs {
     uint32_t batch, k, n;
@@ -1126,6 +1126,8 @@ struct I8NearArgs {
     const float4* error_rows;
     const float* unit;       // the rows', by the rows' scale
     const float4* error_most;   // I8ItemsArgs::error_most
+    uint32_t act;
+    float slope, alpha, lambda;
     const uint32_t* row_flag;
     uint32_t position;
     const uint32_t* index;
@@ -1153,6 +1155,7 @@ template <int V, int T, int R, uint32_t ROOM> __device__ __forceinline__ uint2 i
     __shared__ uint32_t sDead[B], sTop[2 * R * T];
     __shared__ uint16_t sNear[ROOM];
     __shared__ uint32_t sNears, sKth;
+    __shared__ int32_t sNearest;
     const uint32_t tid = threadIdx.x;
     const uint32_t blocks = (a.n + 31) / 32;
     const uint32_t* words = a.words + (uint64_t)b * a.ldw;
@@ -1239,23 +1242,27 @@ template <int V, int T, int R, uint32_t ROOM> __device__ __forceinline__ uint2 i
             }
             t = (n3 >= a.k) ? c3 : (n2 >= a.k) ? c2 : (n1 >= a.k) ? c1 : t;
         }
-        if (tid % kWave == 0) sKth = t;
+        // What can reach the bound, whatever it will be.  The k columns' sums lie no further below their words than what a word is raised by and the
+        // error; their scores, the sums activated, are what another column's score has to reach, and its word lies no further below that than the error.
+        int32_t near = kNoWord + 0x10000;   // (everything)
+        if (t != 0) {
+            const float step = error.w, z = i8_first((uint32_t)i8_sortable((int32_t)(t ^ 0x80000000u))) * step, wide = 1.01f * fmaf(error.x, most.x, error.y * most.y);
+            const float low = z - fabsf(z) * 1.0e-3f - 2e-7f * step - 50.0f * (a.unit[b] * step) * most.w - wide - error.z;
+            const float least = (screen_cut(a, low, error.z) - wide) / step;
+            if (least > -65000.0f && z < 60000.0f * step) {
+                const uint32_t h = __builtin_bit_cast(uint16_t, (_Float16)(least - fabsf(least) * 1.0e-3f - 1.2e-7f));
+                near = i8_sortable((int32_t)(h << 16));
+            }
+        }
+        if (tid % kWave == 0) {
+            sKth = t;
+            sNearest = near;
+        }
     }
     __syncthreads();
     const uint32_t kth = sKth;
     const int32_t t0 = kth != 0 ? (int32_t)(kth ^ 0x80000000u) : kNoWord + 1;
-    // What can reach the bound: a score of the k is no further below its word than what a half is rounded up by, what the place in the sum's lowest bits
-    // raised it by, and the error.
-    int32_t near = kNoWord + 0x10000;
-    if (kth != 0) {
-        const float step = error.w, z = i8_first((uint32_t)i8_sortable(t0)) * step, wide = fmaf(error.x, most.x, error.y * most.y);
-        const float raised = 50.0f * (a.unit[b] * step) * most.w;
-        const float low = (z - fabsf(z) * 2.0e-3f - raised - 2.1f * wide - 2.1f * error.z - 4e-7f * step) / step;
-        if (low > -65000.0f && z < 60000.0f * step) {
-            const uint32_t h = __builtin_bit_cast(uint16_t, (_Float16)(low - fabsf(low) * 1.0e-3f - 1.2e-7f));
-            near = i8_sortable((int32_t)(h << 16));
-        }
-    }
+    int32_t near = sNearest;
     auto listed = [&](int e) __attribute__((always_inline)) -> bool {   // the lane's e-th block (in registers)
         const uint32_t two = __builtin_bit_cast(uint32_t, held[e / 2]);
         return (int32_t)(e % 2 ? two & 0xffff0000u : two << 16) >= near;
@@ -1817,6 +1824,7 @@ static int screen_run_bytes(const ScreenJob& j, const ScreenTable& t, const Scre
     e.error_most = reinterpret_cast<const float4*>(t.stats + 4);
     e.row_flag = j.row_flag; e.position = j.position; e.index = j.index; e.fstart = j.fstart; e.fend = j.fend; e.fidx = j.fidx;
     e.near = w.near; e.near_found = w.near_found;
+    e.act = j.act; e.slope = j.slope; e.alpha = j.alpha; e.lambda = j.lambda;
     const size_t row_lds = (size_t)(j.dim + 127) / 128 * 512;
     if (j.before_last) j.before_last(j.before_last_arg);
     const bool alone = j.n <= 32768;   // (no kernel of its own for the words)

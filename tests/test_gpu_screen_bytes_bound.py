@@ -1,12 +1,15 @@
-"""Searches in bytes: the bound by which words are left out holds where operands are nearly exact in bytes.  Operands whose scores are exact in fp32
-whatever the order of the sums, against a full sort."""
+"""Searches in bytes: the bound by which words are left out holds where operands are nearly exact in bytes, and where activations are flat.
+Operands whose scores are exact in fp32 whatever the order of the sums, against a full sort."""
 
 import numpy as np
 import pytest
 
-from test_gpu_screen_bytes import LINEAR, default_switches, layer, search
+from test_gpu_kept_tables import best
+from test_gpu_screen_bytes import LINEAR, SIGMOID, default_switches, layer, search
 
 pytestmark = pytest.mark.gpu
+
+TANH, RELU = 1, 2
 
 # words looked through by the kernel that scores, by one of their own, and by that with four times as many reads a lane
 WIDTHS = [32768, 131072, 300001]
@@ -35,3 +38,23 @@ def test_words_raised_by_their_places(pkg, dsx, n, starts):
     want = np.sort(np.concatenate([np.arange(b * 32, b * 32 + 32) for b in blocks[28:]]))[:k]
     assert (idx == want).all() and (scores == small / 127).all()
     assert told == 0
+
+
+@pytest.mark.parametrize("n", WIDTHS)
+@pytest.mark.parametrize("act", [SIGMOID, TANH, RELU])
+def test_flat_activations(pkg, dsx, rng, n, act):
+    """Some hundred columns a row of score 1, the sums of which lie far apart; and rows of fewer positive sums than results, the others all 0."""
+    batch, kdim, k = 70, 64, 10
+    print("[case] flat activation %d in bytes n=%d" % (act, n), flush=True)
+    X = rng.permuted(np.tile(np.repeat([-2, 0, 2], [20, 24, 20]), (batch, 1)), axis=1).astype(np.float32)
+    W = 2 * rng.integers(-1, 2, size=(kdim, n)).astype(np.float32)
+    full = X @ W                                            # multiples of 4
+    if act == RELU: level = np.sort(full, axis=1)[:, -6].max()
+    else: level = np.sort(full, axis=1)[:, -200].max() - 18  # 200 columns of a row at 18 and more, none at 15 to 17 or 7 to 9 (where roundings decide)
+    bias = np.full(n, -(level // 4 * 4 + 2), dtype=np.float32)
+    z = full + bias[0]
+    y = np.maximum(z, 0) if act == RELU else np.where(z >= (17 if act == SIGMOID else 9), np.float32(1), np.float32(0))
+    if act != RELU: assert (y.sum(axis=1) >= k).all()
+    keys, vals, _ = layer(pkg, dsx, X, W, bias, act, k)
+    want_keys, want_vals = best(y, k)
+    assert np.array_equal(vals, want_vals) and np.array_equal(keys, want_keys)
