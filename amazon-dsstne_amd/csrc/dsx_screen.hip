@@ -1203,17 +1203,22 @@ template <int V, int T, int R, uint32_t ROOM> __device__ __forceinline__ uint2 i
             }
         asm volatile("" ::: "memory");   // (no more reads in flight than that: the halves have the registers)
     }
+    // (An infinite half says nothing of its column's score - a norm that f16 does not hold, a sum that a half does not - so it counts for no bound: raised
+    // by kUp, the numbers stay in order and infinity becomes the least.)
+    constexpr short kUp = 0x400;
+    typedef uint16_t ushort2v __attribute__((ext_vector_type(2)));
+    auto up = [](short2v x) __attribute__((always_inline)) { return __builtin_bit_cast(short2v, __builtin_bit_cast(ushort2v, x) + (ushort2v){kUp, kUp}); };
     short2v top[R];
 #pragma unroll
     for (int r = 0; r < R; r++) top[r] = short2v{INT16_MIN, INT16_MIN};
     if (!some_dead) {
 #pragma unroll
-        for (int e = 0; e < 2 * V; e++) top[e % R] = __builtin_elementwise_max(top[e % R], held[e]);
+        for (int e = 0; e < 2 * V; e++) top[e % R] = __builtin_elementwise_max(top[e % R], up(held[e]));
     } else {
 #pragma unroll
         for (int e = 0; e < 2 * V; e++) {
             const uint32_t q = e / 2 * T + tid, dead = sDead[q / 8] >> (q % 8 * 4 + e % 2 * 2);
-            short2v x = held[e];
+            short2v x = up(held[e]);
             if (dead & 1u) x[0] = INT16_MIN;
             if (dead & 2u) x[1] = INT16_MIN;
             top[e % R] = __builtin_elementwise_max(top[e % R], x);
@@ -1221,10 +1226,12 @@ template <int V, int T, int R, uint32_t ROOM> __device__ __forceinline__ uint2 i
     }
     // One wavefront searches.  The k-th of the lanes' largest is a word that k columns reach, and seldom much below the k-th of all.
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-        sTop[2 * r * T + tid] = ((uint32_t)(uint16_t)top[r][0] << 16) ^ 0x80000000u;
-        sTop[(2 * r + 1) * T + tid] = ((uint32_t)(uint16_t)top[r][1] << 16) ^ 0x80000000u;
-    }
+    for (int r = 0; r < R; r++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int x = top[r][h];
+            sTop[(2 * r + h) * T + tid] = x > INT16_MIN + kUp ? ((uint32_t)(x - kUp) << 16) ^ 0x80000000u : 0u;
+        }
     __syncthreads();
     if (__builtin_amdgcn_readfirstlane(tid / kWave) == (b >> 8) % (T / kWave)) {
         // (as screen_wave_kth, but for the keys, which stay in LDS)

@@ -1,5 +1,5 @@
-"""Searches in bytes: the bound by which words are left out holds where operands are nearly exact in bytes, and where activations are flat.
-Operands whose scores are exact in fp32 whatever the order of the sums, against a full sort."""
+"""Searches in bytes: the bound by which words are left out holds where operands are nearly exact in bytes, where activations are flat, and where
+the columns of the largest words have the smallest scores.  Operands whose scores are exact in fp32 whatever the order of the sums, against a full sort."""
 
 import numpy as np
 import pytest
@@ -58,3 +58,20 @@ def test_flat_activations(pkg, dsx, rng, n, act):
     keys, vals, _ = layer(pkg, dsx, X, W, bias, act, k)
     want_keys, want_vals = best(y, k)
     assert np.array_equal(vals, want_vals) and np.array_equal(keys, want_keys)
+
+
+@pytest.mark.parametrize("n", WIDTHS)
+@pytest.mark.parametrize("passing", [1, 25, 40])
+def test_columns_that_always_pass(pkg, dsx, rng, n, passing):
+    """Columns whose norms f16 does not hold, so that nothing is known of their scores, which are the lowest there are."""
+    batch, kdim, k = 70, 64, 30
+    print("[case] always passing columns in bytes n=%d passing=%d" % (n, passing), flush=True)
+    X = rng.integers(0, 4, size=(batch, kdim)).astype(np.float32)
+    X[:, 0] = 1
+    W = rng.integers(-3, 4, size=(kdim, n)).astype(np.float32)
+    bias = rng.integers(-40, 41, size=n).astype(np.float32)
+    W[:, rng.permutation(n)[:passing]] = -10000.0
+    keys, vals, told = layer(pkg, dsx, X, W, bias, LINEAR, k)
+    want_keys, want_vals = best(X @ W + bias, k)
+    assert np.array_equal(vals, want_vals) and np.array_equal(keys, want_keys)
+    assert told == 0
