@@ -729,7 +729,7 @@ int dsx_knn_prepare(const float* items, uint32_t rows_padded, uint32_t padding, 
     const uint32_t M = rows_padded - padding;
     const ScreenTable t = screen_table(workspace, dim, rows_padded, true);
     if (int rc = screen_build(t, items, rows_padded, M, dim)) return rc;
-    uint32_t stats[3];
+    uint32_t stats[8];
     DSX_HIP(hipMemcpyAsync(stats, t.stats, sizeof(stats), hipMemcpyDeviceToHost, ctx().stream));
     DSX_HIP(hipStreamSynchronize(ctx().stream));
     ScreenNotes notes{};
@@ -738,7 +738,9 @@ int dsx_knn_prepare(const float* items, uint32_t rows_padded, uint32_t padding, 
     notes.number = stats[2];
     // as where a search makes its own copies
     const float average = notes.number != 0 ? notes.sum / (float)notes.number : 0.0f;
-    if (screen_fits(notes.largest, average)) *prepared = screen_even(notes.largest, average) ? DSX_KNN_FP32_PREPARED_EVEN : DSX_KNN_FP32_PREPARED;
+    // (in bytes an item that is no number adds up to 0, unless sums start from something)
+    const bool even = screen_even(notes.largest, average) && !(t.items8 && stats[6] != 0);
+    if (screen_fits(notes.largest, average)) *prepared = even ? DSX_KNN_FP32_PREPARED_EVEN : DSX_KNN_FP32_PREPARED;
     return DSX_OK;
 }
 

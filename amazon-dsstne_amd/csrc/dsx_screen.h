@@ -154,7 +154,7 @@ struct ScreenJob {
     void (*before_last)(void*);   // called before the kernel that ends with the results is launched (NULL: not)
     void* before_last_arg;
     const void* rows16;       // the table as halves: scores are products of these and of the rows rounded to halves (NULL: of floats); for searches in bytes
-    bool even;                // no bias, no column that always passes, and norms close together (screen_even)
+    bool even;                // no bias, no column that always passes or (where the table has bytes) is no number, and norms close together (screen_even)
 };
 // The rows in f16 (and notes of the table and the rows, NULL: none), then the search itself.
 int screen_rows(const ScreenJob& j, const ScreenTable& t, const ScreenWorkspace& w, ScreenNotes* notes);

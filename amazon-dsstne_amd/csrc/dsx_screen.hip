@@ -60,7 +60,7 @@ __host__ __device__ __forceinline__ float screen_relative(uint32_t dim) { return
 __host__ __device__ __forceinline__ float screen_bias_raise(uint32_t dim) { return ((float)dim + 64.0f) * 6.6e-8f; }
 
 // stats (nearest neighbours): [0] largest norm of a column (the bits of a non-negative float; NaN columns have no part in it: their
-// scores are NaN on every path); [1] sum of the norms of one column in 256, [2] their number; [4], [5], [7] I8ItemsArgs::error_most
+// scores are NaN on every path); [1] sum of the norms of one column in 256, [2] their number; [4], [5], [7] I8ItemsArgs::error_most; [6] I8ItemsArgs::stats
 struct ScreenItemsArgs {
     const float* W;       // [dim][ldw]
     uint64_t ldw;
@@ -247,7 +247,7 @@ struct I8ItemsArgs {
     const _Float16* rows16; // or [n rounded up to 256][ld16]
     uint32_t ld16;
     float* norm;            // [n]; from rows16 it is made here
-    uint32_t* stats;        // from rows16: [0] the largest norm, [6] whether there is one that is no finite number
+    uint32_t* stats;        // [6] whether a norm is no number (from rows16: no finite one); from rows16 [0], the largest, as well
     uint32_t n, dim, pitch32, ld8;
     int8_t* items8;         // [n rounded up to 256][ld8], zero filled
     float* unit;            // [n rounded up to 256 / 32]
@@ -282,6 +282,7 @@ __global__ __launch_bounds__(256) void i8_items_kernel(I8ItemsArgs a)
             float norm, most = 0.0f, sum = 0.0f;
             if constexpr (!HALVES) {
                 norm = a.norm[c];
+                if (norm != norm && lane == 0) a.stats[6] = 1u;
                 if (!(norm < __builtin_inff())) continue;   // always passes, or never: no bytes
             }
             for (uint32_t d = 4 * lane; d < a.ld8; d += 4 * kWave) {
@@ -532,7 +533,7 @@ template <class Args> __device__ __forceinline__ float screen_cut_key(const Args
 }
 
 // The same when k columns score at least t (as a sum); -inf: anything can.
-template <class Args> __device__ __forceinline__ float screen_cut(const Args& a, float t, float e0)
+__device__ __forceinline__ float screen_cut(const ScreenFoldArgs& a, float t, float e0)
 {
     if (!(t > -__builtin_inff())) return -__builtin_inff();
     return screen_cut_key(a, score_key(activate_rt(t, a.act, a.slope, a.alpha, a.lambda)), e0);
@@ -1135,7 +1136,7 @@ struct I8NearArgs {
     const uint64_t* fend;
     const uint32_t* fidx;
     uint2* near;             // [batch][kNearWords] block (kNearDead: its largest sum is a listed column's) and word, as an integer in the order of halves
-    uint2* near_found;       // [batch] how many there are, and the word that k columns reach
+    uint2* near_found;       // [batch] how many there are; the word that k columns reach and the least that is listed (upper halves)
 };
 constexpr uint32_t kNearDead = 0x80000000u;
 constexpr int32_t kNoWord = INT32_MIN;
@@ -1146,8 +1147,8 @@ __device__ __forceinline__ int32_t i8_sortable(int32_t word) { return word ^ ((w
 // A row per workgroup, 4 V words a lane.  Bound by reading them: their first halves alone stay in registers, two in one, so that three or four rows
 // are on a compute unit; what is listed is read once more.  4,096 rows x 1,000,000 columns: 137 us, 3.7 TB/s (255 with whole words in registers, two rows to a compute
 // unit; 191 with four rows and 88 bytes of scratch a lane).
-// V: reads a lane; R: registers of keys that a lane has in the search; ROOM: words that out has room for.  Returns how many there are, and the word that k
-// columns reach; any: whether this lane saw a listed column.
+// V: reads a lane; R: registers of keys that a lane has in the search; ROOM: words that out has room for.  Returns near_found's two; any: whether this lane saw
+// a listed column.
 template <int V, int T, int R, uint32_t ROOM> __device__ __forceinline__ uint2 i8_near(const I8NearArgs& a, uint32_t b, uint2* out, bool& any)
 {
     constexpr int B = V * T * 4 / 32;   // words of a bitmap of blocks
@@ -1255,7 +1256,9 @@ template <int V, int T, int R, uint32_t ROOM> __device__ __forceinline__ uint2 i
         if (t != 0) {
             const float step = error.w, z = i8_first((uint32_t)i8_sortable((int32_t)(t ^ 0x80000000u))) * step, wide = 1.01f * fmaf(error.x, most.x, error.y * most.y);
             const float low = z - fabsf(z) * 1.0e-3f - 2e-7f * step - 50.0f * (a.unit[b] * step) * most.w - wide - error.z;
-            const float least = (screen_cut(a, low, error.z) - wide) / step;
+            // (i8_finish_kernel knows its k-th key but for the lowest 8 bits)
+            const float cut = low > -__builtin_inff() ? screen_cut_key(a, score_key(activate_rt(low, a.act, a.slope, a.alpha, a.lambda)) & ~255u, error.z) : low;
+            const float least = (cut - wide) / step;
             if (least > -65000.0f && z < 60000.0f * step) {
                 const uint32_t h = __builtin_bit_cast(uint16_t, (_Float16)(least - fabsf(least) * 1.0e-3f - 1.2e-7f));
                 near = i8_sortable((int32_t)(h << 16));
@@ -1300,7 +1303,7 @@ template <int V, int T, int R, uint32_t ROOM> __device__ __forceinline__ uint2 i
             const uint32_t block = sNear[i], dead = some_dead ? (sDead[block >> 5] >> (block & 31u) & 1u) * kNearDead : 0u;
             out[i] = make_uint2(block | dead, (uint32_t)i8_sortable((int32_t)words[block]));
         }
-    return make_uint2(nears, (uint32_t)t0);
+    return make_uint2(nears, ((uint32_t)t0 & 0xffff0000u) | (uint32_t)sNearest >> 16);
 }
 
 template <int V>
@@ -1374,7 +1377,7 @@ __global__ __launch_bounds__(256, 4) void i8_finish_kernel(ScreenFoldArgs a, I8N
         return;
     }
     const uint32_t nears = found.x;
-    const int32_t t0 = (int32_t)found.y;
+    const int32_t t0 = (int32_t)(found.y & 0xffff0000u), least = (int32_t)(found.y << 16);
     const bool all = NEAR ? false : nears > kNearWords;   // (more than there was room for: the words are read again; the same for the whole workgroup, as are all of these)
     if (all) {
         for (uint32_t i = tid; i < bitmap; i += T) sDead[i] = 0;
@@ -1460,6 +1463,13 @@ __global__ __launch_bounds__(256, 4) void i8_finish_kernel(ScreenFoldArgs a, I8N
         kept = sCount;
         if (!begun) {
             begun = true;
+            // What is listed was decided by words; now that there are scores it is known whether it was enough.  (A column of the k without a score,
+            // a sum that was raised by more than it should have been.)
+            const float4 most = *e.error_most;
+            if (!all && least > kNoWord + 0x10000 && fmaf(i8_first((uint32_t)i8_sortable(least)), step, fmaf(e1, most.x, e2 * most.y) * 1.000001f) >= cut) {
+                if (tid == 0) screen_flag(a, b);
+                return;
+            }
             each(std::true_type{}, [&](uint32_t block, int32_t x, bool dead, float2 e) {
                 const float wide = fmaf(e1, e.x, e2 * e.y) * 1.000001f;
                 const uint32_t word = (uint32_t)i8_sortable(x);
@@ -1720,7 +1730,7 @@ int screen_build(const ScreenTable& t, const float* W, uint64_t ldw, uint64_t n,
     DSX_LAUNCH_CHECK("screen_items_kernel");
     if (t.items8) {
         I8ItemsArgs e{};
-        e.rows32 = t.rows32; e.norm = t.norm; e.n = (uint32_t)n; e.dim = dim; e.pitch32 = i.pitch32; e.ld8 = i8_ld(dim);
+        e.rows32 = t.rows32; e.norm = t.norm; e.stats = t.stats; e.n = (uint32_t)n; e.dim = dim; e.pitch32 = i.pitch32; e.ld8 = i8_ld(dim);
         e.items8 = (int8_t*)t.items8; e.unit = t.unit8; e.side = t.side8; e.error = t.error8; e.error_most = t.stats + 4;
         hipLaunchKernelGGL((i8_items_kernel<false>), dim3((uint32_t)(knn_f16_rows(n) / 128)), dim3(256), 0, s, e);
         DSX_LAUNCH_CHECK("i8_items_kernel");

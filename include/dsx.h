@@ -376,7 +376,7 @@ int dsx_knn_prepare(const float* items, uint32_t rows_padded, uint32_t padding, 
 #define DSX_KNN_FP16 1
 #define DSX_KNN_SPLIT 2
 #define DSX_KNN_FP32_PREPARED 3
-#define DSX_KNN_FP32_PREPARED_EVEN 4   /* the items' norms lie close together */
+#define DSX_KNN_FP32_PREPARED_EVEN 4   /* the items' norms lie close together (and are numbers, where there are bytes) */
 #define DSX_KNN_FP32_PREPARED_UNSCREENED 5   /* a prepared workspace, whose copies are left alone: searched without screening */
 #define DSX_KNN_FP16_PREPARED 6              /* dsx_knn_prepare_f16 */
 #define DSX_KNN_FP16_PREPARED_UNSCREENED 7   /* the same, left alone */

@@ -1,10 +1,13 @@
-"""Searches in bytes: the bound by which words are left out holds where operands are nearly exact in bytes, where activations are flat, and where
-the columns of the largest words have the smallest scores.  Operands whose scores are exact in fp32 whatever the order of the sums, against a full sort."""
+"""Searches in bytes: the bound by which words are left out holds where operands are nearly exact in bytes, where activations are flat, and where the
+columns of the largest words have no score or a small one.  Operands whose scores are exact in fp32 whatever the order of the sums, against a full sort."""
+
+import ctypes as C
 
 import numpy as np
 import pytest
 
 from test_gpu_kept_tables import best
+from test_gpu_kernels import dev
 from test_gpu_screen_bytes import LINEAR, SIGMOID, default_switches, layer, search
 
 pytestmark = pytest.mark.gpu
@@ -75,3 +78,44 @@ def test_columns_that_always_pass(pkg, dsx, rng, n, passing):
     want_keys, want_vals = best(X @ W + bias, k)
     assert np.array_equal(vals, want_vals) and np.array_equal(keys, want_keys)
     assert told == 0
+
+
+@pytest.mark.parametrize("n", WIDTHS)
+@pytest.mark.parametrize("missing,k", [(1, 1), (10, 10), (5, 10), (3000, 10)])
+def test_items_that_are_no_numbers(pkg, dsx, rng, n, missing, k):
+    """Items along one direction and queries against it: every score is far below 0, which is what the bytes of an item that is no number add up to."""
+    dim, queries = 128, 300
+    print("[case] NaN items in bytes n=%d missing=%d k=%d" % (n, missing, k), flush=True)
+    items = (5 + rng.integers(-1, 2, size=(n, dim))).astype(np.float32)
+    q = -rng.integers(1, 4, size=(queries, dim)).astype(np.float32)
+    want_scores = q @ items.T
+    gone = rng.permutation(n)[:missing]
+    items[gone, rng.integers(0, dim, missing)] = np.nan
+    want_scores[:, gone] = -100000.0
+    scores, idx, repeated = search(pkg, dsx, items, q, k)
+    want, at = best(want_scores, k)
+    assert np.array_equal(idx, at) and np.array_equal(scores, want)
+    assert repeated == 0
+
+
+def test_words_of_columns_without_scores(pkg, dsx, rng):
+    """The same items searched as if all of them were numbers: that what was listed is not enough shows in the scores, and the rows are given up."""
+    n, dim, queries, k = 131072, 128, 300, 10
+    print("[case] NaN items in bytes, taken for even", flush=True)
+    items = (5 + rng.integers(-1, 2, size=(n, dim))).astype(np.float32)
+    q = -rng.integers(1, 4, size=(queries, dim)).astype(np.float32)
+    want_scores = q @ items.T
+    gone = rng.permutation(n)[:k]
+    items[gone, 3] = np.nan
+    want_scores[:, gone] = -100000.0
+    pkg.check(dsx.dsx_testing_set_screen_bytes(1))
+    dI, dQ = dev(pkg, np.ascontiguousarray(items.T)), dev(pkg, q)
+    room = pkg.DeviceArray((dsx.dsx_knn_workspace_bytes_prepared(n, dim, queries, k),), np.uint8)
+    prepared = C.c_int(-1)
+    pkg.check(dsx.dsx_knn_prepare(dI.ptr, n, 0, dim, queries, k, room.ptr, room.nbytes, C.byref(prepared)))
+    assert prepared.value == 3
+    scores, idx = pkg.DeviceArray((queries, k), np.float32), pkg.DeviceArray((queries, k), np.uint32)
+    pkg.check(dsx.dsx_knn_search_host(4, dI.ptr, n, 0, dim, dQ.ptr, queries, k, scores.ptr, idx.ptr, None, None, room.ptr, room.nbytes, None))
+    want, at = best(want_scores, k)
+    assert np.array_equal(idx.numpy(), at) and np.array_equal(scores.numpy(), want)
+    assert dsx.dsx_knn_last_search_repeated() != 0
