@@ -24,6 +24,11 @@ constexpr int kFlagWords = 64;
 static uint32_t* g_layer_flagged = nullptr;
 static const void* g_flag_owner[kFlagWords] = {};
 static int g_flag_next = 0;
+// Behind them, per matrix too, a word that is stored when bytes leave rows open, and what follows from it: how many calls are still to go in halves, and
+// how many were to when it last happened (KnnData does the same).
+constexpr uint32_t kHalvesMost = 1024;
+static uint32_t g_halves_left[kFlagWords] = {}, g_halves_next[kFlagWords] = {};
+static bool g_bytes_last[kFlagWords] = {};   // the last call went in bytes
 
 static void layer_flags_release()
 {
@@ -42,7 +47,31 @@ static int layer_flag_slot(const void* W, bool create)
     g_flag_next = (g_flag_next + 1) % kFlagWords;
     g_flag_owner[i] = W;
     *(volatile uint32_t*)&g_layer_flagged[i] = 0;
+    *(volatile uint32_t*)&g_layer_flagged[kFlagWords + i] = 0;
+    g_halves_left[i] = g_halves_next[i] = 0;
+    g_bytes_last[i] = false;
     return i;
+}
+
+// Whether a call that could go in bytes goes in halves, as rows of a call before it were left open.  (Rows that bytes leave open are computed again in fp32,
+// 32 at a time: little for one of them, several times what halves take where all of a batch are.)
+static bool layer_in_halves(int slot)
+{
+    volatile uint32_t* open = g_layer_flagged + kFlagWords + slot;
+    if (g_halves_left[slot] != 0) {
+        g_halves_left[slot]--;
+        return true;
+    }
+    const bool was_open = *open != 0, before = g_bytes_last[slot];
+    g_bytes_last[slot] = !was_open;
+    if (!was_open) {   // (the call before may not have come that far)
+        if (before) g_halves_next[slot] /= 2;
+        return false;
+    }
+    *open = 0;
+    g_halves_next[slot] = std::min(kHalvesMost, std::max(1u, 4 * g_halves_next[slot]));
+    g_halves_left[slot] = g_halves_next[slot] - 1;
+    return true;
 }
 
 __global__ __launch_bounds__(256) void layer_clear_kernel(uint32_t* p, uint32_t n)
@@ -213,8 +242,8 @@ int dsx_fc_topk_supported(uint32_t ldx, const float* X, uint32_t activation, con
 static int layer_flags_ready()
 {
     if (g_layer_flagged) return DSX_OK;
-    DSX_HIP(hipHostMalloc((void**)&g_layer_flagged, kFlagWords * sizeof(uint32_t), hipHostMallocMapped));
-    for (int i = 0; i < kFlagWords; i++) g_layer_flagged[i] = 0;
+    DSX_HIP(hipHostMalloc((void**)&g_layer_flagged, 2 * kFlagWords * sizeof(uint32_t), hipHostMallocMapped));
+    for (int i = 0; i < 2 * kFlagWords; i++) g_layer_flagged[i] = 0;
     at_shutdown(layer_flags_release);
     return DSX_OK;
 }
@@ -237,7 +266,8 @@ static int fc_topk_common(const float* X, uint32_t ldx, const float* W, const fl
                          activation);
     if (batch == 0) return DSX_OK;
     if (int rc = layer_flags_ready()) return rc;
-    uint32_t* const flag_word = g_layer_flagged + layer_flag_slot(W, true);
+    const int slot = layer_flag_slot(W, true);
+    uint32_t* const flag_word = g_layer_flagged + slot;
     const uint32_t cap = ctx().knobs.fc_topk_candidate_capacity ? ctx().knobs.fc_topk_candidate_capacity : kLayerCandCap;   // tests lower it to reach the overflow path with small inputs
     const uint32_t n0 = layer_first_columns(n, k);
     const bool ranges = n0 < n;
@@ -249,7 +279,8 @@ static int fc_topk_common(const float* X, uint32_t ldx, const float* W, const fl
         reserved = lib_scratch_reserve(ws, layer_layout(nullptr, batch, n0, k, cap, ranges, screened, kdim, n).bytes, "dsx_fc_topk workspace");
     }
     if (reserved) return reserved;
-    const LayerWorkspace w = layer_layout(ws.ptr, batch, n0, k, cap, ranges || screened, screened, kdim, n);
+    LayerWorkspace w = layer_layout(ws.ptr, batch, n0, k, cap, ranges || screened, screened, kdim, n);
+    if (w.screen.words && layer_in_halves(slot)) w.screen = screen_layout(w.screen.rows8, batch, kdim, n, k, false);
     LayerRedo redo{};
     redo.X = X; redo.W = W; redo.bias = bias; redo.ldx = ldx; redo.ldw = n; redo.kdim = kdim; redo.n = n; redo.k = k;
     redo.act = activation;
@@ -267,7 +298,7 @@ static int fc_topk_common(const float* X, uint32_t ldx, const float* W, const fl
         j.bias = bias; j.act = activation; j.slope = redo.slope; j.alpha = redo.alpha; j.lambda = redo.lambda;
         j.position = position; j.index = index; j.fstart = filter_start; j.fend = filter_end; j.fidx = filter_index;
         j.keys = keys; j.values = values;
-        j.row_flag = w.row_flag; j.told = flag_word;
+        j.row_flag = w.row_flag; j.told = flag_word; j.open = flag_word + kFlagWords;
         j.cand = w.cand; j.cand_count = w.cand_count; j.cap = cap; j.overflow = w.overflow;
         j.clear = w.overflow; j.clear_words = 64 + layer_redo_groups(batch);   // (overflow and redo_done)
         if ((rc = screen_rows(j, t, w.screen, nullptr))) return rc;

@@ -96,7 +96,8 @@ ScreenTable screen_table_halves(void* base, uint32_t dim, uint64_t n);
 int screen_build_halves(const ScreenTable& t, const void* items16, uint64_t n, uint32_t dim);
 
 // What a call works in.  columns: how many columns' sums there is room for, all of them or a first block's; screen_run goes by that and not by its
-// own number of columns.
+// own number of columns.  kept: the table has bytes, and the search goes by them where screen_in_bytes says so; one that has to be done again in halves works
+// in the same bytes, laid out with kept = false.
 struct ScreenWorkspace {
     uint32_t columns;
     void* rows16;
@@ -122,10 +123,10 @@ struct ScreenWorkspace {
 ScreenWorkspace screen_layout(void* base, uint32_t batch, uint32_t dim, uint64_t n, uint32_t k, bool kept);
 
 // Nearest neighbours, in pinned memory: the largest norm of the table, a sample of the norms and how many they are; whether a row
-// cannot be screened.
+// cannot be screened, or not in bytes.
 struct ScreenNotes {
     float largest, sum;
-    uint32_t number, flag;
+    uint32_t number, flag, open;
 };
 
 struct ScreenJob {
@@ -145,6 +146,7 @@ struct ScreenJob {
     uint32_t* values2;
     uint32_t* row_flag;       // [batch] set for rows without a result (the caller computes them again), 0 for the others
     uint32_t* told;           // word that is set to 1 with the first of them (may be host memory; may be NULL)
+    uint32_t* open;           // the same for those that a search in halves may have results of, as bytes alone left too much of them open (may be NULL)
     uint64_t* cand;           // [batch][cap]
     uint32_t* cand_count;     // [batch]
     uint32_t cap;

@@ -468,6 +468,7 @@ struct ScreenFoldArgs {
     float slope, alpha, lambda;
     uint32_t* row_flag;
     uint32_t* told;
+    uint32_t* open;
     uint32_t position;
     const uint32_t* index;
     const uint64_t* fstart;
@@ -544,6 +545,13 @@ __device__ __forceinline__ void screen_flag(const ScreenFoldArgs& a, uint32_t b)
     a.row_flag[b] = 1;
     if (a.told) *(volatile uint32_t*)a.told = 1u;
     if (a.admit) a.admit[b] = 0xffffffffu;   // a NaN: nothing more of the row is wanted
+}
+
+// What bytes leave too much of open; halves may not.
+__device__ __forceinline__ void screen_open(const ScreenFoldArgs& a, uint32_t b)
+{
+    a.row_flag[b] = 1;
+    if (a.open) *(volatile uint32_t*)a.open = 1u;
 }
 
 // The row itself into LDS, zero filled to whole rounds of the loop below; first: the caller's component threadIdx.x of it.
@@ -1425,7 +1433,7 @@ __global__ __launch_bounds__(256, 4) void i8_finish_kernel(ScreenFoldArgs a, I8N
     __syncthreads();
     uint32_t count = sCount, scored = count, kept = 0;
     if (count > kBestWords) {
-        if (tid == 0) screen_flag(a, b);
+        if (tid == 0) screen_open(a, b);
         return;
     }
     float cut = 0.0f;
@@ -1467,7 +1475,7 @@ __global__ __launch_bounds__(256, 4) void i8_finish_kernel(ScreenFoldArgs a, I8N
             // a sum that was raised by more than it should have been.)
             const float4 most = *e.error_most;
             if (!all && least > kNoWord + 0x10000 && fmaf(i8_first((uint32_t)i8_sortable(least)), step, fmaf(e1, most.x, e2 * most.y) * 1.000001f) >= cut) {
-                if (tid == 0) screen_flag(a, b);
+                if (tid == 0) screen_open(a, b);
                 return;
             }
             each(std::true_type{}, [&](uint32_t block, int32_t x, bool dead, float2 e) {
@@ -1491,7 +1499,7 @@ __global__ __launch_bounds__(256, 4) void i8_finish_kernel(ScreenFoldArgs a, I8N
         if (tid == 0) sOpened = 0;
         if (!__syncthreads_or(pending != 0)) break;
         if (scored > kBestMost || kept > kBestWords / 2) {
-            if (tid == 0) screen_flag(a, b);
+            if (tid == 0) screen_open(a, b);
             return;
         }
 #pragma unroll
@@ -1685,7 +1693,7 @@ ScreenWorkspace screen_layout(void* base, uint32_t batch, uint32_t dim, uint64_t
         p += align256((size_t)batch * kNearWords * sizeof(uint2));
         w.near_found = (uint2*)p;
         p += align256((size_t)batch * sizeof(uint2));
-        w.bytes = (size_t)(p - (char*)base);
+        w.bytes = std::max((size_t)(p - (char*)base), screen_layout(nullptr, batch, dim, n, k, false).bytes);
         return w;
     }
     // (decided here for every search in this workspace, which may be of fewer columns: pad rows of an item table)
@@ -1819,7 +1827,7 @@ static ScreenFoldArgs fold_args(const ScreenJob& j, const ScreenTable& t)
     ScreenFoldArgs a{};
     a.batch = j.batch; a.k = j.k; a.n = j.n;
     a.act = j.act; a.slope = j.slope; a.alpha = j.alpha; a.lambda = j.lambda;
-    a.row_flag = j.row_flag; a.told = j.told;
+    a.row_flag = j.row_flag; a.told = j.told; a.open = j.open;
     a.position = j.position; a.index = j.index; a.fstart = j.fstart; a.fend = j.fend; a.fidx = j.fidx;
     a.X = j.X; a.ldx = j.ldx; a.dim = j.dim; a.pitch32 = screen_pitch32(j.dim); a.rows32 = t.rows32; a.bias = j.bias;
     a.keys = j.keys; a.values = j.values; a.keys2 = j.keys2; a.values2 = j.values2;

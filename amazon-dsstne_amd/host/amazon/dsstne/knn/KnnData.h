@@ -98,9 +98,10 @@ struct KnnData {
 
 private:
     friend class KnnExactGpu;
-    // Searches that are to go without screening, and how many were to when it last had to be repeated: every repetition doubles the number (64 at
-    // most), every search that went well halves it.
+    // Searches that are to go without screening (unscreenedStorage: or without bytes), and how many were to when one last had to be repeated: every repetition
+    // doubles the number (64 at most), every search that went well halves it.
     uint32_t unscreened = 0, unscreenedNext = 0;
+    int unscreenedStorage = 0;
     // the pinned memory that load put into hResultScores and hResultIndexes
     void* pinnedScores = nullptr;
     void* pinnedIndexes = nullptr;

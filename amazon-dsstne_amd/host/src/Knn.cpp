@@ -357,7 +357,7 @@ void KnnExactGpu::searchDevice(int k, const float* inputs, int size)
     const bool kept = data->workspacePrepared[device] != 0 && !data->dCollectionPartitions.handedOut && !data->dWorkspaces.handedOut;
     const bool halves = data->dataType == DataType::FP16;
     const int storage = data->dataType == DataType::FP32Split ? DSX_KNN_SPLIT
-                        : kept && data->unscreened != 0       ? (halves ? DSX_KNN_FP16_PREPARED_UNSCREENED : DSX_KNN_FP32_PREPARED_UNSCREENED)
+                        : kept && data->unscreened != 0       ? data->unscreenedStorage
                         : kept                                ? data->workspacePrepared[device]
                         : halves                              ? DSX_KNN_FP16
                                                               : DSX_KNN_FP32;
@@ -371,11 +371,19 @@ void KnnExactGpu::searchDevice(int k, const float* inputs, int size)
           "KnnExactGpu::search");
     data->elapsedSgemm[device] = elapsed[0];
     data->elapsedTopK[device] = elapsed[1];
-    if (kept && data->unscreened != 0)
-        data->unscreened--;
-    else if (kept) {
-        data->unscreenedNext = dsx_knn_last_search_repeated() ? std::min(64u, std::max(1u, 2 * data->unscreenedNext)) : data->unscreenedNext / 2;
-        if (dsx_knn_last_search_repeated()) data->unscreened = data->unscreenedNext;
+    if (kept) {
+        const int repeated = dsx_knn_last_search_repeated();
+        if (repeated != 0) {   // (also one without bytes, if halves are not enough any more)
+            data->unscreened = data->unscreenedNext = std::min(64u, std::max(1u, 2 * data->unscreenedNext));
+            const bool even = data->workspacePrepared[device] == DSX_KNN_FP32_PREPARED_EVEN;
+            data->unscreenedStorage = halves          ? DSX_KNN_FP16_PREPARED_UNSCREENED
+                                      : repeated == 1 ? DSX_KNN_FP32_PREPARED_UNSCREENED
+                                      : even          ? DSX_KNN_FP32_PREPARED_EVEN_HALVES
+                                                      : DSX_KNN_FP32_PREPARED_HALVES;
+        } else if (data->unscreened != 0)
+            data->unscreened--;
+        else
+            data->unscreenedNext /= 2;
     }
     if (pinned) return;
     check(dsx_memcpy_d2h(hScores, dScores, bytes), "KnnExactGpu::search");

@@ -342,7 +342,8 @@ int dsx_fc_topk_screened_pays(uint32_t batch, uint32_t k_dim, uint32_t n, uint32
 int dsx_fc_topk_pays(uint32_t batch, uint32_t k_dim, uint32_t n, uint32_t activation, uint32_t k);
 int dsx_fc_topk_supported(uint32_t ldx, const float* X, uint32_t activation, const dsx_act_params* params, const float* filter_mul);
 /* 1 if any row of any dsx_fc_topk call so far had to be recomputed (reset != 0 clears the mark); dsx_fc_topk_flagged_for: the
- * same for the calls with this weight matrix only (the mark is kept per W pointer, for the 64 matrices used last). */
+ * same for the calls with this weight matrix only (the mark is kept per W pointer, for the 64 matrices used last).  Rows of dsx_fc_topk_screened that were
+ * because bytes did not say enough of them leave no mark: the calls that follow go by 16 bits, one at first, and up to 1,024 where it happens again. */
 int dsx_fc_topk_flagged(int reset);
 int dsx_fc_topk_flagged_for(const float* W, int reset);
 
@@ -380,6 +381,8 @@ int dsx_knn_prepare(const float* items, uint32_t rows_padded, uint32_t padding, 
 #define DSX_KNN_FP32_PREPARED_UNSCREENED 5   /* a prepared workspace, whose copies are left alone: searched without screening */
 #define DSX_KNN_FP16_PREPARED 6              /* dsx_knn_prepare_f16 */
 #define DSX_KNN_FP16_PREPARED_UNSCREENED 7   /* the same, left alone */
+#define DSX_KNN_FP32_PREPARED_HALVES 8       /* as DSX_KNN_FP32_PREPARED and _EVEN, but the copy in bytes is left alone: screened in 16 bits */
+#define DSX_KNN_FP32_PREPARED_EVEN_HALVES 9
 int dsx_knn_search_host(int storage, const void* items, uint32_t rows_padded, uint32_t padding, uint32_t dim, const float* queries,
                         uint32_t num_queries, uint32_t k, float* scores, uint32_t* indexes, float* host_scores, uint32_t* host_indexes,
                         void* workspace, size_t workspace_bytes, float* elapsed_ms);
@@ -417,7 +420,8 @@ size_t dsx_knn_workspace_bytes_split(uint32_t rows_padded, uint32_t dim, uint32_
 #define DSX_KNN_PATH_CANDIDATES_REDONE 2  /* a candidate list filled up: repeated block by block */
 int dsx_knn_last_search_path(void);
 /* 1 if the last search was screened in 16 bits or in bytes and found rows that cannot be (thousands of ties, norms beyond f16's range), so that it was repeated
- * without: a caller with more such queries is better off with DSX_KNN_FP32_PREPARED_UNSCREENED. */
+ * without: a caller with more such queries is better off with DSX_KNN_FP32_PREPARED_UNSCREENED (DSX_KNN_FP16_PREPARED_UNSCREENED).  2 if bytes were not enough
+ * (thousands of items whose scores they cannot tell from the k-th) and 16 bits were: DSX_KNN_FP32_PREPARED_HALVES or _EVEN_HALVES. */
 int dsx_knn_last_search_repeated(void);
 /* dsx_knn_search_f16 scores the column ranges after the first block one workgroup per tile, or, when a range has enough item
  * tiles, with workgroups that keep their queries and walk a chunk of the range each (private candidate lists, no atomics on
