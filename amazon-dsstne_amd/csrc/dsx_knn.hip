@@ -739,7 +739,8 @@ int dsx_knn_prepare(const float* items, uint32_t rows_padded, uint32_t padding, 
     *prepared = 0;
     if (!knn_prepares(rows_padded, dim, num_queries, k) || workspace_bytes < dsx_knn_workspace_bytes_prepared(rows_padded, dim, num_queries, k)) return DSX_OK;
     const uint32_t M = rows_padded - padding;
-    const ScreenTable t = screen_table(workspace, dim, rows_padded, true);
+    ScreenTable t = screen_table(workspace, dim, rows_padded, true);
+    if (!screen_in_bytes(num_queries, dim, rows_padded, k)) t.items8 = nullptr;   // (no search of so few goes by them; their place is the table's all the same)
     if (int rc = screen_build(t, items, rows_padded, M, dim)) return rc;
     uint32_t stats[8];
     DSX_HIP(hipMemcpyAsync(stats, t.stats, sizeof(stats), hipMemcpyDeviceToHost, ctx().stream));

@@ -75,7 +75,7 @@ __device__ __forceinline__ float i8_second(uint32_t word)
 }
 
 // The table of a screened search: two row-major copies (f16, fp32), the columns' norms and what they are like; one that is kept holds a copy in bytes
-// as well.  Laid out in screen_table(...).bytes bytes at base, filled by screen_build from W [dim][ldw].
+// as well where searches may go by it.  Laid out in screen_table(...).bytes bytes at base, filled by screen_build from W [dim][ldw].
 struct ScreenTable {
     void* items16;
     float* rows32;

@@ -1609,6 +1609,13 @@ static uint32_t screen_first_columns(uint32_t n, uint32_t k)
 // (what i8_wide_kernel takes, or a whole number of f16_sweep_kernel's pairs of stages)
 static uint32_t i8_ld(uint32_t dim) { return dim > 256 && dim <= 512 ? 512 : (dim + 127) / 128 * 128; }
 
+// What of that is known of a table alone: whether one that is kept holds a copy in bytes.  (Vectors of up to 64 and of 257 to 320 components are mostly padding:
+// 128 bytes beside the 96 to 384 of the other copies, which nothing would read.)
+static bool screen_has_bytes(uint32_t dim, uint64_t n)
+{
+    return n <= kBestColumns && (ctx().knobs.screen_bytes == 1 || (n >= 20000 && 3 * i8_ld(dim) <= 4 * screen_ld(dim)));
+}
+
 // Whether a search with a kept table goes in bytes: many products of a long table, whose bytes are not mostly padding, of which k columns are a small part (else
 // blocks with one candidate hold a second one, and all 32 columns are scored).  Fitted to 1,814 searches and layers (12,000 to 1,000,000 columns, 16 to
 // 1,024 components, 1 to 4,096 rows, k 1 to 200) measured both ways: 3.1 % of the time they could
@@ -1618,11 +1625,10 @@ static uint32_t i8_ld(uint32_t dim) { return dim > 256 && dim <= 512 ? 512 : (di
 // 8 x 256 x 500,000 top 50 114 / 115, 256 x 1,024 x 27,278 top 100 87 / 276.
 bool screen_in_bytes(uint32_t batch, uint32_t dim, uint64_t n, uint32_t k)
 {
-    if (n > kBestColumns || n < 64 * (uint64_t)k || ctx().knobs.screen_bytes == 2) return false;
+    if (!screen_has_bytes(dim, n) || n < 64 * (uint64_t)k || ctx().knobs.screen_bytes == 2) return false;
     if (ctx().knobs.screen_bytes == 1) return true;
-    const uint32_t ld = screen_ld(dim);
-    return !ctx().knobs.fc_topk_first_columns && n >= std::max<uint64_t>(20000, 2500 * (uint64_t)k) && 3 * i8_ld(dim) <= 4 * ld &&
-           (dim <= 512 || batch >= 1024) && (double)batch * (double)n * ld >= (n < 65536 ? 2e10 : 4e9);
+    return !ctx().knobs.fc_topk_first_columns && n >= 2500 * (uint64_t)k && (dim <= 512 || batch >= 1024) &&
+           (double)batch * (double)n * screen_ld(dim) >= (n < 65536 ? 2e10 : 4e9);
 }
 
 ScreenTable screen_table(void* base, uint32_t dim, uint64_t n, bool kept)
@@ -1644,7 +1650,7 @@ ScreenTable screen_table(void* base, uint32_t dim, uint64_t n, bool kept)
     t.unit8 = nullptr;
     t.error8 = nullptr;
     t.side8 = nullptr;
-    if (kept && n <= kBestColumns) {
+    if (kept && screen_has_bytes(dim, n)) {
         t.items8 = p;
         p += align256(rows * i8_ld(dim));
         t.unit8 = (float*)p;

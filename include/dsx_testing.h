@@ -33,7 +33,7 @@ int dsx_testing_occupy(uint32_t workgroups, uint32_t cycles, uint32_t vgprs);
  * depend on it. */
 int dsx_testing_set_screen(int mode);
 /* Screened searches with a kept table: in bytes where that is expected to be the faster way (0, default), wherever it can be (1), never (2).
- * Workspace sizes depend on it. */
+ * Workspaces and tables depend on it: both are made behind the call. */
 int dsx_testing_set_screen_bytes(int mode);
 /* dsx_knn_search*: the events that its stages' times are taken with cannot be made (1; 0, the default: as the device has it). */
 int dsx_testing_set_knn_no_events(int none);

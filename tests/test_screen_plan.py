@@ -53,3 +53,14 @@ def test_where_sums_are_stored(pkg):
                                 (4096, 49663, 1, 0), (4096, 49664, 1, 1), (1024, 65536, 1, 0), (1024, 98304, 10, 0), (1024, 131072, 10, 1), (512, 400000, 1, 1),
                                 (512, 262144, 32, 0), (512, 524288, 32, 1)):
         assert plan(lib, pkg, batch, n, 0, k)[2] == ranges, (batch, n, k)
+
+
+@pytest.mark.parametrize("dim,n,bytes_kept", [(16, 1000000, 0), (64, 1000000, 0), (65, 1000000, 128), (128, 19999, 0), (128, 20000, 128), (256, 300000, 256), (257, 300000, 0),
+                                              (320, 300000, 0), (321, 300000, 512), (1024, 27278, 1024), (128, 1048577, 0)])
+def test_tables_hold_bytes_where_searches_may_go_by_them(pkg, dim, n, bytes_kept):
+    """Beside both copies and the norms: a column's bytes, and 4.7 for units, errors and what sums start from."""
+    lib = pkg.load_library()
+    rows = (n + 255) // 256 * 256
+    others = rows * ((dim + 63) // 64 * 64) * 2 + n * ((dim + 3) // 4 * 4) * 4 + rows * 4 + rows // 64 * 4
+    extra = lib.dsx_screen_table_bytes(n, dim) - others
+    assert 0 <= extra - (rows * (bytes_kept + 4) if bytes_kept else 0) <= (rows if bytes_kept else 0) + 4096
