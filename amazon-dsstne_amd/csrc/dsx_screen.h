@@ -115,6 +115,7 @@ struct ScreenWorkspace {
     float* unit8;
     float4* error8;
     float* side8;             // i8_wide_run's, with the call's biases
+    uint32_t rows;            // whose words there is room for
     uint32_t* words;
     uint2* near;
     uint2* near_found;
@@ -153,7 +154,7 @@ struct ScreenJob {
     uint32_t* overflow;       // scratch word
     uint32_t* clear;          // [clear_words] set to 0 on the way
     uint32_t clear_words;
-    void (*before_last)(void*);   // called before the kernel that ends with the results is launched (NULL: not)
+    void (*before_last)(void*);   // called before the kernel that ends with the (last) results is launched (NULL: not)
     void* before_last_arg;
     const void* rows16;       // the table as halves: scores are products of these and of the rows rounded to halves (NULL: of floats); for searches in bytes
     bool even;                // no bias, no column that always passes or (where the table has bytes) is no number, and norms close together (screen_even)

@@ -1120,6 +1120,7 @@ constexpr uint32_t kBestWords = 2048;    // candidates of a row at a time
 constexpr uint32_t kBestMost = 16384;    // candidates of a row beyond the first k (and as many as it has listed columns): with more it is left open
 constexpr uint32_t kBestColumns = 1u << 20;
 constexpr uint32_t kNearWords = 4096;    // words of a row that are listed
+constexpr uint32_t kAloneColumns = 32768;   // up to here i8_finish_kernel looks through a row's words itself
 
 // Sums of bytes: a word for every 32 columns says what the largest of their sums is at most, whose it is, and what the others are at most.  The columns
 // of the k largest words are scored first; then all columns whose words reach the k-th of those scores, and where the others of a block
@@ -1685,6 +1686,17 @@ ScreenTable screen_table_halves(void* base, uint32_t dim, uint64_t n)
     return t;
 }
 
+// Words of a row, and how many rows' words (and lists) there is room for: 1 GiB of them (6,144 rows of a million columns), else as many as leave equal parts.
+constexpr uint64_t kWordsRoom = (uint64_t)1 << 30;
+static uint64_t i8_row_words(uint64_t n) { return (n + 255) / 256 * 8; }
+static uint32_t i8_rows(uint32_t batch, uint64_t n)
+{
+    const uint64_t row = i8_row_words(n) * sizeof(uint32_t) + (n > kAloneColumns ? (kNearWords + 1) * sizeof(uint2) : 0), most = std::max<uint64_t>(512, kWordsRoom / row / 512 * 512);
+    if (batch <= most) return batch;
+    const uint64_t parts = (batch + most - 1) / most;
+    return (uint32_t)((batch + parts * 512 - 1) / (parts * 512) * 512);   // (whole workgroups' rows)
+}
+
 ScreenWorkspace screen_layout(void* base, uint32_t batch, uint32_t dim, uint64_t n, uint32_t k, bool kept)
 {
     ScreenWorkspace w{};
@@ -1699,12 +1711,15 @@ ScreenWorkspace screen_layout(void* base, uint32_t batch, uint32_t dim, uint64_t
         p += align256((size_t)batch * sizeof(float4));
         w.side8 = (float*)p;
         p += align256(knn_f16_rows(n) / 32 * kI8Side * sizeof(float) + kI8SideSlack);
+        w.rows = i8_rows(batch, n);
         w.words = (uint32_t*)p;
-        p += align256(batch * ((n + 255) / 256 * 8) * sizeof(uint32_t));
-        w.near = (uint2*)p;
-        p += align256((size_t)batch * kNearWords * sizeof(uint2));
-        w.near_found = (uint2*)p;
-        p += align256((size_t)batch * sizeof(uint2));
+        p += align256(w.rows * i8_row_words(n) * sizeof(uint32_t));
+        if (n > kAloneColumns) {
+            w.near = (uint2*)p;
+            p += align256((size_t)w.rows * kNearWords * sizeof(uint2));
+            w.near_found = (uint2*)p;
+            p += align256((size_t)w.rows * sizeof(uint2));
+        }
         w.bytes = std::max((size_t)(p - (char*)base), screen_layout(nullptr, batch, dim, n, k, false).bytes);
         return w;
     }
@@ -1849,39 +1864,56 @@ static ScreenFoldArgs fold_args(const ScreenJob& j, const ScreenTable& t)
 static int screen_run_bytes(const ScreenJob& j, const ScreenTable& t, const ScreenWorkspace& w)
 {
     F16Job f{};
-    f.Q = w.rows8; f.items = t.items8; f.ld = i8_ld(j.dim) / 2; f.batch = j.batch; f.n = j.n;
+    f.items = t.items8; f.ld = i8_ld(j.dim) / 2; f.n = j.n;
     f.norm = t.norm; f.bias = j.bias; f.bias_raise = screen_bias_raise(j.dim);
-    f.scale = w.unit8; f.unit = t.unit8; f.words = w.words; f.ldw = ((uint64_t)j.n + 255) / 256 * 8;
-    const bool starts = j.bias || !j.even;
-    if (int rc = i8_wide_takes(f.ld * 2, j.batch) ? i8_wide_run(f, j.bias ? w.side8 : t.side8, starts) : i8_best_run(f, starts)) return rc;
+    f.unit = t.unit8; f.words = w.words; f.ldw = i8_row_words(j.n);
     ScreenFoldArgs a = fold_args(j, t);
-    a.words = w.words; a.ldw = f.ldw; a.error_items = t.error8; a.error_rows = w.error8; a.near = w.near; a.near_found = w.near_found;
-    I8NearArgs e{};
-    e.batch = j.batch; e.k = j.k; e.n = j.n; e.words = w.words; e.ldw = f.ldw; e.error_rows = w.error8; e.unit = w.unit8;
-    e.error_most = reinterpret_cast<const float4*>(t.stats + 4);
-    e.row_flag = j.row_flag; e.position = j.position; e.index = j.index; e.fstart = j.fstart; e.fend = j.fend; e.fidx = j.fidx;
-    e.near = w.near; e.near_found = w.near_found;
-    e.act = j.act; e.slope = j.slope; e.alpha = j.alpha; e.lambda = j.lambda;
-    const size_t row_lds = (size_t)(j.dim + 127) / 128 * 512;
-    if (j.before_last) j.before_last(j.before_last_arg);
-    const bool alone = j.n <= 32768;   // (no kernel of its own for the words)
-    if (!alone) {
-        if (j.n <= kBestColumns / 4) hipLaunchKernelGGL((i8_near_kernel<4>), dim3(j.batch), dim3(512), 0, ctx().stream, e);
-        else hipLaunchKernelGGL((i8_near_kernel<16>), dim3(j.batch), dim3(512), 0, ctx().stream, e);
-        DSX_LAUNCH_CHECK("i8_near_kernel");
-    }
-    auto finish = [&](auto halves) {
-        constexpr bool H = decltype(halves)::value;
-        if (!alone) hipLaunchKernelGGL((i8_finish_kernel<H, 0>), dim3(j.batch), dim3(256), row_lds, ctx().stream, a, e);
-        else if (j.k <= 32) hipLaunchKernelGGL((i8_finish_kernel<H, 1>), dim3(j.batch), dim3(256), row_lds, ctx().stream, a, e);
-        else hipLaunchKernelGGL((i8_finish_kernel<H, 2>), dim3(j.batch), dim3(256), row_lds, ctx().stream, a, e);
-    };
+    a.words = w.words; a.ldw = f.ldw; a.error_items = t.error8; a.near = w.near; a.near_found = w.near_found;
     if (j.rows16) {
         a.rows16 = (const _Float16*)j.rows16;
         a.ld16 = knn_f16_ld(j.dim);
-        finish(std::true_type{});
-    } else finish(std::false_type{});
-    DSX_LAUNCH_CHECK("i8_finish_kernel");
+    }
+    I8NearArgs e{};
+    e.k = j.k; e.n = j.n; e.words = w.words; e.ldw = f.ldw;
+    e.error_most = reinterpret_cast<const float4*>(t.stats + 4);
+    e.index = j.index; e.fstart = j.fstart; e.fend = j.fend; e.fidx = j.fidx;
+    e.near = w.near; e.near_found = w.near_found;
+    e.act = j.act; e.slope = j.slope; e.alpha = j.alpha; e.lambda = j.lambda;
+    const bool starts = j.bias || !j.even;
+    const size_t row_lds = (size_t)(j.dim + 127) / 128 * 512;
+    const bool alone = j.n <= kAloneColumns;   // (no kernel of its own for the words)
+    for (uint32_t r = 0; r < j.batch; r += w.rows) {
+        const uint32_t rows = std::min(w.rows, j.batch - r);
+        const uint64_t results = (uint64_t)r * j.k;
+        f.Q = (const int8_t*)w.rows8 + (uint64_t)r * i8_ld(j.dim); f.scale = w.unit8 + r; f.batch = rows;
+        if (int rc = i8_wide_takes(f.ld * 2, rows) ? i8_wide_run(f, j.bias ? w.side8 : t.side8, starts) : i8_best_run(f, starts)) return rc;
+        a.batch = e.batch = rows;
+        a.X = j.X + (uint64_t)r * j.ldx;
+        e.error_rows = a.error_rows = w.error8 + r;
+        e.unit = w.unit8 + r;
+        e.row_flag = a.row_flag = j.row_flag + r;
+        a.position = e.position = j.position + r;
+        a.keys = j.keys + results; a.values = j.values + results;
+        if (j.keys2) {
+            a.keys2 = j.keys2 + results;
+            a.values2 = j.values2 + results;
+        }
+        if (j.before_last && r + rows == j.batch) j.before_last(j.before_last_arg);
+        if (!alone) {
+            if (j.n <= kBestColumns / 4) hipLaunchKernelGGL((i8_near_kernel<4>), dim3(rows), dim3(512), 0, ctx().stream, e);
+            else hipLaunchKernelGGL((i8_near_kernel<16>), dim3(rows), dim3(512), 0, ctx().stream, e);
+            DSX_LAUNCH_CHECK("i8_near_kernel");
+        }
+        auto finish = [&](auto halves) {
+            constexpr bool H = decltype(halves)::value;
+            if (!alone) hipLaunchKernelGGL((i8_finish_kernel<H, 0>), dim3(rows), dim3(256), row_lds, ctx().stream, a, e);
+            else if (j.k <= 32) hipLaunchKernelGGL((i8_finish_kernel<H, 1>), dim3(rows), dim3(256), row_lds, ctx().stream, a, e);
+            else hipLaunchKernelGGL((i8_finish_kernel<H, 2>), dim3(rows), dim3(256), row_lds, ctx().stream, a, e);
+        };
+        if (j.rows16) finish(std::true_type{});
+        else finish(std::false_type{});
+        DSX_LAUNCH_CHECK("i8_finish_kernel");
+    }
     return DSX_OK;
 }
 

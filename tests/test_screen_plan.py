@@ -64,3 +64,18 @@ def test_tables_hold_bytes_where_searches_may_go_by_them(pkg, dim, n, bytes_kept
     others = rows * ((dim + 63) // 64 * 64) * 2 + n * ((dim + 3) // 4 * 4) * 4 + rows * 4 + rows // 64 * 4
     extra = lib.dsx_screen_table_bytes(n, dim) - others
     assert 0 <= extra - (rows * (bytes_kept + 4) if bytes_kept else 0) <= (rows if bytes_kept else 0) + 4096
+
+
+@pytest.mark.parametrize("queries", [4096, 16384, 65536])
+def test_words_of_many_rows_have_a_bound(pkg, queries):
+    """What a search in bytes works in beside what one in halves does: 1 GiB, and what its rows take themselves."""
+    lib = pkg.load_library()
+    n, dim, k = 1000000, 128, 100
+    try:
+        for bytes_of in (lambda: lib.dsx_knn_workspace_bytes_prepared(n, dim, queries, k), lambda: lib.dsx_knn_workspace_bytes_f16_prepared(n, dim, queries, k) - n * (dim + 8)):
+            pkg.check(lib.dsx_testing_set_screen_bytes(0))
+            in_bytes = bytes_of()
+            pkg.check(lib.dsx_testing_set_screen_bytes(2))
+            assert in_bytes <= bytes_of() + (1 << 30) + queries * (dim + 24) + (40 << 20)
+    finally:
+        pkg.check(lib.dsx_testing_reset())
