@@ -555,17 +555,23 @@ __device__ __forceinline__ void screen_open(const ScreenFoldArgs& a, uint32_t b)
 }
 
 // The row itself into LDS, zero filled to whole rounds of the loop below; first: the caller's component threadIdx.x of it.
-template <int T, bool HALVES = false> __device__ __forceinline__ void screen_row(const ScreenFoldArgs& a, uint32_t b, float* sX, float first)
+template <int T> __device__ __forceinline__ void screen_row(const ScreenFoldArgs& a, uint32_t b, float* sX, float first)
 {
-    const uint32_t dpad = HALVES ? (a.dim + 127) / 128 * 128 : (a.dim + 63) / 64 * 64;
-    auto as_kept = [](float x) { return HALVES ? (float)(_Float16)x : x; };
-    if (threadIdx.x < dpad) sX[threadIdx.x] = as_kept(first);
-    for (uint32_t d = T + threadIdx.x; d < dpad; d += T) sX[d] = (d < a.dim) ? as_kept(a.X[(uint64_t)b * a.ldx + d]) : 0.0f;
+    const uint32_t dpad = (a.dim + 63) / 64 * 64;
+    if (threadIdx.x < dpad) sX[threadIdx.x] = first;
+    for (uint32_t d = T + threadIdx.x; d < dpad; d += T) sX[d] = (d < a.dim) ? a.X[(uint64_t)b * a.ldx + d] : 0.0f;
+}
+
+// The same as halves, as items of an fp16 table are laid out.
+template <int T> __device__ __forceinline__ void screen_row_halves(const ScreenFoldArgs& a, uint32_t b, _Float16* sX, float first)
+{
+    if (threadIdx.x < a.ld16) sX[threadIdx.x] = (_Float16)first;
+    for (uint32_t d = T + threadIdx.x; d < a.ld16; d += T) sX[d] = (d < a.dim) ? (_Float16)a.X[(uint64_t)b * a.ldx + d] : (_Float16)0.0f;
 }
 
 // The row's candidates sList[from .. count) scored in fp32: their words get the scores' keys, and become 0 where a score is no number.  Sixteen lanes per
 // candidate; the order of a sum depends on nothing but its length.  Every lane of the workgroup calls this.
-template <int T, int STEPS = 2, bool HALVES = false> __device__ __forceinline__ void screen_score(const ScreenFoldArgs& a, uint64_t* sList, uint32_t from, uint32_t count, const float* sX)
+template <int T, int STEPS = 2> __device__ __forceinline__ void screen_score(const ScreenFoldArgs& a, uint64_t* sList, uint32_t from, uint32_t count, const float* sX)
 {
     // (four candidates of a group of lanes at a time: their rows are waited for together)
     constexpr int U = 4;
@@ -578,21 +584,6 @@ template <int T, int STEPS = 2, bool HALVES = false> __device__ __forceinline__ 
             col[u] = ~(uint32_t)sList[min(e0 + T / 16 * u, count - 1)];
             sum[u] = 0.0f;
         }
-        if constexpr (HALVES) {
-#pragma unroll STEPS
-            for (uint32_t d = 8 * sub; d < a.ld16; d += 128) {
-                half8 v[U];
-#pragma unroll
-                for (int u = 0; u < U; u++)
-                    if (u == 0 || e0 + T / 16 * u < count) v[u] = *reinterpret_cast<const half8*>(a.rows16 + (uint64_t)col[u] * a.ld16 + d);
-#pragma unroll
-                for (int u = 0; u < U; u++)
-                    if (u == 0 || e0 + T / 16 * u < count) {
-#pragma unroll
-                        for (int e = 0; e < 8; e++) sum[u] = fmaf(sX[d + e], (float)v[u][e], sum[u]);
-                    }
-            }
-        } else
 #pragma unroll STEPS
         for (uint32_t d = 4 * sub; d < a.pitch32; d += 64) {
             const float4 x = *reinterpret_cast<const float4*>(sX + d);
@@ -618,6 +609,48 @@ template <int T, int STEPS = 2, bool HALVES = false> __device__ __forceinline__ 
                 sList[e0 + T / 16 * u] = (y == y) ? ((uint64_t)score_key(y) << 32) | (uint32_t)~col[u] : 0ull;
             }
         }
+    }
+}
+
+// The same of an fp16 table: exact products, summed by the matrix instruction of the searches that are not screened, in their order (dsx_f16.hip), so that a
+// score has the same bits whichever way a search goes.  A wavefront takes 32 candidates, as the row operand; every column of the other one is the query.
+template <int T> __device__ __forceinline__ void screen_score_halves(const ScreenFoldArgs& a, uint64_t* sList, uint32_t from, uint32_t count, const _Float16* sX)
+{
+    const uint32_t lane = threadIdx.x % kWave, l32 = lane % 32, lhi = lane / 32;
+    for (uint32_t e0 = from + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) * 32; e0 < count; e0 += T / kWave * 32) {
+        const uint32_t col = ~(uint32_t)sList[e0 + l32 < count ? e0 + l32 : e0];   // (no other wavefront's words, which change)
+        const _Float16* row = a.rows16 + (uint64_t)col * a.ld16 + 8 * lhi;
+        floatx16 sums;
+#pragma unroll
+        for (int v = 0; v < 16; v++) sums[v] = 0.0f;
+        auto pieces = [&](half8 (&item)[4], uint32_t d) __attribute__((always_inline)) {
+#pragma unroll
+            for (int s = 0; s < 4; s++) item[s] = *reinterpret_cast<const half8*>(row + d + 16 * s);
+        };
+        auto add = [&](const half8 (&item)[4], uint32_t d) __attribute__((always_inline)) {
+#pragma unroll
+            for (int s = 0; s < 4; s++)
+                sums = __builtin_amdgcn_mfma_f32_32x32x16_f16(item[s], *reinterpret_cast<const half8*>(sX + d + 16 * s + 8 * lhi), sums, 0, 0, 0);
+        };
+        // (ld16 is a multiple of 64; the next 64 components are on their way while these are multiplied, the last ones twice)
+        half8 now[4], next[4];
+        pieces(now, 0);
+#pragma unroll 1
+        for (uint32_t d = 0; d < a.ld16; d += 128) {
+            pieces(next, min(d + 64, a.ld16 - 64));
+            __builtin_amdgcn_sched_barrier(0);
+            add(now, d);
+            if (d + 64 >= a.ld16) break;
+            pieces(now, min(d + 128, a.ld16 - 64));
+            __builtin_amdgcn_sched_barrier(0);
+            add(next, d + 64);
+        }
+        // Result v of a lane is candidate v % 4 + v / 4 * 8 + 4 lhi, the same in all 32 lanes: lane v of them takes it.
+        float y = sums[0];
+#pragma unroll
+        for (int v = 1; v < 16; v++) y = l32 == (uint32_t)v ? sums[v] : y;
+        const uint32_t at = e0 + l32 % 4 + l32 / 4 * 8 + 4 * lhi;
+        if (l32 < 16 && at < count) sList[at] = (y == y) ? ((uint64_t)score_key(y) << 32) | (uint32_t)sList[at] : 0ull;
     }
 }
 
@@ -1372,7 +1405,8 @@ __global__ __launch_bounds__(256, 4) void i8_finish_kernel(ScreenFoldArgs a, I8N
     for (uint32_t i = tid; i < bitmap; i += T) sHot[i] = sMore[i] = 0;
     sBest[tid] = 0;
     if (tid == 0) sCount = sAhead = 0;
-    screen_row<T, HALVES>(a, b, sX, first);
+    if constexpr (HALVES) screen_row_halves<T>(a, b, reinterpret_cast<_Float16*>(sDyn), first);
+    else screen_row<T>(a, b, sX, first);
     bool any = false;
     uint2 found;
     if constexpr (NEAR != 0) found = i8_near<1, T, NEAR, T * 4>(e, b, sNearWords, any);
@@ -1443,7 +1477,8 @@ __global__ __launch_bounds__(256, 4) void i8_finish_kernel(ScreenFoldArgs a, I8N
     uint32_t hot[W], more[W];
     for (;;) {
         // Scores of what is new, and what is left of the list: what is no worse than its k-th.
-        screen_score<T, HALVES ? 2 : 4, HALVES>(a, sList, kept, count, sX);
+        if constexpr (HALVES) screen_score_halves<T>(a, sList, kept, count, reinterpret_cast<const _Float16*>(sDyn));
+        else screen_score<T, 4>(a, sList, kept, count, sX);
         __syncthreads();
         constexpr int L = kBestWords / T;
         uint64_t word[L];
