@@ -151,8 +151,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         for (uint32_t b = 0; b < 4; b++) {
             const uint32_t in_stage = b % NB;
             if (in_stage == 0) {
-                // The stage is there (three requests each for those behind it may not be), and every wavefront is done with the one before the last.
-                asm volatile("s_waitcnt vmcnt(15)" ::: "memory");
+                // The stage is there (three requests each for those behind it may not be), and every wavefront is done with the one before the last: also with
+                // what it has asked LDS for, as the side of that one's last block, whose sums become words behind this barrier as the compiler has it.
+                asm volatile("s_waitcnt vmcnt(15) lgkmcnt(0)" ::: "memory");
                 static_assert(kI8Stages == 8, "3 (kI8Stages - 3) requests");
                 __builtin_amdgcn_s_barrier();
                 asm volatile("" ::: "memory");
