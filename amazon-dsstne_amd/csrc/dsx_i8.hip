@@ -6,7 +6,8 @@
 // the items: 16 KiB of whole rows a stage, from memory straight to LDS in a ring.  So the items are all that moves, once per workgroup, and one
 // 16-byte LDS read feeds two matrix instructions: a stage takes half the LDS cycles that it takes matrix cycles.  (f16_sweep_kernel reads both operands from LDS,
 // 0.75 of a cycle for each matrix cycle, and writes 0.25: 4,096 x 512 x 1,000,000 with starts 2,464 us, 1,907 here; 4,096 x 128 x 1,000,000 without 866, 753.)
-// What bounds it: matrix and vector instructions of a SIMD add up (128 components: 0.50 and 1.09 of 1.52 million cycles, with two wavefronts a SIMD or four), and
+// What bounds it: matrix and vector instructions of a SIMD hardly overlap (128 components, two wavefronts a SIMD or four: 0.50 million cycles of matrix cores busy
+// and 1.09 of vector instructions, at four each, in a kernel of 1.52), and
 // a block's words take 70 vector instructions for each 32 queries, whatever the number of components.
 // The items are the row operand: a lane's sixteen results are sixteen items of one query.  While a block of 32 items is multiplied the sums of the one before
 // it become words; the ring keeps a stage longer for that, for what its sums start from.

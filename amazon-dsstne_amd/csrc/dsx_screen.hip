@@ -27,7 +27,7 @@
 // Searches of long tables that are kept go in bytes (screen_in_bytes): the matrix instructions form products of bytes at twice
 // the rate of halves, and read half as much.  x' = u q, w' = v r with whole numbers q, r of 127 at most; u is a row's unit, v one of 32 columns.  With
 // what the bytes leave out, x = x' + x", w = w' + w", the sum of the products of the bytes is exact and
-//   |s' - s| <= |x"| |w| + |x'| |w"| + (0.1 d + 16) 2^-24 |x| |w| + 3 u v      (the last two: screen_score's roundings, and a start's)
+//   |s' - s| <= |x"| |w| + |x'| |w"| + (1.25 d + 64) 2^-24 |x| |w| + 3 u v      (the last two: a score's roundings in whatever order, and a start's)
 // which is some fifteen times what halves leave open.  A word holds s' as an upper bound, and lies above it by
 //   |word - s'| <= 50 u v + 1e-3 |word|
 // at most: the lowest five bits of the float of 1.5 * 2^23 u v + s' say whose it is, and are taken for the largest they could be (33 units of its last place, a
@@ -614,6 +614,8 @@ template <int T, int STEPS = 2> __device__ __forceinline__ void screen_score(con
 
 // The same of an fp16 table: exact products, summed by the matrix instruction of the searches that are not screened, in their order (dsx_f16.hip), so that a
 // score has the same bits whichever way a search goes.  A wavefront takes 32 candidates, as the row operand; every column of the other one is the query.
+// Bound by the latency of the candidates' rows.  4,096 rows x 1,000,000 x 128 top 100: i8_finish_kernel 146 to 158 us (sixteen lanes a candidate, sums in an order of
+// their own: 152).
 template <int T> __device__ __forceinline__ void screen_score_halves(const ScreenFoldArgs& a, uint64_t* sList, uint32_t from, uint32_t count, const _Float16* sX)
 {
     const uint32_t lane = threadIdx.x % kWave, l32 = lane % 32, lhi = lane / 32;

@@ -325,7 +325,7 @@ int dsx_fc_topk_split(const float* X, uint32_t ldx, const float* W, const void* 
                       uint32_t* values, uint32_t position, const uint32_t* index, const uint64_t* filter_start, const uint64_t* filter_end,
                       const uint32_t* filter_index);
 /* dsx_fc_topk for a caller that keeps the weights' table of the 16-bit screening (two row-major copies of W, 6 bytes per element, and the
- * columns' norms, and a copy in bytes): dsx_screen_table_build fills dsx_screen_table_bytes(n, k_dim) bytes at `table` (device, 256-byte aligned) from W
+ * columns' norms, and where calls may go by it a copy in bytes): dsx_screen_table_build fills dsx_screen_table_bytes(n, k_dim) bytes at `table` (device, 256-byte aligned) from W
  * [k_dim][ldw] on the selected lane's stream; it has to be built again when W changes.  k_dim is 4,096 at most.  The call computes no
  * other results than dsx_fc_topk with its own table does; W is read for rows that have to be computed again.
  * dsx_fc_topk_screened_pays: 1 where this is the fastest way to the top-K of an output layer. */
@@ -399,8 +399,8 @@ int dsx_knn_search_f16(const void* items_f16, uint32_t rows_padded, uint32_t pad
                        float* elapsed_ms);
 size_t dsx_knn_workspace_bytes_f16(uint32_t rows_padded, uint32_t dim, uint32_t num_queries, uint32_t k);
 /* No counterpart in the reference: a copy of the fp16 table in bytes (half its size), by which searches of many queries find what has to be scored; as
- * dsx_knn_prepare, with dsx_knn_workspace_bytes_f16_prepared bytes and the storage DSX_KNN_FP16_PREPARED (*prepared, or 0).  The scores are the same products
- * of halves with fp32 sums. */
+ * dsx_knn_prepare, with dsx_knn_workspace_bytes_f16_prepared bytes and the storage DSX_KNN_FP16_PREPARED (*prepared, or 0).  The scores are the same bits
+ * as dsx_knn_search_f16's. */
 size_t dsx_knn_workspace_bytes_f16_prepared(uint32_t rows_padded, uint32_t dim, uint32_t num_queries, uint32_t k);
 int dsx_knn_prepare_f16(const void* items_f16, uint32_t rows_padded, uint32_t padding, uint32_t dim, uint32_t num_queries, uint32_t k, void* workspace,
                         size_t workspace_bytes, int* prepared);

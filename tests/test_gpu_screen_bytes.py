@@ -204,7 +204,7 @@ def test_search_of_halves(pkg, dsx, rng, form):
     if got[2]:   # the same search
         assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
         return
-    # sums of exact products of halves in two orders: both within dim roundings of the exact sum
+    # both within dim roundings of the exact sum (and the same bits: test_gpu_screen_bytes_halves.py)
     x, w = q.astype(np.float16).astype(np.float64), items.astype(np.float16).astype(np.float64)
     bound = dim * 2.0 ** -24 * np.sqrt((x ** 2).sum(axis=1))[:, None] * np.sqrt((w ** 2).sum(axis=1)).max()
     exact = np.einsum("qd,qkd->qk", x, w[got[1]])
